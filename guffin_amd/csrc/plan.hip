@@ -15,6 +15,7 @@
 #include "common.hpp"
 #include "selection_request.hpp"
 #include "receipt.hpp"
+#include "prefill_run.hpp"
 
 #include <algorithm>
 #include <vector>
@@ -228,7 +229,7 @@ int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t*
                  uint32_t position, const Scratch& s, void* priv_k, void* priv_v, float* out_hidden,
                  float* out_hidden_sums, uint32_t* status) {
     void* st = stream;
-    const uint32_t H = m.hidden, F = m.ffn, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
+    const uint32_t H = m.hidden, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
     const float attn_scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
     // the resident pass is the default where it is the faster one: models with a single KV head (the drafter's
     // small blocks); it can be forced for any model it covers
@@ -493,29 +494,57 @@ namespace guffin {
 namespace {
 
 struct PrefillScratch {
-    float *x, *x1, *u, *q, *kraw, *vraw, *a, *gate, *up, *h, *o;
+    float *x, *x1, *u, *q, *a;
+    float* planes;               // the GEMMs' partial planes
     float *rope_local, *rope_global;
     uint16_t *run_k, *run_v;
-    uint8_t* attn_ws;   // transposed values of the matrix-core attention
+    uint8_t* attn_ws;        // transposed values and the parts' states of the matrix-core attention
     uint8_t* image;
     uint32_t* positions;
     uint64_t bytes;
 };
 
+// the four GEMM launches of a block
+enum { kGemmQkv, kGemmO, kGemmGateUp, kGemmDown };
+struct PrefillLaunch { PrefillMatrix m[3]; uint32_t count, K; PrefillSplit split; };
+
+PrefillLaunch prefill_launch(const guffin_model_desc& m, uint32_t layer, int which, uint32_t rows) {
+    const guffin_layer_desc& L = m.layers[layer];
+    const uint32_t H = m.hidden, F = m.ffn, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
+    static constexpr int first[4] = {0, 3, 4, 6}, count[4] = {3, 1, 2, 1};
+    const uint32_t K[4] = {H, QW, H, F}, N[7] = {QW, KW, KW, H, F, F, H};
+    PrefillLaunch g {};
+    g.count = count[which];
+    g.K = K[which];
+    for (uint32_t i = 0; i < g.count; ++i) g.m[i] = {L.dtype[first[which] + i], L.tiles[first[which] + i], N[first[which] + i]};
+    g.split = prefill_split(g.m, g.count, rows, g.K);
+    return g;
+}
+
 PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, uint8_t* base) {
     Arena ar {base, 0, 0};
-    const uint64_t H = m.hidden, F = m.ffn, QW = uint64_t(m.q_heads) * m.head_dim, KW = uint64_t(m.kv_heads) * m.head_dim;
+    const uint64_t H = m.hidden, QW = uint64_t(m.q_heads) * m.head_dim, KW = uint64_t(m.kv_heads) * m.head_dim;
     PrefillScratch s {};
-    s.x = ar.take<float>(rows * H); s.x1 = ar.take<float>(rows * H); s.u = ar.take<float>(rows * H);
-    s.o = ar.take<float>(rows * H);
+    s.x = ar.take<float>(rows * H); s.x1 = ar.take<float>(rows * H);
+    s.u = ar.take<float>(H > kPrefillMaxWidth ? rows * H : 0);
     s.q = ar.take<float>(rows * QW); s.a = ar.take<float>(rows * QW);
-    s.kraw = ar.take<float>(rows * KW); s.vraw = ar.take<float>(rows * KW);
-    s.gate = ar.take<float>(rows * F); s.up = ar.take<float>(rows * F); s.h = ar.take<float>(rows * F);
+    uint64_t planes = 0;
+    for (uint32_t l = 0; l < m.layer_count; ++l) {
+        if (l && !std::memcmp(m.layers[l].dtype, m.layers[l - 1].dtype, sizeof(m.layers[l].dtype))) continue;
+        for (int which = 0; which < 4; ++which) {
+            const PrefillLaunch g = prefill_launch(m, l, which, rows);
+            uint64_t width = 0;
+            for (uint32_t i = 0; i < g.count; ++i) width += g.m[i].N;
+            planes = std::max(planes, uint64_t(g.split.slices) * rows * width);
+        }
+    }
+    s.planes = ar.take<float>(planes);
     s.rope_local = ar.take<float>(uint64_t(rows) * m.head_dim);
     s.rope_global = ar.take<float>(uint64_t(rows) * m.head_dim);
     s.run_k = ar.take<uint16_t>(rows * KW); s.run_v = ar.take<uint16_t>(rows * KW);
-    // V^T of every token a row may see: at most a full global ring plus the run, in whole 32-token tiles
-    s.attn_ws = ar.take<uint8_t>(uint64_t(m.kv_heads) * m.head_dim * 2 * ((uint64_t(m.ring_global) + rows + 63) & ~uint64_t{31}));
+    // every token a row may see: at most a full ring plus the run, in whole 32-token tiles from an aligned start
+    const uint32_t most = (std::max(m.ring_global, m.sliding_window) + rows + 95) & ~31u;
+    s.attn_ws = ar.take<uint8_t>(prefill_attention_most_bytes(rows, most, m.q_heads, m.kv_heads));
     const uint32_t widest = std::max({m.hidden, m.ffn, m.q_heads * m.head_dim});
     s.image = ar.take<uint8_t>(guffin_hip_prefill_image_bytes(rows, widest));
     s.positions = ar.take<uint32_t>(rows);
@@ -549,7 +578,7 @@ extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* mo
     const PrefillScratch s = prefill_layout(m, rows, static_cast<uint8_t*>(scratch));
     if (s.bytes > scratch_bytes) return fail(GUFFIN_E_CAPACITY, "prefill_rows: scratch arena too small");
     hipStream_t hs = as_stream(stream);
-    const uint32_t H = m.hidden, F = m.ffn, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
+    const uint32_t H = m.hidden, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
     const float attn_scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
     launch(fill_positions_kernel, dim3((rows + 255) / 256), dim3(256), 0, hs, s.positions, rows, position);
     GUFFIN_TRY(check_launch("prefill positions"));
@@ -557,37 +586,73 @@ extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* mo
     GUFFIN_TRY(guffin_hip_rope_table(stream, s.positions, s.rope_global, rows, m.head_dim, m.global_base, m.global_scale));
     GUFFIN_TRY(guffin_hip_embed(stream, m.embed_dtype, m.embed_rows, tokens, s.x, rows, H,
                                 std::sqrt(static_cast<float>(H)), m.vocab, status));
-    GUFFIN_TRY(guffin_hip_rms_norm(stream, s.x, 1, 0, m.layers[0].norm[0], nullptr, s.u, nullptr, rows, H, m.eps, status));
+    const bool fits = H <= kPrefillMaxWidth;   // the norms write the operand image themselves
+    if (fits) {
+        GUFFIN_TRY(prefill_norm(hs, s.x, m.layers[0].norm[0], s.image, rows, H, m.eps, status));
+    } else {
+        GUFFIN_TRY(guffin_hip_rms_norm(stream, s.x, 1, 0, m.layers[0].norm[0], nullptr, s.u, nullptr, rows, H, m.eps, status));
+        GUFFIN_TRY(guffin_hip_prefill_pack(stream, s.u, s.image, rows, H));
+    }
+    // residual + rms(the planes), then the next norm, as the next GEMM's operand or (at the end) the output rows
+    auto joint = [&](uint32_t planes, const float* gamma_post, const float* residual, float* out_residual, const float* gamma_next,
+                     float* out, const RunRows& run) {
+        if (fits)
+            return prefill_joint(hs, s.planes, planes, gamma_post, residual, out_residual, gamma_next, out, out ? nullptr : s.image, rows, H,
+                                 m.eps, run, status);
+        if (run.run_k)
+            GUFFIN_TRY(guffin_hip_publish_run(stream, run.run_k, run.run_v, run.ring_k, run.ring_v, rows, position, run.ring_mask, KW));
+        GUFFIN_TRY(guffin_hip_rms_norm_add_norm(stream, s.planes, planes, uint64_t(rows) * H, gamma_post, residual, out_residual, gamma_next,
+                                                out ? out : s.u, nullptr, rows, H, m.eps, status));
+        return out ? GUFFIN_OK : guffin_hip_prefill_pack(stream, s.u, s.image, rows, H);
+    };
+    PrefillLaunch g[4];
     for (uint32_t l = 0; l < m.layer_count; ++l) {
         const guffin_layer_desc& L = m.layers[l];
-        const bool local = is_local(m, l);
-        const float base = local ? m.local_base : m.global_base, scale = local ? 1.0f : m.global_scale;
-        const uint32_t ring_mask = (local ? m.ring_local : m.ring_global) - 1;
-        GUFFIN_TRY(guffin_hip_prefill_pack(stream, s.u, s.image, rows, H));
-        GUFFIN_TRY(guffin_hip_prefill_gemm(stream, L.dtype[0], L.tiles[0], s.image, s.q, rows, H, QW));
-        GUFFIN_TRY(guffin_hip_prefill_gemm(stream, L.dtype[1], L.tiles[1], s.image, s.kraw, rows, H, KW));
-        GUFFIN_TRY(guffin_hip_prefill_gemm(stream, L.dtype[2], L.tiles[2], s.image, s.vraw, rows, H, KW));
-        GUFFIN_TRY(guffin_hip_qkv_post(stream, s.q, s.kraw, s.vraw, 1, 1, 1, 0, 0, 0, L.norm[1], L.norm[2], s.positions,
-                                       s.q, s.run_k, s.run_v, rows, m.q_heads, m.kv_heads, m.head_dim, m.head_dim, base,
-                                       scale, m.eps, local ? s.rope_local : s.rope_global, status));
-        GUFFIN_TRY(guffin_hip_prefill_attention(stream, s.q, L.ring_k, L.ring_v, s.run_k, s.run_v, s.a, rows, position,
-                                                local ? m.sliding_window : 0u, ring_mask, m.q_heads, m.kv_heads,
-                                                m.head_dim, attn_scale, s.attn_ws));
-        GUFFIN_TRY(guffin_hip_publish_run(stream, s.run_k, s.run_v, L.ring_k, L.ring_v, rows, position, ring_mask, KW));
-        GUFFIN_TRY(guffin_hip_prefill_pack(stream, s.a, s.image, rows, QW));
-        GUFFIN_TRY(guffin_hip_prefill_gemm(stream, L.dtype[3], L.tiles[3], s.image, s.o, rows, QW, H));
-        GUFFIN_TRY(guffin_hip_rms_norm_add_norm(stream, s.o, 1, 0, L.norm[3], s.x, s.x1, L.norm[4], s.u, nullptr, rows, H,
-                                                m.eps, status));
-        GUFFIN_TRY(guffin_hip_prefill_pack(stream, s.u, s.image, rows, H));
-        GUFFIN_TRY(guffin_hip_prefill_gemm(stream, L.dtype[4], L.tiles[4], s.image, s.gate, rows, H, F));
-        GUFFIN_TRY(guffin_hip_prefill_gemm(stream, L.dtype[5], L.tiles[5], s.image, s.up, rows, H, F));
-        GUFFIN_TRY(guffin_hip_geglu(stream, s.gate, s.up, 1, 0, s.h, nullptr, rows, F));
-        GUFFIN_TRY(guffin_hip_prefill_pack(stream, s.h, s.image, rows, F));
-        GUFFIN_TRY(guffin_hip_prefill_gemm(stream, L.dtype[6], L.tiles[6], s.image, s.o, rows, F, H));
+        const bool local = is_local(m, l), same = l && !std::memcmp(L.dtype, m.layers[l - 1].dtype, sizeof(L.dtype));
+        const uint32_t ring_mask = (local ? m.ring_local : m.ring_global) - 1, window = local ? m.sliding_window : 0u;
+        static constexpr int first[4] = {0, 3, 4, 6};
+        for (int which = 0; which < 4; ++which) {
+            if (!same) g[which] = prefill_launch(m, l, which, rows);
+            for (uint32_t i = 0; i < g[which].count; ++i) g[which].m[i].tiles = L.tiles[first[which] + i];
+        }
+        auto gemm = [&](int which, float* const* y) {
+            return prefill_gemm_planes(hs, g[which].m, g[which].count, s.image, y, rows, g[which].K, g[which].split);
+        };
+        if ((reinterpret_cast<uintptr_t>(L.ring_k) | reinterpret_cast<uintptr_t>(L.ring_v)) & 3u)
+            return fail(GUFFIN_E_ALIGN, "prefill_rows: ring rows must be 4-byte aligned");
+        const uint64_t sq = g[kGemmQkv].split.slices, plane = uint64_t(rows) * sq;
+        float* const qkv[3] = {s.planes, s.planes + plane * QW, s.planes + plane * (QW + KW)};
+        GUFFIN_TRY(gemm(kGemmQkv, qkv));
+        const ValueSpan vs = value_span(rows, position, window);
+        const bool matrix = prefill_attention_on_matrix_core(s.q, L.ring_k, L.ring_v, s.run_k, s.run_v, m.q_heads, m.kv_heads);
+        QkvRun qr {};
+        qr.q_planes = qkv[0]; qr.k_planes = qkv[1]; qr.v_planes = qkv[2];
+        qr.q_norm = L.norm[1]; qr.k_norm = L.norm[2]; qr.rope_table = local ? s.rope_local : s.rope_global;
+        qr.q_out = s.q; qr.k_out = s.run_k; qr.v_out = s.run_v;
+        qr.ring_v = static_cast<const uint16_t*>(L.ring_v); qr.vt = reinterpret_cast<uint16_t*>(s.attn_ws);
+        qr.planes = static_cast<uint32_t>(sq); qr.rows = rows; qr.q_heads = m.q_heads; qr.kv_heads = m.kv_heads;
+        qr.position = position; qr.ring_mask = ring_mask; qr.first_visible = vs.first_visible; qr.base32 = vs.base32; qr.T = vs.T;
+        qr.eps = m.eps; qr.status = status;
+        GUFFIN_TRY(prefill_qkv(hs, qr));
+        if (matrix) {
+            GUFFIN_TRY(prefill_attention_run(hs, s.q, L.ring_k, s.run_k, nullptr, s.image, rows, position, window, ring_mask, m.q_heads,
+                                             m.kv_heads, attn_scale, s.attn_ws));
+        } else {
+            GUFFIN_TRY(guffin_hip_prefill_attention(stream, s.q, L.ring_k, L.ring_v, s.run_k, s.run_v, s.a, rows, position, window, ring_mask,
+                                                    m.q_heads, m.kv_heads, m.head_dim, attn_scale, nullptr));
+            GUFFIN_TRY(guffin_hip_prefill_pack(stream, s.a, s.image, rows, QW));
+        }
+        float* const one[1] = {s.planes};
+        GUFFIN_TRY(gemm(kGemmO, one));
+        const RunRows run {s.run_k, s.run_v, L.ring_k, L.ring_v, rows > ring_mask + 1 ? rows - (ring_mask + 1) : 0u, position, ring_mask, KW / 8};
+        GUFFIN_TRY(joint(g[kGemmO].split.slices, L.norm[3], s.x, s.x1, L.norm[4], nullptr, run));
+        float* const gu[2] = {s.planes, s.planes + uint64_t(g[kGemmGateUp].split.slices) * rows * m.ffn};
+        GUFFIN_TRY(gemm(kGemmGateUp, gu));
+        GUFFIN_TRY(prefill_geglu(hs, gu[0], gu[1], g[kGemmGateUp].split.slices, s.image, rows, m.ffn));
+        GUFFIN_TRY(gemm(kGemmDown, one));
         const bool last = l + 1 == m.layer_count;
-        GUFFIN_TRY(guffin_hip_rms_norm_add_norm(stream, s.o, 1, 0, L.norm[5], s.x1, s.x,
-                                                last ? m.out_norm : m.layers[l + 1].norm[0], last ? out_hidden : s.u,
-                                                nullptr, rows, H, m.eps, status));
+        GUFFIN_TRY(joint(g[kGemmDown].split.slices, L.norm[5], s.x1, s.x, last ? m.out_norm : m.layers[l + 1].norm[0],
+                         last ? out_hidden : nullptr, RunRows {}));
     }
     return GUFFIN_OK;
 }

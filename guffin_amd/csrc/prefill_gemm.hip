@@ -1,0 +1,705 @@
+// Prefill GEMM on the matrix core (gfx950): M activation rows times quantised weights.
+//
+// Replaces the reference's prefill matrix path (src/tensor/backends/metal/metal_kernels.mm:1031-1199, dispatch rules
+// metal_command_context.mm:384-401).
+//
+// Operands.  Weights come as the wave tiles of the decode GEMV (64 columns x one block), activations as the image of
+// prefill_image.hpp: fp16 hi and lo halves of x 2^-E.  Both halves of a row meet the same B operand and accumulate in
+// the same fp32 accumulator, so one 16x16x32 matrix instruction covers 16 rows.  B is exact: Q4_K sc * q (<= 945) as one
+// fused multiply-add of the biased quant, Q8_0 the signed quant, Q6_K s * (q - 32) as the nearest fp16 and the exact
+// rest of that rounding (at most one unit of 2049 or more; it meets the hi half only, its product with lo lies below
+// the image's own 22 bits).  A 256-element block accumulates inside the matrix instruction; its d and the span's
+// multiplier are applied in fp32, and Q4_K's -dmin m is one more instruction on the block's group sums.
+//
+// A workgroup is four waves on the same R * 16 rows and four neighbouring column tiles.  The A operand of a 64-element
+// chunk goes from memory to LDS without passing registers, two chunks ahead in three rotating buffers, one barrier per
+// chunk; weights are private to a wave and requested half a block ahead.
+#include "common.hpp"
+#include "prefill_image.hpp"
+#include "prefill_run.hpp"
+
+#include <algorithm>
+
+namespace guffin {
+namespace {
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
+
+constexpr uint32_t kCols = 64;       // columns per wave tile
+
+__host__ __device__ constexpr uint32_t block_bytes(int dtype) {
+    return dtype == GUFFIN_Q8_0 ? 34u : dtype == GUFFIN_Q4_K ? 144u : 210u;
+}
+__host__ __device__ constexpr uint32_t block_elems(int dtype) { return dtype == GUFFIN_Q8_0 ? 32u : 256u; }
+
+// one thread per 8 elements of a row
+__global__ void __launch_bounds__(256)
+prefill_pack_kernel(const float* __restrict__ x, uint8_t* __restrict__ blob, uint32_t M, uint32_t K) {
+    const ImageLayout L = image_layout(M, K);
+    const uint32_t per_row = K / 8;
+    const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= uint64_t(M) * per_row) return;   // whole spans leave together: a span is 4 or 32 aligned threads
+    const uint32_t row = static_cast<uint32_t>(i / per_row), t = static_cast<uint32_t>(i % per_row);
+    const float* src = x + size_t(row) * K + 8 * t;
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = src[k];
+    emit_image_values(v, t, row, L, blob);
+}
+
+__device__ __forceinline__ half8_t as_half8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return __builtin_bit_cast(half8_t, make_uint4(a, b, c, d));
+}
+__device__ __forceinline__ half2_t h2(uint32_t v) { return __builtin_bit_cast(half2_t, v); }
+__device__ __forceinline__ uint32_t u2(half2_t v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ half2_t splat(float f) { const _Float16 h = static_cast<_Float16>(f); return half2_t{h, h}; }
+
+// two bytes of w under the bias 1024, which comes off exactly, as a pair of halves; sel: their
+// places with 0x04 (the bias byte) in between
+__device__ __forceinline__ uint32_t bytes_as_halves(uint32_t w, uint32_t sel, float bias = 1024.f) {
+    return u2(h2(__builtin_amdgcn_perm(0x64646464u, w, sel)) - splat(bias));
+}
+
+// (w & mask) | c is one instruction if it needs no literal (it takes none) and at most one scalar register: the mask is kept
+// in a scalar, c in a vector register.  (Empty asm statements pin them; the instruction itself is the compiler's, whose
+// hazard handling around matrix instructions does not look into an asm statement.)
+__device__ __forceinline__ uint32_t scalar(uint32_t v) { asm("" : "+s"(v)); return v; }
+__device__ __forceinline__ uint32_t and_or(uint32_t w, uint32_t mask, uint32_t c) { return (w & mask) | c; }
+__device__ __forceinline__ uint32_t vector_bias() {
+    uint32_t c = 0x64006400u;
+    asm("" : "+v"(c));
+    return c;
+}
+
+// memory is read through buffer resources: an address is the resource and a wave-uniform offset (scalar registers)
+// plus the lane's 32-bit offset; reads past the end give zeros
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_resource(const void* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
+}
+__device__ __forceinline__ uint4 ld16(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t uniform_off) {
+    const uint4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(lane_off), static_cast<int>(uniform_off), 0);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ uint2 ld8(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t uniform_off) {
+    const uint2_t v = __builtin_amdgcn_raw_buffer_load_b64(r, static_cast<int>(lane_off), static_cast<int>(uniform_off), 0);
+    return make_uint2(v[0], v[1]);
+}
+__device__ __forceinline__ uint32_t ld4(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t uniform_off) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, static_cast<int>(lane_off), static_cast<int>(uniform_off), 0);
+}
+// 64 lanes x 16 (4) bytes straight into LDS at `to` (+ 16 (4) per lane)
+__device__ __forceinline__ void to_lds16(__amdgpu_buffer_rsrc_t r, uint8_t* to, uint32_t lane_off, uint32_t uniform_off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)to, 16, static_cast<int>(lane_off),
+                                             static_cast<int>(uniform_off), 0, 0);
+}
+__device__ __forceinline__ void to_lds4(__amdgpu_buffer_rsrc_t r, uint8_t* to, uint32_t lane_off, uint32_t uniform_off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)to, 4, static_cast<int>(lane_off),
+                                             static_cast<int>(uniform_off), 0, 0);
+}
+// the wave's requests but the N youngest have arrived and its LDS accesses are done, and so have every wave's
+template <int N>
+__device__ __forceinline__ void arrive() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
+struct GemmSegment { const uint8_t* tiles; float* y; uint64_t plane_stride; uint32_t N, dtype, first_group; };
+struct GemmArgs {
+    GemmSegment seg[3];
+    uint32_t segments, M, K;
+    const uint8_t* blob;
+};
+
+// what the workgroup keeps in LDS, R row tiles of 16
+template <int R>
+struct Stage {
+    static constexpr uint32_t kChunk = 4096 * R;              // 2 groups x R tiles x {hi, lo} x 1 KB; three of them
+    static constexpr uint32_t kSums = 3 * kChunk;             // the block's sums image
+    static constexpr uint32_t kMult = kSums + 2048;           // and its multipliers
+    static constexpr uint32_t kHead = kMult + 256;            // the waves' block headers (scales), two blocks
+    static constexpr uint32_t kBytes = kHead + 2 * 4 * 1280;
+};
+
+// The chunk's share of one wave: R of its 4R records.
+template <int R>
+struct Feed {
+    __amdgpu_buffer_rsrc_t img;
+    uint8_t* stage;
+    uint32_t lane16, base, group_stride, wv, last;   // base: this wave's first record of group 0
+    __device__ __forceinline__ void ask(uint32_t chunk, uint32_t buffer) const {
+        const uint32_t c = chunk < last ? chunk : last;   // past the end: the last chunk again, never read
+        const uint32_t from = base + (2 * c + (wv >> 1)) * group_stride;
+        uint8_t* to = stage + buffer * Stage<R>::kChunk + (wv >> 1) * (2048 * R) + (wv & 1) * (1024 * R);
+#pragma unroll
+        for (int i = 0; i < R; ++i) to_lds16(img, to + 1024 * i, lane16, from + 1024 * i);
+    }
+};
+
+template <int R>
+__device__ __forceinline__ void read_half(const uint8_t* group, uint32_t half, uint32_t lane16, half8_t (&a)[R]) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) a[r] = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(group + r * 2048 + half * 1024 + lane16));
+}
+// the schedule of a region of N matrix instructions: V vector instructions and, at first, an LDS read behind each
+template <int N, int V, int D>
+__device__ __forceinline__ void weave() {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (i < D) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// ---- Q4_K ------------------------------------------------------------------------------------------------
+// The B operands of group G (0..7) of a block for column groups 2P, 2P + 1, from its half block's quants and scale words.
+template <int G, int P>
+__device__ __forceinline__ void q4_operands(const uint4 (&q)[4], const uint32_t (&scw)[4], half8_t (&b)[4]) {
+    constexpr bool HIGH = G & 1;
+    constexpr int BYTE = G & 3, WORD = (G >> 1) & 1;
+    const uint32_t bias = vector_bias(), mask = scalar(HIGH ? 0x00F000F0u : 0x000F000Fu);
+#pragma unroll
+    for (int cg = 2 * P; cg < 2 * P + 2; ++cg) {
+        // the scale byte under the bias: 1024 + sc in both halves, then sc and -1024 sc (all exact in fp16); the high
+        // nibbles stay in bits 4-7, where they weigh 16
+        const half2_t sc = h2(__builtin_amdgcn_perm(0x64646464u, scw[cg], 0x04000400u | (BYTE << 16) | BYTE)) - splat(1024.f);
+        const half2_t off = sc * splat(HIGH ? -64.f : -1024.f), mul = HIGH ? sc * splat(0.0625f) : sc;
+        const uint32_t w0 = WORD ? q[cg].z : q[cg].x, w1 = WORD ? q[cg].w : q[cg].y;
+        auto piece = [&](uint32_t w) { return u2(__builtin_elementwise_fma(h2(and_or(w, mask, bias)), mul, off)); };
+        b[cg] = as_half8(piece(w0), piece(w0 >> 8), piece(w1), piece(w1 >> 8));
+    }
+}
+
+template <int R, bool FIRST>
+__device__ __forceinline__ void products(const half8_t (&a)[R], const half8_t (&b)[4], float4_t (&D)[4][R]) {
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+        for (int r = 0; r < R; ++r) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[r], b[cg], FIRST ? zero : D[cg][r], 0, 0, 0);
+}
+
+// A group is two regions of 4R matrix instructions, the hi and the lo halves of A against the same B.  While they run, the
+// next region's A operands come from LDS and the next group's B operands are formed, so a wave by itself keeps the matrix
+// pipe and the vector pipe busy together.  A chunk's last lo half is in registers when its last region starts: there the
+// workgroup meets, the next chunk has arrived and the one after the next but one is asked for in place of the old.
+template <int R>
+__device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& feed, uint8_t* stage, const uint8_t* tile_base,
+                                        uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
+    constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q4_K);
+    constexpr int V = (30 + 4 * R - 1) / (4 * R);   // vector instructions behind each matrix instruction
+    using S = Stage<R>;
+    const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
+    const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
+    uint8_t* const heads = stage + S::kHead + wv * 1280;
+    uint4 q[2][4];
+    uint32_t sc[4];
+    half8_t hi[R], lo[R], b[4], bn[4];
+    float4_t D[4][R];
+    auto ask_half = [&](uint32_t blk, int h, uint4 (&to)[4]) {
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) to[cg] = ld16(tile, lane16, blk * TB + 2048 * cg + 1024 * h);
+    };
+    auto ask_head = [&](uint32_t blk) { to_lds16(tile, heads + (blk & 1) * 5120, lane16, blk * TB + 8192); };
+    // the block's small operands: two waves bring the sums image, one the multipliers
+    auto ask_block = [&](uint32_t blk) {
+        if (wv < 2) to_lds16(feed.img, stage + S::kSums + 1024 * wv, lane16, static_cast<uint32_t>(L.sums_off) + (blk * (L.mpad / 16) + rt0) * 512 + 1024 * wv);
+        else if (wv == 2) to_lds4(feed.img, stage + S::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (blk * L.mpad + rt0 * 16) * 4);
+    };
+    auto scales = [&](uint32_t blk, int half) {
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) {
+            const uint32_t* h = reinterpret_cast<const uint32_t*>(heads + (blk & 1) * 5120 + 256 * cg + j * 16);
+            sc[cg] = half ? (h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u) : h[1] & 0x3F3F3F3Fu;
+        }
+    };
+    ask_half(b0, 0, q[0]);
+    ask_head(b0);
+    feed.ask(4 * b0, 0);
+    asm volatile("" ::: "memory");   // in this order
+    ask_half(b0, 1, q[1]);
+    feed.ask(4 * b0 + 1, 1);
+    asm volatile("" ::: "memory");
+    feed.ask(4 * b0 + 2, 2);
+    arrive<2 * R>();
+    scales(b0, 0);
+    read_half<R>(stage, 0, lane16, hi);
+    q4_operands<0, 0>(q[0], sc, b);
+    q4_operands<0, 1>(q[0], sc, b);
+    uint32_t rd = 0;   // the buffer of the chunk in work
+    for (uint32_t blk = b0; blk < b1; ++blk) {
+        const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
+        auto group = [&]<int G>() {
+            const uint8_t* now = stage + rd * S::kChunk + (G & 1) * (2048 * R);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (G == 3) scales(blk, 1);
+            if constexpr (G == 7) scales(next, 0);
+            read_half<R>(now, 1, lane16, lo);
+            q4_operands<(G + 1) & 7, 0>(q[G == 7 ? 0 : (G + 1) >> 2], sc, bn);
+            products<R, G == 0>(hi, b, D);
+            weave<4 * R, V, R>();
+            if constexpr (G & 1) {
+                arrive<R>();
+                if constexpr (G == 1) { ask_block(blk); ask_head(next); }
+                if constexpr (G == 3) ask_half(next, 0, q[0]);
+                if constexpr (G == 7) ask_half(next, 1, q[1]);
+                feed.ask(4 * blk + (G >> 1) + 3, rd);
+                rd = rd == 2 ? 0 : rd + 1;
+            }
+            const uint8_t* then = stage + rd * S::kChunk + ((G + 1) & 1) * (2048 * R);
+            __builtin_amdgcn_sched_barrier(0);
+            read_half<R>(then, 0, lane16, hi);
+            q4_operands<(G + 1) & 7, 1>(q[G == 7 ? 0 : (G + 1) >> 2], sc, bn);
+            products<R, false>(lo, b, D);
+            weave<4 * R, V, R>();
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg) b[cg] = bn[cg];
+        };
+        group.template operator()<0>();
+        group.template operator()<1>();
+        group.template operator()<2>();
+        group.template operator()<3>();
+        group.template operator()<4>();
+        group.template operator()<5>();
+        group.template operator()<6>();
+        group.template operator()<7>();
+        // block done: -dmin sum_g m_g (sum of group g) as one more instruction per tile, then one scale step
+        half8_t bm[4];
+        float d[4], dmin[4];
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) {
+            const uint4 h = *reinterpret_cast<const uint4*>(heads + (blk & 1) * 5120 + 256 * cg + j * 16);
+            d[cg] = h2f(h.x & 0xFFFFu);
+            dmin[cg] = -32.0f * h2f(h.x >> 16);
+            // minima against the sums' hi (k-slice 0) and lo (k-slice 1) halves; the upper lanes' share is zero
+            const uint32_t in = lane < 32 ? 0xFFFFFFFFu : 0u;
+            const uint32_t mn_a = h.z & 0x3F3F3F3Fu, mn_b = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
+            bm[cg] = as_half8(bytes_as_halves(mn_a, 0x04020400u) & in, bytes_as_halves(mn_a, 0x04030401u) & in,
+                              bytes_as_halves(mn_b, 0x04020400u) & in, bytes_as_halves(mn_b, 0x04030401u) & in);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const half8_t as = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(stage + S::kSums + 512 * r + (lane & 31) * 16));
+            const float4_t mult = *reinterpret_cast<const float4_t*>(stage + S::kMult + 64 * r + 16 * lg);
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg) {
+                const float4_t dm = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, bm[cg], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(mult[i], fmaf(dmin[cg], dm[i], d[cg] * D[cg][r][i]), acc[cg][r][i]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <int R>
+struct GroupA { half8_t hi[R], lo[R]; };
+
+template <int R>
+__device__ __forceinline__ void read_group(const uint8_t* stage, uint32_t lane16, GroupA<R>& a) {
+    read_half<R>(stage, 0, lane16, a.hi);
+    read_half<R>(stage, 1, lane16, a.lo);
+}
+
+// ---- Q6_K ------------------------------------------------------------------------------------------------
+// one 32-group of a half block for column groups 2P, 2P + 1; QD: its number in the half
+template <int R, int QD, bool FIRST>
+__device__ __forceinline__ void q6_group(const GroupA<R>& a, const uint4 (&ql)[4], const uint2 (&qh)[4], const uint2 (&sc)[4],
+                                         uint32_t sel, float4_t (&D)[4][R]) {
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+    const uint32_t bias = vector_bias(), low = scalar(0x000F000Fu), high = scalar(0x00300030u);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        half8_t b[2], rest[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int cg = 2 * p + c;
+            // the int8 scale + 128 under the bias; sel picks the lane's byte of the pair (a scale covers 16 elements)
+            const half2_t s = h2(__builtin_amdgcn_perm(0x64646464u, (QD >> 1) ? sc[cg].y : sc[cg].x, sel + (QD & 1) * 0x00020002u)) - splat(1152.f);
+            const uint32_t w[2] = {(QD & 1) ? ql[cg].z : ql[cg].x, (QD & 1) ? ql[cg].w : ql[cg].y};
+            const uint32_t h[2] = {qh[cg].x, qh[cg].y};
+            uint32_t bw[4], rw[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                constexpr int ls = QD >= 2 ? 4 : 0;
+                const uint32_t wk = w[k >> 1] >> (ls + 8 * (k & 1));
+                constexpr int up = 4 - 2 * QD;   // the two high bits go to bits 4-5
+                const int sh = 8 * (k & 1) - up;
+                const uint32_t hk = sh >= 0 ? h[k >> 1] >> (sh >= 0 ? sh : 0) : h[k >> 1] << (sh < 0 ? -sh : 0);
+                const half2_t q = h2(and_or(wk, low, and_or(hk, high, bias))) - splat(1056.f);
+                const half2_t prod = s * q;                              // nearest
+                bw[k] = u2(prod);
+                rw[k] = u2(__builtin_elementwise_fma(s, q, -prod));      // what that rounding left
+            }
+            b[c] = as_half8(bw[0], bw[1], bw[2], bw[3]);
+            rest[c] = as_half8(rw[0], rw[1], rw[2], rw[3]);
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                D[2 * p + c][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi[r], b[c], FIRST ? zero : D[2 * p + c][r], 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < R; ++r) D[2 * p + c][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.lo[r], b[c], D[2 * p + c][r], 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < R; ++r) D[2 * p + c][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi[r], rest[c], D[2 * p + c][r], 0, 0, 0);
+    }
+}
+
+template <int R>
+__device__ __forceinline__ void q6_walk(const GemmArgs& A, const ImageLayout& L, const Feed<R>& feed, uint8_t* stage,
+                                        const uint8_t* tile_base, uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
+    constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q6_K);
+    const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
+    const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
+    const uint32_t sel = lane >= 32 ? 0x04010401u : 0x04000400u;
+    uint4 ql[2][4];
+    uint2 qh[2][4], sc[2][4];
+    uint32_t dw[4];
+    auto ask_half = [&](uint32_t b, int h, int to) {
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) {
+            ql[to][cg] = ld16(tile, lane16, b * TB + 2048 * cg + 1024 * h);
+            qh[to][cg] = ld8(tile, lane16 + 8 * h, b * TB + 8192 + 1024 * cg);
+            sc[to][cg] = ld8(tile, j * 16 + 8 * h, b * TB + 12288 + 256 * cg);
+        }
+    };
+    auto flip = [&](int to) {   // int8 -> +128
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) { sc[to][cg].x ^= 0x80808080u; sc[to][cg].y ^= 0x80808080u; }
+    };
+    ask_half(b0, 0, 0);
+    feed.ask(4 * b0, 0);
+    asm volatile("" ::: "memory");   // in this order
+    feed.ask(4 * b0 + 1, 1);
+    uint32_t rd = 0, wr = 2;
+    auto next = [&] { rd = rd == 2 ? 0 : rd + 1; wr = wr == 2 ? 0 : wr + 1; };
+    float4_t D[4][R];
+    GroupA<R> a;
+    for (uint32_t b = b0; b < b1; ++b) {
+        const uint32_t bn = b + 1 < b1 ? b + 1 : b;
+        arrive<R>();
+        ask_half(b, 1, 1);
+        if (wv == 0) to_lds4(feed.img, stage + Stage<R>::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (b * L.mpad + rt0 * 16) * 4);
+        feed.ask(4 * b + 2, wr);
+        flip(0);
+        read_group<R>(stage + rd * Stage<R>::kChunk, lane16, a);
+        q6_group<R, 0, true>(a, ql[0], qh[0], sc[0], sel, D);
+        read_group<R>(stage + rd * Stage<R>::kChunk + 2048 * R, lane16, a);
+        q6_group<R, 1, false>(a, ql[0], qh[0], sc[0], sel, D);
+        next();
+        arrive<R>();
+        feed.ask(4 * b + 3, wr);
+        read_group<R>(stage + rd * Stage<R>::kChunk, lane16, a);
+        q6_group<R, 2, false>(a, ql[0], qh[0], sc[0], sel, D);
+        read_group<R>(stage + rd * Stage<R>::kChunk + 2048 * R, lane16, a);
+        q6_group<R, 3, false>(a, ql[0], qh[0], sc[0], sel, D);
+        next();
+        arrive<R>();
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) dw[cg] = ld4(tile, (j >> 1) * 4, b * TB + 13312 + 32 * cg);
+        ask_half(bn, 0, 0);
+        feed.ask(4 * b + 4, wr);
+        flip(1);
+        read_group<R>(stage + rd * Stage<R>::kChunk, lane16, a);
+        q6_group<R, 0, false>(a, ql[1], qh[1], sc[1], sel, D);
+        read_group<R>(stage + rd * Stage<R>::kChunk + 2048 * R, lane16, a);
+        q6_group<R, 1, false>(a, ql[1], qh[1], sc[1], sel, D);
+        next();
+        arrive<R>();
+        feed.ask(4 * b + 5, wr);
+        read_group<R>(stage + rd * Stage<R>::kChunk, lane16, a);
+        q6_group<R, 2, false>(a, ql[1], qh[1], sc[1], sel, D);
+        read_group<R>(stage + rd * Stage<R>::kChunk + 2048 * R, lane16, a);
+        q6_group<R, 3, false>(a, ql[1], qh[1], sc[1], sel, D);
+        next();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float4_t mult = *reinterpret_cast<const float4_t*>(stage + Stage<R>::kMult + 64 * r + 16 * lg);
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg) {
+                const float d = h2f((dw[cg] >> (16 * (j & 1u))) & 0xFFFFu);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(d * mult[i], D[cg][r][i], acc[cg][r][i]);
+            }
+        }
+    }
+}
+
+// grid (row chunks, column groups of 256 over all segments, k-slices), 256 threads.  Consecutive workgroups walk the
+// rows, so that an XCD's L2 keeps its share of the image.
+template <int R, int KINDS>
+__global__ void __launch_bounds__(256, 2)
+prefill_gemm_kernel(GemmArgs A) {
+    __shared__ __attribute__((aligned(16))) uint8_t stage[Stage<R>::kBytes];
+    const ImageLayout L = image_layout(A.M, A.K);
+    const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t s = 0;
+    while (s + 1 < A.segments && blockIdx.y >= A.seg[s + 1].first_group) ++s;
+    const GemmSegment seg = A.seg[s];
+    const uint32_t tile_index = (blockIdx.y - seg.first_group) * 4 + wv, nblk = A.K / 256, rt0 = blockIdx.x * R;
+    const bool valid = tile_index < seg.N / kCols;   // a wave past the last tile works on tile 0 and stores nothing
+    const uint32_t b0 = blockIdx.z * nblk / gridDim.z, b1 = (blockIdx.z + 1) * nblk / gridDim.z;
+    Feed<R> feed;
+    feed.img = make_resource(A.blob, static_cast<uint32_t>(L.bytes));
+    feed.stage = stage;
+    feed.lane16 = lane * 16;
+    feed.group_stride = (L.mpad / 16) * 2048;
+    feed.base = rt0 * 2048 + (wv & 1) * (1024 * R);
+    feed.wv = wv;
+    feed.last = 4 * b1 - 1;
+    float acc[4][R][4];
+#pragma unroll
+    for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[cg][r][i] = 0.f;
+    if (KINDS == 1 || (KINDS == 3 && seg.dtype == GUFFIN_Q4_K))
+        q4_walk<R>(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q4_K)), rt0, b0, b1, acc);
+    else
+        q6_walk<R>(A, L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q6_K)), rt0, b0, b1, acc);
+    // the chunks asked for past the end are still on their way into this workgroup's LDS
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (!valid) return;
+    float* y = seg.y + blockIdx.z * seg.plane_stride;
+    const uint32_t col = tile_index * kCols + (lane & 15), row0 = rt0 * 16 + 4 * (lane >> 4);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t row = row0 + 16 * r + i;
+            if (row < A.M)
+#pragma unroll
+                for (int cg = 0; cg < 4; ++cg) y[size_t(row) * seg.N + col + 16 * cg] = acc[cg][r][i];
+        }
+}
+
+// ---- Q8_0 ------------------------------------------------------------------------------------------------
+// The same workgroup and stages; a 32-element block is one group, so its d and the span's multiplier are applied after
+// the two matrix instructions (hi, lo) of a tile.  grid as above, k-slices in chunks of two blocks.
+template <int R>
+__global__ void __launch_bounds__(256, 2)
+prefill_gemm_q8_kernel(GemmArgs A) {
+    constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q8_0), kSlot = Stage<R>::kChunk + 512;   // chunk, its two groups' multipliers
+    __shared__ __attribute__((aligned(16))) uint8_t stage[3 * kSlot];
+    const ImageLayout L = image_layout(A.M, A.K);
+    const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, lg = lane >> 4;
+    uint32_t s = 0;
+    while (s + 1 < A.segments && blockIdx.y >= A.seg[s + 1].first_group) ++s;
+    const GemmSegment seg = A.seg[s];
+    const uint32_t tile_index = (blockIdx.y - seg.first_group) * 4 + wv, nblk = A.K / 32, rt0 = blockIdx.x * R;
+    const bool valid = tile_index < seg.N / kCols;
+    const uint32_t chunks = (nblk + 1) / 2, c0 = blockIdx.z * chunks / gridDim.z, c1 = (blockIdx.z + 1) * chunks / gridDim.z;
+    const __amdgpu_buffer_rsrc_t img = make_resource(A.blob, static_cast<uint32_t>(L.bytes));
+    const __amdgpu_buffer_rsrc_t tile = make_resource(seg.tiles + size_t(valid ? tile_index : 0) * nblk * TB, nblk * TB);
+    const uint32_t lane16 = lane * 16, group_stride = (L.mpad / 16) * 2048, shift = L.span == 256 ? 3 : 0;
+    const uint32_t base = rt0 * 2048 + (wv & 1) * (1024 * R), mult_off = static_cast<uint32_t>(L.mult_off) + rt0 * 64;
+    auto ask = [&](uint32_t chunk, uint32_t buffer) {
+        const uint32_t c = chunk < c1 ? chunk : c1 - 1;
+        uint8_t* to = stage + buffer * kSlot;
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            to_lds16(img, to + (wv >> 1) * (2048 * R) + (wv & 1) * (1024 * R) + 1024 * i, lane16, base + min(2 * c + (wv >> 1), nblk - 1) * group_stride + 1024 * i);
+        if (wv < 2) to_lds4(img, to + Stage<R>::kChunk + 256 * wv, lane * 4, mult_off + (min(2 * c + wv, nblk - 1) >> shift) * L.mpad * 4);
+    };
+    uint4 q[2][2][2];       // [buffer][group][piece]
+    uint32_t dw[2][2][4];
+    auto ask_weights = [&](uint32_t chunk, int to) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t at = min(2 * chunk + h, nblk - 1) * TB;   // past the end: the last block again, never used
+            q[to][h][0] = ld16(tile, lane16, at);
+            q[to][h][1] = ld16(tile, lane16, at + 1024);
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg) dw[to][h][cg] = ld4(tile, (j >> 1) * 4, at + 2048 + 32 * cg);
+        }
+    };
+    float acc[4][R][4];
+#pragma unroll
+    for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[cg][r][i] = 0.f;
+    ask_weights(c0, 0);
+    ask(c0, 0);
+    asm volatile("" ::: "memory");   // in this order
+    ask(c0 + 1, 1);
+    uint32_t rd = 0, wr = 2;
+    auto chunk = [&](uint32_t c, int now) {
+        arrive<R>();
+        ask_weights(c + 1, now ^ 1);
+        ask(c + 2, wr);
+        const uint8_t* from = stage + rd * kSlot;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (2 * c + h >= nblk) break;   // an odd number of blocks: the last chunk has one
+            GroupA<R> a;
+            read_group<R>(from + h * (2048 * R), lane16, a);
+            half8_t b[4];
+            float d[4];
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg) {
+                const uint4 piece = q[now][h][cg >> 1];
+                const uint32_t w0 = ((cg & 1) ? piece.z : piece.x) ^ 0x80808080u, w1 = ((cg & 1) ? piece.w : piece.y) ^ 0x80808080u;
+                b[cg] = as_half8(bytes_as_halves(w0, 0x04020400u, 1152.f), bytes_as_halves(w0, 0x04030401u, 1152.f),
+                                 bytes_as_halves(w1, 0x04020400u, 1152.f), bytes_as_halves(w1, 0x04030401u, 1152.f));
+                d[cg] = h2f((dw[now][h][cg] >> (16 * (j & 1u))) & 0xFFFFu);
+            }
+            float4_t D[4][R];
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+                for (int r = 0; r < R; ++r) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi[r], b[cg], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+                for (int r = 0; r < R; ++r) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.lo[r], b[cg], D[cg][r], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float4_t mult = *reinterpret_cast<const float4_t*>(from + Stage<R>::kChunk + 256 * h + 64 * r + 16 * lg);
+#pragma unroll
+                for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(d[cg] * mult[i], D[cg][r][i], acc[cg][r][i]);
+            }
+        }
+        rd = rd == 2 ? 0 : rd + 1;
+        wr = wr == 2 ? 0 : wr + 1;
+    };
+    for (uint32_t c = c0; c < c1; c += 2) {
+        chunk(c, 0);
+        if (c + 1 < c1) chunk(c + 1, 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (!valid) return;
+    float* y = seg.y + blockIdx.z * seg.plane_stride;
+    const uint32_t col = tile_index * kCols + j, row0 = rt0 * 16 + 4 * lg;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t row = row0 + 16 * r + i;
+            if (row < A.M)
+#pragma unroll
+                for (int cg = 0; cg < 4; ++cg) y[size_t(row) * seg.N + col + 16 * cg] = acc[cg][r][i];
+        }
+}
+
+int gemm_launch(hipStream_t s, GemmArgs& a, uint32_t slices, uint32_t R) {
+    uint32_t groups = 0, kinds = 0;
+    for (uint32_t i = 0; i < a.segments; ++i) {
+        a.seg[i].first_group = groups;
+        groups += (a.seg[i].N / kCols + 3) / 4;
+        kinds |= a.seg[i].dtype == GUFFIN_Q4_K ? 1u : a.seg[i].dtype == GUFFIN_Q6_K ? 2u : 4u;
+    }
+    const dim3 grid((a.M + 16 * R - 1) / (16 * R), groups, slices), block(256);
+#define GUFFIN_PG(R_) \
+    do { \
+        if (kinds == 1) launch(prefill_gemm_kernel<R_, 1>, grid, block, 0, s, a); \
+        else if (kinds == 2) launch(prefill_gemm_kernel<R_, 2>, grid, block, 0, s, a); \
+        else if (kinds == 3) launch(prefill_gemm_kernel<R_, 3>, grid, block, 0, s, a); \
+        else launch(prefill_gemm_q8_kernel<R_>, grid, block, 0, s, a); \
+    } while (0)
+    if (R == 1) GUFFIN_PG(1); else if (R == 2) GUFFIN_PG(2); else if (R == 3) GUFFIN_PG(3); else GUFFIN_PG(4);
+#undef GUFFIN_PG
+    return check_launch("prefill_gemm");
+}
+
+// Time of a launch by a model of the chip, in microseconds: a workgroup takes `start` to its first product and `block` per 256
+// elements of K (measured, two workgroups on a compute unit; alone it takes three quarters of that), 512 run at once, and a
+// plane costs a write and a read at the memory's rate.
+constexpr float kStart = 3.5f, kBlockQ4[4] = {3.1f, 4.2f, 5.4f, 7.0f}, kBlockQ6[4] = {3.8f, 5.4f, 7.2f, 9.0f}, kPlaneBytesPerUs = 4.0e6f;
+
+PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K, uint32_t most) {
+    uint32_t groups = 0, width = 0;
+    bool q6 = false, q8 = false;
+    for (uint32_t i = 0; i < count; ++i) {
+        groups += (m[i].N / kCols + 3) / 4;
+        width += m[i].N;
+        q6 |= m[i].dtype == GUFFIN_Q6_K;
+        q8 |= m[i].dtype == GUFFIN_Q8_0;
+    }
+    const uint32_t units = q8 ? (K + 63) / 64 : K / 256;   // what a slice is made of
+    PrefillSplit best {1, 1};
+    float least = 0.f;
+    for (uint32_t R = 1; R <= 4; ++R) {
+        const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
+        const float block = (q6 ? kBlockQ6 : kBlockQ4)[R - 1] * (q8 ? 0.3f : 1.0f);
+        for (uint32_t S = 1; S <= std::min(units, most); ++S) {
+            const uint32_t n = chunks * groups * S, rounds = (n + 511) / 512;
+            const float each = kStart + float((units + S - 1) / S) * block * (n <= 256 ? 0.75f : 1.0f);
+            const float cost = each * (rounds == 1 ? 1.0f : std::max(1.0f, 0.5f * (float(rounds) + float(n) / 512.0f)))
+                + float(S) * 8.0f * float(M) * float(width) / kPlaneBytesPerUs;
+            if ((R == 1 && S == 1) || cost < least) { best = {R, S}; least = cost; }
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+PrefillSplit prefill_split(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K) { return split_for(m, count, M, K, 16); }
+
+int prefill_gemm_planes(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M,
+                        uint32_t K, PrefillSplit split) {
+    bool q8 = false, k = false;
+    for (uint32_t i = 0; i < count; ++i) {
+        if (K % block_elems(m[i].dtype) != 0 || m[i].N % kCols != 0) return fail(GUFFIN_E_SHAPE, "prefill_gemm: need K % block == 0 and N % 64 == 0");
+        if (reinterpret_cast<uintptr_t>(m[i].tiles) & 15u) return fail(GUFFIN_E_ALIGN, "prefill_gemm: tiles need 16-byte alignment");
+        (m[i].dtype == GUFFIN_Q8_0 ? q8 : k) = true;
+    }
+    if (image_layout(M, K).bytes >= (size_t(1) << 31)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: the image of M x K exceeds 2 GiB, split the rows");
+    if (q8 && k) {   // the formats' workgroups walk K in different units: a launch each
+        for (uint32_t i = 0; i < count; ++i)
+            if (int rc = prefill_gemm_planes(s, m + i, 1, image, y + i, M, K, split)) return rc;
+        return GUFFIN_OK;
+    }
+    GemmArgs a {};
+    for (uint32_t i = 0; i < count; ++i)
+        a.seg[i] = {static_cast<const uint8_t*>(m[i].tiles), y[i], uint64_t(M) * m[i].N, m[i].N, static_cast<uint32_t>(m[i].dtype), 0};
+    a.segments = count; a.M = M; a.K = K; a.blob = image;
+    return gemm_launch(s, a, split.slices, split.row_tiles);
+}
+}  // namespace guffin
+
+using namespace guffin;
+
+extern "C" uint64_t guffin_hip_prefill_image_bytes(uint32_t M, uint32_t K) {
+    if (M == 0 || K == 0 || K % 32 != 0) return 0;
+    return image_layout(M, K).bytes;
+}
+
+extern "C" int guffin_hip_prefill_pack(void* stream, const float* x, void* image, uint32_t M, uint32_t K) {
+    if (!x || !image) return fail(GUFFIN_E_ARG, "prefill_pack: null pointer");
+    if (M == 0 || K == 0 || K % 32 != 0) return fail(GUFFIN_E_SHAPE, "prefill_pack: K must be a positive multiple of 32");
+    if (reinterpret_cast<uintptr_t>(image) & 255u) return fail(GUFFIN_E_ALIGN, "prefill_pack: the image must be 256-byte aligned");
+    const uint64_t threads = uint64_t(M) * (K / 8);
+    launch(prefill_pack_kernel, dim3(static_cast<uint32_t>((threads + 255) / 256)), dim3(256), 0,
+                       as_stream(stream), x, static_cast<uint8_t*>(image), M, K);
+    return check_launch("prefill_pack");
+}
+
+extern "C" int guffin_hip_prefill_gemm(void* stream, int dtype, const void* tiles, const void* image, float* y,
+                                       uint32_t M, uint32_t K, uint32_t N) {
+    if (!tiles || !image || !y) return fail(GUFFIN_E_ARG, "prefill_gemm: null pointer");
+    if (dtype < GUFFIN_Q8_0 || dtype > GUFFIN_Q6_K) return fail(GUFFIN_E_ARG, "prefill_gemm: unknown dtype");
+    if (M == 0 || K == 0 || N == 0 || K % block_elems(dtype) != 0 || N % kCols != 0)
+        return fail(GUFFIN_E_SHAPE, "prefill_gemm: need K % block == 0 and N % 64 == 0");
+    if ((reinterpret_cast<uintptr_t>(tiles) & 15u) || (reinterpret_cast<uintptr_t>(image) & 255u))
+        return fail(GUFFIN_E_ALIGN, "prefill_gemm: tiles need 16-byte, the image 256-byte alignment");
+    // the kernels address the image with 32-bit offsets
+    if (image_layout(M, K).bytes >= (size_t(1) << 31)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: the image of M x K exceeds 2 GiB, split the rows");
+    GemmArgs a {};
+    a.seg[0] = {static_cast<const uint8_t*>(tiles), y, 0, N, static_cast<uint32_t>(dtype), 0};
+    a.segments = 1; a.M = M; a.K = K; a.blob = static_cast<const uint8_t*>(image);
+    const PrefillMatrix m {dtype, tiles, N};
+    return gemm_launch(as_stream(stream), a, 1, split_for(&m, 1, M, K, 1).row_tiles);
+}

@@ -1,0 +1,275 @@
+// The operators between the GEMMs of a prefill pass (gfx950), each reading the k-slice planes the GEMM before left and
+// writing the operand image the GEMM after reads (prefill_image.hpp), so that no activation crosses memory a second time:
+//
+//   first norm   rms(x)                                       reference: encode_rms_norm
+//   qkv          head norms, NeoX rotation, fp16 narrowing, and the values of every visible token transposed for the
+//                attention                                    gemma_target_runtime.cpp:88-133, metal_kernels.mm:2406-2486
+//   joint        residual + rms(a), then rms of that          gemma_target_runtime.cpp:156-173, 201-213; the joint after the
+//                attention also publishes the run's K/V       attention, when nobody reads the ring rows they replace
+//   geglu        gelu_tanh(gate) * up                         metal_kernels.mm:1827-1843
+#include "common.hpp"
+#include "prefill_image.hpp"
+#include "prefill_run.hpp"
+#include "receipt.hpp"
+
+namespace guffin {
+namespace {
+
+__device__ __forceinline__ float block_total(float v, float* scratch) {
+    v = wave_sum(v);
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, waves = (blockDim.x + 63) >> 6;
+    __syncthreads();  // scratch may still be read from a previous call
+    if (lane == 0) scratch[wv] = v;
+    __syncthreads();
+    float t = 0.f;
+    for (uint32_t i = 0; i < waves; ++i) t += scratch[i];  // same order on every thread
+    return t;
+}
+
+// 8 consecutive floats of `planes` planes, summed in plane order; up to B planes are requested before the first add
+template <int B>
+__device__ __forceinline__ void sum_planes8(const float* p, uint32_t planes, size_t stride, float (&v)[8]) {
+    for (uint32_t s0 = 0; s0 < planes; s0 += B) {
+        float4 a[B], b[B];
+#pragma unroll
+        for (int s = 0; s < B; ++s)
+            if (s0 + s < planes) {
+                a[s] = *reinterpret_cast<const float4*>(p + (s0 + s) * stride);
+                b[s] = *reinterpret_cast<const float4*>(p + (s0 + s) * stride + 4);
+            }
+#pragma unroll
+        for (int s = 0; s < B; ++s)
+            if (s0 + s < planes) {
+                const float w[8] = {a[s].x, a[s].y, a[s].z, a[s].w, b[s].x, b[s].y, b[s].z, b[s].w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = s0 + s == 0 ? w[i] : v[i] + w[i];
+            }
+    }
+}
+__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
+    const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void store8(float* p, const float (&v)[8]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+// the same where the caller's pointer may start at any word
+__device__ __forceinline__ void load8_words(const float* p, float (&v)[8]) {
+    const float4 a = ldf4_a4(p), b = ldf4_a4(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void store8_words(float* p, const float (&v)[8]) {
+    *reinterpret_cast<F4a4*>(p) = F4a4 {v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<F4a4*>(p + 4) = F4a4 {v[4], v[5], v[6], v[7]};
+}
+
+// one workgroup per row, a thread owns 8 consecutive columns
+__global__ void __launch_bounds__(1024)
+prefill_norm_kernel(const float* __restrict__ x, const float* __restrict__ gamma, uint8_t* __restrict__ image, uint32_t rows,
+                    uint32_t width, float eps, uint32_t* __restrict__ status) {
+    __shared__ float scratch[16];
+    const uint32_t r = blockIdx.x, t = threadIdx.x;
+    const bool active = t < width / 8;
+    float v[8] = {}, g[8] = {};
+    if (active) { load8(x + size_t(r) * width + 8 * t, v); load8_words(gamma + 8 * t, g); }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
+    const float inv = 1.0f / sqrtf(block_total(ss, scratch) / static_cast<float>(width) + eps);
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) { v[i] = v[i] * inv * g[i]; bad |= !isfinite(v[i]); }
+    if (active) emit_image_values(v, t, r, image_layout(rows, width), image);
+    if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
+}
+
+// Workgroups [0, rows): one row each.  The rest copy the run's fp16 K/V rows to their ring slots, 16 bytes per thread.
+__global__ void __launch_bounds__(1024)
+prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_stride, const float* __restrict__ gamma_post,
+                     const float* __restrict__ residual, float* __restrict__ out_residual, const float* __restrict__ gamma_next,
+                     float* __restrict__ out_norm, uint8_t* __restrict__ image, uint32_t rows, uint32_t width, float eps,
+                     RunRows run, uint32_t* __restrict__ status) {
+    if (blockIdx.x >= rows) {
+        const uint64_t i = uint64_t(blockIdx.x - rows) * blockDim.x + threadIdx.x;
+        if (i >= uint64_t(rows - run.first_row) * run.row_vec) return;
+        const uint32_t row = run.first_row + static_cast<uint32_t>(i / run.row_vec), c = static_cast<uint32_t>(i % run.row_vec);
+        const size_t dst = size_t((run.position + row) & run.ring_mask) * run.row_vec + c;
+        static_cast<U4a4*>(run.ring_k)[dst] = static_cast<const U4a4*>(run.run_k)[size_t(row) * run.row_vec + c];
+        static_cast<U4a4*>(run.ring_v)[dst] = static_cast<const U4a4*>(run.run_v)[size_t(row) * run.row_vec + c];
+        return;
+    }
+    __shared__ float scratch[16];
+    const uint32_t r = blockIdx.x, t = threadIdx.x;
+    const bool active = t < width / 8;
+    const size_t at = size_t(r) * width + 8 * t;
+    float v[8] = {}, gp[8] = {}, gn[8] = {}, res[8] = {};
+    if (active) {
+        load8_words(gamma_post + 8 * t, gp);
+        load8(residual + at, res);
+        load8_words(gamma_next + 8 * t, gn);
+        sum_planes8<4>(x + at, planes, plane_stride, v);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
+    float inv = 1.0f / sqrtf(block_total(ss, scratch) / static_cast<float>(width) + eps);
+    bool bad = false;
+    ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        v[i] = v[i] * inv * gp[i] + res[i];
+        bad |= !isfinite(v[i]);
+        ss = fmaf(v[i], v[i], ss);
+    }
+    if (active) store8(out_residual + at, v);
+    inv = 1.0f / sqrtf(block_total(ss, scratch) / static_cast<float>(width) + eps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = v[i] * inv * gn[i];
+    if (active) {
+        if (image) emit_image_values(v, t, r, image_layout(rows, width), image);
+        else store8_words(out_norm + at, v);
+    }
+    if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
+}
+
+// one thread per 8 columns of a row
+__global__ void __launch_bounds__(256)
+prefill_geglu_kernel(const float* __restrict__ gate, const float* __restrict__ up, uint32_t planes, size_t plane_stride,
+                     uint8_t* __restrict__ image, uint32_t rows, uint32_t width) {
+    const uint32_t per_row = width / 8;
+    const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= uint64_t(rows) * per_row) return;   // whole spans leave together
+    const uint32_t row = static_cast<uint32_t>(i / per_row), t = static_cast<uint32_t>(i % per_row);
+    float g[8], u[8];
+    sum_planes8<2>(gate + size_t(row) * width + 8 * t, planes, plane_stride, g);
+    sum_planes8<2>(up + size_t(row) * width + 8 * t, planes, plane_stride, u);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) g[k] = geglu_value(g[k], u[k]);
+    emit_image_values(g, t, row, image_layout(rows, width), image);
+}
+
+// Workgroups [0, head_groups): four (row, query or key head) pairs, a wave each.  The rest: 32 visible tokens of one KV
+// head's values each, from the ring or (the run's own, narrowed and kept on the way) from the planes, written transposed.
+__global__ void __launch_bounds__(256)
+prefill_qkv_kernel(QkvRun a) {
+    constexpr uint32_t HD = 256, PITCH = HD + 8;
+    __shared__ __attribute__((aligned(16))) uint16_t tile[32][PITCH];
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    bool bad = false;
+    if (blockIdx.x < a.head_groups) {
+        const uint32_t per_row = a.q_heads + a.kv_heads, p = blockIdx.x * 4 + wv;
+        if (p >= a.rows * per_row) return;
+        const uint32_t r = p / per_row, h = p % per_row;
+        const bool is_q = h < a.q_heads;
+        const uint32_t hh = is_q ? h : h - a.q_heads, heads = is_q ? a.q_heads : a.kv_heads;
+        const size_t off = (size_t(r) * heads + hh) * HD;
+        const size_t stride = size_t(a.rows) * heads * HD;
+        const float* src = (is_q ? a.q_planes : a.k_planes) + off;
+        const float* gamma = is_q ? a.q_norm : a.k_norm;
+        // lane: columns 2 lane, 2 lane + 1 of either half, the pairs that rotate together
+        const float4 rot = reinterpret_cast<const float4*>(a.rope_table)[size_t(r) * (HD / 4) + lane];   // cos, sin of two pairs
+        const float2 g0 = make_float2(gamma[2 * lane], gamma[2 * lane + 1]), g1 = make_float2(gamma[HD / 2 + 2 * lane], gamma[HD / 2 + 2 * lane + 1]);
+        float v[4];
+        for (uint32_t s0 = 0; s0 < a.planes; s0 += 4) {
+            float2 x[4], y[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (s0 + s < a.planes) {
+                    x[s] = *reinterpret_cast<const float2*>(src + (s0 + s) * stride + 2 * lane);
+                    y[s] = *reinterpret_cast<const float2*>(src + (s0 + s) * stride + HD / 2 + 2 * lane);
+                }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (s0 + s < a.planes) {
+                    if (s0 + s == 0) { v[0] = x[s].x; v[1] = x[s].y; v[2] = y[s].x; v[3] = y[s].y; }
+                    else { v[0] += x[s].x; v[1] += x[s].y; v[2] += y[s].x; v[3] += y[s].y; }
+                }
+        }
+        float ss = fmaf(v[0], v[0], fmaf(v[1], v[1], fmaf(v[2], v[2], v[3] * v[3])));
+        const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(HD) + a.eps);
+        v[0] = v[0] * inv * g0.x; v[1] = v[1] * inv * g0.y; v[2] = v[2] * inv * g1.x; v[3] = v[3] * inv * g1.y;
+        const float o0 = __fsub_rn(__fmul_rn(v[0], rot.x), __fmul_rn(v[2], rot.y)), o1 = __fsub_rn(__fmul_rn(v[1], rot.z), __fmul_rn(v[3], rot.w));
+        const float o2 = __fadd_rn(__fmul_rn(v[0], rot.y), __fmul_rn(v[2], rot.x)), o3 = __fadd_rn(__fmul_rn(v[1], rot.w), __fmul_rn(v[3], rot.z));
+        if (is_q) {
+            *reinterpret_cast<float2*>(a.q_out + off + 2 * lane) = make_float2(o0, o1);
+            *reinterpret_cast<float2*>(a.q_out + off + HD / 2 + 2 * lane) = make_float2(o2, o3);
+        } else {
+            auto narrow = [&](float x, float y) {   // round to nearest even, after rotation
+                const _Float16 h0 = static_cast<_Float16>(x), h1 = static_cast<_Float16>(y);
+                bad |= !(isfinite(static_cast<float>(h0)) && isfinite(static_cast<float>(h1)));
+                return uint32_t(__builtin_bit_cast(uint16_t, h0)) | (uint32_t(__builtin_bit_cast(uint16_t, h1)) << 16);
+            };
+            *reinterpret_cast<uint32_t*>(a.k_out + off + 2 * lane) = narrow(o0, o1);
+            *reinterpret_cast<uint32_t*>(a.k_out + off + HD / 2 + 2 * lane) = narrow(o2, o3);
+        }
+    } else {
+        const uint32_t w = blockIdx.x - a.head_groups, kvh = w % a.kv_heads, v0 = (w / a.kv_heads) * 32;
+        const size_t width = size_t(a.kv_heads) * HD, stride = size_t(a.rows) * width;
+        for (uint32_t c = threadIdx.x; c < 32 * (HD / 8); c += 256) {
+            const uint32_t token = c / (HD / 8), d8 = c % (HD / 8), kp = a.base32 + v0 + token;
+            uint4 val = make_uint4(0, 0, 0, 0);   // outside the visible range
+            if (kp >= a.position && kp < a.position + a.rows) {
+                const size_t off = size_t(kp - a.position) * width + kvh * HD + 8 * d8;
+                float f[8];
+                sum_planes8<4>(a.v_planes + off, a.planes, stride, f);
+                uint32_t o[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const _Float16 h0 = static_cast<_Float16>(f[2 * i]), h1 = static_cast<_Float16>(f[2 * i + 1]);
+                    bad |= !(isfinite(static_cast<float>(h0)) && isfinite(static_cast<float>(h1)));
+                    o[i] = uint32_t(__builtin_bit_cast(uint16_t, h0)) | (uint32_t(__builtin_bit_cast(uint16_t, h1)) << 16);
+                }
+                val = make_uint4(o[0], o[1], o[2], o[3]);
+                *reinterpret_cast<uint4*>(a.v_out + off) = val;
+            } else if (kp >= a.first_visible && kp < a.position) {
+                const U4a4 t = *reinterpret_cast<const U4a4*>(a.ring_v + size_t(kp & a.ring_mask) * width + kvh * HD + 8 * d8);
+                val = make_uint4(t.x, t.y, t.z, t.w);
+            }
+            *reinterpret_cast<uint4*>(&tile[token][8 * d8]) = val;
+        }
+        __syncthreads();
+        const uint32_t dim = threadIdx.x;
+        uint32_t o[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) o[t] = uint32_t(tile[2 * t][dim]) | (uint32_t(tile[2 * t + 1][dim]) << 16);
+        uint4* dst = reinterpret_cast<uint4*>(a.vt + (size_t(kvh) * HD + dim) * a.T + v0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dst[i] = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
+    }
+    if (bad && a.status) atomicOr(a.status, GUFFIN_STATUS_KV_NONFINITE);
+}
+
+uint32_t row_threads(uint32_t width) { return (width / 8 + 63) / 64 * 64; }
+
+}  // namespace
+
+int prefill_norm(hipStream_t s, const float* x, const float* gamma, uint8_t* image, uint32_t rows, uint32_t width, float eps, uint32_t* status) {
+    launch(prefill_norm_kernel, dim3(rows), dim3(row_threads(width)), 0, s, x, gamma, image, rows, width, eps, status);
+    return check_launch("prefill_norm");
+}
+
+int prefill_joint(hipStream_t s, const float* x, uint32_t planes, const float* gamma_post, const float* residual, float* out_residual,
+                  const float* gamma_next, float* out_norm, uint8_t* image, uint32_t rows, uint32_t width, float eps, const RunRows& run,
+                  uint32_t* status) {
+    const uint32_t threads = row_threads(width);
+    const uint64_t copies = run.run_k ? uint64_t(rows - run.first_row) * run.row_vec : 0;
+    launch(prefill_joint_kernel, dim3(rows + static_cast<uint32_t>((copies + threads - 1) / threads)), dim3(threads), 0, s, x, planes,
+           size_t(rows) * width, gamma_post, residual, out_residual, gamma_next, out_norm, image, rows, width, eps, run, status);
+    return check_launch("prefill_joint");
+}
+
+int prefill_geglu(hipStream_t s, const float* gate, const float* up, uint32_t planes, uint8_t* image, uint32_t rows, uint32_t width) {
+    const uint64_t threads = uint64_t(rows) * (width / 8);
+    launch(prefill_geglu_kernel, dim3(static_cast<uint32_t>((threads + 255) / 256)), dim3(256), 0, s, gate, up, planes, size_t(rows) * width,
+           image, rows, width);
+    return check_launch("prefill_geglu");
+}
+
+int prefill_qkv(hipStream_t s, QkvRun a) {
+    a.head_groups = (a.rows * (a.q_heads + a.kv_heads) + 3) / 4;
+    launch(prefill_qkv_kernel, dim3(a.head_groups + (a.T / 32) * a.kv_heads), dim3(256), 0, s, a);
+    return check_launch("prefill_qkv");
+}
+
+}  // namespace guffin

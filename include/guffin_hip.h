@@ -489,7 +489,7 @@ int guffin_hip_commit_rows(void* stream, const guffin_model_desc* model, const v
  * and encode_f16_prefill_attention (metal_command_context.hpp:185, metal_kernels.mm:2593-2800).
  *
  * guffin_hip_prefill_pack turns x [M][K] fp32 into the matrix-core operand of M rows (fp16 hi/lo
- * image, per-(row, 32-group) multipliers and sums; guffin_hip_prefill_image_bytes bytes, 256-byte
+ * image, per-(row, block) multipliers and group sums; guffin_hip_prefill_image_bytes bytes, 256-byte
  * aligned); guffin_hip_prefill_gemm multiplies it with a repacked weight matrix, y [M][N] fp32,
  * exact products and fp32 sums like the packed GEMV. */
 uint64_t guffin_hip_prefill_image_bytes(uint32_t M, uint32_t K);
@@ -501,7 +501,7 @@ int guffin_hip_prefill_gemm(void* stream, int dtype, const void* tiles, const vo
  * run_k / run_v [rows][kv_heads*head_dim]; window = 0 for global layers, else the sliding
  * window (the last `window` positions including the row's own).  q, out: [rows][q_heads*256].
  * workspace: guffin_hip_prefill_attention_workspace_bytes bytes (16-byte aligned) for the
- * transposed values of the matrix-core path (q_heads / kv_heads <= 2); NULL selects the
+ * transposed values and the partial results of the matrix-core path (q_heads / kv_heads 1, 2 or 4); NULL selects the
  * vector-unit kernel, which needs none. */
 uint64_t guffin_hip_prefill_attention_workspace_bytes(uint32_t rows, uint32_t position, uint32_t window,
                                                       uint32_t kv_heads, uint32_t head_dim);

@@ -317,3 +317,45 @@ def test_prefill_rows_match_oracle_forward(hip, gfo, kind, rows, position):
             assert np.mean(g == w) >= 0.95
             d = np.abs(g.view(np.float16).astype(np.float32) - w.view(np.float16).astype(np.float32))
             assert d.max() <= 2.0 ** -9 * np.abs(w.view(np.float16).astype(np.float32)).max() + 1e-6
+
+
+@pytest.mark.parametrize("dtype,K,N", [(0, 32, 64), (0, 96, 320), (0, 608, 256), (0, 1024, 64), (1, 256, 256), (1, 1280, 576), (2, 256, 64),
+                                       (2, 1280, 320)])
+@pytest.mark.parametrize("M", [2, 15, 16, 17, 48, 49, 64, 65, 80, 97])
+def test_prefill_gemm_row_tiles(hip, gfo, dtype, K, N, M):
+    """Rows on both sides of every number of 16-row tiles a workgroup takes (one to four, one or two workgroups), with
+    one block of K, an odd number of 32-element blocks, and column tiles that do not fill a workgroup's four.  Bar: the
+    reference's bound for its matrix path on every element (rounding of K + 8 fp32 operations on exact products)."""
+    w = synth.make_weight(dtype, K, N, seed=60 + dtype)
+    x = synth.make_activation(M, K, seed=61)
+    x[M - 1] *= 1e4
+    tiles = hip.repack(dtype, dev(w), K, N)
+    y = hip.prefill_gemm(dtype, tiles, hip.prefill_pack(dev(x)), M, K, N).cpu().numpy()
+    assert_within_operator_bound(gfo, dtype, w, x, y, K, N, matrix_path=True)
+
+
+@pytest.mark.parametrize("kind,rows,position", [("target", 2, 30), ("target", 16, 0), ("target", 17, 90), ("target", 49, 0), ("target", 81, 40),
+                                                ("drafter", 5, 0), ("drafter", 33, 90), ("drafter", 100, 20)])
+def test_prefill_rows_agree_with_decode_at_row_tile_edges(hip, kind, rows, position):
+    """Short runs, whose GEMMs are cut along K and whose attention is cut along the keys (behind a ring that wraps where
+    position + rows exceeds 128 on local blocks), against the decode pass of the last token over the same rings: hidden row
+    within 2e-4 of the row RMS (fp32 sums of exact products in another order, and fp16 K/V rows that may round the other
+    way), its K/V the ring's up to such ties."""
+    import torch
+    from dataclasses import replace
+    from guffin_amd import model
+    base = model.GEMMA3_12B if kind == "target" else model.GEMMA3_270M
+    shape = replace(base, layers=6, vocab=2048, ring_global=256, ring_local=128, sliding_window=96)
+    host = model.HostModel(shape, seed=24, position=position)
+    devm = model.DeviceModel.from_host(host)
+    tokens = dev(np.random.default_rng(19).integers(0, shape.vocab, rows).astype(np.int32))
+    hidden, status = devm.prefill(tokens, position)
+    torch.cuda.synchronize()
+    assert int(status.item()) == 0
+    one, _, pk, pv, st = devm.forward(tokens[rows - 1:].contiguous(), position + rows - 1)
+    assert int(st.item()) == 0
+    want = one.cpu().numpy().astype(np.float64)[0]
+    assert np.max(np.abs(hidden[rows - 1].cpu().numpy() - want)) <= 2e-4 * np.sqrt((want ** 2).mean())
+    for l in range(shape.layers):
+        slot = (position + rows - 1) & (devm.ring_k[l].shape[0] - 1)
+        assert float((devm.ring_k[l][slot] == pk[l, 0]).float().mean()) >= 0.95 and float((devm.ring_v[l][slot] == pv[l, 0]).float().mean()) >= 0.95
