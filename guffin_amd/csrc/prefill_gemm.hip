@@ -69,6 +69,8 @@ __device__ __forceinline__ uint32_t bytes_as_halves(uint32_t w, uint32_t sel, fl
 // hazard handling around matrix instructions does not look into an asm statement.)
 __device__ __forceinline__ uint32_t scalar(uint32_t v) { asm("" : "+s"(v)); return v; }
 __device__ __forceinline__ uint32_t and_or(uint32_t w, uint32_t mask, uint32_t c) { return (w & mask) | c; }
+// a value the compiler takes as it is (it would turn two of the above into two ands and an or3)
+__device__ __forceinline__ uint32_t kept(uint32_t v) { asm("" : "+v"(v)); return v; }
 __device__ __forceinline__ uint32_t vector_bias() {
     uint32_t c = 0x64006400u;
     asm("" : "+v"(c));
@@ -172,11 +174,11 @@ __device__ __forceinline__ void q4_operands(const uint4 (&q)[4], const uint32_t 
     }
 }
 
-template <int R, bool FIRST>
+template <int R, bool FIRST, int C0 = 0, int C1 = 4>
 __device__ __forceinline__ void products(const half8_t (&a)[R], const half8_t (&b)[4], float4_t (&D)[4][R]) {
     const float4_t zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int cg = 0; cg < 4; ++cg)
+    for (int cg = C0; cg < C1; ++cg)
 #pragma unroll
         for (int r = 0; r < R; ++r) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[r], b[cg], FIRST ? zero : D[cg][r], 0, 0, 0);
 }
@@ -294,140 +296,242 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& fee
     }
 }
 
-template <int R>
-struct GroupA { half8_t hi[R], lo[R]; };
-
-template <int R>
-__device__ __forceinline__ void read_group(const uint8_t* stage, uint32_t lane16, GroupA<R>& a) {
-    read_half<R>(stage, 0, lane16, a.hi);
-    read_half<R>(stage, 1, lane16, a.lo);
-}
-
 // ---- Q6_K ------------------------------------------------------------------------------------------------
-// one 32-group of a half block for column groups 2P, 2P + 1; QD: its number in the half
-template <int R, int QD, bool FIRST>
-__device__ __forceinline__ void q6_group(const GroupA<R>& a, const uint4 (&ql)[4], const uint2 (&qh)[4], const uint2 (&sc)[4],
-                                         uint32_t sel, float4_t (&D)[4][R]) {
-    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+// Group QD (0..3) of a half block: the quants q - 32 of column groups C0 .. C1 - 1 as halves
+template <int QD, int C0 = 0, int C1 = 4>
+__device__ __forceinline__ void q6_quants(const uint4 (&ql)[4], const uint2 (&qh)[4], half8_t (&q)[4]) {
     const uint32_t bias = vector_bias(), low = scalar(0x000F000Fu), high = scalar(0x00300030u);
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        half8_t b[2], rest[2];
+    for (int cg = C0; cg < C1; ++cg) {
+        const uint32_t w[2] = {(QD & 1) ? ql[cg].z : ql[cg].x, (QD & 1) ? ql[cg].w : ql[cg].y};
+        const uint32_t h[2] = {qh[cg].x, qh[cg].y};
+        uint32_t o[4];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int cg = 2 * p + c;
-            // the int8 scale + 128 under the bias; sel picks the lane's byte of the pair (a scale covers 16 elements)
-            const half2_t s = h2(__builtin_amdgcn_perm(0x64646464u, (QD >> 1) ? sc[cg].y : sc[cg].x, sel + (QD & 1) * 0x00020002u)) - splat(1152.f);
-            const uint32_t w[2] = {(QD & 1) ? ql[cg].z : ql[cg].x, (QD & 1) ? ql[cg].w : ql[cg].y};
-            const uint32_t h[2] = {qh[cg].x, qh[cg].y};
-            uint32_t bw[4], rw[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                constexpr int ls = QD >= 2 ? 4 : 0;
-                const uint32_t wk = w[k >> 1] >> (ls + 8 * (k & 1));
-                constexpr int up = 4 - 2 * QD;   // the two high bits go to bits 4-5
-                const int sh = 8 * (k & 1) - up;
-                const uint32_t hk = sh >= 0 ? h[k >> 1] >> (sh >= 0 ? sh : 0) : h[k >> 1] << (sh < 0 ? -sh : 0);
-                const half2_t q = h2(and_or(wk, low, and_or(hk, high, bias))) - splat(1056.f);
-                const half2_t prod = s * q;                              // nearest
-                bw[k] = u2(prod);
-                rw[k] = u2(__builtin_elementwise_fma(s, q, -prod));      // what that rounding left
-            }
-            b[c] = as_half8(bw[0], bw[1], bw[2], bw[3]);
-            rest[c] = as_half8(rw[0], rw[1], rw[2], rw[3]);
+        for (int k = 0; k < 4; ++k) {
+            constexpr int ls = QD >= 2 ? 4 : 0, up = 4 - 2 * QD;   // the two high bits go to bits 4-5
+            const int sh = 8 * (k & 1) - up;
+            const uint32_t wk = w[k >> 1] >> (ls + 8 * (k & 1));
+            const uint32_t hk = sh >= 0 ? h[k >> 1] >> (sh >= 0 ? sh : 0) : h[k >> 1] << (sh < 0 ? -sh : 0);
+            o[k] = u2(h2(and_or(wk, low, kept(and_or(hk, high, bias)))) - splat(1056.f));
         }
+        q[cg] = as_half8(o[0], o[1], o[2], o[3]);
+    }
+}
+// times the lane's scale (a scale covers 16 elements; sel picks the lane's byte of the group's pair, int8 + 128 under the
+// bias): q becomes the nearest half of the product, rest what that rounding left
+template <int QD, int C0 = 0, int C1 = 4>
+__device__ __forceinline__ void q6_scaled(const uint2 (&sc)[4], uint32_t sel, half8_t (&q)[4], half8_t (&rest)[4]) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+    for (int cg = C0; cg < C1; ++cg) {
+        const half2_t s = h2(__builtin_amdgcn_perm(0x64646464u, (QD >> 1) ? sc[cg].y : sc[cg].x, sel + (QD & 1) * 0x00020002u)) - splat(1152.f);
+        const uint4 v = __builtin_bit_cast(uint4, q[cg]);
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+        uint32_t p[4], r[4];
 #pragma unroll
-            for (int r = 0; r < R; ++r)
-                D[2 * p + c][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi[r], b[c], FIRST ? zero : D[2 * p + c][r], 0, 0, 0);
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int r = 0; r < R; ++r) D[2 * p + c][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.lo[r], b[c], D[2 * p + c][r], 0, 0, 0);
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int r = 0; r < R; ++r) D[2 * p + c][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi[r], rest[c], D[2 * p + c][r], 0, 0, 0);
+        for (int k = 0; k < 4; ++k) {
+            const half2_t prod = s * h2(x[k]);
+            p[k] = u2(prod);
+            r[k] = u2(__builtin_elementwise_fma(s, h2(x[k]), -prod));
+        }
+        q[cg] = as_half8(p[0], p[1], p[2], p[3]);
+        rest[cg] = as_half8(r[0], r[1], r[2], r[3]);
     }
 }
 
+// Three regions per group: hi against the rest, hi and lo against the products; while they run, the next group's operands
+// are formed (its quants beside the first region, its products and rests beside the second, in place of the rests that are
+// done) and the halves of A that the next region wants are read.  Otherwise as the Q4_K walk.
 template <int R>
-__device__ __forceinline__ void q6_walk(const GemmArgs& A, const ImageLayout& L, const Feed<R>& feed, uint8_t* stage,
-                                        const uint8_t* tile_base, uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
+__device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& feed, uint8_t* stage, const uint8_t* tile_base,
+                                        uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q6_K);
+    constexpr int V0 = (96 + 4 * R - 1) / (4 * R), V1 = (48 + 4 * R - 1) / (4 * R);
+    using S = Stage<R>;
     const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
     const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
     const uint32_t sel = lane >= 32 ? 0x04010401u : 0x04000400u;
+    uint8_t* const heads = stage + S::kHead + wv * 1280;
     uint4 ql[2][4];
-    uint2 qh[2][4], sc[2][4];
-    uint32_t dw[4];
-    auto ask_half = [&](uint32_t b, int h, int to) {
+    uint2 qh[2][4], sc[4];
+    half8_t hi[R], lo[R], b[4], bn[4], rest[4];
+    float4_t D[4][R];
+    auto ask_half = [&](uint32_t blk, int h) {
 #pragma unroll
         for (int cg = 0; cg < 4; ++cg) {
-            ql[to][cg] = ld16(tile, lane16, b * TB + 2048 * cg + 1024 * h);
-            qh[to][cg] = ld8(tile, lane16 + 8 * h, b * TB + 8192 + 1024 * cg);
-            sc[to][cg] = ld8(tile, j * 16 + 8 * h, b * TB + 12288 + 256 * cg);
+            ql[h][cg] = ld16(tile, lane16, blk * TB + 2048 * cg + 1024 * h);
+            qh[h][cg] = ld8(tile, lane16 + 8 * h, blk * TB + 8192 + 1024 * cg);
         }
     };
-    auto flip = [&](int to) {   // int8 -> +128
-#pragma unroll
-        for (int cg = 0; cg < 4; ++cg) { sc[to][cg].x ^= 0x80808080u; sc[to][cg].y ^= 0x80808080u; }
+    auto ask_head = [&](uint32_t blk) {   // the 16 scales of every column, then the columns' d (read beyond the tile: zeros)
+        to_lds16(tile, heads + (blk & 1) * 5120, lane16, blk * TB + 12288);
+        to_lds4(tile, heads + (blk & 1) * 5120 + 1024, lane < 32 ? lane * 4 : 0, blk * TB + 13312);
     };
-    ask_half(b0, 0, 0);
+    auto scales = [&](uint32_t blk, int half) {
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) {
+            const uint2 v = *reinterpret_cast<const uint2*>(heads + (blk & 1) * 5120 + 256 * cg + j * 16 + 8 * half);
+            sc[cg] = make_uint2(v.x ^ 0x80808080u, v.y ^ 0x80808080u);   // int8 -> + 128
+        }
+    };
+    ask_half(b0, 0);
+    ask_head(b0);
+    feed.ask(4 * b0, 0);
+    asm volatile("" ::: "memory");   // in this order
+    ask_half(b0, 1);
+    feed.ask(4 * b0 + 1, 1);
+    asm volatile("" ::: "memory");
+    feed.ask(4 * b0 + 2, 2);
+    arrive<2 * R>();
+    scales(b0, 0);
+    read_half<R>(stage, 0, lane16, hi);
+    q6_quants<0>(ql[0], qh[0], b);
+    q6_scaled<0>(sc, sel, b, rest);
+    uint32_t rd = 0;
+    for (uint32_t blk = b0; blk < b1; ++blk) {
+        const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
+        auto group = [&]<int G>() {
+            constexpr int H = ((G + 1) & 7) >> 2, QD = (G + 1) & 3;   // the next group's half block and place
+            const uint8_t* now = stage + rd * S::kChunk + (G & 1) * (2048 * R);
+            __builtin_amdgcn_sched_barrier(0);
+            read_half<R>(now, 1, lane16, lo);
+            q6_quants<QD>(ql[H], qh[H], bn);
+            products<R, G == 0>(hi, rest, D);
+            weave<4 * R, V0, R>();
+            if constexpr (G == 3) scales(blk, 1);
+            if constexpr (G == 7) scales(next, 0);
+            q6_scaled<QD>(sc, sel, bn, rest);
+            products<R, false>(hi, b, D);
+            weave<4 * R, V1, 0>();
+            if constexpr (G & 1) {
+                arrive<R>();
+                if constexpr (G == 1) {
+                    if (wv == 2) to_lds4(feed.img, stage + S::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (blk * L.mpad + rt0 * 16) * 4);
+                    ask_head(next);
+                }
+                if constexpr (G == 3) ask_half(next, 0);
+                if constexpr (G == 7) ask_half(next, 1);
+                feed.ask(4 * blk + (G >> 1) + 3, rd);
+                rd = rd == 2 ? 0 : rd + 1;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            read_half<R>(stage + rd * S::kChunk + ((G + 1) & 1) * (2048 * R), 0, lane16, hi);
+            products<R, false>(lo, b, D);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg) b[cg] = bn[cg];
+        };
+        group.template operator()<0>();
+        group.template operator()<1>();
+        group.template operator()<2>();
+        group.template operator()<3>();
+        group.template operator()<4>();
+        group.template operator()<5>();
+        group.template operator()<6>();
+        group.template operator()<7>();
+        float d[4];
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg)
+            d[cg] = h2f(*reinterpret_cast<const uint16_t*>(heads + (blk & 1) * 5120 + 1024 + 32 * cg + 2 * j));
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float4_t mult = *reinterpret_cast<const float4_t*>(stage + S::kMult + 64 * r + 16 * lg);
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(d[cg] * mult[i], D[cg][r][i], acc[cg][r][i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// The same for four row tiles, where the accumulators leave no registers for operands formed ahead: column groups by pairs,
+// the compiler's order, and the second wave of the SIMD to fill the gaps (the woven form spills: 2048 x 15360 x 3840 takes
+// 772 us instead of 614).  The workgroup meets at a chunk's start; the chunk after the next is asked for there.
+template <int R>
+__device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, const Feed<R>& feed, uint8_t* stage, const uint8_t* tile_base,
+                                             uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
+    constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q6_K);
+    using S = Stage<R>;
+    const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
+    const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
+    const uint32_t sel = lane >= 32 ? 0x04010401u : 0x04000400u;
+    uint8_t* const heads = stage + S::kHead + wv * 1280;
+    uint4 ql[2][4];
+    uint2 qh[2][4], sc[4];
+    float4_t D[4][R];
+    auto ask_half = [&](uint32_t blk, int h) {
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) {
+            ql[h][cg] = ld16(tile, lane16, blk * TB + 2048 * cg + 1024 * h);
+            qh[h][cg] = ld8(tile, lane16 + 8 * h, blk * TB + 8192 + 1024 * cg);
+        }
+    };
+    auto ask_head = [&](uint32_t blk) {
+        to_lds16(tile, heads + (blk & 1) * 5120, lane16, blk * TB + 12288);
+        to_lds4(tile, heads + (blk & 1) * 5120 + 1024, lane < 32 ? lane * 4 : 0, blk * TB + 13312);
+    };
+    auto scales = [&](uint32_t blk, int half) {
+#pragma unroll
+        for (int cg = 0; cg < 4; ++cg) {
+            const uint2 v = *reinterpret_cast<const uint2*>(heads + (blk & 1) * 5120 + 256 * cg + j * 16 + 8 * half);
+            sc[cg] = make_uint2(v.x ^ 0x80808080u, v.y ^ 0x80808080u);
+        }
+    };
+    ask_half(b0, 0);
+    ask_head(b0);
     feed.ask(4 * b0, 0);
     asm volatile("" ::: "memory");   // in this order
     feed.ask(4 * b0 + 1, 1);
     uint32_t rd = 0, wr = 2;
-    auto next = [&] { rd = rd == 2 ? 0 : rd + 1; wr = wr == 2 ? 0 : wr + 1; };
-    float4_t D[4][R];
-    GroupA<R> a;
-    for (uint32_t b = b0; b < b1; ++b) {
-        const uint32_t bn = b + 1 < b1 ? b + 1 : b;
-        arrive<R>();
-        ask_half(b, 1, 1);
-        if (wv == 0) to_lds4(feed.img, stage + Stage<R>::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (b * L.mpad + rt0 * 16) * 4);
-        feed.ask(4 * b + 2, wr);
-        flip(0);
-        read_group<R>(stage + rd * Stage<R>::kChunk, lane16, a);
-        q6_group<R, 0, true>(a, ql[0], qh[0], sc[0], sel, D);
-        read_group<R>(stage + rd * Stage<R>::kChunk + 2048 * R, lane16, a);
-        q6_group<R, 1, false>(a, ql[0], qh[0], sc[0], sel, D);
-        next();
-        arrive<R>();
-        feed.ask(4 * b + 3, wr);
-        read_group<R>(stage + rd * Stage<R>::kChunk, lane16, a);
-        q6_group<R, 2, false>(a, ql[0], qh[0], sc[0], sel, D);
-        read_group<R>(stage + rd * Stage<R>::kChunk + 2048 * R, lane16, a);
-        q6_group<R, 3, false>(a, ql[0], qh[0], sc[0], sel, D);
-        next();
-        arrive<R>();
+    for (uint32_t blk = b0; blk < b1; ++blk) {
+        const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;
+        auto group = [&]<int G>() {
+            constexpr int H = G >> 2, QD = G & 3;
+            if constexpr ((G & 1) == 0) {
+                arrive<R>();
+                if constexpr (G == 0) {
+                    ask_half(blk, 1);
+                    if (wv == 2) to_lds4(feed.img, stage + S::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (blk * L.mpad + rt0 * 16) * 4);
+                    scales(blk, 0);
+                }
+                if constexpr (G == 2) ask_head(next);
+                if constexpr (G == 4) { ask_half(next, 0); scales(blk, 1); }
+                feed.ask(4 * blk + (G >> 1) + 2, wr);
+            }
+            const uint8_t* from = stage + rd * S::kChunk + (G & 1) * (2048 * R);
+            half8_t hi[R], lo[R], b[4], rest[4];
+            read_half<R>(from, 0, lane16, hi);
+            read_half<R>(from, 1, lane16, lo);
+            auto pair = [&]<int C>() {
+                q6_quants<QD, C, C + 2>(ql[H], qh[H], b);
+                q6_scaled<QD, C, C + 2>(sc, sel, b, rest);
+                products<R, G == 0, C, C + 2>(hi, b, D);
+                products<R, false, C, C + 2>(lo, b, D);
+                products<R, false, C, C + 2>(hi, rest, D);
+            };
+            pair.template operator()<0>();
+            pair.template operator()<2>();
+            if constexpr (G & 1) { rd = rd == 2 ? 0 : rd + 1; wr = wr == 2 ? 0 : wr + 1; }
+        };
+        group.template operator()<0>();
+        group.template operator()<1>();
+        group.template operator()<2>();
+        group.template operator()<3>();
+        group.template operator()<4>();
+        group.template operator()<5>();
+        group.template operator()<6>();
+        group.template operator()<7>();
+        float d[4];
 #pragma unroll
-        for (int cg = 0; cg < 4; ++cg) dw[cg] = ld4(tile, (j >> 1) * 4, b * TB + 13312 + 32 * cg);
-        ask_half(bn, 0, 0);
-        feed.ask(4 * b + 4, wr);
-        flip(1);
-        read_group<R>(stage + rd * Stage<R>::kChunk, lane16, a);
-        q6_group<R, 0, false>(a, ql[1], qh[1], sc[1], sel, D);
-        read_group<R>(stage + rd * Stage<R>::kChunk + 2048 * R, lane16, a);
-        q6_group<R, 1, false>(a, ql[1], qh[1], sc[1], sel, D);
-        next();
-        arrive<R>();
-        feed.ask(4 * b + 5, wr);
-        read_group<R>(stage + rd * Stage<R>::kChunk, lane16, a);
-        q6_group<R, 2, false>(a, ql[1], qh[1], sc[1], sel, D);
-        read_group<R>(stage + rd * Stage<R>::kChunk + 2048 * R, lane16, a);
-        q6_group<R, 3, false>(a, ql[1], qh[1], sc[1], sel, D);
-        next();
+        for (int cg = 0; cg < 4; ++cg)
+            d[cg] = h2f(*reinterpret_cast<const uint16_t*>(heads + (blk & 1) * 5120 + 1024 + 32 * cg + 2 * j));
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const float4_t mult = *reinterpret_cast<const float4_t*>(stage + Stage<R>::kMult + 64 * r + 16 * lg);
+            const float4_t mult = *reinterpret_cast<const float4_t*>(stage + S::kMult + 64 * r + 16 * lg);
 #pragma unroll
-            for (int cg = 0; cg < 4; ++cg) {
-                const float d = h2f((dw[cg] >> (16 * (j & 1u))) & 0xFFFFu);
+            for (int cg = 0; cg < 4; ++cg)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(d * mult[i], D[cg][r][i], acc[cg][r][i]);
-            }
+                for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(d[cg] * mult[i], D[cg][r][i], acc[cg][r][i]);
         }
     }
 }
@@ -463,8 +567,10 @@ prefill_gemm_kernel(GemmArgs A) {
             for (int i = 0; i < 4; ++i) acc[cg][r][i] = 0.f;
     if (KINDS == 1 || (KINDS == 3 && seg.dtype == GUFFIN_Q4_K))
         q4_walk<R>(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q4_K)), rt0, b0, b1, acc);
+    else if constexpr (R == 4)
+        q6_walk_wide<R>(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q6_K)), rt0, b0, b1, acc);
     else
-        q6_walk<R>(A, L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q6_K)), rt0, b0, b1, acc);
+        q6_walk<R>(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q6_K)), rt0, b0, b1, acc);
     // the chunks asked for past the end are still on their way into this workgroup's LDS
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!valid) return;
@@ -541,8 +647,9 @@ prefill_gemm_q8_kernel(GemmArgs A) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             if (2 * c + h >= nblk) break;   // an odd number of blocks: the last chunk has one
-            GroupA<R> a;
-            read_group<R>(from + h * (2048 * R), lane16, a);
+            half8_t hi[R], lo[R];
+            read_half<R>(from + h * (2048 * R), 0, lane16, hi);
+            read_half<R>(from + h * (2048 * R), 1, lane16, lo);
             half8_t b[4];
             float d[4];
 #pragma unroll
@@ -557,11 +664,11 @@ prefill_gemm_q8_kernel(GemmArgs A) {
 #pragma unroll
             for (int cg = 0; cg < 4; ++cg)
 #pragma unroll
-                for (int r = 0; r < R; ++r) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi[r], b[cg], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                for (int r = 0; r < R; ++r) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[r], b[cg], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
             for (int cg = 0; cg < 4; ++cg)
 #pragma unroll
-                for (int r = 0; r < R; ++r) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.lo[r], b[cg], D[cg][r], 0, 0, 0);
+                for (int r = 0; r < R; ++r) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[r], b[cg], D[cg][r], 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const float4_t mult = *reinterpret_cast<const float4_t*>(from + Stage<R>::kChunk + 256 * h + 64 * r + 16 * lg);
@@ -613,30 +720,36 @@ int gemm_launch(hipStream_t s, GemmArgs& a, uint32_t slices, uint32_t R) {
     return check_launch("prefill_gemm");
 }
 
-// Time of a launch by a model of the chip, in microseconds: a workgroup takes `start` to its first product and `block` per 256
-// elements of K (measured, two workgroups on a compute unit; alone it takes three quarters of that), 512 run at once, and a
-// plane costs a write and a read at the memory's rate.
-constexpr float kStart = 3.5f, kBlockQ4[4] = {3.1f, 4.2f, 5.4f, 7.0f}, kBlockQ6[4] = {3.8f, 5.4f, 7.2f, 9.0f}, kPlaneBytesPerUs = 4.0e6f;
+// Time of a launch by a model of the chip, in microseconds: `start` from the launch to the first product and from the last one
+// to the end, then every compute unit (256) works off its share of the workgroups at `unit` per slice unit -- 256 elements
+// of K, 64 for Q8_0 --, and a plane costs a write here and a read in the next operator.  Constants fitted to sweeps
+// over 4 to 1000 rows of both models' shapes; the choice was within 4 % of the best pair of each.
+constexpr float kStart[4] = {5.0f, 6.2f, 7.5f, 8.5f};
+constexpr float kUnit[3][4] = {{0.6f, 0.82f, 1.0f, 1.35f}, {2.3f, 2.7f, 3.2f, 3.8f}, {2.8f, 3.3f, 4.0f, 4.8f}};   // Q8_0, Q4_K, Q6_K
+constexpr float kPlaneBytesPerUs = 5.0e6f;
 
 PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K, uint32_t most) {
     uint32_t groups = 0, width = 0;
-    bool q6 = false, q8 = false;
+    float unit[4] = {};   // of a workgroup, the mean over the launch
+    bool q8 = false;
     for (uint32_t i = 0; i < count; ++i) {
-        groups += (m[i].N / kCols + 3) / 4;
+        const uint32_t n = (m[i].N / kCols + 3) / 4;
+        groups += n;
         width += m[i].N;
-        q6 |= m[i].dtype == GUFFIN_Q6_K;
         q8 |= m[i].dtype == GUFFIN_Q8_0;
+        for (int r = 0; r < 4; ++r) unit[r] += float(n) * kUnit[m[i].dtype][r];
     }
     const uint32_t units = q8 ? (K + 63) / 64 : K / 256;   // what a slice is made of
     PrefillSplit best {1, 1};
     float least = 0.f;
     for (uint32_t R = 1; R <= 4; ++R) {
         const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
-        const float block = (q6 ? kBlockQ6 : kBlockQ4)[R - 1] * (q8 ? 0.3f : 1.0f);
-        for (uint32_t S = 1; S <= std::min(units, most); ++S) {
-            const uint32_t n = chunks * groups * S, rounds = (n + 511) / 512;
-            const float each = kStart + float((units + S - 1) / S) * block * (n <= 256 ? 0.75f : 1.0f);
-            const float cost = each * (rounds == 1 ? 1.0f : std::max(1.0f, 0.5f * (float(rounds) + float(n) / 512.0f)))
+        for (uint32_t S = 1; S <= std::max(1u, std::min(units, most)); ++S) {
+            const uint32_t n = chunks * groups * S;
+            // one workgroup per compute unit leaves gaps that a second one fills; the last, partly filled turn overlaps the
+            // one before it: half of it counts
+            const float turns = std::max(1.22f, 0.5f * (float((n + 255) / 256) + float(n) / 256.0f));
+            const float cost = kStart[R - 1] + turns * float((units + S - 1) / S) * unit[R - 1] / float(groups)
                 + float(S) * 8.0f * float(M) * float(width) / kPlaneBytesPerUs;
             if ((R == 1 && S == 1) || cost < least) { best = {R, S}; least = cost; }
         }
