@@ -173,7 +173,9 @@ __device__ __forceinline__ void split_half8(const float (&x)[8], uint4& hi, uint
 // key range is cut into parts, the parts' states
 struct AttentionOut { float* rows; uint8_t* image; float* part_o; float* part_ml; };
 constexpr float kProbScale = 1024.0f;   // probabilities enter the matrix instruction times 2^10
-constexpr uint32_t kTileQueries = 32;   // (row, head) pairs of a workgroup: two A tiles
+constexpr float kLog2e = 1.44269504088896340736f;
+// scores are kept times log2(e), so that the exponential is one instruction (v_exp_f32, an ulp; it flushes what is below 2^-126)
+__device__ __forceinline__ float exp2_of(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // one (row, head): 8 consecutive output dimensions in 32 consecutive lanes
 __device__ __forceinline__ void emit_attention(const AttentionOut& to, const float (&v)[8], uint32_t row, uint32_t rows, uint32_t head,
@@ -188,121 +190,152 @@ __device__ __forceinline__ void emit_attention(const AttentionOut& to, const flo
     }
 }
 
-// grid (ceil(rows * group / 32), kv_heads, parts), 4 waves.  A workgroup serves 32 (row, head) pairs of one KV head -- the
-// group's heads of 32 / group consecutive rows, as two A tiles of 16 pairs -- and one part of the key range.  Each wave walks
-// its own 32-token tiles (tile index = wave mod 4) with its own online softmax state and its own output accumulators; the
-// four states are merged at the end.  A run of few rows is cut into parts so that the chip is full; their states are
-// merged by prefill_attention_merge_kernel.
+// grid (ceil(rows * group / (16 NT)), kv_heads, parts), 4 waves.  A workgroup serves 16 NT (row, head) pairs of one KV head
+// -- the group's heads of 16 NT / group consecutive rows, as NT A tiles of 16 pairs -- and one part of the key range.  Each
+// wave walks its own 32-token tiles (tile index = wave mod 4) with its own online softmax state and its own output
+// accumulators; the four states are merged at the end.  A run of few rows is cut into parts so that the chip is full; their
+// states are merged by prefill_attention_merge_kernel.
 //   scores   S = Q K^T: queries (scaled, fp16 hi + lo, staged once in LDS in operand order) as A,
 //            keys straight from their fp16 rows as B (a lane reads 8 dims of one key per MFMA)
+//   softmax  a tile that every row sees whole needs no masks, and the accumulators are rescaled only where a maximum moved
 //   values   O += P V: probabilities times 2^10 as fp16 hi + lo through a wave-private LDS
 //            transpose as A, V^T rows as B
+template <int NT>
 __global__ void __launch_bounds__(256, 2)
 prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __restrict__ ring_k,
                               const uint16_t* __restrict__ run_k, const uint16_t* __restrict__ vt,
                               AttentionOut to, uint32_t rows, uint32_t position, uint32_t window,
                               uint32_t ring_mask, uint32_t q_heads, uint32_t kv_heads, float scale,
                               uint32_t base32, uint32_t T, uint32_t group_shift) {
-    constexpr int HD = 256, NT = 2;
+    constexpr int HD = 256;
+    constexpr uint32_t kPairs = 16 * NT;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     // [NT][8 k-steps][hi, lo][64 lanes] 16-byte query operands, later the merge buffer
     uint8_t* qa = lds;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 15, lg = lane >> 4;
-    float* pt = reinterpret_cast<float*>(lds + NT * 16384) + wave * (NT * 16 * 32);  // [NT][16 pairs][32 tokens]
-    float* ml = reinterpret_cast<float*>(lds + NT * 16384 + 4 * NT * 16 * 32 * 4);   // [32 pairs][2] for the merge
-    const uint32_t kvh = blockIdx.y, r0 = blockIdx.x * (kTileQueries >> group_shift), group = 1u << group_shift;
+    float* pt = reinterpret_cast<float*>(lds + NT * 16384) + wave * (kPairs * 32);   // [NT][16 pairs][32 tokens]
+    float* ml = reinterpret_cast<float*>(lds + NT * 16384 + 4 * kPairs * 32 * 4);    // [pairs][2] for the merge
+    const uint32_t kvh = blockIdx.y, r0 = blockIdx.x * (kPairs >> group_shift), group = 1u << group_shift;
     const size_t row_stride = size_t(kv_heads) * HD;
-    const uint32_t last_row = min(r0 + (kTileQueries >> group_shift), rows) - 1;
+    const uint32_t last_row = min(r0 + (kPairs >> group_shift), rows) - 1;
     const uint32_t hi_pos = position + last_row;
     const uint32_t lo_first = (window && position + r0 + 1 > window) ? position + r0 + 1 - window : 0;
+    const uint32_t last_first = (window && hi_pos + 1 > window) ? hi_pos + 1 - window : 0;   // of the last row
     const uint32_t tile_lo = (lo_first - base32) / 32, tiles = (hi_pos - base32) / 32 + 1 - tile_lo;
     const uint32_t begin = tile_lo + blockIdx.z * tiles / gridDim.z, end = tile_lo + (blockIdx.z + 1) * tiles / gridDim.z;
 
-    for (uint32_t idx = threadIdx.x; idx < kTileQueries * 32; idx += 256) {
+    auto ask_keys = [&](uint32_t ti, uint4 (&kb)[2][8]) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const uint32_t kp = min(base32 + 32 * ti + 16 * c + j, hi_pos);
+            const uint16_t* krow = (kp >= position ? run_k + size_t(kp - position) * row_stride
+                                                   : ring_k + size_t(kp & ring_mask) * row_stride) + kvh * HD + 8 * lg;
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks) kb[c][ks] = *reinterpret_cast<const uint4*>(krow + 32 * ks);
+        }
+    };
+    uint4 kb[2][8];
+    // one A tile leaves registers for the next keys beside the values: the first ones travel while the queries are staged
+    if constexpr (NT == 1) ask_keys(min(begin + wave, tile_lo + tiles - 1), kb);
+    for (uint32_t idx = threadIdx.x; idx < kPairs * 32; idx += 256) {
         const uint32_t m = idx / 32, c8 = idx % 32;
         const uint32_t row = min(r0 + (m >> group_shift), rows - 1), head = kvh * group + (m & (group - 1));
         const float* src = q + (size_t(row) * q_heads + head) * HD + 8 * c8;
         const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
-        const float x[8] = {a.x * scale, a.y * scale, a.z * scale, a.w * scale, b.x * scale, b.y * scale, b.z * scale, b.w * scale};
+        const float f = scale * kLog2e;
+        const float x[8] = {a.x * f, a.y * f, a.z * f, a.w * f, b.x * f, b.y * f, b.z * f, b.w * f};
         uint4 hi, lo;
         split_half8(x, hi, lo);
         uint8_t* dst = qa + (((m >> 4) * 8 + c8 / 4) * 2) * 1024 + ((m & 15) + 16 * (c8 % 4)) * 16;
         *reinterpret_cast<uint4*>(dst) = hi;
         *reinterpret_cast<uint4*>(dst + 1024) = lo;
     }
-    __syncthreads();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the keys stay on their way
 
     float m[NT][4], l[NT][4];
     float4_t O[NT][16];
-    uint32_t pos_r[NT][4], first_r[NT][4];
 #pragma unroll
     for (int g = 0; g < NT; ++g) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            m[g][r] = -INFINITY; l[g][r] = 0.f;
-            const uint32_t row = r0 + ((16 * g + 4 * lg + r) >> group_shift);
-            pos_r[g][r] = row < rows ? position + row : 0u;  // a padding row sees nothing: first > pos
-            first_r[g][r] = row < rows ? ((window && position + row + 1 > window) ? position + row + 1 - window : 0u) : 1u;
-        }
+        for (int r = 0; r < 4; ++r) { m[g][r] = -INFINITY; l[g][r] = 0.f; }
 #pragma unroll
         for (int dt = 0; dt < 16; ++dt) O[g][dt] = float4_t{0.f, 0.f, 0.f, 0.f};
     }
     for (uint32_t ti = begin + wave; ti < end; ti += 4) {
         const uint32_t t0 = base32 + 32 * ti;
+        if constexpr (NT > 1) ask_keys(ti, kb);
         float4_t S[NT][2];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            __builtin_amdgcn_sched_barrier(0);
-            const uint32_t kp = min(t0 + 16 * c + j, hi_pos);
-            const uint16_t* krow = (kp >= position ? run_k + size_t(kp - position) * row_stride
-                                                   : ring_k + size_t(kp & ring_mask) * row_stride) + kvh * HD + 8 * lg;
-            uint4 kb[8];
+        for (int ks = 0; ks < 8; ++ks)
 #pragma unroll
-            for (int ks = 0; ks < 8; ++ks) kb[ks] = *reinterpret_cast<const uint4*>(krow + 32 * ks);
+            for (int half = 0; half < 2; ++half)
 #pragma unroll
-            for (int g = 0; g < NT; ++g) {
-                float4_t acc = {0.f, 0.f, 0.f, 0.f};
+                for (int g = 0; g < NT; ++g) {
+                    const half8_t a = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(qa + ((g * 8 + ks) * 2 + half) * 1024 + lane * 16));
 #pragma unroll
-                for (int ks = 0; ks < 8; ++ks) {
-                    const uint8_t* ap = qa + ((g * 8 + ks) * 2) * 1024 + lane * 16;
-                    const half8_t kv = __builtin_bit_cast(half8_t, kb[ks]);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(ap)), kv, acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(ap + 1024)), kv, acc, 0, 0, 0);
+                    for (int c = 0; c < 2; ++c)
+                        S[g][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8_t, kb[c][ks]),
+                                                                         ks + half == 0 ? float4_t{0.f, 0.f, 0.f, 0.f} : S[g][c], 0, 0, 0);
                 }
-                S[g][c] = acc;
-            }
-        }
-        // online softmax of the lane group's four pairs of a tile; a pair's 32 scores sit in 16 lanes x 2
+        if constexpr (NT > 1) __builtin_amdgcn_sched_barrier(0);   // the keys' registers become the values'
+        const uint16_t* vcol = vt + (size_t(kvh) * HD + j) * T + (t0 - base32) + 8 * lg;
+        uint4 vb[8];
+        auto ask_values = [&](int first) {
 #pragma unroll
-        for (int g = 0; g < NT; ++g) {
+            for (int i = 0; i < 8; ++i) vb[i] = *reinterpret_cast<const uint4*>(vcol + size_t(16 * (first + i)) * T);
+        };
+        ask_values(0);
+        // online softmax of the lane group's four pairs of a tile; a pair's 32 scores sit in 16 lanes x 2
+        if (!(t0 >= last_first && t0 + 31 <= position + r0)) {
+#pragma unroll
+            for (int g = 0; g < NT; ++g)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t row = r0 + ((16 * g + 4 * lg + r) >> group_shift), pos = position + row;
+                    const uint32_t first = (window && pos + 1 > window) ? pos + 1 - window : 0u;
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const uint32_t kp = t0 + 16 * c + j;
+                        if (!(row < rows && kp <= pos && kp >= first)) S[g][c][r] = -INFINITY;
+                    }
+                }
+        }
+        float top[NT][4];
+        bool moved = false;
+#pragma unroll
+        for (int g = 0; g < NT; ++g)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                float sv[2];
+                top[g][r] = fmaxf(m[g][r], row16_max(fmaxf(S[g][0][r], S[g][1][r])));
+                moved |= top[g][r] > m[g][r];
+            }
+        if (__ballot(moved)) {
 #pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    const uint32_t kp = t0 + 16 * c + j;
-                    const bool visible = kp <= pos_r[g][r] && kp >= first_r[g][r] && kp <= hi_pos;
-                    sv[c] = visible ? S[g][c][r] : -INFINITY;
+            for (int g = 0; g < NT; ++g)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float resc = top[g][r] == -INFINITY ? 1.f : exp2_of(m[g][r] - top[g][r]);
+                    l[g][r] *= resc;
+                    m[g][r] = top[g][r];
+#pragma unroll
+                    for (int dt = 0; dt < 16; ++dt) O[g][dt][r] *= resc;
                 }
-                const float tmax = row16_max(fmaxf(sv[0], sv[1]));
-                const float new_m = fmaxf(m[g][r], tmax);
-                const float resc = new_m == -INFINITY ? 1.f : expf(m[g][r] - new_m);
-                const float p0 = sv[0] == -INFINITY ? 0.f : expf(sv[0] - new_m);
-                const float p1 = sv[1] == -INFINITY ? 0.f : expf(sv[1] - new_m);
-                const float add = row16_sum(p0 + p1);
-                l[g][r] = l[g][r] * resc + add;
-                m[g][r] = new_m;
+        }
 #pragma unroll
-                for (int dt = 0; dt < 16; ++dt) O[g][dt][r] *= resc;
+        for (int g = 0; g < NT; ++g)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float from = m[g][r] == -INFINITY ? 0.f : m[g][r];   // nothing seen yet: every score is -inf
+                const float p0 = exp2_of(S[g][0][r] - from), p1 = exp2_of(S[g][1][r] - from);
+                l[g][r] += row16_sum(p0 + p1);
                 pt[(g * 16 + 4 * lg + r) * 32 + j] = p0 * kProbScale;
                 pt[(g * 16 + 4 * lg + r) * 32 + 16 + j] = p1 * kProbScale;
             }
-        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        half8_t pa_hi[NT], pa_lo[NT];
+        half8_t pa[NT][2];
 #pragma unroll
         for (int g = 0; g < NT; ++g) {
             const float* src = pt + (g * 16 + j) * 32 + 8 * lg;  // A lane (pair j, tokens 8 lg .. 8 lg + 7)
@@ -310,20 +343,25 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
             const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
             uint4 hi, lo;
             split_half8(x, hi, lo);
-            pa_hi[g] = __builtin_bit_cast(half8_t, hi);
-            pa_lo[g] = __builtin_bit_cast(half8_t, lo);
+            pa[g][0] = __builtin_bit_cast(half8_t, hi);
+            pa[g][1] = __builtin_bit_cast(half8_t, lo);
         }
-        const uint16_t* vcol = vt + (size_t(kvh) * HD + j) * T + (t0 - base32) + 8 * lg;
+        auto values = [&](int first) {
 #pragma unroll
-        for (int dt = 0; dt < 16; ++dt) {
-            if (dt % 8 == 0) __builtin_amdgcn_sched_barrier(0);   // eight value operands in flight: all sixteen cost the second wave
-            const half8_t vb = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(vcol + size_t(16 * dt) * T));
+            for (int half = 0; half < 2; ++half)
 #pragma unroll
-            for (int g = 0; g < NT; ++g) {
-                O[g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa_hi[g], vb, O[g][dt], 0, 0, 0);
-                O[g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa_lo[g], vb, O[g][dt], 0, 0, 0);
-            }
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int g = 0; g < NT; ++g)
+                        O[g][first + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[g][half], __builtin_bit_cast(half8_t, vb[i]), O[g][first + i], 0, 0, 0);
+        };
+        values(0);
+        if constexpr (NT > 1) __builtin_amdgcn_sched_barrier(0);
+        ask_values(8);
+        if constexpr (NT == 1) {
+            if (ti + 4 < end) ask_keys(ti + 4, kb);
         }
+        values(8);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -341,8 +379,8 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
                 if (w > 0) {
                     const float mo = ml[(g * 16 + 4 * lg + r) * 2], lo_ = ml[(g * 16 + 4 * lg + r) * 2 + 1];
                     const float M = fmaxf(m[g][r], mo);
-                    mine = m[g][r] == -INFINITY ? 0.f : expf(m[g][r] - M);
-                    theirs = mo == -INFINITY ? 0.f : expf(mo - M);
+                    mine = m[g][r] == -INFINITY ? 0.f : exp2_of(m[g][r] - M);
+                    theirs = mo == -INFINITY ? 0.f : exp2_of(mo - M);
                     l[g][r] = l[g][r] * mine + lo_ * theirs;
                     m[g][r] = M;
                 }
@@ -367,7 +405,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         }
     }
     __syncthreads();
-    for (uint32_t idx = threadIdx.x; idx < kTileQueries * 32; idx += 256) {   // 32 consecutive lanes: one (row, head)
+    for (uint32_t idx = threadIdx.x; idx < kPairs * 32; idx += 256) {   // 32 consecutive lanes: one (row, head)
         const uint32_t p = idx / 32, c8 = idx % 32, i = p & 15;
         const uint32_t row = r0 + (p >> group_shift), head = kvh * group + (p & (group - 1));
         if (row >= rows) continue;
@@ -403,7 +441,7 @@ prefill_attention_merge_kernel(AttentionOut to, uint32_t rows, uint32_t q_heads,
 #pragma unroll 4
     for (uint32_t p = 0; p < parts; ++p) {
         const size_t at = p * stride + pair;
-        const float mp = to.part_ml[2 * at], w = mp == -INFINITY ? 0.f : expf(mp - M);   // a part can hold no visible token
+        const float mp = to.part_ml[2 * at], w = mp == -INFINITY ? 0.f : exp2_of(mp - M);   // a part can hold no visible token
         den += w * to.part_ml[2 * at + 1];
         const float4 a = *reinterpret_cast<const float4*>(to.part_o + at * HD + 8 * c8), b = *reinterpret_cast<const float4*>(to.part_o + at * HD + 8 * c8 + 4);
         v[0] = fmaf(w, a.x, v[0]); v[1] = fmaf(w, a.y, v[1]); v[2] = fmaf(w, a.z, v[2]); v[3] = fmaf(w, a.w, v[3]);
@@ -480,10 +518,14 @@ extern "C" int guffin_hip_publish_run(void* stream, const void* run_k, const voi
 }
 
 namespace {
-// parts of the key range: enough workgroups for two per compute unit, every wave of a part with a tile of its own
-uint32_t attention_parts(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_t group) {
-    const uint32_t workgroups = ((rows * group + kTileQueries - 1) / kTileQueries) * kv_heads;
-    return std::max(1u, std::min(512u / workgroups, T / 128));
+// A tiles of a workgroup and parts of the key range.  Two tiles read a key and a value row once for twice the queries, so they
+// stay while they leave a workgroup per compute unit; a short run takes single tiles (half the accumulators, half the merge)
+// and parts: two workgroups per compute unit, every wave of a part with a tile of its own.
+struct AttentionCut { uint32_t tiles, parts; };
+AttentionCut attention_cut(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_t group) {
+    const uint32_t pairs = rows * group, twos = (pairs + 31) / 32 * kv_heads, ones = (pairs + 15) / 16 * kv_heads;
+    if (twos >= 256) return {2, 1};
+    return {1, std::max(1u, std::min(512u / ones, T / 128))};
 }
 uint64_t transposed_bytes(uint32_t T, uint32_t kv_heads) { return (uint64_t(kv_heads) * 256 * T * 2 + 255) & ~uint64_t{255}; }
 }  // namespace
@@ -495,7 +537,7 @@ extern "C" uint64_t guffin_hip_prefill_attention_workspace_bytes(uint32_t rows, 
     const uint32_t T = value_span(rows, position, window).T;
     uint64_t states = 0;
     for (uint32_t group = 1; group <= 4; group *= 2) {
-        const uint64_t parts = attention_parts(rows, T, kv_heads, group);
+        const uint64_t parts = attention_cut(rows, T, kv_heads, group).parts;
         if (parts > 1) states = std::max(states, parts * rows * kv_heads * group * (256 + 2) * 4);
     }
     return transposed_bytes(T, kv_heads) + states;
@@ -511,7 +553,7 @@ bool prefill_attention_on_matrix_core(const void* q, const void* ring_k, const v
 }
 
 uint64_t prefill_attention_most_bytes(uint32_t rows, uint32_t T, uint32_t q_heads, uint32_t kv_heads) {
-    const uint64_t parts = attention_parts(rows, T, kv_heads, q_heads / kv_heads);
+    const uint64_t parts = attention_cut(rows, T, kv_heads, q_heads / kv_heads).parts;
     return transposed_bytes(T, kv_heads) + (parts > 1 ? parts * rows * q_heads * (256 + 2) * 4 : 0);
 }
 
@@ -520,13 +562,16 @@ int prefill_attention_run(hipStream_t s, const float* q, const void* ring_k, con
                           void* workspace) {
     const ValueSpan vs = value_span(rows, position, window);
     const uint32_t group = q_heads / kv_heads, shift = group == 1 ? 0 : group == 2 ? 1 : 2;
-    const uint32_t parts = attention_parts(rows, vs.T, kv_heads, group);
+    const auto [nt, parts] = attention_cut(rows, vs.T, kv_heads, group);
     float* states = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + transposed_bytes(vs.T, kv_heads));
     const AttentionOut to {out, image, states, states + size_t(parts) * rows * q_heads * 256};
-    constexpr size_t lds = 2 * 16384 + 4 * 2 * 16 * 32 * 4 + kTileQueries * 2 * 4;
-    launch(prefill_attention_mfma_kernel, dim3((rows * group + kTileQueries - 1) / kTileQueries, kv_heads, parts), dim3(256), lds, s, q,
-           static_cast<const uint16_t*>(ring_k), static_cast<const uint16_t*>(run_k), static_cast<const uint16_t*>(workspace), to, rows, position,
-           window, ring_mask, q_heads, kv_heads, scale, vs.base32, vs.T, shift);
+    const size_t lds = nt * (16384 + 4 * 16 * 32 * 4 + 16 * 2 * 4);
+    const dim3 grid((rows * group + 16 * nt - 1) / (16 * nt), kv_heads, parts);
+#define GUFFIN_PA(NT_) launch(prefill_attention_mfma_kernel<NT_>, grid, dim3(256), lds, s, q, static_cast<const uint16_t*>(ring_k), \
+                              static_cast<const uint16_t*>(run_k), static_cast<const uint16_t*>(workspace), to, rows, position, window, \
+                              ring_mask, q_heads, kv_heads, scale, vs.base32, vs.T, shift)
+    if (nt == 1) GUFFIN_PA(1); else GUFFIN_PA(2);
+#undef GUFFIN_PA
     if (int rc = check_launch("prefill_attention_mfma")) return rc;
     if (parts == 1) return GUFFIN_OK;
     launch(prefill_attention_merge_kernel, dim3((rows * q_heads + 7) / 8), dim3(256), 0, s, to, rows, q_heads, parts);
