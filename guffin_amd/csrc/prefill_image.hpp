@@ -33,8 +33,10 @@ __host__ __device__ inline ImageLayout image_layout(uint32_t M, uint32_t K) {
 }
 
 // Elements 8t .. 8t+7 of row `row` (t counts along K).  The lanes of a span (32 or 4 consecutive t in consecutive,
-// aligned lanes) must run it together.
-__device__ __forceinline__ void emit_image_values(const float (&v)[8], uint32_t t, uint32_t row, const ImageLayout& L, uint8_t* blob) {
+// aligned lanes) must run it together.  records: where a workgroup that holds 8 rows of eight groups collects their pieces of the
+// records (16 KB of LDS) instead of writing 16 bytes at a time to lines that it shares with other rows.
+__device__ __forceinline__ void emit_image_values(const float (&v)[8], uint32_t t, uint32_t row, const ImageLayout& L, uint8_t* blob,
+                                                  uint8_t* records = nullptr) {
     constexpr int order[8] = {0, 2, 1, 3, 4, 6, 5, 7};
     const uint32_t g = t >> 2, s = t & 3u;
     float sum = v[0], m = fabsf(v[0]);
@@ -80,7 +82,8 @@ __device__ __forceinline__ void emit_image_values(const float (&v)[8], uint32_t 
         }
         hi[p] = hw; lo[p] = lw;
     }
-    uint8_t* base = blob + (size_t(g) * (L.mpad / 16) + tile) * 2048 + (i16 + 16 * s) * 16;
+    uint8_t* base = records ? records + (g & 7u) * 2048 : blob + (size_t(g) * (L.mpad / 16) + tile) * 2048;
+    base += (i16 + 16 * s) * 16;
     *reinterpret_cast<uint4*>(base) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
     *reinterpret_cast<uint4*>(base + 1024) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
 }

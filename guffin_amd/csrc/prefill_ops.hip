@@ -108,7 +108,7 @@ prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_
         load8_words(gamma_post + 8 * t, gp);
         load8(residual + at, res);
         load8_words(gamma_next + 8 * t, gn);
-        sum_planes8<4>(x + at, planes, plane_stride, v);
+        sum_planes8<8>(x + at, planes, plane_stride, v);
     }
     float ss = 0.f;
 #pragma unroll
@@ -133,20 +133,31 @@ prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_
     if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
 }
 
-// one thread per 8 columns of a row
+// grid (width / 256, ceil(rows / 8)): 8 rows of 256 columns, a thread 8 of them; the rows' operand pieces leave together, whole
+// 128-byte lines.  (With every thread's 16 bytes written where they belong, into lines shared by workgroups of several XCDs,
+// 2048 x 15360 took 145 us instead of 65.)
 __global__ void __launch_bounds__(256)
 prefill_geglu_kernel(const float* __restrict__ gate, const float* __restrict__ up, uint32_t planes, size_t plane_stride,
                      uint8_t* __restrict__ image, uint32_t rows, uint32_t width) {
-    const uint32_t per_row = width / 8;
-    const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= uint64_t(rows) * per_row) return;   // whole spans leave together
-    const uint32_t row = static_cast<uint32_t>(i / per_row), t = static_cast<uint32_t>(i % per_row);
-    float g[8], u[8];
-    sum_planes8<2>(gate + size_t(row) * width + 8 * t, planes, plane_stride, g);
-    sum_planes8<2>(up + size_t(row) * width + 8 * t, planes, plane_stride, u);
+    __shared__ __attribute__((aligned(16))) uint8_t records[8 * 2048];
+    const ImageLayout L = image_layout(rows, width);
+    const uint32_t t0 = blockIdx.x * 32, c = threadIdx.x & 31, valid = min(32u, width / 8 - t0), row = blockIdx.y * 8 + (threadIdx.x >> 5);
+    if (row < rows && c < valid) {
+        float g[8], u[8];
+        const size_t at = size_t(row) * width + 8 * (t0 + c);
+        sum_planes8<4>(gate + at, planes, plane_stride, g);
+        sum_planes8<4>(up + at, planes, plane_stride, u);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) g[k] = geglu_value(g[k], u[k]);
-    emit_image_values(g, t, row, image_layout(rows, width), image);
+        for (int k = 0; k < 8; ++k) g[k] = geglu_value(g[k], u[k]);
+        emit_image_values(g, t0 + c, row, L, image, records);
+    }
+    __syncthreads();
+    // 8 rows of a record's k-slice are 128 contiguous bytes; padding rows' places hold what they held: nobody looks at them
+    const uint32_t tile = blockIdx.y >> 1, half = (blockIdx.y & 1) * 128;
+    for (uint32_t k = threadIdx.x; k < (valid / 4) * 64; k += 256) {
+        const uint32_t g = k >> 6, at = ((k >> 3) & 7) * 256 + half + (k & 7) * 16;   // hi or lo and k-slice, row
+        *reinterpret_cast<uint4*>(image + (size_t(t0 / 4 + g) * (L.mpad / 16) + tile) * 2048 + at) = *reinterpret_cast<const uint4*>(records + g * 2048 + at);
+    }
 }
 
 // Workgroups [0, head_groups): four (row, query or key head) pairs, a wave each.  The rest: 32 visible tokens of one KV
@@ -260,9 +271,7 @@ int prefill_joint(hipStream_t s, const float* x, uint32_t planes, const float* g
 }
 
 int prefill_geglu(hipStream_t s, const float* gate, const float* up, uint32_t planes, uint8_t* image, uint32_t rows, uint32_t width) {
-    const uint64_t threads = uint64_t(rows) * (width / 8);
-    launch(prefill_geglu_kernel, dim3(static_cast<uint32_t>((threads + 255) / 256)), dim3(256), 0, s, gate, up, planes, size_t(rows) * width,
-           image, rows, width);
+    launch(prefill_geglu_kernel, dim3((width + 255) / 256, (rows + 7) / 8), dim3(256), 0, s, gate, up, planes, size_t(rows) * width, image, rows, width);
     return check_launch("prefill_geglu");
 }
 
