@@ -83,6 +83,20 @@ SHAPES = [
 ]
 
 
+@pytest.mark.parametrize("dtype,K,N", [(0, 32, 64), (0, 512, 64), (0, 544, 128), (0, 992, 64), (1, 256, 64), (1, 1024, 128), (1, 1280, 64),
+                                       (1, 1792, 64), (2, 256, 128), (2, 768, 64), (2, 1280, 192)])
+@pytest.mark.parametrize("offset", [0, 2, 6])
+def test_repack_of_ragged_block_runs(hip, dtype, K, N, offset):
+    """Numbers of blocks that fill a workgroup's share once, exactly and with every kind of rest, from streams that start
+    at any 16-bit word; every byte against the inverse map (unpack)."""
+    import torch
+    w = synth.make_weight(dtype, K, N, seed=40 + dtype)
+    buf = torch.zeros(w.size + 16, dtype=torch.uint8, device="cuda")
+    buf[offset:offset + w.size] = dev(w)
+    tiles = hip.repack(dtype, buf[offset:offset + w.size], K, N)
+    assert np.array_equal(hip.unpack(dtype, tiles, K, N).cpu().numpy(), w)
+
+
 @pytest.mark.parametrize("dtype,K,N", SHAPES)
 @pytest.mark.parametrize("rows", [1, 2])
 def test_packed_gemv_parity(hip, gfo, dtype, K, N, rows):
