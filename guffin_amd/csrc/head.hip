@@ -388,7 +388,9 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
         remaining -= s_above;
     }
     const uint32_t bound = prefix;
-    // ---- collect ----------------------------------------------------------------------------------
+    // ---- collect: this workgroup's keys into LDS, then one reservation in the row's list for all of them ----
+    if (tid == 0) s_count = 0;
+    __syncthreads();
     bool bad = false;
 #pragma unroll
     for (uint32_t u = 0; u < kCollectTile / 1024; ++u) {
@@ -401,17 +403,18 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
             key = make_key(v, t);
             hit = static_cast<uint32_t>(key >> 32) >= bound;
         }
-        const uint64_t mask = __ballot(hit);
-        if (mask) {
-            const int leader = __ffsll(static_cast<long long>(mask)) - 1;
-            uint32_t base = 0;
-            if (lane == uint32_t(leader))
-                base = __hip_atomic_fetch_add(counter, static_cast<uint32_t>(__popcll(mask)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            base = __shfl(base, leader, kWave);
-            const uint32_t at = base + static_cast<uint32_t>(__popcll(mask & ((uint64_t{1} << lane) - 1)));
-            if (hit && at < kCollectCap) __hip_atomic_store(list + at, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (hit) {
+            const uint32_t at = atomicAdd(&s_count, 1u);
+            if (at < kCollectCap) sel[at] = key;
         }
     }
+    __syncthreads();
+    const uint32_t found = s_count;   // above kCollectCap: the row's counter shows it too, and nobody reads the list
+    if (tid == 0 && found) s_bin = __hip_atomic_fetch_add(counter, found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (found)
+        for (uint32_t i = tid; i < min(found, kCollectCap); i += blockDim.x)
+            if (s_bin + i < kCollectCap) __hip_atomic_store(list + s_bin + i, sel[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (bad && status) atomicOr(status + row, GUFFIN_STATUS_NONFINITE);
     // ---- the last workgroup of the row to get here finishes it -----------------------------------------
     __builtin_amdgcn_s_waitcnt(0);
@@ -428,12 +431,14 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
         for (uint32_t i = tid; i < n; i += blockDim.x) sel[i] = __hip_atomic_load(list + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (n <= 512) {
             __syncthreads();
-            for (uint32_t i = tid; i < n; i += blockDim.x) {
-                const uint64_t k = sel[i];
-                uint32_t rank = 0;
-                for (uint32_t j = 0; j < n; ++j) rank += sel[j] > k;
-                if (rank < retain) keys[rank] = k;
-            }
+            // the workgroup's 1024 threads over n keys: 2, 4, 8 or 16 neighbouring lanes count for one of them
+            const uint32_t shift = n <= 64 ? 4 : n <= 128 ? 3 : n <= 256 ? 2 : 1, i = tid >> shift, part = tid & ((1u << shift) - 1);
+            const uint64_t k = i < n ? sel[i] : 0;
+            uint32_t rank = 0;
+#pragma unroll 8
+            for (uint32_t j = part; j < n; j += 1u << shift) rank += sel[j] > k;
+            for (uint32_t o = 1; o < (1u << shift); o <<= 1) rank += __shfl_xor(rank, o, kWave);
+            if (i < n && part == 0 && rank < retain) keys[rank] = k;
         } else {
             for (uint32_t i = n + tid; i < kCollectCap; i += blockDim.x) sel[i] = 0;
             bitonic_desc(sel, kCollectCap);
