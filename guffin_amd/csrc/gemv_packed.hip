@@ -172,9 +172,10 @@ __global__ void unpack_kernel(const uint16_t* __restrict__ src, uint16_t* __rest
     }
 }
 
-// One workgroup per row writes the row's activation receipt (sums, multipliers, image).
+// Receipt (sums, multipliers, image) of a row, 2048 elements per workgroup: one trip to memory whatever the width.
 __global__ void __launch_bounds__(256) group_sums_kernel(const float* __restrict__ x, void* __restrict__ receipt, uint32_t K, uint32_t rows) {
-    emit_receipt(x + size_t(blockIdx.x) * K, 0, K, blockIdx.x, rows, K, receipt);
+    const uint32_t k0 = blockIdx.y * 2048, count = min(2048u, K - k0);
+    emit_receipt(x + size_t(blockIdx.x) * K + k0, k0, count, blockIdx.x, rows, K, receipt);
 }
 
 __global__ void reduce_partials_kernel(const float* __restrict__ part, float* __restrict__ y, uint32_t S, uint32_t count) {
@@ -433,7 +434,7 @@ extern "C" int guffin_hip_group_sums(void* stream, const float* x, float* xsums,
     if (!x || !xsums) return fail(GUFFIN_E_ARG, "group_sums: null pointer");
     if (rows == 0 || rows > 2 || K == 0 || K % 32 != 0) return fail(GUFFIN_E_SHAPE, "group_sums: K must be a positive multiple of 32, rows 1 or 2");
     if (reinterpret_cast<uintptr_t>(xsums) & 255u) return fail(GUFFIN_E_ALIGN, "group_sums: the receipt must be 256-byte aligned");
-    launch(group_sums_kernel, dim3(rows), dim3(256), 0, as_stream(stream), x, xsums, K, rows);
+    launch(group_sums_kernel, dim3(rows, (K + 2047) / 2048), dim3(256), 0, as_stream(stream), x, xsums, K, rows);
     return check_launch("group_sums");
 }
 

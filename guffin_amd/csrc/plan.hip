@@ -508,18 +508,41 @@ struct PrefillScratch {
 enum { kGemmQkv, kGemmO, kGemmGateUp, kGemmDown };
 struct PrefillLaunch { PrefillMatrix m[3]; uint32_t count, K; PrefillSplit split; };
 
-PrefillLaunch prefill_launch(const guffin_model_desc& m, uint32_t layer, int which, uint32_t rows) {
-    const guffin_layer_desc& L = m.layers[layer];
-    const uint32_t H = m.hidden, F = m.ffn, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
-    static constexpr int first[4] = {0, 3, 4, 6}, count[4] = {3, 1, 2, 1};
-    const uint32_t K[4] = {H, QW, H, F}, N[7] = {QW, KW, KW, H, F, F, H};
-    PrefillLaunch g {};
-    g.count = count[which];
-    g.K = K[which];
-    for (uint32_t i = 0; i < g.count; ++i) g.m[i] = {L.dtype[first[which] + i], L.tiles[first[which] + i], N[first[which] + i]};
-    g.split = prefill_split(g.m, g.count, rows, g.K);
-    return g;
-}
+// A block's launches; their splits depend on its seven formats, of which a model has few sets: worked out once per set and call.
+class PrefillLaunches {
+  public:
+    PrefillLaunches(const guffin_model_desc& model, uint32_t rows) : m_(model), rows_(rows) {}
+    PrefillLaunch operator()(uint32_t layer, int which) {
+        const guffin_layer_desc& L = m_.layers[layer];
+        const uint32_t H = m_.hidden, F = m_.ffn, QW = m_.q_heads * m_.head_dim, KW = m_.kv_heads * m_.head_dim;
+        static constexpr int first[4] = {0, 3, 4, 6}, count[4] = {3, 1, 2, 1};
+        const uint32_t K[4] = {H, QW, H, F}, N[7] = {QW, KW, KW, H, F, F, H};
+        auto launch_of = [&](int w) {
+            PrefillLaunch g {};
+            g.count = count[w];
+            g.K = K[w];
+            for (uint32_t i = 0; i < g.count; ++i) g.m[i] = {L.dtype[first[w] + i], L.tiles[first[w] + i], N[first[w] + i]};
+            return g;
+        };
+        size_t at = 0;
+        while (at < sets_.size() && std::memcmp(sets_[at].dtype, L.dtype, sizeof(L.dtype)) != 0) ++at;
+        if (at == sets_.size()) {
+            Set s {};
+            std::memcpy(s.dtype, L.dtype, sizeof(L.dtype));
+            for (int w = 0; w < 4; ++w) { const PrefillLaunch g = launch_of(w); s.split[w] = prefill_split(g.m, g.count, rows_, g.K); }
+            sets_.push_back(s);
+        }
+        PrefillLaunch g = launch_of(which);
+        g.split = sets_[at].split[which];
+        return g;
+    }
+
+  private:
+    struct Set { int32_t dtype[7]; PrefillSplit split[4]; };
+    const guffin_model_desc& m_;
+    uint32_t rows_;
+    std::vector<Set> sets_;
+};
 
 PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, uint8_t* base) {
     Arena ar {base, 0, 0};
@@ -529,10 +552,10 @@ PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, uint8_t
     s.u = ar.take<float>(H > kPrefillMaxWidth ? rows * H : 0);
     s.q = ar.take<float>(rows * QW); s.a = ar.take<float>(rows * QW);
     uint64_t planes = 0;
+    PrefillLaunches launches(m, rows);
     for (uint32_t l = 0; l < m.layer_count; ++l) {
-        if (l && !std::memcmp(m.layers[l].dtype, m.layers[l - 1].dtype, sizeof(m.layers[l].dtype))) continue;
         for (int which = 0; which < 4; ++which) {
-            const PrefillLaunch g = prefill_launch(m, l, which, rows);
+            const PrefillLaunch g = launches(l, which);
             uint64_t width = 0;
             for (uint32_t i = 0; i < g.count; ++i) width += g.m[i].N;
             planes = std::max(planes, uint64_t(g.split.slices) * rows * width);
@@ -605,16 +628,12 @@ extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* mo
                                                 out ? out : s.u, nullptr, rows, H, m.eps, status));
         return out ? GUFFIN_OK : guffin_hip_prefill_pack(stream, s.u, s.image, rows, H);
     };
-    PrefillLaunch g[4];
+    PrefillLaunches launches(m, rows);
     for (uint32_t l = 0; l < m.layer_count; ++l) {
         const guffin_layer_desc& L = m.layers[l];
-        const bool local = is_local(m, l), same = l && !std::memcmp(L.dtype, m.layers[l - 1].dtype, sizeof(L.dtype));
+        const bool local = is_local(m, l);
         const uint32_t ring_mask = (local ? m.ring_local : m.ring_global) - 1, window = local ? m.sliding_window : 0u;
-        static constexpr int first[4] = {0, 3, 4, 6};
-        for (int which = 0; which < 4; ++which) {
-            if (!same) g[which] = prefill_launch(m, l, which, rows);
-            for (uint32_t i = 0; i < g[which].count; ++i) g[which].m[i].tiles = L.tiles[first[which] + i];
-        }
+        const PrefillLaunch g[4] = {launches(l, kGemmQkv), launches(l, kGemmO), launches(l, kGemmGateUp), launches(l, kGemmDown)};
         auto gemm = [&](int which, float* const* y) {
             return prefill_gemm_planes(hs, g[which].m, g[which].count, s.image, y, rows, g[which].K, g[which].split);
         };

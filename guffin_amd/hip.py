@@ -1,5 +1,6 @@
 """ctypes binding of libguffin_hip.so over torch device tensors."""
 import ctypes as C
+import functools
 import os
 
 import torch
@@ -32,6 +33,53 @@ def lib():
         _lib.guffin_hip_last_error.restype = C.c_char_p
         _lib.guffin_hip_arch.restype = C.c_char_p
     return _lib
+
+
+class _Calls:
+    """The entry points of the small operators with their argument types declared once: pointers are plain integers, and a
+    call costs about a microsecond of the host instead of five (these operators run for less than their call used to
+    take).  A prototype of its own per function leaves the attributes of the library object as callers know them."""
+
+    P, U, Q, F, I = C.c_void_p, C.c_uint32, C.c_uint64, C.c_float, C.c_int
+    SIGNATURES = {
+        "guffin_hip_group_sums": (I, P, P, P, U, U),
+        "guffin_hip_gemv_packed": (I, P, I, P, P, P, P, P, U, U, U),
+        "guffin_hip_repack": (I, P, I, P, P, U, U),
+        "guffin_hip_select_candidates": (I, P, P, U, U, U, P, P, P, P, P),
+        "guffin_hip_argmax": (I, P, P, U, U, P, P, P, P),
+        "guffin_hip_draft_law": (I, P, P, U, P, Q, Q, P, P, P, P, P),
+        "guffin_hip_spec_accept": (I, P, P, P, P, P, Q, Q, P, P, P),
+        "guffin_hip_receipt_bytes": (Q, U, U),
+        "guffin_hip_gemv_packed_slices": (U, I, U, U),
+        "guffin_hip_packed_bytes": (Q, I, U, U),
+        "guffin_hip_select_workspace_bytes": (Q, U, U, U),
+        "guffin_hip_draft_law_workspace_bytes": (Q, U),
+        "guffin_hip_forward_scratch_bytes": (Q, P, U, U),
+        "guffin_hip_forward_rows": (I, P, P, P, U, U, P, Q, P, P, P, P, P),
+        "guffin_hip_prefill_scratch_bytes": (Q, P, U),
+        "guffin_hip_prefill_rows": (I, P, P, P, U, U, P, Q, P, P),
+        "guffin_hip_h1_step": (I, P, P, P, P, Q, P, P, P, P, P, P),
+    }
+
+    def __getattr__(self, name):
+        fn = C.CFUNCTYPE(*self.SIGNATURES[name])((name, lib()))
+        setattr(self, name, fn)   # found at once from now on
+        return fn
+
+
+_calls = _Calls()
+
+
+def _raw_stream():
+    return _current_stream(torch.cuda.current_device())
+
+
+# the current stream's handle without a Stream object around it
+_current_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+
+
+def _at(t):
+    return t.data_ptr() if t is not None else None
 
 
 def check(rc):
@@ -111,7 +159,7 @@ class Chain:
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(_raw_stream())
 
 
 def _p(t):
@@ -133,14 +181,14 @@ def gemv(dtype, w, x, N, out=None):
     return out
 
 
+@functools.lru_cache(maxsize=1024)
 def packed_bytes(dtype, K, N):
-    lib().guffin_hip_packed_bytes.restype = C.c_uint64
-    return lib().guffin_hip_packed_bytes(dtype, K, N)
+    return _calls.guffin_hip_packed_bytes(dtype, K, N)
 
 
 def repack(dtype, canonical, K, N):
     tiles = torch.empty_like(canonical)
-    check(lib().guffin_hip_repack(_stream(), dtype, _p(canonical), _p(tiles), K, N))
+    check(_calls.guffin_hip_repack(_raw_stream(), dtype, canonical.data_ptr(), tiles.data_ptr(), K, N))
     return tiles
 
 
@@ -150,19 +198,20 @@ def unpack(dtype, tiles, K, N):
     return canonical
 
 
+@functools.lru_cache(maxsize=1024)
 def receipt_bytes(rows, K):
-    lib().guffin_hip_receipt_bytes.restype = C.c_uint64
-    n = lib().guffin_hip_receipt_bytes(rows, K)
+    n = _calls.guffin_hip_receipt_bytes(rows, K)
     if n == 0:
         raise GuffinError(-2, "receipt: K must be a positive multiple of 32 and rows 1 or 2")
     return n
 
 
 def _receipt(rows, K, device):
-    """New receipt blob; the returned [rows, K/16 + K/32] view of its sums starts at the blob's first byte."""
-    blob = torch.zeros(receipt_bytes(rows, K) // 4, dtype=torch.float32, device=device)
+    """New receipt blob; the returned [rows, K/16 + K/32] view of its sums starts at the blob's first byte.  The operator
+    that is given it writes all of it that is ever read."""
+    blob = torch.empty(receipt_bytes(rows, K) // 4, dtype=torch.float32, device=device)
     n = K // 16 + K // 32
-    return blob[:rows * n].view(rows, n)
+    return blob.as_strided((rows, n), (n, 1))
 
 
 def receipt_parts(sums, rows, K):
@@ -183,24 +232,31 @@ def group_sums(x, out=None):
     rows, K = x.shape
     if out is None:
         out = _receipt(rows, K, x.device)
-    check(lib().guffin_hip_group_sums(_stream(), _p(x), _p(out), rows, K))
+    check(_calls.guffin_hip_group_sums(_raw_stream(), x.data_ptr(), out.data_ptr(), rows, K))
     return out
 
 
+@functools.lru_cache(maxsize=1024)
 def gemv_packed_slices(dtype, K, N):
-    lib().guffin_hip_gemv_packed_slices.restype = C.c_uint32
-    return lib().guffin_hip_gemv_packed_slices(dtype, K, N)
+    return _calls.guffin_hip_gemv_packed_slices(dtype, K, N)
 
 
 def gemv_packed(dtype, tiles, x, xsums, N, partials=None, out=None, reduce=True):
     rows, K = x.shape
-    S = gemv_packed_slices(dtype, K, N)
-    if partials is None:
-        partials = torch.empty((S, rows, N), dtype=torch.float32, device=x.device)
-    if reduce and out is None:
-        out = torch.empty((rows, N), dtype=torch.float32, device=x.device)
-    check(lib().guffin_hip_gemv_packed(_stream(), dtype, _p(tiles), _p(x), _p(xsums), _p(partials),
-                                       _p(out) if reduce else C.c_void_p(0), rows, K, N))
+    if partials is None or (reduce and out is None):
+        # a single plane is the result itself; several and their sum are one allocation
+        S = gemv_packed_slices(dtype, K, N)
+        planes, sum_rows = (S if partials is None else 0), (rows if reduce and out is None else 0)
+        if S == 1 and reduce and partials is None:
+            partials = out = torch.empty((rows, N), dtype=torch.float32, device=x.device) if out is None else out
+        else:
+            both = torch.empty((planes * rows + sum_rows, N), dtype=torch.float32, device=x.device)
+            if partials is None:
+                partials = both[:planes * rows].view(S, rows, N)
+            if sum_rows:
+                out = both[planes * rows:]
+    check(_calls.guffin_hip_gemv_packed(_raw_stream(), dtype, tiles.data_ptr(), x.data_ptr(), xsums.data_ptr(), partials.data_ptr(),
+                                        out.data_ptr() if reduce else None, rows, K, N))
     return out if reduce else partials
 
 
@@ -401,16 +457,27 @@ def _bytes(n, device="cuda"):
     return torch.zeros(int(n), dtype=torch.uint8, device=device)
 
 
+def _zeroed(device, *nbytes):
+    """Cleared byte buffers of the given sizes, one allocation and one fill between them."""
+    starts = [0]
+    for n in nbytes:
+        starts.append(starts[-1] + (int(n) + 15) // 16 * 16)
+    blob = torch.zeros(starts[-1], dtype=torch.uint8, device=device)
+    return [blob[at:at + int(n)] for at, n in zip(starts, nbytes)]
+
+
 def select_candidates(logits, retain, history=None, history_count=None, status=None, result=None):
     rows, vocab = logits.shape
-    lib().guffin_hip_select_workspace_bytes.restype = C.c_uint64
-    ws = _bytes(lib().guffin_hip_select_workspace_bytes(rows, vocab, retain))
+    ws = torch.empty(_calls.guffin_hip_select_workspace_bytes(rows, vocab, retain), dtype=torch.uint8, device="cuda")
+    if result is None and status is None:
+        result, status = _zeroed("cuda", rows * candidates_dtype.itemsize, 4 * rows)
+        status = status.view(torch.int32)
     if result is None:
         result = _bytes(rows * candidates_dtype.itemsize)
     if status is None:
         status = torch.zeros(rows, dtype=torch.int32, device=logits.device)
-    check(lib().guffin_hip_select_candidates(_stream(), _p(logits), rows, vocab, retain, _p(history),
-                                             _p(history_count), _p(ws), _p(result), _p(status)))
+    check(_calls.guffin_hip_select_candidates(_raw_stream(), logits.data_ptr(), rows, vocab, retain, _at(history), _at(history_count),
+                                              ws.data_ptr(), result.data_ptr(), status.data_ptr()))
     return result, status
 
 
@@ -459,26 +526,28 @@ def candidates_to_numpy(result):
 
 def argmax(logits, status=None):
     rows, vocab = logits.shape
-    ws = _bytes(rows * 256 * 8)
-    token = torch.zeros(rows, dtype=torch.int32, device=logits.device)
-    logit = torch.zeros(rows, dtype=torch.float32, device=logits.device)
-    check(lib().guffin_hip_argmax(_stream(), _p(logits), rows, vocab, _p(ws), _p(token), _p(logit), _p(status)))
+    ws = torch.empty(rows * 256 * 8, dtype=torch.uint8, device="cuda")
+    token = torch.empty(rows, dtype=torch.int32, device=logits.device)
+    logit = torch.empty(rows, dtype=torch.float32, device=logits.device)
+    check(_calls.guffin_hip_argmax(_raw_stream(), logits.data_ptr(), rows, vocab, ws.data_ptr(), token.data_ptr(), logit.data_ptr(), _at(status)))
     return token, logit
 
 
 def draft_law(logits, options, seed=0, step=0, draws=None, law=None, proposal=None, status=None, workspace=None):
     vocab = logits.numel()
-    lib().guffin_hip_draft_law_workspace_bytes.restype = C.c_uint64
     if workspace is None:
-        workspace = _bytes(lib().guffin_hip_draft_law_workspace_bytes(vocab))
+        workspace = torch.empty(_calls.guffin_hip_draft_law_workspace_bytes(vocab), dtype=torch.uint8, device="cuda")
+    if law is None and proposal is None and status is None:
+        law, proposal, status = _zeroed("cuda", law_dtype.itemsize, 4, 4)
+        proposal, status = proposal.view(torch.int32), status.view(torch.int32)
     if law is None:
         law = _bytes(law_dtype.itemsize)
     if proposal is None:
         proposal = torch.zeros(1, dtype=torch.int32, device=logits.device)
     if status is None:
         status = torch.zeros(1, dtype=torch.int32, device=logits.device)
-    check(lib().guffin_hip_draft_law(_stream(), _p(logits), vocab, C.byref(options), C.c_uint64(seed),
-                                     C.c_uint64(step), _p(draws), _p(workspace), _p(law), _p(proposal), _p(status)))
+    check(_calls.guffin_hip_draft_law(_raw_stream(), logits.data_ptr(), vocab, C.byref(options), seed, step, _at(draws), workspace.data_ptr(),
+                                      law.data_ptr(), proposal.data_ptr(), status.data_ptr()))
     return law, proposal, status
 
 
@@ -585,8 +654,8 @@ def spec_accept_history(cands, law, history, history_count, proposal, options, s
 def spec_accept(cands, law, proposal, options, seed=0, step=0, draws=None, result=None, status=None):
     if result is None:
         result = _bytes(result_dtype.itemsize)
-    check(lib().guffin_hip_spec_accept(_stream(), _p(cands), _p(law), _p(proposal), C.byref(options),
-                                       C.c_uint64(seed), C.c_uint64(step), _p(draws), _p(result), _p(status)))
+    check(_calls.guffin_hip_spec_accept(_raw_stream(), cands.data_ptr(), law.data_ptr(), proposal.data_ptr(), C.byref(options), seed, step,
+                                        _at(draws), result.data_ptr(), _at(status)))
     return result
 
 

@@ -358,20 +358,19 @@ class DeviceModel:
         """Runs len(tokens) rows; returns (hidden, hidden_sums, priv_k, priv_v)."""
         sh = self.shape
         rows = tokens.numel()
-        lib = hip.lib()
-        lib.guffin_hip_forward_scratch_bytes.restype = C.c_uint64
-        nbytes = lib.guffin_hip_forward_scratch_bytes(C.byref(self.desc), rows, position)
+        nbytes = hip._calls.guffin_hip_forward_scratch_bytes(C.byref(self.desc), rows, position)
         if nbytes == 0:
-            raise hip.GuffinError(-1, lib.guffin_hip_last_error().decode())
-        scratch = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
-        pk, pv = self.private_rows(rows)
-        hidden = torch.zeros((rows, sh.hidden), dtype=torch.float32, device="cuda")
+            raise hip.GuffinError(-1, hip.lib().guffin_hip_last_error().decode())
+        # the pass writes whatever it reads and all of what it returns: nothing here is cleared
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        pk = torch.empty((sh.layers, rows, sh.kv_width), dtype=torch.float16, device="cuda")
+        pv = torch.empty_like(pk)
+        hidden = torch.empty((rows, sh.hidden), dtype=torch.float32, device="cuda")
         sums = hip._receipt(rows, sh.hidden, "cuda")
         if status is None:
             status = hip.new_status()
-        hip.check(lib.guffin_hip_forward_rows(hip._stream(), C.byref(self.desc), hip._p(tokens), rows, position,
-                                              hip._p(scratch), C.c_uint64(nbytes), hip._p(pk), hip._p(pv),
-                                              hip._p(hidden), hip._p(sums), hip._p(status)))
+        hip.check(hip._calls.guffin_hip_forward_rows(hip._raw_stream(), C.byref(self.desc), tokens.data_ptr(), rows, position, scratch.data_ptr(),
+                                                     nbytes, pk.data_ptr(), pv.data_ptr(), hidden.data_ptr(), sums.data_ptr(), status.data_ptr()))
         return hidden, sums, pk, pv, status
 
 
@@ -379,17 +378,15 @@ class DeviceModel:
         """Ingests len(tokens) rows at `position` (rings are updated); returns the output-normed rows."""
         sh = self.shape
         rows = tokens.numel()
-        lib = hip.lib()
-        lib.guffin_hip_prefill_scratch_bytes.restype = C.c_uint64
-        nbytes = lib.guffin_hip_prefill_scratch_bytes(C.byref(self.desc), rows)
+        nbytes = hip._calls.guffin_hip_prefill_scratch_bytes(C.byref(self.desc), rows)
         if nbytes == 0:
-            raise hip.GuffinError(-1, lib.guffin_hip_last_error().decode())
-        scratch = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
-        hidden = torch.zeros((rows, sh.hidden), dtype=torch.float32, device="cuda")
+            raise hip.GuffinError(-1, hip.lib().guffin_hip_last_error().decode())
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        hidden = torch.empty((rows, sh.hidden), dtype=torch.float32, device="cuda")
         if status is None:
             status = hip.new_status()
-        hip.check(lib.guffin_hip_prefill_rows(hip._stream(), C.byref(self.desc), hip._p(tokens), rows, position,
-                                              hip._p(scratch), C.c_uint64(nbytes), hip._p(hidden), hip._p(status)))
+        hip.check(hip._calls.guffin_hip_prefill_rows(hip._raw_stream(), C.byref(self.desc), tokens.data_ptr(), rows, position, scratch.data_ptr(),
+                                                     nbytes, hidden.data_ptr(), status.data_ptr()))
         return hidden, status
 
 
@@ -431,10 +428,9 @@ class H1Plan:
     def step(self, step=None):
         if step is not None:
             self.desc.step = step
-        hip.check(hip.lib().guffin_hip_h1_step(hip._stream(), C.byref(self.desc), hip._p(self.root),
-                                               hip._p(self.scratch), C.c_uint64(self.nbytes), hip._p(self.d_pk),
-                                               hip._p(self.d_pv), hip._p(self.t_pk), hip._p(self.t_pv),
-                                               hip._p(self.result), hip._p(self.status)))
+        hip.check(hip._calls.guffin_hip_h1_step(hip._raw_stream(), C.byref(self.desc), self.root.data_ptr(), self.scratch.data_ptr(),
+                                                self.nbytes, self.d_pk.data_ptr(), self.d_pv.data_ptr(), self.t_pk.data_ptr(),
+                                                self.t_pv.data_ptr(), self.result.data_ptr(), self.status.data_ptr()))
 
     def read_result(self):
         return self.result.cpu().numpy().view(hip.result_dtype)[0]
