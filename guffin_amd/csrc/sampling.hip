@@ -89,20 +89,24 @@ __device__ __forceinline__ bool options_valid(const SamplerOptions& o) {
 }
 
 // Sums whose order matters, one lane's work over LDS: eight operands are read before the first of their adds, so the chain is
-// one of additions, not of LDS reads (64 doubles: 2.7 -> 0.6 us).  Past the end a zero is added, which changes nothing.
+// one of additions, not of LDS reads.  v holds zeros from n up to the next multiple of eight: adding them changes nothing.
 // running[i] = v[0] + ... + v[i]; returns the total
 template <typename T>
-__device__ __forceinline__ T ordered_sums(const T* v, uint32_t n, T* running) {
-    T sum = T(0);
+__device__ __forceinline__ T ordered_sums(const T* __restrict__ v, uint32_t n, T* __restrict__ running) {
+    T sum = T(0), x[8], next[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) x[k] = v[k];
     for (uint32_t i0 = 0; i0 < n; i0 += 8) {
-        T x[8];
+        const uint32_t ahead = i0 + 8 < n ? i0 + 8 : i0;
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) x[k] = i0 + k < n ? v[i0 + k] : T(0);
+        for (uint32_t k = 0; k < 8; ++k) next[k] = v[ahead + k];
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) {
-            sum += x[k];
-            if (running && i0 + k < n) running[i0 + k] = sum;
-        }
+        for (uint32_t k = 0; k < 8; ++k) { sum += x[k]; x[k] = sum; }
+        if (running)
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) running[i0 + k] = x[k];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) x[k] = next[k];
     }
     return sum;
 }
@@ -216,16 +220,18 @@ draft_law_kernel(const Candidates* __restrict__ top, SamplerOptions opt, uint64_
     if (t == 0) {  // descending-tail top-p / min-p in the reference's sequential order
         // the tail sums from the last entry down; the last of them, in slot 0 (always kept), is the total: the
         // same adds in the same order
-        float tail = 0.f;
-        for (uint32_t j0 = n; j0 > 0; j0 = j0 > 8 ? j0 - 8 : 0) {   // eight reads ahead of their adds
-            float x[8];
+        float tail = 0.f, x[8], next[8];
+        const uint32_t top = (n + 7) & ~7u;   // past the end zeros
 #pragma unroll
-            for (uint32_t k = 0; k < 8; ++k) x[k] = k < j0 ? weight[j0 - 1 - k] : 0.f;
+        for (uint32_t k = 0; k < 8; ++k) x[k] = weight[top - 1 - k];
+        for (uint32_t j0 = top; j0 > 0; j0 -= 8) {   // eight reads ahead of their adds
+            const uint32_t ahead = j0 > 8 ? j0 - 8 : 8;
 #pragma unroll
-            for (uint32_t k = 0; k < 8; ++k) {
-                tail = __fadd_rn(tail, x[k]);
-                if (k < j0) running[j0 - 1 - k] = tail;
-            }
+            for (uint32_t k = 0; k < 8; ++k) next[k] = weight[ahead - 1 - k];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) { tail = __fadd_rn(tail, x[k]); x[k] = tail; }
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) { running[j0 - 1 - k] = x[k]; x[k] = next[k]; }
         }
     }
     __syncthreads();
@@ -534,12 +540,16 @@ __device__ int prepare_distribution(const Candidates* cand, const SamplerOptions
         float logit = sc.raw[t];
         bool dup = false;
         if (!isfinite(logit)) atomicMin(&sc.err, -4);
+        // every lane walks the whole record without a branch, so that the reads run ahead (with a loop of its own length and
+        // an exit per lane this step alone took 3.6 us of the kernel)
+        bool differs = false;
 #pragma unroll 8
-        for (uint32_t j = 0; j < t; ++j)
-            if (sc.tok[j] == token) {
-                dup = true;
-                if (sc.raw[j] != logit) atomicMin(&sc.err, -5);
-            }
+        for (uint32_t j = 0; j < n; ++j) {
+            const bool same = (sc.tok[j] == token) & (j < t);
+            dup |= same;
+            differs |= same & (sc.raw[j] != logit);
+        }
+        if (differs) atomicMin(&sc.err, -5);
         if (!dup) {
             for (uint32_t h = 0; h < history_count; ++h)
                 if (sc.hist[h] == token) {
@@ -568,12 +578,13 @@ __device__ int prepare_distribution(const Candidates* cand, const SamplerOptions
     }
     __syncthreads();
     if (opt.temperature == 0.f) {
-        if (t == 0) { out.count = 1; out.total = 1.0; out.weight[0] = 1.0; }
+        if (t == 0) { out.count = 1; out.total = 1.0; }
+        if (t < kMaxTopK) out.weight[t] = t == 0 ? 1.0 : 0.0;
         __syncthreads();
         return 0;
     }
     const float max_logit = sc.logit[0];
-    if (t < count) sc.w[t] = exp(static_cast<double>(__fsub_rn(sc.logit[t], max_logit)));
+    if (t < kMaxTopK) sc.w[t] = t < count ? exp(static_cast<double>(__fsub_rn(sc.logit[t], max_logit))) : 0.0;
     __syncthreads();
     if (t == 0) {
         ordered_sums(sc.w, count, sc.run);
@@ -589,8 +600,8 @@ __device__ int prepare_distribution(const Candidates* cand, const SamplerOptions
     }
     __syncthreads();
     count = sc.kept < sc.cut ? sc.kept : sc.cut;
-    if (t < count)
-        out.weight[t] = exp(static_cast<double>(__fsub_rn(sc.logit[t], max_logit)) / static_cast<double>(opt.temperature));
+    if (t < kMaxTopK)   // zeros behind the last entry, for the sums
+        out.weight[t] = t < count ? exp(static_cast<double>(__fsub_rn(sc.logit[t], max_logit)) / static_cast<double>(opt.temperature)) : 0.0;
     __syncthreads();
     if (t == 0) {
         const double norm = ordered_sums(out.weight, count, static_cast<double*>(nullptr));
@@ -625,7 +636,7 @@ __device__ double validated_total(const Prepared& p, Scratch& sc) {
             for (uint32_t i0 = 0; i0 < count; i0 += 8) {   // a zero past the end changes neither total nor correction
                 double x[8];
 #pragma unroll
-                for (uint32_t k = 0; k < 8; ++k) x[k] = i0 + k < count ? p.weight[i0 + k] : 0.0;
+                for (uint32_t k = 0; k < 8; ++k) x[k] = p.weight[i0 + k];
 #pragma unroll
                 for (uint32_t k = 0; k < 8; ++k) {
                     const double w = x[k];
@@ -649,7 +660,7 @@ __device__ uint32_t select_prepared(const Prepared& p, double draw) {
     for (uint32_t i0 = 0; i0 < p.count; i0 += 8) {
         double x[8];
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) x[k] = i0 + k < p.count ? p.weight[i0 + k] : 0.0;
+        for (uint32_t k = 0; k < 8; ++k) x[k] = p.weight[i0 + k];
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
             cumulative += x[k];
@@ -771,6 +782,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
             if (w < (t >> 6)) at += wave_count[w];
             entries += wave_count[w];
         }
+        if (t >= entries && t < kMaxTopK) residual.weight[t] = 0.0;
         if (more) { residual.token[at] = target.token[t]; residual.weight[at] = diff[t]; }
         __syncthreads();
         if (t == 0) {
