@@ -45,6 +45,20 @@ int resident_launch(hipStream_t stream, const guffin_model_desc& m, uint32_t row
                     const void* u_receipt_in, float* x_out, float* u_out, void* u_receipt_out, uint32_t max_ring_tokens,
                     uint32_t* status);
 
+// ---- K/V rows of every block of a model between its rings and a flat block of rows (prefill.hip) ---------------
+// flat_k / flat_v: [layer][flat_rows][kv width], position p in row p & (flat_rows - 1), flat_rows a power of two.  Save and
+// Restore copy positions [first, first + count); Publish saves them and then puts row path[i] of the private rows
+// [layer][priv_rows][kv width] at position first + i.
+enum class KvMove { Save, Restore, Publish };
+constexpr uint32_t kMovePath = 8;   // rows a Publish may take
+int kv_move_rows(hipStream_t s, const guffin_model_desc& m, KvMove move, void* flat_k, void* flat_v, uint32_t flat_rows, uint32_t first,
+                 uint32_t count, const void* priv_k = nullptr, const void* priv_v = nullptr, uint32_t priv_rows = 0,
+                 const uint32_t* path = nullptr);
+
+// guffin_hip_commit_rows of every row, with the rows' final states kept: kept[row] = hidden[row] unless kept is null (plan.hip)
+int commit_rows_keeping(void* stream, const guffin_model_desc& m, const void* priv_k, const void* priv_v, void* const* ring_k_table,
+                        void* const* ring_v_table, const uint32_t* accepted, uint32_t position, uint32_t rows, const float* hidden, float* kept);
+
 // ---- attention with a host-known schedule (attention.hip), used by the block graph of plan.hip --------
 int qkv_attention_scheduled(void* stream, const float* q_raw, const float* k_raw, const float* v_raw, uint32_t planes,
                             uint64_t q_plane_stride, uint64_t k_plane_stride, uint64_t v_plane_stride, const float* q_norm,

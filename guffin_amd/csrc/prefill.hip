@@ -478,7 +478,77 @@ __global__ void kv_cache_copy_kernel(const U4a4* __restrict__ src_k, const U4a4*
     dst_v[to] = src_v[from];
 }
 
+// The same for every block of a model in one launch: a few rows of a few KB per block are a launch's latency and nothing else, and
+// a launch per block made the drafter's transaction and the ticket's commit 18 to 96 of them (48 blocks, two rows: 96 launches
+// -> 1).  A Publish reads, saves and overwrites a ring piece in one thread.
+constexpr uint32_t kMoveLayers = 64;   // blocks per launch: their rings travel as kernel arguments
+struct MoveRings { U4a4* k[kMoveLayers]; U4a4* v[kMoveLayers]; uint64_t local; };
+struct MovePath { uint32_t row[kMovePath]; };
+template <KvMove MOVE>
+__global__ void kv_move_kernel(const MoveRings rings, U4a4* __restrict__ flat_k, U4a4* __restrict__ flat_v, uint32_t flat_rows,
+                               const U4a4* __restrict__ priv_k, const U4a4* __restrict__ priv_v, uint32_t priv_rows, const MovePath path,
+                               uint32_t first, uint32_t mask_local, uint32_t mask_global, uint32_t row_vec) {
+    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x, layer = blockIdx.y, t = blockIdx.z;
+    if (c >= row_vec) return;
+    const uint32_t mask = (rings.local >> layer) & 1u ? mask_local : mask_global, position = first + t;
+    const size_t ring = size_t(position & mask) * row_vec + c, flat = (size_t(layer) * flat_rows + (position & (flat_rows - 1u))) * row_vec + c;
+    U4a4 *rk = rings.k[layer] + ring, *rv = rings.v[layer] + ring;
+    if constexpr (MOVE == KvMove::Restore) {
+        *rk = flat_k[flat];
+        *rv = flat_v[flat];
+    } else {
+        flat_k[flat] = *rk;
+        flat_v[flat] = *rv;
+        if constexpr (MOVE == KvMove::Publish) {
+            const size_t from = (size_t(layer) * priv_rows + path.row[t]) * row_vec + c;
+            *rk = priv_k[from];
+            *rv = priv_v[from];
+        }
+    }
+}
+
 }  // namespace
+
+int kv_move_rows(hipStream_t s, const guffin_model_desc& m, KvMove move, void* flat_k, void* flat_v, uint32_t flat_rows, uint32_t first,
+                 uint32_t count, const void* priv_k, const void* priv_v, uint32_t priv_rows, const uint32_t* path) {
+    if (count == 0) return GUFFIN_OK;
+    const uint32_t kvw = m.kv_heads * m.head_dim, row_vec = kvw / 8;
+    if (count > flat_rows || count > m.ring_local || count > m.ring_global)
+        return fail(GUFFIN_E_CAPACITY, "kv_move_rows: more rows than one side holds");
+    MovePath rows {};
+    if (move == KvMove::Publish) {
+        if (count > kMovePath) return fail(GUFFIN_E_CAPACITY, "kv_move_rows: a path of at most 8 rows");
+        for (uint32_t i = 0; i < count; ++i) rows.row[i] = path[i];
+    }
+    for (uint32_t l = 0; l < m.layer_count; ++l) {   // nothing moves unless everything can
+        const guffin_layer_desc& L = m.layers[l];
+        if (!L.ring_k || !L.ring_v) return fail(GUFFIN_E_ARG, "kv_move_rows: every layer needs its rings");
+        if ((reinterpret_cast<uintptr_t>(L.ring_k) | reinterpret_cast<uintptr_t>(L.ring_v)) & 3u)
+            return fail(GUFFIN_E_ALIGN, "kv_move_rows: rows must be 4-byte aligned");
+    }
+    for (uint32_t l0 = 0; l0 < m.layer_count; l0 += kMoveLayers) {
+        const uint32_t n = std::min(kMoveLayers, m.layer_count - l0);
+        MoveRings r {};
+        for (uint32_t i = 0; i < n; ++i) {
+            const guffin_layer_desc& L = m.layers[l0 + i];
+            r.k[i] = static_cast<U4a4*>(L.ring_k);
+            r.v[i] = static_cast<U4a4*>(L.ring_v);
+            if (layer_is_local(m.global_period, l0 + i)) r.local |= uint64_t{1} << i;
+        }
+        const size_t flat_at = size_t(l0) * flat_rows * row_vec, priv_at = size_t(l0) * priv_rows * row_vec;
+        U4a4 *fk = static_cast<U4a4*>(flat_k) + flat_at, *fv = static_cast<U4a4*>(flat_v) + flat_at;
+        const U4a4 *pk = priv_k ? static_cast<const U4a4*>(priv_k) + priv_at : nullptr, *pv = priv_v ? static_cast<const U4a4*>(priv_v) + priv_at : nullptr;
+        const dim3 grid((row_vec + 255) / 256, n, count), block(std::min(row_vec, 256u));
+#define GUFFIN_MOVE(M) launch(kv_move_kernel<M>, grid, block, 0, s, r, fk, fv, flat_rows, pk, pv, priv_rows, rows, first, m.ring_local - 1, m.ring_global - 1, row_vec)
+        if (move == KvMove::Save) GUFFIN_MOVE(KvMove::Save);
+        else if (move == KvMove::Restore) GUFFIN_MOVE(KvMove::Restore);
+        else GUFFIN_MOVE(KvMove::Publish);
+#undef GUFFIN_MOVE
+        if (int rc = check_launch("kv_move_rows")) return rc;
+    }
+    return GUFFIN_OK;
+}
+
 }  // namespace guffin
 
 using namespace guffin;

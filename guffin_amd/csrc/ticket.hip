@@ -67,23 +67,9 @@ void clear_transaction(guffin_verify_ticket* t) {
     t->provisional_count = 0;
 }
 
-struct LayerRing { void* k; void* v; uint32_t mask; };
-LayerRing ring_of(const guffin_model_desc& m, uint32_t layer) {
-    const bool local = layer_is_local(m.global_period, layer);  // the same rule as the forward pass it commits for
-    return {m.layers[layer].ring_k, m.layers[layer].ring_v, (local ? m.ring_local : m.ring_global) - 1u};
-}
-
 // restores ring rows [position + first, position + first + count) of every layer from the backup rows
 int restore_rows(hipStream_t s, const guffin_verify_ticket* t, uint32_t first, uint32_t count) {
-    const guffin_model_desc& m = *t->target;
-    const uint32_t kvw = m.kv_heads * m.head_dim;
-    for (uint32_t l = 0; l < m.layer_count; ++l) {
-        const LayerRing r = ring_of(m, l);
-        const uint16_t* bk = static_cast<const uint16_t*>(t->backup_k) + size_t(l) * kMaxTicketRows * kvw;
-        const uint16_t* bv = static_cast<const uint16_t*>(t->backup_v) + size_t(l) * kMaxTicketRows * kvw;
-        GUFFIN_TRY(guffin_hip_kv_cache_copy(s, bk, bv, r.k, r.v, t->position + first, count, kMaxTicketRows - 1u, r.mask, kvw));
-    }
-    return GUFFIN_OK;
+    return kv_move_rows(s, *t->target, KvMove::Restore, t->backup_k, t->backup_v, kMaxTicketRows, t->position + first, count);
 }
 
 }  // namespace
@@ -238,30 +224,16 @@ extern "C" int guffin_hip_ticket_provisional_commit(void* stream, guffin_verify_
             return fail(GUFFIN_E_ARG, "ticket_provisional_commit: selected nodes are not one causal path");
     }
     const guffin_model_desc& m = *t->target;
-    const uint32_t kvw = m.kv_heads * m.head_dim;
     hipStream_t hs = as_stream(stream);
     for (uint32_t i = 0; i < kMaxTicketRows; ++i) t->provisional_path[i] = i < count ? path[i] : 0u;
-    int rc = GUFFIN_OK;
-    if (hipMemcpyAsync(t->selected, t->provisional_path, count * sizeof(uint32_t), hipMemcpyHostToDevice, hs) != hipSuccess)
-        rc = fail(GUFFIN_E_HIP, "ticket_provisional_commit: upload failed");
-    // backups read the durable rows of every layer before any selected private row is published
-    for (uint32_t l = 0; rc == GUFFIN_OK && l < m.layer_count; ++l) {
-        const LayerRing r = ring_of(m, l);
-        uint16_t* bk = static_cast<uint16_t*>(t->backup_k) + size_t(l) * kMaxTicketRows * kvw;
-        uint16_t* bv = static_cast<uint16_t*>(t->backup_v) + size_t(l) * kMaxTicketRows * kvw;
-        rc = guffin_hip_kv_cache_copy(stream, r.k, r.v, bk, bv, t->position, count, r.mask, kMaxTicketRows - 1u, kvw);
-    }
-    const bool rings_touched = rc == GUFFIN_OK;
-    for (uint32_t l = 0; rc == GUFFIN_OK && l < m.layer_count; ++l) {
-        const LayerRing r = ring_of(m, l);
-        const uint16_t* pk = static_cast<const uint16_t*>(t->priv_k) + size_t(l) * t->rows * kvw;
-        const uint16_t* pv = static_cast<const uint16_t*>(t->priv_v) + size_t(l) * t->rows * kvw;
-        rc = guffin_hip_kv_scatter(stream, pk, pv, t->selected, r.k, r.v, t->position, count, kvw, r.mask);
-    }
+    // every durable row goes to its backup row before the selected private row takes its place
+    int rc = kv_move_rows(hs, m, KvMove::Publish, t->backup_k, t->backup_v, kMaxTicketRows, t->position, count, t->priv_k, t->priv_v,
+                          t->rows, t->provisional_path);
+    const bool rings_touched = rc == GUFFIN_OK || rc == GUFFIN_E_HIP;
     if (rc == GUFFIN_OK && hipStreamSynchronize(hs) != hipSuccess) rc = fail(GUFFIN_E_HIP, "ticket_provisional_commit: wait failed");
     if (rc != GUFFIN_OK) {
-        // some rings may hold the pass's rows and some not (:586-590); before the first scatter
-        // nothing durable has changed and the ticket stays completed
+        // some rings may hold the pass's rows and some not (:586-590); a move that was refused changed nothing durable
+        // and the ticket stays completed
         if (rings_touched) t->state = GUFFIN_TXN_POISONED;
         return rc;
     }

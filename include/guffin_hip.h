@@ -783,7 +783,7 @@ typedef struct guffin_verify_ticket {
     void* priv_k; void* priv_v;              /* device, [blocks][rows][kv width] fp16: the pass's own rows */
     void* backup_k; void* backup_v;          /* device, [blocks][4][kv width] fp16: ring rows a commit overwrites */
     uint32_t* tokens;                        /* device u32[4]: the rows' tokens */
-    uint32_t* selected;                      /* device u32[4]: the selected path */
+    uint32_t* selected;                      /* device u32[4]; a commit's path travels with its launch, nothing is written here */
     void* candidates;                        /* device, 4 candidate records */
     uint32_t* status;                        /* device u32[5]: the pass's status word, one selection status per row */
     uint32_t retain;                         /* candidates kept per row (top_k), 1..320 */
