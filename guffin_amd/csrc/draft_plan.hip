@@ -18,9 +18,12 @@
 // went back to.  Same observable behaviour: an aborted or truncated suffix leaves every ring row as it was, and
 // logits after a commit equal those of a plain replay of the kept tokens.
 //
-// Every call is host-synchronous (it returns when its device work is done); the path that is timed is
-// guffin_hip_h1_step, which needs none of this.
+// Every call is host-synchronous (it returns when its device work is done), but inside a call the host waits once: the
+// passes and laws of up to kBatch tokens are enqueued behind each other, a drafted token passing from law to embedding in
+// device memory, and the status word is read when all of them are done (run_batch).  Waiting for every pass and law, and
+// a copy launch per block, took 1.4 of the 5.0 ms of six passes and four proposals of an 18-block drafter.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
@@ -34,7 +37,12 @@ namespace {
 constexpr uint32_t kDefaultTransactionRows = 32;   // when the caller names none (the reference's callers use 96 or 256)
 constexpr uint32_t kMaxHorizon = 23;        // external_speculation_max_horizon
 constexpr uint64_t kLawBytes = 8 + 256 * 4 + 257 * 8;
+constexpr uint32_t kBatch = kMaxHorizon + 1;   // passes between two looks at the status word; no more than a transaction holds
+constexpr uint32_t kHistory = 64;              // the sampler's window
 struct Draws { uint32_t word, pad; double u_accept, u_residual, u_next; };
+// What a call uploads, in one copy: the input tokens of a batch, the draws, and the sampler's window with the drafted tokens
+// behind it: chain[kHistory + i] is drafted token i, and the window before it the up to 64 words that precede it
+struct Staging { Draws draws[kMaxHorizon]; uint32_t tokens[kBatch]; uint32_t chain[kHistory + kMaxHorizon]; };
 
 struct Carve {
     uint8_t* base; uint64_t used;
@@ -50,8 +58,8 @@ struct Buffers {
     uint8_t* forward; uint64_t forward_bytes;
     uint16_t *priv_k, *priv_v, *backup_k, *backup_v;
     float *hidden, *hidden_sums, *hidden_saved, *sums_saved, *txn_hidden, *logits, *parts, *scores;
-    uint32_t *tokens, *drafted, *history, *status, *proposal;
-    Draws* draws;
+    Staging* staging;
+    uint32_t* status;
     uint8_t *law_ws, *law;
     uint64_t* cdf;
     void **ring_k_table, **ring_v_table;
@@ -81,12 +89,8 @@ Buffers carve(const guffin_model_desc& m, uint32_t arena, void* workspace, uint6
     b.logits = c.take<float>(2 * uint64_t(m.vocab));
     b.parts = c.take<float>(uint64_t(std::max(1u, guffin_hip_gemv_packed_slices(m.head_dtype, m.hidden, m.vocab))) * 2 * m.vocab);
     b.scores = c.take<float>(m.vocab);
-    b.tokens = c.take<uint32_t>(2);
-    b.drafted = c.take<uint32_t>(kMaxHorizon + 1);
-    b.history = c.take<uint32_t>(64);
+    b.staging = c.take<Staging>(1);
     b.status = c.take<uint32_t>(1);
-    b.proposal = c.take<uint32_t>(1);
-    b.draws = c.take<Draws>(kMaxHorizon);
     b.law_ws = c.take<uint8_t>(guffin_hip_draft_law_any_workspace_bytes(m.vocab));
     b.law = c.take<uint8_t>(kLawBytes);
     b.cdf = c.take<uint64_t>(uint64_t(m.vocab) + 1);
@@ -111,83 +115,122 @@ int poison(guffin_draft_plan* p, int code, const char* what) {
 
 // ring rows [first, end) of every layer to the backup arena (save) or back (restore)
 int move_rows(hipStream_t s, const guffin_draft_plan* p, const Buffers& b, uint32_t first, uint32_t end, bool save) {
-    const guffin_model_desc& m = *p->model;
     if (end <= first) return GUFFIN_OK;
-    const uint64_t kvw = uint64_t(m.kv_heads) * m.head_dim;
-    for (uint32_t l = 0; l < m.layer_count; ++l) {
-        const uint32_t ring_mask = (layer_is_local(m.global_period, l) ? m.ring_local : m.ring_global) - 1;
-        const uint32_t arena = p->transaction_arena;
-        void* bk = b.backup_k + uint64_t(l) * arena * kvw;
-        void* bv = b.backup_v + uint64_t(l) * arena * kvw;
-        void* rk = m.layers[l].ring_k;
-        void* rv = m.layers[l].ring_v;
-        const int rc = save ? guffin_hip_kv_cache_copy(s, rk, rv, bk, bv, first, end - first, ring_mask, arena - 1, kvw)
-                            : guffin_hip_kv_cache_copy(s, bk, bv, rk, rv, first, end - first, arena - 1, ring_mask, kvw);
-        if (rc) return rc;
-    }
-    return GUFFIN_OK;
+    return kv_move_rows(s, *p->model, save ? KvMove::Save : KvMove::Restore, b.backup_k, b.backup_v, p->transaction_arena, first, end - first);
 }
 
-// one pass of `rows` tokens (already in b.tokens) at the materialized frontier, published to the rings
-int forward(hipStream_t s, guffin_draft_plan* p, const Buffers& b, uint32_t rows) {
+// one pass of the token at `token` (device memory) at the materialized frontier, published to the rings
+int forward(hipStream_t s, guffin_draft_plan* p, const Buffers& b, const uint32_t* token) {
     const guffin_model_desc& m = *p->model;
     const uint32_t at = p->materialized;
-    if (p->transaction_active && at + rows > p->backup_end) {   // rows below backup_end already hold the originals
-        const uint32_t first = std::max(at, p->backup_end);
-        GUFFIN_TRY(move_rows(s, p, b, first, at + rows, true));
-        p->backup_end = at + rows;
-    }
-    // The resident pass can give up a wait (a device shared with other work): its rows, and whatever else it
-    // raised in the status word, are then not to be trusted.  These calls are host-synchronous anyway: the status
-    // word is read before and after such a pass and, if the bit came up, put back, the resident form is switched
-    // off for the process and the pass runs again, one launch per operator.
-    const bool watched = resident_chosen(m, rows) && g_forward_mode == 0;
-    uint32_t before = 0, after = 0;
-    if (watched && (hipStreamSynchronize(s) != hipSuccess || hipMemcpy(&before, b.status, 4, hipMemcpyDeviceToHost) != hipSuccess))
-        return fail(GUFFIN_E_HIP, "draft_plan: the stream failed");
-    GUFFIN_TRY(guffin_hip_forward_rows(s, &m, b.tokens, rows, at, b.forward, b.forward_bytes, b.priv_k, b.priv_v, b.hidden,
+    GUFFIN_TRY(guffin_hip_forward_rows(s, &m, token, 1, at, b.forward, b.forward_bytes, b.priv_k, b.priv_v, b.hidden,
                                        b.hidden_sums, b.status));
-    if (watched) {
-        if (hipStreamSynchronize(s) != hipSuccess || hipMemcpy(&after, b.status, 4, hipMemcpyDeviceToHost) != hipSuccess)
-            return fail(GUFFIN_E_HIP, "draft_plan: the pass failed");
-        if ((after & GUFFIN_STATUS_SYNC) && !(before & GUFFIN_STATUS_SYNC)) {
-            resident_note_status(after);
-            if (hipMemcpy(b.status, &before, 4, hipMemcpyHostToDevice) != hipSuccess) return fail(GUFFIN_E_HIP, "draft_plan: the pass failed");
-            GUFFIN_TRY(guffin_hip_forward_rows(s, &m, b.tokens, rows, at, b.forward, b.forward_bytes, b.priv_k, b.priv_v, b.hidden,
-                                               b.hidden_sums, b.status));
-        }
-    }
-    GUFFIN_TRY(guffin_hip_commit_rows(s, &m, b.priv_k, b.priv_v, b.ring_k_table, b.ring_v_table, nullptr, at, rows));
-    if (p->transaction_active   // the rows' final normalised states, by their place in the transaction
-        && hipMemcpyAsync(b.txn_hidden + uint64_t(at - p->checkpoint_materialized) * m.hidden, b.hidden, uint64_t(rows) * m.hidden * 4,
-                          hipMemcpyDeviceToDevice, s) != hipSuccess)
-        return fail(GUFFIN_E_HIP, "draft_plan: keeping the rows' final states failed");
-    p->materialized = at + rows;
-    p->last_rows = rows;
+    // a transaction keeps the rows' final normalised states by their place in it
+    float* kept = p->transaction_active ? b.txn_hidden + uint64_t(at - p->checkpoint_materialized) * m.hidden : nullptr;
+    GUFFIN_TRY(commit_rows_keeping(s, m, b.priv_k, b.priv_v, b.ring_k_table, b.ring_v_table, nullptr, at, 1, b.hidden, kept));
+    p->materialized = at + 1;
+    p->last_rows = 1;
     p->logits_valid = 0;
     p->hidden_valid = 1;
     return GUFFIN_OK;
 }
 
+int read_status(hipStream_t s, const Buffers& b, uint32_t* status) {
+    return hipMemcpyWithStream(status, b.status, 4, hipMemcpyDeviceToHost, s) == hipSuccess ? GUFFIN_OK : GUFFIN_E_HIP;
+}
+
 int finish(hipStream_t s, guffin_draft_plan* p, const Buffers& b, const char* what) {
     uint32_t status = 0;
-    if (hipStreamSynchronize(s) != hipSuccess || hipMemcpy(&status, b.status, 4, hipMemcpyDeviceToHost) != hipSuccess)
-        return poison(p, GUFFIN_E_HIP, what);
+    if (read_status(s, b, &status)) return poison(p, GUFFIN_E_HIP, what);
     if (status != 0) return poison(p, GUFFIN_E_NUMERIC, what);
     return GUFFIN_OK;
+}
+
+// the output rows of the pass at the frontier, kept across a transaction so that an abort leaves the plan able to
+// draft from (or read the logits of) the prefix it returns to; rows and receipt lie behind each other on both sides
+int copy_frontier(hipStream_t s, const guffin_model_desc& m, const Buffers& b, bool save) {
+    const size_t bytes = (b.hidden_sums - b.hidden) * 4 + guffin_hip_receipt_bytes(2, m.hidden);
+    if (hipMemcpyAsync(save ? b.hidden_saved : b.hidden, save ? b.hidden : b.hidden_saved, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess)
+        return fail(GUFFIN_E_HIP, "draft_plan: copying the frontier rows failed");
+    return GUFFIN_OK;
+}
+
+// the final state at `position`, which the open transaction ran or began on, back to b.hidden / b.hidden_sums
+int restore_frontier(hipStream_t s, guffin_draft_plan* p, const Buffers& b, uint32_t position) {
+    const guffin_model_desc& m = *p->model;
+    p->hidden_valid = p->logits_valid = 0;
+    if (position > p->checkpoint_materialized) {
+        const float* kept = b.txn_hidden + uint64_t(position - 1 - p->checkpoint_materialized) * m.hidden;
+        if (hipMemcpyAsync(b.hidden, kept, uint64_t(m.hidden) * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
+            return fail(GUFFIN_E_HIP, "draft_plan: restoring the frontier's state failed");
+        GUFFIN_TRY(guffin_hip_group_sums(s, b.hidden, b.hidden_sums, 1, m.hidden));
+        p->last_rows = 1;
+        p->hidden_valid = 1;
+    } else if (p->checkpoint_hidden_valid) {
+        GUFFIN_TRY(copy_frontier(s, m, b, false));
+        p->last_rows = p->checkpoint_last_rows;
+        p->hidden_valid = 1;
+    }
+    return GUFFIN_OK;
+}
+
+// Enqueues `body` (up to `rows` passes from the materialized frontier on, with the laws between them), waits once and looks at
+// the status word.  Two things can make a batch run again, from the ring rows and the final state it began with:
+//   - the resident pass gave up a wait (a device shared with other work): its rows, and whatever else it raised in the status
+//     word, are not to be trusted; the resident form is switched off for the process and the batch runs one launch per operator;
+//   - a law's support did not fit the compact form (status bit 32): body(true) runs the laws with the full-vocabulary kernels
+//     behind the compact one, which otherwise are fourteen launches per proposal that find nothing to do.
+// The ring rows a batch overwrites go to the backup arena first, inside a transaction (where they may already be) and, for a
+// batch that may have to run again, outside one.  poisoned: the plan after an error, as for every pass that fails.
+template <typename Body>
+int run_batch(hipStream_t s, guffin_draft_plan* p, const Buffers& b, uint32_t rows, const char* what, Body body) {
+    const guffin_model_desc& m = *p->model;
+    const uint32_t first = p->materialized, end = first + rows;
+    const bool watched = resident_chosen(m, 1) && g_forward_mode == 0;
+    if (p->transaction_active) {
+        if (end > p->backup_end) {   // rows below backup_end already hold the originals
+            if (int rc = move_rows(s, p, b, std::max(first, p->backup_end), end, true)) { p->poisoned = 1; return rc; }
+            p->backup_end = end;
+        }
+    } else if (watched) {
+        if (int rc = move_rows(s, p, b, first, end, true)) { p->poisoned = 1; return rc; }
+    }
+    constexpr uint32_t kOverflow = 32u;   // the compact law's support overflow
+    bool full_laws = false, given_up = false;
+    for (;;) {
+        if (int rc = body(full_laws)) { p->poisoned = 1; return rc; }
+        uint32_t status = 0;
+        if (read_status(s, b, &status)) return poison(p, GUFFIN_E_HIP, what);
+        if (status == 0) return GUFFIN_OK;
+        const bool again_plain = watched && !given_up && (status & GUFFIN_STATUS_SYNC) != 0;
+        const bool again_full = !again_plain && p->transaction_active && !full_laws && (status & kOverflow) != 0;
+        if (!again_plain && !again_full) return poison(p, GUFFIN_E_NUMERIC, what);
+        if (again_plain) { resident_note_status(status); given_up = true; }
+        full_laws |= again_full;
+        if (hipMemsetAsync(b.status, 0, 4, s) != hipSuccess) return poison(p, GUFFIN_E_HIP, what);
+        if (int rc = move_rows(s, p, b, first, end, false)) { p->poisoned = 1; return rc; }
+        p->materialized = first;
+        p->hidden_valid = p->logits_valid = 0;
+        if (p->transaction_active)
+            if (int rc = restore_frontier(s, p, b, first)) { p->poisoned = 1; return rc; }
+    }
 }
 
 // host tokens through the blocks one row per pass, a pending token first: a token's rows and logits then do
 // not depend on how the caller grouped its appends (a two-row pass sums attention partitions and norms in
 // another order than two one-row passes), which is what lets a commit be compared with a replay bit for bit
-int ingest(hipStream_t s, guffin_draft_plan* p, const Buffers& b, const uint32_t* tokens, uint32_t count) {
+int ingest(hipStream_t s, guffin_draft_plan* p, const Buffers& b, const uint32_t* tokens, uint32_t count, const char* what) {
     std::vector<uint32_t> input;
     if (p->has_pending) input.push_back(p->pending_token);
     input.insert(input.end(), tokens, tokens + count);
-    for (size_t i = 0; i < input.size(); ++i) {
-        if (hipMemcpyWithStream(b.tokens, input.data() + i, 4, hipMemcpyHostToDevice, s) != hipSuccess)
+    for (uint32_t i0 = 0; i0 < input.size(); i0 += kBatch) {
+        const uint32_t n = std::min(kBatch, static_cast<uint32_t>(input.size()) - i0);
+        if (hipMemcpyWithStream(b.staging->tokens, input.data() + i0, n * 4, hipMemcpyHostToDevice, s) != hipSuccess)
             return poison(p, GUFFIN_E_HIP, "draft_plan: token upload failed");
-        if (int rc = forward(s, p, b, 1)) { p->poisoned = 1; return rc; }
+        GUFFIN_TRY(run_batch(s, p, b, n, what, [&](bool) {
+            for (uint32_t i = 0; i < n; ++i) GUFFIN_TRY(forward(s, p, b, b.staging->tokens + i));
+            return int(GUFFIN_OK);
+        }));
     }
     p->has_pending = 0;
     p->position = p->materialized;
@@ -279,16 +322,6 @@ extern "C" int guffin_hip_draft_plan_reset(void* stream, guffin_draft_plan* plan
     return GUFFIN_OK;
 }
 
-// the output rows of the pass at the frontier, kept across a transaction so that an abort leaves the plan able to
-// draft from (or read the logits of) the prefix it returns to
-static int copy_frontier(hipStream_t s, const guffin_model_desc& m, const Buffers& b, bool save) {
-    const size_t hidden_bytes = 2 * size_t(m.hidden) * 4, sums_bytes = guffin_hip_receipt_bytes(2, m.hidden);
-    if (hipMemcpyAsync(save ? b.hidden_saved : b.hidden, save ? b.hidden : b.hidden_saved, hidden_bytes, hipMemcpyDeviceToDevice, s) != hipSuccess
-        || hipMemcpyAsync(save ? b.sums_saved : b.hidden_sums, save ? b.hidden_sums : b.sums_saved, sums_bytes, hipMemcpyDeviceToDevice, s) != hipSuccess)
-        return fail(GUFFIN_E_HIP, "draft_plan: copying the frontier rows failed");
-    return GUFFIN_OK;
-}
-
 extern "C" int guffin_hip_draft_plan_begin_transaction(void* stream, guffin_draft_plan* plan) {
     GUFFIN_TRY(usable(plan, "draft_plan_begin_transaction: null pointer"));
     if (plan->transaction_active) return fail(GUFFIN_E_STATE, "draft_plan_begin_transaction: a transaction is already open");
@@ -343,24 +376,10 @@ extern "C" int guffin_hip_draft_plan_truncate(void* stream, guffin_draft_plan* p
         const Buffers b = carve(plan);
         hipStream_t s = as_stream(stream);
         if (int rc = move_rows(s, plan, b, position, plan->backup_end, false)) { plan->poisoned = 1; return rc; }
-        GUFFIN_TRY(finish(s, plan, b, "draft_plan_truncate: restoring the ring rows failed"));
         plan->backup_end = std::min(plan->backup_end, position);
         plan->materialized = position;
-        plan->hidden_valid = plan->logits_valid = 0;
         // the frontier's final state: a row this transaction ran, or the one the transaction began on
-        const guffin_model_desc& m = *plan->model;
-        if (position > plan->checkpoint_materialized) {
-            const float* kept = b.txn_hidden + uint64_t(position - 1 - plan->checkpoint_materialized) * m.hidden;
-            if (hipMemcpyAsync(b.hidden, kept, uint64_t(m.hidden) * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
-                return poison(plan, GUFFIN_E_HIP, "draft_plan_truncate: restoring the frontier's state failed");
-            if (int rc = guffin_hip_group_sums(s, b.hidden, b.hidden_sums, 1, m.hidden)) { plan->poisoned = 1; return rc; }
-            plan->last_rows = 1;
-            plan->hidden_valid = 1;
-        } else if (plan->checkpoint_hidden_valid) {
-            if (int rc = copy_frontier(s, m, b, false)) { plan->poisoned = 1; return rc; }
-            plan->last_rows = plan->checkpoint_last_rows;
-            plan->hidden_valid = 1;
-        }
+        if (int rc = restore_frontier(s, plan, b, position)) { plan->poisoned = 1; return rc; }
         GUFFIN_TRY(finish(s, plan, b, "draft_plan_truncate: restoring the frontier's state failed"));
     }
     plan->has_pending = 0;    // position <= materialized now: whatever was pending lay beyond it
@@ -388,8 +407,7 @@ extern "C" int guffin_hip_draft_plan_append(void* stream, guffin_draft_plan* pla
     GUFFIN_TRY(capacity_check(plan, count + (plan->has_pending ? 1u : 0u), "draft_plan_append: the context is full"));
     const Buffers b = carve(plan);
     hipStream_t s = as_stream(stream);
-    GUFFIN_TRY(ingest(s, plan, b, tokens, count));
-    return finish(s, plan, b, "draft_plan_append: the pass raised the device status");
+    return ingest(s, plan, b, tokens, count, "draft_plan_append: the pass raised the device status");
 }
 
 // A saved emission of this drafter put back after its prefix was replayed: known, but not run (:75-77).
@@ -429,38 +447,43 @@ extern "C" int guffin_hip_draft_plan_propose(void* stream, guffin_draft_plan* pl
     const guffin_model_desc& m = *plan->model;
     const Buffers b = carve(plan);
     hipStream_t s = as_stream(stream);
-    if (plan->has_pending) GUFFIN_TRY(ingest(s, plan, b, nullptr, 0));
-    std::vector<Draws> draws(horizon);
-    for (uint32_t i = 0; i < horizon; ++i) draws[i] = {words[i], 0, 0.5, 0.5, 0.5};
-    if (hipMemcpyWithStream(b.draws, draws.data(), horizon * sizeof(Draws), hipMemcpyHostToDevice, s) != hipSuccess)
+    Staging up {};
+    const bool pending = plan->has_pending != 0;
+    for (uint32_t i = 0; i < horizon; ++i) up.draws[i] = {words[i], 0, 0.5, 0.5, 0.5};
+    if (pending) up.tokens[0] = plan->pending_token;
+    for (uint32_t i = 0; i < history_count; ++i) up.chain[kHistory - history_count + i] = history[i];
+    if (hipMemcpyWithStream(b.staging, &up, sizeof(up), hipMemcpyHostToDevice, s) != hipSuccess)
         return poison(plan, GUFFIN_E_HIP, "draft_plan_propose: upload failed");
-    std::vector<uint32_t> window(history, history + history_count);
     const bool penalise = opt.repetition_penalty != 1.0f;
     Options law_options = opt;
     law_options.repetition_penalty = 1.0f;   // applied to the scores below, as gd_process does before the law
-    for (uint32_t i = 0; i < horizon; ++i) {
-        if (int rc = ensure_logits(s, plan, b)) { plan->poisoned = 1; return rc; }
-        const float* logits = b.logits + uint64_t(plan->last_rows - 1) * m.vocab;
-        if (penalise && !window.empty()) {
-            if (hipMemcpyWithStream(b.history, window.data(), window.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess)
-                return poison(plan, GUFFIN_E_HIP, "draft_plan_propose: upload failed");
-            if (int rc = guffin_hip_draft_process(s, logits, m.vocab, b.history, static_cast<uint32_t>(window.size()),
-                                                  opt.repetition_penalty, b.scores)) { plan->poisoned = 1; return rc; }
-            logits = b.scores;
+    // what guffin_hip_draft_law takes; options out of range are guffin_hip_draft_law_any's to refuse
+    const bool compact = opt.temperature > 0.f && std::isfinite(opt.temperature) && opt.top_k >= 1 && opt.top_k <= 64 && opt.top_p > 0.f
+                      && opt.top_p <= 1.f && opt.min_p >= 0.f && opt.min_p <= 1.f;
+    GUFFIN_TRY(run_batch(s, plan, b, horizon - 1 + (pending ? 1u : 0u), "draft_plan_propose: a pass or a law raised the device status", [&](bool full_laws) {
+        if (pending) GUFFIN_TRY(forward(s, plan, b, b.staging->tokens));
+        for (uint32_t i = 0; i < horizon; ++i) {
+            GUFFIN_TRY(ensure_logits(s, plan, b));
+            const float* logits = b.logits + uint64_t(plan->last_rows - 1) * m.vocab;
+            const uint32_t window = std::min(kHistory, history_count + i);
+            uint32_t* token = b.staging->chain + kHistory + i;
+            if (penalise && window != 0) {
+                GUFFIN_TRY(guffin_hip_draft_process(s, logits, m.vocab, token - window, window, opt.repetition_penalty, b.scores));
+                logits = b.scores;
+            }
+            if (compact && !full_laws)
+                GUFFIN_TRY(guffin_hip_draft_law(s, logits, m.vocab, &law_options, 0, 0, b.staging->draws + i, b.law_ws, b.law, token, b.status));
+            else
+                GUFFIN_TRY(guffin_hip_draft_law_any(s, logits, m.vocab, &law_options, 0, 0, b.staging->draws + i, b.law_ws, b.law, b.cdf,
+                                                    token, b.status));
+            if (i + 1 < horizon) GUFFIN_TRY(forward(s, plan, b, token));
         }
-        if (int rc = guffin_hip_draft_law_any(s, logits, m.vocab, &law_options, 0, 0, b.draws + i, b.law_ws, b.law, b.cdf,
-                                              b.tokens, b.status)) { plan->poisoned = 1; return rc; }
-        GUFFIN_TRY(finish(s, plan, b, "draft_plan_propose: the law raised the device status"));
-        if (hipMemcpy(&drafted[i], b.tokens, 4, hipMemcpyDeviceToHost) != hipSuccess)
-            return poison(plan, GUFFIN_E_HIP, "draft_plan_propose: read-back failed");
-        if (window.size() == 64) window.erase(window.begin());
-        window.push_back(drafted[i]);
-        if (i + 1 < horizon) {           // b.tokens[0] holds the drafted token: run it
-            if (int rc = forward(s, plan, b, 1)) { plan->poisoned = 1; return rc; }
-            plan->position = plan->materialized;
-        }
-    }
-    GUFFIN_TRY(finish(s, plan, b, "draft_plan_propose: the pass raised the device status"));
+        return int(GUFFIN_OK);
+    }));
+    plan->has_pending = 0;
+    plan->position = plan->materialized;
+    if (hipMemcpyWithStream(drafted, b.staging->chain + kHistory, horizon * 4, hipMemcpyDeviceToHost, s) != hipSuccess)
+        return poison(plan, GUFFIN_E_HIP, "draft_plan_propose: read-back failed");
     plan->pending_token = drafted[horizon - 1];
     plan->has_pending = 1;
     plan->position = plan->materialized + 1;

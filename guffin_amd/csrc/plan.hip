@@ -292,11 +292,16 @@ int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t*
     return GUFFIN_OK;
 }
 
-// publishes the verified rows: row 0 always, row 1 if the proposal was accepted
+// publishes the verified rows: row 0 always, row 1 if the proposal was accepted; the first block's workgroups also keep the
+// row's final state where the caller asks for it
 __global__ void commit_rows_kernel(const uint16_t* priv_k, const uint16_t* priv_v, uint16_t* const* ring_k,
                                    uint16_t* const* ring_v, const uint32_t* accepted, uint32_t position, uint32_t rows,
-                                   uint32_t row_width, uint32_t mask_local, uint32_t mask_global, uint32_t global_period) {
+                                   uint32_t row_width, uint32_t mask_local, uint32_t mask_global, uint32_t global_period,
+                                   const float* hidden, float* kept, uint32_t hidden_width) {
     const uint32_t layer = blockIdx.y, row = blockIdx.z;
+    if (kept && layer == 0)
+        for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < hidden_width; c += gridDim.x * blockDim.x)
+            kept[size_t(row) * hidden_width + c] = hidden[size_t(row) * hidden_width + c];
     const uint32_t publish = accepted ? 1u + (*accepted != 0u) : rows;
     if (row >= publish || row >= rows) return;
     const bool local = layer_is_local(global_period, layer);
@@ -475,18 +480,24 @@ extern "C" int guffin_hip_forward_tree_rows(void* stream, const guffin_model_des
     return GUFFIN_OK;
 }
 
+int guffin::commit_rows_keeping(void* stream, const guffin_model_desc& m, const void* priv_k, const void* priv_v,
+                                void* const* ring_k_table, void* const* ring_v_table, const uint32_t* accepted, uint32_t position,
+                                uint32_t rows, const float* hidden, float* kept) {
+    const uint32_t KW = m.kv_heads * m.head_dim;
+    launch(commit_rows_kernel, dim3((KW + 255) / 256, m.layer_count, rows), dim3(256), 0,
+                       as_stream(stream), static_cast<const uint16_t*>(priv_k), static_cast<const uint16_t*>(priv_v),
+                       reinterpret_cast<uint16_t* const*>(ring_k_table), reinterpret_cast<uint16_t* const*>(ring_v_table),
+                       accepted, position, rows, KW, m.ring_local - 1, m.ring_global - 1, m.global_period, hidden, kept, m.hidden);
+    return check_launch("commit_rows");
+}
+
 extern "C" int guffin_hip_commit_rows(void* stream, const guffin_model_desc* model, const void* priv_k,
                                       const void* priv_v, void* const* ring_k_table, void* const* ring_v_table,
                                       const uint32_t* accepted, uint32_t position, uint32_t rows) {
     GUFFIN_TRY(validate_model(model));
     if (!priv_k || !priv_v || !ring_k_table || !ring_v_table) return fail(GUFFIN_E_ARG, "commit_rows: null pointer");
     if (rows == 0 || rows > 2) return fail(GUFFIN_E_SHAPE, "commit_rows: rows must be 1 or 2");
-    const uint32_t KW = model->kv_heads * model->head_dim;
-    launch(commit_rows_kernel, dim3((KW + 255) / 256, model->layer_count, rows), dim3(256), 0,
-                       as_stream(stream), static_cast<const uint16_t*>(priv_k), static_cast<const uint16_t*>(priv_v),
-                       reinterpret_cast<uint16_t* const*>(ring_k_table), reinterpret_cast<uint16_t* const*>(ring_v_table),
-                       accepted, position, rows, KW, model->ring_local - 1, model->ring_global - 1, model->global_period);
-    return check_launch("commit_rows");
+    return commit_rows_keeping(stream, *model, priv_k, priv_v, ring_k_table, ring_v_table, accepted, position, rows, nullptr, nullptr);
 }
 
 // ---- prefill: a run of rows through every block --------------------------------------------

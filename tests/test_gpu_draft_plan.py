@@ -378,3 +378,37 @@ def test_the_transaction_capacity_is_the_callers(hip, scaled_world):
     plan.abort_transaction()
     assert plan.position == 70 and same_caches(snapshot(plan, shape), before)
     assert np.array_equal(plan.read_logits().view(np.uint32), logits.view(np.uint32))
+
+
+@pytest.mark.parametrize("penalty,history_length", [(1.0, 0), (1.3, 62)])
+@pytest.mark.parametrize("kind", ["scaled", "reference"])
+def test_a_chain_equals_its_laws_one_by_one(hip, kind, penalty, history_length):
+    """A chain's passes and laws are enqueued together; draft i is what the law of the logits after draft i-1 selects when it is
+    asked for alone.  The reference fixture's logits tie thousands of tokens, so its compact laws overflow and the chain runs
+    again with the full-vocabulary law; the 62-token history slides out of the sampler's window of 64 inside the chain."""
+    import torch
+    from guffin_amd import model
+    world = world_of(kind)
+    device = model.DeviceModel.from_host(world.host)
+    plan = model.DraftPlan(device)
+    plan.append(world.stream(10))
+    before = snapshot(plan, world.shape)
+    history = [int(t) for t in world.stream(history_length)]
+    words = [int(w) for w in np.random.default_rng(8).integers(0, 2 ** 32, 5)]
+    plan.begin_transaction()
+    drafted = plan.propose(words, hip.SamplerOptions(0.9, 40, 0.95, 0.02, penalty), history)
+    assert plan.materialized_position == 14 and plan.position == 15
+    plan.abort_transaction()
+    assert same_caches(snapshot(plan, world.shape), before)
+    window = list(history)
+    plain = hip.SamplerOptions(0.9, 40, 0.95, 0.02, 1.0)
+    for i, word in enumerate(words):
+        logits = torch.from_numpy(plan.read_logits()).cuda()
+        if penalty != 1.0 and window:
+            logits = hip.draft_process(logits, torch.tensor(window[-64:], dtype=torch.int32, device="cuda"), penalty)
+        draws = np.zeros(1, dtype=[("word", "<u4"), ("pad", "<u4"), ("u", "<f8", 3)])
+        draws["word"], draws["u"] = word, 0.5
+        _, _, proposal, status = hip.draft_law_any(logits, plain, draws=torch.from_numpy(draws.view(np.uint8)).cuda())
+        assert int(status) == 0 and drafted[i] == int(proposal.cpu().numpy().view(np.uint32)[0]), (kind, i)
+        window.append(drafted[i])
+        plan.append([drafted[i]])
