@@ -352,8 +352,9 @@ __global__ void __launch_bounds__(256)
 geglu_kernel(const float* __restrict__ gate, const float* __restrict__ up, uint32_t planes, size_t plane_stride,
              float* __restrict__ out, float* __restrict__ out_sums, uint32_t width) {
     extern __shared__ float lds[];  // [chunk] when sums are requested
-    // grid: (chunks_per_row, rows); a chunk is a multiple of 32 columns
-    const uint32_t chunk = (width + gridDim.x - 1) / gridDim.x;
+    // grid: (chunks_per_row, rows); with a receipt a chunk is a multiple of 32 columns
+    uint32_t chunk = (width + gridDim.x - 1) / gridDim.x;
+    if (out_sums) chunk = (chunk + 31u) & ~31u;
     const uint32_t c0 = blockIdx.x * chunk, c1 = c0 + chunk < width ? c0 + chunk : width;
     const size_t rbase = size_t(blockIdx.y) * width;
     for (uint32_t c = c0 + threadIdx.x; c < c1; c += blockDim.x) {
