@@ -32,7 +32,7 @@ namespace {
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
-constexpr int kMaxRows = 2;
+constexpr int kMaxRows = 4;   // query rows of a launch: 2 through the entry points, 4 for the fused form of a block graph pass
 
 struct AttnArgs {
     const float* q;              // [rows][q_heads][hd]
@@ -150,8 +150,8 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
                  "s"(a.planes), "s"(a.q_stride), "s"(a.k_stride), "s"(a.v_stride), "s"(a.q_norm), "s"(a.k_norm), "s"(a.rope),
                  "s"(a.priv_k_out), "s"(a.priv_v_out));
     asm volatile("" :: "s"(a.eps), "s"(a.status), "s"(a.inline_schedule), "s"(a.sched[0][0]), "s"(a.sched[0][1]),
-                 "s"(a.sched[0][2]), "s"(a.sched[0][3]), "s"(a.sched[kMaxRows - 1][0]), "s"(a.sched[kMaxRows - 1][1]),
-                 "s"(a.sched[kMaxRows - 1][2]), "s"(a.sched[kMaxRows - 1][3]), "s"(a.amask[0]), "s"(a.amask[kMaxRows - 1]));
+                 "s"(a.sched[0][2]), "s"(a.sched[0][3]), "s"(a.sched[ROWS - 1][0]), "s"(a.sched[ROWS - 1][1]),
+                 "s"(a.sched[ROWS - 1][2]), "s"(a.sched[ROWS - 1][3]), "s"(a.amask[0]), "s"(a.amask[ROWS - 1]));
     const uint32_t row_stride = a.kv_heads * HD;  // in halves
 
     // fused: the query rows of this wave (w, w+kAW, ..) are requested first; their addresses need
@@ -245,17 +245,23 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
     };
 
     if constexpr (FUSED) {
-        // wave w prepares query rows w, w+kAW, ..; the last 2 ROWS waves prepare the private rows' key / value
-        // (row i/2, key for even i) when this partition holds it; every load is issued before any arithmetic
-        HeadRow kvr;
-        const uint32_t ki = wv - (kAW - 2 * ROWS);   // wraps for the waves below: pr >= ROWS then
-        const uint32_t pr = ki >> 1, pt = n_ring + pr;
-        const bool is_key = (ki & 1u) == 0;
-        const bool mine = wv >= uint32_t(kAW - 2 * ROWS) && pr < ROWS && pr < a.private_rows && pt >= t0 && pt < t1;
-        const size_t kv_off = (size_t(pr) * a.kv_heads + kvh) * HD;
-        if (mine)
-            load_head_row(kvr, (is_key ? a.k_raw : a.v_raw) + kv_off, a.planes, is_key ? a.k_stride : a.v_stride,
-                          is_key ? a.k_norm : nullptr, is_key ? a.rope + size_t(pr) * (HD / 2) : nullptr, lane);
+        // wave w prepares query rows w, w+kAW, ..; the last 2 ROWS waves (with more than that many rows, every wave two
+        // of them) prepare the private rows' key / value (row i/2, key for even i) when this partition holds it; every
+        // load is issued before any arithmetic
+        constexpr int KI = (2 * ROWS + kAW - 1) / kAW;
+        constexpr uint32_t kFirst = KI == 1 ? kAW - 2 * ROWS : 0;
+        HeadRow kvr[KI];
+        bool mine[KI];
+#pragma unroll
+        for (int i = 0; i < KI; ++i) {
+            const uint32_t ki = wv - kFirst + kAW * i;   // wraps for the waves below: pr >= ROWS then
+            const uint32_t pr = ki >> 1, pt = n_ring + pr;
+            const bool is_key = (ki & 1u) == 0;
+            mine[i] = wv >= kFirst && pr < ROWS && pr < a.private_rows && pt >= t0 && pt < t1;
+            if (mine[i])
+                load_head_row(kvr[i], (is_key ? a.k_raw : a.v_raw) + (size_t(pr) * a.kv_heads + kvh) * HD, a.planes, is_key ? a.k_stride : a.v_stride,
+                              is_key ? a.k_norm : nullptr, is_key ? a.rope + size_t(pr) * (HD / 2) : nullptr, lane);
+        }
 #pragma unroll
         for (int i = 0; i < QI; ++i) {
             const uint32_t item = wv + kAW * i;
@@ -265,12 +271,17 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
                 for (int c = 0; c < 4; ++c) q_s[item * HD + lane + 64 * c] = qr[i].v[c];
             }
         }
-        if (mine) {
-            finish_head_row(kvr, is_key && a.k_norm != nullptr, is_key, a.eps);
+#pragma unroll
+        for (int i = 0; i < KI; ++i) {
+            if (!mine[i]) continue;
+            const uint32_t ki = wv - kFirst + kAW * i, pr = ki >> 1;
+            const bool is_key = (ki & 1u) == 0;
+            const size_t kv_off = (size_t(pr) * a.kv_heads + kvh) * HD;
+            finish_head_row(kvr[i], is_key && a.k_norm != nullptr, is_key, a.eps);
             bool bad = false;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                const _Float16 hv = static_cast<_Float16>(kvr.v[c]);  // round-to-nearest-even, after rotation
+                const _Float16 hv = static_cast<_Float16>(kvr[i].v[c]);  // round-to-nearest-even, after rotation
                 bad |= !isfinite(static_cast<float>(hv));
                 const uint16_t bits = __builtin_bit_cast(uint16_t, hv);
                 (is_key ? k_s : v_s)[pr][lane + 64 * c] = bits;
@@ -482,9 +493,9 @@ int launch_partial(hipStream_t s, const AttnArgs& a) {
     constexpr int kAW = attention_waves(NQ);
     const bool fused = a.q_raw != nullptr;
     const size_t lds = (size_t(NQ) * a.span + size_t(kAW) * NQ * 256 + (fused ? size_t(NQ) * 256 : 0)) * sizeof(float);
-    if (fused)
+    if (fused || ROWS > 2)
         launch((attn_partial_kernel<ROWS, GROUP, 256, true>), dim3(a.partitions, a.kv_heads), dim3(64 * kAW), lds, s, a);
-    else
+    else if constexpr (ROWS <= 2)
         launch((attn_partial_kernel<ROWS, GROUP, 256, false>), dim3(a.partitions, a.kv_heads), dim3(64 * kAW), lds, s, a);
     return check_launch("attention_partial");
 }
@@ -537,7 +548,7 @@ int attention_decode(void* stream, const float* q, const FusedInputs* fused, con
                      float scale, uint32_t* status, const uint32_t* host_schedule = nullptr, const uint32_t* host_amask = nullptr) {
     if ((!q && !fused) || !ring_k || !ring_v || !priv_k || !priv_v || !schedule || !ancestors || !out || !partial_out || !partial_ml)
         return fail(GUFFIN_E_ARG, "attention_decode: null pointer");
-    if (rows == 0 || rows > kMaxRows || private_rows > 32) return fail(GUFFIN_E_SHAPE, "attention_decode: rows must be 1 or 2, private rows <= 32");
+    if (rows == 0 || rows > (fused && host_schedule ? uint32_t(kMaxRows) : 2u) || private_rows > 32) return fail(GUFFIN_E_SHAPE, "attention_decode: rows must be 1 or 2, private rows <= 32");
     if (head_dim != 256) return fail(GUFFIN_E_SHAPE, "attention_decode: head_dim must be 256");
     if (reinterpret_cast<uintptr_t>(out_sums) & 255u) return fail(GUFFIN_E_ALIGN, "attention_decode: the receipt must be 256-byte aligned");
     if (kv_heads == 0 || q_heads % kv_heads != 0) return fail(GUFFIN_E_SHAPE, "attention_decode: q_heads must be a multiple of kv_heads");
@@ -586,6 +597,10 @@ int attention_decode(void* stream, const float* q, const FusedInputs* fused, con
         case 12: rc = launch_partial<2, 1>(s, a); break;
         case 21: rc = launch_partial<1, 2>(s, a); break;
         case 22: rc = launch_partial<2, 2>(s, a); break;
+        case 13: rc = launch_partial<3, 1>(s, a); break;
+        case 14: rc = launch_partial<4, 1>(s, a); break;
+        case 23: rc = launch_partial<3, 2>(s, a); break;
+        case 24: rc = launch_partial<4, 2>(s, a); break;
         case 41: rc = launch_partial<1, 4>(s, a); break;
         case 42: rc = launch_partial<2, 4>(s, a); break;
         default: return fail(GUFFIN_E_SHAPE, "attention_decode: q_heads / kv_heads must be 1, 2 or 4");

@@ -45,6 +45,19 @@ int resident_launch(hipStream_t stream, const guffin_model_desc& m, uint32_t row
                     const void* u_receipt_in, float* x_out, float* u_out, void* u_receipt_out, uint32_t max_ring_tokens,
                     uint32_t* status);
 
+// ---- streaming products of 3 and 4 rows (gemv_wide.hip) -------------------------------------------------------
+constexpr uint32_t kWideRows = 4;
+// The work split of a streaming product over `tiles` column tiles of `nblk` blocks (gemv_packed.hip): blocks per wave, waves per
+// workgroup (at most max_w) and planes left to the consumer; waves_per_cu waves are assumed to fit a CU.
+struct GemvSplit { uint32_t bps, W, planes; };
+GemvSplit gemv_split(uint32_t nblk, uint32_t tiles, uint32_t max_w, uint32_t waves_per_cu);
+uint32_t gemv_wide_planes(uint32_t count, const int* dtypes, const uint32_t* N, uint32_t K);
+// partials[i]: [planes][rows][N[i]]; y (one matrix): the planes' sum [rows][N]
+int gemv_wide(hipStream_t s, uint32_t count, const int* dtypes, const void* const* tiles, const uint32_t* N, float* const* partials,
+              const float* xsums, float* y, uint32_t rows, uint32_t K);
+int gateup_wide(hipStream_t s, int dtype, const void* gate_tiles, const void* up_tiles, const float* xsums, float* h, float* h_sums,
+                uint32_t rows, uint32_t K, uint32_t F);
+
 // ---- K/V rows of every block of a model between its rings and a flat block of rows (prefill.hip) ---------------
 // flat_k / flat_v: [layer][flat_rows][kv width], position p in row p & (flat_rows - 1), flat_rows a power of two.  Save and
 // Restore copy positions [first, first + count); Publish saves them and then puts row path[i] of the private rows
@@ -54,6 +67,13 @@ constexpr uint32_t kMovePath = 8;   // rows a Publish may take
 int kv_move_rows(hipStream_t s, const guffin_model_desc& m, KvMove move, void* flat_k, void* flat_v, uint32_t flat_rows, uint32_t first,
                  uint32_t count, const void* priv_k = nullptr, const void* priv_v = nullptr, uint32_t priv_rows = 0,
                  const uint32_t* path = nullptr);
+
+// ---- a whole verify tree of up to 4 rows in one pass (plan.hip) -----------------------------------------------------
+bool tree_pass_fits(const guffin_model_desc& m);
+uint64_t tree_pass_bytes(const guffin_model_desc& m, uint32_t position);   // scratch of a tree at that position
+int forward_tree_pass(hipStream_t stream, const guffin_model_desc& m, const uint32_t* tokens, uint32_t rows, uint32_t position,
+                      const uint32_t* depths, const uint32_t* parents, void* scratch, uint64_t scratch_bytes, void* priv_k, void* priv_v,
+                      float* out_hidden, float* out_hidden_sums, uint32_t* status);
 
 // guffin_hip_commit_rows of every row, with the rows' final states kept: kept[row] = hidden[row] unless kept is null (plan.hip)
 int commit_rows_keeping(void* stream, const guffin_model_desc& m, const void* priv_k, const void* priv_v, void* const* ring_k_table,

@@ -315,7 +315,7 @@ float* g_scratch_ptr[kMaxDevices] = {};
 // Work split of a launch over `tiles` column tiles of `nblk` blocks each: blocks per wave so
 // that the chip holds about four waves per SIMD, waves per workgroup (k-slices reduced in LDS,
 // at most max_w) and planes (k-slices left to the consumer), preferring one workgroup per CU.
-struct Split { uint32_t bps, W, planes; };
+using Split = GemvSplit;
 Split choose_split(uint32_t nblk, uint32_t tiles, uint32_t max_w, uint32_t waves_per_cu = 0) {
     // a kernel capped at 8 waves per workgroup is register-bound: a CU holds 8 of its waves, not 16
     if (waves_per_cu == 0) waves_per_cu = max_w < 16 ? 8 : 16;
@@ -367,6 +367,8 @@ int launch_packed(hipStream_t s, const uint8_t* w, const float* x, const float* 
 }
 
 }  // namespace
+
+GemvSplit gemv_split(uint32_t nblk, uint32_t tiles, uint32_t max_w, uint32_t waves_per_cu) { return choose_split(nblk, tiles, max_w, waves_per_cu); }
 
 // Called by guffin_hip_init with `device` current: the split heuristics' CU count and this device's
 // address of the static scratch array.

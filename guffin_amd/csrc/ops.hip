@@ -461,7 +461,7 @@ extern "C" int guffin_hip_rms_norm(void* stream, const float* x, uint32_t planes
                                    uint32_t rows, uint32_t width, float eps, uint32_t* status) {
     if (!x || !gamma || !y) return fail(GUFFIN_E_ARG, "rms_norm: null pointer");
     if (rows == 0 || width == 0 || planes == 0) return fail(GUFFIN_E_SHAPE, "rms_norm: empty shape");
-    if (y_sums && (width % 32 != 0 || rows > 2)) return fail(GUFFIN_E_SHAPE, "rms_norm: a receipt needs width % 32 == 0 and rows <= 2");
+    if (y_sums && (width % 32 != 0 || rows > kWideRows)) return fail(GUFFIN_E_SHAPE, "rms_norm: a receipt needs width % 32 == 0 and rows <= 4");
     if (reinterpret_cast<uintptr_t>(y_sums) & 255u) return fail(GUFFIN_E_ALIGN, "rms_norm: the receipt must be 256-byte aligned");
     if (!(eps > 0.f)) return fail(GUFFIN_E_ARG, "rms_norm: epsilon must be positive");
     if (!aligned4(x) || !aligned4(y) || !aligned4(gamma)) return fail(GUFFIN_E_ALIGN, "rms_norm: fp32 pointers must be 4-byte aligned");
@@ -479,7 +479,7 @@ extern "C" int guffin_hip_rms_norm_add_norm(void* stream, const float* x, uint32
     if (!x || !gamma_post || !residual || !out_residual || !gamma_next || !out_norm)
         return fail(GUFFIN_E_ARG, "rms_norm_add_norm: null pointer");
     if (rows == 0 || width == 0 || planes == 0) return fail(GUFFIN_E_SHAPE, "rms_norm_add_norm: empty shape");
-    if (out_sums && (width % 32 != 0 || rows > 2)) return fail(GUFFIN_E_SHAPE, "rms_norm_add_norm: a receipt needs width % 32 == 0 and rows <= 2");
+    if (out_sums && (width % 32 != 0 || rows > kWideRows)) return fail(GUFFIN_E_SHAPE, "rms_norm_add_norm: a receipt needs width % 32 == 0 and rows <= 4");
     if (reinterpret_cast<uintptr_t>(out_sums) & 255u) return fail(GUFFIN_E_ALIGN, "rms_norm_add_norm: the receipt must be 256-byte aligned");
     if (!(eps > 0.f)) return fail(GUFFIN_E_ARG, "rms_norm_add_norm: epsilon must be positive");
     auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
@@ -580,7 +580,7 @@ extern "C" int guffin_hip_geglu(void* stream, const float* gate, const float* up
                                 float* out, float* out_sums, uint32_t rows, uint32_t width) {
     if (!gate || !up || !out) return fail(GUFFIN_E_ARG, "geglu: null pointer");
     if (rows == 0 || width == 0 || planes == 0) return fail(GUFFIN_E_SHAPE, "geglu: empty shape");
-    if (out_sums && (width % 32 != 0 || rows > 2)) return fail(GUFFIN_E_SHAPE, "geglu: a receipt needs width % 32 == 0 and rows <= 2");
+    if (out_sums && (width % 32 != 0 || rows > kWideRows)) return fail(GUFFIN_E_SHAPE, "geglu: a receipt needs width % 32 == 0 and rows <= 4");
     if (reinterpret_cast<uintptr_t>(out_sums) & 255u) return fail(GUFFIN_E_ALIGN, "geglu: the receipt must be 256-byte aligned");
     // chunks of 512 columns (a multiple of 32) per workgroup
     const uint32_t chunk = 512, chunks = (width + chunk - 1) / chunk;

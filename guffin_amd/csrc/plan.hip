@@ -38,7 +38,7 @@ struct Arena {
     }
 };
 
-// private rows a verify tree may hold (rows of one pass are at most 2; a tree takes several passes)
+// private rows a verify tree may hold
 constexpr uint32_t kMaxTreeSlots = 8;
 
 struct Scratch {
@@ -53,19 +53,31 @@ struct Scratch {
     uint64_t bytes;
 };
 
-uint32_t slices(int dtype, uint32_t K, uint32_t N) { return guffin_hip_gemv_packed_slices(dtype, K, N); }
+// Planes a projection of `rows` rows leaves: up to two rows run the kernels of gemv_packed.hip, three and four those of
+// gemv_wide.hip, which fetch and unpack the weights once for all of them.
+uint32_t slices(int dtype, uint32_t K, uint32_t N, uint32_t rows) {
+    return rows > 2 ? gemv_wide_planes(1, &dtype, &N, K) : guffin_hip_gemv_packed_slices(dtype, K, N);
+}
+uint32_t slices(uint32_t count, const int* dtypes, const uint32_t* N, uint32_t K, uint32_t rows) {
+    return rows > 2 ? gemv_wide_planes(count, dtypes, N, K) : guffin_hip_gemv_packed_multi_slices(count, dtypes, N, K);
+}
+int project(void* st, uint32_t count, const int* dtypes, const void* const* tiles, const uint32_t* N, float* const* parts, const float* x,
+            const float* xs, uint32_t rows, uint32_t K) {
+    if (rows > 2) return gemv_wide(as_stream(st), count, dtypes, tiles, N, parts, xs, nullptr, rows, K);
+    return guffin_hip_gemv_packed_multi(st, count, dtypes, tiles, N, parts, x, xs, rows, K);
+}
 // floats in the activation receipt of `rows` rows of `width`
 uint64_t receipt_floats(uint32_t rows, uint32_t width) { return receipt_layout(rows, width).bytes / 4; }
 // floats from the start of a [rows][width] block to its receipt (256-byte aligned) and the total
 uint64_t hidden_receipt_offset(uint32_t rows, uint32_t width) { return (uint64_t(rows) * width + 63) & ~uint64_t{63}; }
 uint64_t hidden_with_receipt(uint32_t rows, uint32_t width) { return hidden_receipt_offset(rows, width) + receipt_floats(rows, width); }
-uint32_t qkv_slices(const guffin_layer_desc& L, uint32_t H, uint32_t QW, uint32_t KW) {
+uint32_t qkv_slices(const guffin_layer_desc& L, uint32_t H, uint32_t QW, uint32_t KW, uint32_t rows) {
     const uint32_t n[3] = {QW, KW, KW};
-    return guffin_hip_gemv_packed_multi_slices(3, L.dtype, n, H);
+    return slices(3, L.dtype, n, H, rows);
 }
-uint32_t ffn_slices(const guffin_layer_desc& L, uint32_t H, uint32_t F) {
+uint32_t ffn_slices(const guffin_layer_desc& L, uint32_t H, uint32_t F, uint32_t rows) {
     const uint32_t n[2] = {F, F};
-    return guffin_hip_gemv_packed_multi_slices(2, L.dtype + 4, n, H);
+    return slices(2, L.dtype + 4, n, H, rows);
 }
 
 bool is_local(const guffin_model_desc& m, uint32_t layer) { return layer_is_local(m.global_period, layer); }
@@ -96,8 +108,8 @@ Scratch layout(const guffin_model_desc& m, uint32_t rows, uint32_t position, uin
     uint64_t pa = 0, pb = 0, pc = 0;
     for (uint32_t l = 0; l < m.layer_count; ++l) {
         const guffin_layer_desc& L = m.layers[l];
-        auto need = [&](int i, uint32_t K, uint32_t N) { return uint64_t(slices(L.dtype[i], K, N)) * rows * N; };
-        const uint64_t sq = qkv_slices(L, H, QW, KW), sf = ffn_slices(L, H, F);
+        auto need = [&](int i, uint32_t K, uint32_t N) { return uint64_t(slices(L.dtype[i], K, N, rows)) * rows * N; };
+        const uint64_t sq = qkv_slices(L, H, QW, KW, rows), sf = ffn_slices(L, H, F, rows);
         pa = std::max({pa, sq * rows * QW, need(3, QW, H), sf * rows * F, need(6, F, H)});
         pb = std::max({pb, sq * rows * KW, sf * rows * F});
         pc = std::max(pc, sq * rows * KW);
@@ -146,24 +158,26 @@ void row_schedule(const guffin_model_desc& m, uint32_t layer, uint32_t position,
 }
 
 // positions, ancestors, the per-layer attention schedule of `rows` contiguous rows and the two
-// rotation tables (local and global frequency base) of the pass
+// rotation tables (local and global frequency base) of the pass.  depths: byte r is row r's distance from `position`
+// (r itself for contiguous rows; a tree's schedule travels with its launches, it asks for no layers here)
 __global__ void stage_rows_kernel(uint32_t* positions, uint32_t* ancestors, uint32_t* schedule, uint32_t rows,
-                                  uint32_t position, uint32_t layers, uint32_t window, uint32_t global_period,
+                                  uint32_t position, uint32_t depths, uint32_t layers, uint32_t window, uint32_t global_period,
                                   float2* rope_local, float2* rope_global, uint32_t rope_dim, float local_base,
                                   float global_base, float global_scale, uint32_t* sync, uint32_t sync_words) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < sync_words) sync[i] = 0u;   // barrier counters of the resident pass start at zero
     const uint32_t half = rope_dim / 2;
+    auto at = [&](uint32_t row) { return position + ((depths >> (8 * row)) & 255u); };
     if (i < rows * half) {
         float c, s;
         if (global_period > 1) {  // a model without local blocks has no local base
-            rope_sincos(position + i / half, i % half, rope_dim, local_base, 1.0f, c, s);
+            rope_sincos(at(i / half), i % half, rope_dim, local_base, 1.0f, c, s);
             rope_local[i] = make_float2(c, s);
         }
-        rope_sincos(position + i / half, i % half, rope_dim, global_base, global_scale, c, s);
+        rope_sincos(at(i / half), i % half, rope_dim, global_base, global_scale, c, s);
         rope_global[i] = make_float2(c, s);
     }
-    if (i < rows) { positions[i] = position + i; ancestors[i] = i; }
+    if (i < rows) { positions[i] = at(i); ancestors[i] = i; }
     if (i >= layers * rows) return;
     const uint32_t layer = i / rows, row = i % rows;
     uint32_t words[4];
@@ -201,44 +215,54 @@ int block_tail(void* st, const guffin_model_desc& m, uint32_t l, const Scratch& 
                float* out_hidden_sums, uint32_t* status) {
     const guffin_layer_desc& L = m.layers[l];
     const uint32_t H = m.hidden, F = m.ffn, QW = m.q_heads * m.head_dim;
-    GUFFIN_TRY(guffin_hip_gemv_packed(st, L.dtype[3], L.tiles[3], s.a, s.as, s.part_a, nullptr, rows, QW, H));
+    GUFFIN_TRY(project(st, 1, L.dtype + 3, L.tiles + 3, &H, &s.part_a, s.a, s.as, rows, QW));
     // x1 = x + rms(o, post_attention_norm); u = rms(x1, ffn_norm)
-    GUFFIN_TRY(guffin_hip_rms_norm_add_norm(st, s.part_a, slices(L.dtype[3], QW, H), uint64_t(rows) * H, L.norm[3],
+    GUFFIN_TRY(guffin_hip_rms_norm_add_norm(st, s.part_a, slices(L.dtype[3], QW, H, rows), uint64_t(rows) * H, L.norm[3],
                                             s.x, s.x1, L.norm[4], s.u, s.us, rows, H, m.eps, status));
     if (L.dtype[4] == L.dtype[5] && L.dtype[4] != GUFFIN_Q6_K) {
-        GUFFIN_TRY(guffin_hip_gateup_geglu(st, L.dtype[4], L.tiles[4], L.tiles[5], s.u, s.us, s.h, s.hs, rows, H, F));
+        if (rows > 2) GUFFIN_TRY(gateup_wide(as_stream(st), L.dtype[4], L.tiles[4], L.tiles[5], s.us, s.h, s.hs, rows, H, F));
+        else GUFFIN_TRY(guffin_hip_gateup_geglu(st, L.dtype[4], L.tiles[4], L.tiles[5], s.u, s.us, s.h, s.hs, rows, H, F));
     } else {
         const int dt[2] = {L.dtype[4], L.dtype[5]};
         const void* tl[2] = {L.tiles[4], L.tiles[5]};
         const uint32_t n[2] = {F, F};
         float* parts[2] = {s.part_a, s.part_b};
-        GUFFIN_TRY(guffin_hip_gemv_packed_multi(st, 2, dt, tl, n, parts, s.u, s.us, rows, H));
-        GUFFIN_TRY(guffin_hip_geglu(st, s.part_a, s.part_b, ffn_slices(L, H, F), uint64_t(rows) * F, s.h, s.hs, rows, F));
+        GUFFIN_TRY(project(st, 2, dt, tl, n, parts, s.u, s.us, rows, H));
+        GUFFIN_TRY(guffin_hip_geglu(st, s.part_a, s.part_b, ffn_slices(L, H, F, rows), uint64_t(rows) * F, s.h, s.hs, rows, F));
     }
-    GUFFIN_TRY(guffin_hip_gemv_packed(st, L.dtype[6], L.tiles[6], s.h, s.hs, s.part_a, nullptr, rows, F, H));
+    GUFFIN_TRY(project(st, 1, L.dtype + 6, L.tiles + 6, &H, &s.part_a, s.h, s.hs, rows, F));
     // x = x1 + rms(down, post_ffw_norm); u = rms(x, next block's attn_norm | output_norm)
     const bool last = l + 1 == m.layer_count;
     const float* gamma_next = last ? m.out_norm : m.layers[l + 1].norm[0];
-    GUFFIN_TRY(guffin_hip_rms_norm_add_norm(st, s.part_a, slices(L.dtype[6], F, H), uint64_t(rows) * H, L.norm[5],
+    GUFFIN_TRY(guffin_hip_rms_norm_add_norm(st, s.part_a, slices(L.dtype[6], F, H, rows), uint64_t(rows) * H, L.norm[5],
                                             s.x1, s.x, gamma_next, last ? out_hidden : s.u,
                                             last ? out_hidden_sums : s.us, rows, H, m.eps, status));
     return GUFFIN_OK;
 }
 
+// tree: the rows are one whole verify tree instead of a run: row r stands at position + depth[r] and attends the ring
+// below `position` (through its window) and the rows of ancestors[r], a bit each, itself among them
+struct TreeRows { uint32_t depth[kWideRows], ancestors[kWideRows]; };
+
 int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t* tokens, uint32_t rows,
                  uint32_t position, const Scratch& s, void* priv_k, void* priv_v, float* out_hidden,
-                 float* out_hidden_sums, uint32_t* status) {
+                 float* out_hidden_sums, uint32_t* status, const TreeRows* tree = nullptr) {
     void* st = stream;
     const uint32_t H = m.hidden, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
     const float attn_scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
     // the resident pass is the default where it is the faster one: models with a single KV head (the drafter's
     // small blocks); it can be forced for any model it covers
-    const bool resident = s.exchange != nullptr && resident_chosen(m, rows);
+    const bool resident = s.exchange != nullptr && resident_chosen(m, rows) && !tree;
     if (g_forward_mode == 2 && !resident) return fail(GUFFIN_E_SHAPE, "forward: the resident pass does not cover this model");
     const uint32_t sync_words = resident ? s.sync_words : 0u;
     const uint32_t n_stage = std::max({m.layer_count * rows, rows * (m.head_dim / 2), sync_words});
+    uint32_t depths = 0x03020100u;
+    if (tree) {
+        depths = 0;
+        for (uint32_t r = 0; r < rows; ++r) depths |= tree->depth[r] << (8 * r);
+    }
     launch(stage_rows_kernel, dim3((n_stage + 63) / 64), dim3(64), 0, stream, s.positions, s.ancestors,
-                       s.schedule, rows, position, m.layer_count, m.sliding_window, m.global_period,
+                       s.schedule, rows, position, depths, tree ? 0u : m.layer_count, m.sliding_window, m.global_period,
                        reinterpret_cast<float2*>(s.rope_local), reinterpret_cast<float2*>(s.rope_global), m.head_dim,
                        m.local_base, m.global_base, m.global_scale, s.sync, sync_words);
     GUFFIN_TRY(check_launch("stage_rows"));
@@ -272,14 +296,21 @@ int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t*
             const void* tl[3] = {L.tiles[0], L.tiles[1], L.tiles[2]};
             const uint32_t n[3] = {QW, KW, KW};
             float* parts[3] = {s.part_a, s.part_b, s.part_c};
-            GUFFIN_TRY(guffin_hip_gemv_packed_multi(st, 3, dt, tl, n, parts, s.u, s.us, rows, H));
-            const uint32_t sq = qkv_slices(L, H, QW, KW);
+            GUFFIN_TRY(project(st, 3, dt, tl, n, parts, s.u, s.us, rows, H));
+            const uint32_t sq = qkv_slices(L, H, QW, KW, rows);
             if (sq == 0) return fail(GUFFIN_E_SHAPE, "forward: q, k and v must share the block length");
             // head norms, rotation, fp16 K/V rows and the attention itself in one pass over the planes; the
             // rows are contiguous and the position is the host's, so the schedule words stage_rows_kernel
             // writes are known here too and travel with the launch
-            uint32_t host_schedule[2][4], host_amask[2];
-            for (uint32_t row = 0; row < rows; ++row) row_schedule(m, l, position, row, host_schedule[row], host_amask[row]);
+            uint32_t host_schedule[kWideRows][4] = {}, host_amask[kWideRows] = {};
+            for (uint32_t row = 0; row < rows; ++row) {
+                if (!tree) { row_schedule(m, l, position, row, host_schedule[row], host_amask[row]); continue; }
+                const uint32_t p = position + tree->depth[row];
+                const uint32_t window_start = (local && p >= m.sliding_window) ? p + 1 - m.sliding_window : 0;
+                const uint32_t base_first = std::min(window_start, position);
+                host_schedule[row][0] = base_first; host_schedule[row][1] = position - base_first;
+                host_amask[row] = tree->ancestors[row];
+            }
             GUFFIN_TRY(qkv_attention_scheduled(st, s.part_a, s.part_b, s.part_c, sq, uint64_t(rows) * QW, uint64_t(rows) * KW,
                                                uint64_t(rows) * KW, L.norm[1], L.norm[2],
                                                local ? s.rope_local : s.rope_global, m.eps, L.ring_k, L.ring_v, pk, pv,
@@ -391,7 +422,36 @@ extern "C" int guffin_hip_forward_rows(void* stream, const guffin_model_desc* mo
                         out_hidden_sums, status);
 }
 
-// ---- rows of a verify tree -------------------------------------------------------------------
+// ---- a whole verify tree in one pass -----------------------------------------------------------
+// Up to four rows through the wide products.  Two query heads a KV head at most: the attention of four rows over more
+// would not fit its registers; such a model's trees run as passes of two rows below.
+bool guffin::tree_pass_fits(const guffin_model_desc& m) { return m.kv_heads != 0 && m.q_heads % m.kv_heads == 0 && m.q_heads / m.kv_heads <= 2; }
+
+uint64_t guffin::tree_pass_bytes(const guffin_model_desc& m, uint32_t position) {
+    if (validate_model(&m) || !tree_pass_fits(m)) return 0;
+    return std::max(layout(m, 3, position, nullptr).bytes, layout(m, 4, position, nullptr).bytes);
+}
+
+int guffin::forward_tree_pass(hipStream_t stream, const guffin_model_desc& m, const uint32_t* tokens, uint32_t rows, uint32_t position,
+                              const uint32_t* depths, const uint32_t* parents, void* scratch, uint64_t scratch_bytes, void* priv_k,
+                              void* priv_v, float* out_hidden, float* out_hidden_sums, uint32_t* status) {
+    GUFFIN_TRY(validate_model(&m));
+    if (rows == 0 || rows > kWideRows || !tree_pass_fits(m)) return fail(GUFFIN_E_SHAPE, "forward_tree_pass: at most 4 rows, at most 2 query heads per KV head");
+    if (m.global_period > 1 && m.sliding_window <= rows) return fail(GUFFIN_E_SHAPE, "forward_tree_pass: the sliding window must exceed the tree's depth");
+    TreeRows tree {};
+    uint32_t deepest = 0;
+    for (uint32_t r = 0; r < rows; ++r) {
+        tree.depth[r] = depths[r];
+        tree.ancestors[r] = (r == 0 ? 0u : tree.ancestors[parents[r]]) | 1u << r;   // rows come in topological order
+        deepest = std::max(deepest, depths[r]);
+    }
+    GUFFIN_TRY(check_ring_capacity(m, position, deepest + 1, "forward_tree_pass: the rows do not fit the KV rings"));
+    const Scratch s = layout(m, rows, position, static_cast<uint8_t*>(scratch));
+    if (s.bytes > scratch_bytes) return fail(GUFFIN_E_CAPACITY, "forward_tree_pass: scratch arena too small");
+    return forward_rows(stream, m, tokens, rows, position, s, priv_k, priv_v, out_hidden, out_hidden_sums, status, &tree);
+}
+
+// ---- rows of a verify tree, two at a time --------------------------------------------------------
 // One pass of 1 or 2 rows whose parents may be any earlier row of the tree: a row's token list is the ring
 // below `base_position` (through the layer's window) followed by its ancestors among the tree's private
 // rows, itself last.  The rows' own K/V go to consecutive private slots; attention reads every slot an
@@ -461,8 +521,8 @@ extern "C" int guffin_hip_forward_tree_rows(void* stream, const guffin_model_des
         const void* tl[3] = {L.tiles[0], L.tiles[1], L.tiles[2]};
         const uint32_t n[3] = {QW, KW, KW};
         float* parts[3] = {s.part_a, s.part_b, s.part_c};
-        GUFFIN_TRY(guffin_hip_gemv_packed_multi(stream, 3, dt, tl, n, parts, s.u, s.us, rows, H));
-        const uint32_t sq = qkv_slices(L, H, QW, KW);
+        GUFFIN_TRY(project(stream, 3, dt, tl, n, parts, s.u, s.us, rows, H));
+        const uint32_t sq = qkv_slices(L, H, QW, KW, rows);
         if (sq == 0) return fail(GUFFIN_E_SHAPE, "forward_tree_rows: q, k and v must share the block length");
         // head norms, rotation and fp16 narrowing into the rows' own slots, then attention over ring and slots
         GUFFIN_TRY(guffin_hip_qkv_post(stream, s.part_a, s.part_b, s.part_c, sq, sq, sq, uint64_t(rows) * QW, uint64_t(rows) * KW,
@@ -716,9 +776,9 @@ StepBuffers carve_step(const guffin_h1_desc* d, void* scratch) {
     b.t_scratch = ar.take<uint8_t>(b.t_bytes);
     b.d_hidden = ar.take<float>(hidden_with_receipt(dr, D.hidden));
     b.t_hidden = ar.take<float>(hidden_with_receipt(2, T.hidden));
-    b.q_parts = ar.take<float>(uint64_t(slices(D.head_dtype, D.hidden, D.vocab)) * dr * D.vocab);
+    b.q_parts = ar.take<float>(uint64_t(slices(D.head_dtype, D.hidden, D.vocab, dr)) * dr * D.vocab);
     b.q_logits = ar.take<float>(uint64_t(dr) * D.vocab);
-    b.p_parts = ar.take<float>(uint64_t(slices(T.head_dtype, T.hidden, V)) * 2 * V);
+    b.p_parts = ar.take<float>(uint64_t(slices(T.head_dtype, T.hidden, V, 2)) * 2 * V);
     b.p_logits = ar.take<float>(2 * V);
     b.law_ws = ar.take<uint8_t>(guffin_hip_draft_law_workspace_bytes(D.vocab));
     b.sel_ws = ar.take<uint8_t>(guffin_hip_select_workspace_bytes(2, V, d->top_k + kHistoryWindow));

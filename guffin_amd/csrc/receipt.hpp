@@ -4,12 +4,13 @@
 //                                      reference's producers emit the same kind of receipt for
 //                                      its Q4_K kernels, metal_kernels.mm:16-27)
 //   mult   float [rows][K/32]          per 32-group multiplier 2^(E+24) of the image below
-//   image  half  [K/32][4][32]         matrix-core operand: variant 2r = hi, 2r+1 = lo of row r,
+//   image  half  [K/32][V][32]         matrix-core operand, V = 4 variants for up to two rows and 8 for three or four:
+//                                      variant 2r = hi, 2r+1 = lo of row r,
 //                                      hi + lo = x * 2^-E to 22 bits, E chosen per 32-group so that
 //                                      |x| 2^-E < 2^15; inside a group the 8 halves of k-slice s
 //                                      (elements 8s..8s+7) sit at 8s + {0,2,1,3,4,6,5,7}, the
 //                                      order in which nibble pairs fall out of a weight dword
-// All three start on 256-byte boundaries of one blob; K must be a multiple of 32.
+// All three start on 256-byte boundaries of one blob; K must be a multiple of 32.  Three rows are laid out as four.
 #pragma once
 #include "common.hpp"
 
@@ -26,10 +27,11 @@ __device__ __forceinline__ float geglu_value(float g, float u) {
 struct ReceiptLayout { size_t mult_off, image_off, bytes; };
 
 __host__ __device__ inline ReceiptLayout receipt_layout(uint32_t rows, uint32_t K) {
-    const size_t sums = size_t(rows) * (K / 16 + K / 32) * 4;
+    const uint32_t laid = rows > 2 ? 4u : rows;
+    const size_t sums = size_t(laid) * (K / 16 + K / 32) * 4;
     const size_t mult = (sums + 255) & ~size_t{255};
-    const size_t image = (mult + size_t(rows) * (K / 32) * 4 + 255) & ~size_t{255};
-    return {mult, image, image + size_t(K / 32) * 256};
+    const size_t image = (mult + size_t(laid) * (K / 32) * 4 + 255) & ~size_t{255};
+    return {mult, image, image + size_t(K / 32) * (rows > 2 ? 512 : 256)};
 }
 
 // One item: the 8 consecutive activations v[] of row r, elements k0 + 8t .. k0 + 8t + 7.  The four
@@ -72,10 +74,10 @@ __device__ __forceinline__ void emit_receipt_values(const float (&v)[8], uint32_
             }
             hi[p] = hw; lo[p] = lw;
         }
-        uint8_t* base = image + (size_t(g) * 4 + 2 * r) * 64 + s * 16;
+        uint8_t* base = image + (size_t(g) * (rows > 2 ? 8 : 4) + 2 * r) * 64 + s * 16;
         *reinterpret_cast<uint4*>(base) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
         *reinterpret_cast<uint4*>(base + 64) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-        if (rows == 1) {  // the operand always has four variants; a single row leaves two empty
+        if ((rows & 1u) && r + 1 == rows) {  // the operand has four or eight variants; an odd row count leaves two empty
             *reinterpret_cast<uint4*>(base + 128) = make_uint4(0, 0, 0, 0);
             *reinterpret_cast<uint4*>(base + 192) = make_uint4(0, 0, 0, 0);
         }

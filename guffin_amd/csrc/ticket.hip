@@ -12,8 +12,9 @@
 // it is about to overwrite into the backup rows, then scatters the selected private rows into the
 // rings; finalize keeps a prefix of them and restores the rest.  The rows of a pass are a chain of 1 or
 // 2 rows (one launch sequence of the block graph) or a tree of up to 4 rows in topological order (row r's
-// parent is any earlier row), which runs in passes of 2 rows whose attention reads the earlier rows'
-// private K/V; a provisional commit takes any root-to-node path.  Nothing is allocated: every buffer is
+// parent is any earlier row), which runs in one pass that fetches the weights once for all of them (a model with more
+// than two query heads per KV head: in passes of 2 rows whose attention reads the earlier rows' private K/V); a
+// provisional commit takes any root-to-node path.  Nothing is allocated: every buffer is
 // the caller's.
 #include <cstddef>
 #include "common.hpp"
@@ -39,13 +40,14 @@ Arena arena_of(const guffin_model_desc& m, uint32_t position, uint32_t retain) {
     Arena a {};
     const uint32_t rows = kMaxTicketRows;
     uint64_t off = 0;
-    // a pass has at most 2 rows; a tree pass sizes its arena at the deepest position a row can take
+    // a chain's pass has at most 2 rows; a tree pass sizes its arena at the deepest position a row can take
     a.forward = off; off += aligned(std::max({guffin_hip_forward_scratch_bytes(&m, 2, position),
                                               guffin_hip_forward_scratch_bytes(&m, 2, position + kMaxTicketRows),
-                                              guffin_hip_forward_scratch_bytes(&m, 1, position + kMaxTicketRows)}));
+                                              guffin_hip_forward_scratch_bytes(&m, 1, position + kMaxTicketRows), tree_pass_bytes(m, position)}));
     a.hidden_receipt = (uint64_t(rows) * m.hidden + 63) & ~uint64_t{63};
     a.hidden = off; off += aligned(a.hidden_receipt * 4 + receipt_layout(rows, m.hidden).bytes);
-    const uint32_t slices = guffin_hip_gemv_packed_slices(m.head_dtype, m.hidden, m.vocab);
+    const int head_dtype = m.head_dtype;
+    const uint32_t slices = std::max(guffin_hip_gemv_packed_slices(head_dtype, m.hidden, m.vocab), gemv_wide_planes(1, &head_dtype, &m.vocab, m.hidden));
     a.parts = off; off += aligned(uint64_t(slices) * rows * m.vocab * 4);
     a.pass_receipt = off; off += aligned(receipt_layout(2, m.hidden).bytes);
     a.logits = off; off += aligned(uint64_t(rows) * m.vocab * 4);
@@ -157,6 +159,13 @@ extern "C" int guffin_hip_ticket_submit(void* stream, guffin_verify_ticket* t) {
                                          t->priv_v, hidden, hidden_sums, t->status);
         if (rc == GUFFIN_OK)
             rc = guffin_hip_gemv_packed(stream, m.head_dtype, m.head_tiles, hidden, hidden_sums, parts, logits, t->rows, m.hidden, m.vocab);
+    } else if (tree_pass_fits(m)) {
+        if (rc == GUFFIN_OK)
+            rc = forward_tree_pass(hs, m, t->tokens, t->rows, t->position, t->depths, t->parents, base + a.forward, a.hidden - a.forward,
+                                   t->priv_k, t->priv_v, hidden, hidden_sums, t->status);
+        const int head_dtype = m.head_dtype;
+        const void* head = m.head_tiles;
+        if (rc == GUFFIN_OK) rc = gemv_wide(hs, 1, &head_dtype, &head, &m.vocab, &parts, hidden_sums, logits, t->rows, m.hidden);
     } else {
         // passes of two rows in row order; a row's ancestor list is its path from the root, itself last
         float* pass_receipt = reinterpret_cast<float*>(base + a.pass_receipt);

@@ -802,8 +802,8 @@ int guffin_hip_ticket_encode(guffin_verify_ticket* ticket, const uint32_t* row_t
 /* The same for a tree of up to 4 rows in topological order (VerifierTopologyDescriptor,
  * include/local_gguf_engine/engine/target_verifier.hpp): parents[0] = GUFFIN_TICKET_ROOT, parents[r] < r.  Row r is
  * verified at cache position `position` + its depth and attends the ring and its ancestors among the rows.  A chain
- * of 1 or 2 rows runs as guffin_hip_ticket_encode runs it (one pass); any other tree runs in passes of 2 rows
- * through guffin_hip_forward_tree_rows.  guffin_hip_ticket_provisional_commit then takes any root-to-node path. */
+ * of 1 or 2 rows runs as guffin_hip_ticket_encode runs it; any other tree is one pass of its own too, or, with more than two
+ * query heads per KV head, passes of 2 rows through guffin_hip_forward_tree_rows.  guffin_hip_ticket_provisional_commit then takes any root-to-node path. */
 int guffin_hip_ticket_encode_tree(guffin_verify_ticket* ticket, const uint32_t* row_tokens, const uint32_t* parents,
                                   uint32_t rows, uint32_t position);
 int guffin_hip_ticket_submit(void* stream, guffin_verify_ticket* ticket);

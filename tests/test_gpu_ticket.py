@@ -254,3 +254,51 @@ def test_three_row_tree_against_the_oracle_and_every_path(hip, gfo):
     ticket.provisional_commit([0, 1, 2])
     ticket.discard()
     assert_rings(target, kept)
+
+
+@pytest.mark.parametrize("position", [0, 5, 1023])
+@pytest.mark.parametrize("parents", [(None, 0, 0), (None, 0, 1, 0), (None, 0, 1, 2)])
+@pytest.mark.parametrize("kind", ["12b", "mixed", "q8_0", "one_head"])
+def test_a_tree_in_one_pass_equals_its_chains(hip, kind, parents, position):
+    """Trees of 3 and 4 rows run as one pass over the wide products (Q4_K, Q6_K, both in a launch, Q8_0; ragged column groups and
+    K slices) and the attention of 3 and 4 rows.  Every row's path from the root, taken as a chain of one-row passes over rings that
+    hold its ancestors, must give the same row: the products are exact on both sides, so the rows differ by the order of their fp32
+    sums only (1e-3 of the largest logit and nearly all fp16 patterns equal, as between the one-row and the resident pass)."""
+    import torch
+    from guffin_amd import model, synth
+    shape = replace(model.GEMMA3_12B, layers=6, vocab=2048, ring_global=2048)
+    if kind == "mixed":   # every projection in the other K-quant now and then: mixed q/k/v launches, gate/up without the fused form
+        shape = replace(shape, hidden=768, ffn=1280, dtypes=(synth.Q4_K, synth.Q6_K, synth.Q4_K, synth.Q6_K, synth.Q6_K, synth.Q4_K, synth.Q4_K))
+    elif kind == "q8_0":
+        shape = replace(shape, hidden=640, ffn=1088, q_heads=4, kv_heads=2, dtypes=(synth.Q8_0,) * 7, embed_dtype=synth.Q8_0)
+    elif kind == "one_head":   # one query head per KV head
+        shape = replace(shape, hidden=512, ffn=768, q_heads=4, kv_heads=4)
+    host = model.HostModel(shape, seed=9, position=position, untied_head=True)
+    target = model.DeviceModel.from_host(host)
+    ticket = model.VerifyTicket(target, position + 4)
+    tokens = [17, 1999, 42, 7][:len(parents)]
+    before = rings(target)
+    ticket.encode_tree(tokens, list(parents), position)
+    ticket.submit()
+    assert ticket.complete() == 0
+    assert_rings(target, before)
+    got, kvw, rows = ticket.read_candidates(), shape.kv_width, len(parents)
+    priv_k = ticket.priv_k.view(-1)[:shape.layers * rows * kvw].view(shape.layers, rows, kvw).clone()
+    priv_v = ticket.priv_v.view(-1)[:shape.layers * rows * kvw].view(shape.layers, rows, kvw).clone()
+    for row in range(rows):
+        path, node = [], row
+        while node is not None:
+            path.insert(0, node)
+            node = parents[node]
+        for depth, node in enumerate(path):
+            tok = torch.tensor([tokens[node]], dtype=torch.int32, device="cuda")
+            hidden, sums, pk, pv, status = target.forward(tok, position + depth)
+            publish([(k, v) for k, v in zip(target.ring_k, target.ring_v)], target, pk, pv, position + depth, [0])
+        assert int(status) == 0
+        logits = hip.gemv_packed(int(shape.embed_dtype), target.head_tiles, hidden, sums, shape.vocab)
+        want = hip.candidates_to_numpy(hip.select_candidates(logits, 64)[0])[0]["values"]
+        assert np.allclose(got[row]["values"]["logit"][:64], want["logit"][:64], rtol=0, atol=1e-3 * float(np.abs(want["logit"][:64]).max()))
+        assert np.mean((priv_k[:, row] == pk[:, 0]).cpu().numpy()) >= 0.95 and np.mean((priv_v[:, row] == pv[:, 0]).cpu().numpy()) >= 0.95
+        for (k, v), (bk, bv) in zip(zip(target.ring_k, target.ring_v), before):
+            k.copy_(bk)
+            v.copy_(bv)
