@@ -18,11 +18,16 @@
 //   Q6_K 13440 B : pieces 0..7 ql, 8..11 qh, piece 12 = 16 int8 scales, then 64 x fp16 d
 //   Q8_0  2176 B : pieces 0..1 quants, then 64 x fp16 d
 //
-// GEMV: one v_mfma_f32_16x16x32_f16 per 32 elements and column group.  B = the quants as fp16
-// subnormals (an integer n < 1024 in a half is exactly n*2^-24, and the matrix core honours
-// subnormal inputs), A = the activation image of the producer's receipt (hi/lo fp16 split of
-// x * 2^-E per 32-group, four variants = two rows), so every product is exact and sums are
-// fp32.  Block scales are applied to the per-group sums in fp32 by the lane that owns the
+// GEMV: B = the quants as fp16 patterns below 2048 (an integer n < 2048 in a half is exactly n*2^-24, and the matrix
+// core honours subnormal inputs), A = the activation image of the producer's receipt (hi/lo fp16 split of x * 2^-E per
+// 32-group, four variants = two rows), so every product is exact and sums are fp32.  Q8_0: one v_mfma_f32_16x16x32_f16
+// per 32 elements and column group of 16.  Q4_K, Q6_K: v_mfma_f32_4x4x4_16b_f16, the same rate in useful products
+// (sixteen column groups of 4 side by side, no repeated A rows), a lane owning one column from its quants to its sum: no
+// selection among column groups (128 of 496 vector instructions of a Q4_K tile), no masked half-groups and lane exchanges
+// for Q6_K, and the operand of a 256-element block in 8 registers instead of 32, so it is requested ahead of every tile.
+// With the 16x16x32 form / now (us): gate + up 3840 -> 15360 on two rows 17.3 / 15.2, on one 16.2 / 14.5, down
+// 15360 -> 3840 on two rows 13.0 / 11.3, q/k/v 8.2 / 7.4: what a launch streams does not change, its unpack is what
+// does not overlap.  Block scales are applied to the per-group sums in fp32 by the lane that owns the
 // column; the offset terms (-dmin*m for Q4_K, -32 for Q6_K, -128 for the biased Q8_0 bytes)
 // use the receipt's 16- / 32-sums.  K is cut into slices: up to 16 slices are the waves of
 // one workgroup, combined in wave order through LDS; the remaining S "planes" go to

@@ -5,6 +5,9 @@
 #include "common.hpp"
 #include "receipt.hpp"
 
+#include <type_traits>
+#include <utility>
+
 namespace guffin {
 namespace {
 
@@ -25,15 +28,14 @@ __device__ __forceinline__ uint32_t odd_bytes(uint32_t v) { return __builtin_amd
 // =======================================================================================
 // Q4_K
 // =======================================================================================
-// Matrix-core path.  A wave covers 64 columns x one 256-element block as four column groups
-// of 16; lane (j = lane % 16, s = lane / 16) holds, for every column group, the bytes 8s..8s+7
-// of each 32-byte quant chunk of column 16*cg + j, and owns column `lane` for the scales and
-// the result.  For each 32-element sub-block and column group one v_mfma_f32_16x16x32_f16
-// multiplies the activation image (A: 16 rows = the 4 variants hi/lo x row, repeated; lane
-// (i, s) holds variant i % 4, k-slice s) with the nibbles as fp16 subnormals (B: q * 2^-24,
-// or 16q * 2^-24 for high nibbles, both exact).  Every lane group then holds the four variant
-// sums of the 16 columns of that group; lane group g keeps those of column group g and scales
-// them by d*sc of its own column in fp32.  The -dmin*m term uses the 32-sums.
+// Matrix-core path (Q4_K and Q6_K).  A wave covers 64 columns x one 256-element block; lane l owns column l for everything: its
+// quants, its scales, its result.  One v_mfma_f32_4x4x4_16b_f16 multiplies four elements of every column with the four variants
+// (hi/lo x row) of the activation image: sixteen 4x4 products side by side, block l / 4 of the B side holding the columns of lanes
+// 4 (l / 4) .. + 3, the A side one block of four elements broadcast to all sixteen (CBSZ 4, ABID the block).  So a lane's 8 bytes
+// of the image, block l / 4 for variant l % 4, are the operand of 64 elements, and 8 registers that of a whole 256-element block.
+// B: the quants as fp16 bit patterns below 2048 (q * 2^-24 times a power of two, exact).  Eight chained instructions are a 32-group
+// (four a 16-element half of Q6_K), and every lane finds the four variant sums of its own column in its own registers; it scales them
+// by d*sc in fp32.  The -dmin*m term uses the 32-sums.
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
@@ -45,42 +47,54 @@ __device__ __forceinline__ uint4 stream_load(const uint8_t* p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+
+// bytes from the start of a 256-element tile to the pieces of the lane's column: its 16-byte pieces lie 256 bytes apart (k-slices),
+// 16 columns side by side, the column groups 2048 bytes apart (1024 for the high bits of Q6_K)
+__device__ __forceinline__ uint32_t column_at(uint32_t lane) { return (lane >> 4) * 2048u + (lane & 15u) * 16u; }
+
+// q[4 h + s]: k-slice s of chunks 2h and 2h + 1
 struct Q4Tile { uint4 q[8]; uint4 hdr; };
 
 // Loads come back in the order of their requests: the scales and the pieces of the first four sub-blocks go
 // first, so that their products run while the other half of the tile is still on its way.
-__device__ __forceinline__ void load_tile(Q4Tile& t, const uint8_t* p) {
-    t.hdr = stream_load(p + 8192);
+__device__ __forceinline__ void load_tile(Q4Tile& t, const uint8_t* tile, uint32_t lane) {
+    t.hdr = stream_load(tile + 8192 + lane * 16);
+    const uint8_t* p = tile + column_at(lane);
 #pragma unroll
-    for (int i = 0; i < 8; i += 2) t.q[i] = stream_load(p + 1024 * i);
-#pragma unroll
-    for (int i = 1; i < 8; i += 2) t.q[i] = stream_load(p + 1024 * i);
+    for (int i = 0; i < 8; ++i) t.q[i] = stream_load(p + 1024 * (i >> 2) + 256 * (i & 3));
 }
 
 __device__ __forceinline__ half8_t as_half8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
     return __builtin_bit_cast(half8_t, make_uint4(a, b, c, d));
 }
 
-// image: this block's 8 groups of the activation image, already offset for this lane;
-// mult / xs32: this block's 8 multipliers / 32-sums of row 0 (rows `per_mult` / `per_row` apart)
-struct Q4Operand { half8_t a[8]; };
-__device__ __forceinline__ void load_operand(Q4Operand& o, const uint8_t* __restrict__ image) {
+// The operand of a 256-element block: groups 2p and 2p + 1 in a[p], A-side block 8 (g % 2) + i holding elements 4i .. 4i + 3 of
+// group g.  image: this block's 8 groups of the activation image, already offset for this lane.
+struct BlockOperand { half4_t a[4]; };
+__device__ __forceinline__ uint32_t operand_lane(uint32_t lane) { return (lane >> 5) * 256u + (lane & 3u) * 64u + ((lane >> 2) & 7u) * 8u; }
+__device__ __forceinline__ void load_operand(BlockOperand& o, const uint8_t* __restrict__ image) {
 #pragma unroll
-    for (int g = 0; g < 8; ++g) o.a[g] = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(image + 256 * g));
+    for (int p = 0; p < 4; ++p) o.a[p] = __builtin_bit_cast(half4_t, *reinterpret_cast<const uint2*>(image + 512 * p));
 }
+template <int BLOCK>
+__device__ __forceinline__ float4_t mac4(half4_t a, uint32_t b0, uint32_t b1, float4_t c) {
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(a, __builtin_bit_cast(half4_t, make_uint2(b0, b1)), c, 4, BLOCK, 0);
+}
+template <typename F, int... I>
+__device__ __forceinline__ void each_slice(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
 
+// mult / xs32: this block's 8 multipliers / 32-sums of row 0 (rows `per_mult` / `per_row` apart)
 template <int R>
-__device__ __forceinline__ void compute_tile(const Q4Tile& t, const Q4Operand& op,
+__device__ __forceinline__ void compute_tile(const Q4Tile& t, const BlockOperand& op,
                                              const float* __restrict__ mult, uint32_t per_mult,
-                                             const float* __restrict__ xs32, uint32_t per_row,
-                                             uint32_t lane_group, float (&acc)[R]) {
-    const half8_t (&a)[8] = op.a;
+                                             const float* __restrict__ xs32, uint32_t per_row, float (&acc)[R]) {
     const float d = h2f(t.hdr.x & 0xFFFFu), dmin = h2f(t.hdr.x >> 16);
     const uint32_t s0 = t.hdr.y, s1 = t.hdr.z, s2 = t.hdr.w;
     const uint32_t sc_a = s0 & 0x3F3F3F3Fu, mn_a = s1 & 0x3F3F3F3Fu;
     const uint32_t sc_b = (s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u);
     const uint32_t mn_b = ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u);
-    const float d_q = d * 0.0625f;  // nibbles enter as 16 q
+    const float d_lo = d * (1.f / 128), d_hi = d * (1.f / 16);  // nibbles enter as 128 q and 16 q
     float mt[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) mt[r] = 0.f;
@@ -88,26 +102,25 @@ __device__ __forceinline__ void compute_tile(const Q4Tile& t, const Q4Operand& o
 #pragma unroll
     for (int ch = 0; ch < 4; ++ch) {  // 32-byte chunk: sub-blocks 2ch (low nibbles) and 2ch+1 (high)
         float4_t lo = zero, hi = zero;
-#pragma unroll
-        for (int cg = 0; cg < 4; ++cg) {
-            const uint4 piece = t.q[2 * cg + (ch >> 1)];
+        each_slice([&](auto slice) {
+            constexpr int S = slice;
+            const uint4 piece = t.q[4 * (ch >> 1) + S];
             const uint32_t w0 = (ch & 1) ? piece.z : piece.x, w1 = (ch & 1) ? piece.w : piece.y;
-            // every nibble sits in bits 4-7 of its half (16 q as a bit pattern below 2048, which reads as
-            // 16 q 2^-24): the matrix instruction does not normalise such operands, so a pattern with leading
-            // zeros loses that many bits of every product it meets once the products of a sum are aligned.
-            // (In bits 0-3 the low nibbles cost up to 200 eps of a group's sum|q x| on activations with a wide
-            // range inside the group; bits 6-9 would gain two more bits for one more shift per word.)
-            constexpr uint32_t M = 0x00F000F0u;
-            const half8_t blo = as_half8((w0 << 4) & M, (w0 >> 4) & M, (w1 << 4) & M, (w1 >> 4) & M);
-            const half8_t bhi = as_half8(w0 & M, (w0 >> 8) & M, w1 & M, (w1 >> 8) & M);
-            const float4_t dlo = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[2 * ch], blo, zero, 0, 0, 0);
-            const float4_t dhi = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[2 * ch + 1], bhi, zero, 0, 0, 0);
-            if (lane_group == uint32_t(cg)) { lo = dlo; hi = dhi; }
-        }
+            // low nibbles sit in bits 7-10 of their half, high ones in bits 4-7 (128 q and 16 q as bit patterns below 2048, which
+            // read as n 2^-24): the matrix instruction does not normalise such operands, so a pattern with leading zeros loses
+            // that many bits of every product it meets once the products of a sum are aligned.  (Where the low nibbles go costs
+            // the same; the high ones further up would take one more shift per word.  Both in bits 4-7: rms error on
+            // activations with a 512-fold range, K = 3840, 5.2e-7 of the result's rms.)
+            constexpr uint32_t L = 0x07800780u, M = 0x00F000F0u;
+            lo = mac4<2 * S>(op.a[ch], (w0 << 7) & L, (w0 >> 1) & L, lo);
+            hi = mac4<8 + 2 * S>(op.a[ch], w0 & M, (w0 >> 8) & M, hi);
+            lo = mac4<2 * S + 1>(op.a[ch], (w1 << 7) & L, (w1 >> 1) & L, lo);
+            hi = mac4<8 + 2 * S + 1>(op.a[ch], w1 & M, (w1 >> 8) & M, hi);
+        }, std::make_integer_sequence<int, 4>{});
         const uint32_t scw = ch < 2 ? sc_a : sc_b, mnw = ch < 2 ? mn_a : mn_b;
         const float sc_lo = (ch & 1) ? ub2(scw) : ub0(scw), sc_hi = (ch & 1) ? ub3(scw) : ub1(scw);
         const float mn_lo = (ch & 1) ? ub2(mnw) : ub0(mnw), mn_hi = (ch & 1) ? ub3(mnw) : ub1(mnw);
-        const float f_lo = d_q * sc_lo, f_hi = d_q * sc_hi;
+        const float f_lo = d_lo * sc_lo, f_hi = d_hi * sc_hi;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const float m_lo = mult[r * per_mult + 2 * ch], m_hi = mult[r * per_mult + 2 * ch + 1];
@@ -124,33 +137,20 @@ __device__ __forceinline__ void compute_tile(const Q4Tile& t, const Q4Operand& o
 // =======================================================================================
 // Q6_K
 // =======================================================================================
-// Same operand scheme as Q4_K with two differences.  A scale covers 16 elements, so the A rows
-// of one 32-element MFMA are split: rows 0-3 carry the variants with the second 16 elements
-// zeroed, rows 4-7 the other half (rows 8-15 repeat them); lane group g then holds the sums of
-// k-half g % 2.  Lane (j, g) owns columns 32*(g/2) + j and + 16 for that k-half, keeps column
-// groups 2*(g/2) and 2*(g/2)+1, and the two k-halves are added across lanes at the end.
-struct Q6Tile { uint4 ql[8]; uint4 qh[4]; uint4 sc[2]; uint32_t d[2]; };
+// Same operand scheme as Q4_K; a scale covers 16 elements, so a 32-group is two chains of four instructions.
+// ql[4 n + s]: k-slice s of half n; qh[s]: k-slice s of both halves
+struct Q6Tile { uint4 ql[8]; uint4 qh[4]; uint4 sc; uint32_t d; };
 
-// EARLY: the request order of the Q4_K tile (what the first 128 elements need, then the low nibbles of the other
-// half).  It pays where the operand groups are requested ahead of the tile; the one-tile-at-a-time walk reads
-// them behind the tile, where a group's wait covers every earlier request anyway, and is slower with it.
-template <bool EARLY>
-__device__ __forceinline__ void load_tile(Q6Tile& t, const uint8_t* p, uint32_t lane) {
+// What the first 128 elements need goes first, then the low nibbles of the other half.
+__device__ __forceinline__ void load_tile(Q6Tile& t, const uint8_t* tile, uint32_t lane) {
+    const uint8_t* p = tile + column_at(lane);
+    const uint8_t* ph = tile + 8192 + (lane >> 4) * 1024u + (lane & 15u) * 16u;
+    t.sc = *reinterpret_cast<const uint4*>(tile + 12288 + lane * 16);
+    t.d = *reinterpret_cast<const uint16_t*>(tile + 13312 + lane * 2);
 #pragma unroll
-    for (int i = 0; i < 8; i += EARLY ? 2 : 1) t.ql[i] = stream_load(p + 1024 * i);
+    for (int i = 0; i < 4; ++i) { t.ql[i] = stream_load(p + 256 * i); t.qh[i] = stream_load(ph + 256 * i); }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) t.qh[i] = stream_load(p + 8192 + 1024 * i);
-    const uint8_t* base = p - lane * 16;
-    const uint32_t col = 32u * (lane >> 5) + (lane & 15u);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        t.sc[c] = *reinterpret_cast<const uint4*>(base + 12288 + (col + 16 * c) * 16);
-        t.d[c] = *reinterpret_cast<const uint16_t*>(base + 13312 + (col + 16 * c) * 2);
-    }
-    if constexpr (EARLY) {
-#pragma unroll
-        for (int i = 1; i < 8; i += 2) t.ql[i] = stream_load(p + 1024 * i);
-    }
+    for (int i = 4; i < 8; ++i) t.ql[i] = stream_load(p + 1024 + 256 * (i & 3));
 }
 
 __device__ __forceinline__ float sbyte(uint32_t w, int i) {
@@ -158,85 +158,56 @@ __device__ __forceinline__ float sbyte(uint32_t w, int i) {
 }
 
 template <int R>
-__device__ __forceinline__ void compute_tile(const Q6Tile& t, const uint8_t* __restrict__ image, uint32_t keep,
+__device__ __forceinline__ void compute_tile(const Q6Tile& t, const BlockOperand& op,
                                              const float* __restrict__ mult, uint32_t per_mult,
-                                             const float* __restrict__ xs16, uint32_t per_row,
-                                             uint32_t lane, float (&acc)[2][R]) {
-    const uint32_t khalf = (lane >> 4) & 1u;
-    const bool upper = lane >= 32;
+                                             const float* __restrict__ xs16, uint32_t per_row, float (&acc)[2][R]) {
     const float4_t zero = {0.f, 0.f, 0.f, 0.f};
-    float part[2][R], off[2][R];
+    float part[2][R], off[2][R];   // of the first and of the second halves of the groups: two sums half as long
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int r = 0; r < R; ++r) { part[c][r] = 0.f; off[c][r] = 0.f; }
-#pragma unroll
-    for (int g = 0; g < 8; ++g) {  // 32-element group: half n, quadrant qd
-        const int n = g >> 2, qd = g & 3;
-        uint4 av = *reinterpret_cast<const uint4*>(image + 256 * g);
-        av.x &= keep; av.y &= keep; av.z &= keep; av.w &= keep;
-        const half8_t a = __builtin_bit_cast(half8_t, av);
-        float4_t D[4];
-#pragma unroll
-        for (int cg = 0; cg < 4; ++cg) {
-            const uint4 lq = t.ql[2 * cg + n], hq = t.qh[cg];
-            const uint32_t w0 = (qd & 1) ? lq.z : lq.x, w1 = (qd & 1) ? lq.w : lq.y;
-            const uint32_t h0 = n ? hq.z : hq.x, h1 = n ? hq.w : hq.y;
-            const int ls = qd >= 2 ? 4 : 0;  // nibble shift
-            uint32_t b[4];
+    for (int r = 0; r < R; ++r) part[0][r] = part[1][r] = off[0][r] = off[1][r] = 0.f;
+    each_slice([&](auto group) {  // 32-element group: half n, quadrant qd
+        constexpr int G = group, n = G >> 2, qd = G & 3, ls = qd >= 2 ? 4 : 0, AT = 8 * (G & 1);
+        float4_t first = zero, second = zero;
+        auto slice_operand = [&](int s, uint32_t (&b)[4]) {
+            const uint4 lq = t.ql[4 * n + s], hq = t.qh[s];
+            const uint32_t w[2] = {(qd & 1) ? lq.z : lq.x, (qd & 1) ? lq.w : lq.y};
+            const uint32_t h[2] = {n ? hq.z : hq.x, n ? hq.w : hq.y};
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
-                const uint32_t w = k ? w1 : w0, h = k ? h1 : h0;
                 // the 6-bit quant sits in bits 4-9 of its half (16 q as a bit pattern: see the Q4_K tile)
-                const uint32_t lo0 = (ls ? w : w << 4) & 0x00F000F0u, lo1 = (w >> (ls + 4)) & 0x00F000F0u;
+                const uint32_t lo0 = (ls ? w[k] : w[k] << 4) & 0x00F000F0u, lo1 = (w[k] >> (ls + 4)) & 0x00F000F0u;
                 // 2-bit field of quadrant qd moved to bits 8-9 of each half
-                const uint32_t hs0 = h << (8 - 2 * qd);
-                const uint32_t hs1 = qd == 0 ? h : h >> (2 * qd);
+                const uint32_t hs0 = h[k] << (8 - 2 * qd), hs1 = qd == 0 ? h[k] : h[k] >> (2 * qd);
                 b[2 * k] = (hs0 & 0x03000300u) | lo0;
                 b[2 * k + 1] = (hs1 & 0x03000300u) | lo1;
             }
-            D[cg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, as_half8(b[0], b[1], b[2], b[3]), zero, 0, 0, 0);
-        }
-        const float4_t da = upper ? D[2] : D[0], db = upper ? D[3] : D[1];
-        // int8 scale of 16-element group 2g + khalf for the lane's two columns
-        const int word = g >> 1;  // scales 4*word .. 4*word+3 hold groups 2g-(g&1)*2 ...
-        float sc[2];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const uint32_t wv = word == 0 ? t.sc[c].x : word == 1 ? t.sc[c].y : word == 2 ? t.sc[c].z : t.sc[c].w;
-            const float s_even = sbyte(wv, 2 * (g & 1)), s_odd = sbyte(wv, 2 * (g & 1) + 1);
-            sc[c] = khalf ? s_odd : s_even;
-        }
+        };
+        each_slice([&](auto slice) {   // slices s (first 16 elements) and s + 2 (second)
+            constexpr int S = slice;
+            uint32_t b[4], c[4];
+            slice_operand(S, b);
+            slice_operand(S + 2, c);
+            first = mac4<AT + 2 * S>(op.a[G >> 1], b[0], b[1], first);
+            second = mac4<AT + 2 * S + 4>(op.a[G >> 1], c[0], c[1], second);
+            first = mac4<AT + 2 * S + 1>(op.a[G >> 1], b[2], b[3], first);
+            second = mac4<AT + 2 * S + 5>(op.a[G >> 1], c[2], c[3], second);
+        }, std::make_integer_sequence<int, 2>{});
+        const uint32_t wv = (G >> 1) == 0 ? t.sc.x : (G >> 1) == 1 ? t.sc.y : (G >> 1) == 2 ? t.sc.z : t.sc.w;
+        const float s_first = sbyte(wv, 2 * (G & 1)), s_second = sbyte(wv, 2 * (G & 1) + 1);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const float m = mult[r * per_mult + g];
-            const float s16_first = xs16[r * per_row + 2 * g], s16_second = xs16[r * per_row + 2 * g + 1];
-            const float s16 = khalf ? s16_second : s16_first;
-            part[0][r] = fmaf(sc[0] * m, da[2 * r] + da[2 * r + 1], part[0][r]);
-            part[1][r] = fmaf(sc[1] * m, db[2 * r] + db[2 * r + 1], part[1][r]);
-            off[0][r] = fmaf(sc[0], s16, off[0][r]);
-            off[1][r] = fmaf(sc[1], s16, off[1][r]);
+            const float m = mult[r * per_mult + G];
+            part[0][r] = fmaf(s_first * m, first[2 * r] + first[2 * r + 1], part[0][r]);
+            part[1][r] = fmaf(s_second * m, second[2 * r] + second[2 * r + 1], part[1][r]);
+            off[0][r] = fmaf(s_first, xs16[r * per_row + 2 * G], off[0][r]);
+            off[1][r] = fmaf(s_second, xs16[r * per_row + 2 * G + 1], off[1][r]);
         }
-    }
+    }, std::make_integer_sequence<int, 8>{});
+    const float d = h2f(t.d);
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const float d = h2f(t.d[c]);
+    for (int half = 0; half < 2; ++half)
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[c][r] = fmaf(d, fmaf(-32.0f, off[c][r], 0.0625f * part[c][r]), acc[c][r]);
-    }
-}
-
-// adds the two k-halves and hands every lane the sum of its own column
-template <int R>
-__device__ __forceinline__ void q6_gather(const float (&acc2)[2][R], uint32_t lane, float (&acc)[R]) {
-    const uint32_t src = 32u * (lane >> 5) + (lane & 15u);  // lane (j, group 2*(q/2)) holds column 16q + j as a (q even) or b
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float a = acc2[0][r] + __shfl_xor(acc2[0][r], 16, kWave);
-        const float b = acc2[1][r] + __shfl_xor(acc2[1][r], 16, kWave);
-        const float ga = __shfl(a, src, kWave), gb = __shfl(b, src, kWave);
-        acc[r] = ((lane >> 4) & 1u) ? gb : ga;
-    }
+        for (int r = 0; r < R; ++r) acc[half][r] = fmaf(d, fmaf(-32.0f, off[half][r], 0.0625f * part[half][r]), acc[half][r]);
 }
 
 // =======================================================================================
@@ -299,43 +270,45 @@ __device__ __forceinline__ void run_blocks_at(const uint8_t* __restrict__ tiles,
     // lane (i = lane % 16, s = lane / 16) of the A operand: variant i % 4, k-slice s
     const uint8_t* image = blob + L.image_off + (lane & 3u) * 64u + (lane >> 4) * 16u;
     const uint32_t ob1 = ob0 + count;
-    if constexpr (DTYPE == GUFFIN_Q4_K) {
-        // the first block's operand (a hit in the caches) is requested ahead of the weight tiles, which
-        // come from HBM: behind them it would cost every wave a second trip before its first product
-        Q4Tile cur, nxt;
-        Q4Operand op;
-        if (count) { load_operand(op, image + size_t(ob0) * 2048u); load_tile(cur, tp); }
-        for (uint32_t b = ob0; b < ob1; ++b) {
-            if (b + 1 < ob1) load_tile(nxt, tp + size_t(b + 1 - ob0) * TB);
-            if (b != ob0) load_operand(op, image + size_t(b) * 2048u);
-            compute_tile<R>(cur, op, mult + b * 8u, K / 32, xs + b * 8u, per_row, lane >> 4, acc);
-            cur = nxt;
+    if constexpr (DTYPE != GUFFIN_Q8_0) {
+        using Tile = std::conditional_t<DTYPE == GUFFIN_Q4_K, Q4Tile, Q6Tile>;
+        constexpr uint32_t xs_block = DTYPE == GUFFIN_Q4_K ? 8 : 16;
+        const uint8_t* im = blob + L.image_off + operand_lane(lane);
+        float halves[2][R];   // Q6_K
+        auto product = [&](const Tile& t, const BlockOperand& o, uint32_t b) {
+            const float *mb = mult + b * 8u, *xb = xs + b * xs_block;
+            if constexpr (DTYPE == GUFFIN_Q6_K) compute_tile<R>(t, o, mb, K / 32, xb, per_row, halves);
+            else compute_tile<R>(t, o, mb, K / 32, xb, per_row, acc);
+        };
+        if constexpr (DTYPE == GUFFIN_Q6_K) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) halves[0][r] = halves[1][r] = 0.f;
         }
-    } else if constexpr (DTYPE == GUFFIN_Q6_K) {
-        // A rows 0-3 / 8-11 see the first 16 elements of a group, rows 4-7 / 12-15 the second 16
-        const uint32_t keep = (((lane & 15u) >> 2) & 1u) == (lane >> 5) ? 0xFFFFFFFFu : 0u;
-        float acc2[2][R];
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int r = 0; r < R; ++r) acc2[c][r] = 0.f;
-        // (this tile and its operand together do not fit the registers: the operand is read group by group)
+        // a block's operand (a hit in the caches) is requested ahead of its weight tile, which comes from HBM:
+        // behind it it would cost the wave a second trip before its first product
         if constexpr (SINGLE) {  // one tile in registers at a time: 16 waves fit a workgroup
             for (uint32_t b = ob0; b < ob1; ++b) {
-                Q6Tile cur;
-                load_tile<false>(cur, tp + size_t(b - ob0) * TB, lane);
-                compute_tile<R>(cur, image + size_t(b) * 2048u, keep, mult + b * 8u, K / 32, xs + b * 16u, per_row, lane, acc2);
+                Tile cur;
+                BlockOperand op;
+                load_operand(op, im + size_t(b) * 2048u);
+                load_tile(cur, tiles + size_t(b - ob0) * TB, lane);
+                product(cur, op, b);
             }
         } else {
-            Q6Tile cur, nxt;
-            if (count) load_tile<true>(cur, tp, lane);
+            Tile cur, nxt;
+            BlockOperand op, on;
+            if (count) { load_operand(op, im + size_t(ob0) * 2048u); load_tile(cur, tiles, lane); }
             for (uint32_t b = ob0; b < ob1; ++b) {
-                if (b + 1 < ob1) load_tile<true>(nxt, tp + size_t(b + 1 - ob0) * TB, lane);
-                compute_tile<R>(cur, image + size_t(b) * 2048u, keep, mult + b * 8u, K / 32, xs + b * 16u, per_row, lane, acc2);
+                if (b + 1 < ob1) { load_operand(on, im + size_t(b + 1) * 2048u); load_tile(nxt, tiles + size_t(b + 1 - ob0) * TB, lane); }
+                product(cur, op, b);
                 cur = nxt;
+                op = on;
             }
         }
-        q6_gather<R>(acc2, lane, acc);
+        if constexpr (DTYPE == GUFFIN_Q6_K) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[r] = halves[0][r] + halves[1][r];
+        }
     } else {
         Q8Tile cur, nxt;
         auto operand = [&](uint32_t b) { return __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(image + size_t(b) * 256u)); };
