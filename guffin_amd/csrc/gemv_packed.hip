@@ -38,6 +38,8 @@
 #include "receipt.hpp"
 #include "gemv_tiles.hpp"
 
+#include <algorithm>
+
 namespace guffin {
 namespace {
 
@@ -73,10 +75,11 @@ __device__ __forceinline__ uint32_t tile_offset(uint32_t o, uint32_t l) {
     }
 }
 
-// Canonical stream -> tiles.  A workgroup takes 64 columns x up to kRepackBlocks blocks: every column's run of blocks is read
+// Canonical stream -> tiles.  A workgroup takes 64 columns x up to repack_blocks blocks: every column's run of blocks is read
 // as the consecutive dwords it is and laid out in LDS one block after the other, then the tiles are written in 16-byte
 // pieces, lane after lane, so both sides move whole lines.  (One thread per 16-bit word, scattered over the tile's lines,
-// reached 1.5 TB/s on 15360 x 3840 Q6_K.)  grid (N / 64, ceil(nblk / blocks)), 256 threads.
+// reached 1.5 TB/s on 15360 x 3840 Q6_K.)  grid (N / 64, ceil(nblk / per)), 256 threads; `per` blocks, at most repack_blocks.
+// Matrices that would leave CUs idle take fewer blocks a workgroup: a workgroup's time is its walk over its blocks.
 constexpr uint32_t repack_blocks(int dtype) { return dtype == GUFFIN_Q8_0 ? 16 : dtype == GUFFIN_Q4_K ? 4 : 2; }
 // a block in LDS: an odd number of dwords, so that 64 columns fall on different banks; a Q8_0 block starts 2 bytes in, which
 // puts its quants on dword boundaries
@@ -85,12 +88,12 @@ struct __attribute__((packed, aligned(2))) U1a2 { uint32_t x; };
 
 template <int DTYPE>
 __global__ void __launch_bounds__(256)
-repack_tiles_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t nblk) {
+repack_tiles_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t nblk, uint32_t per) {
     constexpr uint32_t BB = block_bytes(DTYPE), NB = repack_blocks(DTYPE), PITCH = repack_pitch(DTYPE), TB = kTileCols * BB;
     // dwords of a block from byte `SKIP` on; what is left (Q8_0's d in front, Q6_K's d behind) is one 16-bit word
     constexpr uint32_t DW = BB / 4, SKIP = DTYPE == GUFFIN_Q8_0 ? 2 : 0, UNITS = DW + (BB % 4 ? 1 : 0);
     __shared__ uint32_t lds[kTileCols * NB * PITCH];
-    const uint32_t b0 = blockIdx.y * NB, nb = min(NB, nblk - b0);
+    const uint32_t b0 = blockIdx.y * per, nb = min(per, nblk - b0);
     const uint8_t* base = src + (size_t(blockIdx.x) * kTileCols * nblk + b0) * BB;
     constexpr int AHEAD = 8;
     const uint32_t units = kTileCols * nb * UNITS;
@@ -411,8 +414,9 @@ static int repack_common(void* stream, int dtype, const void* src, void* dst, ui
     if (to_tiles) {
         const uint8_t* from = static_cast<const uint8_t*>(src);
         uint8_t* to = static_cast<uint8_t*>(dst);
-#define GUFFIN_REPACK(DT) \
-        launch(repack_tiles_kernel<DT>, dim3(N / kTileCols, (nblk + repack_blocks(DT) - 1) / repack_blocks(DT)), dim3(256), 0, s, from, to, nblk)
+        const uint32_t tiles = N / kTileCols, wgs = 2 * uint32_t(g_cus);   // two workgroups a CU, if the matrix has that many blocks
+        const uint32_t per = std::clamp(static_cast<uint32_t>((uint64_t(tiles) * nblk + wgs - 1) / wgs), 1u, repack_blocks(dtype));
+#define GUFFIN_REPACK(DT) launch(repack_tiles_kernel<DT>, dim3(tiles, (nblk + per - 1) / per), dim3(256), 0, s, from, to, nblk, per)
         if (dtype == GUFFIN_Q4_K) GUFFIN_REPACK(GUFFIN_Q4_K);
         else if (dtype == GUFFIN_Q6_K) GUFFIN_REPACK(GUFFIN_Q6_K);
         else GUFFIN_REPACK(GUFFIN_Q8_0);
