@@ -30,7 +30,6 @@ int check_launch(const char* what) {
 int gemv_init(int cu_count);
 int ops_init(int cu_count);
 int gemv_packed_init(int device, int cu_count);
-int gemv_wide_init();
 int head_init();
 
 }  // namespace guffin
@@ -57,7 +56,7 @@ extern "C" int guffin_hip_init(int device) {
     if (gemv_init(prop.multiProcessorCount) != 0 || ops_init(prop.multiProcessorCount) != 0 || head_init() != 0)
         return fail(GUFFIN_E_HIP, "init: could not raise a kernel's dynamic LDS limit");
     resident_init(prop.multiProcessorCount);
-    if (gemv_packed_init(device, prop.multiProcessorCount) != 0 || gemv_wide_init() != 0)
+    if (gemv_packed_init(device, prop.multiProcessorCount) != 0)
         return fail(GUFFIN_E_HIP, "init: could not take the address of the static scratch array on this device");
     return GUFFIN_OK;
 }

@@ -25,9 +25,9 @@
 // (sixteen column groups of 4 side by side, no repeated A rows), a lane owning one column from its quants to its sum: no
 // selection among column groups (128 of 496 vector instructions of a Q4_K tile), no masked half-groups and lane exchanges
 // for Q6_K, and the operand of a 256-element block in 8 registers instead of 32, so it is requested ahead of every tile.
-// With the 16x16x32 form / now (us): gate + up 3840 -> 15360 on two rows 17.3 / 15.2, on one 16.2 / 14.5, down
-// 15360 -> 3840 on two rows 13.0 / 11.3, q/k/v 8.2 / 7.4: what a launch streams does not change, its unpack is what
-// does not overlap.  Block scales are applied to the per-group sums in fp32 by the lane that owns the
+// With the 16x16x32 form / now (us): gate + up 3840 -> 15360 on two rows 17.3 / 15.2, on one 16.2 / 14.6, down
+// 15360 -> 3840 on two rows 13.0 / 10.8, q/k/v 8.2 / 7.2, the 262144-row Q6_K head 143 / 130: what a launch streams does
+// not change, its unpack is what does not overlap.  Block scales are applied to the per-group sums in fp32 by the lane that owns the
 // column; the offset terms (-dmin*m for Q4_K, -32 for Q6_K, -128 for the biased Q8_0 bytes)
 // use the receipt's 16- / 32-sums.  K is cut into slices: up to 16 slices are the waves of
 // one workgroup, combined in wave order through LDS; the remaining S "planes" go to
@@ -242,7 +242,7 @@ gemv_q6k_single_kernel(const uint8_t* __restrict__ wt, const float* __restrict__
     const uint32_t slice = blockIdx.y * c.W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t b0 = min(slice, c.nblk), b1 = min(b0 + 1u, c.nblk);
     float acc[R];
-    run_blocks<GUFFIN_Q6_K, R, true>(wt, x, xsums, c.K, c.nblk, blockIdx.x, b0, b1, acc);
+    run_blocks<GUFFIN_Q6_K, R, kWalkOne>(wt, x, xsums, c.K, c.nblk, blockIdx.x, b0, b1, acc);
     finish_tile<R>(acc, part, N, blockIdx.x, blockIdx.y, c.W);
 }
 

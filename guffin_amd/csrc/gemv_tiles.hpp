@@ -69,13 +69,22 @@ __device__ __forceinline__ half8_t as_half8(uint32_t a, uint32_t b, uint32_t c, 
     return __builtin_bit_cast(half8_t, make_uint4(a, b, c, d));
 }
 
-// The operand of a 256-element block: groups 2p and 2p + 1 in a[p], A-side block 8 (g % 2) + i holding elements 4i .. 4i + 3 of
-// group g.  image: this block's 8 groups of the activation image, already offset for this lane.
-struct BlockOperand { half4_t a[4]; };
-__device__ __forceinline__ uint32_t operand_lane(uint32_t lane) { return (lane >> 5) * 256u + (lane & 3u) * 64u + ((lane >> 2) & 7u) * 8u; }
-__device__ __forceinline__ void load_operand(BlockOperand& o, const uint8_t* __restrict__ image) {
+// The operand of a 256-element block: groups 2p and 2p + 1 in a[set][p], A-side block 8 (g % 2) + i holding elements 4i .. 4i + 3
+// of group g; one set of four variants for up to two rows, two for three and four.  image: this block's 8 groups of the activation
+// image, already offset for this lane.
+constexpr int operand_sets(int rows) { return rows > 2 ? 2 : 1; }
+template <int R> struct BlockOperand { half4_t a[operand_sets(R)][4]; };
+template <int R>
+__device__ __forceinline__ uint32_t operand_lane(uint32_t lane) {
+    return (lane >> 5) * (256u * operand_sets(R)) + (lane & 3u) * 64u + ((lane >> 2) & 7u) * 8u;
+}
+template <int R>
+__device__ __forceinline__ void load_operand(BlockOperand<R>& o, const uint8_t* __restrict__ image) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) o.a[p] = __builtin_bit_cast(half4_t, *reinterpret_cast<const uint2*>(image + 512 * p));
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int set = 0; set < operand_sets(R); ++set)
+            o.a[set][p] = __builtin_bit_cast(half4_t, *reinterpret_cast<const uint2*>(image + 512 * operand_sets(R) * p + 256 * set));
 }
 template <int BLOCK>
 __device__ __forceinline__ float4_t mac4(half4_t a, uint32_t b0, uint32_t b1, float4_t c) {
@@ -86,7 +95,7 @@ __device__ __forceinline__ void each_slice(F f, std::integer_sequence<int, I...>
 
 // mult / xs32: this block's 8 multipliers / 32-sums of row 0 (rows `per_mult` / `per_row` apart)
 template <int R>
-__device__ __forceinline__ void compute_tile(const Q4Tile& t, const BlockOperand& op,
+__device__ __forceinline__ void compute_tile(const Q4Tile& t, const BlockOperand<R>& op,
                                              const float* __restrict__ mult, uint32_t per_mult,
                                              const float* __restrict__ xs32, uint32_t per_row, float (&acc)[R]) {
     const float d = h2f(t.hdr.x & 0xFFFFu), dmin = h2f(t.hdr.x >> 16);
@@ -101,7 +110,9 @@ __device__ __forceinline__ void compute_tile(const Q4Tile& t, const BlockOperand
     const float4_t zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ch = 0; ch < 4; ++ch) {  // 32-byte chunk: sub-blocks 2ch (low nibbles) and 2ch+1 (high)
-        float4_t lo = zero, hi = zero;
+        float4_t lo[operand_sets(R)], hi[operand_sets(R)];
+#pragma unroll
+        for (int set = 0; set < operand_sets(R); ++set) lo[set] = hi[set] = zero;
         each_slice([&](auto slice) {
             constexpr int S = slice;
             const uint4 piece = t.q[4 * (ch >> 1) + S];
@@ -112,10 +123,18 @@ __device__ __forceinline__ void compute_tile(const Q4Tile& t, const BlockOperand
             // the same; the high ones further up would take one more shift per word.  Both in bits 4-7: rms error on
             // activations with a 512-fold range, K = 3840, 5.2e-7 of the result's rms.)
             constexpr uint32_t L = 0x07800780u, M = 0x00F000F0u;
-            lo = mac4<2 * S>(op.a[ch], (w0 << 7) & L, (w0 >> 1) & L, lo);
-            hi = mac4<8 + 2 * S>(op.a[ch], w0 & M, (w0 >> 8) & M, hi);
-            lo = mac4<2 * S + 1>(op.a[ch], (w1 << 7) & L, (w1 >> 1) & L, lo);
-            hi = mac4<8 + 2 * S + 1>(op.a[ch], w1 & M, (w1 >> 8) & M, hi);
+            const uint32_t l[4] = {(w0 << 7) & L, (w0 >> 1) & L, (w1 << 7) & L, (w1 >> 1) & L};
+            const uint32_t u[4] = {w0 & M, (w0 >> 8) & M, w1 & M, (w1 >> 8) & M};
+#pragma unroll
+            for (int set = 0; set < operand_sets(R); ++set) {
+                lo[set] = mac4<2 * S>(op.a[set][ch], l[0], l[1], lo[set]);
+                hi[set] = mac4<8 + 2 * S>(op.a[set][ch], u[0], u[1], hi[set]);
+            }
+#pragma unroll
+            for (int set = 0; set < operand_sets(R); ++set) {
+                lo[set] = mac4<2 * S + 1>(op.a[set][ch], l[2], l[3], lo[set]);
+                hi[set] = mac4<8 + 2 * S + 1>(op.a[set][ch], u[2], u[3], hi[set]);
+            }
         }, std::make_integer_sequence<int, 4>{});
         const uint32_t scw = ch < 2 ? sc_a : sc_b, mnw = ch < 2 ? mn_a : mn_b;
         const float sc_lo = (ch & 1) ? ub2(scw) : ub0(scw), sc_hi = (ch & 1) ? ub3(scw) : ub1(scw);
@@ -124,8 +143,8 @@ __device__ __forceinline__ void compute_tile(const Q4Tile& t, const BlockOperand
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const float m_lo = mult[r * per_mult + 2 * ch], m_hi = mult[r * per_mult + 2 * ch + 1];
-            acc[r] = fmaf(f_lo * m_lo, lo[2 * r] + lo[2 * r + 1], acc[r]);
-            acc[r] = fmaf(f_hi * m_hi, hi[2 * r] + hi[2 * r + 1], acc[r]);
+            acc[r] = fmaf(f_lo * m_lo, lo[r >> 1][2 * (r & 1)] + lo[r >> 1][2 * (r & 1) + 1], acc[r]);
+            acc[r] = fmaf(f_hi * m_hi, hi[r >> 1][2 * (r & 1)] + hi[r >> 1][2 * (r & 1) + 1], acc[r]);
             mt[r] = fmaf(mn_lo, xs32[r * per_row + 2 * ch], mt[r]);
             mt[r] = fmaf(mn_hi, xs32[r * per_row + 2 * ch + 1], mt[r]);
         }
@@ -158,7 +177,7 @@ __device__ __forceinline__ float sbyte(uint32_t w, int i) {
 }
 
 template <int R>
-__device__ __forceinline__ void compute_tile(const Q6Tile& t, const BlockOperand& op,
+__device__ __forceinline__ void compute_tile(const Q6Tile& t, const BlockOperand<R>& op,
                                              const float* __restrict__ mult, uint32_t per_mult,
                                              const float* __restrict__ xs16, uint32_t per_row, float (&acc)[2][R]) {
     const float4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -167,7 +186,9 @@ __device__ __forceinline__ void compute_tile(const Q6Tile& t, const BlockOperand
     for (int r = 0; r < R; ++r) part[0][r] = part[1][r] = off[0][r] = off[1][r] = 0.f;
     each_slice([&](auto group) {  // 32-element group: half n, quadrant qd
         constexpr int G = group, n = G >> 2, qd = G & 3, ls = qd >= 2 ? 4 : 0, AT = 8 * (G & 1);
-        float4_t first = zero, second = zero;
+        float4_t first[operand_sets(R)], second[operand_sets(R)];
+#pragma unroll
+        for (int set = 0; set < operand_sets(R); ++set) first[set] = second[set] = zero;
         auto slice_operand = [&](int s, uint32_t (&b)[4]) {
             const uint4 lq = t.ql[4 * n + s], hq = t.qh[s];
             const uint32_t w[2] = {(qd & 1) ? lq.z : lq.x, (qd & 1) ? lq.w : lq.y};
@@ -187,18 +208,24 @@ __device__ __forceinline__ void compute_tile(const Q6Tile& t, const BlockOperand
             uint32_t b[4], c[4];
             slice_operand(S, b);
             slice_operand(S + 2, c);
-            first = mac4<AT + 2 * S>(op.a[G >> 1], b[0], b[1], first);
-            second = mac4<AT + 2 * S + 4>(op.a[G >> 1], c[0], c[1], second);
-            first = mac4<AT + 2 * S + 1>(op.a[G >> 1], b[2], b[3], first);
-            second = mac4<AT + 2 * S + 5>(op.a[G >> 1], c[2], c[3], second);
+#pragma unroll
+            for (int set = 0; set < operand_sets(R); ++set) {
+                first[set] = mac4<AT + 2 * S>(op.a[set][G >> 1], b[0], b[1], first[set]);
+                second[set] = mac4<AT + 2 * S + 4>(op.a[set][G >> 1], c[0], c[1], second[set]);
+            }
+#pragma unroll
+            for (int set = 0; set < operand_sets(R); ++set) {
+                first[set] = mac4<AT + 2 * S + 1>(op.a[set][G >> 1], b[2], b[3], first[set]);
+                second[set] = mac4<AT + 2 * S + 5>(op.a[set][G >> 1], c[2], c[3], second[set]);
+            }
         }, std::make_integer_sequence<int, 2>{});
         const uint32_t wv = (G >> 1) == 0 ? t.sc.x : (G >> 1) == 1 ? t.sc.y : (G >> 1) == 2 ? t.sc.z : t.sc.w;
         const float s_first = sbyte(wv, 2 * (G & 1)), s_second = sbyte(wv, 2 * (G & 1) + 1);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const float m = mult[r * per_mult + G];
-            part[0][r] = fmaf(s_first * m, first[2 * r] + first[2 * r + 1], part[0][r]);
-            part[1][r] = fmaf(s_second * m, second[2 * r] + second[2 * r + 1], part[1][r]);
+            part[0][r] = fmaf(s_first * m, first[r >> 1][2 * (r & 1)] + first[r >> 1][2 * (r & 1) + 1], part[0][r]);
+            part[1][r] = fmaf(s_second * m, second[r >> 1][2 * (r & 1)] + second[r >> 1][2 * (r & 1) + 1], part[1][r]);
             off[0][r] = fmaf(s_first, xs16[r * per_row + 2 * G], off[0][r]);
             off[1][r] = fmaf(s_second, xs16[r * per_row + 2 * G + 1], off[1][r]);
         }
@@ -253,7 +280,10 @@ __device__ __forceinline__ void compute_tile(const Q8Tile& t, const half8_t a,
 // One wave: `count` consecutive blocks of one column tile, the first at `tiles` (its 64 x block bytes),
 // against the operand blocks ob0 .. ob0 + count - 1 of the receipt `xsums` (a blob laid out for R rows
 // of K activations, in global memory or in LDS); returns the per-lane column sums.
-template <int DTYPE, int R, bool SINGLE = false>
+// How a wave walks its blocks.  Ahead: the next block's tile and operand are requested before a block's products (two tiles in
+// registers).  One: the run has at most one block.  Serial: one tile in registers at a time.
+constexpr int kWalkAhead = 0, kWalkOne = 1, kWalkSerial = 2;
+template <int DTYPE, int R, int WALK = kWalkAhead>
 __device__ __forceinline__ void run_blocks_at(const uint8_t* __restrict__ tiles, const float* __restrict__ xsums,
                                               uint32_t K, uint32_t ob0, uint32_t count, float (&acc)[R],
                                               uint32_t lane = threadIdx.x & 63) {
@@ -273,9 +303,10 @@ __device__ __forceinline__ void run_blocks_at(const uint8_t* __restrict__ tiles,
     if constexpr (DTYPE != GUFFIN_Q8_0) {
         using Tile = std::conditional_t<DTYPE == GUFFIN_Q4_K, Q4Tile, Q6Tile>;
         constexpr uint32_t xs_block = DTYPE == GUFFIN_Q4_K ? 8 : 16;
-        const uint8_t* im = blob + L.image_off + operand_lane(lane);
+        constexpr uint32_t image_block = 2048u * operand_sets(R);
+        const uint8_t* im = blob + L.image_off + operand_lane<R>(lane);
         float halves[2][R];   // Q6_K
-        auto product = [&](const Tile& t, const BlockOperand& o, uint32_t b) {
+        auto product = [&](const Tile& t, const BlockOperand<R>& o, uint32_t b) {
             const float *mb = mult + b * 8u, *xb = xs + b * xs_block;
             if constexpr (DTYPE == GUFFIN_Q6_K) compute_tile<R>(t, o, mb, K / 32, xb, per_row, halves);
             else compute_tile<R>(t, o, mb, K / 32, xb, per_row, acc);
@@ -286,23 +317,43 @@ __device__ __forceinline__ void run_blocks_at(const uint8_t* __restrict__ tiles,
         }
         // a block's operand (a hit in the caches) is requested ahead of its weight tile, which comes from HBM:
         // behind it it would cost the wave a second trip before its first product
-        if constexpr (SINGLE) {  // one tile in registers at a time: 16 waves fit a workgroup
+        if constexpr (WALK == kWalkSerial) {
             for (uint32_t b = ob0; b < ob1; ++b) {
                 Tile cur;
-                BlockOperand op;
-                load_operand(op, im + size_t(b) * 2048u);
+                BlockOperand<R> op;
+                load_operand<R>(op, im + size_t(b) * image_block);
                 load_tile(cur, tiles + size_t(b - ob0) * TB, lane);
                 product(cur, op, b);
             }
+        } else if (WALK == kWalkOne || count <= 1) {
+            if (count) {
+                Tile only;
+                BlockOperand<R> op;
+                load_operand<R>(op, im + size_t(ob0) * image_block);
+                load_tile(only, tiles, lane);
+                product(only, op, ob0);
+            }
         } else {
-            Tile cur, nxt;
-            BlockOperand op, on;
-            if (count) { load_operand(op, im + size_t(ob0) * 2048u); load_tile(cur, tiles, lane); }
-            for (uint32_t b = ob0; b < ob1; ++b) {
-                if (b + 1 < ob1) { load_operand(on, im + size_t(b + 1) * 2048u); load_tile(nxt, tiles + size_t(b + 1 - ob0) * TB, lane); }
-                product(cur, op, b);
-                cur = nxt;
-                op = on;
+            // Two tiles by name, the next block's requests always in front of a block's products: behind a branch the compiler has
+            // to count as if they had not been made, and a block waits for the next one's tile; copied from one name to the
+            // other, it waits for all of it.  Past the last block every lane asks for the same words of the first.
+            Tile even, odd;
+            BlockOperand<R> even_op, odd_op;
+            auto request = [&](Tile& t, BlockOperand<R>& o, uint32_t b) {
+                const bool there = b < ob1;
+                const uint32_t at = there ? b : ob0, l = there ? lane : 0u;
+                load_operand<R>(o, blob + L.image_off + operand_lane<R>(l) + size_t(at) * image_block);
+                load_tile(t, tiles + size_t(at - ob0) * TB, l);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            request(even, even_op, ob0);
+            for (uint32_t b = ob0;; b += 2) {
+                request(odd, odd_op, b + 1);
+                product(even, even_op, b);
+                if (b + 1 >= ob1) break;
+                request(even, even_op, b + 2);
+                product(odd, odd_op, b + 1);
+                if (b + 2 >= ob1) break;
             }
         }
         if constexpr (DTYPE == GUFFIN_Q6_K) {
@@ -366,12 +417,12 @@ __device__ __forceinline__ void run_blocks_ahead(const Q8Ahead& ahead, const uin
 }
 
 // One wave: blocks [b0, b1) of column tile `ct` of a whole matrix whose operand is the receipt of its K inputs.
-template <int DTYPE, int R, bool SINGLE = false>
+template <int DTYPE, int R, int WALK = kWalkAhead>
 __device__ __forceinline__ void run_blocks(const uint8_t* __restrict__ wt, const float* __restrict__ x,
                                            const float* __restrict__ xsums, uint32_t K, uint32_t nblk,
                                            uint32_t ct, uint32_t b0, uint32_t b1, float (&acc)[R]) {
     constexpr uint32_t TB = kTileCols * block_bytes(DTYPE);
-    run_blocks_at<DTYPE, R, SINGLE>(wt + (size_t(ct) * nblk + b0) * TB, xsums, K, b0, b1 > b0 ? b1 - b0 : 0u, acc);
+    run_blocks_at<DTYPE, R, WALK>(wt + (size_t(ct) * nblk + b0) * TB, xsums, K, b0, b1 > b0 ? b1 - b0 : 0u, acc);
 }
 
 }  // namespace

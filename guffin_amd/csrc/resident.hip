@@ -216,7 +216,7 @@ __device__ __forceinline__ void wave_blocks(const Ctx& c, uint32_t dtype, const 
         if (dtype == GUFFIN_Q4_K) {
             run_blocks_at<GUFFIN_Q4_K, R>(tiles, opnd, K, ob0, count, acc, lane);
         } else {
-            run_blocks_at<GUFFIN_Q6_K, R, true>(tiles, opnd, K, ob0, count, acc, lane);
+            run_blocks_at<GUFFIN_Q6_K, R, kWalkSerial>(tiles, opnd, K, ob0, count, acc, lane);
         }
     } else {
         run_blocks_at<GUFFIN_Q8_0, R>(tiles, opnd, K, ob0, count, acc, lane);

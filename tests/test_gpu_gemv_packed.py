@@ -285,3 +285,25 @@ def test_packed_rejects_bad_arguments(hip):
                         torch.zeros((3, 24), dtype=torch.float32, device="cuda"), 64)
     with pytest.raises(hip.GuffinError):
         hip.gemv_packed(1, w[8:], x, torch.zeros((1, 24), dtype=torch.float32, device="cuda"), 64)
+
+
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("blocks", [1, 2, 3, 5])
+@pytest.mark.parametrize("rows", [1, 2])
+def test_waves_that_walk_one_to_five_blocks(hip, gfo, dtype, blocks, rows):
+    """So many column tiles that a wave takes whole runs of blocks: odd and even counts, and the last, shorter run.  Bound: 24 fp32
+    roundings of the sum of absolute products (4 adds a matrix instruction's chain, the group sums, the walk)."""
+    K, tiles = 256 * blocks, 2600
+    N = 64 * tiles
+    w = np.tile(synth.make_weight(dtype, K, 320, seed=80 + blocks), tiles // 5)   # columns repeat every five tiles
+    x = synth.make_activation(rows, K, seed=81)
+    xd = dev(x)
+    y = hip.gemv_packed(dtype, hip.repack(dtype, dev(w), K, N), xd, hip.group_sums(xd), N).cpu().numpy().reshape(rows, tiles // 5, 320)
+    dense = gfo.dequant(dtype, w[:w.size // (tiles // 5)]).reshape(320, K).astype(np.float64)
+    want, weight = x.astype(np.float64) @ dense.T, np.abs(x).astype(np.float64) @ np.abs(dense).T
+    # Q6_K evaluates s (sum q x - 32 sum x): both terms round, |q| + 32 for |q - 32|
+    slack = 24 * 2.0 ** -24 * (weight if dtype == 1 else weight + 64 * np.abs(x).sum(1, keepdims=True) * np.abs(dense).max() / 32)
+    if dtype == 1:   # d sc sum q x - dmin m sum x apart until the end of a block: either is at most the largest weight times sum |x|
+        slack = slack + 24 * 2.0 ** -24 * 2 * np.abs(x).sum(1, keepdims=True) * np.abs(dense).max()
+    assert np.all(np.abs(y - want[:, None, :]) <= slack[:, None, :]), float(np.abs(y - want[:, None, :]).max())
+    assert np.array_equal(y, np.broadcast_to(y[:, :1], y.shape))   # equal columns, equal bits, wherever their tile lies
