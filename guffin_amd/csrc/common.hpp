@@ -61,9 +61,9 @@ int gateup_wide(hipStream_t s, int dtype, const void* gate_tiles, const void* up
 // ---- K/V rows of every block of a model between its rings and a flat block of rows (prefill.hip) ---------------
 // flat_k / flat_v: [layer][flat_rows][kv width], position p in row p & (flat_rows - 1), flat_rows a power of two.  Save and
 // Restore copy positions [first, first + count); Publish saves them and then puts row path[i] of the private rows
-// [layer][priv_rows][kv width] at position first + i.
-enum class KvMove { Save, Restore, Publish };
-constexpr uint32_t kMovePath = 8;   // rows a Publish may take
+// [layer][priv_rows][kv width] at position first + i; Put does that without saving (no flat block).
+enum class KvMove { Save, Restore, Publish, Put };
+constexpr uint32_t kMovePath = 8;   // rows a Publish or Put may take
 int kv_move_rows(hipStream_t s, const guffin_model_desc& m, KvMove move, void* flat_k, void* flat_v, uint32_t flat_rows, uint32_t first,
                  uint32_t count, const void* priv_k = nullptr, const void* priv_v = nullptr, uint32_t priv_rows = 0,
                  const uint32_t* path = nullptr);

@@ -91,7 +91,7 @@ uint32_t max_tokens_for(const guffin_model_desc& m, uint32_t layer, uint32_t pos
     return position + rows;
 }
 
-Scratch layout(const guffin_model_desc& m, uint32_t rows, uint32_t position, uint8_t* base) {
+Scratch layout(const guffin_model_desc& m, uint32_t rows, uint32_t position, uint8_t* base, bool with_resident = true) {
     Arena ar {base, 0, 0};
     const uint32_t H = m.hidden, F = m.ffn, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
     Scratch s {};
@@ -132,7 +132,7 @@ Scratch layout(const guffin_model_desc& m, uint32_t rows, uint32_t position, uin
     s.positions = ar.take<uint32_t>(rows);
     s.ancestors = ar.take<uint32_t>(uint64_t(rows) * kMaxTreeSlots);   // a chain uses `rows` of them, a tree pass one list per row
     s.schedule = ar.take<uint32_t>(uint64_t(m.layer_count) * rows * 4);
-    if (resident_fits(m, rows)) {
+    if (with_resident && resident_fits(m, rows)) {
         s.exchange = ar.take<uint8_t>(resident_scratch_bytes(m, rows));
         s.sync_words = resident_sync_words(m);
         s.sync = ar.take<uint32_t>(s.sync_words);
@@ -646,6 +646,31 @@ PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, uint8_t
     return s;
 }
 
+// A run of up to four rows goes through the streaming products of a verify pass, which read the weights at the memory's rate,
+// and its K/V rows to the rings in one launch at the end.  12B shapes behind 700 tokens, us, with the tiled GEMMs / so: 2 rows
+// 5107 / 2966, 3 rows 5187 / 3531, 4 rows 5198 / 3602 (5 rows: 5221, two passes would take 6570).  For the models a tree pass covers, whose blocks'
+// matrices run in shared launches, and where the caller's arena (sized for the tiled form) holds the pass.
+struct ShortRun { uint16_t *priv_k, *priv_v; uint64_t bytes; };
+bool short_run_fits(const guffin_model_desc& m, uint32_t rows) {
+    if (rows > kWideRows || !tree_pass_fits(m) || g_forward_mode == 2 || resident_chosen(m, rows)) return false;
+    if (rows > m.ring_local || rows > m.ring_global || (m.global_period > 1 && m.sliding_window <= rows)) return false;
+    for (uint32_t l = 0; l < m.layer_count; ++l) {
+        const int32_t* d = m.layers[l].dtype;
+        auto length = [&](int i) { return d[i] == GUFFIN_Q8_0 ? 32u : 256u; };
+        if (length(0) != length(1) || length(0) != length(2) || length(4) != length(5)) return false;
+    }
+    return true;
+}
+ShortRun short_run_layout(const guffin_model_desc& m, uint32_t rows, uint32_t position, uint8_t* base) {
+    Arena ar {base, layout(m, rows, position, nullptr, false).bytes, 0};
+    const uint64_t words = uint64_t(m.layer_count) * rows * m.kv_heads * m.head_dim;
+    ShortRun r {};
+    r.priv_k = ar.take<uint16_t>(words);
+    r.priv_v = ar.take<uint16_t>(words);
+    r.bytes = ar.used;
+    return r;
+}
+
 __global__ void fill_positions_kernel(uint32_t* positions, uint32_t rows, uint32_t position) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < rows) positions[i] = position + i;
@@ -672,6 +697,18 @@ extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* mo
     const PrefillScratch s = prefill_layout(m, rows, static_cast<uint8_t*>(scratch));
     if (s.bytes > scratch_bytes) return fail(GUFFIN_E_CAPACITY, "prefill_rows: scratch arena too small");
     hipStream_t hs = as_stream(stream);
+    if (short_run_fits(m, rows)) {
+        uint8_t* base = static_cast<uint8_t*>(scratch);
+        const ShortRun r = short_run_layout(m, rows, position, base);
+        if (r.bytes <= scratch_bytes) {
+            for (uint32_t l = 0; l < m.layer_count; ++l)
+                if ((reinterpret_cast<uintptr_t>(m.layers[l].ring_k) | reinterpret_cast<uintptr_t>(m.layers[l].ring_v)) & 3u)
+                    return fail(GUFFIN_E_ALIGN, "prefill_rows: ring rows must be 4-byte aligned");
+            GUFFIN_TRY(forward_rows(hs, m, tokens, rows, position, layout(m, rows, position, base, false), r.priv_k, r.priv_v, out_hidden, nullptr, status));
+            const uint32_t path[kWideRows] = {0, 1, 2, 3};
+            return kv_move_rows(hs, m, KvMove::Put, nullptr, nullptr, 0, position, rows, r.priv_k, r.priv_v, rows, path);
+        }
+    }
     const uint32_t H = m.hidden, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
     const float attn_scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
     launch(fill_positions_kernel, dim3((rows + 255) / 256), dim3(256), 0, hs, s.positions, rows, position);

@@ -497,9 +497,11 @@ __global__ void kv_move_kernel(const MoveRings rings, U4a4* __restrict__ flat_k,
         *rk = flat_k[flat];
         *rv = flat_v[flat];
     } else {
-        flat_k[flat] = *rk;
-        flat_v[flat] = *rv;
-        if constexpr (MOVE == KvMove::Publish) {
+        if constexpr (MOVE != KvMove::Put) {
+            flat_k[flat] = *rk;
+            flat_v[flat] = *rv;
+        }
+        if constexpr (MOVE == KvMove::Publish || MOVE == KvMove::Put) {
             const size_t from = (size_t(layer) * priv_rows + path.row[t]) * row_vec + c;
             *rk = priv_k[from];
             *rv = priv_v[from];
@@ -513,10 +515,10 @@ int kv_move_rows(hipStream_t s, const guffin_model_desc& m, KvMove move, void* f
                  uint32_t count, const void* priv_k, const void* priv_v, uint32_t priv_rows, const uint32_t* path) {
     if (count == 0) return GUFFIN_OK;
     const uint32_t kvw = m.kv_heads * m.head_dim, row_vec = kvw / 8;
-    if (count > flat_rows || count > m.ring_local || count > m.ring_global)
+    if ((move != KvMove::Put && count > flat_rows) || count > m.ring_local || count > m.ring_global)
         return fail(GUFFIN_E_CAPACITY, "kv_move_rows: more rows than one side holds");
     MovePath rows {};
-    if (move == KvMove::Publish) {
+    if (move == KvMove::Publish || move == KvMove::Put) {
         if (count > kMovePath) return fail(GUFFIN_E_CAPACITY, "kv_move_rows: a path of at most 8 rows");
         for (uint32_t i = 0; i < count; ++i) rows.row[i] = path[i];
     }
@@ -536,12 +538,13 @@ int kv_move_rows(hipStream_t s, const guffin_model_desc& m, KvMove move, void* f
             if (layer_is_local(m.global_period, l0 + i)) r.local |= uint64_t{1} << i;
         }
         const size_t flat_at = size_t(l0) * flat_rows * row_vec, priv_at = size_t(l0) * priv_rows * row_vec;
-        U4a4 *fk = static_cast<U4a4*>(flat_k) + flat_at, *fv = static_cast<U4a4*>(flat_v) + flat_at;
+        U4a4 *fk = flat_k ? static_cast<U4a4*>(flat_k) + flat_at : nullptr, *fv = flat_v ? static_cast<U4a4*>(flat_v) + flat_at : nullptr;
         const U4a4 *pk = priv_k ? static_cast<const U4a4*>(priv_k) + priv_at : nullptr, *pv = priv_v ? static_cast<const U4a4*>(priv_v) + priv_at : nullptr;
         const dim3 grid((row_vec + 255) / 256, n, count), block(std::min(row_vec, 256u));
 #define GUFFIN_MOVE(M) launch(kv_move_kernel<M>, grid, block, 0, s, r, fk, fv, flat_rows, pk, pv, priv_rows, rows, first, m.ring_local - 1, m.ring_global - 1, row_vec)
         if (move == KvMove::Save) GUFFIN_MOVE(KvMove::Save);
         else if (move == KvMove::Restore) GUFFIN_MOVE(KvMove::Restore);
+        else if (move == KvMove::Put) GUFFIN_MOVE(KvMove::Put);
         else GUFFIN_MOVE(KvMove::Publish);
 #undef GUFFIN_MOVE
         if (int rc = check_launch("kv_move_rows")) return rc;

@@ -359,3 +359,40 @@ def test_prefill_rows_agree_with_decode_at_row_tile_edges(hip, kind, rows, posit
     for l in range(shape.layers):
         slot = (position + rows - 1) & (devm.ring_k[l].shape[0] - 1)
         assert float((devm.ring_k[l][slot] == pk[l, 0]).float().mean()) >= 0.95 and float((devm.ring_v[l][slot] == pv[l, 0]).float().mean()) >= 0.95
+
+
+@pytest.mark.parametrize("position", [0, 20, 95, 125, 200])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4])
+@pytest.mark.parametrize("kind", ["target", "mixed", "drafter"])
+def test_the_shortest_runs_agree_with_a_longer_one(hip, kind, rows, position):
+    """Runs of up to four rows take the verify pass' products where the model allows: their hidden rows and ring rows are those
+    of the first rows of a five-row run through the tiled GEMMs (2e-4 of the row RMS: fp32 sums in another order, and fp16 K/V
+    rows that may round the other way), and, on up to two rows of a model without a resident pass, the verify pass' bits."""
+    import torch
+    from dataclasses import replace
+    from guffin_amd import model
+    base = model.GEMMA3_270M if kind == "drafter" else model.GEMMA3_12B
+    shape = replace(base, layers=6, vocab=2048, ring_global=2048, ring_local=128, sliding_window=96)
+    if kind == "mixed":
+        shape = replace(shape, layer_dtypes=tuple(shape.dtypes if l % 2 == 0 else tuple(1 for _ in shape.dtypes) for l in range(6)))
+    host = model.HostModel(shape, seed=31, position=position)
+    short, long = model.DeviceModel.from_host(host), model.DeviceModel.from_host(host)
+    tokens = dev(np.random.default_rng(23).integers(0, shape.vocab, 5).astype(np.int32))
+    before = short.forward(tokens[:rows].contiguous(), position) if rows <= 2 else None
+    got, status = short.prefill(tokens[:rows].contiguous(), position)
+    want, status_long = long.prefill(tokens, position)
+    torch.cuda.synchronize()
+    assert int(status.item()) == 0 and int(status_long.item()) == 0
+    want = want[:rows].cpu().numpy().astype(np.float64)
+    assert np.all(np.abs(got.cpu().numpy() - want) <= 2e-4 * np.sqrt((want ** 2).mean(axis=1, keepdims=True)))
+    if before is not None and kind != "drafter":
+        assert torch.equal(got, before[0])
+    for l in range(shape.layers):
+        cap = short.ring_k[l].shape[0]
+        ours = [(position + r) & (cap - 1) for r in range(rows)]
+        theirs = [(position + r) & (cap - 1) for r in range(5)]
+        for mine, other in ((short.ring_k[l], long.ring_k[l]), (short.ring_v[l], long.ring_v[l])):
+            for s in ours:
+                assert float((mine[s] == other[s]).float().mean()) >= 0.95
+            rest = [s for s in range(cap) if s not in theirs]
+            assert torch.equal(mine[rest], other[rest])   # nothing else moves
