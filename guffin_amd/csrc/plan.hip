@@ -648,8 +648,8 @@ PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, uint8_t
 
 // A run of up to four rows goes through the streaming products of a verify pass, which read the weights at the memory's rate,
 // and its K/V rows to the rings in one launch at the end.  12B shapes behind 700 tokens, us, with the tiled GEMMs / so: 2 rows
-// 5107 / 2966, 3 rows 5187 / 3531, 4 rows 5198 / 3602 (5 rows: 5221, two passes would take 6570).  For the models a tree pass covers, whose blocks'
-// matrices run in shared launches, and where the caller's arena (sized for the tiled form) holds the pass.
+// 5107 / 2966, 3 rows 5187 / 3531, 4 rows 5198 / 3602 (5 rows: 5221, two passes would take 6570).  For the models a tree pass
+// covers, whose blocks' matrices run in shared launches, and where the caller's arena (sized for the tiled form) holds the pass.
 struct ShortRun { uint16_t *priv_k, *priv_v; uint64_t bytes; };
 bool short_run_fits(const guffin_model_desc& m, uint32_t rows) {
     if (rows > kWideRows || !tree_pass_fits(m) || g_forward_mode == 2 || resident_chosen(m, rows)) return false;
