@@ -334,26 +334,24 @@ __device__ __forceinline__ void run_blocks_at(const uint8_t* __restrict__ tiles,
                 product(only, op, ob0);
             }
         } else {
-            // Two tiles by name, the next block's requests always in front of a block's products: behind a branch the compiler has
-            // to count as if they had not been made, and a block waits for the next one's tile; copied from one name to the
-            // other, it waits for all of it.  Past the last block every lane asks for the same words of the first.
+            // Two tiles by name, and a copy of the products for the run's end: behind a branch around the next block's requests the
+            // compiler has to count as if they had not been made, and a block waits for the next one's tile; copied from one name
+            // to the other, it waits for all of it.
             Tile even, odd;
             BlockOperand<R> even_op, odd_op;
             auto request = [&](Tile& t, BlockOperand<R>& o, uint32_t b) {
-                const bool there = b < ob1;
-                const uint32_t at = there ? b : ob0, l = there ? lane : 0u;
-                load_operand<R>(o, blob + L.image_off + operand_lane<R>(l) + size_t(at) * image_block);
-                load_tile(t, tiles + size_t(at - ob0) * TB, l);
+                load_operand<R>(o, im + size_t(b) * image_block);
+                load_tile(t, tiles + size_t(b - ob0) * TB, lane);
                 __builtin_amdgcn_sched_barrier(0);
             };
             request(even, even_op, ob0);
-            for (uint32_t b = ob0;; b += 2) {
+            for (uint32_t b = ob0;; b += 2) {   // (two blocks at least)
                 request(odd, odd_op, b + 1);
                 product(even, even_op, b);
-                if (b + 1 >= ob1) break;
+                if (b + 2 >= ob1) { product(odd, odd_op, b + 1); break; }
                 request(even, even_op, b + 2);
                 product(odd, odd_op, b + 1);
-                if (b + 2 >= ob1) break;
+                if (b + 3 >= ob1) { product(even, even_op, b + 2); break; }
             }
         }
         if constexpr (DTYPE == GUFFIN_Q6_K) {
