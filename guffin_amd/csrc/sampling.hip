@@ -732,10 +732,13 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
     bool holds_proposal = false;
     uint64_t mass = 0;
     if (!rc && t < target.count) {
-        mass = q[t] = law_mass(q_law, full_cdf, vocab, target.token[t], nullptr, target_to_draft);
+        q[t] = law_mass(q_law, full_cdf, vocab, target.token[t], nullptr, target_to_draft);
+        // A mass is a difference of two edges: over edges out of order it wraps, and the sum of the masses may still be 2^32.
+        // Counted as at most 2^32 + 1 each, 256 of them cannot wrap, and their sum, which as one of whole numbers does not
+        // depend on the order, passes 2^32 exactly where some prefix does or some mass by itself.
+        mass = q[t] <= kMassTotal ? q[t] : kMassTotal + 1;
         holds_proposal = target.token[t] == proposal;
     }
-    // masses are whole numbers: their sum does not depend on the order, and it passes 2^32 where some prefix does
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mass += __shfl_xor(mass, o, kWave);
     if ((t & 63u) == 0) wave_mass[t >> 6] = mass;

@@ -34,6 +34,21 @@ def law_record(dtype, pairs, edit=None):
     return law
 
 
+# Edges of a law over three tokens whose last one is the whole: masses are differences of edges, so they always sum to it
+# modulo 2^64, however wrong the edges between are.  One above the total, one below its predecessor, one far above.
+INTERIOR_EDGES = ([0, TOTAL // 2, 2 * TOTAL, TOTAL], [0, TOTAL // 2, TOTAL // 4, TOTAL], [0, TOTAL // 2, U64_MAX - 7, TOTAL])
+INTERIOR_ROW = [(0, 0.5), (1, 0.25), (2, 0.0)]
+
+
+def interior_case(edges, draws):
+    """`edges` as the compact law of tokens 0, 1, 2, all of them in the target; the proposal's own mass is in order."""
+    def edit(law):
+        for i, edge in enumerate(edges):
+            law["cdf"][i] = edge
+    return dict(rows=[INTERIOR_ROW] * 2, history=[[], []], law=[(0, 1), (1, 1), (2, 1)], edit=edit, proposal=0,
+                options=(1.0, 3, 1.0, 0.0, 1.0), draws=draws, code=23)
+
+
 def uniform4():
     return [(t, TOTAL // 4) for t in range(4)]
 
@@ -134,6 +149,9 @@ def fault_cases():
     with_(1, options=(float("nan"), 2, 1.0, 0.0, 1.0))
     with_(1, options=(0.8, 2, 1.0, 0.0, 0.0))
     with_(2, rows=[[], []])
+    for edges in INTERIOR_EDGES:
+        for ua in (0.0, 0.99):   # what would be accepted and what would go to the residual
+            out.append(interior_case(edges, (ua, 0.5, 0.5)))
     return out
 
 

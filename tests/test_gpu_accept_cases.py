@@ -20,7 +20,7 @@ def hip():
     return module
 
 
-def device_run(hip, case, cdf=None):
+def device_run(hip, case, cdf=None, target_to_draft=None):
     import torch
     cands = np.zeros(2, hip.candidates_dtype)
     for r, row in enumerate(case["rows"]):
@@ -40,7 +40,10 @@ def device_run(hip, case, cdf=None):
     status = torch.zeros(1, dtype=torch.int32, device="cuda")
     proposal = torch.tensor([case["proposal"]], dtype=torch.int64, device="cuda").to(torch.int32)
     options = hip.SamplerOptions(*case["options"])
-    if cdf is not None:
+    if target_to_draft is not None:
+        out = hip.spec_accept_mapped(up(cands), up(law), target_to_draft, proposal, options, draws=up(draws), status=status, full_cdf=cdf,
+                                     vocab=0 if cdf is None else cdf.numel() - 1)
+    elif cdf is not None:
         out = hip.spec_accept_law(up(cands), up(law), cdf, proposal, options, draws=up(draws), status=status)
     else:
         out = hip.spec_accept_history(up(cands), up(law), up(hist), up(counts), proposal, options, draws=up(draws), status=status)
@@ -98,3 +101,24 @@ def test_sparse_target_against_a_32000_token_table(hip, gfo):
     case = dict(rows=[row, row], history=[[], []], law=[], edit=full, proposal=40000, options=o, draws=(0.3, 0.5, 0.5))
     got, status = device_run(hip, case, cdf_dev)
     assert int(got["status"]) == 22 and status & STATUS_LAW_INVALID
+
+
+@pytest.mark.parametrize("form", ["full", "mapped", "mapped_full"])
+def test_a_broken_edge_inside_a_law_is_refused_in_every_form(hip, form):
+    """The laws whose masses still sum to 2^32 (the compact form is among the fault cases; the oracle's answers are
+    tests/test_oracle_accept_cases.py's), each table also with its edges in order, which is decided."""
+    import torch
+    t2d = torch.arange(3, dtype=torch.int32, device="cuda") if form != "full" else None
+    for edges in cases.INTERIOR_EDGES + ([0, cases.TOTAL // 2, cases.TOTAL // 2, cases.TOTAL],):
+        for ua in (0.0, 0.99):
+            case = cases.interior_case(edges, (ua, 0.5, 0.5))
+            cdf = None
+            if form != "mapped":
+                cdf = torch.from_numpy(np.array(edges, np.uint64).view(np.int64)).cuda()
+                case["edit"] = lambda law: law.__setitem__("count", 0xFFFFFFFF)
+            got, status = device_run(hip, case, cdf, t2d)
+            if edges in cases.INTERIOR_EDGES:
+                assert int(got["status"]) == 23 and status & STATUS_LAW_INVALID, edges
+                assert int(got["accepted"]) == 0 and int(got["token"]) == 0xFFFFFFFF and int(got["next_root"]) == 0xFFFFFFFF
+            else:
+                assert int(got["status"]) == 0 and status == 0

@@ -63,3 +63,16 @@ def test_malformed_laws_rows_and_draws_fail_closed(gfo):
     for case in cases.fault_cases():
         rc, got = run(gfo, case)
         assert rc == -case["code"], (case.get("edit"), case["proposal"], case["draws"], case["options"], rc)
+
+
+@pytest.mark.parametrize("edges", cases.INTERIOR_EDGES)
+def test_a_broken_edge_inside_a_law_is_refused_in_every_form(gfo, edges):
+    """Full table, mapped compact law and mapped full table; the compact law is among the fault cases."""
+    row, options, draws = np.array(cases.INTERIOR_ROW, gfo.token_logit), gfo.SamplerOptions(1.0, 3, 1.0, 0.0, 1.0), (0.0, 0.5, 0.5)
+    cdf, t2d = np.array(edges, np.uint64), np.arange(3, dtype=np.int32)
+    assert gfo.spec_accept_full(row, row, cdf, 0, options, *draws)[0] == -23
+    assert gfo.spec_accept_full_mapped(row, row, cdf, t2d, 0, options, *draws)[0] == -23
+    case = cases.interior_case(edges, draws)
+    record = cases.law_record(np.dtype([("count", np.uint32), ("pad", np.uint32), ("ids", np.uint32, (256,)), ("cdf", np.uint64, (257,))]),
+                              case["law"], case["edit"])
+    assert gfo.spec_accept_mapped(row, (), row, (), gfo.DraftLaw.from_buffer_copy(record.tobytes()), t2d, 0, options, *draws)[0] == -23
