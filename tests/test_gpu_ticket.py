@@ -302,3 +302,23 @@ def test_a_tree_in_one_pass_equals_its_chains(hip, kind, parents, position):
         for (k, v), (bk, bv) in zip(zip(target.ring_k, target.ring_v), before):
             k.copy_(bk)
             v.copy_(bv)
+
+
+@pytest.mark.parametrize("parents", [(None, 0, 0), (None, 0, 1), (None, 0, 0, 1)])
+def test_a_tree_runs_in_every_forward_mode(hip, target, parents):
+    """The resident pass covers chains of one and two rows; trees run per operator, also where the resident pass is asked for."""
+    from guffin_amd import model
+    ticket = model.VerifyTicket(target, POSITION + 4)
+    tokens, before, got = [17, 1999, 42, 7][:len(parents)], rings(target), []
+    try:
+        for mode in (1, 2):
+            hip.set_forward_mode(mode)
+            ticket.encode_tree(tokens, list(parents), POSITION)
+            ticket.submit()
+            assert ticket.complete() == 0
+            got.append(ticket.read_candidates()[:len(tokens)])
+            ticket.discard()
+    finally:
+        hip.set_forward_mode(0)
+    assert np.array_equal(got[0]["count"], got[1]["count"]) and np.array_equal(got[0]["values"], got[1]["values"])
+    assert_rings(target, before)
