@@ -174,8 +174,10 @@ __device__ __forceinline__ void split_half8(const float (&x)[8], uint4& hi, uint
 struct AttentionOut { float* rows; uint8_t* image; float* part_o; float* part_ml; };
 constexpr float kProbScale = 1024.0f;   // probabilities enter the matrix instruction times 2^10
 constexpr float kLog2e = 1.44269504088896340736f;
-// scores are kept times log2(e), so that the exponential is one instruction (v_exp_f32, an ulp; it flushes what is below 2^-126)
-__device__ __forceinline__ float exp2_of(float x) { return __builtin_amdgcn_exp2f(x); }
+// e^x of a difference of scores: v_exp_f32 (an ulp; it flushes what is below 2^-126) behind a multiplication by log2(e).  That
+// stands here, where it costs the difference one rounding, and not at the queries, where every operand would be rounded once
+// more ahead of the product and lose half a bit of its range, nor at the maxima, whose rounding is not small beside large scores.
+__device__ __forceinline__ float exp_of(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
 // one (row, head): 8 consecutive output dimensions in 32 consecutive lanes
 __device__ __forceinline__ void emit_attention(const AttentionOut& to, const float (&v)[8], uint32_t row, uint32_t rows, uint32_t head,
@@ -243,8 +245,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         const uint32_t row = min(r0 + (m >> group_shift), rows - 1), head = kvh * group + (m & (group - 1));
         const float* src = q + (size_t(row) * q_heads + head) * HD + 8 * c8;
         const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
-        const float f = scale * kLog2e;
-        const float x[8] = {a.x * f, a.y * f, a.z * f, a.w * f, b.x * f, b.y * f, b.z * f, b.w * f};
+        const float x[8] = {a.x * scale, a.y * scale, a.z * scale, a.w * scale, b.x * scale, b.y * scale, b.z * scale, b.w * scale};
         uint4 hi, lo;
         split_half8(x, hi, lo);
         uint8_t* dst = qa + (((m >> 4) * 8 + c8 / 4) * 2) * 1024 + ((m & 15) + 16 * (c8 % 4)) * 16;
@@ -265,19 +266,27 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
     for (uint32_t ti = begin + wave; ti < end; ti += 4) {
         const uint32_t t0 = base32 + 32 * ti;
         if constexpr (NT > 1) ask_keys(ti, kb);
-        float4_t S[NT][2];
+        // A sum rounds at the size it has grown to: the hi halves of the first four steps are one chain; the other takes the lo
+        // halves, whose sums are small, and from the fifth step on both.
+        float4_t S[NT][2], rest[NT][2];
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks)
 #pragma unroll
-            for (int half = 0; half < 2; ++half)
+            for (int half = 1; half >= 0; --half)
 #pragma unroll
                 for (int g = 0; g < NT; ++g) {
                     const half8_t a = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(qa + ((g * 8 + ks) * 2 + half) * 1024 + lane * 16));
 #pragma unroll
-                    for (int c = 0; c < 2; ++c)
-                        S[g][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8_t, kb[c][ks]),
-                                                                         ks + half == 0 ? float4_t{0.f, 0.f, 0.f, 0.f} : S[g][c], 0, 0, 0);
+                    for (int c = 0; c < 2; ++c) {
+                        float4_t& sum = half == 0 && ks < 4 ? S[g][c] : rest[g][c];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8_t, kb[c][ks]),
+                                                                     ks == 0 ? float4_t{0.f, 0.f, 0.f, 0.f} : sum, 0, 0, 0);
+                    }
                 }
+#pragma unroll
+        for (int g = 0; g < NT; ++g)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) S[g][c] += rest[g][c];
         if constexpr (NT > 1) __builtin_amdgcn_sched_barrier(0);   // the keys' registers become the values'
         const uint16_t* vcol = vt + (size_t(kvh) * HD + j) * T + (t0 - base32) + 8 * lg;
         uint4 vb[8];
@@ -315,7 +324,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
             for (int g = 0; g < NT; ++g)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float resc = top[g][r] == -INFINITY ? 1.f : exp2_of(m[g][r] - top[g][r]);
+                    const float resc = top[g][r] == -INFINITY ? 1.f : exp_of(m[g][r] - top[g][r]);
                     l[g][r] *= resc;
                     m[g][r] = top[g][r];
 #pragma unroll
@@ -327,7 +336,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float from = m[g][r] == -INFINITY ? 0.f : m[g][r];   // nothing seen yet: every score is -inf
-                const float p0 = exp2_of(S[g][0][r] - from), p1 = exp2_of(S[g][1][r] - from);
+                const float p0 = exp_of(S[g][0][r] - from), p1 = exp_of(S[g][1][r] - from);
                 l[g][r] += row16_sum(p0 + p1);
                 pt[(g * 16 + 4 * lg + r) * 32 + j] = p0 * kProbScale;
                 pt[(g * 16 + 4 * lg + r) * 32 + 16 + j] = p1 * kProbScale;
@@ -375,21 +384,19 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         for (int g = 0; g < NT; ++g)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                float mine = 1.f, theirs = 0.f;
-                if (w > 0) {
-                    const float mo = ml[(g * 16 + 4 * lg + r) * 2], lo_ = ml[(g * 16 + 4 * lg + r) * 2 + 1];
-                    const float M = fmaxf(m[g][r], mo);
-                    mine = m[g][r] == -INFINITY ? 0.f : exp2_of(m[g][r] - M);
-                    theirs = mo == -INFINITY ? 0.f : exp2_of(mo - M);
-                    l[g][r] = l[g][r] * mine + lo_ * theirs;
-                    m[g][r] = M;
-                }
+                float* slots = ob + (g * 64 + r) * 64 + lane;   // [dt][4][64]
+                if (w == 0) {
 #pragma unroll
-                for (int dt = 0; dt < 16; ++dt) {
-                    float* slot = ob + (((g * 16 + dt) * 4 + r) * 64 + lane);
-                    const float v = O[g][dt][r] * mine + (w > 0 ? *slot * theirs : 0.f);
-                    *slot = v;
+                    for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r];
+                    continue;
                 }
+                const float mo = ml[(g * 16 + 4 * lg + r) * 2], lo_ = ml[(g * 16 + 4 * lg + r) * 2 + 1];
+                const float M = fmaxf(m[g][r], mo);
+                const float mine = m[g][r] == -INFINITY ? 0.f : exp_of(m[g][r] - M), theirs = mo == -INFINITY ? 0.f : exp_of(mo - M);
+                l[g][r] = l[g][r] * mine + lo_ * theirs;
+                m[g][r] = M;
+#pragma unroll
+                for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r] * mine + slots[dt * 256] * theirs;
             }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -441,7 +448,7 @@ prefill_attention_merge_kernel(AttentionOut to, uint32_t rows, uint32_t q_heads,
 #pragma unroll 4
     for (uint32_t p = 0; p < parts; ++p) {
         const size_t at = p * stride + pair;
-        const float mp = to.part_ml[2 * at], w = mp == -INFINITY ? 0.f : exp2_of(mp - M);   // a part can hold no visible token
+        const float mp = to.part_ml[2 * at], w = mp == -INFINITY ? 0.f : exp_of(mp - M);   // a part can hold no visible token
         den += w * to.part_ml[2 * at + 1];
         const float4 a = *reinterpret_cast<const float4*>(to.part_o + at * HD + 8 * c8), b = *reinterpret_cast<const float4*>(to.part_o + at * HD + 8 * c8 + 4);
         v[0] = fmaf(w, a.x, v[0]); v[1] = fmaf(w, a.y, v[1]); v[2] = fmaf(w, a.z, v[2]); v[3] = fmaf(w, a.w, v[3]);

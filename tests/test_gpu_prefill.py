@@ -276,6 +276,63 @@ def test_prefill_attention_reference_cases(hip, rows, origin, window, capacity, 
         assert abs(float(out[1, 0]) ) > 1e-3       # the retained fp32 query decides row 1
 
 
+def double_attention(q, ring_k, ring_v, run_k, run_v, position, window, mask, q_heads, kv_heads, scale):
+    """The same in 64 bits, from device tensors to a device tensor."""
+    import torch
+    rows, hd = q.shape[0], 256
+    first = max(0, position + 1 - window) if window else 0
+    held = torch.arange(first, position, device="cuda") & mask
+    K, V = (torch.cat([ring[held], run]).double().view(-1, kv_heads, hd) for ring, run in ((ring_k, run_k), (ring_v, run_v)))
+    token, own = torch.arange(first, position + rows, device="cuda"), position + torch.arange(rows, device="cuda")
+    visible = token[None] <= own[:, None]
+    if window:
+        visible &= token[None] > own[:, None] - window
+    out = torch.empty((rows, q_heads, hd), dtype=torch.float64, device="cuda")
+    for h in range(q_heads):
+        g = h // (q_heads // kv_heads)
+        s = (q.double().view(rows, q_heads, hd)[:, h] @ K[:, g].T.contiguous()) * scale
+        out[:, h] = torch.softmax(s.masked_fill(~visible, -float("inf")), -1) @ V[:, g].contiguous()
+    return out.view(rows, -1)
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,rows,position,window,cap", [(4, 1, 200, 300, 256, 256), (16, 8, 333, 0, 1024, 1024), (16, 8, 37, 900, 0, 1024)])
+@pytest.mark.parametrize("spread", [16.0, 100.0])
+def test_prefill_attention_scores_are_as_close_as_plain_fp32(hip, q_heads, kv_heads, rows, position, window, cap, spread):
+    """Large scores (spread times a standard normal one), whose error is all that the output shows, on the matrix core (queries in two
+    halves of fp16, two chains of eight instructions) and by plain fp32 arithmetic (the kernel for rows the matrix core cannot take),
+    both against 64 bits.  In units of u^2, u = 2.5e-8 the rms of one fp32 rounding: plain chains of 64 products (four heads per
+    key head) round for 33 and chains of 32 (two) for 17; an instruction rounds for 4.7 (measured) times the share its accumulator has
+    already grown to, 11 over both chains, and the query's 22 bits, the chains' sum and the probabilities' 22 bits add 6 at most.
+    So no more than plain fp32's error with four heads, and with two no more than sqrt(17 / 17) of it, a quarter on top."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(17)
+    rn = lambda *shape: torch.randn(shape, device="cuda", generator=gen)
+    q = spread * rn(rows, q_heads * 256)
+    held = [rn(n, kv_heads * 256).half() for n in (cap, cap, rows, rows)]
+    want = double_attention(q, *held, position, window, cap - 1, q_heads, kv_heads, 0.0625)
+    rms = []
+    for matrix_core in (True, False):
+        out = hip.prefill_attention(q, *held, position, window, cap - 1, q_heads, kv_heads, 256, 0.0625, matrix_core=matrix_core)
+        rms.append(float((out.double() - want).pow(2).mean().sqrt()))
+    assert rms[0] <= (1.0 if q_heads == 4 * kv_heads else 1.25) * rms[1], rms
+
+
+def test_prefill_attention_takes_queries_up_to_the_range_of_a_half(hip):
+    """A query element of 60 000 after the scale (a half holds 65 504) against keys small enough for ordinary scores."""
+    import torch
+    rows, width = 20, 256
+    q = torch.zeros((rows, 4 * width), device="cuda")
+    q[:, 7::256] = 960000.0
+    run_k = torch.zeros((rows, width), dtype=torch.float16, device="cuda")
+    run_k[:, 7] = torch.arange(rows, device="cuda") * 2.0 ** -17
+    run_v = torch.randn((rows, width), device="cuda").half()
+    ring = torch.zeros((64, width), dtype=torch.float16, device="cuda")
+    out = hip.prefill_attention(q, ring, ring, run_k, run_v, 0, 0, 63, 4, 1, 256, 0.0625)
+    want = double_attention(q, ring, ring, run_k, run_v, 0, 0, 63, 4, 1, 0.0625)
+    assert float((out.double() - want).abs().max()) <= 2e-6 * float(want.abs().max())   # scores below 10: the bar of the cases above
+
+
 def test_publish_run_keeps_the_newest_rows(hip):
     import torch
     rows, width, cap, position = 40, 256, 16, 9
