@@ -8,8 +8,16 @@
 // the same fp32 accumulator, so one 16x16x32 matrix instruction covers 16 rows.  B is exact: Q4_K sc * q (<= 945) as one
 // fused multiply-add of the biased quant, Q8_0 the signed quant, Q6_K s * (q - 32) as the nearest fp16 and the exact
 // rest of that rounding (at most one unit of 2049 or more; it meets the hi half only, its product with lo lies below
-// the image's own 22 bits).  A 256-element block accumulates inside the matrix instruction; its d and the span's
+// the image's own 22 bits).  A block's sums accumulate inside the matrix instruction; its d and the span's
 // multiplier are applied in fp32, and Q4_K's -dmin m is one more instruction on the block's group sums.
+//
+// Precision.  A matrix instruction rounds at the size its accumulator has grown to (some 4.7 times, going by the error), so
+// the order of a chain counts: Q4_K takes a group's lo half ahead of its hi half and ends a chain after half a block.  rms
+// error against 64 bits in 1e-7 of the result's rms, 333 rows, K = 3840 (Q4_K), 15360 (Q6_K), 2048 (Q8_0): normal activations
+// 1.51, 2.16, 1.61; of a 512-fold range 1.57, 2.20, 1.65; every 97th 200-fold 1.63, 2.29, 1.68; all positive 0.87, 2.16, 1.59.
+// (Kernels of 8 rows, hi and lo in accumulators of their own and Q6_K's -32 a term by itself: 1.56, 3.80, 2.68; 2.24, 4.10,
+// 2.74; 3.31, 12.7, 2.88; 0.88, 6.34, 5.21.  Q4_K hi before lo over whole blocks: 1.78, 1.84, 1.87, 0.78, and 4 % faster.  Its
+// minima or quants as denormal halves need no bias, but the instruction then drops the places they lack: 1.59 on normal ones.)
 //
 // A workgroup is four waves on the same R * 16 rows and four neighbouring column tiles.  The A operand of a 64-element
 // chunk goes from memory to LDS without passing registers, two chunks ahead in three rotating buffers, one barrier per
@@ -71,8 +79,7 @@ __device__ __forceinline__ uint32_t scalar(uint32_t v) { asm("" : "+s"(v)); retu
 __device__ __forceinline__ uint32_t and_or(uint32_t w, uint32_t mask, uint32_t c) { return (w & mask) | c; }
 // a value the compiler takes as it is (it would turn two of the above into two ands and an or3)
 __device__ __forceinline__ uint32_t kept(uint32_t v) { asm("" : "+v"(v)); return v; }
-__device__ __forceinline__ uint32_t vector_bias() {
-    uint32_t c = 0x64006400u;
+__device__ __forceinline__ uint32_t vector_bias(uint32_t c = 0x64006400u) {
     asm("" : "+v"(c));
     return c;
 }
@@ -161,15 +168,15 @@ template <int G, int P>
 __device__ __forceinline__ void q4_operands(const uint4 (&q)[4], const uint32_t (&scw)[4], half8_t (&b)[4]) {
     constexpr bool HIGH = G & 1;
     constexpr int BYTE = G & 3, WORD = (G >> 1) & 1;
-    const uint32_t bias = vector_bias(), mask = scalar(HIGH ? 0x00F000F0u : 0x000F000Fu);
+    // the quant under a bias whose last place is the quant's: 1024 + q, or 64 + q where the high nibbles stay in bits 4-7
+    const uint32_t bias = vector_bias(HIGH ? 0x54005400u : 0x64006400u), mask = scalar(HIGH ? 0x00F000F0u : 0x000F000Fu);
 #pragma unroll
     for (int cg = 2 * P; cg < 2 * P + 2; ++cg) {
-        // the scale byte under the bias: 1024 + sc in both halves, then sc and -1024 sc (all exact in fp16); the high
-        // nibbles stay in bits 4-7, where they weigh 16
+        // the scale byte under the bias: 1024 + sc in both halves, then sc and -bias sc (all exact in fp16)
         const half2_t sc = h2(__builtin_amdgcn_perm(0x64646464u, scw[cg], 0x04000400u | (BYTE << 16) | BYTE)) - splat(1024.f);
-        const half2_t off = sc * splat(HIGH ? -64.f : -1024.f), mul = HIGH ? sc * splat(0.0625f) : sc;
+        const half2_t off = sc * splat(HIGH ? -64.f : -1024.f);
         const uint32_t w0 = WORD ? q[cg].z : q[cg].x, w1 = WORD ? q[cg].w : q[cg].y;
-        auto piece = [&](uint32_t w) { return u2(__builtin_elementwise_fma(h2(and_or(w, mask, bias)), mul, off)); };
+        auto piece = [&](uint32_t w) { return u2(__builtin_elementwise_fma(h2(and_or(w, mask, bias)), sc, off)); };
         b[cg] = as_half8(piece(w0), piece(w0 >> 8), piece(w1), piece(w1 >> 8));
     }
 }
@@ -192,6 +199,10 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& fee
                                         uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q4_K);
     constexpr int V = (30 + 4 * R - 1) / (4 * R);   // vector instructions behind each matrix instruction
+    // Up to three row tiles the fold is woven in as well: a tile's beside the next tile's products, the last one's beside the
+    // second half's first products.  Four leave no registers for that (2048 x 3840 x 15360: 446 us against 440 by itself).
+    constexpr bool WOVEN = R < 4;
+    constexpr int VA = (30 + 32 * (R - 1) + 4 * R - 1) / (4 * R), VB = (62 + 4 * R - 1) / (4 * R);
     using S = Stage<R>;
     const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
     const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
@@ -227,24 +238,52 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& fee
     feed.ask(4 * b0 + 2, 2);
     arrive<2 * R>();
     scales(b0, 0);
-    read_half<R>(stage, 0, lane16, hi);
+    read_half<R>(stage, 1, lane16, lo);
     q4_operands<0, 0>(q[0], sc, b);
     q4_operands<0, 1>(q[0], sc, b);
     uint32_t rd = 0;   // the buffer of the chunk in work
     for (uint32_t blk = b0; blk < b1; ++blk) {
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
+        float dh[4];   // the first half's sums leave their chain for acc (no bias term yet)
+        auto fold_scales = [&] {
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg)
+                dh[cg] = h2f(*reinterpret_cast<const uint16_t*>(heads + (blk & 1) * 5120 + 256 * cg + j * 16));
+        };
+        auto fold = [&](int r) {
+            const float4_t mult = *reinterpret_cast<const float4_t*>(stage + S::kMult + 64 * r + 16 * lg);
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(dh[cg] * mult[i], D[cg][r][i], acc[cg][r][i]);
+        };
         auto group = [&]<int G>() {
             const uint8_t* now = stage + rd * S::kChunk + (G & 1) * (2048 * R);
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (G == 3) scales(blk, 1);
+            if constexpr (WOVEN && G == 3) fold_scales();
             if constexpr (G == 7) scales(next, 0);
-            read_half<R>(now, 1, lane16, lo);
+            read_half<R>(now, 0, lane16, hi);
             q4_operands<(G + 1) & 7, 0>(q[G == 7 ? 0 : (G + 1) >> 2], sc, bn);
-            products<R, G == 0>(hi, b, D);
-            weave<4 * R, V, R>();
+            if constexpr (WOVEN && G == 4) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    if (r + 1 == R) fold(r);
+#pragma unroll
+                    for (int cg = 0; cg < 4; ++cg) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[r], b[cg], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                }
+                weave<4 * R, VB, R>();
+            } else {
+                products<R, (G & 3) == 0>(lo, b, D);
+                weave<4 * R, V, R>();
+            }
             if constexpr (G & 1) {
                 arrive<R>();
-                if constexpr (G == 1) { ask_block(blk); ask_head(next); }
+                if constexpr (G == 1) {
+                    ask_block(blk);
+                    ask_head(next);
+                    asm volatile("" ::: "memory");   // in this order: the fold reads the multipliers behind the next meeting
+                }
                 if constexpr (G == 3) ask_half(next, 0, q[0]);
                 if constexpr (G == 7) ask_half(next, 1, q[1]);
                 feed.ask(4 * blk + (G >> 1) + 3, rd);
@@ -252,10 +291,20 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& fee
             }
             const uint8_t* then = stage + rd * S::kChunk + ((G + 1) & 1) * (2048 * R);
             __builtin_amdgcn_sched_barrier(0);
-            read_half<R>(then, 0, lane16, hi);
+            read_half<R>(then, 1, lane16, lo);
             q4_operands<(G + 1) & 7, 1>(q[G == 7 ? 0 : (G + 1) >> 2], sc, bn);
-            products<R, false>(lo, b, D);
-            weave<4 * R, V, R>();
+            if constexpr (WOVEN && G == 3) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+#pragma unroll
+                    for (int cg = 0; cg < 4; ++cg) D[cg][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[r], b[cg], D[cg][r], 0, 0, 0);
+                    if (r > 0) fold(r - 1);
+                }
+                weave<4 * R, VA, R>();
+            } else {
+                products<R, false>(hi, b, D);
+                weave<4 * R, V, R>();
+            }
 #pragma unroll
             for (int cg = 0; cg < 4; ++cg) b[cg] = bn[cg];
         };
@@ -263,6 +312,11 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& fee
         group.template operator()<1>();
         group.template operator()<2>();
         group.template operator()<3>();
+        if constexpr (!WOVEN) {
+            fold_scales();
+#pragma unroll
+            for (int r = 0; r < R; ++r) fold(r);
+        }
         group.template operator()<4>();
         group.template operator()<5>();
         group.template operator()<6>();
@@ -274,12 +328,11 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& fee
         for (int cg = 0; cg < 4; ++cg) {
             const uint4 h = *reinterpret_cast<const uint4*>(heads + (blk & 1) * 5120 + 256 * cg + j * 16);
             d[cg] = h2f(h.x & 0xFFFFu);
-            dmin[cg] = -32.0f * h2f(h.x >> 16);
-            // minima against the sums' hi (k-slice 0) and lo (k-slice 1) halves; the upper lanes' share is zero
-            const uint32_t in = lane < 32 ? 0xFFFFFFFFu : 0u;
+            dmin[cg] = -16.0f * h2f(h.x >> 16);   // the group sums are in units of 32, and twice in dm
+            // minima against the sums' hi (k-slices 0 and 2) and lo (1 and 3) halves
             const uint32_t mn_a = h.z & 0x3F3F3F3Fu, mn_b = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
-            bm[cg] = as_half8(bytes_as_halves(mn_a, 0x04020400u) & in, bytes_as_halves(mn_a, 0x04030401u) & in,
-                              bytes_as_halves(mn_b, 0x04020400u) & in, bytes_as_halves(mn_b, 0x04030401u) & in);
+            bm[cg] = as_half8(bytes_as_halves(mn_a, 0x04020400u), bytes_as_halves(mn_a, 0x04030401u),
+                              bytes_as_halves(mn_b, 0x04020400u), bytes_as_halves(mn_b, 0x04030401u));
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -723,7 +776,8 @@ int gemm_launch(hipStream_t s, GemmArgs& a, uint32_t slices, uint32_t R) {
 // Time of a launch by a model of the chip, in microseconds: `start` from the launch to the first product and from the last one
 // to the end, then every compute unit (256) works off its share of the workgroups at `unit` per slice unit -- 256 elements
 // of K, 64 for Q8_0 --, and a plane costs a write here and a read in the next operator.  Constants fitted to sweeps
-// over 4 to 1000 rows of both models' shapes; the choice was within 4 % of the best pair of each.
+// over 4 to 1000 rows of both models' shapes.  Against the best pair of a sweep of 5 to 2048 rows, planes counted: the 12B
+// shapes' launches 1 % longer on the mean, 12 % at most (64 rows); the drafter's, 4 to 30 us of them, 5 % and 45 %.
 constexpr float kStart[4] = {5.0f, 6.2f, 7.5f, 8.5f};
 constexpr float kUnit[3][4] = {{0.6f, 0.82f, 1.0f, 1.35f}, {2.3f, 2.7f, 3.2f, 3.8f}, {2.8f, 3.3f, 4.0f, 4.8f}};   // Q8_0, Q4_K, Q6_K
 constexpr float kPlaneBytesPerUs = 5.0e6f;

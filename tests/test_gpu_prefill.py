@@ -60,6 +60,31 @@ def test_prefill_gemm_keeps_all_f32_operand_information(hip, gfo, dtype):
     assert_f32_information(gfo, dtype, w, x, inner, y, width, columns)
 
 
+@pytest.mark.parametrize("rows", [37, 128, 333])
+def test_prefill_gemm_sums_against_64_bits(hip, rows):
+    """Q4_K at K = 3840 on normal activations.  With u = 2.5e-8, the rms of one fp32 rounding, a chain of 30 updates of the row's
+    sum costs 16 u^2 of squared error beside the result's, a block's own two roundings 2 u^2, the operand's 22 bits 2 u^2, and a
+    matrix instruction 4.7 u^2 (measured) times the share its accumulator has already grown to, 14 u^2 over chains of eight:
+    1.46e-7 in all, 1.6e-7 with a tenth on top.  (Chains of sixteen, a whole block, measured 1.8e-7.)"""
+    import torch
+    K, N = 3840, 512
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(23)
+    raw = torch.randint(0, 256, (N * (K // 256), 144), dtype=torch.uint8, device="cuda", generator=gen)
+    scales = (0.02 * torch.randn((raw.shape[0], 2), device="cuda", generator=gen)).abs().half()
+    raw[:, :4] = scales.view(torch.uint8)
+    packed, quants = raw[:, 4:16].int(), raw[:, 16:].view(-1, 4, 1, 32)
+    sc = torch.cat([packed[:, :4] & 63, (packed[:, 8:] & 15) | ((packed[:, :4] >> 6) << 4)], 1).double()
+    mn = torch.cat([packed[:, 4:8] & 63, (packed[:, 8:] >> 4) | ((packed[:, 4:8] >> 6) << 4)], 1).double()
+    q = torch.cat([quants & 15, quants >> 4], 2).reshape(-1, 8, 32).double()
+    d = scales.double()
+    w = (d[:, :1, None] * sc[:, :, None] * q - d[:, 1:, None] * mn[:, :, None]).reshape(N, K)
+    x = torch.randn((rows, K), device="cuda", generator=gen)
+    want = x.double() @ w.T.contiguous()
+    y = hip.prefill_gemm(1, hip.repack(1, raw.view(-1), K, N), hip.prefill_pack(x), rows, K, N).double()
+    assert float(((y - want).pow(2).mean() / want.pow(2).mean()).sqrt()) <= 1.6e-7
+
+
 def test_prefill_gemm_down_projection_shape(hip, gfo):
     """Q6_K at the down projection's K = 15360 (60 blocks per column, the longest chain of LDS
     stages and weight prefetches) with an odd number of column tiles and rows in every row group."""
