@@ -50,6 +50,7 @@ constexpr uint32_t kWideRows = 4;
 // The work split of a streaming product over `tiles` column tiles of `nblk` blocks (gemv_packed.hip): blocks per wave, waves per
 // workgroup (at most max_w) and planes left to the consumer; waves_per_cu waves are assumed to fit a CU.
 struct GemvSplit { uint32_t bps, W, planes; };
+uint32_t compute_units();   // of the device the library was initialised on (256 before that)
 GemvSplit gemv_split(uint32_t nblk, uint32_t tiles, uint32_t max_w, uint32_t waves_per_cu);
 uint32_t gemv_wide_planes(uint32_t count, const int* dtypes, const uint32_t* N, uint32_t K);
 // partials[i]: [planes][rows][N[i]]; y (one matrix): the planes' sum [rows][N]

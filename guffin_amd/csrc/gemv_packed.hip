@@ -376,6 +376,7 @@ int launch_packed(hipStream_t s, const uint8_t* w, const float* x, const float* 
 
 }  // namespace
 
+uint32_t compute_units() { return static_cast<uint32_t>(g_cus); }
 GemvSplit gemv_split(uint32_t nblk, uint32_t tiles, uint32_t max_w, uint32_t waves_per_cu) { return choose_split(nblk, tiles, max_w, waves_per_cu); }
 
 // Called by guffin_hip_init with `device` current: the split heuristics' CU count and this device's

@@ -604,8 +604,9 @@ namespace {
 struct AttentionCut { uint32_t tiles, parts; };
 AttentionCut attention_cut(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_t group) {
     const uint32_t pairs = rows * group, twos = (pairs + 31) / 32 * kv_heads, ones = (pairs + 15) / 16 * kv_heads;
-    if (twos >= 256) return {2, 1};
-    return {1, std::max(1u, std::min(512u / ones, T / 128))};
+    const uint32_t cus = compute_units();
+    if (twos >= cus) return {2, 1};
+    return {1, std::max(1u, std::min(2 * cus / ones, T / 128))};
 }
 uint64_t transposed_bytes(uint32_t T, uint32_t kv_heads) { return (uint64_t(kv_heads) * 256 * T * 2 + 255) & ~uint64_t{255}; }
 }  // namespace

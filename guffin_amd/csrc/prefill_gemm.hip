@@ -774,7 +774,7 @@ int gemm_launch(hipStream_t s, GemmArgs& a, uint32_t slices, uint32_t R) {
 }
 
 // Time of a launch by a model of the chip, in microseconds: `start` from the launch to the first product and from the last one
-// to the end, then every compute unit (256) works off its share of the workgroups at `unit` per slice unit -- 256 elements
+// to the end, then every compute unit works off its share of the workgroups at `unit` per slice unit -- 256 elements
 // of K, 64 for Q8_0 --, and a plane costs a write here and a read in the next operator.  Constants fitted to sweeps
 // over 4 to 1000 rows of both models' shapes.  Against the best pair of a sweep of 5 to 2048 rows, planes counted: the 12B
 // shapes' launches 1 % longer on the mean, 12 % at most (64 rows); the drafter's, 4 to 30 us of them, 5 % and 45 %.
@@ -794,6 +794,7 @@ PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint3
         for (int r = 0; r < 4; ++r) unit[r] += float(n) * kUnit[m[i].dtype][r];
     }
     const uint32_t units = q8 ? (K + 63) / 64 : K / 256;   // what a slice is made of
+    const uint32_t cus = compute_units();
     PrefillSplit best {1, 1};
     float least = 0.f;
     for (uint32_t R = 1; R <= 4; ++R) {
@@ -802,7 +803,7 @@ PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint3
             const uint32_t n = chunks * groups * S;
             // one workgroup per compute unit leaves gaps that a second one fills; the last, partly filled turn overlaps the
             // one before it: half of it counts
-            const float turns = std::max(1.22f, 0.5f * (float((n + 255) / 256) + float(n) / 256.0f));
+            const float turns = std::max(1.22f, 0.5f * (float((n + cus - 1) / cus) + float(n) / float(cus)));
             const float cost = kStart[R - 1] + turns * float((units + S - 1) / S) * unit[R - 1] / float(groups)
                 + float(S) * 8.0f * float(M) * float(width) / kPlaneBytesPerUs;
             if ((R == 1 && S == 1) || cost < least) { best = {R, S}; least = cost; }
