@@ -25,8 +25,8 @@
 // (sixteen column groups of 4 side by side, no repeated A rows), a lane owning one column from its quants to its sum: no
 // selection among column groups (128 of 496 vector instructions of a Q4_K tile), no masked half-groups and lane exchanges
 // for Q6_K, and the operand of a 256-element block in 8 registers instead of 32, so it is requested ahead of every tile.
-// With the 16x16x32 form / now (us): gate + up 3840 -> 15360 on two rows 17.3 / 14.9, on one 16.2 / 14.3, down
-// 15360 -> 3840 on two rows 13.0 / 10.8, q/k/v 8.2 / 7.2, the 262144-row Q6_K head 143 / 130: what a launch streams does
+// With the 16x16x32 form / now (us): gate + up 3840 -> 15360 on two rows 17.3 / 14.2, on one 16.2 / 14.3, down
+// 15360 -> 3840 on two rows 13.0 / 10.7, q/k/v 8.2 / 6.9, the 262144-row Q6_K head 143 / 124: what a launch streams does
 // not change, its unpack is what does not overlap.  Block scales are applied to the per-group sums in fp32 by the lane that owns the
 // column; the offset terms (-dmin*m for Q4_K, -32 for Q6_K, -128 for the biased Q8_0 bytes)
 // use the receipt's 16- / 32-sums.  K is cut into slices: up to 16 slices are the waves of

@@ -1,14 +1,12 @@
-// Chunked prefill on the matrix core (gfx950): M rows x quantised weights, and causal GQA
-// attention over the fp16 KV rings for a run of consecutive positions.
+// Causal GQA attention of a run of rows over the fp16 KV rings (gfx950), and the moves of K/V rows around it.
 //
-// Replaces the reference's prefill matrix path (src/tensor/backends/metal/metal_kernels.mm:
-// 1031-1199, dispatch rules metal_command_context.mm:384-401) and encode_f16_prefill_attention
-// (metal_command_context.hpp:185, kernels metal_kernels.mm:2593-2800).
+// Replaces the reference's encode_f16_prefill_attention (src/tensor/backends/metal/metal_command_context.hpp:185, kernels
+// metal_kernels.mm:2593-2800).
 //
-// Attention.  A workgroup serves 16 consecutive query rows of one KV head (all query heads of the
-// group) and walks the visible key range in tiles of 32 tokens through LDS with an online
-// softmax, fp32 math on fp16 keys/values: positions before the run come from the ring, the run's
-// own positions from its private rows, which are published to the ring afterwards.
+// prefill_attention_mfma_kernel runs on the matrix core for one, two or four query heads per KV head; prefill_attention_kernel
+// on the vector unit takes rows it cannot (other alignments, no workspace).  Positions before the run come from the ring,
+// the run's own from its private rows, which are published to the ring afterwards.  Both walk the visible key range in tiles
+// of 32 tokens with an online softmax, fp32 math on fp16 keys and values.
 #include "common.hpp"
 #include "prefill_image.hpp"
 #include "prefill_run.hpp"

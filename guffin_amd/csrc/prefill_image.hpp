@@ -4,7 +4,8 @@
 //   img  : half  [K/32][Mpad/16][hi, lo][64 lanes][8]   one 1 KB record per (32-group, 16 rows, half) in the order the
 //                                        matrix instruction wants its A operand: lane (i, s) = i + 16 s holds k-slice s
 //                                        (elements 8s..8s+7) of row i, inside it the halves at {0,2,1,3,4,6,5,7}
-//   mult : float [K/span][Mpad]          2^E of (row, span); hi + lo = x 2^-E to 22 bits, |x| 2^-E < 2^15
+//   mult : float [K/span][Mpad]          2^E of (row, span); |x| 2^-E < 2^15 and hi + lo = x 2^-E to 22 bits, for what lies
+//                                        below 2^-18 of the span's largest to 2^-40 of that
 //   sums : half  [K/256][Mpad/16][32 lanes][8]   (K % 256 == 0) the 8 group sums of a 256-element block times 2^-(E+5), lane
 //                                        i the hi and lane 16 + i the lo half of row i, group t at {0,2,1,3,4,6,5,7}[t]
 //

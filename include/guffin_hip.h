@@ -446,7 +446,8 @@ int guffin_hip_forward_tree_rows(void* stream, const guffin_model_desc* model, c
 /* How guffin_hip_forward_rows (and so guffin_hip_h1_step, the sessions and the tickets) runs the blocks:
  * 0 (default) the resident pass for models with one KV head that fit it (measured faster there), else one
  * launch per operator; 1 always one launch per operator; 2 the resident pass for every model it covers
- * (1 or 8 KV heads of 256, hidden width <= 4096, one block length per model), else GUFFIN_E_SHAPE.  The resident pass keeps one workgroup per CU for a
+ * (1 or 8 KV heads of 256, hidden width <= 4096, one block length per model), else GUFFIN_E_SHAPE.  Verify trees other than chains
+ * of 1 or 2 rows have no resident form and run one launch per operator in every mode.  The resident pass keeps one workgroup per CU for a
  * group of blocks, gives each of the 8 XCDs one KV head (models with 8 KV heads; one XCD for a single KV
  * head) and moves a block's intermediate rows through that XCD's L2; only the two reductions of a block
  * cross XCDs.  Every wait in it is bounded by the spin limit (polls of a counter): a workgroup that gives up
