@@ -1,0 +1,999 @@
+// The block graph of a decode pass (one or two rows) of a narrow Q8_0 model with one KV head -- the drafter -- as one launch of
+// up to 24 blocks on the 32 CUs of one XCD.
+//
+// Operator order per block: the drafter's forward (src/engine/gemma3_draft.mm:888-972).  The placement and the bounded waits are
+// those of resident.hip; as there, workgroups hand over through the XCD's L2: plain stores, a counter, reads past the L1.
+//
+// What bounds it: a chain of 18 x 5 phases, each a hand-over (1.05 us: a 256-byte store, its acknowledgement, arrival, poll) and
+// one to two microseconds of dependent steps; the weights alone (5.9 MB a block at the 1.3 TB/s that one XCD takes) would be 4.5
+// us a block.  So the design is about what lies between two hand-overs:
+//
+//   * A wave works from its operand to its partial sums by itself.  It owns three blocks of the hidden width: it sums their
+//     planes, keeps their residual in registers and forms their operand (a norm pair needs the others for its two sums only, a
+//     meeting each); it merges just the attention outputs that its own two o-projection blocks want and loads just the GeGLU
+//     values of its own down blocks.
+//   * Products are exact integers: the quants are int8 as they lie in the tile, an activation is four int8 digits of a 31-bit
+//     fixed-point number per group of 32, and v_mfma_i32_4x4x4_16b_i8 multiplies a column's four weights with the four digits
+//     of four elements: eight instructions a block, nothing to unpack, no bias to take off again, sums without rounding.  (The
+//     fp16 form of the other kernels: some 60 vector instructions a block, 22 bits of an activation.)
+//   * A wave's weights of a whole block of the model (15 tiles) have registers of their own and are asked for most of a block
+//     ahead, a few tiles behind each phase's own operands and never during a hand-over (which then takes 1.9 us).
+//   * Weights are read through the caches' ordinary policy: non-temporal requests take 1200 cycles instead of 700 to come back
+//     (2176-byte tiles, one XCD), which is 47 us of a pass.
+//   * The eighth wave has no weights.  It adds the workers' partial sums, stores them, waits for that store alone, arrives
+//     and polls; so nobody's wait for a store or for the counter includes a weight request.
+//   * Attention: a wave a query (four waves are one a SIMD: eight would share the issue slots), a token per 16 lanes with a
+//     running softmax of their own, merged over lanes by register swaps; a list's first 20 tokens lie in LDS before the phase.
+//
+// 270M-shaped model, one row at position 150 / 600 / 4096: 299 / 303 / 356 us; two rows: 394 / 415 / 463.  (resident_blocks_kernel,
+// three launches: 606 / 621 / 652 and 777 / 816 / 888.)  rms error of the hidden row against 64 bits, one block, where no K/V
+// rounding falls the other way: 5.3-8e-8, as before.
+#include "common.hpp"
+#include "receipt.hpp"
+#include "resident.hpp"
+
+#include <algorithm>
+#include <cmath>
+
+namespace guffin {
+namespace {
+
+constexpr uint32_t kWaves = 8, kThreads = 64 * kWaves;
+constexpr uint32_t kWorkers = 7;          // waves with weights; the last one publishes
+constexpr uint32_t kParts = 3;            // parts of K in the o and down projections
+constexpr uint32_t kMaxWidth = 640;       // hidden width: three blocks a worker
+constexpr uint32_t kMaxFfn = 2048;        // a gate / up tile pair a workgroup
+constexpr int kOwn = 3, kOwnO = 2, kOwnDown = 4;          // blocks per worker: of the hidden width, of o, of down
+constexpr uint32_t kTile = 64 * 34;       // a wave tile of one Q8_0 block (gemv_packed.hip has the layout)
+constexpr uint32_t kChunk = 20;           // tokens whose keys and values lie in LDS (a window of 512: 17 a workgroup)
+
+constexpr uint32_t kSyncStride = 64;      // words between the counters of consecutive launches
+constexpr uint32_t kLayers = 24;          // blocks per launch (their pointers travel as kernel arguments)
+
+struct DLayer {
+    const uint8_t* tiles[7];                 // q k v o gate up down
+    const float* weights[6];                 // post_attention_norm, ffn_norm, post_ffw_norm, the norm that follows the block, q_norm, k_norm
+    const uint16_t *ring_k, *ring_v;
+    uint32_t local, ring_mask;
+};
+struct DArgs {
+    DLayer layer[kLayers];
+    uint32_t layers, H, F;
+    float eps, scale;
+    uint8_t* exchange;                       // the hand-over buffers; offsets of its regions, all of them
+    uint32_t qkv_at, out_at, ml_at, o_at, d_at, h_at, exchange_bytes;
+    uint32_t* sync;                          // one cleared counter
+    const float *x_in, *u_in;
+    float *x_out, *u_out; void* u_receipt_out;   // written after the last block
+    const float2 *rope_local, *rope_global;
+    const uint32_t *schedule, *ancestors;    // of the launch's first block on
+    uint16_t *priv_k, *priv_v;               // [block][row][256], of the launch's first block on
+    uint32_t* status;
+    uint32_t spin_limit;
+    unsigned long long* stamps;              // profiling aid: 8 clock readings per block from workgroup 0, or null
+};
+
+typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
+typedef int i4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+
+template <int R>
+struct Shared {
+    float red[kWorkers][2][R][64];                 // the workers' column sums (gate and up)
+    float sums[2][R][kWaves];                      // their parts of a row's two sums of squares
+    float2 rope[2][R][kHd / 2];                    // local, global
+    uint32_t opnd[kWorkers][R][128];               // a worker's operand: an element's four digits a word
+    float mult[kWorkers][R][4];
+    float head[kWaves][kHd];                       // a wave's query (then its output, where several waves share a query)
+    float2 ml[kWaves];
+    uint16_t k_s[kChunk][kHd], v_s[kChunk][kHd];   // ring rows of a chunk of this workgroup's tokens
+    uint16_t kp_s[R][kHd], vp_s[R][kHd];           // the private rows among them
+    float weight[kWorkers][R][kGroups];            // a worker's partition weights, those of lane group g at 8 g ..
+    uint32_t schedule[kLayers][R][4];      // first ring position, ring count, private rows attended (a bit each)
+    uint32_t dead;
+};
+
+// the workgroup meets; LDS accesses are done, loads stay in flight
+__device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// what this wave wrote to LDS may be read by its other lanes
+__device__ __forceinline__ void own_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// everything this wave has asked for is there (what it asks for next does not hold up what the chain waits for)
+__device__ __forceinline__ void arrived() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// the other operand order of the xor-16 / xor-32 exchange, on the vector unit
+__device__ __forceinline__ float swap16_sum(float v) {
+    const u2_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r.x) + __uint_as_float(r.y);
+}
+__device__ __forceinline__ float swap32_sum(float v) {
+    const u2_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r.x) + __uint_as_float(r.y);
+}
+__device__ __forceinline__ float swap16_max(float v) {
+    const u2_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
+}
+__device__ __forceinline__ float swap32_max(float v) {
+    const u2_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
+}
+__device__ __forceinline__ float lanes_sum(float v) { return swap32_sum(swap16_sum(row16_sum(v))); }
+
+// ---- weights ---------------------------------------------------------------------------------------------
+// A lane's column of one block: its 32 quants in order, its scale.
+struct Tile { u2_t q[4]; uint32_t d; };
+__device__ __forceinline__ uint32_t tile_lane(uint32_t lane) { return (lane >> 5) * 1024u + (lane & 15u) * 16u + ((lane >> 4) & 1u) * 8u; }
+using Global = const __attribute__((address_space(1))) uint8_t*;   // (a generic pointer's loads would count as LDS accesses too)
+__device__ __forceinline__ void load_tile(Tile& t, Global tile, uint32_t lane) {
+    Global p = tile + tile_lane(lane);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) t.q[s] = *reinterpret_cast<const __attribute__((address_space(1))) u2_t*>(p + 256 * s);
+    t.d = *reinterpret_cast<const __attribute__((address_space(1))) uint16_t*>(tile + 2048 + lane * 2);
+}
+// Block i of a run of `count`; past its end the last one again, unused, so that every wave makes the same requests.  (The uniform
+// part of an address stays in scalar registers: left to itself the compiler adds it to the lane's part and keeps the sums of all
+// fifteen tiles in vector registers over the loop.)
+__device__ __forceinline__ void ask_tile(Tile& t, const uint8_t* run, uint32_t i, uint32_t count, uint32_t lane) {
+    Global p = (Global)run + (i < count ? i : max(count, 1u) - 1u) * kTile;
+    asm("" : "+s"(p));
+    load_tile(t, p, lane);
+    asm volatile("" ::: "memory");   // here and not elsewhere
+}
+
+// ---- activations -----------------------------------------------------------------------------------------
+// Fixed point for a group of 32: |x| < 2^(e+1) with e the exponent of the group's largest, n = x 2^(29-e), |n| < 2^30.  The four
+// int8 digits of n (n = sum d_k 256^k, each in [-128, 127]) are the bytes of n + 0x00808080 with the lower three's top bits
+// flipped.  A group with an infinity or a NaN gets a NaN for its multiplier.
+struct GroupScale { float scale, mult; };
+__device__ __forceinline__ GroupScale group_scale(uint32_t largest) {   // bits of the group's largest magnitude
+    const uint32_t eb = min(max(largest >> 23, 30u), 254u);
+    return {__uint_as_float((283u - eb) << 23), __uint_as_float(largest >= 0x7F800000u ? 0x7FC00000u : (eb - 29u) << 23)};
+}
+__device__ __forceinline__ uint32_t digits(float x, float scale) { return (static_cast<uint32_t>(static_cast<int>(x * scale)) + 0x00808080u) ^ 0x00808080u; }
+__device__ __forceinline__ uint32_t magnitude(float v) { return __float_as_uint(v) & 0x7FFFFFFFu; }
+
+// Four consecutive elements a lane, a group in eight aligned lanes; quad `at` of the wave's operand if `mine`.
+__device__ __forceinline__ void put_quad(const f4_t v, uint32_t at, bool mine, uint32_t* opnd, float* mult) {
+    uint32_t m = max(max(magnitude(v.x), magnitude(v.y)), max(magnitude(v.z), magnitude(v.w)));
+    m = max(m, lane_cross_u32<0xB1, 0xF>(m));
+    m = max(m, lane_cross_u32<0x4E, 0xF>(m));
+    m = max(m, lane_cross_u32<0x141, 0xF>(m));
+    const GroupScale g = group_scale(m);
+    if (mine) {
+        *reinterpret_cast<uint4*>(opnd + 4 * at) = make_uint4(digits(v.x, g.scale), digits(v.y, g.scale), digits(v.z, g.scale), digits(v.w, g.scale));
+        if ((at & 7u) == 0) mult[at >> 3] = g.mult;
+    }
+}
+// The matrix operand of blocks 2v, 2v + 1: lane 4 i + k holds digit k of elements 4i .. 4i + 3.
+template <int V>
+__device__ __forceinline__ void read_operand(int (&a)[V], const uint32_t* opnd, uint32_t lane) {
+    const uint32_t k = lane & 3u, low = 0x0c0c0000u | (k + 4u) << 8 | k, high = (k + 4u) << 24 | k << 16 | 0x00000c0cu;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const uint4 w = *reinterpret_cast<const uint4*>(opnd + 64 * v + 4 * (lane >> 2));
+        a[v] = static_cast<int>(__builtin_amdgcn_perm(w.y, w.x, low) | __builtin_amdgcn_perm(w.w, w.z, high));
+    }
+}
+
+// digit sums by weight, the small ones first
+__device__ __forceinline__ float digit_value(const i4_t D) {
+    float f = fmaf(static_cast<float>(D[1]), 256.f, static_cast<float>(D[0]));
+    f = fmaf(static_cast<float>(D[2]), 65536.f, f);
+    return fmaf(static_cast<float>(D[3]), 16777216.f, f);
+}
+// elements 4 STEP .. 4 STEP + 3 of every block: the chains of the blocks side by side
+template <int STEP, int N, int R, int V, int I = 0>
+__device__ __forceinline__ void step(const Tile (&t)[N], const int (&a)[R][V], i4_t (&D)[N][R]) {
+    if constexpr (I < N) {
+        const int w = static_cast<int>((STEP & 1) ? t[I].q[STEP >> 1].y : t[I].q[STEP >> 1].x);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            D[I][r] = __builtin_amdgcn_mfma_i32_4x4x4i8(a[r][I >> 1], w, STEP == 0 ? i4_t{0, 0, 0, 0} : D[I][r], 4, 8 * (I & 1) + STEP, 0);
+        step<STEP, N, R, V, I + 1>(t, a, D);
+    }
+}
+template <int N, int R, int V, int STEP = 0>
+__device__ __forceinline__ void steps(const Tile (&t)[N], const int (&a)[R][V], i4_t (&D)[N][R]) {
+    if constexpr (STEP < 8) { step<STEP>(t, a, D); steps<N, R, V, STEP + 1>(t, a, D); }
+}
+// this lane's column over the wave's `count` blocks, in block order
+template <int N, int R>
+__device__ __forceinline__ void fold(const Tile (&t)[N], uint32_t count, const i4_t (&D)[N][R], const float (*mult)[4], float (&acc)[R]) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float d = h2f(t[i].d);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float sum = fmaf(d * mult[r][i], digit_value(D[i][r]), acc[r]);
+            acc[r] = uint32_t(i) < count ? sum : acc[r];
+        }
+    }
+}
+
+// how `total` items are dealt to `ways`: the first ones get one more
+struct Share { uint32_t first, count; };
+__device__ __forceinline__ Share share_of(uint32_t total, uint32_t ways, uint32_t i) {
+    const uint32_t base = total / ways, more = total % ways;
+    return {i * base + min(i, more), base + (i < more ? 1u : 0u)};
+}
+
+// ---- attention -------------------------------------------------------------------------------------------
+// The tokens of a block's rows (union of the rows' ring ranges, then the private rows) and this workgroup's part of them.
+template <int R>
+struct Tokens { uint32_t u_first, n_ring, t0, t1, mask, first[R], end[R], attends[R]; };
+
+template <int R>
+__device__ __forceinline__ Tokens<R> tokens_of(const Shared<R>& sh, uint32_t l, uint32_t mask, uint32_t slot) {
+    Tokens<R> t;
+    uint32_t first = 0xFFFFFFFFu, end = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t f = uniform(sh.schedule[l][r][0]), n = uniform(sh.schedule[l][r][1]);
+        t.first[r] = f; t.end[r] = f + n; t.attends[r] = uniform(sh.schedule[l][r][2]);
+        if (n) { first = min(first, f); end = max(end, f + n); }
+    }
+    t.u_first = end ? first : 0u;
+    t.n_ring = end ? end - first : 0u;
+    const uint32_t total = t.n_ring + R, per = (total + kGroups - 1) / kGroups;
+    t.t0 = min(slot * per, total); t.t1 = min(t.t0 + per, total);
+    t.mask = mask;
+    return t;
+}
+
+// A worker's share of a chunk: up to three of its 20 pairs of rows (ten of keys, ten of values), half a wave a row.  Asked for
+// through a buffer resource: lanes past the last token ask beyond its end, which reads zeros and touches no memory.
+struct Rows { uint4 v[3]; };
+template <int R>
+__device__ __forceinline__ void ask_rows(Rows& to, const uint16_t* ring_k, const uint16_t* ring_v, const Tokens<R>& t, uint32_t chunk, uint32_t wave, uint32_t lane) {
+#pragma unroll
+    for (uint32_t i = 0; i < 3; ++i) {
+        const uint32_t pair = wave + kWorkers * i, row = 2 * (pair % (kChunk / 2)) + (lane >> 5), token = chunk + row;
+        const __amdgpu_buffer_rsrc_t ring = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pair < kChunk / 2 ? ring_k : ring_v), 0,
+                                                                              static_cast<int>((t.mask + 1) * (2 * kHd)), 0x00020000);
+        const bool there = pair < kChunk && token < t.t1 && token < t.n_ring;
+        const int at = there ? static_cast<int>(((t.u_first + token) & t.mask) * (2 * kHd) + 16 * (lane & 31u)) : -1024;
+        to.v[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ring, at, 0, 0));
+    }
+}
+template <int R>
+__device__ __forceinline__ void put_rows(Shared<R>& sh, const Rows& from, uint32_t wave, uint32_t lane) {
+#pragma unroll
+    for (uint32_t i = 0; i < 3; ++i) {
+        const uint32_t pair = wave + kWorkers * i, row = 2 * (pair % (kChunk / 2)) + (lane >> 5);
+        if (pair < kChunk) *reinterpret_cast<uint4*>(&(pair < kChunk / 2 ? sh.k_s : sh.v_s)[row][8 * (lane & 31u)]) = from.v[i];
+    }
+}
+
+// Head norm and rotation of 256 values, dimensions 2l, 2l+1, 128 + 2l, 128 + 2l + 1 a lane.
+struct HeadNorm { float2 lo, hi; };
+__device__ __forceinline__ HeadNorm load_head_norm(const float* p, uint32_t lane) {
+    HeadNorm g;
+    g.lo = make_float2(p[2 * lane], p[2 * lane + 1]); g.hi = make_float2(p[128 + 2 * lane], p[128 + 2 * lane + 1]);
+    return g;
+}
+__device__ __forceinline__ void norm_rotate(float (&v)[4], const HeadNorm& gamma, const float2* rope, float eps, uint32_t lane) {
+    const float ss = lanes_sum(fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0]))));
+    const float inv = 1.0f / sqrtf(ss / 256.0f + eps);
+    const float g[4] = {gamma.lo.x, gamma.lo.y, gamma.hi.x, gamma.hi.y};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = v[k] * inv * g[k];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const float2 cs = rope[2 * lane + k];
+        const float first = v[k], second = v[k + 2];
+        v[k] = __fsub_rn(__fmul_rn(first, cs.x), __fmul_rn(second, cs.y));
+        v[k + 2] = __fadd_rn(__fmul_rn(first, cs.y), __fmul_rn(second, cs.x));
+    }
+}
+
+template <int R, int G>
+struct Pass {
+    static constexpr int NQ = R * G;
+    static constexpr uint32_t CW = (G + 2) * kHd, TA = 4 * G + 8;
+    // Four or eight waves attend, a query each (two or four of them, where there are fewer queries): four are one a SIMD, and
+    // eight would share its issue slots.
+    static constexpr uint32_t WPQ = NQ < 4 ? 4 / NQ : 1, ATTENDING = WPQ * NQ;
+    static constexpr uint32_t STEP = 4 * WPQ;                                  // tokens of a round
+    static constexpr uint32_t PREPARING = ATTENDING + 2 * R <= kWorkers ? ATTENDING : 0;   // first wave of those that prepare private rows
+    const DArgs& a;
+    Shared<R>& sh;
+    uint32_t lane;
+    const uint32_t wave, slot;
+    uint32_t generation = 0;
+    __amdgpu_buffer_rsrc_t exchange;
+
+    // What another workgroup stored during this launch: past this CU's L1 (sc1), which nothing invalidates, from the L2.
+    static constexpr int kPast = 16;
+    __device__ __forceinline__ f4_t ld4(uint32_t at, uint32_t floats) const {
+        return __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(exchange, static_cast<int>(4 * floats), static_cast<int>(at), kPast));
+    }
+    __device__ __forceinline__ float2 ld2(uint32_t at, uint32_t floats) const {
+        return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(exchange, static_cast<int>(4 * floats), static_cast<int>(at), kPast));
+    }
+    __device__ __forceinline__ void st(uint32_t at, uint32_t floats, float v) const {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
+    }
+    __device__ __forceinline__ void st2(uint32_t at, uint32_t floats, float2 v) const {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2_t, v), exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
+    }
+    __device__ __forceinline__ void st4(uint32_t at, uint32_t floats, f4_t v) const {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, v), exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
+    }
+
+    __device__ __forceinline__ void enter() { lane = opaque(lane); }   // or every address that depends on the lane alone is kept in a register over the loop
+    __device__ __forceinline__ void stamp(uint32_t l, uint32_t phase) const {
+        if (a.stamps && slot == 0 && lane == 0) a.stamps[l * 16 + phase] = wall_clock64();
+    }
+
+    // The last wave: its stores are in the L2, then the arrival, then the wait for the other workgroups.  A wait that gives up
+    // raises the status bit, and the workgroup waits no more for the rest of the launch.
+    __device__ __forceinline__ void arrive_and_wait() {
+        __builtin_amdgcn_s_waitcnt(0);
+        generation += 1;
+        if (lane == 0 && !sh.dead) {
+            __hip_atomic_fetch_add(a.sync, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            const uint32_t target = kGroups * generation;
+            uint32_t spins = 0;
+            while (__hip_atomic_load(a.sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+                if (++spins > a.spin_limit) {
+                    sh.dead = 1u;
+                    atomicOr(a.status, GUFFIN_STATUS_SYNC);
+                    break;
+                }
+            }
+        }
+        asm volatile("" ::: "memory");
+    }
+    __device__ __forceinline__ float workers_sum(int matrix, int r) const {
+        float s = sh.red[0][matrix][r][lane];
+#pragma unroll
+        for (uint32_t w = 1; w < kWorkers; ++w) s += sh.red[w][matrix][r][lane];
+        return s;
+    }
+
+    // What a wave's part in a block's attention needs and does not depend on the pass, asked for a phase ahead.
+    __device__ __forceinline__ HeadNorm ask_gamma(const DLayer& L) const {
+        const bool key = PREPARING >= ATTENDING && wave >= PREPARING && wave < PREPARING + 2 * R;
+        return load_head_norm(L.weights[key ? 5 : 4], lane);
+    }
+
+    // Every query of the rows against this workgroup's tokens.  The first chunk's rows lie in LDS, `rows` holds this worker's share
+    // of the second one; a token per 16 lanes, lane s of them with dimensions 8s .. 8s+7 and 128 + 8s .. 128 + 8s + 7.
+    template <typename First, typename Second>
+    __device__ __forceinline__ void attend(uint32_t l, const DLayer& L, const Tokens<R>& t, const HeadNorm& gamma, Rows& rows, First first_request, Second second_request) {
+        constexpr uint32_t ROUNDS = (kChunk + STEP - 1) / STEP;
+        const uint32_t query = wave / WPQ, r = R > 1 ? query / G : 0, s16 = lane & 15u;
+        const float2* rope = sh.rope[L.local ? 0 : 1][0];
+        // the private rows' keys and values are the work of the workgroup whose tokens they are, a wave each
+        const bool owner = t.t1 > t.n_ring && t.t1 > t.t0;
+        const uint32_t pr = (wave - PREPARING) >> 1;
+        const bool prepares = owner && wave >= PREPARING && wave < PREPARING + 2 * R && t.n_ring + pr >= t.t0 && t.n_ring + pr < t.t1;
+        const bool is_key = ((wave - PREPARING) & 1u) == 0;
+        float2 v0 = make_float2(0.f, 0.f), v1 = v0, p0 = v0, p1 = v0;
+        HeadNorm key_gamma = gamma;
+        if (wave < ATTENDING) {
+            const uint32_t own = r * CW + (query % G) * kHd + 2 * lane;
+            v0 = ld2(a.qkv_at, own); v1 = ld2(a.qkv_at, own + 128);
+        }
+        if (prepares) {
+            const uint32_t src = pr * CW + (is_key ? G : G + 1) * kHd + 2 * lane;
+            p0 = ld2(a.qkv_at, src); p1 = ld2(a.qkv_at, src + 128);
+            if (PREPARING < ATTENDING && is_key) key_gamma = load_head_norm(L.weights[5], lane);
+        }
+        arrived();
+        first_request();
+        float* q_s = sh.head[wave];
+        if (wave < ATTENDING) {
+            float v[4] = {v0.x, v0.y, v1.x, v1.y};
+            norm_rotate(v, gamma, rope + r * (kHd / 2), a.eps, lane);
+            *reinterpret_cast<float2*>(q_s + 2 * lane) = make_float2(v[0] * a.scale, v[1] * a.scale);
+            *reinterpret_cast<float2*>(q_s + 128 + 2 * lane) = make_float2(v[2] * a.scale, v[3] * a.scale);
+        }
+        if (prepares) {
+            float pv[4] = {p0.x, p0.y, p1.x, p1.y};
+            if (is_key) norm_rotate(pv, key_gamma, rope + pr * (kHd / 2), a.eps, lane);
+            bool bad = false;
+            uint32_t bits[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const _Float16 hv = static_cast<_Float16>(pv[k]);
+                bad |= !isfinite(static_cast<float>(hv));
+                bits[k] = __builtin_bit_cast(uint16_t, hv);
+            }
+            uint16_t* to = (is_key ? sh.kp_s : sh.vp_s)[pr];
+            uint16_t* out = (is_key ? a.priv_k : a.priv_v) + (size_t(l) * R + pr) * kHd;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t d = (k >> 1) * 128 + 2 * lane + (k & 1);
+                to[d] = static_cast<uint16_t>(bits[k]);
+                out[d] = static_cast<uint16_t>(bits[k]);
+            }
+            if (bad) atomicOr(a.status, GUFFIN_STATUS_KV_NONFINITE);
+        }
+        if (owner) meet(); else own_lds();
+        second_request();
+        f4_t q[4];
+        const uint32_t first = t.first[R > 1 && r ? R - 1 : 0], end = t.end[R > 1 && r ? R - 1 : 0], attends = t.attends[R > 1 && r ? R - 1 : 0];
+        float m = -INFINITY, sum = 0.f, acc[16];
+        if (wave < ATTENDING) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = *reinterpret_cast<const f4_t*>(q_s + 128 * (k >> 1) + 8 * s16 + 4 * (k & 1));
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+        for (uint32_t chunk = t.t0; chunk < t.t1; chunk += kChunk) {
+            const uint32_t chunk_end = min(chunk + kChunk, t.t1);
+            if (wave < ATTENDING) {
+                const uint32_t mine = 4 * (wave % WPQ) + (lane >> 4);   // this lane's token of a round, from the chunk's first
+                float s[ROUNDS];
+                // a token's row: a private one, or the chunk's (past the last token zeros, or what the chunk before left)
+                auto row_at = [&](uint32_t at, const uint16_t (*ring)[kHd], const uint16_t (*priv)[kHd]) {
+                    return (owner && chunk + at >= t.n_ring && chunk + at < t.t1 ? priv[chunk + at - t.n_ring] : ring[min(at, kChunk - 1)]) + 8 * s16;
+                };
+#pragma unroll
+                for (uint32_t u = 0; u < ROUNDS; ++u) {
+                    s[u] = -INFINITY;
+                    if (chunk + STEP * u + 4 * (wave % WPQ) < chunk_end) {
+                        const uint32_t at = STEP * u + mine, token = chunk + at;
+                        const uint16_t* key = row_at(at, sh.k_s, sh.kp_s);
+                        float d[2];
+#pragma unroll
+                        for (int p = 0; p < 2; ++p) {
+                            const uint4 k4 = *reinterpret_cast<const uint4*>(key + 128 * p);
+                            const uint32_t w[4] = {k4.x, k4.y, k4.z, k4.w};
+                            d[p] = 0.f;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const half2_t h2 = __builtin_bit_cast(half2_t, w[i]);
+                                d[p] = fmaf(static_cast<float>(h2.x), q[2 * p + (i >> 1)][2 * (i & 1)], d[p]);
+                                d[p] = fmaf(static_cast<float>(h2.y), q[2 * p + (i >> 1)][2 * (i & 1) + 1], d[p]);
+                            }
+                        }
+                        const float dot = row16_sum(d[0] + d[1]);
+                        const uint32_t pos = t.u_first + token;
+                        const bool valid = token < chunk_end && (token >= t.n_ring ? ((attends >> (token - t.n_ring)) & 1u) != 0 : (pos >= first && pos < end));
+                        s[u] = valid ? dot : -INFINITY;
+                    }
+                }
+                float top = m;
+#pragma unroll
+                for (uint32_t u = 0; u < ROUNDS; ++u) top = fmaxf(top, s[u]);
+                const float base = top == -INFINITY ? 0.f : top;   // nothing attended so far: every weight is zero
+                if (chunk != t.t0) {
+                    const float keep = expf(m - base);
+                    sum *= keep;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[i] *= keep;
+                }
+                m = top;
+#pragma unroll
+                for (uint32_t u = 0; u < ROUNDS; ++u) {
+                    if (chunk + STEP * u + 4 * (wave % WPQ) < chunk_end) {
+                        const uint32_t at = STEP * u + mine;
+                        const uint16_t* value = row_at(at, sh.v_s, sh.vp_s);
+                        const float p = expf(s[u] - base);
+                        sum += p;
+                        if (chunk + at < chunk_end) {
+#pragma unroll
+                            for (int b = 0; b < 2; ++b) {
+                                const uint4 v4 = *reinterpret_cast<const uint4*>(value + 128 * b);
+                                const uint32_t w[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) {
+                                    const half2_t h2 = __builtin_bit_cast(half2_t, w[i]);
+                                    acc[8 * b + 2 * i] = fmaf(static_cast<float>(h2.x), p, acc[8 * b + 2 * i]);
+                                    acc[8 * b + 2 * i + 1] = fmaf(static_cast<float>(h2.y), p, acc[8 * b + 2 * i + 1]);
+                                }
+                            }
+                        }
+                    }
+                }
+            }
+            if (chunk + kChunk < t.t1) {   // a longer list: the next chunk takes this one's place
+                meet();
+                if (wave < kWorkers) {
+                    put_rows<R>(sh, rows, wave, lane);
+                    ask_rows<R>(rows, L.ring_k, L.ring_v, t, chunk + 2 * kChunk, wave, lane);
+                }
+                meet();
+            }
+        }
+        if (wave >= ATTENDING) return;
+        // the four token groups of the wave: a common maximum, then halves of the values exchanged for halves of the lanes
+        const float top = swap32_max(swap16_max(m)), base = top == -INFINITY ? 0.f : top, f = expf(m - base);
+        sum = swap32_sum(swap16_sum(sum * f));
+        float e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const u2_t x = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i] * f), __float_as_uint(acc[i + 8] * f), false, false);
+            e[i] = __uint_as_float(x.x) + __uint_as_float(x.y);
+        }
+        f4_t o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const u2_t x = __builtin_amdgcn_permlane16_swap(__float_as_uint(e[i]), __float_as_uint(e[i + 4]), false, false);
+            o[i] = __uint_as_float(x.x) + __uint_as_float(x.y);
+        }
+        const uint32_t at = (lane >> 5) * 128 + 8 * s16 + ((lane >> 4) & 1u) * 4;
+        if constexpr (WPQ == 1) {
+            st4(a.out_at, (slot * NQ + query) * kHd + at, o);
+            if (lane == 0) st2(a.ml_at, (slot * NQ + query) * 2, make_float2(top, sum));
+            arrived();
+        } else {
+            own_lds();   // the query has been read
+            *reinterpret_cast<f4_t*>(q_s + at) = o;
+            if (lane == 0) sh.ml[wave] = make_float2(top, sum);
+        }
+    }
+
+    // the last wave, where several share a query: the queries' outputs over this workgroup's tokens
+    __device__ __forceinline__ void publish_attention() {
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+            float top = sh.ml[n * WPQ].x;
+#pragma unroll
+            for (uint32_t j = 1; j < WPQ; ++j) top = fmaxf(top, sh.ml[n * WPQ + j].x);
+            const float base = top == -INFINITY ? 0.f : top;
+            f4_t o = {0.f, 0.f, 0.f, 0.f};
+            float sum = 0.f;
+#pragma unroll
+            for (uint32_t j = 0; j < WPQ; ++j) {
+                const float2 mj = sh.ml[n * WPQ + j];
+                const float f = expf(mj.x - base);
+                const f4_t oj = *reinterpret_cast<const f4_t*>(&sh.head[n * WPQ + j][4 * lane]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = fmaf(oj[i], f, o[i]);
+                sum = fmaf(mj.y, f, sum);
+            }
+            st4(a.out_at, (slot * NQ + n) * kHd + 4 * lane, o);
+            if (lane == 0) st2(a.ml_at, (slot * NQ + n) * 2, make_float2(top, sum));
+        }
+    }
+
+    // A worker's quads of a row: those of its own blocks, one a lane.
+    struct Own { Share blocks; bool on; uint32_t at; };
+    // The last of a row's sum of squares, over the workers' parts.  Every wave meets here.
+    __device__ __forceinline__ float row_total(int which, int r) const {
+        const f4_t lo = *reinterpret_cast<const f4_t*>(&sh.sums[which][r][0]), hi = *reinterpret_cast<const f4_t*>(&sh.sums[which][r][4]);
+        return ((lo.x + lo.y) + (lo.z + lo.w)) + ((hi.x + hi.y) + hi.z);
+    }
+    // x = x + rms(planes, post); the operand of this worker's blocks from rms(x, next).  Two meetings.
+    // outputs: also written to memory (the state after the last block of the launch).
+    template <typename First, typename Second, typename Third>
+    __device__ __forceinline__ void norm_pair(uint32_t planes, const f4_t& post, const f4_t& next, f4_t (&x)[R], const Own& own,
+                                              bool outputs, First first_request, Second second_request, Third third_request) {
+        const uint32_t H = a.H;
+        f4_t v[R], p1[R], p2[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            v[r] = ld4(planes, r * H + own.at);
+            p1[r] = ld4(planes, (R + r) * H + own.at);
+            p2[r] = ld4(planes, (2 * R + r) * H + own.at);
+        }
+        arrived();
+        first_request();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            v[r] = v[r] + p1[r] + p2[r];
+            float ss = (v[r].x * v[r].x + v[r].y * v[r].y) + (v[r].z * v[r].z + v[r].w * v[r].w);
+            ss = swap16_sum(row16_sum(own.on ? ss : 0.f));   // 24 lanes at most
+            if (lane == 0) sh.sums[0][r][wave] = ss;
+        }
+        meet();
+        second_request();
+        bool bad = false;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float inv = 1.0f / sqrtf(row_total(0, r) / static_cast<float>(H) + a.eps);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                x[r][i] = v[r][i] * inv * post[i] + x[r][i];
+                bad |= !isfinite(x[r][i]);
+            }
+            float ss = (x[r].x * x[r].x + x[r].y * x[r].y) + (x[r].z * x[r].z + x[r].w * x[r].w);
+            ss = swap16_sum(row16_sum(own.on ? ss : 0.f));
+            if (lane == 0) sh.sums[1][r][wave] = ss;
+        }
+        meet();
+        third_request();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float inv = 1.0f / sqrtf(row_total(1, r) / static_cast<float>(H) + a.eps);
+            f4_t u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) u[i] = x[r][i] * inv * next[i];
+            put_quad(u, lane, own.on, sh.opnd[wave][r], sh.mult[wave][r]);
+            if (outputs) {
+                float* row = sh.head[wave];   // attention is over: room for the wave's part of the row
+                if (own.on) {
+                    *reinterpret_cast<f4_t*>(a.x_out + size_t(r) * H + own.at) = x[r];
+                    *reinterpret_cast<f4_t*>(a.u_out + size_t(r) * H + own.at) = u;
+                    *reinterpret_cast<f4_t*>(row + 4 * lane) = u;
+                }
+                own_lds();
+                if (a.u_receipt_out && lane < 4 * own.blocks.count) {
+                    float y[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) y[i] = row[8 * lane + i];
+                    emit_receipt_values(y, 32 * own.blocks.first, lane, r, R, H, a.u_receipt_out);
+                }
+                own_lds();
+            }
+        }
+        if (bad && own.on) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
+        own_lds();
+    }
+
+    // ---- the eighth wave -------------------------------------------------------------------------------------
+    __device__ __forceinline__ void publisher() {
+        const uint32_t tiles = a.H / 64, part = uniform(slot / tiles), column = (slot - part * tiles) * 64 + lane;
+        for (uint32_t l = 0; l < a.layers; ++l) {
+            const DLayer& L = a.layer[l];
+            enter();
+            const Tokens<R> t = tokens_of<R>(sh, l, L.ring_mask, slot);
+            Rows none;
+            const HeadNorm gamma = ask_gamma(L);
+            stamp(l, 0);
+            meet();
+            if (slot < TA)
+#pragma unroll
+                for (int r = 0; r < R; ++r) st(a.qkv_at, r * CW + slot * 64 + lane, workers_sum(0, r));
+            arrive_and_wait();
+            stamp(l, 1);
+            meet();
+            attend(l, L, t, gamma, none, [] {}, [] {});
+            meet();
+            if constexpr (WPQ > 1) publish_attention();
+            arrive_and_wait();
+            stamp(l, 2);
+            meet();
+            // o-projection
+            meet();
+            stamp(l, 3);
+            if (part < kParts)
+#pragma unroll
+                for (int r = 0; r < R; ++r) st(a.o_at, (part * R + r) * a.H + column, workers_sum(0, r));
+            arrive_and_wait();
+            stamp(l, 4);
+            meet();
+            // norm pair, gate and up
+            meet();
+            meet();
+            meet();
+            stamp(l, 5);
+            if (slot < a.F / 64)
+#pragma unroll
+                for (int r = 0; r < R; ++r) st(a.h_at, r * a.F + slot * 64 + lane, geglu_value(workers_sum(0, r), workers_sum(1, r)));
+            arrive_and_wait();
+            stamp(l, 6);
+            meet();
+            // down
+            meet();
+            if (part < kParts)
+#pragma unroll
+                for (int r = 0; r < R; ++r) st(a.d_at, (part * R + r) * a.H + column, workers_sum(0, r));
+            arrive_and_wait();
+            stamp(l, 7);
+            meet();
+            // norm pair
+            meet();
+            meet();
+        }
+    }
+
+    // ---- the seven others ------------------------------------------------------------------------------------
+    __device__ __forceinline__ void worker() {
+        const uint32_t H = a.H, F = a.F, nb_h = H / 32, tiles = H / 64;
+        Own own;
+        own.blocks = share_of(nb_h, kWorkers, wave);             // blocks of the hidden width
+        own.blocks.first = min(own.blocks.first, nb_h - 1);      // (no blocks: the last one's requests, unused)
+        own.on = lane < 8 * own.blocks.count;
+        own.at = 32 * own.blocks.first + (own.on ? 4 * lane : 0u);
+        // q/k/v: a column tile a workgroup (workgroups past the last one repeat some tile's requests, unused)
+        const uint32_t qt = slot % TA;
+        const int qm = qt < 4 * G ? 0 : (qt < 4 * G + 4 ? 1 : 2);
+        const uint32_t q_tile = qm == 0 ? qt : qm == 1 ? qt - 4 * G : qt - 4 * G - 4;
+        const uint32_t q_at = uniform((q_tile * nb_h + own.blocks.first) * kTile);
+        // o: a column tile and a part of K, blocks by pairs (64 elements lie in one head)
+        const uint32_t row_part = uniform(slot / tiles), part = row_part < kParts ? row_part : 0, tile = slot - row_part * tiles;
+        const Share o_part = share_of(4 * G, kParts, part);
+        const bool o_on = wave < o_part.count;
+        const uint32_t o_pair = uniform(o_part.first + (o_on ? wave : 0u));
+        const uint32_t o_at = uniform((tile * (8 * G) + 2 * o_pair) * kTile);
+        // gate and up: a tile pair a workgroup
+        const uint32_t g_at = uniform(((slot % (F / 64)) * nb_h + own.blocks.first) * kTile);
+        // down: a column tile and a part of K
+        const Share d_part = share_of(F / 32, kParts, part), d_own = share_of(d_part.count, kWorkers, wave);
+        const uint32_t d_first = uniform(min(d_part.first + d_own.first, F / 32 - 1)), d_at = uniform((tile * (F / 32) + d_first) * kTile);
+
+        // Requests: a tile here and a tile there.  A wave's three to six at once, all waves at the same time, are 50 to 90 KB a
+        // workgroup, which one XCD takes 1.1 to 2 us to fetch (1.3 TB/s); in front of a phase's products that is what the products
+        // wait for, behind them what the last wave's store and poll do.
+        Tile tq[kOwn], to[kOwnO], tg[kOwn], tu[kOwn], td[kOwnDown];
+        f4_t post, next, x[R];
+        Rows rows;
+        HeadNorm gamma;
+        auto ask_q = [&](const DLayer& from, int i) { ask_tile(tq[i], from.tiles[qm] + q_at, i, own.blocks.count, lane); };
+        auto ask_o = [&](const DLayer& from, int i) { ask_tile(to[i], from.tiles[3] + o_at, i, 2, lane); };
+        auto ask_gate = [&](const DLayer& from, int i) { ask_tile(tg[i], from.tiles[4] + g_at, i, own.blocks.count, lane); };
+        auto ask_up = [&](const DLayer& from, int i) { ask_tile(tu[i], from.tiles[5] + g_at, i, own.blocks.count, lane); };
+        auto ask_down = [&](const DLayer& from, int i) { ask_tile(td[i], from.tiles[6] + d_at, i, d_own.count, lane); };
+        {
+            const DLayer& L = a.layer[0];
+#pragma unroll
+            for (int i = 0; i < kOwn; ++i) ask_q(L, i);
+            for (int i = 0; i < kOwnO; ++i) ask_o(L, i);
+            for (int i = 0; i < kOwn; ++i) ask_gate(L, i);
+            for (int i = 0; i < 1; ++i) ask_up(L, i);
+            const Tokens<R> t = tokens_of<R>(sh, 0, L.ring_mask, slot);
+            ask_rows<R>(rows, L.ring_k, L.ring_v, t, t.t0, wave, lane);
+            gamma = ask_gamma(L);
+        }
+        auto norm_weights = [&](const float* p, const float* n) {
+            const float4 vp = ldf4_a4(p + own.at), vn = ldf4_a4(n + own.at);
+            post = f4_t{vp.x, vp.y, vp.z, vp.w}; next = f4_t{vn.x, vn.y, vn.z, vn.w};
+        };
+        // the rows and the operand that the launch starts from
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            x[r] = *reinterpret_cast<const f4_t*>(a.x_in + size_t(r) * H + own.at);
+            const f4_t u = *reinterpret_cast<const f4_t*>(a.u_in + size_t(r) * H + own.at);
+            put_quad(u, lane, own.on, sh.opnd[wave][r], sh.mult[wave][r]);
+        }
+        own_lds();
+        auto publish = [&](const float (&acc)[R], int matrix) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) sh.red[wave][matrix][r][lane] = acc[r];
+        };
+        for (uint32_t l = 0; l < a.layers; ++l) {
+            const DLayer& L = a.layer[l];
+            const uint32_t ln = l + 1 < a.layers ? l + 1 : l;   // past the last block: this one's again, unused
+            const DLayer& N = a.layer[ln];
+            enter();
+            float acc[R];
+            // ---- q, k, v -----------------------------------------------------------------------------------
+            {
+                int op[R][2];
+                i4_t D[kOwn][R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) read_operand(op[r], sh.opnd[wave][r], lane);
+                steps(tq, op, D);
+                fold(tq, own.blocks.count, D, sh.mult[wave], acc);
+                publish(acc, 0);
+            }
+            put_rows<R>(sh, rows, wave, lane);
+            meet();
+            const Tokens<R> t = tokens_of<R>(sh, l, L.ring_mask, slot);
+            if (t.t0 + kChunk < t.t1) ask_rows<R>(rows, L.ring_k, L.ring_v, t, t.t0 + kChunk, wave, lane);
+            meet();
+            // ---- attention ---------------------------------------------------------------------------------
+            attend(l, L, t, gamma, rows, [&] { ask_up(L, 1); }, [&] { ask_up(L, 2); });
+            ask_down(L, 0);
+            ask_down(L, 1);
+            meet();
+            meet();
+            // ---- merge of the partitions for this wave's 64 elements, o-projection ------------------------
+            {
+                // 16 lanes hold the 64 elements, four each; lane group g the partitions 4 i + g
+                const uint32_t head = (64 * o_pair) / kHd, dim = (64 * o_pair) % kHd, g = lane >> 4, s16 = lane & 15u;
+                f4_t pv[R][kGroups / 4];
+                float2 ml[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const uint32_t n = r * G + head;
+                    ml[r] = ld2(a.ml_at, ((lane & 31u) * NQ + n) * 2);
+#pragma unroll
+                    for (uint32_t i = 0; i < kGroups / 4; ++i)
+                        pv[r][i] = ld4(a.out_at + (4 * i * NQ * kHd + n * kHd + dim) * 4, g * (NQ * kHd) + 4 * s16);
+                }
+                arrived();
+                ask_down(L, 2);
+                norm_weights(L.weights[0], L.weights[1]);
+                float den[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    float top = ml[r].y > 0.f ? ml[r].x : -INFINITY;
+                    top = swap16_max(row16_max(top));
+                    const float w = ml[r].y > 0.f ? expf(ml[r].x - top) : 0.f;
+                    den[r] = swap16_sum(row16_sum(w * ml[r].y));
+                    if (lane < kGroups) sh.weight[wave][r][8 * (lane & 3u) + (lane >> 2)] = w;
+                }
+                own_lds();
+                bool bad = false;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const f4_t w0 = *reinterpret_cast<const f4_t*>(&sh.weight[wave][r][8 * g]), w1 = *reinterpret_cast<const f4_t*>(&sh.weight[wave][r][8 * g + 4]);
+                    f4_t e = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (uint32_t i = 0; i < kGroups / 4; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) e[j] = fmaf(i < 4 ? w0[i & 3] : w1[i & 3], pv[r][i][j], e[j]);
+                    // element 4 s16 + g is left in this lane
+                    const u2_t x = __builtin_amdgcn_permlane32_swap(__float_as_uint(e.x), __float_as_uint(e.z), false, false);
+                    const u2_t y = __builtin_amdgcn_permlane32_swap(__float_as_uint(e.y), __float_as_uint(e.w), false, false);
+                    const u2_t z = __builtin_amdgcn_permlane16_swap(__float_as_uint(__uint_as_float(x.x) + __uint_as_float(x.y)),
+                                                                    __float_as_uint(__uint_as_float(y.x) + __uint_as_float(y.y)), false, false);
+                    const float v = (__uint_as_float(z.x) + __uint_as_float(z.y)) / den[r];
+                    bad |= o_on && !isfinite(v);
+                    uint32_t m = magnitude(v);
+                    m = max(m, lane_cross_u32<0xB1, 0xF>(m));
+                    m = max(m, lane_cross_u32<0x4E, 0xF>(m));
+                    m = max(m, lane_cross_u32<0x141, 0xF>(m));
+                    const u2_t m16 = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+                    m = max(m16.x, m16.y);
+                    const u2_t m32 = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+                    const GroupScale scale = group_scale(max(m32.x, m32.y));
+                    sh.opnd[wave][r][4 * s16 + g] = digits(v, scale.scale);
+                    if ((lane & 0x37u) == 0) sh.mult[wave][r][s16 >> 3] = scale.mult;
+                }
+                if (bad) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
+                ask_down(L, 3);
+                own_lds();
+                int op[R][1];
+                i4_t D[kOwnO][R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) read_operand(op[r], sh.opnd[wave][r], lane);
+                steps(to, op, D);
+                fold(to, o_on ? 2u : 0u, D, sh.mult[wave], acc);
+                publish(acc, 0);
+            }
+            meet();
+            meet();
+            // ---- x1 = x + rms(o, post_attention_norm); rms(x1, ffn_norm); gate and up ---------------------
+            norm_pair(a.o_at, post, next, x, own, false, [&] { ask_o(N, 0); ask_o(N, 1); }, [] {}, [] {});
+            {
+                int op[R][2];
+                i4_t D[kOwn][R], E[kOwn][R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) read_operand(op[r], sh.opnd[wave][r], lane);
+                steps(tg, op, D);
+                steps(tu, op, E);
+                fold(tg, own.blocks.count, D, sh.mult[wave], acc);
+                publish(acc, 0);
+                fold(tu, own.blocks.count, E, sh.mult[wave], acc);
+                publish(acc, 1);
+            }
+            meet();
+            meet();
+            // ---- down --------------------------------------------------------------------------------------
+            {
+                f4_t hv[R];
+                const uint32_t at = 32 * d_first + 4 * min(lane, 8 * max(d_own.count, 1u) - 1);
+#pragma unroll
+                for (int r = 0; r < R; ++r) hv[r] = ld4(a.h_at, r * F + at);
+                arrived();
+                ask_q(N, 0);
+                ask_q(N, 1);
+                ask_q(N, 2);
+                norm_weights(L.weights[2], L.weights[3]);
+#pragma unroll
+                for (int r = 0; r < R; ++r) put_quad(hv[r], lane, lane < 8 * d_own.count, sh.opnd[wave][r], sh.mult[wave][r]);
+                ask_gate(N, 0);
+                own_lds();
+                int op[R][2];
+                i4_t D[kOwnDown][R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) read_operand(op[r], sh.opnd[wave][r], lane);
+                steps(td, op, D);
+                fold(td, d_own.count, D, sh.mult[wave], acc);
+                publish(acc, 0);
+            }
+            meet();
+            const Tokens<R> tn = tokens_of<R>(sh, ln, N.ring_mask, slot);
+            meet();
+            // ---- x = x1 + rms(down, post_ffw_norm); rms(x, next block's attn_norm or the output norm) -----
+            norm_pair(a.d_at, post, next, x, own, l + 1 == a.layers && slot == 0, [&] { ask_gate(N, 1); },
+                      [&] { ask_gate(N, 2); ask_rows<R>(rows, N.ring_k, N.ring_v, tn, tn.t0, wave, lane); gamma = ask_gamma(N); }, [&] { ask_up(N, 0); });
+        }
+    }
+};
+
+template <int R, int G>
+__global__ void __launch_bounds__(kThreads) drafter_blocks_kernel(const DArgs a) {
+    __shared__ __attribute__((aligned(256))) Shared<R> sh;
+    if (xcc_id() != 0) return;   // the model has one KV head: the other XCDs leave at once
+    const uint32_t lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+    Pass<R, G> pass {a, sh, lane, wave, blockIdx.x / 8, 0, __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, static_cast<int>(a.exchange_bytes), 0x00020000)};
+    // The arguments' lines, once, all at a time: they come from far, and a block's pointers otherwise cost a wait at each first use.
+    {
+        uint64_t seen = 0;
+        const uint64_t* words = reinterpret_cast<const uint64_t*>(&a);
+#pragma unroll
+        for (uint32_t i = 0; i < sizeof(DArgs) / 64; ++i) seen ^= words[8 * i];
+        asm volatile("" ::"s"(seen));
+    }
+    // the rotations and the schedules
+    if (threadIdx.x == 0) sh.dead = 0;
+    for (uint32_t i = threadIdx.x; i < 2 * R * (kHd / 2); i += kThreads) {
+        const uint32_t at = i % (R * (kHd / 2));
+        (&sh.rope[0][0][0])[i] = i < R * (kHd / 2) ? a.rope_local[at] : a.rope_global[at];
+    }
+    for (uint32_t i = threadIdx.x; i < a.layers * R; i += kThreads) {
+        const uint32_t* s = a.schedule + 4 * i;
+        uint32_t attends = 0;
+        for (uint32_t k = 0; k < s[3]; ++k) attends |= 1u << a.ancestors[s[2] + k];
+        uint32_t* to = sh.schedule[i / R][i % R];
+        to[0] = s[0]; to[1] = s[1]; to[2] = attends;
+    }
+    __syncthreads();
+    if (wave == kWorkers) pass.publisher();
+    else pass.worker();
+}
+
+}  // namespace
+
+// Widths whose tiles a workgroup's waves hold: three blocks of the hidden width a worker, a gate / up pair a workgroup.
+bool drafter_pass_fits(const guffin_model_desc& m) {
+    if (m.kv_heads != 1 || m.head_dim != kHd || (m.q_heads != 1 && m.q_heads != 2 && m.q_heads != 4)) return false;
+    if (uint64_t(std::max(m.ring_local, m.ring_global)) * 2 * kHd >= (uint64_t(1) << 31)) return false;   // 32-bit offsets into a ring
+    if (m.hidden % 64 || m.hidden > kMaxWidth || m.ffn % 64 || m.ffn > kMaxFfn) return false;
+    for (uint32_t l = 0; l < m.layer_count; ++l)
+        for (int i = 0; i < 7; ++i)
+            if (m.layers[l].dtype[i] != GUFFIN_Q8_0) return false;
+    return true;
+}
+
+int drafter_pass(hipStream_t stream, const guffin_model_desc& m, uint32_t rows, const DrafterPass& p) {
+    DArgs a {};
+    a.H = m.hidden; a.F = m.ffn; a.eps = m.eps; a.scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
+    a.exchange = p.exchange;
+    const uint32_t NQ = rows * m.q_heads;
+    uint32_t used = 0;
+    auto take = [&](uint32_t floats) {   // regions start on cache lines of their own
+        const uint32_t at = used;
+        used += (floats * 4 + 255) & ~255u;
+        return at;
+    };
+    a.qkv_at = take(rows * (m.q_heads + 2) * kHd);
+    a.out_at = take(kGroups * NQ * kHd);
+    a.ml_at = take(kGroups * NQ * 2);
+    a.o_at = take(kParts * rows * m.hidden);
+    a.d_at = take(kParts * rows * m.hidden);
+    a.h_at = take(rows * m.ffn);
+    a.exchange_bytes = used;
+    if (used > resident_scratch_bytes(m, rows)) return fail(GUFFIN_E_CAPACITY, "drafter pass: exchange buffers");
+    a.rope_local = reinterpret_cast<const float2*>(p.rope_local); a.rope_global = reinterpret_cast<const float2*>(p.rope_global);
+    a.ancestors = p.ancestors; a.status = p.status; a.spin_limit = g_spin_limit;
+    for (uint32_t first = 0, n = 0; first < m.layer_count; first += kLayers, ++n) {
+        a.layers = std::min(kLayers, m.layer_count - first);
+        for (uint32_t i = 0; i < a.layers; ++i) {
+            const uint32_t l = first + i;
+            const guffin_layer_desc& L = m.layers[l];
+            DLayer& d = a.layer[i];
+            for (int k = 0; k < 7; ++k) d.tiles[k] = static_cast<const uint8_t*>(L.tiles[k]);
+            for (int k = 0; k < 3; ++k) d.weights[k] = L.norm[3 + k];
+            d.weights[3] = l + 1 == m.layer_count ? m.out_norm : m.layers[l + 1].norm[0];
+            d.weights[4] = L.norm[1]; d.weights[5] = L.norm[2];
+            d.ring_k = static_cast<const uint16_t*>(L.ring_k); d.ring_v = static_cast<const uint16_t*>(L.ring_v);
+            d.local = layer_is_local(m.global_period, l) ? 1u : 0u;
+            d.ring_mask = (d.local ? m.ring_local : m.ring_global) - 1;
+        }
+        const bool last = first + a.layers == m.layer_count;
+        a.sync = p.sync + n * kSyncStride;
+        a.schedule = p.schedule + size_t(first) * rows * 4;
+        a.priv_k = static_cast<uint16_t*>(p.priv_k) + size_t(first) * rows * kHd;
+        a.priv_v = static_cast<uint16_t*>(p.priv_v) + size_t(first) * rows * kHd;
+        a.x_in = p.x; a.u_in = p.u; a.x_out = p.x;
+        a.u_out = last ? p.out_hidden : p.u;
+        a.u_receipt_out = last ? p.out_sums : nullptr;
+        a.stamps = g_resident_stamps ? g_resident_stamps + size_t(first) * 16 : nullptr;
+        switch (rows * 10 + m.q_heads) {
+            case 11: launch(drafter_blocks_kernel<1, 1>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+            case 12: launch(drafter_blocks_kernel<1, 2>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+            case 14: launch(drafter_blocks_kernel<1, 4>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+            case 21: launch(drafter_blocks_kernel<2, 1>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+            case 22: launch(drafter_blocks_kernel<2, 2>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+            case 24: launch(drafter_blocks_kernel<2, 4>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+            default: return fail(GUFFIN_E_SHAPE, "drafter pass: unsupported head grouping");
+        }
+        if (int rc = check_launch("drafter_blocks")) return rc;
+    }
+    return GUFFIN_OK;
+}
+
+}  // namespace guffin

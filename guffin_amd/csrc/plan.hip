@@ -13,6 +13,7 @@
 // caller can capture a whole step into a HIP graph.
 #include <cstddef>
 #include "common.hpp"
+#include "resident.hpp"
 #include "selection_request.hpp"
 #include "receipt.hpp"
 #include "prefill_run.hpp"
@@ -269,6 +270,9 @@ int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t*
     GUFFIN_TRY(guffin_hip_embed(st, m.embed_dtype, m.embed_rows, tokens, s.x, rows, H,
                                 std::sqrt(static_cast<float>(H)), m.vocab, status));
     GUFFIN_TRY(guffin_hip_rms_norm(st, s.x, 1, 0, m.layers[0].norm[0], nullptr, s.u, s.us, rows, H, m.eps, status));
+    if (resident && drafter_pass_fits(m))
+        return drafter_pass(stream, m, rows, {s.exchange, s.sync, s.rope_local, s.rope_global, s.schedule, s.ancestors, priv_k, priv_v,
+                                              s.x, s.u, out_hidden, out_hidden_sums, status});
     if (resident) {
         // groups of blocks, each one launch whose workgroups stay on the chip; the residual rows and the
         // normalised rows' receipt pass from launch to launch through s.x / s.us

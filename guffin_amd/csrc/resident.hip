@@ -14,7 +14,8 @@
 // addresses this CU has not read before in the launch (a set of exchange buffers per block, so that no line
 // of the L1 can be stale).  Across XCDs the partial planes are written through (sc1 stores)
 // and read with sc1 loads after a two-level barrier (XCD counter, then one device counter).
-// A model with one KV head (the drafter) runs on the 32 CUs of XCD 0; the others leave at once.
+// A model with one KV head runs on the 32 CUs of XCD 0; the others leave at once.  (A narrow Q8_0 one, the drafter, has a pass of
+// its own, drafter_pass.hip.)
 //
 // Every wait is bounded: a workgroup that gives up raises GUFFIN_STATUS_SYNC, stops waiting for the
 // rest of the launch and still runs to the end, so the grid always drains.  Placement (workgroup i
@@ -24,6 +25,7 @@
 #include "common.hpp"
 #include "receipt.hpp"
 #include "gemv_tiles.hpp"
+#include "resident.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -31,13 +33,10 @@
 namespace guffin {
 namespace {
 
-constexpr uint32_t kGroups = 32;        // workgroups per XCD
 constexpr uint32_t kWaves = 8;          // waves per workgroup: two per SIMD, 256 registers each
 constexpr uint32_t kThreads = 512;
-constexpr uint32_t kGrid = 256;
 constexpr uint32_t kRowThreads = 256;   // threads that hold one row of the residual stream (two runs of 8 columns each)
 constexpr uint32_t kRowItems = 2;       // runs of 8 columns per thread: run i of thread t covers columns 8 * (t + 256 i) ..
-constexpr uint32_t kHd = 256;
 constexpr uint32_t kSyncWords = 64 * (2 * 8 + 2);   // per launch: 8 counter lines, 8 flag lines, device counter, spare
 
 struct RLayer {
@@ -71,12 +70,6 @@ struct RArgs {
     uint32_t set_floats, vec_floats;   // floats between the exchange buffers of consecutive blocks; floats of one `vec`
     unsigned long long* stamps;   // profiling aid: 8 clock readings per block from workgroup 0, or null
 };
-
-__device__ __forceinline__ uint32_t xcc_id() {
-    uint32_t v;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(v));
-    return v & 0xFu;
-}
 
 // ---- loads of data another workgroup wrote during this launch ----------------------------------
 // Plain vector loads: every call site indexes by thread, so none is served by the scalar cache, and the

@@ -473,7 +473,8 @@ int guffin_hip_set_spin_limit(uint32_t polls);
  * 100 MHz clock at the start of each block's q/k/v projection, attention, o-projection, first norm pair,
  * gate/up, down projection, second norm pair, and at the block's end (words 0-7 of the block), and inside the
  * first norm pair after the device-wide wait, the slice sums, the XCD-wide wait and the first row sum (words
- * 8-11).  NULL (default) switches it off. */
+ * 8-11).  The drafter's own pass stores words 0-7 when q/k/v, the attention, the o-projection, its sums, the first norm pair with
+ * gate/up, their sums, the down projection and the second norm pair begin.  NULL (default) switches it off. */
 int guffin_hip_set_resident_stamps(void* device_words);
 
 /* Publishes private rows into the rings of every layer at slot (position + row) & mask: all

@@ -1,0 +1,92 @@
+"""The drafter's pass on one XCD (drafter_pass.hip) at the edges of what it covers, against the launch-per-operator pass on the
+same model and rows and against the CPU oracle: head groupings (how many waves share a query), widths where workers have no
+blocks or the column tiles leave workgroups idle, token lists of one chunk of 20 a workgroup, of just more and of several,
+windows that begin inside a ring, more blocks than a launch takes.
+
+Bounds as for the resident pass (test_gpu_resident.py): the same products and sums of them in another order, 1e-4 of the row
+RMS; 1e-3 against the oracle; fp16 K/V rows equal but for roundings that fall the other way, none off by more than a step."""
+from dataclasses import replace
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from guffin_amd import hip as module
+    module.init(0)
+    yield module
+    module.set_forward_mode(0)
+
+
+def rel_rms(got, want):
+    want = want.astype(np.float64)
+    scale = np.sqrt((want ** 2).mean(axis=-1, keepdims=True)) + 1e-30
+    return float(np.max(np.abs(got.astype(np.float64) - want) / scale))
+
+
+# heads, hidden, ffn, layers, rows, position
+CASES = [(4, 640, 2048, 2, 1, 0), (4, 640, 2048, 2, 2, 0), (4, 640, 2048, 2, 1, 511), (4, 640, 2048, 2, 2, 512),
+         (4, 640, 2048, 1, 1, 639), (4, 640, 2048, 1, 2, 638), (4, 640, 2048, 1, 1, 640), (4, 640, 2048, 7, 2, 1400),
+         (2, 640, 2048, 2, 1, 700), (2, 640, 2048, 2, 2, 31), (1, 640, 2048, 2, 1, 700), (1, 640, 2048, 2, 2, 63),
+         (4, 64, 256, 2, 1, 100), (4, 64, 256, 2, 2, 20), (2, 256, 512, 2, 2, 90), (1, 576, 1792, 2, 1, 33),
+         (4, 512, 1024, 2, 2, 300), (4, 64, 256, 26, 1, 70), (2, 64, 256, 25, 2, 5)]
+
+
+@pytest.mark.parametrize("heads,hidden,ffn,layers,rows,position", CASES)
+def test_the_pass_equals_the_per_operator_pass(hip, gfo, heads, hidden, ffn, layers, rows, position):
+    import torch
+    from guffin_amd import model
+    # every second block global, so that short models see lists beyond the window too
+    shape = replace(model.GEMMA3_270M, layers=layers, vocab=1024, ring_global=2048, q_heads=heads, hidden=hidden, ffn=ffn,
+                    global_period=2)
+    host = model.HostModel(shape, seed=3 + layers + heads, position=position)
+    devm = model.DeviceModel.from_host(host)
+    tokens = torch.tensor([17, 999][:rows], dtype=torch.int32, device="cuda")
+    print("drafter pass", heads, hidden, ffn, layers, rows, position, flush=True)
+    hip.set_forward_mode(1)
+    want = devm.forward(tokens, position)
+    torch.cuda.synchronize()
+    hip.set_forward_mode(2)
+    got = devm.forward(tokens, position)
+    again = devm.forward(tokens, position)
+    torch.cuda.synchronize()
+    hip.set_forward_mode(0)
+    assert int(want[4].item()) == 0 and int(got[4].item()) == 0
+    for g, a in zip((got[0], got[2], got[3]), (again[0], again[2], again[3])):
+        assert torch.equal(g, a)
+    # A chain of 25 narrow blocks: a K/V element that two sums put on either side of a rounding (relative difference e: 2^12 e of
+    # them, the spacing of halves being 2^-11 or more) is off by 2^-11 and every later block goes on with that.  The bound is the
+    # oracle's then, and the share of equal patterns, which that difference no longer bounds, is not asked for.
+    deep = layers > 7
+    loose = 1e-3 if deep else 1e-4
+    assert rel_rms(got[0].cpu().numpy(), want[0].cpu().numpy()) <= loose
+    for g, w in ((got[2], want[2]), (got[3], want[3])):
+        gb, wb = g.view(torch.int16).cpu().numpy(), w.view(torch.int16).cpu().numpy()
+        assert deep or np.mean(gb == wb) >= 0.98
+        d = np.abs(g.float().cpu().numpy() - w.float().cpu().numpy())
+        assert d.max() <= 2.0 ** -9 * float(w.float().abs().max()) + 1e-6
+    oracle, _, _ = gfo.forward(host, tokens.cpu().numpy().view(np.uint32), position, threads=8)
+    assert rel_rms(got[0].cpu().numpy(), oracle) <= 1e-3
+
+
+def test_a_row_keeps_a_nan_and_says_so(hip):
+    """A non-finite row in a ring's values reaches the hidden row and the status word, as in the per-operator pass: an operand
+    group with a NaN has no fixed-point digits, its multiplier carries the NaN instead."""
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=2, vocab=1024, ring_global=1024)
+    devm = model.DeviceModel.from_host(model.HostModel(shape, seed=9, position=100))
+    devm.ring_v[0][50].fill_(float("nan"))
+    tokens = torch.tensor([5], dtype=torch.int32, device="cuda")
+    words = []
+    for mode in (1, 2):
+        hip.set_forward_mode(mode)
+        out = devm.forward(tokens, 100)
+        torch.cuda.synchronize()
+        words.append(int(out[4].item()))
+        assert not bool(torch.isfinite(out[0]).any())
+    hip.set_forward_mode(0)
+    assert words[0] != 0 and words[0] == words[1]
