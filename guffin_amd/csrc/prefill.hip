@@ -190,6 +190,12 @@ __device__ __forceinline__ void emit_attention(const AttentionOut& to, const flo
     }
 }
 
+// whether the merge of a workgroup's waves has room for all of their outputs, and its LDS
+template <int NT> constexpr bool kMergeAtOnce = NT == 1;
+constexpr uint32_t attention_lds(uint32_t nt) {
+    return nt == 1 ? 4 * 16384 + 5 * 16 * 2 * 4 : nt * (16384 + 4 * 16 * 32 * 4 + 16 * 2 * 4);
+}
+
 // grid (ceil(rows * group / (16 NT)), kv_heads, parts), 4 waves.  A workgroup serves 16 NT (row, head) pairs of one KV head
 // -- the group's heads of 16 NT / group consecutive rows, as NT A tiles of 16 pairs -- and one part of the key range.  Each
 // wave walks its own 32-token tiles (tile index = wave mod 4) with its own online softmax state and its own output
@@ -261,9 +267,17 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
 #pragma unroll
         for (int dt = 0; dt < 16; ++dt) O[g][dt] = float4_t{0.f, 0.f, 0.f, 0.f};
     }
+    constexpr int VB = NT > 1 ? 8 : 16;   // one A tile: all values of a tile in registers, asked for ahead of the scores
     for (uint32_t ti = begin + wave; ti < end; ti += 4) {
         const uint32_t t0 = base32 + 32 * ti;
         if constexpr (NT > 1) ask_keys(ti, kb);
+        const uint16_t* vcol = vt + (size_t(kvh) * HD + j) * T + (t0 - base32) + 8 * lg;
+        uint4 vb[VB];
+        auto ask_values = [&](int first) {
+#pragma unroll
+            for (int i = 0; i < VB; ++i) vb[i] = *reinterpret_cast<const uint4*>(vcol + size_t(16 * (first + i)) * T);
+        };
+        if constexpr (NT == 1) ask_values(0);
         // A sum rounds at the size it has grown to: the hi halves of the first four steps are one chain; the other takes the lo
         // halves, whose sums are small, and from the fifth step on both.
         float4_t S[NT][2], rest[NT][2];
@@ -286,13 +300,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
 #pragma unroll
             for (int c = 0; c < 2; ++c) S[g][c] += rest[g][c];
         if constexpr (NT > 1) __builtin_amdgcn_sched_barrier(0);   // the keys' registers become the values'
-        const uint16_t* vcol = vt + (size_t(kvh) * HD + j) * T + (t0 - base32) + 8 * lg;
-        uint4 vb[8];
-        auto ask_values = [&](int first) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) vb[i] = *reinterpret_cast<const uint4*>(vcol + size_t(16 * (first + i)) * T);
-        };
-        ask_values(0);
+        if constexpr (NT > 1) ask_values(0);
         // online softmax of the lane group's four pairs of a tile; a pair's 32 scores sit in 16 lanes x 2
         if (!(t0 >= last_first && t0 + 31 <= position + r0)) {
 #pragma unroll
@@ -357,56 +365,87 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
 #pragma unroll
             for (int half = 0; half < 2; ++half)
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
+                for (int i = 0; i < VB; ++i)
 #pragma unroll
                     for (int g = 0; g < NT; ++g)
                         O[g][first + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[g][half], __builtin_bit_cast(half8_t, vb[i]), O[g][first + i], 0, 0, 0);
         };
-        values(0);
-        if constexpr (NT > 1) __builtin_amdgcn_sched_barrier(0);
-        ask_values(8);
         if constexpr (NT == 1) {
             if (ti + 4 < end) ask_keys(ti + 4, kb);
+            values(0);
+        } else {
+            values(0);
+            __builtin_amdgcn_sched_barrier(0);
+            ask_values(8);
+            values(8);
         }
-        values(8);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     // merge the four waves' states in wave order through LDS (the query operands are dead now)
     float* ob = reinterpret_cast<float*>(qa);  // [(g * 16 + dt) * 4 + r][lane]
-    for (uint32_t w = 0; w < 4; ++w) {
+    constexpr uint32_t kWaveSlots = NT * 4096;   // of one wave's outputs
+    if constexpr (kMergeAtOnce<NT>) {
+        // every wave's outputs have room: scaled to the common maximum by their own wave, summed by whoever stores them.  (One
+        // wave behind the other over the same slots, as below: three more passes over them.  With the values asked for ahead of the scores 12 rows at
+        // position 100 take 11.1 instead of 12.4 us, 37 at 1500 16.1 instead of 16.8.)
+        float* states = reinterpret_cast<float*>(lds + 4 * kWaveSlots * 4);   // [wave][pair][2]
+        ml = states + 4 * kPairs * 2;
         __syncthreads();
-        if (wave != w) continue;
+        if (j == 0)
 #pragma unroll
-        for (int g = 0; g < NT; ++g)
+            for (int r = 0; r < 4; ++r) *reinterpret_cast<float2*>(states + (wave * kPairs + 4 * lg + r) * 2) = make_float2(m[0][r], l[0][r]);
+        __syncthreads();
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float* slots = ob + (g * 64 + r) * 64 + lane;   // [dt][4][64]
-                if (w == 0) {
+        for (int r = 0; r < 4; ++r) {
+            float2 st[4];
 #pragma unroll
-                    for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r];
-                    continue;
-                }
-                const float mo = ml[(g * 16 + 4 * lg + r) * 2], lo_ = ml[(g * 16 + 4 * lg + r) * 2 + 1];
-                const float M = fmaxf(m[g][r], mo);
-                const float mine = m[g][r] == -INFINITY ? 0.f : exp_of(m[g][r] - M), theirs = mo == -INFINITY ? 0.f : exp_of(mo - M);
-                l[g][r] = l[g][r] * mine + lo_ * theirs;
-                m[g][r] = M;
+            for (int w = 0; w < 4; ++w) st[w] = *reinterpret_cast<const float2*>(states + (w * kPairs + 4 * lg + r) * 2);
+            const float M = fmaxf(fmaxf(st[0].x, st[1].x), fmaxf(st[2].x, st[3].x));
+            float den = 0.f;
 #pragma unroll
-                for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r] * mine + slots[dt * 256] * theirs;
-            }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (j == 0) {
+            for (int w = 0; w < 4; ++w) den += st[w].x == -INFINITY ? 0.f : st[w].y * exp_of(st[w].x - M);
+            const float mine = m[0][r] == -INFINITY ? 0.f : exp_of(m[0][r] - M);
+            float* slots = ob + wave * kWaveSlots + r * 64 + lane;
 #pragma unroll
+            for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[0][dt][r] * mine;
+            if (wave == 0 && j == 0) *reinterpret_cast<float2*>(ml + (4 * lg + r) * 2) = make_float2(M, den);
+        }
+    } else {
+        for (uint32_t w = 0; w < 4; ++w) {
+            __syncthreads();
+            if (wave != w) continue;
+    #pragma unroll
             for (int g = 0; g < NT; ++g)
-#pragma unroll
+    #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    ml[(g * 16 + 4 * lg + r) * 2] = m[g][r];
-                    ml[(g * 16 + 4 * lg + r) * 2 + 1] = l[g][r];
+                    float* slots = ob + (g * 64 + r) * 64 + lane;   // [dt][4][64]
+                    if (w == 0) {
+    #pragma unroll
+                        for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r];
+                        continue;
+                    }
+                    const float mo = ml[(g * 16 + 4 * lg + r) * 2], lo_ = ml[(g * 16 + 4 * lg + r) * 2 + 1];
+                    const float M = fmaxf(m[g][r], mo);
+                    const float mine = m[g][r] == -INFINITY ? 0.f : exp_of(m[g][r] - M), theirs = mo == -INFINITY ? 0.f : exp_of(mo - M);
+                    l[g][r] = l[g][r] * mine + lo_ * theirs;
+                    m[g][r] = M;
+    #pragma unroll
+                    for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r] * mine + slots[dt * 256] * theirs;
                 }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (j == 0) {
+    #pragma unroll
+                for (int g = 0; g < NT; ++g)
+    #pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        ml[(g * 16 + 4 * lg + r) * 2] = m[g][r];
+                        ml[(g * 16 + 4 * lg + r) * 2 + 1] = l[g][r];
+                    }
+            }
         }
     }
     __syncthreads();
@@ -417,7 +456,10 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         const float* src = ob + ((((p >> 4) * 16 + (c8 >> 1)) * 4 + (i & 3)) * 64 + 8 * (c8 & 1) + 16 * (i >> 2));
         float v[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = src[k];
+        for (int k = 0; k < 8; ++k) {
+            v[k] = src[k];
+            if constexpr (kMergeAtOnce<NT>) v[k] += src[kWaveSlots + k] + src[2 * kWaveSlots + k] + src[3 * kWaveSlots + k];
+        }
         if (gridDim.z == 1) {
             const float den = ml[p * 2 + 1] * kProbScale;
 #pragma unroll
@@ -440,17 +482,39 @@ prefill_attention_merge_kernel(AttentionOut to, uint32_t rows, uint32_t q_heads,
     const uint32_t pair = blockIdx.x * 8 + threadIdx.x / 32, c8 = threadIdx.x % 32;
     if (pair >= rows * q_heads) return;
     const size_t stride = size_t(rows) * q_heads;
-    float M = -INFINITY;
-    for (uint32_t p = 0; p < parts; ++p) M = fmaxf(M, to.part_ml[2 * (p * stride + pair)]);
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, den = 0.f;
-#pragma unroll 4
-    for (uint32_t p = 0; p < parts; ++p) {
-        const size_t at = p * stride + pair;
-        const float mp = to.part_ml[2 * at], w = mp == -INFINITY ? 0.f : exp_of(mp - M);   // a part can hold no visible token
-        den += w * to.part_ml[2 * at + 1];
-        const float4 a = *reinterpret_cast<const float4*>(to.part_o + at * HD + 8 * c8), b = *reinterpret_cast<const float4*>(to.part_o + at * HD + 8 * c8 + 4);
-        v[0] = fmaf(w, a.x, v[0]); v[1] = fmaf(w, a.y, v[1]); v[2] = fmaf(w, a.z, v[2]); v[3] = fmaf(w, a.w, v[3]);
-        v[4] = fmaf(w, b.x, v[4]); v[5] = fmaf(w, b.y, v[5]); v[6] = fmaf(w, b.z, v[6]); v[7] = fmaf(w, b.w, v[7]);
+    // a lane a part's state, 32 at a time: their maximum and weights are two reductions instead of a walk of one trip a part
+    const float2* states = reinterpret_cast<const float2*>(to.part_ml);
+    auto top_of = [](float x) { x = row16_max(x); return fmaxf(x, __shfl_xor(x, 16, kWave)); };
+    auto sum_of = [](float x) { x = row16_sum(x); return x + __shfl_xor(x, 16, kWave); };
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, den = 0.f, M = -INFINITY;
+    for (uint32_t p0 = 0; p0 < parts; p0 += 32) {
+        const float2 st = p0 + c8 < parts ? states[(p0 + c8) * stride + pair] : make_float2(-INFINITY, 0.f);   // a part can hold no visible token
+        const float top = fmaxf(M, top_of(st.x)), base = top == -INFINITY ? 0.f : top;
+        if (p0) {
+            const float keep = exp_of(M - base);
+            den *= keep;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] *= keep;
+        }
+        M = top;
+        const float w = exp_of(st.x - base);
+        den += sum_of(w * st.y);
+        const uint32_t n = min(parts - p0, 32u);
+        for (uint32_t i0 = 0; i0 < n; i0 += 8) {
+            float4 a[8], b[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) {
+                const float* src = to.part_o + ((p0 + min(i0 + i, n - 1)) * stride + pair) * HD + 8 * c8;
+                a[i] = *reinterpret_cast<const float4*>(src); b[i] = *reinterpret_cast<const float4*>(src + 4);
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) {
+                const float wi = __shfl(w, (threadIdx.x & 32u) + min(i0 + i, 31u), kWave), f = i0 + i < n ? wi : 0.f;
+                if (f == 0.f) continue;   // nothing of a part without tokens, whatever it left
+                v[0] = fmaf(f, a[i].x, v[0]); v[1] = fmaf(f, a[i].y, v[1]); v[2] = fmaf(f, a[i].z, v[2]); v[3] = fmaf(f, a[i].w, v[3]);
+                v[4] = fmaf(f, b[i].x, v[4]); v[5] = fmaf(f, b[i].y, v[5]); v[6] = fmaf(f, b[i].z, v[6]); v[7] = fmaf(f, b[i].w, v[7]);
+            }
+        }
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] /= den * kProbScale;
@@ -606,6 +670,12 @@ AttentionCut attention_cut(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_
     if (twos >= cus) return {2, 1};
     return {1, std::max(1u, std::min(2 * cus / ones, T / 128))};
 }
+// more than 64 KB of LDS a workgroup has to be allowed once per kernel
+int allow_attention_lds() {
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_attention_mfma_kernel<1>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, attention_lds(1));
+    return allowed == hipSuccess ? GUFFIN_OK : fail(GUFFIN_E_HIP, "prefill_attention: could not raise the dynamic LDS limit");
+}
 uint64_t transposed_bytes(uint32_t T, uint32_t kv_heads) { return (uint64_t(kv_heads) * 256 * T * 2 + 255) & ~uint64_t{255}; }
 }  // namespace
 
@@ -644,7 +714,8 @@ int prefill_attention_run(hipStream_t s, const float* q, const void* ring_k, con
     const auto [nt, parts] = attention_cut(rows, vs.T, kv_heads, group);
     float* states = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + transposed_bytes(vs.T, kv_heads));
     const AttentionOut to {out, image, states, states + size_t(parts) * rows * q_heads * 256};
-    const size_t lds = nt * (16384 + 4 * 16 * 32 * 4 + 16 * 2 * 4);
+    const uint32_t lds = attention_lds(nt);
+    if (int rc = allow_attention_lds()) return rc;
     const dim3 grid((rows * group + 16 * nt - 1) / (16 * nt), kv_heads, parts);
 #define GUFFIN_PA(NT_) launch(prefill_attention_mfma_kernel<NT_>, grid, dim3(256), lds, s, q, static_cast<const uint16_t*>(ring_k), \
                               static_cast<const uint16_t*>(run_k), static_cast<const uint16_t*>(workspace), to, rows, position, window, \

@@ -85,7 +85,10 @@ prefill_norm_kernel(const float* __restrict__ x, const float* __restrict__ gamma
 }
 
 // Workgroups [0, rows): one row each.  The rest copy the run's fp16 K/V rows to their ring slots, 16 bytes per thread.
-__global__ void __launch_bounds__(1024)
+// B planes are requested at a time: a short run has up to 16 and few workgroups, and is bound by the trips (37 rows, 15 planes:
+// 8.4 us by eights, 8.1 at once; 12 rows 8.0 and 7.5); THREADS: the widest row's.
+template <int B, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_stride, const float* __restrict__ gamma_post,
                      const float* __restrict__ residual, float* __restrict__ out_residual, const float* __restrict__ gamma_next,
                      float* __restrict__ out_norm, uint8_t* __restrict__ image, uint32_t rows, uint32_t width, float eps,
@@ -108,7 +111,7 @@ prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_
         load8_words(gamma_post + 8 * t, gp);
         load8(residual + at, res);
         load8_words(gamma_next + 8 * t, gn);
-        sum_planes8<8>(x + at, planes, plane_stride, v);
+        sum_planes8<B>(x + at, planes, plane_stride, v);
     }
     float ss = 0.f;
 #pragma unroll
@@ -160,16 +163,20 @@ prefill_geglu_kernel(const float* __restrict__ gate, const float* __restrict__ u
     }
 }
 
-// Workgroups [0, head_groups): four (row, query or key head) pairs, a wave each.  The rest: 32 visible tokens of one KV
+// Workgroups [0, head_groups): sixteen (row, query or key head) pairs, a wave each.  The rest: 32 visible tokens of one KV
 // head's values each, from the ring or (the run's own, narrowed and kept on the way) from the planes, written transposed.
-__global__ void __launch_bounds__(256)
+// Bound by its trips in a short run, so a thread has eight elements of one token and asks for eight planes at a time (with four
+// tokens one behind the other, by fours, 15 planes were sixteen trips: 12 rows at position 100 9.1 us, 37 at 1500 11.8, 2048 at 0 30.0; now
+// 6.4, 7.5 and 29.0).
+constexpr uint32_t kQkvThreads = 1024;
+__global__ void __launch_bounds__(kQkvThreads)
 prefill_qkv_kernel(QkvRun a) {
     constexpr uint32_t HD = 256, PITCH = HD + 8;
     __shared__ __attribute__((aligned(16))) uint16_t tile[32][PITCH];
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     bool bad = false;
     if (blockIdx.x < a.head_groups) {
-        const uint32_t per_row = a.q_heads + a.kv_heads, p = blockIdx.x * 4 + wv;
+        const uint32_t per_row = a.q_heads + a.kv_heads, p = blockIdx.x * (kQkvThreads / 64) + wv;
         if (p >= a.rows * per_row) return;
         const uint32_t r = p / per_row, h = p % per_row;
         const bool is_q = h < a.q_heads;
@@ -182,16 +189,16 @@ prefill_qkv_kernel(QkvRun a) {
         const float4 rot = reinterpret_cast<const float4*>(a.rope_table)[size_t(r) * (HD / 4) + lane];   // cos, sin of two pairs
         const float2 g0 = make_float2(gamma[2 * lane], gamma[2 * lane + 1]), g1 = make_float2(gamma[HD / 2 + 2 * lane], gamma[HD / 2 + 2 * lane + 1]);
         float v[4];
-        for (uint32_t s0 = 0; s0 < a.planes; s0 += 4) {
-            float2 x[4], y[4];
+        for (uint32_t s0 = 0; s0 < a.planes; s0 += 8) {
+            float2 x[8], y[8];
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+            for (int s = 0; s < 8; ++s)
                 if (s0 + s < a.planes) {
                     x[s] = *reinterpret_cast<const float2*>(src + (s0 + s) * stride + 2 * lane);
                     y[s] = *reinterpret_cast<const float2*>(src + (s0 + s) * stride + HD / 2 + 2 * lane);
                 }
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+            for (int s = 0; s < 8; ++s)
                 if (s0 + s < a.planes) {
                     if (s0 + s == 0) { v[0] = x[s].x; v[1] = x[s].y; v[2] = y[s].x; v[3] = y[s].y; }
                     else { v[0] += x[s].x; v[1] += x[s].y; v[2] += y[s].x; v[3] += y[s].y; }
@@ -217,13 +224,14 @@ prefill_qkv_kernel(QkvRun a) {
     } else {
         const uint32_t w = blockIdx.x - a.head_groups, kvh = w % a.kv_heads, v0 = (w / a.kv_heads) * 32;
         const size_t width = size_t(a.kv_heads) * HD, stride = size_t(a.rows) * width;
-        for (uint32_t c = threadIdx.x; c < 32 * (HD / 8); c += 256) {
-            const uint32_t token = c / (HD / 8), d8 = c % (HD / 8), kp = a.base32 + v0 + token;
+        static_assert(kQkvThreads == 32 * (HD / 8), "a thread: eight elements of a token");
+        {
+            const uint32_t token = threadIdx.x / (HD / 8), d8 = threadIdx.x % (HD / 8), kp = a.base32 + v0 + token;
             uint4 val = make_uint4(0, 0, 0, 0);   // outside the visible range
             if (kp >= a.position && kp < a.position + a.rows) {
                 const size_t off = size_t(kp - a.position) * width + kvh * HD + 8 * d8;
                 float f[8];
-                sum_planes8<4>(a.v_planes + off, a.planes, stride, f);
+                sum_planes8<8>(a.v_planes + off, a.planes, stride, f);
                 uint32_t o[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -240,13 +248,11 @@ prefill_qkv_kernel(QkvRun a) {
             *reinterpret_cast<uint4*>(&tile[token][8 * d8]) = val;
         }
         __syncthreads();
-        const uint32_t dim = threadIdx.x;
-        uint32_t o[16];
+        const uint32_t dim = threadIdx.x >> 2, t0 = 8 * (threadIdx.x & 3);   // four threads: a dimension's 32 tokens
+        uint32_t o[4];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) o[t] = uint32_t(tile[2 * t][dim]) | (uint32_t(tile[2 * t + 1][dim]) << 16);
-        uint4* dst = reinterpret_cast<uint4*>(a.vt + (size_t(kvh) * HD + dim) * a.T + v0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dst[i] = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
+        for (int t = 0; t < 4; ++t) o[t] = uint32_t(tile[t0 + 2 * t][dim]) | (uint32_t(tile[t0 + 2 * t + 1][dim]) << 16);
+        *reinterpret_cast<uint4*>(a.vt + (size_t(kvh) * HD + dim) * a.T + v0 + t0) = make_uint4(o[0], o[1], o[2], o[3]);
     }
     if (bad && a.status) atomicOr(a.status, GUFFIN_STATUS_KV_NONFINITE);
 }
@@ -265,8 +271,13 @@ int prefill_joint(hipStream_t s, const float* x, uint32_t planes, const float* g
                   uint32_t* status) {
     const uint32_t threads = row_threads(width);
     const uint64_t copies = run.run_k ? uint64_t(rows - run.first_row) * run.row_vec : 0;
-    launch(prefill_joint_kernel, dim3(rows + static_cast<uint32_t>((copies + threads - 1) / threads)), dim3(threads), 0, s, x, planes,
-           size_t(rows) * width, gamma_post, residual, out_residual, gamma_next, out_norm, image, rows, width, eps, run, status);
+    const dim3 grid(rows + static_cast<uint32_t>((copies + threads - 1) / threads));
+    if (planes > 8 && threads <= 512)
+        launch(prefill_joint_kernel<16, 512>, grid, dim3(threads), 0, s, x, planes, size_t(rows) * width, gamma_post, residual, out_residual,
+               gamma_next, out_norm, image, rows, width, eps, run, status);
+    else
+        launch(prefill_joint_kernel<8, 1024>, grid, dim3(threads), 0, s, x, planes, size_t(rows) * width, gamma_post, residual, out_residual,
+               gamma_next, out_norm, image, rows, width, eps, run, status);
     return check_launch("prefill_joint");
 }
 
@@ -276,8 +287,8 @@ int prefill_geglu(hipStream_t s, const float* gate, const float* up, uint32_t pl
 }
 
 int prefill_qkv(hipStream_t s, QkvRun a) {
-    a.head_groups = (a.rows * (a.q_heads + a.kv_heads) + 3) / 4;
-    launch(prefill_qkv_kernel, dim3(a.head_groups + (a.T / 32) * a.kv_heads), dim3(256), 0, s, a);
+    a.head_groups = (a.rows * (a.q_heads + a.kv_heads) + kQkvThreads / 64 - 1) / (kQkvThreads / 64);
+    launch(prefill_qkv_kernel, dim3(a.head_groups + (a.T / 32) * a.kv_heads), dim3(kQkvThreads), 0, s, a);
     return check_launch("prefill_qkv");
 }
 
