@@ -167,6 +167,13 @@ __device__ __forceinline__ void weave() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// the lane's number, worked out where it stands
+__device__ __forceinline__ uint32_t lane_again() {
+    uint32_t none = 0;
+    asm volatile("" : "+s"(none));
+    return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none));
+}
+
 // ---- Q4_K ------------------------------------------------------------------------------------------------
 // The B operands of group G (0..7) of a block for column groups 2P, 2P + 1, from its half block's quants and scale words.
 template <int G, int P>
@@ -200,7 +207,7 @@ __device__ __forceinline__ void products(const half8_t (&a)[R], const half8_t (&
 // pipe and the vector pipe busy together.  A chunk's last lo half is in registers when its last region starts: there the
 // workgroup meets, the next chunk has arrived and the one after the next but one is asked for in place of the old.
 template <int R>
-__device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& feed, uint8_t* stage, const uint8_t* tile_base,
+__device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint8_t* stage, const uint8_t* tile_base,
                                         uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q4_K);
     constexpr int V = (30 + 4 * R - 1) / (4 * R);   // vector instructions behind each matrix instruction
@@ -209,7 +216,8 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& fee
     constexpr bool WOVEN = R < 4;
     constexpr int VA = (30 + 32 * (R - 1) + 4 * R - 1) / (4 * R), VB = (62 + 4 * R - 1) / (4 * R);
     using S = Stage<R>;
-    const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
+    const uint32_t wv = feed.wv;
+    uint32_t lane = lane_again(), j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
     const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
     uint8_t* const heads = stage + S::kHead + wv * 1280;
     uint4 q[2][4];
@@ -248,6 +256,7 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, const Feed<R>& fee
     q4_operands<0, 1>(q[0], sc, b);
     uint32_t rd = 0;   // the buffer of the chunk in work
     for (uint32_t blk = b0; blk < b1; ++blk) {
+        if constexpr (!WOVEN) { lane = lane_again(); j = lane & 15; lg = lane >> 4; lane16 = feed.lane16 = lane * 16; }   // no register to keep addresses in
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
         float dh[4];   // the first half's sums leave their chain for acc (no bias term yet)
         auto fold_scales = [&] {
@@ -510,7 +519,7 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, const Feed<R>
                                              uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q6_K);
     using S = Stage<R>;
-    const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
+    const uint32_t lane = lane_again(), wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
     const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
     const uint32_t sel = lane >= 32 ? 0x04010401u : 0x04000400u;
     uint8_t* const heads = stage + S::kHead + wv * 1280;
@@ -601,7 +610,7 @@ __global__ void __launch_bounds__(256, 2)
 prefill_gemm_kernel(GemmArgs A) {
     __shared__ __attribute__((aligned(16))) uint8_t stage[Stage<R>::kBytes];
     const ImageLayout L = image_layout(A.M, A.K);
-    const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t s = 0;
     while (s + 1 < A.segments && blockIdx.y >= A.seg[s + 1].first_group) ++s;
     const GemmSegment seg = A.seg[s];
@@ -611,7 +620,7 @@ prefill_gemm_kernel(GemmArgs A) {
     Feed<R> feed;
     feed.img = make_resource(A.blob, static_cast<uint32_t>(L.bytes));
     feed.stage = stage;
-    feed.lane16 = lane * 16;
+    feed.lane16 = lane_again() * 16;
     feed.group_stride = (L.mpad / 16) * 2048;
     feed.base = rt0 * 2048 + (wv & 1) * (1024 * R);
     feed.wv = wv;
@@ -633,7 +642,7 @@ prefill_gemm_kernel(GemmArgs A) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!valid) return;
     float* y = seg.y + blockIdx.z * seg.plane_stride;
-    const uint32_t col = tile_index * kCols + (lane & 15), row0 = rt0 * 16 + 4 * (lane >> 4);
+    const uint32_t at = lane_again(), col = tile_index * kCols + (at & 15), row0 = rt0 * 16 + 4 * (at >> 4);
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
