@@ -30,7 +30,7 @@ __device__ __forceinline__ uint64_t make_key(float logit, uint32_t token) {
     const uint32_t ordered = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
     return (uint64_t(ordered) << 32) | (0xFFFFFFFFu - token);
 }
-[[maybe_unused]] __device__ __forceinline__ float key_logit(uint64_t key) {
+__device__ __forceinline__ float key_logit(uint64_t key) {
     const uint32_t o = static_cast<uint32_t>(key >> 32);
     return __uint_as_float((o & 0x80000000u) ? (o & 0x7FFFFFFFu) : ~o);
 }
@@ -89,7 +89,7 @@ __device__ __forceinline__ void hist_add(uint32_t* hist, bool valid, uint32_t bi
     uint64_t todo = __ballot(valid);
     for (int it = 0; it < 8 && todo; ++it) {
         const int leader = __ffsll(static_cast<long long>(todo)) - 1;
-        const uint32_t b0 = __shfl(bin, leader, kWave);
+        const uint32_t b0 = __builtin_amdgcn_readlane(bin, leader);
         const uint64_t same = __ballot(valid && bin == b0) & todo;
         if (lane == uint32_t(leader)) atomicAdd(&hist[b0], static_cast<uint32_t>(__popcll(same)));
         todo &= ~same;
@@ -98,19 +98,24 @@ __device__ __forceinline__ void hist_add(uint32_t* hist, bool valid, uint32_t bi
 }
 
 // Writes one row of the result from its `retain` selected keys (candidate order) and appends the logits of
-// the row's history tokens; all threads of the workgroup call it after the keys are complete.
+// the row's history tokens; all threads of the workgroup call it after the keys are complete.  raised: the row's status word;
+// whole: the record is new memory, what it does not use becomes zero.
 __device__ void emit_candidates(const uint64_t* keys, uint32_t retain, uint32_t row, const float* __restrict__ logits,
                                 uint32_t vocab, float divisor, const uint32_t* __restrict__ history,
-                                const uint32_t* __restrict__ history_count, uint32_t row_stride, uint32_t history_stride,
+                                uint32_t hc, uint32_t history_stride, uint32_t raised, bool whole,
                                 Candidates* __restrict__ result, uint32_t* __restrict__ status) {
     __syncthreads();
     Candidates& out = result[row];
-    const uint32_t hc = history_count ? history_count[size_t(row) * row_stride] : 0;
     for (uint32_t i = threadIdx.x; i < retain; i += blockDim.x) {
         const uint32_t token = key_token(keys[i]);
+        // the key holds the value's bits but for a zero's sign and what adding zero does to a NaN: those are read again
+        float v = key_logit(keys[i]);
+        if (!(v < 0.f || v > 0.f)) v = logits[size_t(row) * vocab + token] / divisor;
         out.values[i].token = token;
-        out.values[i].logit = logits[size_t(row) * vocab + token] / divisor;  // the native value, not the key's
+        out.values[i].logit = v;
     }
+    if (whole)
+        for (uint32_t i = retain + hc + threadIdx.x; i < 384; i += blockDim.x) { out.values[i].token = 0; out.values[i].logit = 0.f; }
     uint32_t st = 0;
     for (uint32_t i = threadIdx.x; i < hc; i += blockDim.x) {
         const uint32_t token = history[size_t(row) * history_stride + i];
@@ -126,10 +131,13 @@ __device__ void emit_candidates(const uint64_t* keys, uint32_t retain, uint32_t 
         }
     }
     if (st && status) atomicOr(status + row, st);
-    __syncthreads();
+    if (hc && status) {
+        raised |= __syncthreads_or(st & GUFFIN_STATUS_BAD_TOKEN) ? GUFFIN_STATUS_BAD_TOKEN : 0u;
+        raised |= __syncthreads_or(st & GUFFIN_STATUS_NONFINITE) ? GUFFIN_STATUS_NONFINITE : 0u;
+    }
     if (threadIdx.x == 0) {
         out.count = retain + hc;
-        out.status = status ? status[row] : 0;
+        out.status = raised;
     }
 }
 
@@ -142,7 +150,7 @@ __global__ void __launch_bounds__(1024)
 topk_merge_kernel(const float* __restrict__ logits, const uint64_t* __restrict__ survivors, uint32_t n_survivors,
                   uint32_t tile_keep, uint32_t vocab, uint32_t retain_cap, float divisor, const uint32_t* __restrict__ history,
                   const uint32_t* __restrict__ history_count, const uint32_t* __restrict__ row_retain, uint32_t row_stride,
-                  uint32_t history_stride, Candidates* __restrict__ result, uint32_t* __restrict__ status) {
+                  uint32_t history_stride, bool whole, Candidates* __restrict__ result, uint32_t* __restrict__ status) {
     __shared__ uint32_t hist[256];
     __shared__ uint64_t sel[512];
     __shared__ uint64_t keys[512];  // selected keys in candidate order
@@ -156,6 +164,7 @@ topk_merge_kernel(const float* __restrict__ logits, const uint64_t* __restrict__
         const uint32_t want = row_retain[size_t(row) * row_stride];
         retain = want < 1 ? 1 : (want < retain_cap ? want : retain_cap);
     }
+    const uint32_t hc = history_count ? history_count[size_t(row) * row_stride] : 0, raised = status ? status[row] : 0;
     const uint64_t* src = survivors + size_t(row) * n_survivors;
     // up to kMine keys per thread stay in registers (8 for the verify pass's lists, 34 for the 257 per
     // tile that the proposal law asks for); longer survivor lists are re-read from memory in every pass
@@ -282,7 +291,7 @@ topk_merge_kernel(const float* __restrict__ logits, const uint64_t* __restrict__
             keys[rank] = k;
         }
     }
-    emit_candidates(keys, retain, row, logits, vocab, divisor, history, history_count, row_stride, history_stride, result, status);
+    emit_candidates(keys, retain, row, logits, vocab, divisor, history, hc, history_stride, raised, whole, result, status);
 }
 
 // ---- selection by threshold ------------------------------------------------------------------
@@ -291,15 +300,27 @@ topk_merge_kernel(const float* __restrict__ logits, const uint64_t* __restrict__
 // maximum is at or below the retain-th largest logit of the row, so only logits at or above it can be
 // selected, and on anything but massively tied rows they are few more than `retain`.  Two launches:
 //   segment_max_kernel       the ordered score bits of every segment's maximum; clears the row's counters
-//   threshold_select_kernel  every workgroup finds the bound for itself (a 4-pass radix select over at most
-//                            1024 words), collects the keys of its 4096 logits that reach it into the row's
-//                            list, and the workgroup that finishes last sorts the list and writes the row
-// The list and the counters move with device-scope accesses (the workgroups sit on different L2s), every
+//   threshold_select_kernel  (`sure` != 0: the best `sure` logits and every tie with the last of them are all the caller
+//                            needs, and as many of the following, up to `retain`, as come with the bound for those.)  Every workgroup finds the bound for itself (a radix select over at most 1024
+//                            words that stops as soon as few maxima lie between it and the exact one),
+//                            collects the keys of its 4096 logits that reach it, and the workgroup that
+//                            finishes last sorts all of them and writes the row
+// What bounds the second is the chain of trips to memory behind one another (the workgroups sit on different
+// L2s, so what they exchange moves with device-scope accesses).  A workgroup therefore has places of its own
+// for kSlots keys and its count, stored without asking anybody; only what does not fit goes through a
+// reservation in the row's common list, and the last workgroup asks for counts and places at once.  Its
+// logits lie 64 apart from its neighbours', so that a run of equal or large ones is dealt to all.  Every
 // workgroup waits for its own stores before it counts itself done, and nobody waits for anybody: the last
-// arrival is whoever draws the last ticket.  A row whose list overflows (more than kCollectCap logits tie
-// into the bound) is selected exactly, and slowly, by a radix select over the whole row in that workgroup.
+// arrival is whoever draws the last ticket.  A row whose common list overflows, or with more than kCollectCap
+// keys, is selected exactly, and slowly, by a radix select over the whole row in that workgroup.
+// 262144 logits: 64 of two rows 9.5 us (10.6 with an exact bound and every key through one reservation), what a compact law
+// of 64 needs of one row 9.5 (15.4 with its best 257 in order).
 constexpr uint32_t kSeg = 256, kMaxSegs = 1024, kCollectTile = 4096, kCollectCap = 2048;
-constexpr uint32_t kThresholdRowWords = kMaxSegs + 4 + 2 * kCollectCap;   // segment maxima, counter, done, pad, list
+constexpr uint32_t kMaxCollectors = kMaxSegs * kSeg / kCollectTile, kSlots = 16;
+// segment maxima; common list's length, workgroups done, pad; the workgroups' counts, their places, the common list
+constexpr uint32_t kThresholdRowWords = kMaxSegs + 4 + 2 * kCollectCap;
+constexpr uint32_t kCommonCap = kCollectCap - kMaxCollectors / 2 - kMaxCollectors * kSlots;
+static_assert(kMaxCollectors == 64, "a wave scans the workgroups' counts");
 
 __device__ __forceinline__ uint32_t ordered_bits(float v) {
     const uint32_t b = __float_as_uint(v + 0.0f);
@@ -307,11 +328,13 @@ __device__ __forceinline__ uint32_t ordered_bits(float v) {
 }
 
 __global__ void __launch_bounds__(256)
-segment_max_kernel(const float* __restrict__ logits, uint32_t vocab, uint32_t segs, float divisor, uint32_t* __restrict__ ws) {
+segment_max_kernel(const float* __restrict__ logits, uint32_t vocab, uint32_t segs, float divisor, uint32_t* __restrict__ ws,
+                   uint32_t* __restrict__ new_status) {
     const uint32_t row = blockIdx.y, lane = threadIdx.x & 63;
     const uint32_t seg = blockIdx.x * 4 + (threadIdx.x >> 6);
     uint32_t* row_ws = ws + size_t(row) * kThresholdRowWords;
     if (blockIdx.x == 0 && threadIdx.x < 4) row_ws[kMaxSegs + threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 4 && new_status) new_status[row] = 0;
     if (seg >= segs) return;
     const float* lr = logits + size_t(row) * vocab;
     uint32_t best = 0;
@@ -329,7 +352,7 @@ segment_max_kernel(const float* __restrict__ logits, uint32_t vocab, uint32_t se
 
 // the bin (highest first) that holds the `remaining`-th largest entry of a 256-bin histogram; first wave only
 __device__ __forceinline__ void find_bin(const uint32_t* hist, uint32_t remaining, uint32_t lane, uint32_t& s_bin,
-                                         uint32_t& s_above) {
+                                         uint32_t& s_above, uint32_t& s_in) {
     uint32_t c[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) c[j] = hist[255 - 4 * lane - j];
@@ -339,62 +362,69 @@ __device__ __forceinline__ void find_bin(const uint32_t* hist, uint32_t remainin
     if (above < remaining && remaining <= incl) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            if (remaining <= above + c[j]) { s_bin = 255 - 4 * lane - j; s_above = above; break; }
+            if (remaining <= above + c[j]) { s_bin = 255 - 4 * lane - j; s_above = above; s_in = c[j]; break; }
             above += c[j];
         }
     }
 }
 
+template <typename T>
+__device__ __forceinline__ T shared_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T>
+__device__ __forceinline__ void shared_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 __global__ void __launch_bounds__(1024)
-threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32_t segs, uint32_t retain_cap, float divisor,
-                        const uint32_t* __restrict__ history, const uint32_t* __restrict__ history_count,
+threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32_t segs, uint32_t retain_cap, uint32_t sure,
+                        float divisor, const uint32_t* __restrict__ history, const uint32_t* __restrict__ history_count,
                         const uint32_t* __restrict__ row_retain, uint32_t row_stride, uint32_t history_stride,
                         uint32_t* __restrict__ ws, Candidates* __restrict__ result, uint32_t* __restrict__ status,
-                        bool suppressed_ok) {
+                        bool suppressed_ok, bool whole) {
     __shared__ uint32_t hist[256];
     __shared__ uint64_t sel[kCollectCap];
     __shared__ uint64_t keys[512];
-    __shared__ uint32_t s_bin, s_above, s_last, s_count;
+    __shared__ uint32_t s_bin, s_above, s_in, s_last, s_count;
     const uint32_t row = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    uint32_t* row_ws = ws + size_t(row) * kThresholdRowWords;
+    uint32_t* counter = row_ws + kMaxSegs;
+    uint32_t* done = counter + 1;
+    uint32_t* counts = counter + 4;
+    uint64_t* places = reinterpret_cast<uint64_t*>(counts + kMaxCollectors);
+    uint64_t* common = places + kMaxCollectors * kSlots;
+    const float* lr = logits + size_t(row) * vocab;
+    // this workgroup's logits are requested before the bound is worked out
+    auto token_of = [&](uint32_t u) { return ((u * (blockDim.x / 64) + (tid >> 6)) * gridDim.x + blockIdx.x) * 64 + lane; };
+    float mine[kCollectTile / 1024];
+#pragma unroll
+    for (uint32_t u = 0; u < kCollectTile / 1024; ++u) mine[u] = token_of(u) < vocab ? lr[token_of(u)] : 0.f;
+    const uint32_t word = tid < segs ? row_ws[tid] : 0u;
     uint32_t retain = retain_cap;
     if (row_retain) {
         const uint32_t want = row_retain[size_t(row) * row_stride];
         retain = want < 1 ? 1 : (want < retain_cap ? want : retain_cap);
     }
-    uint32_t* row_ws = ws + size_t(row) * kThresholdRowWords;
-    uint32_t* counter = row_ws + kMaxSegs;
-    uint32_t* done = counter + 1;
-    uint64_t* list = reinterpret_cast<uint64_t*>(row_ws + kMaxSegs + 4);
-    const float* lr = logits + size_t(row) * vocab;
-    // this workgroup's logits are requested before the bound is worked out
-    float mine[kCollectTile / 1024];
-#pragma unroll
-    for (uint32_t u = 0; u < kCollectTile / 1024; ++u) {
-        const uint32_t t = blockIdx.x * kCollectTile + u * 1024 + tid;
-        mine[u] = t < vocab ? lr[t] : 0.f;
-    }
-    // ---- the bound: the retain-th largest segment maximum (segs >= retain by the launch's condition) ----
-    const uint32_t word = tid < segs ? row_ws[tid] : 0u;
-    uint32_t prefix = 0, remaining = retain;
-    for (int pass = 0; pass < 4; ++pass) {
-        const int shift = 24 - 8 * pass;
+    const uint32_t hc = history_count ? history_count[size_t(row) * row_stride] : 0;
+    // ---- the bound: at or below the largest segment maximum but `least` - 1 (there are as many by the launch's condition), with
+    // no more than an eighth of `least` maxima too many above it; every further byte would cost a pass, most rows stop after two
+    const uint32_t least = sure ? sure : retain;
+    uint32_t prefix = 0, remaining = least, shift = 24;
+    for (;; shift -= 8) {
         if (tid < 256) hist[tid] = 0;
         __syncthreads();
-        hist_add(hist, tid < segs && (pass == 0 || (word >> (shift + 8)) == prefix), (word >> shift) & 255u, lane);
+        hist_add(hist, tid < segs && (shift == 24 || (word >> (shift + 8)) == prefix), (word >> shift) & 255u, lane);
         __syncthreads();
-        if (tid < 64) find_bin(hist, remaining, lane, s_bin, s_above);
+        if (tid < 64) find_bin(hist, remaining, lane, s_bin, s_above, s_in);
+        if (tid == 0) s_count = 0;
         __syncthreads();
         prefix = (prefix << 8) | s_bin;
         remaining -= s_above;
+        if (shift == 0 || s_in - remaining <= least / 8) break;
     }
-    const uint32_t bound = prefix;
-    // ---- collect: this workgroup's keys into LDS, then one reservation in the row's list for all of them ----
-    if (tid == 0) s_count = 0;
-    __syncthreads();
+    const uint32_t bound = prefix << shift;
+    // ---- collect: this workgroup's keys into LDS, then into its places and, past them, the row's common list ----
     bool bad = false;
 #pragma unroll
     for (uint32_t u = 0; u < kCollectTile / 1024; ++u) {
-        const uint32_t t = blockIdx.x * kCollectTile + u * 1024 + tid;
+        const uint32_t t = token_of(u);
         bool hit = false;
         uint64_t key = 0;
         if (t < vocab) {
@@ -409,12 +439,16 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
         }
     }
     __syncthreads();
-    const uint32_t found = s_count;   // above kCollectCap: the row's counter shows it too, and nobody reads the list
-    if (tid == 0 && found) s_bin = __hip_atomic_fetch_add(counter, found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (found)
-        for (uint32_t i = tid; i < min(found, kCollectCap); i += blockDim.x)
-            if (s_bin + i < kCollectCap) __hip_atomic_store(list + s_bin + i, sel[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t found = s_count;
+    if (tid < kSlots && tid < found) shared_store(places + blockIdx.x * kSlots + tid, sel[tid]);
+    if (tid == kSlots) shared_store(counts + blockIdx.x, found);
+    if (found > kSlots) {
+        const uint32_t more = found - kSlots;   // beyond the list: the row's counter shows it too, and nobody reads the list
+        if (tid == 0) s_bin = __hip_atomic_fetch_add(counter, more, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        for (uint32_t i = tid; i < min(more, kCommonCap); i += blockDim.x)
+            if (s_bin + i < kCommonCap) shared_store(common + s_bin + i, sel[kSlots + i]);
+    }
     if (bad && status) atomicOr(status + row, GUFFIN_STATUS_NONFINITE);
     // ---- the last workgroup of the row to get here finishes it -----------------------------------------
     __builtin_amdgcn_s_waitcnt(0);
@@ -426,19 +460,31 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
     }
     __syncthreads();
     if (!s_last) return;
-    const uint32_t n = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (n <= kCollectCap) {
-        for (uint32_t i = tid; i < n; i += blockDim.x) sel[i] = __hip_atomic_load(list + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // every wave scans the counts for itself; a thread takes one place
+    const uint32_t count = lane < gridDim.x ? shared_load(counts + lane) : 0;
+    const uint32_t owner = tid / kSlots, raised = status ? shared_load(status + row) : 0;
+    const uint64_t place = owner < gridDim.x ? shared_load(places + tid) : 0;   // its collector may have left it as it was
+    const uint32_t kept = min(count, kSlots), upto = wave_inclusive_scan(kept), all = wave_inclusive_scan(count);
+    const uint32_t n = __builtin_amdgcn_readlane(all, 63), placed = __builtin_amdgcn_readlane(upto, 63);
+    const uint32_t own_kept = __shfl(kept, owner, kWave), own_upto = __shfl(upto, owner, kWave);
+    static_assert(kMaxCollectors * kSlots == 1024, "a place per thread");
+    if (n <= kCollectCap && n - placed <= kCommonCap) {
+        if (tid % kSlots < own_kept) sel[own_upto - own_kept + tid % kSlots] = place;
+        for (uint32_t i = tid; i < n - placed; i += blockDim.x) sel[placed + i] = shared_load(common + i);
         if (n <= 512) {
             __syncthreads();
             // the workgroup's 1024 threads over n keys: 2, 4, 8 or 16 neighbouring lanes count for one of them
-            const uint32_t shift = n <= 64 ? 4 : n <= 128 ? 3 : n <= 256 ? 2 : 1, i = tid >> shift, part = tid & ((1u << shift) - 1);
+            const uint32_t part_bits = n <= 64 ? 4 : n <= 128 ? 3 : n <= 256 ? 2 : 1, i = tid >> part_bits, part = tid & ((1u << part_bits) - 1);
             const uint64_t k = i < n ? sel[i] : 0;
             uint32_t rank = 0;
 #pragma unroll 8
-            for (uint32_t j = part; j < n; j += 1u << shift) rank += sel[j] > k;
-            for (uint32_t o = 1; o < (1u << shift); o <<= 1) rank += __shfl_xor(rank, o, kWave);
+            for (uint32_t j = part; j < n; j += 1u << part_bits) rank += sel[j] > k;
+            rank += lane_cross_u32<0xB1, 0xF>(rank);                        // the neighbour,
+            if (part_bits >= 2) rank += lane_cross_u32<0x4E, 0xF>(rank);    // the pair, the four, the eight beside
+            if (part_bits >= 3) rank += lane_cross_u32<0x141, 0xF>(rank);
+            if (part_bits >= 4) rank += lane_cross_u32<0x140, 0xF>(rank);
             if (i < n && part == 0 && rank < retain) keys[rank] = k;
+            retain = min(retain, n);   // fewer only where the call is sure of fewer
         } else {
             for (uint32_t i = n + tid; i < kCollectCap; i += blockDim.x) sel[i] = 0;
             bitonic_desc(sel, kCollectCap);
@@ -449,16 +495,16 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
         uint64_t kprefix = 0;
         uint32_t left = retain;
         for (int pass = 0; pass < 8; ++pass) {
-            const int shift = 56 - 8 * pass;
+            const int down = 56 - 8 * pass;
             if (tid < 256) hist[tid] = 0;
             __syncthreads();
             for (uint32_t i0 = 0; i0 < vocab; i0 += blockDim.x) {   // whole waves stay converged
                 const uint32_t i = i0 + tid;
                 const uint64_t k = i < vocab ? make_key(lr[i] / divisor, i) : 0;
-                hist_add(hist, i < vocab && (pass == 0 || (k >> (shift + 8)) == kprefix), static_cast<uint32_t>(k >> shift) & 255u, lane);
+                hist_add(hist, i < vocab && (pass == 0 || (k >> (down + 8)) == kprefix), static_cast<uint32_t>(k >> down) & 255u, lane);
             }
             __syncthreads();
-            if (tid < 64) find_bin(hist, left, lane, s_bin, s_above);
+            if (tid < 64) find_bin(hist, left, lane, s_bin, s_above, s_in);
             __syncthreads();
             kprefix = (kprefix << 8) | s_bin;
             left -= s_above;
@@ -476,7 +522,12 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
             keys[rank] = k;
         }
     }
-    emit_candidates(keys, retain, row, logits, vocab, divisor, history, history_count, row_stride, history_stride, result, status);
+    emit_candidates(keys, retain, row, logits, vocab, divisor, history, hc, history_stride, raised, whole, result, status);
+}
+
+__global__ void clear_words_kernel(uint32_t* words, uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) words[i] = 0;
 }
 
 // ---- verify-row input validation --------------------------------------------------------------
@@ -581,7 +632,15 @@ namespace guffin {
 int select_candidates_scaled(hipStream_t s, const float* logits, uint32_t rows, uint32_t vocab, uint32_t retain,
                              float divisor, const uint32_t* history, const uint32_t* history_count,
                              void* workspace, void* result, uint32_t* status, bool suppressed_ok = false,
-                             const uint32_t* row_retain = nullptr, uint32_t row_stride = 1);
+                             const uint32_t* row_retain = nullptr, uint32_t row_stride = 1, uint32_t sure = 0, bool fresh = false);
+}
+
+extern "C" int guffin_hip_select_candidates_fresh(void* stream, const float* logits, uint32_t rows, uint32_t vocab,
+                                                  uint32_t retain, const uint32_t* history, const uint32_t* history_count,
+                                                  void* workspace, void* result, uint32_t* status) {
+    if (!status) return fail(GUFFIN_E_ARG, "select_candidates_fresh: null pointer");
+    return select_candidates_scaled(as_stream(stream), logits, rows, vocab, retain, 1.0f, history, history_count,
+                                    workspace, result, status, false, nullptr, 1, 0, true);
 }
 
 extern "C" int guffin_hip_select_candidates(void* stream, const float* logits, uint32_t rows, uint32_t vocab,
@@ -594,7 +653,7 @@ extern "C" int guffin_hip_select_candidates(void* stream, const float* logits, u
 int guffin::select_candidates_scaled(hipStream_t s, const float* logits, uint32_t rows, uint32_t vocab,
                                      uint32_t retain, float divisor, const uint32_t* history,
                                      const uint32_t* history_count, void* workspace, void* result, uint32_t* status,
-                                     bool suppressed_ok, const uint32_t* row_retain, uint32_t row_stride) {
+                                     bool suppressed_ok, const uint32_t* row_retain, uint32_t row_stride, uint32_t sure, bool fresh) {
     if (!logits || !workspace || !result) return fail(GUFFIN_E_ARG, "select_candidates: null pointer");
     if (rows == 0 || vocab == 0) return fail(GUFFIN_E_SHAPE, "select_candidates: empty shape");
     if (retain == 0 || retain > 320) return fail(GUFFIN_E_CAPACITY, "select_candidates: retain must be in [1, 320] (top_k <= 256 plus 64 history tokens)");
@@ -605,24 +664,26 @@ int guffin::select_candidates_scaled(hipStream_t s, const float* logits, uint32_
     const uint32_t segs = (vocab + kSeg - 1) / kSeg;
     if (segs <= kMaxSegs && segs >= 2 * keep) {   // large vocabulary: a bound from the segment maxima, then one pass
         uint32_t* words = static_cast<uint32_t*>(workspace);
-        launch(segment_max_kernel, dim3((segs + 3) / 4, rows), dim3(256), 0, s, logits, vocab, segs, divisor, words);
+        launch(segment_max_kernel, dim3((segs + 3) / 4, rows), dim3(256), 0, s, logits, vocab, segs, divisor, words,
+               fresh ? status : nullptr);
         if (int rc = check_launch("select_candidates(segment maxima)")) return rc;
         launch(threshold_select_kernel, dim3((vocab + kCollectTile - 1) / kCollectTile, rows), dim3(1024), 0, s,
-                           logits, vocab, segs, keep, divisor, history, history_count, row_retain, row_stride,
-                           row_stride == 1 ? 64u : row_stride, words, static_cast<Candidates*>(result), status, suppressed_ok);
+                           logits, vocab, segs, keep, sure, divisor, history, history_count, row_retain, row_stride,
+                           row_stride == 1 ? 64u : row_stride, words, static_cast<Candidates*>(result), status, suppressed_ok, fresh);
         return check_launch("select_candidates(threshold)");
     }
+    if (fresh) launch(clear_words_kernel, dim3((rows + 63) / 64), dim3(64), 0, s, status, rows);
     uint64_t* surv = static_cast<uint64_t*>(workspace);
     launch(topk_tile_kernel, dim3(tiles, rows), dim3(1024), 0, s, logits, surv, vocab, keep, divisor, status, suppressed_ok);
     if (int rc = check_launch("select_candidates(tile)")) return rc;
     if (tiles * keep <= 8 * 1024)
         launch(topk_merge_kernel<8>, dim3(rows), dim3(1024), 0, s, logits, surv, tiles * keep, keep, vocab,
                            keep, divisor, history, history_count, row_retain, row_stride, row_stride == 1 ? 64u : row_stride,
-                           static_cast<Candidates*>(result), status);
+                           fresh, static_cast<Candidates*>(result), status);
     else
         launch(topk_merge_kernel<34>, dim3(rows), dim3(1024), 0, s, logits, surv, tiles * keep, keep, vocab,
                            keep, divisor, history, history_count, row_retain, row_stride, row_stride == 1 ? 64u : row_stride,
-                           static_cast<Candidates*>(result), status);
+                           fresh, static_cast<Candidates*>(result), status);
     return check_launch("select_candidates(merge)");
 }
 

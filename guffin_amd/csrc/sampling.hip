@@ -142,22 +142,6 @@ __device__ __forceinline__ void rank_sort_ascending(uint64_t* keys, uint32_t n) 
     if (t < n) keys[rank] = mine;
     __syncthreads();
 }
-// Descending, keys distinct except for zeros (padding and dropped duplicates), which end up behind the others in
-// the first `span` places.
-__device__ __forceinline__ void rank_sort_descending(uint64_t* keys, uint32_t n, uint32_t span) {
-    __syncthreads();
-    const uint32_t t = threadIdx.x;
-    const uint64_t mine = t < n ? keys[t] : 0;
-    uint32_t rank = 0;
-    if (mine != 0)
-#pragma unroll 8
-        for (uint32_t j = 0; j < n; ++j) rank += keys[j] > mine;
-    __syncthreads();
-    if (t < span) keys[t] = 0;
-    __syncthreads();
-    if (mine != 0) keys[rank] = mine;
-    __syncthreads();
-}
 
 __device__ __forceinline__ uint64_t score_key(float score, uint32_t token) {
     const uint32_t b = __float_as_uint(score + 0.0f);
@@ -171,7 +155,8 @@ __device__ __forceinline__ uint64_t score_key(float score, uint32_t token) {
 __global__ void __launch_bounds__(256)
 draft_law_kernel(const Candidates* __restrict__ top, SamplerOptions opt, uint64_t seed, uint64_t step,
                  const StepDraws* __restrict__ injected, DraftLaw* __restrict__ law,
-                 uint32_t* __restrict__ proposal, uint32_t* __restrict__ status, uint32_t* __restrict__ full_error) {
+                 uint32_t* __restrict__ proposal, uint32_t* __restrict__ status, uint32_t* __restrict__ full_error, bool whole) {
+    // whole: the law is new memory, what it does not use becomes zero
     // full_error != nullptr: the full-vocabulary kernels follow, guarded by law->count; a support of
     // more than 256 ties then hands over to them instead of failing
     __shared__ uint64_t keys[256];
@@ -179,16 +164,19 @@ draft_law_kernel(const Candidates* __restrict__ top, SamplerOptions opt, uint64_
     __shared__ uint64_t edge[257];
     __shared__ uint32_t s_n, s_first, s_bad, s_chosen;
     const uint32_t t = threadIdx.x;
-    const uint32_t avail = top->count;
-    // every thread fetches its own entry once; the single-lane sections below work on LDS only
+    // the record (always whole in memory) comes in one trip: every thread fetches its own entry, counted or not, and the
+    // single-lane sections below work on LDS only
+    const uint32_t avail = top->count, raised = top->status;
+    const float found_logit = top->values[t].logit, more = top->values[256].logit;
+    const uint32_t found_token = top->values[t].token;
     const bool usable = options_valid(opt) && opt.temperature > 0.f && opt.top_k <= 64 && avail >= 1;
     const uint32_t k = usable ? (opt.top_k < avail ? opt.top_k : avail) : 1u;
-    const float cutoff = usable ? top->values[k - 1].logit : 0.f;
-    const float first_logit = usable ? top->values[0].logit : 0.f;
-    const float my_logit = t < avail ? top->values[t].logit : -INFINITY;
-    const uint32_t my_token = t < avail ? top->values[t].token : 0u;
+    const float my_logit = t < avail ? found_logit : -INFINITY;
+    const uint32_t my_token = t < avail ? found_token : 0u;
     if (t == 0) { s_first = 256u; s_bad = 0; s_chosen = 0xFFFFFFFFu; }
+    score[t] = my_logit;
     __syncthreads();
+    const float cutoff = usable ? score[k - 1] : 0.f, first_logit = usable ? score[0] : 0.f;
     // entries are sorted by (score desc, token asc): the support is a prefix, its length the first
     // entry that is below the cutoff or -inf
     if (!(t < avail && !(my_logit < cutoff) && my_logit != -INFINITY)) atomicMin(&s_first, t);
@@ -196,11 +184,10 @@ draft_law_kernel(const Candidates* __restrict__ top, SamplerOptions opt, uint64_
     if (t == 0) {
         uint32_t st = 0, n = 0;
         if (!usable) st = GUFFIN_STATUS_LAW_INVALID;
-        if (top->status & GUFFIN_STATUS_NONFINITE) st = GUFFIN_STATUS_LAW_INVALID | GUFFIN_STATUS_NONFINITE;
+        if (raised & GUFFIN_STATUS_NONFINITE) st = GUFFIN_STATUS_LAW_INVALID | GUFFIN_STATUS_NONFINITE;
         if (!st) {
             n = s_first;
             if (n == 256u && avail > 256u) {   // all 256 are in: a 257th eligible entry overflows the compact law
-                const float more = top->values[256].logit;
                 if (!(more < cutoff) && more != -INFINITY) n = 257u;
             }
             if (n == 0) st = GUFFIN_STATUS_LAW_INVALID;  // nothing eligible
@@ -213,7 +200,10 @@ draft_law_kernel(const Candidates* __restrict__ top, SamplerOptions opt, uint64_
     }
     __syncthreads();
     const uint32_t n = s_n;
-    if (n == 0) return;
+    if (n == 0) {
+        if (whole) { law->ids[t] = 0; law->cdf[t] = 0; if (t == 0) { law->pad = 0; law->cdf[256] = 0; } }
+        return;
+    }
     score[t] = t < n ? my_logit : -INFINITY;
     weight[t] = t < n ? law_exp(my_logit - first_logit) : 0.f;
     __syncthreads();
@@ -278,6 +268,9 @@ draft_law_kernel(const Candidates* __restrict__ top, SamplerOptions opt, uint64_
         if (uint64_t(d.word) >= last && uint64_t(d.word) < next) s_chosen = static_cast<uint32_t>(keys[t] >> 32);
         law->ids[t] = static_cast<uint32_t>(keys[t] >> 32);
         law->cdf[t + 1] = next;
+    } else if (whole) {
+        law->ids[t] = 0;
+        law->cdf[t + 1] = 0;
     }
     __syncthreads();
     if (t == 0) {
@@ -498,176 +491,63 @@ law_cdf_select_kernel(uint32_t vocab, bool greedy, uint64_t seed, uint64_t step,
 }
 
 // =========================================================================================
-// Target law (prepare_token_distribution) — whole workgroup, 512 threads
+// Target law (prepare_token_distribution) of the two candidate rows, and the accept / residual decision
 // =========================================================================================
+// One workgroup of two teams, a candidate row each: whether row 1 is wanted is known only at the end, and by then its law is
+// ready.  The kernel is a chain of short dependent steps, so what it costs is their number: everything is requested at once;
+// duplicates and places come out of one walk over the record; a sum whose order matters is one lane's, the compensated sum of
+// the same terms another wave's beside it and the masses of q a third's; running sums are kept, so that a draw is found by all
+// lanes at once; at temperatures of 1 and 0 the tempered weights are the raw ones and their sums are not taken twice.
+// An accepted proposal over 64 candidates takes 12.0 us (25.0 with a row after the other, and a step after the other inside).
+constexpr uint32_t kTeam = kMaxCandidates;   // threads of a row, a candidate each
+
 struct Prepared {
     uint32_t count;
     double total;
     uint32_t token[kMaxTopK];
-    double weight[kMaxTopK];
+    double weight[kMaxTopK];         // zeros behind the last entry
+    double run[kMaxTopK];            // running sums of the weights, in index order
 };
 
-struct Scratch {
-    uint64_t keys[512];
-    float logit[512];
-    double w[kMaxTopK];
-    double run[kMaxTopK];            // running sums of w, taken by one lane in index order
-    uint32_t tok[kMaxCandidates];    // the candidate record, staged once
+struct RowScratch {
+    uint64_t keys[kMaxCandidates], sorted[kMaxCandidates];
     float raw[kMaxCandidates];
+    double w[kMaxTopK];              // raw weights, zeros behind the last entry
+    double compensated[kMaxTopK];    // compensated running sums of the weights
     uint32_t hist[kHistoryCap];
     uint32_t kept, cut;              // ends of the top-p and min-p prefixes
-    uint32_t flag;
-    double value;
+    uint32_t dup, unique, flag, pick;
     int err;
 };
 
-// returns 0 or a negative error; result in `out` (shared); uses all threads.  Sums whose order matters are
-// taken by one lane over LDS; divisions, comparisons and exponentials are spread over the lanes.
-__device__ int prepare_distribution(const Candidates* cand, const SamplerOptions& opt, const uint32_t* history,
-                                    uint32_t history_count, Scratch& sc, Prepared& out) {
-    const uint32_t t = threadIdx.x, n = cand->count;
-    if (t == 0) sc.err = (!options_valid(opt) ? -1 : (n == 0 || n > kMaxCandidates) ? -2 : history_count > 64 ? -3 : 0);
-    __syncthreads();
-    if (sc.err) return sc.err;
-    const uint32_t request_top_k = opt.temperature == 0.f ? 1u : opt.top_k;
-    if (t < n) { sc.tok[t] = cand->values[t].token; sc.raw[t] = cand->values[t].logit; }
-    if (t < history_count) sc.hist[t] = history[t];
-    __syncthreads();
-    // dedup (a later duplicate must carry the same logit), repetition penalty, sort key
-    uint64_t key = 0;
-    if (t < n) {
-        const uint32_t token = sc.tok[t];
-        float logit = sc.raw[t];
-        bool dup = false;
-        if (!isfinite(logit)) atomicMin(&sc.err, -4);
-        // every lane walks the whole record without a branch, so that the reads run ahead (with a loop of its own length and
-        // an exit per lane this step alone took 3.6 us of the kernel)
-        bool differs = false;
-#pragma unroll 8
-        for (uint32_t j = 0; j < n; ++j) {
-            const bool same = (sc.tok[j] == token) & (j < t);
-            dup |= same;
-            differs |= same & (sc.raw[j] != logit);
-        }
-        if (differs) atomicMin(&sc.err, -5);
-        if (!dup) {
-            for (uint32_t h = 0; h < history_count; ++h)
-                if (sc.hist[h] == token) {
-                    logit = logit < 0.f ? __fmul_rn(logit, opt.repetition_penalty) : __fdiv_rn(logit, opt.repetition_penalty);
-                    break;
-                }
-            key = score_key(logit, token);
-        }
-    }
-    if (t < 512) sc.keys[t] = key;
-    __syncthreads();
-    if (sc.err) return sc.err;
-    uint32_t span = 64;   // the sort covers the record only (a real key is never 0, the padding is)
-    while (span < n) span <<= 1;
-    rank_sort_descending(sc.keys, n, span);
-    // unique count = number of non-zero keys (a real key is never 0: ordered(logit) has a set bit)
-    uint32_t mine = (t < span && sc.keys[t] != 0) ? 1u : 0u;
-    const uint32_t unique = __syncthreads_count(mine);
-    if (unique < request_top_k) return -6;
-    uint32_t count = unique < request_top_k ? unique : request_top_k;
-    // logits back from the sorted keys
-    if (t < count) {
-        const uint32_t o = static_cast<uint32_t>(sc.keys[t] >> 32);
-        sc.logit[t] = __uint_as_float((o & 0x80000000u) ? (o & 0x7FFFFFFFu) : ~o);
-        out.token[t] = 0xFFFFFFFFu - static_cast<uint32_t>(sc.keys[t]);
-    }
-    __syncthreads();
-    if (opt.temperature == 0.f) {
-        if (t == 0) { out.count = 1; out.total = 1.0; }
-        if (t < kMaxTopK) out.weight[t] = t == 0 ? 1.0 : 0.0;
-        __syncthreads();
-        return 0;
-    }
-    const float max_logit = sc.logit[0];
-    if (t < kMaxTopK) sc.w[t] = t < count ? exp(static_cast<double>(__fsub_rn(sc.logit[t], max_logit))) : 0.0;
-    __syncthreads();
-    if (t == 0) {
-        ordered_sums(sc.w, count, sc.run);
-        sc.kept = count; sc.cut = count;
-    }
-    __syncthreads();
-    {
-        // top-p keeps entries up to and including the first whose running share reaches top_p; min-p then
-        // keeps the leading entries (the first always) whose weight is at least min_p
-        const double total = sc.run[count - 1];
-        if (t + 1 < count && !(sc.run[t] / total < static_cast<double>(opt.top_p))) atomicMin(&sc.kept, t + 1);
-        if (opt.min_p > 0.f && t >= 1 && t < count && !(sc.w[t] >= static_cast<double>(opt.min_p))) atomicMin(&sc.cut, t);
-    }
-    __syncthreads();
-    count = sc.kept < sc.cut ? sc.kept : sc.cut;
-    if (t < kMaxTopK)   // zeros behind the last entry, for the sums
-        out.weight[t] = t < count ? exp(static_cast<double>(__fsub_rn(sc.logit[t], max_logit)) / static_cast<double>(opt.temperature)) : 0.0;
-    __syncthreads();
-    if (t == 0) {
-        const double norm = ordered_sums(out.weight, count, static_cast<double*>(nullptr));
-        out.count = count;
-        out.total = norm;
-        sc.err = (!isfinite(norm) || norm <= 0.0) ? -7 : 0;
-    }
-    __syncthreads();
-    return sc.err;
-}
-
-// Neumaier-compensated total with the reference's consistency checks; all threads call it (the quotients
-// are checked per lane, the compensated sum is one lane's), every thread gets the result: -1 when invalid.
-__device__ double validated_total(const Prepared& p, Scratch& sc) {
-    const uint32_t t = threadIdx.x;
-    __syncthreads();
-    const uint32_t count = p.count;
-    const double stored = p.total;
-    const bool shape_ok = !(count == 0 || count > kMaxTopK || !isfinite(stored) || stored <= 0.0);
-    if (t == 0) sc.flag = 0;
-    __syncthreads();
-    if (shape_ok && t < count) {
-        const double w = p.weight[t];
-        const double prob = w / stored;  // the stored probability is exactly this quotient
-        if (!isfinite(prob) || prob < 0.0 || prob > 1.0 || !isfinite(w) || w < 0.0) sc.flag = 1;
-    }
-    __syncthreads();
-    if (t == 0) {
-        double result = -1.0;
-        if (shape_ok && !sc.flag) {
-            double total = 0.0, correction = 0.0;
-            for (uint32_t i0 = 0; i0 < count; i0 += 8) {   // a zero past the end changes neither total nor correction
-                double x[8];
+// Neumaier's compensated sum over v[0] ... v[i], for every i; zeros past the end change nothing
+__device__ __forceinline__ void compensated_sums(const double* __restrict__ v, uint32_t n, double* __restrict__ out) {
+    double total = 0.0, correction = 0.0, x[8];
+    for (uint32_t i0 = 0; i0 < n; i0 += 8) {
 #pragma unroll
-                for (uint32_t k = 0; k < 8; ++k) x[k] = p.weight[i0 + k];
-#pragma unroll
-                for (uint32_t k = 0; k < 8; ++k) {
-                    const double w = x[k];
-                    const double sum = total + w;
-                    correction += total >= w ? (total - sum) + w : (w - sum) + total;
-                    total = sum;
-                }
-            }
-            total += correction;
-            const double tol = static_cast<double>(count) * 2.220446049250313e-16 * total;
-            if (isfinite(total) && total > 0.0 && !(fabs(total - stored) > tol)) result = total;
-        }
-        sc.value = result;
-    }
-    __syncthreads();
-    return sc.value;
-}
-
-__device__ uint32_t select_prepared(const Prepared& p, double draw) {
-    double cumulative = 0.0;
-    for (uint32_t i0 = 0; i0 < p.count; i0 += 8) {
-        double x[8];
-#pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) x[k] = p.weight[i0 + k];
+        for (uint32_t k = 0; k < 8; ++k) x[k] = v[i0 + k];
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
-            cumulative += x[k];
-            if (i0 + k < p.count && draw < cumulative) return p.token[i0 + k];
+            const double w = x[k], sum = total + w;
+            correction += total >= w ? (total - sum) + w : (w - sum) + total;
+            total = sum;
+            x[k] = total + correction;
         }
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) out[i0 + k] = x[k];
     }
-    return p.token[p.count - 1];
+}
+// the reference's consistency check of a law's stored total against its compensated sum
+__device__ __forceinline__ bool total_holds(double total, double stored, uint32_t count) {
+    const double tol = static_cast<double>(count) * 2.220446049250313e-16 * total;
+    return isfinite(total) && total > 0.0 && !(fabs(total - stored) > tol);
+}
+__device__ __forceinline__ bool total_usable(uint32_t count, double stored) {
+    return !(count == 0 || count > kMaxTopK || !isfinite(stored) || stored <= 0.0);
+}
+__device__ __forceinline__ bool weight_usable(double w, double stored) {
+    const double prob = w / stored;  // the stored probability is exactly this quotient
+    return isfinite(prob) && !(prob < 0.0) && !(prob > 1.0) && isfinite(w) && !(w < 0.0);
 }
 
 // target_to_draft: null when both sides share one vocabulary; else the law lives in draft ids and a
@@ -699,142 +579,255 @@ __device__ uint64_t law_mass(const LawCopy& law, const uint64_t* full_cdf, uint3
     return law.cdf[lo + 1] - law.cdf[lo];
 }
 
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(2 * kTeam)
 spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restrict__ law,
                    const uint64_t* __restrict__ full_cdf, uint32_t vocab, const uint32_t* __restrict__ history,
                    const uint32_t* __restrict__ history_count, const uint32_t* __restrict__ proposal_ptr, SamplerOptions opt, uint64_t seed, uint64_t step,
                    const StepDraws* __restrict__ injected, SpecResult* __restrict__ result,
                    uint32_t* __restrict__ status, const int32_t* __restrict__ target_to_draft) {
-    __shared__ Scratch sc;
-    __shared__ Prepared target, residual;
+    __shared__ RowScratch scratch[2];
+    __shared__ Prepared prepared[2], residual;
     __shared__ uint64_t q[kMaxTopK];
     __shared__ double diff[kMaxTopK];
-    __shared__ double s_proposed, s_acceptance;
-    __shared__ int s_code;
-    __shared__ uint32_t s_accepted, s_draw_residual;
+    __shared__ double s_acceptance;
+    __shared__ uint64_t s_begin, s_mass;
     __shared__ LawCopy q_law;
-    __shared__ uint64_t wave_mass[8];
-    __shared__ uint32_t wave_count[8];
-    const uint32_t t = threadIdx.x;
-    const uint32_t proposal = *proposal_ptr;
+    __shared__ uint64_t wave_mass[2 * kTeam / 64];
+    __shared__ uint32_t wave_count[2 * kTeam / 64];
+    const uint32_t team = __builtin_amdgcn_readfirstlane(threadIdx.x / kTeam), t = threadIdx.x - team * kTeam, lane = t & 63;
+    RowScratch& sc = scratch[team];
+    Prepared& out = prepared[team];
+    // ---- everything in one trip: a row's record, its history and the compact law are always whole in memory ----
+    const Candidates* cand = &rows[team];
+    const uint32_t n = cand->count;
+    const uint32_t token = cand->values[t].token;
+    const float raw = cand->values[t].logit;
+    const uint32_t history_n = history ? history_count[team] : 0u;
+    const uint32_t past = history && t < kHistoryCap ? history[team * kHistoryCap + t] : 0u;
+    const uint32_t law_id = team == 0 && t < 256 ? law->ids[t] : 0u;
+    const uint64_t law_edge = team == 0 && t < 257 ? law->cdf[t] : 0u;
+    const uint32_t law_count = law->count, proposal = *proposal_ptr;
     const StepDraws d = injected ? *injected : step_draws(seed, step);
-    // the compact law comes in once, every word by its own lane (the record is always whole in memory):
-    // the gathers below search it in LDS instead of through a chain of dependent trips to memory
-    if (t < 256) { q_law.ids[t] = law->ids[t]; q_law.cdf[t] = law->cdf[t]; }
-    if (t == 256) { q_law.cdf[256] = law->cdf[256]; q_law.count = law->count; }
+    if (team == 0 && t < 256) q_law.ids[t] = law_id;
+    if (team == 0 && t < 257) q_law.cdf[t] = law_edge;
     if (t == 0) {
-        result->accepted = 0; result->token = 0xFFFFFFFFu; result->next_root = 0xFFFFFFFFu; result->status = 0;
-        result->acceptance_probability = 0.0; result->residual_total = 0.0; result->residual_count = 0;
-        result->proposal = proposal;
+        sc.err = !options_valid(opt) ? -1 : (n == 0 || n > kMaxCandidates) ? -2 : history_n > kHistoryCap ? -3 : 0;
+        sc.dup = 0; sc.unique = 0; sc.flag = 0; sc.pick = 0xFFFFFFFFu;
+        if (team == 0) { q_law.count = law_count; s_acceptance = 0.0; }
     }
-    // history: [2][64] token ids and their counts per row (null: no repetition history)
-    int rc = prepare_distribution(&rows[0], opt, history, history ? history_count[0] : 0u, sc, target);
+    if (t < kHistoryCap) sc.hist[t] = past;
+    __syncthreads();
+    // ---- repetition penalty and sort key ------------------------------------------------------------------
+    int rc = sc.err;
+    const uint32_t entries = rc ? 0u : n;
+    uint64_t key = 0;
+    if (t < entries) {
+        float logit = raw;
+        for (uint32_t h = 0; h < history_n; ++h)
+            if (sc.hist[h] == token) {
+                logit = logit < 0.f ? __fmul_rn(logit, opt.repetition_penalty) : __fdiv_rn(logit, opt.repetition_penalty);
+                break;
+            }
+        key = score_key(logit, token);
+        sc.keys[t] = key;
+        sc.raw[t] = raw;
+    }
+    __syncthreads();
+    if (t < entries && !isfinite(raw)) atomicMin(&sc.err, -4);
+    // ---- places: the keys ahead of one's own, counted by four neighbouring lanes where the team has them to spare ----
+    {
+        const bool fours = entries <= kTeam / 4;
+        const uint32_t i = fours ? t >> 2 : t, from = fours ? t & 3u : 0u, by = fours ? 4u : 1u;
+        const uint64_t own = i < entries ? sc.keys[i] : 0;
+        uint32_t rank = 0, same = 0;
+#pragma unroll 8
+        for (uint32_t j = from; j < entries; j += by) {
+            const uint64_t other = sc.keys[j];
+            rank += other > own;
+            same += static_cast<uint32_t>(other) == static_cast<uint32_t>(own);   // one's own token, once
+        }
+        if (fours) {
+            rank += lane_cross_u32<0xB1, 0xF>(rank); rank += lane_cross_u32<0x4E, 0xF>(rank);
+            same += lane_cross_u32<0xB1, 0xF>(same); same += lane_cross_u32<0x4E, 0xF>(same);
+        }
+        if (i < entries && from == 0) {
+            if (same > 1) sc.dup = 1;
+            sc.sorted[rank] = own;
+        }
+        if (t == 0) sc.unique = entries;
+    }
+    __syncthreads();
+    if (scratch[0].dup | scratch[1].dup) {
+        // a token more than once: the first entry stays, a later one must carry the same logit
+        bool drop = false, differs = false;
+        if (t < entries)
+            for (uint32_t j = 0; j < t; ++j) {
+                const bool same = static_cast<uint32_t>(sc.keys[j]) == static_cast<uint32_t>(key);
+                drop |= same;
+                differs |= same & (sc.raw[j] != raw);
+            }
+        if (differs) atomicMin(&sc.err, -5);
+        __syncthreads();
+        if (drop) key = 0;   // a real key of a finite logit is never 0
+        if (t < entries) sc.keys[t] = key;
+        sc.sorted[t] = 0;
+        if (t == 0) sc.unique = 0;
+        __syncthreads();
+        if (key != 0) {
+            uint32_t rank = 0;
+            for (uint32_t j = 0; j < entries; ++j) rank += sc.keys[j] > key;
+            sc.sorted[rank] = key;
+            atomicAdd(&sc.unique, 1u);
+        }
+        __syncthreads();
+    }
+    // ---- raw weights of the best top_k -----------------------------------------------------------------------
+    rc = sc.err;
+    const uint32_t request_top_k = opt.temperature == 0.f ? 1u : opt.top_k;
+    if (!rc && sc.unique < request_top_k) rc = -6;
+    uint32_t count = rc ? 0u : request_top_k;
+    const bool plain = opt.temperature == 1.f || opt.temperature == 0.f;
+    float below = 0.f;   // how far the entry's logit lies under the best
+    if (t < kMaxTopK) {
+        double w = 0.0;
+        if (t < count) {
+            const uint64_t mine = sc.sorted[t];
+            below = __fsub_rn(key_score(mine), key_score(sc.sorted[0]));
+            out.token[t] = key_token(mine);
+            w = exp(static_cast<double>(below));
+        }
+        sc.w[t] = w;
+    }
+    if (t == 0) { sc.kept = count; sc.cut = count; }
+    __syncthreads();
+    if (t == 0) ordered_sums(sc.w, count, out.run);
+    if (team == 0) {
+        if (t == 64 && plain) compensated_sums(sc.w, count, sc.compensated);
+        if (!target_to_draft && t >= 128 && t - 128 < count) q[t - 128] = law_mass(q_law, full_cdf, vocab, out.token[t - 128], nullptr);
+    } else if (t == 128) {
+        uint64_t begin = 0;   // a law that failed leaves no proposal
+        s_mass = scratch[0].err || proposal == 0xFFFFFFFFu ? 0 : law_mass(q_law, full_cdf, vocab, proposal, &begin, target_to_draft);
+        s_begin = begin;
+    }
+    __syncthreads();
+    // ---- top-p keeps entries up to and including the first whose running share reaches top_p; min-p then keeps the leading
+    // entries (the first always) whose weight is at least min_p
+    if (count) {
+        const double total = out.run[count - 1];
+        if (t + 1 < count && !(out.run[t] / total < static_cast<double>(opt.top_p))) atomicMin(&sc.kept, t + 1);
+        if (opt.min_p > 0.f && t >= 1 && t < count && !(sc.w[t] >= static_cast<double>(opt.min_p))) atomicMin(&sc.cut, t);
+    }
+    __syncthreads();
+    count = sc.kept < sc.cut ? sc.kept : sc.cut;
+    if (plain) {
+        if (t < kMaxTopK) out.weight[t] = t < count ? sc.w[t] : 0.0;
+    } else {
+        if (t < kMaxTopK) out.weight[t] = t < count ? exp(static_cast<double>(below) / static_cast<double>(opt.temperature)) : 0.0;
+        __syncthreads();
+        if (t == 0) ordered_sums(out.weight, count, out.run);
+        if (t == 64 && team == 0) compensated_sums(out.weight, count, sc.compensated);
+        __syncthreads();
+    }
+    const double norm = count ? out.run[count - 1] : 0.0;
+    if (!rc && (!isfinite(norm) || norm <= 0.0)) rc = -7;
+    if (t == 0) { out.count = rc ? 0u : count; out.total = norm; if (team == 1) sc.err = rc; }
+    // ---- the checks of both laws, and what the proposal weighs in each ------------------------------------------
+    // (from here on team 0's threads work on row 0's law; team 1 follows through the barriers)
+    const bool head = team == 0;
     bool holds_proposal = false;
     uint64_t mass = 0;
-    if (!rc && t < target.count) {
-        q[t] = law_mass(q_law, full_cdf, vocab, target.token[t], nullptr, target_to_draft);
+    if (head && !rc && t < count) {
+        // through a vocabulary map only the tokens that stay are looked up
+        if (target_to_draft) q[t] = law_mass(q_law, full_cdf, vocab, out.token[t], nullptr, target_to_draft);
         // A mass is a difference of two edges: over edges out of order it wraps, and the sum of the masses may still be 2^32.
         // Counted as at most 2^32 + 1 each, 256 of them cannot wrap, and their sum, which as one of whole numbers does not
         // depend on the order, passes 2^32 exactly where some prefix does or some mass by itself.
         mass = q[t] <= kMassTotal ? q[t] : kMassTotal + 1;
-        holds_proposal = target.token[t] == proposal;
+        holds_proposal = out.token[t] == proposal;
+        if (!weight_usable(out.weight[t], norm)) sc.flag = 1;
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mass += __shfl_xor(mass, o, kWave);
-    if ((t & 63u) == 0) wave_mass[t >> 6] = mass;
+    if (lane == 0) wave_mass[threadIdx.x >> 6] = mass;
     const bool in_target = __syncthreads_or(holds_proposal) != 0;
-    const double normalization = rc ? -1.0 : validated_total(target, sc);
-    __syncthreads();
-    if (t == 0) {
-        int code = rc;
+    // ---- from here every thread follows row 0's decision ---------------------------------------------------------
+    const Prepared& target = prepared[0];
+    int code = head ? rc : 0;
+    double proposed = 0.0, normalization = -1.0;
+    if (head && !code) {
         auto unit = [](double u) { return isfinite(u) && u >= 0.0 && u < 1.0; };
-        if (!code && (!unit(d.u_accept) || !unit(d.u_residual) || !unit(d.u_next))) code = -20;
-        if (!code && normalization < 0.0) code = -21;
-        uint64_t begin = 0, proposal_mass = 0;
-        if (!code) {
-            proposal_mass = law_mass(q_law, full_cdf, vocab, proposal, &begin, target_to_draft);
-            if (proposal_mass == 0 || proposal_mass > kMassTotal || begin > kMassTotal - proposal_mass) code = -22;
-        }
-        if (!code) {
-            uint64_t gathered = 0;
-            for (int w = 0; w < 8; ++w) gathered += wave_mass[w];
-            if (gathered > kMassTotal) code = -23;
-            if (!code && !in_target && proposal_mass > kMassTotal - gathered) code = -24;
-        }
-        s_code = code;
-        s_accepted = 0;
-        s_draw_residual = 0;
-        s_acceptance = 0.0;
-        s_proposed = static_cast<double>(proposal_mass) / static_cast<double>(kMassTotal);
+        normalization = scratch[0].compensated[count - 1];
+        const bool valid = total_usable(count, norm) && !sc.flag && total_holds(normalization, norm, count);
+        uint64_t gathered = 0;
+        for (uint32_t w = 0; w < kTeam / 64; ++w) gathered += wave_mass[w];
+        if (!unit(d.u_accept) || !unit(d.u_residual) || !unit(d.u_next)) code = -20;
+        else if (!valid) code = -21;
+        else if (s_mass == 0 || s_mass > kMassTotal || s_begin > kMassTotal - s_mass) code = -22;
+        else if (gathered > kMassTotal) code = -23;
+        else if (!in_target && s_mass > kMassTotal - gathered) code = -24;
+        proposed = static_cast<double>(s_mass) / static_cast<double>(kMassTotal);
     }
+    // p, p / q of the proposal and p - q per lane; then the entries with an excess, in order, without gaps
+    bool more = false;
+    if (head && !code && t < count) {
+        const double p = target.weight[t] / normalization;
+        if (target.token[t] == proposal) s_acceptance = fmin(1.0, p / proposed);   // tokens are distinct
+        diff[t] = p - static_cast<double>(q[t]) / static_cast<double>(kMassTotal);
+        more = !(diff[t] <= 0.0);
+    }
+    const uint64_t ahead = __ballot(more);
+    if (lane == 0) wave_count[threadIdx.x >> 6] = static_cast<uint32_t>(__popcll(ahead));
     __syncthreads();
-    if (s_code == 0) {
-        // p, p / q of the proposal and p - q per lane; the residual's order and sum stay one lane's
-        if (t < target.count) {
-            const double p = target.weight[t] / normalization;
-            if (target.token[t] == proposal) s_acceptance = fmin(1.0, p / s_proposed);   // tokens are distinct
-            diff[t] = p - static_cast<double>(q[t]) / static_cast<double>(kMassTotal);
-        }
-        // the entries with an excess, in order, without gaps
-        const bool more = t < target.count && !(diff[t] <= 0.0);
-        const uint64_t ahead = __ballot(more);
-        if ((t & 63u) == 0) wave_count[t >> 6] = static_cast<uint32_t>(__popcll(ahead));
-        __syncthreads();
-        uint32_t at = static_cast<uint32_t>(__popcll(ahead & ((uint64_t{1} << (t & 63u)) - 1))), entries = 0;
-        for (uint32_t w = 0; w < 8; ++w) {
-            if (w < (t >> 6)) at += wave_count[w];
-            entries += wave_count[w];
-        }
-        if (t >= entries && t < kMaxTopK) residual.weight[t] = 0.0;
+    uint32_t at = static_cast<uint32_t>(__popcll(ahead & ((uint64_t{1} << lane) - 1))), excess = 0;
+    for (uint32_t w = 0; w < kTeam / 64; ++w) {
+        if (w < (t >> 6)) at += wave_count[w];
+        excess += wave_count[w];
+    }
+    if (head) {
+        if (t >= excess && t < kMaxTopK) residual.weight[t] = 0.0;
         if (more) { residual.token[at] = target.token[t]; residual.weight[at] = diff[t]; }
-        __syncthreads();
-        if (t == 0) {
-            int code = 0;
-            const double acceptance = s_acceptance;
-            residual.count = entries;
-            residual.total = ordered_sums(residual.weight, entries, static_cast<double*>(nullptr));
-            if (residual.count == 0 && acceptance < 1.0) code = -25;
-            result->acceptance_probability = acceptance;
-            result->residual_total = residual.total;
-            result->residual_count = residual.count;
-            if (!code) {
-                if (d.u_accept < acceptance) {
-                    s_accepted = 1;
-                    result->accepted = 1; result->token = proposal; result->next_root = proposal;
-                } else {
-                    s_draw_residual = 1;
-                }
-            }
-            s_code = code;
-        }
-        __syncthreads();
-        if (s_draw_residual) {
-            const double residual_total = validated_total(residual, sc);
-            if (t == 0) {
-                if (residual_total < 0.0) {
-                    s_code = -26;
-                } else {
-                    const uint32_t tok = select_prepared(residual, d.u_residual * residual.total);
-                    result->token = tok; result->next_root = tok;
-                }
-            }
-            __syncthreads();
-        }
+        if (t == 0) sc.flag = 0;
     }
-    if (s_code == 0 && s_accepted) {
-        // a fully accepted chain leaves row 1's candidates to seed the next root
-        rc = prepare_distribution(&rows[1], opt, history ? history + 64 : nullptr, history ? history_count[1] : 0u, sc, target);
-        if (t == 0) {
-            if (rc) s_code = rc - 100;
-            else result->next_root = opt.temperature == 0.f ? target.token[0]
-                                                             : select_prepared(target, d.u_next * target.total);
+    __syncthreads();
+    if (head && t == 0) ordered_sums(residual.weight, excess, residual.run);
+    if (head && t == 64) compensated_sums(residual.weight, excess, sc.compensated);
+    __syncthreads();
+    const double acceptance = s_acceptance, residual_total = excess ? residual.run[excess - 1] : 0.0;
+    const bool decided = code == 0;
+    bool accepted = false;
+    if (head && decided) {
+        if (excess == 0 && acceptance < 1.0) code = -25;
+        else accepted = d.u_accept < acceptance;
+    }
+    // ---- the draw: row 1's law behind an accepted proposal, the residual otherwise ---------------------------------
+    if (head && code == 0) {
+        if (accepted) {
+            const Prepared& after = prepared[1];
+            if (scratch[1].err) code = scratch[1].err - 100;
+            else if (t < after.count && d.u_next * after.total < after.run[t]) atomicMin(&sc.pick, t);
+        } else {
+            if (!total_usable(excess, residual_total) || !total_holds(sc.compensated[excess - 1], residual_total, excess)) code = -26;
+            else if (t < excess) {
+                if (!weight_usable(residual.weight[t], residual_total)) sc.flag = 1;
+                if (d.u_residual * residual_total < residual.run[t]) atomicMin(&sc.pick, t);
+            }
         }
     }
     __syncthreads();
-    if (t == 0 && s_code != 0) {
-        result->status = static_cast<uint32_t>(-s_code);
-        result->token = 0xFFFFFFFFu; result->next_root = 0xFFFFFFFFu; result->accepted = 0;
-        if (status) atomicOr(status, GUFFIN_STATUS_LAW_INVALID);
+    if (threadIdx.x == 0) {
+        if (!code && !accepted && sc.flag) code = -26;
+        const Prepared& from = accepted ? prepared[1] : residual;
+        const uint32_t length = accepted ? prepared[1].count : excess;
+        const uint32_t drawn = code ? 0xFFFFFFFFu : from.token[opt.temperature == 0.f && accepted ? 0u : min(sc.pick, length - 1)];
+        result->accepted = !code && accepted;
+        result->token = code ? 0xFFFFFFFFu : accepted ? proposal : drawn;
+        result->next_root = drawn;
+        result->status = static_cast<uint32_t>(-code);
+        result->acceptance_probability = decided ? acceptance : 0.0;
+        result->residual_total = decided ? residual_total : 0.0;
+        result->residual_count = decided ? excess : 0u;
+        result->proposal = proposal;
+        if (code && status) atomicOr(status, GUFFIN_STATUS_LAW_INVALID);
     }
 }
 
@@ -843,7 +836,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
 int select_candidates_scaled(hipStream_t s, const float* logits, uint32_t rows, uint32_t vocab, uint32_t retain,
                              float divisor, const uint32_t* history, const uint32_t* history_count,
                              void* workspace, void* result, uint32_t* status, bool suppressed_ok = false,
-                             const uint32_t* row_retain = nullptr, uint32_t row_stride = 1);
+                             const uint32_t* row_retain = nullptr, uint32_t row_stride = 1, uint32_t sure = 0, bool fresh = false);
 
 }  // namespace guffin
 
@@ -886,16 +879,16 @@ bool compact_options(const SamplerOptions& o) { return o.temperature > 0.f && o.
 
 int launch_compact_law(hipStream_t s, const float* logits, uint32_t vocab, const SamplerOptions& opt, uint64_t seed,
                        uint64_t step, const void* injected_draws, void* workspace, void* law, uint32_t* proposal,
-                       uint32_t* status, uint32_t* full_error, bool suppressed_ok = false) {
+                       uint32_t* status, uint32_t* full_error, bool suppressed_ok = false, bool fresh = false) {
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     Candidates* top = reinterpret_cast<Candidates*>(ws + ((guffin_hip_select_workspace_bytes(1, vocab, 257) + 15) & ~uint64_t{15}));
-    // the k-th best score and every tie with it: the best 257 scores decide both
+    // the k-th best score and every tie with it, up to one more than a compact law holds, decide it
     if (int rc = select_candidates_scaled(s, logits, 1, vocab, vocab < 257 ? vocab : 257, opt.temperature, nullptr,
-                                          nullptr, ws, top, status, suppressed_ok))
+                                          nullptr, ws, top, status, suppressed_ok, nullptr, 1, opt.top_k, fresh))
         return rc;
     launch(draft_law_kernel, dim3(1), dim3(256), 0, s, top, opt, seed, step,
                        static_cast<const StepDraws*>(injected_draws), static_cast<DraftLaw*>(law), proposal, status,
-                       full_error);
+                       full_error, fresh);
     return check_launch("draft_law");
 }
 
@@ -927,9 +920,9 @@ int launch_full_law(hipStream_t s, const float* logits, uint32_t vocab, const Sa
 
 }  // namespace
 
-extern "C" int guffin_hip_draft_law(void* stream, const float* logits, uint32_t vocab, const void* options,
-                                    uint64_t seed, uint64_t step, const void* injected_draws, void* workspace,
-                                    void* law, uint32_t* proposal, uint32_t* status) {
+namespace {
+int draft_law_compact(void* stream, const float* logits, uint32_t vocab, const void* options, uint64_t seed, uint64_t step,
+                      const void* injected_draws, void* workspace, void* law, uint32_t* proposal, uint32_t* status, bool fresh) {
     if (!logits || !options || !workspace || !law || !proposal || !status) return fail(GUFFIN_E_ARG, "draft_law: null pointer");
     if (vocab < 1) return fail(GUFFIN_E_SHAPE, "draft_law: empty vocabulary");
     if (reinterpret_cast<uintptr_t>(workspace) & 7u) return fail(GUFFIN_E_ALIGN, "draft_law: workspace must be 8-byte aligned");
@@ -937,7 +930,20 @@ extern "C" int guffin_hip_draft_law(void* stream, const float* logits, uint32_t 
     if (!compact_options(opt))
         return fail(GUFFIN_E_ARG, "draft_law: the compact law needs temperature > 0 and top_k in [1, 64]");
     return launch_compact_law(as_stream(stream), logits, vocab, opt, seed, step, injected_draws, workspace, law,
-                              proposal, status, nullptr);
+                              proposal, status, nullptr, false, fresh);
+}
+}  // namespace
+
+extern "C" int guffin_hip_draft_law(void* stream, const float* logits, uint32_t vocab, const void* options,
+                                    uint64_t seed, uint64_t step, const void* injected_draws, void* workspace,
+                                    void* law, uint32_t* proposal, uint32_t* status) {
+    return draft_law_compact(stream, logits, vocab, options, seed, step, injected_draws, workspace, law, proposal, status, false);
+}
+
+extern "C" int guffin_hip_draft_law_fresh(void* stream, const float* logits, uint32_t vocab, const void* options,
+                                          uint64_t seed, uint64_t step, const void* injected_draws, void* workspace,
+                                          void* law, uint32_t* proposal, uint32_t* status) {
+    return draft_law_compact(stream, logits, vocab, options, seed, step, injected_draws, workspace, law, proposal, status, true);
 }
 
 namespace guffin {
@@ -1088,7 +1094,7 @@ extern "C" int guffin_hip_spec_accept_mapped(void* stream, const void* target_ca
     if (!target_candidates || !law || !proposal || !options || !result) return fail(GUFFIN_E_ARG, "spec_accept: null pointer");
     if ((history == nullptr) != (history_count == nullptr)) return fail(GUFFIN_E_ARG, "spec_accept: history needs its counts");
     const SamplerOptions opt = *static_cast<const SamplerOptions*>(options);
-    launch(spec_accept_kernel, dim3(1), dim3(512), 0, as_stream(stream),
+    launch(spec_accept_kernel, dim3(1), dim3(2 * kTeam), 0, as_stream(stream),
                        static_cast<const Candidates*>(target_candidates), static_cast<const DraftLaw*>(law), full_cdf,
                        vocab, history, history_count, proposal, opt, seed, step,
                        static_cast<const StepDraws*>(injected_draws), static_cast<SpecResult*>(result), status,

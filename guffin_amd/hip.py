@@ -45,8 +45,10 @@ class _Calls:
         "guffin_hip_group_sums": (I, P, P, P, U, U),
         "guffin_hip_gemv_packed": (I, P, I, P, P, P, P, P, U, U, U),
         "guffin_hip_repack": (I, P, I, P, P, U, U),
+        "guffin_hip_select_candidates_fresh": (I, P, P, U, U, U, P, P, P, P, P),
         "guffin_hip_select_candidates": (I, P, P, U, U, U, P, P, P, P, P),
         "guffin_hip_argmax": (I, P, P, U, U, P, P, P, P),
+        "guffin_hip_draft_law_fresh": (I, P, P, U, P, Q, Q, P, P, P, P, P),
         "guffin_hip_draft_law": (I, P, P, U, P, Q, Q, P, P, P, P, P),
         "guffin_hip_spec_accept": (I, P, P, P, P, P, Q, Q, P, P, P),
         "guffin_hip_receipt_bytes": (Q, U, U),
@@ -444,6 +446,7 @@ result_dtype = _np.dtype([("accepted", _np.uint32), ("token", _np.uint32), ("nex
                           ("status", _np.uint32), ("acceptance_probability", _np.float64),
                           ("residual_total", _np.float64), ("residual_count", _np.uint32),
                           ("proposal", _np.uint32)])
+_candidates_bytes, _law_bytes = candidates_dtype.itemsize, law_dtype.itemsize
 draws_dtype = _np.dtype([("word", _np.uint32), ("pad", _np.uint32), ("u_accept", _np.float64),
                          ("u_residual", _np.float64), ("u_next", _np.float64)])
 
@@ -457,27 +460,30 @@ def _bytes(n, device="cuda"):
     return torch.zeros(int(n), dtype=torch.uint8, device=device)
 
 
-def _zeroed(device, *nbytes):
-    """Cleared byte buffers of the given sizes, one allocation and one fill between them."""
-    starts = [0]
-    for n in nbytes:
-        starts.append(starts[-1] + (int(n) + 15) // 16 * 16)
-    blob = torch.zeros(starts[-1], dtype=torch.uint8, device=device)
-    return [blob[at:at + int(n)] for at, n in zip(starts, nbytes)]
+@functools.lru_cache(maxsize=1024)
+def _select_workspace_bytes(rows, vocab, retain):
+    return _calls.guffin_hip_select_workspace_bytes(rows, vocab, retain)
+
+
+@functools.lru_cache(maxsize=1024)
+def _draft_law_workspace_bytes(vocab):
+    return _calls.guffin_hip_draft_law_workspace_bytes(vocab)
 
 
 def select_candidates(logits, retain, history=None, history_count=None, status=None, result=None):
     rows, vocab = logits.shape
-    ws = torch.empty(_calls.guffin_hip_select_workspace_bytes(rows, vocab, retain), dtype=torch.uint8, device="cuda")
-    if result is None and status is None:
-        result, status = _zeroed("cuda", rows * candidates_dtype.itemsize, 4 * rows)
-        status = status.view(torch.int32)
+    ws = torch.empty(_select_workspace_bytes(rows, vocab, retain), dtype=torch.uint8, device="cuda")
+    call = _calls.guffin_hip_select_candidates
+    if result is None and status is None:   # both new: the kernels clear what they do not write, no fill runs before them
+        result = torch.empty(rows * _candidates_bytes, dtype=torch.uint8, device="cuda")
+        status = torch.empty(rows, dtype=torch.int32, device="cuda")
+        call = _calls.guffin_hip_select_candidates_fresh
     if result is None:
-        result = _bytes(rows * candidates_dtype.itemsize)
+        result = _bytes(rows * _candidates_bytes)
     if status is None:
         status = torch.zeros(rows, dtype=torch.int32, device=logits.device)
-    check(_calls.guffin_hip_select_candidates(_raw_stream(), logits.data_ptr(), rows, vocab, retain, _at(history), _at(history_count),
-                                              ws.data_ptr(), result.data_ptr(), status.data_ptr()))
+    check(call(_raw_stream(), logits.data_ptr(), rows, vocab, retain, _at(history), _at(history_count), ws.data_ptr(), result.data_ptr(),
+               status.data_ptr()))
     return result, status
 
 
@@ -536,18 +542,21 @@ def argmax(logits, status=None):
 def draft_law(logits, options, seed=0, step=0, draws=None, law=None, proposal=None, status=None, workspace=None):
     vocab = logits.numel()
     if workspace is None:
-        workspace = torch.empty(_calls.guffin_hip_draft_law_workspace_bytes(vocab), dtype=torch.uint8, device="cuda")
-    if law is None and proposal is None and status is None:
-        law, proposal, status = _zeroed("cuda", law_dtype.itemsize, 4, 4)
-        proposal, status = proposal.view(torch.int32), status.view(torch.int32)
+        workspace = torch.empty(_draft_law_workspace_bytes(vocab), dtype=torch.uint8, device="cuda")
+    call = _calls.guffin_hip_draft_law
+    if law is None and proposal is None and status is None:   # all new, as in select_candidates
+        law = torch.empty(_law_bytes, dtype=torch.uint8, device="cuda")
+        proposal = torch.empty(1, dtype=torch.int32, device="cuda")
+        status = torch.empty(1, dtype=torch.int32, device="cuda")
+        call = _calls.guffin_hip_draft_law_fresh
     if law is None:
-        law = _bytes(law_dtype.itemsize)
+        law = _bytes(_law_bytes)
     if proposal is None:
         proposal = torch.zeros(1, dtype=torch.int32, device=logits.device)
     if status is None:
         status = torch.zeros(1, dtype=torch.int32, device=logits.device)
-    check(_calls.guffin_hip_draft_law(_raw_stream(), logits.data_ptr(), vocab, C.byref(options), seed, step, _at(draws), workspace.data_ptr(),
-                                      law.data_ptr(), proposal.data_ptr(), status.data_ptr()))
+    check(call(_raw_stream(), logits.data_ptr(), vocab, C.byref(options), seed, step, _at(draws), workspace.data_ptr(), law.data_ptr(),
+               proposal.data_ptr(), status.data_ptr()))
     return law, proposal, status
 
 
@@ -653,7 +662,7 @@ def spec_accept_history(cands, law, history, history_count, proposal, options, s
 
 def spec_accept(cands, law, proposal, options, seed=0, step=0, draws=None, result=None, status=None):
     if result is None:
-        result = _bytes(result_dtype.itemsize)
+        result = torch.empty(result_dtype.itemsize, dtype=torch.uint8, device="cuda")   # the kernel writes every word
     check(_calls.guffin_hip_spec_accept(_raw_stream(), cands.data_ptr(), law.data_ptr(), proposal.data_ptr(), C.byref(options), seed, step,
                                         _at(draws), result.data_ptr(), _at(status)))
     return result

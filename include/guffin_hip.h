@@ -250,6 +250,11 @@ uint64_t guffin_hip_select_workspace_bytes(uint32_t rows, uint32_t vocab, uint32
 int guffin_hip_select_candidates(void* stream, const float* logits, uint32_t rows, uint32_t vocab,
                                  uint32_t retain, const uint32_t* history, const uint32_t* history_count,
                                  void* workspace, void* result, uint32_t* status);
+/* The same into memory that nothing has cleared: status (not NULL) starts from 0 and the places of `values` that a row does
+ * not use become zero. */
+int guffin_hip_select_candidates_fresh(void* stream, const float* logits, uint32_t rows, uint32_t vocab,
+                                       uint32_t retain, const uint32_t* history, const uint32_t* history_count,
+                                       void* workspace, void* result, uint32_t* status);
 /* The token ids a verify pass reads on the device against the ids the host planned: a row whose id is
  * outside the vocabulary or differs sets GUFFIN_STATUS_BAD_TOKEN in the one status word.  Replaces
  * encode_verifier_input_validation (metal_command_context.hpp:221; verifier_input_validate_u32_kernel,
@@ -311,6 +316,11 @@ uint64_t guffin_hip_draft_law_workspace_bytes(uint32_t vocab);
 int guffin_hip_draft_law(void* stream, const float* logits, uint32_t vocab, const void* options,
                          uint64_t seed, uint64_t step, const void* injected_draws, void* workspace,
                          void* law, uint32_t* proposal, uint32_t* status);
+/* The same into memory that nothing has cleared: status starts from 0 and the words of the law that it does not use
+ * become zero. */
+int guffin_hip_draft_law_fresh(void* stream, const float* logits, uint32_t vocab, const void* options,
+                               uint64_t seed, uint64_t step, const void* injected_draws, void* workspace,
+                               void* law, uint32_t* proposal, uint32_t* status);
 /* scores[i] = logits[i] with the repetition penalty on the tokens of the sampler history (divided
  * when >= 0, multiplied when negative): what the drafter's gd_process does before its law is built
  * (src/engine/gemma3_draft.mm:186-204); the law entry points then take `scores` for logits.

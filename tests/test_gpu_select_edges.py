@@ -1,0 +1,73 @@
+"""Selection against a bound, where its stages change over: keys past a collector's own places, past the row's common list
+(992 keys) and past what is sorted in LDS (2048), ties across the last place, zeros of both signs, and results in memory that
+held something else.  The order (logit descending, token ascending) is exact, so the oracle is a stable sort on the host."""
+import numpy as np
+import pytest
+import torch
+
+from guffin_amd import hip
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _init():
+    hip.init(0)
+
+
+def rows_of(kind, vocab, rng):
+    x = rng.standard_normal((2, vocab)).astype(np.float32)
+    if kind == "zeros":
+        x = np.where(rng.random(x.shape) < 0.5, np.float32(0.0), np.float32(-0.0))
+        x[:, : vocab // 2] -= np.float32(1.0)
+    elif kind.startswith("run"):          # a run of equal logits above the rest, ending inside the answer or far beyond it
+        n = int(kind[3:])
+        x[0, 1000:1000 + n] = 9.0
+        x[1, vocab - n:] = 9.0
+    elif kind.startswith("spread"):       # the same, dealt to all collectors
+        n = int(kind[6:])
+        for r in range(2):
+            x[r, rng.permutation(vocab)[:n]] = 9.0
+    elif kind == "narrow":                # all within one step of the bound's first bytes
+        x = 100.0 + x * np.float32(1e-4)
+    return x
+
+
+@pytest.mark.parametrize("vocab", [32768, 131585, 262144])
+@pytest.mark.parametrize("retain", [1, 17, 64])
+@pytest.mark.parametrize("kind", ["normal", "narrow", "zeros", "run15", "run300", "run1100", "run2049", "spread1023", "spread1100", "spread2500"])
+def test_selection_is_a_stable_sort(kind, retain, vocab):
+    x = rows_of(kind, vocab, np.random.default_rng(retain + vocab))
+    junk = torch.full((1 << 20,), 0x5A, dtype=torch.uint8, device="cuda")   # what the next buffers may be cut from
+    del junk
+    got, status = hip.select_candidates(torch.from_numpy(x).cuda(), retain)
+    got = hip.candidates_to_numpy(got)
+    assert status.cpu().tolist() == [0, 0]
+    for r in range(2):
+        want = np.argsort(-x[r], kind="stable")[:retain]
+        values = got[r]["values"]
+        assert (int(got[r]["count"]), int(got[r]["status"])) == (retain, 0)
+        assert np.array_equal(values["token"][:retain], want.astype(np.uint32))
+        assert np.array_equal(values["logit"][:retain].view(np.uint32), x[r][want].view(np.uint32))   # a zero's sign too
+        assert not values["token"][retain:].any() and not values["logit"][retain:].view(np.uint32).any()
+
+
+@pytest.mark.parametrize("top_k", [1, 5, 64])
+@pytest.mark.parametrize("ties", [0, 1, 40, 200, 300])
+def test_the_law_holds_every_tie_with_the_last_place(ties, top_k):
+    """`ties` logits beyond the top_k-th equal it: all of them are in the law, or it is refused where they pass 256."""
+    rng = np.random.default_rng(ties)
+    x = rng.standard_normal(262144).astype(np.float32)
+    order = np.argsort(-x, kind="stable")
+    x[order[top_k - 1:top_k + ties]] = x[order[top_k - 1]]
+    law, proposal, status = hip.draft_law(torch.from_numpy(x).cuda(), hip.SamplerOptions(1.0, top_k, 1.0, 0.0, 1.0), seed=3, step=1)
+    law = law.cpu().numpy().view(hip.law_dtype)[0]
+    n = top_k + ties
+    if n > 256:
+        assert int(law["count"]) == 0 and int(status.item()) != 0 and proposal.item() == -1
+        assert not law["ids"].any() and not law["cdf"].any()
+    else:
+        assert int(law["count"]) == n and int(status.item()) == 0
+        assert np.array_equal(law["ids"][:n], np.sort(np.flatnonzero(x >= x[order[top_k - 1]])).astype(np.uint32))
+        assert int(law["cdf"][0]) == 0 and int(law["cdf"][n]) == 1 << 32
+        assert not law["ids"][n:].any() and not law["cdf"][n + 1:].any()
