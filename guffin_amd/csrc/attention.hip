@@ -110,12 +110,6 @@ __device__ __forceinline__ void finish_head_row(HeadRow& h, bool norm, bool rota
     }
 }
 
-// A workgroup barrier for data that moves through LDS: it waits for this wave's LDS operations only.
-// (__syncthreads() also waits for every vector load in flight -- here the key rows requested before the
-// queries are prepared and the value rows requested before the softmax, which are meant to stay in flight
-// across it.)  Nothing a wave stores to global memory in this kernel is read by another wave of the launch.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 __device__ __forceinline__ float dot2(float acc, uint32_t packed_half2, float a, float b) {
     const half2_t h = __builtin_bit_cast(half2_t, packed_half2);
     acc = fmaf(static_cast<float>(h.x), a, acc);
@@ -124,8 +118,17 @@ __device__ __forceinline__ float dot2(float acc, uint32_t packed_half2, float a,
 
 // waves of a partition's workgroup: two per SIMD.  With eight the queries and the private rows' key / value are
 // prepared by different waves, and a 32-token partition is one round of keys and two of values per wave.
-// (Eight query rows keep four waves: their per-wave output slots would not fit 64 KB of LDS otherwise.)
-constexpr int attention_waves(int queries) { return queries <= 4 ? 8 : 4; }
+// (Sixteen queries keep four waves: their per-wave output slots would take all of the LDS otherwise.  Eight take 73-81 KB, for
+// one workgroup on a compute unit as it is; with four waves a local layer of four rows took 15.4 us instead of 9.4.)
+constexpr int attention_waves(int queries) { return queries <= 8 ? 8 : 4; }
+
+// Where a dimension lies among the 256 floats of a query in LDS: a lane reads dimensions 8 seg .. 8 seg + 7 of each half of the
+// row in four pieces of 16 bytes, and a piece of 16 lanes is 256 bytes without a gap (in the row's own order, every other 16
+// bytes, two lanes share each bank).  With the halves of a wave combined by lane swaps, not shuffles through LDS, a local layer
+// of one row went from 7.4 to 6.3 us, of two from 10.4 to 8.0.
+__device__ __forceinline__ uint32_t query_place(uint32_t d) {
+    return ((d >> 7) * 2 + ((d >> 2) & 1)) * 64 + ((d >> 3) & 15) * 4 + (d & 3);
+}
 
 template <int ROWS, int GROUP, int HD, bool FUSED>
 __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_partial_kernel(AttnArgs a) {
@@ -268,7 +271,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
             if (item < NQ) {
                 finish_head_row(qr[i], a.q_norm != nullptr, true, a.eps);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) q_s[item * HD + lane + 64 * c] = qr[i].v[c];
+                for (int c = 0; c < 4; ++c) q_s[item * HD + query_place(lane + 64 * c)] = qr[i].v[c] * a.scale;
             }
         }
 #pragma unroll
@@ -297,10 +300,17 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
             const uint32_t r = n / group, g = n % group;
-            const float* qp = FUSED ? q_s + n * HD + seg * 8
-                                    : a.q + (size_t(r) * a.q_heads + kvh * group + g) * HD + seg * 8;
+            if constexpr (FUSED) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) { qv[n][i] = qp[i] * a.scale; qv[n][8 + i] = qp[HD / 2 + i] * a.scale; }
+                for (int c = 0; c < 4; ++c) {
+                    const float4 p = *reinterpret_cast<const float4*>(q_s + n * HD + c * 64 + seg * 4);
+                    qv[n][4 * c] = p.x; qv[n][4 * c + 1] = p.y; qv[n][4 * c + 2] = p.z; qv[n][4 * c + 3] = p.w;
+                }
+            } else {
+                const float* qp = a.q + (size_t(r) * a.q_heads + kvh * group + g) * HD + seg * 8;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) { qv[n][i] = qp[i] * a.scale; qv[n][8 + i] = qp[HD / 2 + i] * a.scale; }
+            }
         }
         // U rounds stay in flight for the whole walk: a slot is asked for its next row (U rounds on) as soon as its
         // row has been read, so a long partition streams instead of filling and draining once per batch
@@ -387,27 +397,31 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
         }
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
+            // one swap per pair of dimensions: the lower lanes end with both halves' even one, the upper with the odd one
+            float both[4];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[n][i] += __shfl_xor(acc[n][i], 32, kWave);
-            if (hsel == 0) {
-                float* mp = merge + (wv * NQ + n) * HD + dl;
-                *reinterpret_cast<float4*>(mp) = make_float4(acc[n][0], acc[n][1], acc[n][2], acc[n][3]);
-                *reinterpret_cast<float4*>(mp + 4) = make_float4(acc[n][4], acc[n][5], acc[n][6], acc[n][7]);
+            for (int i = 0; i < 4; ++i) {
+                const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[n][2 * i]), __float_as_uint(acc[n][2 * i + 1]), false, false);
+                both[i] = both_sum({p[0], p[1]});
             }
+            *reinterpret_cast<float4*>(merge + (wv * NQ + n) * HD + hsel * (HD / 2) + (lane & 31) * 4) = make_float4(both[0], both[1], both[2], both[3]);
         }
     }
     lds_barrier();
-    for (uint32_t i = threadIdx.x; i < NQ * HD; i += 64 * kAW) {
-        const uint32_t n = i / HD, d = i % HD;
-        float pair[kAW / 2];   // waves in pairs, the pairs in order
+    for (uint32_t i = threadIdx.x; i < NQ * (HD / 2); i += 64 * kAW) {
+        const uint32_t n = i / (HD / 2), d = i % (HD / 2);   // dimensions 2d and 2d + 1
+        auto total = [&](const float* at) {
+            float pair[kAW / 2];   // waves in pairs, the pairs in order
 #pragma unroll
-        for (int w = 0; w < kAW; w += 2) pair[w / 2] = merge[(w * NQ + n) * HD + d] + merge[((w + 1) * NQ + n) * HD + d];
-        float v = pair[0] + pair[1];
+            for (int w = 0; w < kAW; w += 2) pair[w / 2] = at[(w * NQ + n) * HD] + at[((w + 1) * NQ + n) * HD];
+            float v = pair[0] + pair[1];
 #pragma unroll
-        for (int w = 2; w < kAW / 2; w += 2) v += pair[w] + pair[w + 1];
+            for (int w = 2; w < kAW / 2; w += 2) v += pair[w] + pair[w + 1];
+            return v;
+        };
         const uint32_t r = n / group, g = n % group, head = kvh * group + g;
         const size_t slot = (size_t(r) * a.q_heads + head) * a.partitions + part;
-        a.part_out[slot * HD + d] = v;
+        *reinterpret_cast<F2a4*>(a.part_out + slot * HD + 2 * d) = {total(merge + d), total(merge + HD / 2 + d)};
         if (d == 0) { a.part_ml[slot * 2] = s_max[n]; a.part_ml[slot * 2 + 1] = s_sum[n]; }
     }
 }
@@ -416,7 +430,8 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
 // Each thread owns one output dimension.  The outputs of the first 64 partitions are requested at
 // once, before the weights exist (indices beyond the last partition read the last one again and
 // meet a zero weight), so up to 64 partitions cost one trip to memory; weights and denominators
-// terms are formed once, in parallel, in LDS.
+// terms are formed once, in parallel, in LDS, while the outputs are on their way.  (4.7 us of
+// 32 partitions; 4.8 with barriers that wait for them.)
 constexpr int kMergeAhead = 64;
 template <int AHEAD>
 __global__ void __launch_bounds__(256)
@@ -446,7 +461,7 @@ attn_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ 
     for (uint32_t p = threadIdx.x + 256; p < partitions; p += 256) if (ml[2 * p + 1] > 0.f) m = fmaxf(m, ml[2 * p]);
     m = wave_max(m);
     if (lane == 0) red[wv] = m;
-    __syncthreads();
+    lds_barrier();
     const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     for (uint32_t p = threadIdx.x; p < slots; p += 256) {
         const bool first = p == threadIdx.x;
@@ -454,7 +469,7 @@ attn_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ 
         wgt[p] = l > 0.f ? expf((first ? own.x : ml[2 * p]) - M) : 0.f;
         lsum[p] = l;
     }
-    __syncthreads();
+    lds_barrier();
     float denom = 0.f, acc0 = 0.f;
 #pragma unroll
     for (int q = 0; q < AHEAD; ++q) {
@@ -481,7 +496,7 @@ attn_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ 
     }
     if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
     if (out_sums) {
-        __syncthreads();
+        lds_barrier();
         // receipt of the attention output row [q_heads*hd], the o-projection's input
         emit_receipt(rowbuf, (rh % q_heads) * hd, hd, rh / q_heads, gridDim.x / q_heads, q_heads * hd, out_sums);
     }
@@ -493,6 +508,16 @@ int launch_partial(hipStream_t s, const AttnArgs& a) {
     constexpr int kAW = attention_waves(NQ);
     const bool fused = a.q_raw != nullptr;
     const size_t lds = (size_t(NQ) * a.span + size_t(kAW) * NQ * 256 + (fused ? size_t(NQ) * 256 : 0)) * sizeof(float);
+    if constexpr (kAW * NQ * 256 * sizeof(float) >= 64 * 1024) {   // more than a launch gets unasked, allowed once per kernel
+        static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_partial_kernel<ROWS, GROUP, 256, true>),
+                                                              hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+        if (allowed != hipSuccess || lds > 96 * 1024) return fail(GUFFIN_E_HIP, "attention_partial: could not raise the dynamic LDS limit");
+    }
+    if constexpr (kAW * NQ * 256 * sizeof(float) >= 64 * 1024 && ROWS <= 2) {
+        static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_partial_kernel<ROWS, GROUP, 256, false>),
+                                                              hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+        if (allowed != hipSuccess) return fail(GUFFIN_E_HIP, "attention_partial: could not raise the dynamic LDS limit");
+    }
     if (fused || ROWS > 2)
         launch((attn_partial_kernel<ROWS, GROUP, 256, true>), dim3(a.partitions, a.kv_heads), dim3(64 * kAW), lds, s, a);
     else if constexpr (ROWS <= 2)

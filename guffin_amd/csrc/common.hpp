@@ -94,6 +94,7 @@ struct __attribute__((packed, aligned(4))) U4a4 { uint32_t x, y, z, w; };
 struct __attribute__((packed, aligned(2))) U4a2 { uint32_t x, y, z, w; };
 struct __attribute__((packed, aligned(2))) U2a2 { uint32_t x, y; };
 struct __attribute__((packed, aligned(4))) F4a4 { float x, y, z, w; };
+struct __attribute__((packed, aligned(4))) F2a4 { float x, y; };
 
 __device__ __forceinline__ uint4 ld16_a4(const uint8_t* p) {
     const U4a4 t = *reinterpret_cast<const U4a4*>(p);
@@ -135,8 +136,9 @@ __device__ __forceinline__ float sb3(uint32_t v) { return static_cast<float>(sta
 
 // Sums and maxima over the 16 lanes of a row on the vector unit's lane-crossing modifiers (two quad permutations,
 // then the mirror of 8 and of 16 lanes: every lane ends with the row's total), and over the wave with two more
-// steps through the LDS crossbar.  A crossbar shuffle costs a wave that is alone on its SIMD more than a hundred
-// cycles, and the reductions sit in dependent chains; every lane of the wave must be active.
+// steps that swap neighbouring rows and halves of the wave.  A shuffle through the LDS crossbar would cost a wave that is
+// alone on its SIMD more than a hundred cycles, and the reductions sit in dependent chains; every lane of the wave must be
+// active.
 template <int CTRL>
 __device__ __forceinline__ float lane_cross(float v) {   // a lane outside the modifier's reach reads 0
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
@@ -148,6 +150,18 @@ __device__ __forceinline__ float row16_sum(float v) {
     v += lane_cross<0x140>(v);   // row_mirror
     return v;
 }
+// the values of this lane's row and of the row beside it (xor 16 lanes), the even row's first; the same for the wave's halves
+struct Both { uint32_t a, b; };
+__device__ __forceinline__ Both rows_beside(uint32_t v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return {r[0], r[1]};
+}
+__device__ __forceinline__ Both halves_beside(uint32_t v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return {r[0], r[1]};
+}
+__device__ __forceinline__ float both_sum(Both p) { return __uint_as_float(p.a) + __uint_as_float(p.b); }
+__device__ __forceinline__ float both_max(Both p) { return fmaxf(__uint_as_float(p.a), __uint_as_float(p.b)); }
 __device__ __forceinline__ float row16_max(float v) {
     v = fmaxf(v, lane_cross<0xB1>(v));
     v = fmaxf(v, lane_cross<0x4E>(v));
@@ -175,20 +189,24 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     v = max(v, lane_cross_u32<0x4E, 0xF>(v));
     v = max(v, lane_cross_u32<0x141, 0xF>(v));
     v = max(v, lane_cross_u32<0x140, 0xF>(v));
-    v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), 16, kWave)));
-    return max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), 32, kWave)));
+    const Both rows = rows_beside(v);
+    const Both halves = halves_beside(max(rows.a, rows.b));
+    return max(halves.a, halves.b);
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
-    v = row16_sum(v);
-    v += __shfl_xor(v, 16, kWave);
-    return v + __shfl_xor(v, 32, kWave);
+    v = both_sum(rows_beside(__float_as_uint(row16_sum(v))));
+    return both_sum(halves_beside(__float_as_uint(v)));
 }
 __device__ __forceinline__ float wave_max(float v) {
-    v = row16_max(v);
-    v = fmaxf(v, __shfl_xor(v, 16, kWave));
-    return fmaxf(v, __shfl_xor(v, 32, kWave));
+    v = both_max(rows_beside(__float_as_uint(row16_max(v))));
+    return both_max(halves_beside(__float_as_uint(v)));
 }
+
+// A workgroup barrier for data that moves through LDS: it waits for this wave's LDS operations only.  (__syncthreads() also
+// waits for every load and store to memory under way: for operands of later steps that were requested ahead, and for results on
+// their way out, a trip to memory in the middle of a chain.)  What waves exchange through memory needs the other.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Sum of `planes` partial planes in plane order; loads are issued four at a time so that the
 // adds, not the memory latency, form the dependent chain.
