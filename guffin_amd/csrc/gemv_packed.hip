@@ -303,11 +303,8 @@ gateup_geglu_kernel(const uint8_t* __restrict__ gate_tiles, const uint8_t* __res
         h[size_t(r) * F + blockIdx.x * kTileCols + lane] = v;
         vals[r * 64 + lane] = v;
     }
-    __syncthreads();
-    if (h_receipt) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) emit_receipt(vals + r * 64, blockIdx.x * kTileCols, kTileCols, r, R, F, h_receipt);
-    }
+    lds_barrier();   // h is on its way out and nobody here reads it
+    if (h_receipt && wave < uint32_t(R)) emit_receipt(vals + wave * 64, blockIdx.x * kTileCols, kTileCols, wave, R, F, h_receipt, lane, 64);
 }
 
 int g_cus = 256;

@@ -137,8 +137,8 @@ gateup_wide_kernel(const uint8_t* __restrict__ gate_tiles, const uint8_t* __rest
         h[size_t(i >> 6) * F + blockIdx.x * kTileCols + (i & 63u)] = v;
         vals[i] = v;
     }
-    __syncthreads();
-    for (uint32_t r = 0; r < c.rows; ++r) emit_receipt(vals + r * 64, blockIdx.x * kTileCols, kTileCols, r, c.rows, F, h_receipt);
+    lds_barrier();   // h is on its way out and nobody here reads it
+    if (wave < c.rows) emit_receipt(vals + wave * 64, blockIdx.x * kTileCols, kTileCols, wave, c.rows, F, h_receipt, lane, 64);
 }
 
 __global__ void wide_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, uint32_t planes, uint32_t count) {

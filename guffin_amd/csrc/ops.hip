@@ -107,7 +107,7 @@ rms_norm_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_strid
         second(c, gamma[c], residual ? residual[size_t(r) * width + c] : 0.f);
     if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
     if (y_sums) {
-        __syncthreads();
+        lds_barrier();   // y is on its way out and nobody here reads it
         emit_receipt(row, 0, width, r, gridDim.x, width, y_sums);
     }
 }
@@ -170,7 +170,7 @@ rms_norm_add_norm_kernel(const float* __restrict__ x, uint32_t planes, size_t pl
     for (uint32_t c = threadIdx.x + PF * blockDim.x; c < width; c += blockDim.x) third(c, gamma_next[c]);
     if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
     if (out_sums) {
-        __syncthreads();
+        lds_barrier();
         emit_receipt(row, 0, width, r, gridDim.x, width, out_sums);
     }
 }
@@ -373,7 +373,7 @@ geglu_kernel(const float* __restrict__ gate, const float* __restrict__ up, uint3
         if (out_sums) lds[c - c0] = v;
     }
     if (out_sums) {
-        __syncthreads();
+        lds_barrier();
         emit_receipt(lds, c0, c1 - c0, blockIdx.y, gridDim.y, width, out_sums);
     }
 }

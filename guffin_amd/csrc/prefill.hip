@@ -484,8 +484,8 @@ prefill_attention_merge_kernel(AttentionOut to, uint32_t rows, uint32_t q_heads,
     const size_t stride = size_t(rows) * q_heads;
     // a lane a part's state, 32 at a time: their maximum and weights are two reductions instead of a walk of one trip a part
     const float2* states = reinterpret_cast<const float2*>(to.part_ml);
-    auto top_of = [](float x) { x = row16_max(x); return fmaxf(x, __shfl_xor(x, 16, kWave)); };
-    auto sum_of = [](float x) { x = row16_sum(x); return x + __shfl_xor(x, 16, kWave); };
+    auto top_of = [](float x) { return both_max(rows_beside(__float_as_uint(row16_max(x)))); };
+    auto sum_of = [](float x) { return both_sum(rows_beside(__float_as_uint(row16_sum(x)))); };
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, den = 0.f, M = -INFINITY;
     for (uint32_t p0 = 0; p0 < parts; p0 += 32) {
         const float2 st = p0 + c8 < parts ? states[(p0 + c8) * stride + pair] : make_float2(-INFINITY, 0.f);   // a part can hold no visible token

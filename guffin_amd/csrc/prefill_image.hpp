@@ -48,7 +48,7 @@ __device__ __forceinline__ void emit_image_values(const float (&v)[8], uint32_t 
     if (L.span == 256) {
         m = fmaxf(m, lane_cross<0x141>(m));
         m = fmaxf(m, lane_cross<0x140>(m));
-        m = fmaxf(m, __shfl_xor(m, 16, kWave));
+        m = both_max(rows_beside(__float_as_uint(m)));
     }
     // biased exponent of the span's maximum, clamped so that both scale factors are normal floats
     uint32_t eb = __float_as_uint(m) >> 23;

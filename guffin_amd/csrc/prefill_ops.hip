@@ -15,12 +15,12 @@
 namespace guffin {
 namespace {
 
+// scratch: nobody else's, and used once
 __device__ __forceinline__ float block_total(float v, float* scratch) {
     v = wave_sum(v);
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, waves = (blockDim.x + 63) >> 6;
-    __syncthreads();  // scratch may still be read from a previous call
     if (lane == 0) scratch[wv] = v;
-    __syncthreads();
+    lds_barrier();
     float t = 0.f;
     for (uint32_t i = 0; i < waves; ++i) t += scratch[i];  // same order on every thread
     return t;
@@ -102,7 +102,7 @@ prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_
         static_cast<U4a4*>(run.ring_v)[dst] = static_cast<const U4a4*>(run.run_v)[size_t(row) * run.row_vec + c];
         return;
     }
-    __shared__ float scratch[16];
+    __shared__ float scratch[2][16];
     const uint32_t r = blockIdx.x, t = threadIdx.x;
     const bool active = t < width / 8;
     const size_t at = size_t(r) * width + 8 * t;
@@ -116,7 +116,7 @@ prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
-    float inv = 1.0f / sqrtf(block_total(ss, scratch) / static_cast<float>(width) + eps);
+    float inv = 1.0f / sqrtf(block_total(ss, scratch[0]) / static_cast<float>(width) + eps);
     bool bad = false;
     ss = 0.f;
 #pragma unroll
@@ -125,8 +125,8 @@ prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_
         bad |= !isfinite(v[i]);
         ss = fmaf(v[i], v[i], ss);
     }
+    inv = 1.0f / sqrtf(block_total(ss, scratch[1]) / static_cast<float>(width) + eps);
     if (active) store8(out_residual + at, v);
-    inv = 1.0f / sqrtf(block_total(ss, scratch) / static_cast<float>(width) + eps);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = v[i] * inv * gn[i];
     if (active) {
@@ -154,7 +154,7 @@ prefill_geglu_kernel(const float* __restrict__ gate, const float* __restrict__ u
         for (int k = 0; k < 8; ++k) g[k] = geglu_value(g[k], u[k]);
         emit_image_values(g, t0 + c, row, L, image, records);
     }
-    __syncthreads();
+    lds_barrier();   // what went to memory already is read by nobody here
     // 8 rows of a record's k-slice are 128 contiguous bytes; padding rows' places hold what they held: nobody looks at them
     const uint32_t tile = blockIdx.y >> 1, half = (blockIdx.y & 1) * 128;
     for (uint32_t k = threadIdx.x; k < (valid / 4) * 64; k += 256) {
@@ -247,7 +247,7 @@ prefill_qkv_kernel(QkvRun a) {
             }
             *reinterpret_cast<uint4*>(&tile[token][8 * d8]) = val;
         }
-        __syncthreads();
+        lds_barrier();
         const uint32_t dim = threadIdx.x >> 2, t0 = 8 * (threadIdx.x & 3);   // four threads: a dimension's 32 tokens
         uint32_t o[4];
 #pragma unroll
