@@ -478,7 +478,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
 // the parts' states of every (row, head), merged in part order; 32 lanes per pair
 __global__ void __launch_bounds__(256)
 prefill_attention_merge_kernel(AttentionOut to, uint32_t rows, uint32_t q_heads, uint32_t parts) {
-    constexpr uint32_t HD = 256;
+    constexpr uint32_t HD = 256, kAhead = 12;   // parts asked for at once
     const uint32_t pair = blockIdx.x * 8 + threadIdx.x / 32, c8 = threadIdx.x % 32;
     if (pair >= rows * q_heads) return;
     const size_t stride = size_t(rows) * q_heads;
@@ -500,15 +500,18 @@ prefill_attention_merge_kernel(AttentionOut to, uint32_t rows, uint32_t q_heads,
         const float w = exp_of(st.x - base);
         den += sum_of(w * st.y);
         const uint32_t n = min(parts - p0, 32u);
-        for (uint32_t i0 = 0; i0 < n; i0 += 8) {
-            float4 a[8], b[8];
+        for (uint32_t i0 = 0; i0 < n; i0 += kAhead) {
+            float4 a[kAhead], b[kAhead];
 #pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) {
-                const float* src = to.part_o + ((p0 + min(i0 + i, n - 1)) * stride + pair) * HD + 8 * c8;
-                a[i] = *reinterpret_cast<const float4*>(src); b[i] = *reinterpret_cast<const float4*>(src + 4);
+            for (uint32_t i = 0; i < kAhead; ++i) {
+                a[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (i0 + i < n) {
+                    const float* src = to.part_o + ((p0 + i0 + i) * stride + pair) * HD + 8 * c8;
+                    a[i] = *reinterpret_cast<const float4*>(src); b[i] = *reinterpret_cast<const float4*>(src + 4);
+                }
             }
 #pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) {
+            for (uint32_t i = 0; i < kAhead; ++i) {
                 const float wi = __shfl(w, (threadIdx.x & 32u) + min(i0 + i, 31u), kWave), f = i0 + i < n ? wi : 0.f;
                 if (f == 0.f) continue;   // nothing of a part without tokens, whatever it left
                 v[0] = fmaf(f, a[i].x, v[0]); v[1] = fmaf(f, a[i].y, v[1]); v[2] = fmaf(f, a[i].z, v[2]); v[3] = fmaf(f, a[i].w, v[3]);
@@ -668,7 +671,9 @@ AttentionCut attention_cut(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_
     const uint32_t pairs = rows * group, twos = (pairs + 31) / 32 * kv_heads, ones = (pairs + 15) / 16 * kv_heads;
     const uint32_t cus = compute_units();
     if (twos >= cus) return {2, 1};
-    return {1, std::max(1u, std::min(2 * cus / ones, T / 128))};
+    // (one tile more than a wave each would be a second round for one of them: 37 rows behind 1500 tokens, 34 tiles in eight
+    // parts 16.4 us, in nine 14.4; a second part costs the launch that merges them, more than a second round)
+    return {1, std::max(1u, std::min(2 * cus / ones, T < 256 ? 1 : (T + 127) / 128))};
 }
 // more than 64 KB of LDS a workgroup has to be allowed once per kernel
 int allow_attention_lds() {
