@@ -435,9 +435,8 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
 constexpr int kMergeAhead = 64;
 template <int AHEAD>
 __global__ void __launch_bounds__(256)
-attn_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ part_ml, float* __restrict__ out,
-                  float* __restrict__ out_sums, uint32_t partitions, uint32_t hd, uint32_t q_heads,
-                  uint32_t* __restrict__ status) {
+attn_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ part_ml, uint32_t partitions, uint32_t hd, uint32_t q_heads,
+                  uint32_t rows, float* __restrict__ out, float* __restrict__ out_sums, uint32_t* __restrict__ status) {
     extern __shared__ float wgt[];  // [max(partitions, 64)] weights, then as many partition sums l_p
     __shared__ float red[4];
     __shared__ float rowbuf[1024];
@@ -478,7 +477,7 @@ attn_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ 
     }
     for (uint32_t p = AHEAD; p < partitions; ++p) denom = fmaf(wgt[p], lsum[p], denom);
     bool bad = false;
-    for (uint32_t d = threadIdx.x; d < hd; d += blockDim.x) {
+    for (uint32_t d = threadIdx.x; d < hd; d += 256) {
         float acc = 0.f;
         uint32_t p = 0;
         if (d == d0) { acc = acc0; p = partitions < uint32_t(AHEAD) ? partitions : uint32_t(AHEAD); }
@@ -498,7 +497,7 @@ attn_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ 
     if (out_sums) {
         lds_barrier();
         // receipt of the attention output row [q_heads*hd], the o-projection's input
-        emit_receipt(rowbuf, (rh % q_heads) * hd, hd, rh / q_heads, gridDim.x / q_heads, q_heads * hd, out_sums);
+        emit_receipt(rowbuf, (rh % q_heads) * hd, hd, rh / q_heads, rows, q_heads * hd, out_sums, threadIdx.x, 256);
     }
 }
 
@@ -633,11 +632,11 @@ int attention_decode(void* stream, const float* q, const FusedInputs* fused, con
     if (rc) return rc;
     // the outputs requested ahead: 32 when the partitions are that few (a local layer), else 64
     if (a.partitions <= 32)
-        launch(attn_merge_kernel<32>, dim3(rows * q_heads), dim3(256), 2 * 32 * sizeof(float), s, partial_out, partial_ml, out,
-                           out_sums, a.partitions, head_dim, q_heads, status);
+        launch(attn_merge_kernel<32>, dim3(rows * q_heads), dim3(256), 2 * 32 * sizeof(float), s, partial_out, partial_ml, a.partitions,
+               head_dim, q_heads, rows, out, out_sums, status);
     else
-        launch(attn_merge_kernel<kMergeAhead>, dim3(rows * q_heads), dim3(256), 2 * std::max<uint32_t>(a.partitions, kMergeAhead) * sizeof(float), s, partial_out, partial_ml, out,
-                           out_sums, a.partitions, head_dim, q_heads, status);
+        launch(attn_merge_kernel<kMergeAhead>, dim3(rows * q_heads), dim3(256), 2 * std::max<uint32_t>(a.partitions, kMergeAhead) * sizeof(float), s, partial_out, partial_ml, a.partitions,
+               head_dim, q_heads, rows, out, out_sums, status);
     return check_launch("attention_merge");
 }
 }  // namespace

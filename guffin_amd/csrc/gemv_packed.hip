@@ -196,7 +196,10 @@ __global__ void reduce_partials_kernel(const float* __restrict__ part, float* __
 
 // Workgroup = W waves over consecutive k-slices of one column tile; the W per-lane sums are
 // combined through LDS in wave order and written as one plane.  grid = (tiles, planes).
-struct PackedCfg { uint32_t K, nblk, bps, W; };
+// The arguments of these kernels lie as they do because the first fourteen words of a launch's arguments are in registers
+// when a wave starts (a build flag), if nothing but words and pointers stands among them: what the first requests need goes
+// first, as words of its own, and what only the stores need goes last.  Behind a struct they were a trip to memory ahead of
+// every first request.
 
 template <int R>
 __device__ __forceinline__ void finish_tile(float (&acc)[R], float* __restrict__ part, uint32_t N, uint32_t ct,
@@ -225,55 +228,53 @@ constexpr int kMixed = 3;  // Q4_K and Q6_K matrices in one launch
 
 template <int DTYPE, int R>
 __global__ void __launch_bounds__(64 * max_waves(DTYPE))
-gemv_packed_kernel(const uint8_t* __restrict__ wt, const float* __restrict__ x, const float* __restrict__ xsums,
-                   float* __restrict__ part, uint32_t N, PackedCfg c) {
-    const uint32_t slice = blockIdx.y * c.W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t b0 = min(slice * c.bps, c.nblk), b1 = min(b0 + c.bps, c.nblk);
+gemv_packed_kernel(const uint8_t* __restrict__ wt, const float* __restrict__ xsums, uint32_t K, uint32_t bps, uint32_t W, uint32_t N,
+                   float* __restrict__ part) {
+    const uint32_t slice = blockIdx.y * W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nblk = K / block_elems(DTYPE);
+    const uint32_t b0 = min(slice * bps, nblk), b1 = min(b0 + bps, nblk);
     float acc[R];
-    run_blocks<DTYPE, R>(wt, x, xsums, c.K, c.nblk, blockIdx.x, b0, b1, acc);
-    finish_tile<R>(acc, part, N, blockIdx.x, blockIdx.y, c.W);
+    run_blocks<DTYPE, R>(wt, xsums, K, nblk, blockIdx.x, b0, b1, acc);
+    finish_tile<R>(acc, part, N, blockIdx.x, blockIdx.y, W);
 }
 
 // Q6_K with one block per wave and 16 waves per workgroup (shapes whose split leaves every wave a single block)
 template <int R>
 __global__ void __launch_bounds__(1024)
-gemv_q6k_single_kernel(const uint8_t* __restrict__ wt, const float* __restrict__ x, const float* __restrict__ xsums,
-                       float* __restrict__ part, uint32_t N, PackedCfg c) {
-    const uint32_t slice = blockIdx.y * c.W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t b0 = min(slice, c.nblk), b1 = min(b0 + 1u, c.nblk);
+gemv_q6k_single_kernel(const uint8_t* __restrict__ wt, const float* __restrict__ xsums, uint32_t K, uint32_t W, uint32_t N,
+                       float* __restrict__ part) {
+    const uint32_t slice = blockIdx.y * W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nblk = K / block_elems(GUFFIN_Q6_K);
+    const uint32_t b0 = min(slice, nblk), b1 = min(b0 + 1u, nblk);
     float acc[R];
-    run_blocks<GUFFIN_Q6_K, R, kWalkOne>(wt, x, xsums, c.K, c.nblk, blockIdx.x, b0, b1, acc);
-    finish_tile<R>(acc, part, N, blockIdx.x, blockIdx.y, c.W);
+    run_blocks<GUFFIN_Q6_K, R, kWalkOne>(wt, xsums, K, nblk, blockIdx.x, b0, b1, acc);
+    finish_tile<R>(acc, part, N, blockIdx.x, blockIdx.y, W);
 }
 
 // Several matrices that share the activation rows (q/k/v, gate/up) in one launch: the column
 // tiles of all matrices sit side by side along grid x.  COUNT also names the instantiation
-// so that profiles tell q/k/v (3) from gate/up (2).
-struct MultiMeta { uint32_t N[3], dtype[3], tile_end[3]; };
-
+// so that profiles tell q/k/v (3) from gate/up (2).  end0, end1: the tiles of the first matrix, of the first two; dtypes: a byte each.
 template <int R, int COUNT, int MODE>
 __global__ void __launch_bounds__(64 * max_waves(MODE == kMixed ? GUFFIN_Q6_K : MODE))
 gemv_packed_multi_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2,
-                         float* __restrict__ p0, float* __restrict__ p1, float* __restrict__ p2,
-                         const float* __restrict__ x, const float* __restrict__ xsums, MultiMeta m, PackedCfg c) {
+                         const float* __restrict__ xsums, uint32_t end0, uint32_t end1, uint32_t dtypes, uint32_t K, uint32_t bps, uint32_t W,
+                         uint32_t n0, uint32_t n1, uint32_t n2, float* __restrict__ p0, float* __restrict__ p1, float* __restrict__ p2) {
     uint32_t which = 0;
-    if (COUNT > 1 && blockIdx.x >= m.tile_end[0]) which = 1;
-    if (COUNT > 2 && blockIdx.x >= m.tile_end[1]) which = 2;
-    const uint32_t first = which == 0 ? 0 : m.tile_end[which - 1];
+    if (COUNT > 1 && blockIdx.x >= end0) which = 1;
+    if (COUNT > 2 && blockIdx.x >= end1) which = 2;
+    const uint32_t first = which == 0 ? 0 : which == 1 ? end0 : end1;
     const uint8_t* __restrict__ wt = which == 0 ? t0 : which == 1 ? t1 : t2;
     float* __restrict__ part = which == 0 ? p0 : which == 1 ? p1 : p2;
-    const uint32_t ct = blockIdx.x - first, N = m.N[which];
-    [[maybe_unused]] const uint32_t dtype = m.dtype[which];
-    const uint32_t slice = blockIdx.y * c.W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t b0 = min(slice * c.bps, c.nblk), b1 = min(b0 + c.bps, c.nblk);
+    const uint32_t ct = blockIdx.x - first, N = which == 0 ? n0 : which == 1 ? n1 : n2;
+    [[maybe_unused]] const uint32_t dtype = (dtypes >> (8 * which)) & 0xFFu;
+    const uint32_t slice = blockIdx.y * W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t nblk = K / block_elems(MODE == kMixed ? GUFFIN_Q4_K : MODE), b0 = min(slice * bps, nblk), b1 = min(b0 + bps, nblk);
     float acc[R];
     if constexpr (MODE == kMixed) {
-        if (dtype == GUFFIN_Q4_K) run_blocks<GUFFIN_Q4_K, R>(wt, x, xsums, c.K, c.nblk, ct, b0, b1, acc);
-        else run_blocks<GUFFIN_Q6_K, R>(wt, x, xsums, c.K, c.nblk, ct, b0, b1, acc);
+        if (dtype == GUFFIN_Q4_K) run_blocks<GUFFIN_Q4_K, R>(wt, xsums, K, nblk, ct, b0, b1, acc);
+        else run_blocks<GUFFIN_Q6_K, R>(wt, xsums, K, nblk, ct, b0, b1, acc);
     } else {
-        run_blocks<MODE, R>(wt, x, xsums, c.K, c.nblk, ct, b0, b1, acc);
+        run_blocks<MODE, R>(wt, xsums, K, nblk, ct, b0, b1, acc);
     }
-    finish_tile<R>(acc, part, N, ct, blockIdx.y, c.W);
+    finish_tile<R>(acc, part, N, ct, blockIdx.y, W);
 }
 
 // gate and up projections of one column tile in one workgroup (waves [0, W) gate, [W, 2W) up,
@@ -282,23 +283,24 @@ gemv_packed_multi_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restri
 template <int DTYPE, int R>
 __global__ void __launch_bounds__(1024)
 gateup_geglu_kernel(const uint8_t* __restrict__ gate_tiles, const uint8_t* __restrict__ up_tiles,
-                    const float* __restrict__ x, const float* __restrict__ xsums, float* __restrict__ h,
-                    void* __restrict__ h_receipt, uint32_t F, PackedCfg c) {
+                    const float* __restrict__ xsums, uint32_t K, uint32_t bps, uint32_t W, uint32_t F, float* __restrict__ h,
+                    void* __restrict__ h_receipt) {
     __shared__ float red[16 * 2 * 64];
     __shared__ float vals[2 * 64];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const bool is_up = wave >= c.W;
-    const uint32_t slice = is_up ? wave - c.W : wave;
-    const uint32_t b0 = min(slice * c.bps, c.nblk), b1 = min(b0 + c.bps, c.nblk);
+    const uint32_t nblk = K / block_elems(DTYPE);
+    const bool is_up = wave >= W;
+    const uint32_t slice = is_up ? wave - W : wave;
+    const uint32_t b0 = min(slice * bps, nblk), b1 = min(b0 + bps, nblk);
     float acc[R];
-    run_blocks<DTYPE, R>(is_up ? up_tiles : gate_tiles, x, xsums, c.K, c.nblk, blockIdx.x, b0, b1, acc);
+    run_blocks<DTYPE, R>(is_up ? up_tiles : gate_tiles, xsums, K, nblk, blockIdx.x, b0, b1, acc);
 #pragma unroll
     for (int r = 0; r < R; ++r) red[(wave * R + r) * 64 + lane] = acc[r];
     __syncthreads();
     if (threadIdx.x < R * 64) {
         const uint32_t r = threadIdx.x >> 6;
-        float g = red[r * 64 + lane], u = red[(c.W * R + r) * 64 + lane];
-        for (uint32_t w = 1; w < c.W; ++w) { g += red[(w * R + r) * 64 + lane]; u += red[((c.W + w) * R + r) * 64 + lane]; }
+        float g = red[r * 64 + lane], u = red[(W * R + r) * 64 + lane];
+        for (uint32_t w = 1; w < W; ++w) { g += red[(w * R + r) * 64 + lane]; u += red[((W + w) * R + r) * 64 + lane]; }
         const float v = geglu_value(g, u);
         h[size_t(r) * F + blockIdx.x * kTileCols + lane] = v;
         vals[r * 64 + lane] = v;
@@ -352,22 +354,21 @@ PackedPlan packed_plan(int dtype, uint32_t nblk, uint32_t tiles) {
 }
 
 template <int DTYPE>
-int launch_packed(hipStream_t s, const uint8_t* w, const float* x, const float* xsums, float* part,
+int launch_packed(hipStream_t s, const uint8_t* w, const float* xsums, float* part,
                   uint32_t rows, uint32_t K, uint32_t N) {
     const uint32_t nblk = K / block_elems(DTYPE);
     const PackedPlan plan = packed_plan(DTYPE, nblk, N / kTileCols);
     const Split sp = plan.sp;
-    const PackedCfg c {K, nblk, sp.bps, sp.W};
     const dim3 grid(N / kTileCols, sp.planes), block(sp.W * 64);
     if constexpr (DTYPE == GUFFIN_Q6_K) {
         if (plan.single) {
-            if (rows == 2) launch((gemv_q6k_single_kernel<2>), grid, block, 0, s, w, x, xsums, part, N, c);
-            else launch((gemv_q6k_single_kernel<1>), grid, block, 0, s, w, x, xsums, part, N, c);
+            if (rows == 2) launch((gemv_q6k_single_kernel<2>), grid, block, 0, s, w, xsums, K, sp.W, N, part);
+            else launch((gemv_q6k_single_kernel<1>), grid, block, 0, s, w, xsums, K, sp.W, N, part);
             return check_launch("gemv_packed");
         }
     }
-    if (rows == 2) launch((gemv_packed_kernel<DTYPE, 2>), grid, block, 0, s, w, x, xsums, part, N, c);
-    else launch((gemv_packed_kernel<DTYPE, 1>), grid, block, 0, s, w, x, xsums, part, N, c);
+    if (rows == 2) launch((gemv_packed_kernel<DTYPE, 2>), grid, block, 0, s, w, xsums, K, sp.bps, sp.W, N, part);
+    else launch((gemv_packed_kernel<DTYPE, 1>), grid, block, 0, s, w, xsums, K, sp.bps, sp.W, N, part);
     return check_launch("gemv_packed");
 }
 
@@ -492,7 +493,7 @@ extern "C" int guffin_hip_gemv_packed_multi(void* stream, uint32_t count, const 
         if (!tiles[0] || !partials[0]) return fail(GUFFIN_E_ARG, "gemv_packed_multi: null pointer");
         return guffin_hip_gemv_packed(stream, dtypes[0], tiles[0], x, xsums, partials[0], nullptr, rows, K, N[0]);
     }
-    MultiMeta m {};
+    uint32_t n[3] = {N[0], N[0], N[0]}, ends[2] = {0, 0}, formats = 0;
     const uint8_t* t[3] = {nullptr, nullptr, nullptr};
     float* p[3] = {nullptr, nullptr, nullptr};
     uint32_t tile_end = 0;
@@ -500,14 +501,16 @@ extern "C" int guffin_hip_gemv_packed_multi(void* stream, uint32_t count, const 
         if (!tiles[i] || !partials[i]) return fail(GUFFIN_E_ARG, "gemv_packed_multi: null pointer");
         if (reinterpret_cast<uintptr_t>(tiles[i]) & 15u) return fail(GUFFIN_E_ALIGN, "gemv_packed_multi: tiles must be 16-byte aligned");
         tile_end += N[i] / kTileCols;
-        m.N[i] = N[i]; m.dtype[i] = static_cast<uint32_t>(dtypes[i]); m.tile_end[i] = tile_end;
+        n[i] = N[i];
+        formats |= static_cast<uint32_t>(dtypes[i]) << (8 * i);
+        if (i < 2) ends[i] = tile_end;
         t[i] = static_cast<const uint8_t*>(tiles[i]); p[i] = partials[i];
     }
-    for (uint32_t i = count; i < 3; ++i) { t[i] = t[0]; p[i] = p[0]; m.tile_end[i] = tile_end; m.N[i] = m.N[0]; m.dtype[i] = m.dtype[0]; }
-    const PackedCfg c {K, K / block_elems(dtypes[0]), sp.bps, sp.W};
+    for (uint32_t i = count; i < 3; ++i) { t[i] = t[0]; p[i] = p[0]; }
     const dim3 grid(tile_end, sp.planes), block(sp.W * 64);
     hipStream_t s = as_stream(stream);
-#define GUFFIN_MULTI(R_, C_, M_) launch((gemv_packed_multi_kernel<R_, C_, M_>), grid, block, 0, s, t[0], t[1], t[2], p[0], p[1], p[2], x, xsums, m, c)
+#define GUFFIN_MULTI(R_, C_, M_) launch((gemv_packed_multi_kernel<R_, C_, M_>), grid, block, 0, s, t[0], t[1], t[2], xsums, ends[0], ends[1], formats, K, sp.bps, sp.W, \
+                                        n[0], n[1], n[2], p[0], p[1], p[2])
 #define GUFFIN_MULTI_MODE(R_, C_) do { \
         if (mode == GUFFIN_Q4_K) GUFFIN_MULTI(R_, C_, GUFFIN_Q4_K); else if (mode == GUFFIN_Q6_K) GUFFIN_MULTI(R_, C_, GUFFIN_Q6_K); \
         else if (mode == GUFFIN_Q8_0) GUFFIN_MULTI(R_, C_, GUFFIN_Q8_0); else GUFFIN_MULTI(R_, C_, kMixed); } while (0)
@@ -534,12 +537,11 @@ extern "C" int guffin_hip_gateup_geglu(void* stream, int dtype, const void* gate
         sp.bps = (nblk + 7) / 8;
         sp.W = (nblk + sp.bps - 1) / sp.bps;
     }
-    const PackedCfg c {K, nblk, sp.bps, sp.W};
     const dim3 grid(tiles), block(2 * sp.W * 64);
     hipStream_t s = as_stream(stream);
     const uint8_t* g = static_cast<const uint8_t*>(gate_tiles);
     const uint8_t* u = static_cast<const uint8_t*>(up_tiles);
-#define GUFFIN_GU(D_, R_) launch((gateup_geglu_kernel<D_, R_>), grid, block, 0, s, g, u, x, xsums, h, h_sums, F, c)
+#define GUFFIN_GU(D_, R_) launch((gateup_geglu_kernel<D_, R_>), grid, block, 0, s, g, u, xsums, K, sp.bps, sp.W, F, h, h_sums)
     if (dtype == GUFFIN_Q4_K) { if (rows == 2) GUFFIN_GU(GUFFIN_Q4_K, 2); else GUFFIN_GU(GUFFIN_Q4_K, 1); }
     else { if (rows == 2) GUFFIN_GU(GUFFIN_Q8_0, 2); else GUFFIN_GU(GUFFIN_Q8_0, 1); }
 #undef GUFFIN_GU
@@ -559,9 +561,9 @@ extern "C" int guffin_hip_gemv_packed(void* stream, int dtype, const void* tiles
     hipStream_t s = as_stream(stream);
     float* out = (y && S == 1) ? y : partials;  // a single plane is the result: no second launch
     int rc;
-    if (dtype == GUFFIN_Q4_K) rc = launch_packed<GUFFIN_Q4_K>(s, w, x, xsums, out, rows, K, N);
-    else if (dtype == GUFFIN_Q6_K) rc = launch_packed<GUFFIN_Q6_K>(s, w, x, xsums, out, rows, K, N);
-    else rc = launch_packed<GUFFIN_Q8_0>(s, w, x, xsums, out, rows, K, N);
+    if (dtype == GUFFIN_Q4_K) rc = launch_packed<GUFFIN_Q4_K>(s, w, xsums, out, rows, K, N);
+    else if (dtype == GUFFIN_Q6_K) rc = launch_packed<GUFFIN_Q6_K>(s, w, xsums, out, rows, K, N);
+    else rc = launch_packed<GUFFIN_Q8_0>(s, w, xsums, out, rows, K, N);
     if (rc || !y || S == 1) return rc;
     const uint32_t count = rows * N;
     launch(reduce_partials_kernel, dim3((count + 255) / 256), dim3(256), 0, s, partials, y, S, count);

@@ -416,8 +416,7 @@ __device__ __forceinline__ void run_blocks_ahead(const Q8Ahead& ahead, const uin
 
 // One wave: blocks [b0, b1) of column tile `ct` of a whole matrix whose operand is the receipt of its K inputs.
 template <int DTYPE, int R, int WALK = kWalkAhead>
-__device__ __forceinline__ void run_blocks(const uint8_t* __restrict__ wt, const float* __restrict__ x,
-                                           const float* __restrict__ xsums, uint32_t K, uint32_t nblk,
+__device__ __forceinline__ void run_blocks(const uint8_t* __restrict__ wt, const float* __restrict__ xsums, uint32_t K, uint32_t nblk,
                                            uint32_t ct, uint32_t b0, uint32_t b1, float (&acc)[R]) {
     constexpr uint32_t TB = kTileCols * block_bytes(DTYPE);
     run_blocks_at<DTYPE, R, WALK>(wt + (size_t(ct) * nblk + b0) * TB, xsums, K, b0, b1 > b0 ? b1 - b0 : 0u, acc);

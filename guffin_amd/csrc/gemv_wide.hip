@@ -59,7 +59,7 @@ __device__ __forceinline__ void run_wide(const uint8_t* __restrict__ wt, const f
     constexpr uint32_t TB = kTileCols * block_bytes(DTYPE);
     if constexpr (DTYPE != GUFFIN_Q8_0) {
         float acc[kWideRows];
-        run_blocks<DTYPE, kWideRows, WALK>(wt, nullptr, xsums, K, nblk, ct, b0, b1, acc);
+        run_blocks<DTYPE, kWideRows, WALK>(wt, xsums, K, nblk, ct, b0, b1, acc);
 #pragma unroll
         for (uint32_t r = 0; r < kWideRows; ++r) red[r * 64 + lane] = acc[r];
     } else {
@@ -87,34 +87,34 @@ __device__ __forceinline__ void run_wide(const uint8_t* __restrict__ wt, const f
     }
 }
 
-struct WideCfg { uint32_t K, nblk, bps, W, rows; };
-struct WideMeta { const uint8_t* tiles[3]; float* part[3]; uint32_t N[3], dtype[3], tile_end[3]; };
-
-// Up to three matrices of the same rows, their column tiles side by side along grid x; grid y: planes.
+// Up to three matrices of the same rows, their column tiles side by side along grid x; grid y: planes.  (The arguments' order: as
+// for the kernels of gemv_packed.hip.)  end0, end1: the tiles of the first matrix, of the first two; dtypes: a byte each.
 template <int MODE, uint32_t WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
-gemv_wide_kernel(const float* __restrict__ xsums, const WideMeta m, const WideCfg c) {
+gemv_wide_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const float* __restrict__ xsums,
+                 uint32_t end0, uint32_t end1, uint32_t dtypes, uint32_t K, uint32_t bps, uint32_t W, uint32_t rows, uint32_t n0, uint32_t n1,
+                 uint32_t n2, float* __restrict__ p0, float* __restrict__ p1, float* __restrict__ p2) {
     __shared__ float red[WAVES * kWideRows * 64];
-    const uint32_t which = blockIdx.x >= m.tile_end[1] ? 2u : blockIdx.x >= m.tile_end[0] ? 1u : 0u;
-    const uint8_t* wt = which == 0 ? m.tiles[0] : which == 1 ? m.tiles[1] : m.tiles[2];
-    float* part = which == 0 ? m.part[0] : which == 1 ? m.part[1] : m.part[2];
-    const uint32_t N = which == 0 ? m.N[0] : which == 1 ? m.N[1] : m.N[2];
-    [[maybe_unused]] const uint32_t dtype = which == 0 ? m.dtype[0] : which == 1 ? m.dtype[1] : m.dtype[2];
-    const uint32_t ct = blockIdx.x - (which == 0 ? 0u : which == 1 ? m.tile_end[0] : m.tile_end[1]);
+    const uint32_t which = blockIdx.x >= end1 ? 2u : blockIdx.x >= end0 ? 1u : 0u;
+    const uint8_t* wt = which == 0 ? t0 : which == 1 ? t1 : t2;
+    float* part = which == 0 ? p0 : which == 1 ? p1 : p2;
+    const uint32_t N = which == 0 ? n0 : which == 1 ? n1 : n2, nblk = K / block_elems(MODE == kWideMixed ? GUFFIN_Q4_K : MODE);
+    [[maybe_unused]] const uint32_t dtype = (dtypes >> (8 * which)) & 0xFFu;
+    const uint32_t ct = blockIdx.x - (which == 0 ? 0u : which == 1 ? end0 : end1);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const uint32_t slice = blockIdx.y * c.W + wave, b0 = min(slice * c.bps, c.nblk), b1 = min(b0 + c.bps, c.nblk);
+    const uint32_t slice = blockIdx.y * W + wave, b0 = min(slice * bps, nblk), b1 = min(b0 + bps, nblk);
     float* own = red + wave * kWideRows * 64;
     if constexpr (MODE == kWideMixed) {
-        if (dtype == GUFFIN_Q4_K) run_wide<GUFFIN_Q4_K, (WAVES > kWideWaves ? kWalkOne : kWalkAhead)>(wt, xsums, c.K, c.nblk, ct, b0, b1, own, lane);
-        else run_wide<GUFFIN_Q6_K, (WAVES > kWideWaves ? kWalkOne : kWalkAhead)>(wt, xsums, c.K, c.nblk, ct, b0, b1, own, lane);
+        if (dtype == GUFFIN_Q4_K) run_wide<GUFFIN_Q4_K, (WAVES > kWideWaves ? kWalkOne : kWalkAhead)>(wt, xsums, K, nblk, ct, b0, b1, own, lane);
+        else run_wide<GUFFIN_Q6_K, (WAVES > kWideWaves ? kWalkOne : kWalkAhead)>(wt, xsums, K, nblk, ct, b0, b1, own, lane);
     } else {
-        run_wide<MODE, (WAVES > kWideWaves ? kWalkOne : kWalkAhead)>(wt, xsums, c.K, c.nblk, ct, b0, b1, own, lane);
+        run_wide<MODE, (WAVES > kWideWaves ? kWalkOne : kWalkAhead)>(wt, xsums, K, nblk, ct, b0, b1, own, lane);
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < c.rows * 64; i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < rows * 64; i += 64 * W) {
         float t = red[i];
-        for (uint32_t w = 1; w < c.W; ++w) t += red[w * kWideRows * 64 + i];
-        part[(size_t(blockIdx.y) * c.rows + (i >> 6)) * N + ct * kTileCols + (i & 63u)] = t;
+        for (uint32_t w = 1; w < W; ++w) t += red[w * kWideRows * 64 + i];
+        part[(size_t(blockIdx.y) * rows + (i >> 6)) * N + ct * kTileCols + (i & 63u)] = t;
     }
 }
 
@@ -122,23 +122,25 @@ gemv_wide_kernel(const float* __restrict__ xsums, const WideMeta m, const WideCf
 template <int DTYPE>
 __global__ void __launch_bounds__(64 * kWideWaves)
 gateup_wide_kernel(const uint8_t* __restrict__ gate_tiles, const uint8_t* __restrict__ up_tiles, const float* __restrict__ xsums,
-                   float* __restrict__ h, void* __restrict__ h_receipt, uint32_t F, const WideCfg c) {
+                   uint32_t K, uint32_t bps, uint32_t W, uint32_t F, uint32_t rows, float* __restrict__ h,
+                   void* __restrict__ h_receipt) {
     __shared__ float red[kWideWaves * kWideRows * 64];
     __shared__ float vals[kWideRows * 64];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const bool is_up = wave >= c.W;
-    const uint32_t slice = is_up ? wave - c.W : wave, b0 = min(slice * c.bps, c.nblk), b1 = min(b0 + c.bps, c.nblk);
-    run_wide<DTYPE>(is_up ? up_tiles : gate_tiles, xsums, c.K, c.nblk, blockIdx.x, b0, b1, red + wave * kWideRows * 64, lane);
+    const uint32_t nblk = K / block_elems(DTYPE);
+    const bool is_up = wave >= W;
+    const uint32_t slice = is_up ? wave - W : wave, b0 = min(slice * bps, nblk), b1 = min(b0 + bps, nblk);
+    run_wide<DTYPE>(is_up ? up_tiles : gate_tiles, xsums, K, nblk, blockIdx.x, b0, b1, red + wave * kWideRows * 64, lane);
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < c.rows * 64; i += blockDim.x) {
-        float g = red[i], u = red[c.W * kWideRows * 64 + i];
-        for (uint32_t w = 1; w < c.W; ++w) { g += red[w * kWideRows * 64 + i]; u += red[(c.W + w) * kWideRows * 64 + i]; }
+    for (uint32_t i = threadIdx.x; i < rows * 64; i += 128 * W) {
+        float g = red[i], u = red[W * kWideRows * 64 + i];
+        for (uint32_t w = 1; w < W; ++w) { g += red[w * kWideRows * 64 + i]; u += red[(W + w) * kWideRows * 64 + i]; }
         const float v = geglu_value(g, u);
         h[size_t(i >> 6) * F + blockIdx.x * kTileCols + (i & 63u)] = v;
         vals[i] = v;
     }
     lds_barrier();   // h is on its way out and nobody here reads it
-    if (wave < c.rows) emit_receipt(vals + wave * 64, blockIdx.x * kTileCols, kTileCols, wave, c.rows, F, h_receipt, lane, 64);
+    if (wave < rows) emit_receipt(vals + wave * 64, blockIdx.x * kTileCols, kTileCols, wave, rows, F, h_receipt, lane, 64);
 }
 
 __global__ void wide_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, uint32_t planes, uint32_t count) {
@@ -178,28 +180,30 @@ int gemv_wide(hipStream_t s, uint32_t count, const int* dtypes, const void* cons
     GemvSplit sp {};
     int mode = 0;
     if (int rc = wide_split(count, dtypes, N, K, &sp, &mode)) return rc;
-    WideMeta m {};
-    uint32_t end = 0;
+    const uint8_t* t[3];
+    float* p[3];
+    uint32_t n[3], ends[3], end = 0, formats = 0;
     for (uint32_t i = 0; i < 3; ++i) {
         const uint32_t k = i < count ? i : 0;
         if (i < count) end += N[i] / kTileCols;
-        m.tiles[i] = static_cast<const uint8_t*>(tiles[k]); m.part[i] = partials[k]; m.N[i] = N[k];
-        m.dtype[i] = static_cast<uint32_t>(dtypes[k]); m.tile_end[i] = end;
+        t[i] = static_cast<const uint8_t*>(tiles[k]); p[i] = partials[k]; n[i] = N[k]; ends[i] = end;
+        formats |= static_cast<uint32_t>(dtypes[k]) << (8 * i);
     }
-    if (y && sp.planes == 1) m.part[0] = y;   // one plane is the result
-    const WideCfg c {K, K / block_elems(dtypes[0]), sp.bps, sp.W, rows};
+    if (y && sp.planes == 1) p[0] = y;   // one plane is the result
     const dim3 grid(end, sp.planes), block(64 * sp.W);
-#define GUFFIN_WIDE(M_) do { if (sp.bps == 1) launch((gemv_wide_kernel<M_, 16>), grid, block, 0, s, xsums, m, c); \
-        else launch((gemv_wide_kernel<M_, kWideWaves>), grid, block, 0, s, xsums, m, c); } while (0)
+#define GUFFIN_WIDE(M_) do { if (sp.bps == 1) launch((gemv_wide_kernel<M_, 16>), grid, block, 0, s, GUFFIN_WIDE_ARGS); \
+        else launch((gemv_wide_kernel<M_, kWideWaves>), grid, block, 0, s, GUFFIN_WIDE_ARGS); } while (0)
+#define GUFFIN_WIDE_ARGS t[0], t[1], t[2], xsums, ends[0], ends[1], formats, K, sp.bps, sp.W, rows, n[0], n[1], n[2], p[0], p[1], p[2]
     if (mode == GUFFIN_Q4_K) GUFFIN_WIDE(GUFFIN_Q4_K);
     else if (mode == GUFFIN_Q6_K) GUFFIN_WIDE(GUFFIN_Q6_K);
     else if (mode == GUFFIN_Q8_0) GUFFIN_WIDE(GUFFIN_Q8_0);
     else GUFFIN_WIDE(kWideMixed);
+#undef GUFFIN_WIDE_ARGS
 #undef GUFFIN_WIDE
     if (int rc = check_launch("gemv_wide")) return rc;
     if (!y || sp.planes == 1) return GUFFIN_OK;
-    const uint32_t n = rows * N[0];
-    launch(wide_reduce_kernel, dim3((n + 255) / 256), dim3(256), 0, s, partials[0], y, sp.planes, n);
+    const uint32_t elements = rows * N[0];
+    launch(wide_reduce_kernel, dim3((elements + 255) / 256), dim3(256), 0, s, partials[0], y, sp.planes, elements);
     return check_launch("gemv_wide_reduce");
 }
 
@@ -213,11 +217,10 @@ int gateup_wide(hipStream_t s, int dtype, const void* gate_tiles, const void* up
         sp.bps = (nblk + kWideWaves / 2 - 1) / (kWideWaves / 2);
         sp.W = (nblk + sp.bps - 1) / sp.bps;
     }
-    const WideCfg c {K, nblk, sp.bps, sp.W, rows};
     const dim3 grid(F / kTileCols), block(2 * sp.W * 64);
     const uint8_t *g = static_cast<const uint8_t*>(gate_tiles), *u = static_cast<const uint8_t*>(up_tiles);
-    if (dtype == GUFFIN_Q4_K) launch(gateup_wide_kernel<GUFFIN_Q4_K>, grid, block, 0, s, g, u, xsums, h, static_cast<void*>(h_sums), F, c);
-    else launch(gateup_wide_kernel<GUFFIN_Q8_0>, grid, block, 0, s, g, u, xsums, h, static_cast<void*>(h_sums), F, c);
+    if (dtype == GUFFIN_Q4_K) launch(gateup_wide_kernel<GUFFIN_Q4_K>, grid, block, 0, s, g, u, xsums, K, sp.bps, sp.W, F, rows, h, static_cast<void*>(h_sums));
+    else launch(gateup_wide_kernel<GUFFIN_Q8_0>, grid, block, 0, s, g, u, xsums, K, sp.bps, sp.W, F, rows, h, static_cast<void*>(h_sums));
     return check_launch("gateup_wide");
 }
 

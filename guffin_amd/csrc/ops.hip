@@ -188,11 +188,10 @@ __device__ __forceinline__ float4 ld4(const float* p, bool on) {
 __device__ __forceinline__ void unpack4(const float4& a, float* o) { o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; }
 
 __global__ void __launch_bounds__(1024)
-rms_norm_add_norm_regs_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_stride,
-                              const float* __restrict__ gamma_post, const float* __restrict__ residual,
-                              float* __restrict__ out_residual, const float* __restrict__ gamma_next,
-                              float* __restrict__ out_norm, float* __restrict__ out_sums, uint32_t width,
-                              float eps, uint32_t* __restrict__ status) {
+rms_norm_add_norm_regs_kernel(const float* __restrict__ x, const float* __restrict__ residual, const float* __restrict__ gamma_post,
+                              const float* __restrict__ gamma_next, size_t plane_stride, uint32_t planes, uint32_t width,
+                              float eps, uint32_t rows, float* __restrict__ out_residual,
+                              float* __restrict__ out_norm, float* __restrict__ out_sums, uint32_t* __restrict__ status) {
     __shared__ float scratch[2][16];   // the waves' sums: of the first norm, of the second
     const uint32_t r = blockIdx.x, item = threadIdx.x;
     const bool active = item < width / 8;
@@ -201,7 +200,7 @@ rms_norm_add_norm_regs_kernel(const float* __restrict__ x, uint32_t planes, size
         if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = own;
         lds_barrier();
         float t = 0.f;
-        for (uint32_t i = 0; i < blockDim.x >> 6; ++i) t += sums[i];  // same order on every thread
+        for (uint32_t i = 0; i < (width + 511) / 512; ++i) t += sums[i];  // same order on every thread
         return t;
     };
     const size_t col = active ? item * 8u : 0u, at = size_t(r) * width + col;
@@ -251,7 +250,7 @@ rms_norm_add_norm_regs_kernel(const float* __restrict__ x, uint32_t planes, size
         *reinterpret_cast<float4*>(out_residual + at + 4) = make_float4(v[4], v[5], v[6], v[7]);
         *reinterpret_cast<float4*>(out_norm + at) = make_float4(y[0], y[1], y[2], y[3]);
         *reinterpret_cast<float4*>(out_norm + at + 4) = make_float4(y[4], y[5], y[6], y[7]);
-        if (out_sums) emit_receipt_values(y, 0, item, r, gridDim.x, width, out_sums);
+        if (out_sums) emit_receipt_values(y, 0, item, r, rows, width, out_sums);
     }
     if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
 }
@@ -494,9 +493,8 @@ extern "C" int guffin_hip_rms_norm_add_norm(void* stream, const float* x, uint32
     if (planes <= uint32_t(kFastPlanes) && width % 8 == 0 && width / 8 <= 1024 && (!out_sums || width % 32 == 0)
         && plane_stride % 4 == 0 && a16(x) && a16(gamma_post) && a16(residual) && a16(out_residual) && a16(gamma_next) && a16(out_norm)) {
         const uint32_t threads = (width / 8 + 63) / 64 * 64;
-        launch(rms_norm_add_norm_regs_kernel, dim3(rows), dim3(threads), 0, as_stream(stream), x, planes,
-                           static_cast<size_t>(plane_stride), gamma_post, residual, out_residual, gamma_next, out_norm,
-                           out_sums, width, eps, status);
+        launch(rms_norm_add_norm_regs_kernel, dim3(rows), dim3(threads), 0, as_stream(stream), x, residual, gamma_post, gamma_next,
+                           static_cast<size_t>(plane_stride), planes, width, eps, rows, out_residual, out_norm, out_sums, status);
         return check_launch("rms_norm_add_norm");
     }
     const size_t lds = (size_t(width) + 16) * 4;

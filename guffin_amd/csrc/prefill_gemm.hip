@@ -118,12 +118,24 @@ __device__ __forceinline__ uint2_t from_lds8(const uint8_t* at) { return *reinte
 template <int N>
 __device__ __forceinline__ void arrive() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
 
-struct GemmSegment { const uint8_t* tiles; float* y; uint64_t plane_stride; uint32_t N, dtype, first_group; };
+// What a launch brings.  A kernel takes it as words and pointers in this order: the first fourteen words of a launch's arguments
+// are in registers when a wave starts (a build flag), as long as no struct stands among them.
 struct GemmArgs {
-    GemmSegment seg[3];
-    uint32_t segments, M, K;
+    const uint8_t* tiles[3];
     const uint8_t* blob;
+    uint32_t M, K, columns[3];   // column tiles of 64 of each matrix, 0: no such matrix
+    uint32_t form;               // k-slices, and the matrices' formats in the upper bytes
+    float* y[3];
 };
+// the matrix of a workgroup and its first column tile there
+struct GemmSegment { const uint8_t* tiles; float* y; uint32_t columns, dtype, first; };
+__device__ __forceinline__ GemmSegment segment_of(uint32_t group, const uint8_t* t0, const uint8_t* t1, const uint8_t* t2, uint32_t n0, uint32_t n1,
+                                                  uint32_t n2, uint32_t form, float* y0, float* y1, float* y2) {
+    const uint32_t g1 = (n0 + 3) / 4, g2 = g1 + (n1 + 3) / 4;
+    if (group < g1) return {t0, y0, n0, (form >> 8) & 0xFFu, 4 * group};
+    if (group < g2) return {t1, y1, n1, (form >> 16) & 0xFFu, 4 * (group - g1)};
+    return {t2, y2, n2, form >> 24, 4 * (group - g2)};
+}
 
 // what the workgroup keeps in LDS, R row tiles of 16
 template <int R>
@@ -607,18 +619,18 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, const Feed<R>
 // rows, so that an XCD's L2 keeps its share of the image.
 template <int R, int KINDS>
 __global__ void __launch_bounds__(256, 2)
-prefill_gemm_kernel(GemmArgs A) {
+prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const uint8_t* __restrict__ blob,
+                    uint32_t M, uint32_t K, uint32_t n0, uint32_t n1, uint32_t n2, uint32_t form, float* __restrict__ y0,
+                    float* __restrict__ y1, float* __restrict__ y2) {
     __shared__ __attribute__((aligned(16))) uint8_t stage[Stage<R>::kBytes];
-    const ImageLayout L = image_layout(A.M, A.K);
+    const ImageLayout L = image_layout(M, K);
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint32_t s = 0;
-    while (s + 1 < A.segments && blockIdx.y >= A.seg[s + 1].first_group) ++s;
-    const GemmSegment seg = A.seg[s];
-    const uint32_t tile_index = (blockIdx.y - seg.first_group) * 4 + wv, nblk = A.K / 256, rt0 = blockIdx.x * R;
-    const bool valid = tile_index < seg.N / kCols;   // a wave past the last tile works on tile 0 and stores nothing
-    const uint32_t b0 = blockIdx.z * nblk / gridDim.z, b1 = (blockIdx.z + 1) * nblk / gridDim.z;
+    const GemmSegment seg = segment_of(blockIdx.y, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
+    const uint32_t tile_index = seg.first + wv, nblk = K / 256, rt0 = blockIdx.x * R, slices = form & 0xFFu;
+    const bool valid = tile_index < seg.columns;   // a wave past the last tile works on tile 0 and stores nothing
+    const uint32_t b0 = blockIdx.z * nblk / slices, b1 = (blockIdx.z + 1) * nblk / slices;
     Feed<R> feed;
-    feed.img = make_resource(A.blob, static_cast<uint32_t>(L.bytes));
+    feed.img = make_resource(blob, static_cast<uint32_t>(L.bytes));
     feed.stage = stage;
     feed.lane16 = lane_again() * 16;
     feed.group_stride = (L.mpad / 16) * 2048;
@@ -641,16 +653,17 @@ prefill_gemm_kernel(GemmArgs A) {
     // the chunks asked for past the end are still on their way into this workgroup's LDS
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!valid) return;
-    float* y = seg.y + blockIdx.z * seg.plane_stride;
+    const uint32_t N = seg.columns * kCols;
+    float* y = seg.y + blockIdx.z * (uint64_t(M) * N);
     const uint32_t at = lane_again(), col = tile_index * kCols + (at & 15), row0 = rt0 * 16 + 4 * (at >> 4);
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t row = row0 + 16 * r + i;
-            if (row < A.M)
+            if (row < M)
 #pragma unroll
-                for (int cg = 0; cg < 4; ++cg) y[size_t(row) * seg.N + col + 16 * cg] = acc[cg][r][i];
+                for (int cg = 0; cg < 4; ++cg) y[size_t(row) * N + col + 16 * cg] = acc[cg][r][i];
         }
 }
 
@@ -659,18 +672,18 @@ prefill_gemm_kernel(GemmArgs A) {
 // the two matrix instructions (hi, lo) of a tile.  grid as above, k-slices in chunks of two blocks.
 template <int R>
 __global__ void __launch_bounds__(256, 2)
-prefill_gemm_q8_kernel(GemmArgs A) {
+prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const uint8_t* __restrict__ blob,
+                    uint32_t M, uint32_t K, uint32_t n0, uint32_t n1, uint32_t n2, uint32_t form, float* __restrict__ y0,
+                    float* __restrict__ y1, float* __restrict__ y2) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q8_0), kSlot = Stage<R>::kChunk + 512;   // chunk, its two groups' multipliers
     __shared__ __attribute__((aligned(16))) uint8_t stage[3 * kSlot];
-    const ImageLayout L = image_layout(A.M, A.K);
+    const ImageLayout L = image_layout(M, K);
     const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, lg = lane >> 4;
-    uint32_t s = 0;
-    while (s + 1 < A.segments && blockIdx.y >= A.seg[s + 1].first_group) ++s;
-    const GemmSegment seg = A.seg[s];
-    const uint32_t tile_index = (blockIdx.y - seg.first_group) * 4 + wv, nblk = A.K / 32, rt0 = blockIdx.x * R;
-    const bool valid = tile_index < seg.N / kCols;
-    const uint32_t chunks = (nblk + 1) / 2, c0 = blockIdx.z * chunks / gridDim.z, c1 = (blockIdx.z + 1) * chunks / gridDim.z;
-    const __amdgpu_buffer_rsrc_t img = make_resource(A.blob, static_cast<uint32_t>(L.bytes));
+    const GemmSegment seg = segment_of(blockIdx.y, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
+    const uint32_t tile_index = seg.first + wv, nblk = K / 32, rt0 = blockIdx.x * R, slices = form & 0xFFu;
+    const bool valid = tile_index < seg.columns;
+    const uint32_t chunks = (nblk + 1) / 2, c0 = blockIdx.z * chunks / slices, c1 = (blockIdx.z + 1) * chunks / slices;
+    const __amdgpu_buffer_rsrc_t img = make_resource(blob, static_cast<uint32_t>(L.bytes));
     const __amdgpu_buffer_rsrc_t tile = make_resource(seg.tiles + size_t(valid ? tile_index : 0) * nblk * TB, nblk * TB);
     const uint32_t lane16 = lane * 16, group_stride = (L.mpad / 16) * 2048, shift = L.span == 256 ? 3 : 0;
     const uint32_t base = rt0 * 2048 + (wv & 1) * (1024 * R), mult_off = static_cast<uint32_t>(L.mult_off) + rt0 * 64;
@@ -754,36 +767,45 @@ prefill_gemm_q8_kernel(GemmArgs A) {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!valid) return;
-    float* y = seg.y + blockIdx.z * seg.plane_stride;
+    const uint32_t N = seg.columns * kCols;
+    float* y = seg.y + blockIdx.z * (uint64_t(M) * N);
     const uint32_t col = tile_index * kCols + j, row0 = rt0 * 16 + 4 * lg;
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t row = row0 + 16 * r + i;
-            if (row < A.M)
+            if (row < M)
 #pragma unroll
-                for (int cg = 0; cg < 4; ++cg) y[size_t(row) * seg.N + col + 16 * cg] = acc[cg][r][i];
+                for (int cg = 0; cg < 4; ++cg) y[size_t(row) * N + col + 16 * cg] = acc[cg][r][i];
         }
 }
 
-int gemm_launch(hipStream_t s, GemmArgs& a, uint32_t slices, uint32_t R) {
+int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M, uint32_t K,
+                uint32_t slices, uint32_t R) {
+    if (count > 3 || slices > 255) return fail(GUFFIN_E_SHAPE, "prefill_gemm: at most three matrices and 255 slices");
+    GemmArgs a {};
+    a.blob = image; a.M = M; a.K = K; a.form = slices;
     uint32_t groups = 0, kinds = 0;
-    for (uint32_t i = 0; i < a.segments; ++i) {
-        a.seg[i].first_group = groups;
-        groups += (a.seg[i].N / kCols + 3) / 4;
-        kinds |= a.seg[i].dtype == GUFFIN_Q4_K ? 1u : a.seg[i].dtype == GUFFIN_Q6_K ? 2u : 4u;
+    for (uint32_t i = 0; i < count; ++i) {
+        a.tiles[i] = static_cast<const uint8_t*>(m[i].tiles); a.y[i] = y[i];
+        a.columns[i] = m[i].N / kCols;
+        a.form |= static_cast<uint32_t>(m[i].dtype) << (8 * (i + 1));
+        groups += (a.columns[i] + 3) / 4;
+        kinds |= m[i].dtype == GUFFIN_Q4_K ? 1u : m[i].dtype == GUFFIN_Q6_K ? 2u : 4u;
     }
-    const dim3 grid((a.M + 16 * R - 1) / (16 * R), groups, slices), block(256);
+    const dim3 grid((M + 16 * R - 1) / (16 * R), groups, slices), block(256);
+#define GUFFIN_PG_ARGS a.tiles[0], a.tiles[1], a.tiles[2], a.blob, a.M, a.K, a.columns[0], a.columns[1], a.columns[2], a.form, a.y[0], a.y[1], a.y[2]
 #define GUFFIN_PG(R_) \
     do { \
-        if (kinds == 1) launch(prefill_gemm_kernel<R_, 1>, grid, block, 0, s, a); \
-        else if (kinds == 2) launch(prefill_gemm_kernel<R_, 2>, grid, block, 0, s, a); \
-        else if (kinds == 3) launch(prefill_gemm_kernel<R_, 3>, grid, block, 0, s, a); \
-        else launch(prefill_gemm_q8_kernel<R_>, grid, block, 0, s, a); \
+        if (kinds == 1) launch(prefill_gemm_kernel<R_, 1>, grid, block, 0, s, GUFFIN_PG_ARGS); \
+        else if (kinds == 2) launch(prefill_gemm_kernel<R_, 2>, grid, block, 0, s, GUFFIN_PG_ARGS); \
+        else if (kinds == 3) launch(prefill_gemm_kernel<R_, 3>, grid, block, 0, s, GUFFIN_PG_ARGS); \
+        else launch(prefill_gemm_q8_kernel<R_>, grid, block, 0, s, GUFFIN_PG_ARGS); \
     } while (0)
     if (R == 1) GUFFIN_PG(1); else if (R == 2) GUFFIN_PG(2); else if (R == 3) GUFFIN_PG(3); else GUFFIN_PG(4);
 #undef GUFFIN_PG
+#undef GUFFIN_PG_ARGS
     return check_launch("prefill_gemm");
 }
 
@@ -844,11 +866,7 @@ int prefill_gemm_planes(hipStream_t s, const PrefillMatrix* m, uint32_t count, c
             if (int rc = prefill_gemm_planes(s, m + i, 1, image, y + i, M, K, split)) return rc;
         return GUFFIN_OK;
     }
-    GemmArgs a {};
-    for (uint32_t i = 0; i < count; ++i)
-        a.seg[i] = {static_cast<const uint8_t*>(m[i].tiles), y[i], uint64_t(M) * m[i].N, m[i].N, static_cast<uint32_t>(m[i].dtype), 0};
-    a.segments = count; a.M = M; a.K = K; a.blob = image;
-    return gemm_launch(s, a, split.slices, split.row_tiles);
+    return gemm_launch(s, m, count, image, y, M, K, split.slices, split.row_tiles);
 }
 }  // namespace guffin
 
@@ -879,9 +897,6 @@ extern "C" int guffin_hip_prefill_gemm(void* stream, int dtype, const void* tile
         return fail(GUFFIN_E_ALIGN, "prefill_gemm: tiles need 16-byte, the image 256-byte alignment");
     // the kernels address the image with 32-bit offsets
     if (image_layout(M, K).bytes >= (size_t(1) << 31)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: the image of M x K exceeds 2 GiB, split the rows");
-    GemmArgs a {};
-    a.seg[0] = {static_cast<const uint8_t*>(tiles), y, 0, N, static_cast<uint32_t>(dtype), 0};
-    a.segments = 1; a.M = M; a.K = K; a.blob = static_cast<const uint8_t*>(image);
     const PrefillMatrix m {dtype, tiles, N};
-    return gemm_launch(as_stream(stream), a, 1, split_for(&m, 1, M, K, 1).row_tiles);
+    return gemm_launch(as_stream(stream), &m, 1, static_cast<const uint8_t*>(image), &y, M, K, 1, split_for(&m, 1, M, K, 1).row_tiles);
 }
