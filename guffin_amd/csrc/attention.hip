@@ -131,13 +131,18 @@ __device__ __forceinline__ uint32_t query_place(uint32_t d) {
 }
 
 template <int ROWS, int GROUP, int HD, bool FUSED>
-__global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_partial_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_partial_kernel(const uint16_t* __restrict__ ring_k, const float* __restrict__ q_raw, const float* __restrict__ q_norm,
+                                                                                const float2* __restrict__ rope, size_t q_stride, uint32_t host_first,
+                                                                                uint32_t host_ring, uint32_t cut, uint32_t form, AttnArgs a) {
+    // What the first requests need comes in words of its own, in registers when a wave starts (see the kernels of
+    // gemv_packed.hip); the struct is a trip away.
     static_assert(HD == 256, "head dimension 256 (16 lanes x 16 dims)");
     constexpr int NQ = ROWS * GROUP;
     constexpr int kAW = attention_waves(NQ);
+    const uint32_t tp = 16 * (cut & 31u), span = 16 * ((cut >> 5) & 31u);
     extern __shared__ float lds[];
     float* sc = lds;                          // [NQ][tp] scores, then probabilities
-    float* merge = lds + NQ * a.span;         // [kAW][NQ][HD]
+    float* merge = lds + NQ * span;           // [kAW][NQ][HD]
     float* q_s = merge + kAW * NQ * HD;       // fused: [NQ][HD] prepared queries
     __shared__ float s_max[NQ], s_sum[NQ];
     __shared__ __attribute__((aligned(16))) uint16_t k_s[FUSED ? ROWS : 1][HD], v_s[FUSED ? ROWS : 1][HD];
@@ -145,17 +150,11 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
     const uint32_t part = blockIdx.x, kvh = blockIdx.y;
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     constexpr uint32_t group = GROUP;
-    // Every launch argument is asked for here, in one go: left to their first uses, the scalar loads of a
-    // 300-byte argument block are spread over the blocks of the prologue, one dependent trip each.
-    asm volatile("" :: "s"(a.q), "s"(a.ring_k), "s"(a.ring_v), "s"(a.priv_k), "s"(a.priv_v), "s"(a.schedule), "s"(a.ancestors),
-                 "s"(a.part_out), "s"(a.part_ml), "s"(a.rows), "s"(a.q_heads), "s"(a.kv_heads), "s"(a.ring_mask), "s"(a.tp),
-                 "s"(a.span), "s"(a.partitions), "s"(a.private_rows), "s"(a.scale), "s"(a.q_raw), "s"(a.k_raw), "s"(a.v_raw),
-                 "s"(a.planes), "s"(a.q_stride), "s"(a.k_stride), "s"(a.v_stride), "s"(a.q_norm), "s"(a.k_norm), "s"(a.rope),
-                 "s"(a.priv_k_out), "s"(a.priv_v_out));
-    asm volatile("" :: "s"(a.eps), "s"(a.status), "s"(a.inline_schedule), "s"(a.sched[0][0]), "s"(a.sched[0][1]),
-                 "s"(a.sched[0][2]), "s"(a.sched[0][3]), "s"(a.sched[ROWS - 1][0]), "s"(a.sched[ROWS - 1][1]),
-                 "s"(a.sched[ROWS - 1][2]), "s"(a.sched[ROWS - 1][3]), "s"(a.amask[0]), "s"(a.amask[ROWS - 1]));
-    const uint32_t row_stride = a.kv_heads * HD;  // in halves
+    const uint32_t partitions = cut >> 16;
+    const uint32_t ring_mask = static_cast<uint32_t>((uint64_t{1} << ((cut >> 10) & 63u)) - 1);
+    const uint32_t kv_heads = form & 0xFFFFu, planes = (form >> 16) & 0x7FFFu, q_heads = kv_heads * GROUP;
+    const bool scheduled = form >> 31;   // the host knows the rows' token lists
+    const uint32_t row_stride = kv_heads * HD;  // in halves
 
     // fused: the query rows of this wave (w, w+kAW, ..) are requested first; their addresses need
     // nothing but the launch arguments, so they travel together with the schedule below
@@ -167,34 +166,31 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
             const uint32_t item = wv + kAW * i;
             if (item < NQ) {
                 const uint32_t r = item / group, head = kvh * group + item % group;
-                load_head_row(qr[i], a.q_raw + (size_t(r) * a.q_heads + head) * HD, a.planes, a.q_stride, a.q_norm,
-                              a.rope + size_t(r) * (HD / 2), lane);
+                load_head_row(qr[i], q_raw + (size_t(r) * q_heads + head) * HD, planes, q_stride, q_norm, rope + size_t(r) * (HD / 2), lane);
             }
         }
     }
 
     // merged virtual token list
-    uint32_t u_first = 0xFFFFFFFFu, u_end = 0;
+    uint32_t u_first = host_first, n_ring = host_ring;
     uint32_t bfirst[ROWS], bend[ROWS], amask[ROWS];
+    if (!scheduled) {
+        uint32_t u_end = 0;
+        u_first = 0xFFFFFFFFu;
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-        bfirst[r] = 0; bend[r] = 0; amask[r] = 0;
-        if (a.inline_schedule) {
-            bfirst[r] = a.sched[r][0]; bend[r] = a.sched[r][0] + a.sched[r][1];
-            if (a.sched[r][1]) { u_first = min(u_first, bfirst[r]); u_end = max(u_end, bend[r]); }
-            amask[r] = a.amask[r];
-        } else {
+        for (int r = 0; r < ROWS; ++r) {
             const uint32_t* s = a.schedule + 4 * r;
-            bfirst[r] = s[0]; bend[r] = s[0] + s[1];
+            bfirst[r] = s[0]; bend[r] = s[0] + s[1]; amask[r] = 0;
             if (s[1]) { u_first = min(u_first, s[0]); u_end = max(u_end, s[0] + s[1]); }
             for (uint32_t i = 0; i < s[3]; ++i) amask[r] |= 1u << a.ancestors[s[2] + i];
         }
+        if (u_end == 0) { u_first = 0; }
+        n_ring = u_end - u_first;
     }
-    if (u_end == 0) { u_first = 0; }
-    const uint32_t n_ring = u_end - u_first, n_total = n_ring + a.private_rows;
+    const uint32_t private_rows = FUSED ? uint32_t(ROWS) : a.private_rows, n_total = n_ring + private_rows;
     // the last partition takes what is left (at most `span` tokens: the launch has one partition fewer when a
     // handful of tokens -- the private rows -- would otherwise need a workgroup of their own on a full chip)
-    const uint32_t t0 = part * a.tp, t1 = part + 1 == a.partitions ? min(t0 + a.span, n_total) : min(t0 + a.tp, n_total);
+    const uint32_t t0 = part * tp, t1 = part + 1 == partitions ? min(t0 + span, n_total) : min(t0 + tp, n_total);
 
     // ---- keys: four rounds of loads are issued before their dot products so that a wave keeps
     // 16 key rows (8 KB) in flight (a round is 4 tokens per wave, 4 kAW per workgroup); in fused mode the first
@@ -213,7 +209,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
             const bool is_priv = t >= n_ring;
             if (FUSED && is_priv) return;  // taken from LDS once prepared
             const uint16_t* kp = is_priv ? a.priv_k + size_t(t - n_ring) * row_stride
-                                         : a.ring_k + size_t((u_first + t) & a.ring_mask) * row_stride;
+                                         : ring_k + size_t((u_first + t) & ring_mask) * row_stride;
             kp += kvh * HD + seg * 8;
             // (4-byte aligned requests: a caller's K/V view may start at any word of its parent allocation)
             k0[u] = ld16_a4(reinterpret_cast<const uint8_t*>(kp)); k1[u] = ld16_a4(reinterpret_cast<const uint8_t*>(kp + HD / 2));
@@ -224,6 +220,16 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
         for (int u = 0; u < U; ++u) load_key_round(u, tb);
     };
     if constexpr (FUSED) load_keys(tb_first);
+    // Every other launch argument is asked for here, in one go: left to their first uses, the scalar loads of a
+    // 300-byte argument block are spread over the blocks of the prologue, one dependent trip each.
+    asm volatile("" :: "s"(a.q), "s"(a.priv_k), "s"(a.priv_v), "s"(a.ring_v), "s"(a.part_out), "s"(a.part_ml), "s"(a.private_rows), "s"(a.scale),
+                 "s"(a.k_raw), "s"(a.v_raw), "s"(a.k_stride), "s"(a.v_stride), "s"(a.k_norm), "s"(a.priv_k_out), "s"(a.priv_v_out),
+                 "s"(a.eps), "s"(a.status), "s"(a.sched[0][0]), "s"(a.sched[0][1]), "s"(a.sched[ROWS - 1][0]), "s"(a.sched[ROWS - 1][1]),
+                 "s"(a.amask[0]), "s"(a.amask[ROWS - 1]));
+    if (scheduled) {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) { bfirst[r] = a.sched[r][0]; bend[r] = a.sched[r][0] + a.sched[r][1]; amask[r] = a.amask[r]; }
+    }
     // ---- values: a half wave covers one value row (32 lanes x 8 dims, 16-byte loads), a wave two
     // tokens per round, four rounds in flight; in fused mode the first batch is requested while
     // the softmax runs
@@ -238,7 +244,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
             const bool is_priv = t >= n_ring;
             if (FUSED && is_priv) return;  // taken from LDS once prepared
             const uint16_t* vp = is_priv ? a.priv_v + size_t(t - n_ring) * row_stride
-                                         : a.ring_v + size_t((u_first + t) & a.ring_mask) * row_stride;
+                                         : a.ring_v + size_t((u_first + t) & ring_mask) * row_stride;
             vv[u] = ld16_a4(reinterpret_cast<const uint8_t*>(vp + kvh * HD + dl));
         }
     };
@@ -260,16 +266,16 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
             const uint32_t ki = wv - kFirst + kAW * i;   // wraps for the waves below: pr >= ROWS then
             const uint32_t pr = ki >> 1, pt = n_ring + pr;
             const bool is_key = (ki & 1u) == 0;
-            mine[i] = wv >= kFirst && pr < ROWS && pr < a.private_rows && pt >= t0 && pt < t1;
+            mine[i] = wv >= kFirst && pr < ROWS && pr < private_rows && pt >= t0 && pt < t1;
             if (mine[i])
-                load_head_row(kvr[i], (is_key ? a.k_raw : a.v_raw) + (size_t(pr) * a.kv_heads + kvh) * HD, a.planes, is_key ? a.k_stride : a.v_stride,
-                              is_key ? a.k_norm : nullptr, is_key ? a.rope + size_t(pr) * (HD / 2) : nullptr, lane);
+                load_head_row(kvr[i], (is_key ? a.k_raw : a.v_raw) + (size_t(pr) * kv_heads + kvh) * HD, planes, is_key ? a.k_stride : a.v_stride,
+                              is_key ? a.k_norm : nullptr, is_key ? rope + size_t(pr) * (HD / 2) : nullptr, lane);
         }
 #pragma unroll
         for (int i = 0; i < QI; ++i) {
             const uint32_t item = wv + kAW * i;
             if (item < NQ) {
-                finish_head_row(qr[i], a.q_norm != nullptr, true, a.eps);
+                finish_head_row(qr[i], q_norm != nullptr, true, a.eps);
 #pragma unroll
                 for (int c = 0; c < 4; ++c) q_s[item * HD + query_place(lane + 64 * c)] = qr[i].v[c] * a.scale;
             }
@@ -279,7 +285,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
             if (!mine[i]) continue;
             const uint32_t ki = wv - kFirst + kAW * i, pr = ki >> 1;
             const bool is_key = (ki & 1u) == 0;
-            const size_t kv_off = (size_t(pr) * a.kv_heads + kvh) * HD;
+            const size_t kv_off = (size_t(pr) * kv_heads + kvh) * HD;
             finish_head_row(kvr[i], is_key && a.k_norm != nullptr, is_key, a.eps);
             bool bad = false;
 #pragma unroll
@@ -307,7 +313,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
                     qv[n][4 * c] = p.x; qv[n][4 * c + 1] = p.y; qv[n][4 * c + 2] = p.z; qv[n][4 * c + 3] = p.w;
                 }
             } else {
-                const float* qp = a.q + (size_t(r) * a.q_heads + kvh * group + g) * HD + seg * 8;
+                const float* qp = a.q + (size_t(r) * q_heads + kvh * group + g) * HD + seg * 8;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) { qv[n][i] = qp[i] * a.scale; qv[n][8 + i] = qp[HD / 2 + i] * a.scale; }
             }
@@ -315,11 +321,11 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
         // U rounds stay in flight for the whole walk: a slot is asked for its next row (U rounds on) as soon as its
         // row has been read, so a long partition streams instead of filling and draining once per batch
         if constexpr (!FUSED) load_keys(tb_first);
-        for (uint32_t tb = tb_first; tb < t0 + a.span; tb += 4 * kAW * U) {
+        for (uint32_t tb = tb_first; tb < t0 + span; tb += 4 * kAW * U) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const uint32_t t = tb + 4 * kAW * u;
-                if (t >= t0 + a.span) break;
+                if (t >= t0 + span) break;
                 const bool in_range = t < t1, is_priv = t >= n_ring;
                 const uint32_t pos = u_first + t, prow = t - n_ring;
                 if (FUSED && in_range && is_priv) {
@@ -327,7 +333,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
                     k0[u] = *reinterpret_cast<const uint4*>(kp); k1[u] = *reinterpret_cast<const uint4*>(kp + HD / 2);
                 }
                 const uint32_t kw[8] = {k0[u].x, k0[u].y, k0[u].z, k0[u].w, k1[u].x, k1[u].y, k1[u].z, k1[u].w};
-                if (tb + 4 * kAW * U < t0 + a.span) load_key_round(u, tb + 4 * kAW * U);
+                if (tb + 4 * kAW * U < t0 + span) load_key_round(u, tb + 4 * kAW * U);
                 float s[NQ];
 #pragma unroll
                 for (int n = 0; n < NQ; ++n) {
@@ -342,7 +348,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
                         const uint32_t r = n / group;
                         const bool valid = in_range && (is_priv ? ((amask[r] >> prow) & 1u) != 0
                                                                 : (pos >= bfirst[r] && pos < bend[r]));
-                        sc[n * a.span + (t - t0)] = valid ? s[n] : -INFINITY;
+                        sc[n * span + (t - t0)] = valid ? s[n] : -INFINITY;
                     }
                 }
             }
@@ -354,13 +360,13 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
     // ---- softmax over the partition, one wave per query ----------------------------------
     for (uint32_t n = wv; n < NQ; n += kAW) {
         float m = -INFINITY;
-        for (uint32_t i = lane; i < a.span; i += 64) m = fmaxf(m, sc[n * a.span + i]);
+        for (uint32_t i = lane; i < span; i += 64) m = fmaxf(m, sc[n * span + i]);
         m = wave_max(m);
         float l = 0.f;
-        for (uint32_t i = lane; i < a.span; i += 64) {
-            const float v = sc[n * a.span + i];
+        for (uint32_t i = lane; i < span; i += 64) {
+            const float v = sc[n * span + i];
             const float p = v == -INFINITY ? 0.f : expf(v - m);
-            sc[n * a.span + i] = p;
+            sc[n * span + i] = p;
             l += p;
         }
         l = wave_sum(l);
@@ -385,7 +391,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
                 if (tb + 2 * kAW * UV < t1) load_value_round(u, tb + 2 * kAW * UV);
 #pragma unroll
                 for (int n = 0; n < NQ; ++n) {
-                    const float p = sc[n * a.span + (t - t0)];
+                    const float p = sc[n * span + (t - t0)];
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const half2_t h = __builtin_bit_cast(half2_t, w4[i]);
@@ -420,7 +426,7 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
             return v;
         };
         const uint32_t r = n / group, g = n % group, head = kvh * group + g;
-        const size_t slot = (size_t(r) * a.q_heads + head) * a.partitions + part;
+        const size_t slot = (size_t(r) * q_heads + head) * partitions + part;
         *reinterpret_cast<F2a4*>(a.part_out + slot * HD + 2 * d) = {total(merge + d), total(merge + HD / 2 + d)};
         if (d == 0) { a.part_ml[slot * 2] = s_max[n]; a.part_ml[slot * 2 + 1] = s_sum[n]; }
     }
@@ -506,6 +512,16 @@ int launch_partial(hipStream_t s, const AttnArgs& a) {
     constexpr int NQ = ROWS * GROUP;
     constexpr int kAW = attention_waves(NQ);
     const bool fused = a.q_raw != nullptr;
+    if (a.partitions > 0xFFFFu || a.kv_heads > 0xFFFFu || a.planes > 0x7FFFu) return fail(GUFFIN_E_SHAPE, "attention: more partitions, KV heads or planes than a launch takes");
+    uint32_t first = 0xFFFFFFFFu, end = 0;   // of the rows' token lists together, where they are known here
+    for (int r = 0; r < ROWS && a.inline_schedule; ++r)
+        if (a.sched[r][1]) { first = std::min(first, a.sched[r][0]); end = std::max(end, a.sched[r][0] + a.sched[r][1]); }
+    if (end == 0) first = 0;
+    const uint32_t ring = end - first;
+    uint32_t cap = 0;
+    while (cap < 32 && (a.ring_mask >> cap)) ++cap;
+    const uint32_t cut = a.tp / 16 | a.span / 16 << 5 | cap << 10 | a.partitions << 16;
+    const uint32_t form = a.kv_heads | a.planes << 16 | a.inline_schedule << 31;
     const size_t lds = (size_t(NQ) * a.span + size_t(kAW) * NQ * 256 + (fused ? size_t(NQ) * 256 : 0)) * sizeof(float);
     if constexpr (kAW * NQ * 256 * sizeof(float) >= 64 * 1024) {   // more than a launch gets unasked, allowed once per kernel
         static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_partial_kernel<ROWS, GROUP, 256, true>),
@@ -518,9 +534,11 @@ int launch_partial(hipStream_t s, const AttnArgs& a) {
         if (allowed != hipSuccess) return fail(GUFFIN_E_HIP, "attention_partial: could not raise the dynamic LDS limit");
     }
     if (fused || ROWS > 2)
-        launch((attn_partial_kernel<ROWS, GROUP, 256, true>), dim3(a.partitions, a.kv_heads), dim3(64 * kAW), lds, s, a);
+        launch((attn_partial_kernel<ROWS, GROUP, 256, true>), dim3(a.partitions, a.kv_heads), dim3(64 * kAW), lds, s, a.ring_k, a.q_raw, a.q_norm,
+               a.rope, a.q_stride, first, ring, cut, form, a);
     else if constexpr (ROWS <= 2)
-        launch((attn_partial_kernel<ROWS, GROUP, 256, false>), dim3(a.partitions, a.kv_heads), dim3(64 * kAW), lds, s, a);
+        launch((attn_partial_kernel<ROWS, GROUP, 256, false>), dim3(a.partitions, a.kv_heads), dim3(64 * kAW), lds, s, a.ring_k, a.q_raw, a.q_norm,
+               a.rope, a.q_stride, first, ring, cut, form, a);
     return check_launch("attention_partial");
 }
 

@@ -374,16 +374,15 @@ template <typename T>
 __device__ __forceinline__ void shared_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 __global__ void __launch_bounds__(1024)
-threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32_t segs, uint32_t retain_cap, uint32_t sure,
-                        float divisor, const uint32_t* __restrict__ history, const uint32_t* __restrict__ history_count,
-                        const uint32_t* __restrict__ row_retain, uint32_t row_stride, uint32_t history_stride,
-                        uint32_t* __restrict__ ws, Candidates* __restrict__ result, uint32_t* __restrict__ status,
-                        bool suppressed_ok, bool whole) {
+threshold_select_kernel(const float* __restrict__ logits, uint32_t* __restrict__ ws, uint32_t vocab, uint32_t segs, uint32_t retain_cap,
+                        uint32_t sure, float divisor, uint32_t row_stride, const uint32_t* __restrict__ history_count,
+                        const uint32_t* __restrict__ row_retain, const uint32_t* __restrict__ history, uint32_t history_stride,
+                        Candidates* __restrict__ result, uint32_t* __restrict__ status, bool suppressed_ok, bool whole) {
     __shared__ uint32_t hist[256];
     __shared__ uint64_t sel[kCollectCap];
     __shared__ uint64_t keys[512];
     __shared__ uint32_t s_bin, s_above, s_in, s_last, s_count;
-    const uint32_t row = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const uint32_t row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, collectors = (vocab + kCollectTile - 1) / kCollectTile;
     uint32_t* row_ws = ws + size_t(row) * kThresholdRowWords;
     uint32_t* counter = row_ws + kMaxSegs;
     uint32_t* done = counter + 1;
@@ -392,7 +391,7 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
     uint64_t* common = places + kMaxCollectors * kSlots;
     const float* lr = logits + size_t(row) * vocab;
     // this workgroup's logits are requested before the bound is worked out
-    auto token_of = [&](uint32_t u) { return ((u * (blockDim.x / 64) + (tid >> 6)) * gridDim.x + blockIdx.x) * 64 + lane; };
+    auto token_of = [&](uint32_t u) { return ((u * (1024 / 64) + (tid >> 6)) * collectors + blockIdx.x) * 64 + lane; };
     float mine[kCollectTile / 1024];
 #pragma unroll
     for (uint32_t u = 0; u < kCollectTile / 1024; ++u) mine[u] = token_of(u) < vocab ? lr[token_of(u)] : 0.f;
@@ -446,7 +445,7 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
         const uint32_t more = found - kSlots;   // beyond the list: the row's counter shows it too, and nobody reads the list
         if (tid == 0) s_bin = __hip_atomic_fetch_add(counter, more, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
-        for (uint32_t i = tid; i < min(more, kCommonCap); i += blockDim.x)
+        for (uint32_t i = tid; i < min(more, kCommonCap); i += 1024)
             if (s_bin + i < kCommonCap) shared_store(common + s_bin + i, sel[kSlots + i]);
     }
     if (bad && status) atomicOr(status + row, GUFFIN_STATUS_NONFINITE);
@@ -455,22 +454,22 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
     __syncthreads();
     if (tid == 0) {
         const uint32_t before = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = before + 1 == gridDim.x;
+        s_last = before + 1 == collectors;
         s_count = 0;
     }
     __syncthreads();
     if (!s_last) return;
     // every wave scans the counts for itself; a thread takes one place
-    const uint32_t count = lane < gridDim.x ? shared_load(counts + lane) : 0;
+    const uint32_t count = lane < collectors ? shared_load(counts + lane) : 0;
     const uint32_t owner = tid / kSlots, raised = status ? shared_load(status + row) : 0;
-    const uint64_t place = owner < gridDim.x ? shared_load(places + tid) : 0;   // its collector may have left it as it was
+    const uint64_t place = owner < collectors ? shared_load(places + tid) : 0;   // its collector may have left it as it was
     const uint32_t kept = min(count, kSlots), upto = wave_inclusive_scan(kept), all = wave_inclusive_scan(count);
     const uint32_t n = __builtin_amdgcn_readlane(all, 63), placed = __builtin_amdgcn_readlane(upto, 63);
     const uint32_t own_kept = __shfl(kept, owner, kWave), own_upto = __shfl(upto, owner, kWave);
     static_assert(kMaxCollectors * kSlots == 1024, "a place per thread");
     if (n <= kCollectCap && n - placed <= kCommonCap) {
         if (tid % kSlots < own_kept) sel[own_upto - own_kept + tid % kSlots] = place;
-        for (uint32_t i = tid; i < n - placed; i += blockDim.x) sel[placed + i] = shared_load(common + i);
+        for (uint32_t i = tid; i < n - placed; i += 1024) sel[placed + i] = shared_load(common + i);
         if (n <= 512) {
             __syncthreads();
             // the workgroup's 1024 threads over n keys: 2, 4, 8 or 16 neighbouring lanes count for one of them
@@ -486,9 +485,9 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
             if (i < n && part == 0 && rank < retain) keys[rank] = k;
             retain = min(retain, n);   // fewer only where the call is sure of fewer
         } else {
-            for (uint32_t i = n + tid; i < kCollectCap; i += blockDim.x) sel[i] = 0;
+            for (uint32_t i = n + tid; i < kCollectCap; i += 1024) sel[i] = 0;
             bitonic_desc(sel, kCollectCap);
-            for (uint32_t i = tid; i < retain; i += blockDim.x) keys[i] = sel[i];
+            for (uint32_t i = tid; i < retain; i += 1024) keys[i] = sel[i];
         }
     } else {
         // more ties than the list holds: an 8-pass radix select over the whole row's keys, exact and slow
@@ -498,7 +497,7 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
             const int down = 56 - 8 * pass;
             if (tid < 256) hist[tid] = 0;
             __syncthreads();
-            for (uint32_t i0 = 0; i0 < vocab; i0 += blockDim.x) {   // whole waves stay converged
+            for (uint32_t i0 = 0; i0 < vocab; i0 += 1024) {   // whole waves stay converged
                 const uint32_t i = i0 + tid;
                 const uint64_t k = i < vocab ? make_key(lr[i] / divisor, i) : 0;
                 hist_add(hist, i < vocab && (pass == 0 || (k >> (down + 8)) == kprefix), static_cast<uint32_t>(k >> down) & 255u, lane);
@@ -510,12 +509,12 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t vocab, uint32
             left -= s_above;
         }
         // kprefix is the retain-th largest key (keys are unique): everything above it, then it
-        for (uint32_t i = tid; i < vocab; i += blockDim.x) {
+        for (uint32_t i = tid; i < vocab; i += 1024) {
             const uint64_t k = make_key(lr[i] / divisor, i);
             if (k >= kprefix) sel[atomicAdd(&s_count, 1u)] = k;
         }
         __syncthreads();
-        for (uint32_t i = tid; i < retain; i += blockDim.x) {
+        for (uint32_t i = tid; i < retain; i += 1024) {
             const uint64_t k = sel[i];
             uint32_t rank = 0;
             for (uint32_t j = 0; j < retain; ++j) rank += sel[j] > k;
@@ -668,8 +667,8 @@ int guffin::select_candidates_scaled(hipStream_t s, const float* logits, uint32_
                fresh ? status : nullptr);
         if (int rc = check_launch("select_candidates(segment maxima)")) return rc;
         launch(threshold_select_kernel, dim3((vocab + kCollectTile - 1) / kCollectTile, rows), dim3(1024), 0, s,
-                           logits, vocab, segs, keep, sure, divisor, history, history_count, row_retain, row_stride,
-                           row_stride == 1 ? 64u : row_stride, words, static_cast<Candidates*>(result), status, suppressed_ok, fresh);
+                           logits, words, vocab, segs, keep, sure, divisor, row_stride, history_count, row_retain, history,
+                           row_stride == 1 ? 64u : row_stride, static_cast<Candidates*>(result), status, suppressed_ok, fresh);
         return check_launch("select_candidates(threshold)");
     }
     if (fresh) launch(clear_words_kernel, dim3((rows + 63) / 64), dim3(64), 0, s, status, rows);

@@ -210,9 +210,10 @@ template <int NT>
 __global__ void __launch_bounds__(256, 2)
 prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __restrict__ ring_k,
                               const uint16_t* __restrict__ run_k, const uint16_t* __restrict__ vt,
-                              AttentionOut to, uint32_t rows, uint32_t position, uint32_t window,
-                              uint32_t ring_mask, uint32_t q_heads, uint32_t kv_heads, float scale,
-                              uint32_t base32, uint32_t T, uint32_t group_shift) {
+                              uint32_t rows, uint32_t position, uint32_t window, uint32_t ring_mask, uint32_t base32, uint32_t form,
+                              float scale, uint32_t T, AttentionOut to) {
+    // (the arguments' order: what the first requests need goes first, see the kernels of gemv_packed.hip)
+    const uint32_t kv_heads = form & 0xFFFFu, group_shift = (form >> 16) & 3u, q_heads = kv_heads << group_shift, parts = form >> 18;
     constexpr int HD = 256;
     constexpr uint32_t kPairs = 16 * NT;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -229,7 +230,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
     const uint32_t lo_first = (window && position + r0 + 1 > window) ? position + r0 + 1 - window : 0;
     const uint32_t last_first = (window && hi_pos + 1 > window) ? hi_pos + 1 - window : 0;   // of the last row
     const uint32_t tile_lo = (lo_first - base32) / 32, tiles = (hi_pos - base32) / 32 + 1 - tile_lo;
-    const uint32_t begin = tile_lo + blockIdx.z * tiles / gridDim.z, end = tile_lo + (blockIdx.z + 1) * tiles / gridDim.z;
+    const uint32_t begin = tile_lo + blockIdx.z * tiles / parts, end = tile_lo + (blockIdx.z + 1) * tiles / parts;
 
     auto ask_keys = [&](uint32_t ti, uint4 (&kb)[2][8]) {
 #pragma unroll
@@ -460,7 +461,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
             v[k] = src[k];
             if constexpr (kMergeAtOnce<NT>) v[k] += src[kWaveSlots + k] + src[2 * kWaveSlots + k] + src[3 * kWaveSlots + k];
         }
-        if (gridDim.z == 1) {
+        if (parts == 1) {
             const float den = ml[p * 2 + 1] * kProbScale;
 #pragma unroll
             for (int k = 0; k < 8; ++k) v[k] /= den;
@@ -477,13 +478,14 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
 
 // the parts' states of every (row, head), merged in part order; 32 lanes per pair
 __global__ void __launch_bounds__(256)
-prefill_attention_merge_kernel(AttentionOut to, uint32_t rows, uint32_t q_heads, uint32_t parts) {
+prefill_attention_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, uint32_t rows, uint32_t q_heads, uint32_t parts,
+                               AttentionOut to) {
     constexpr uint32_t HD = 256, kAhead = 12;   // parts asked for at once
     const uint32_t pair = blockIdx.x * 8 + threadIdx.x / 32, c8 = threadIdx.x % 32;
     if (pair >= rows * q_heads) return;
     const size_t stride = size_t(rows) * q_heads;
     // a lane a part's state, 32 at a time: their maximum and weights are two reductions instead of a walk of one trip a part
-    const float2* states = reinterpret_cast<const float2*>(to.part_ml);
+    const float2* states = reinterpret_cast<const float2*>(part_ml);
     auto top_of = [](float x) { return both_max(rows_beside(__float_as_uint(row16_max(x)))); };
     auto sum_of = [](float x) { return both_sum(rows_beside(__float_as_uint(row16_sum(x)))); };
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, den = 0.f, M = -INFINITY;
@@ -506,7 +508,7 @@ prefill_attention_merge_kernel(AttentionOut to, uint32_t rows, uint32_t q_heads,
             for (uint32_t i = 0; i < kAhead; ++i) {
                 a[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (i0 + i < n) {
-                    const float* src = to.part_o + ((p0 + i0 + i) * stride + pair) * HD + 8 * c8;
+                    const float* src = part_o + ((p0 + i0 + i) * stride + pair) * HD + 8 * c8;
                     a[i] = *reinterpret_cast<const float4*>(src); b[i] = *reinterpret_cast<const float4*>(src + 4);
                 }
             }
@@ -717,19 +719,21 @@ int prefill_attention_run(hipStream_t s, const float* q, const void* ring_k, con
     const ValueSpan vs = value_span(rows, position, window);
     const uint32_t group = q_heads / kv_heads, shift = group == 1 ? 0 : group == 2 ? 1 : 2;
     const auto [nt, parts] = attention_cut(rows, vs.T, kv_heads, group);
+    if (kv_heads > 0xFFFFu) return fail(GUFFIN_E_SHAPE, "prefill_attention: more KV heads than a grid has rows");
     float* states = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + transposed_bytes(vs.T, kv_heads));
     const AttentionOut to {out, image, states, states + size_t(parts) * rows * q_heads * 256};
     const uint32_t lds = attention_lds(nt);
     if (int rc = allow_attention_lds()) return rc;
     const dim3 grid((rows * group + 16 * nt - 1) / (16 * nt), kv_heads, parts);
+    const uint32_t form = kv_heads | (shift << 16) | (parts << 18);   // at most two parts a compute unit
 #define GUFFIN_PA(NT_) launch(prefill_attention_mfma_kernel<NT_>, grid, dim3(256), lds, s, q, static_cast<const uint16_t*>(ring_k), \
-                              static_cast<const uint16_t*>(run_k), static_cast<const uint16_t*>(workspace), to, rows, position, window, \
-                              ring_mask, q_heads, kv_heads, scale, vs.base32, vs.T, shift)
+                              static_cast<const uint16_t*>(run_k), static_cast<const uint16_t*>(workspace), rows, position, window, ring_mask, \
+                              vs.base32, form, scale, vs.T, to)
     if (nt == 1) GUFFIN_PA(1); else GUFFIN_PA(2);
 #undef GUFFIN_PA
     if (int rc = check_launch("prefill_attention_mfma")) return rc;
     if (parts == 1) return GUFFIN_OK;
-    launch(prefill_attention_merge_kernel, dim3((rows * q_heads + 7) / 8), dim3(256), 0, s, to, rows, q_heads, parts);
+    launch(prefill_attention_merge_kernel, dim3((rows * q_heads + 7) / 8), dim3(256), 0, s, to.part_o, to.part_ml, rows, q_heads, parts, to);
     return check_launch("prefill_attention_merge");
 }
 }  // namespace guffin

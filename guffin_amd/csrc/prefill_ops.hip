@@ -15,10 +15,10 @@
 namespace guffin {
 namespace {
 
-// scratch: nobody else's, and used once
-__device__ __forceinline__ float block_total(float v, float* scratch) {
+// scratch: nobody else's, and used once; waves: of the workgroup
+__device__ __forceinline__ float block_total(float v, float* scratch, uint32_t waves) {
     v = wave_sum(v);
-    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, waves = (blockDim.x + 63) >> 6;
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (lane == 0) scratch[wv] = v;
     lds_barrier();
     float t = 0.f;
@@ -76,7 +76,7 @@ prefill_norm_kernel(const float* __restrict__ x, const float* __restrict__ gamma
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
-    const float inv = 1.0f / sqrtf(block_total(ss, scratch) / static_cast<float>(width) + eps);
+    const float inv = 1.0f / sqrtf(block_total(ss, scratch, (width + 511) / 512) / static_cast<float>(width) + eps);
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < 8; ++i) { v[i] = v[i] * inv * g[i]; bad |= !isfinite(v[i]); }
@@ -89,12 +89,12 @@ prefill_norm_kernel(const float* __restrict__ x, const float* __restrict__ gamma
 // 8.4 us by eights, 8.1 at once; 12 rows 8.0 and 7.5); THREADS: the widest row's.
 template <int B, int THREADS>
 __global__ void __launch_bounds__(THREADS)
-prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_stride, const float* __restrict__ gamma_post,
-                     const float* __restrict__ residual, float* __restrict__ out_residual, const float* __restrict__ gamma_next,
-                     float* __restrict__ out_norm, uint8_t* __restrict__ image, uint32_t rows, uint32_t width, float eps,
-                     RunRows run, uint32_t* __restrict__ status) {
+prefill_joint_kernel(const float* __restrict__ x, const float* __restrict__ residual, const float* __restrict__ gamma_post,
+                     const float* __restrict__ gamma_next, size_t plane_stride, uint32_t planes, uint32_t width, uint32_t rows, float eps,
+                     float* __restrict__ out_residual, float* __restrict__ out_norm, uint8_t* __restrict__ image, RunRows run,
+                     uint32_t* __restrict__ status) {
     if (blockIdx.x >= rows) {
-        const uint64_t i = uint64_t(blockIdx.x - rows) * blockDim.x + threadIdx.x;
+        const uint64_t i = uint64_t(blockIdx.x - rows) * ((width + 511) / 512 * 64) + threadIdx.x;
         if (i >= uint64_t(rows - run.first_row) * run.row_vec) return;
         const uint32_t row = run.first_row + static_cast<uint32_t>(i / run.row_vec), c = static_cast<uint32_t>(i % run.row_vec);
         const size_t dst = size_t((run.position + row) & run.ring_mask) * run.row_vec + c;
@@ -116,7 +116,7 @@ prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
-    float inv = 1.0f / sqrtf(block_total(ss, scratch[0]) / static_cast<float>(width) + eps);
+    float inv = 1.0f / sqrtf(block_total(ss, scratch[0], (width + 511) / 512) / static_cast<float>(width) + eps);
     bool bad = false;
     ss = 0.f;
 #pragma unroll
@@ -125,7 +125,7 @@ prefill_joint_kernel(const float* __restrict__ x, uint32_t planes, size_t plane_
         bad |= !isfinite(v[i]);
         ss = fmaf(v[i], v[i], ss);
     }
-    inv = 1.0f / sqrtf(block_total(ss, scratch[1]) / static_cast<float>(width) + eps);
+    inv = 1.0f / sqrtf(block_total(ss, scratch[1], (width + 511) / 512) / static_cast<float>(width) + eps);
     if (active) store8(out_residual + at, v);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = v[i] * inv * gn[i];
@@ -170,36 +170,39 @@ prefill_geglu_kernel(const float* __restrict__ gate, const float* __restrict__ u
 // 6.4, 7.5 and 29.0).
 constexpr uint32_t kQkvThreads = 1024;
 __global__ void __launch_bounds__(kQkvThreads)
-prefill_qkv_kernel(QkvRun a) {
+prefill_qkv_kernel(const float* __restrict__ q_planes, const float* __restrict__ k_planes, const float* __restrict__ v_planes,
+                   const uint16_t* __restrict__ ring_v, uint32_t rows, uint32_t head_groups, uint32_t planes, uint32_t kv_heads, uint32_t position,
+                   uint32_t base32, QkvRun a) {
+    // (the struct holds them as well, but arrives a trip later: see the kernels of gemv_packed.hip)
     constexpr uint32_t HD = 256, PITCH = HD + 8;
     __shared__ __attribute__((aligned(16))) uint16_t tile[32][PITCH];
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     bool bad = false;
-    if (blockIdx.x < a.head_groups) {
-        const uint32_t per_row = a.q_heads + a.kv_heads, p = blockIdx.x * (kQkvThreads / 64) + wv;
-        if (p >= a.rows * per_row) return;
+    if (blockIdx.x < head_groups) {
+        const uint32_t per_row = a.q_heads + kv_heads, p = blockIdx.x * (kQkvThreads / 64) + wv;
+        if (p >= rows * per_row) return;
         const uint32_t r = p / per_row, h = p % per_row;
         const bool is_q = h < a.q_heads;
-        const uint32_t hh = is_q ? h : h - a.q_heads, heads = is_q ? a.q_heads : a.kv_heads;
+        const uint32_t hh = is_q ? h : h - a.q_heads, heads = is_q ? a.q_heads : kv_heads;
         const size_t off = (size_t(r) * heads + hh) * HD;
-        const size_t stride = size_t(a.rows) * heads * HD;
-        const float* src = (is_q ? a.q_planes : a.k_planes) + off;
+        const size_t stride = size_t(rows) * heads * HD;
+        const float* src = (is_q ? q_planes : k_planes) + off;
         const float* gamma = is_q ? a.q_norm : a.k_norm;
         // lane: columns 2 lane, 2 lane + 1 of either half, the pairs that rotate together
         const float4 rot = reinterpret_cast<const float4*>(a.rope_table)[size_t(r) * (HD / 4) + lane];   // cos, sin of two pairs
         const float2 g0 = make_float2(gamma[2 * lane], gamma[2 * lane + 1]), g1 = make_float2(gamma[HD / 2 + 2 * lane], gamma[HD / 2 + 2 * lane + 1]);
         float v[4];
-        for (uint32_t s0 = 0; s0 < a.planes; s0 += 8) {
+        for (uint32_t s0 = 0; s0 < planes; s0 += 8) {
             float2 x[8], y[8];
 #pragma unroll
             for (int s = 0; s < 8; ++s)
-                if (s0 + s < a.planes) {
+                if (s0 + s < planes) {
                     x[s] = *reinterpret_cast<const float2*>(src + (s0 + s) * stride + 2 * lane);
                     y[s] = *reinterpret_cast<const float2*>(src + (s0 + s) * stride + HD / 2 + 2 * lane);
                 }
 #pragma unroll
             for (int s = 0; s < 8; ++s)
-                if (s0 + s < a.planes) {
+                if (s0 + s < planes) {
                     if (s0 + s == 0) { v[0] = x[s].x; v[1] = x[s].y; v[2] = y[s].x; v[3] = y[s].y; }
                     else { v[0] += x[s].x; v[1] += x[s].y; v[2] += y[s].x; v[3] += y[s].y; }
                 }
@@ -222,16 +225,16 @@ prefill_qkv_kernel(QkvRun a) {
             *reinterpret_cast<uint32_t*>(a.k_out + off + HD / 2 + 2 * lane) = narrow(o2, o3);
         }
     } else {
-        const uint32_t w = blockIdx.x - a.head_groups, kvh = w % a.kv_heads, v0 = (w / a.kv_heads) * 32;
-        const size_t width = size_t(a.kv_heads) * HD, stride = size_t(a.rows) * width;
+        const uint32_t w = blockIdx.x - head_groups, kvh = w % kv_heads, v0 = (w / kv_heads) * 32;
+        const size_t width = size_t(kv_heads) * HD, stride = size_t(rows) * width;
         static_assert(kQkvThreads == 32 * (HD / 8), "a thread: eight elements of a token");
         {
-            const uint32_t token = threadIdx.x / (HD / 8), d8 = threadIdx.x % (HD / 8), kp = a.base32 + v0 + token;
+            const uint32_t token = threadIdx.x / (HD / 8), d8 = threadIdx.x % (HD / 8), kp = base32 + v0 + token;
             uint4 val = make_uint4(0, 0, 0, 0);   // outside the visible range
-            if (kp >= a.position && kp < a.position + a.rows) {
-                const size_t off = size_t(kp - a.position) * width + kvh * HD + 8 * d8;
+            if (kp >= position && kp < position + rows) {
+                const size_t off = size_t(kp - position) * width + kvh * HD + 8 * d8;
                 float f[8];
-                sum_planes8<8>(a.v_planes + off, a.planes, stride, f);
+                sum_planes8<8>(v_planes + off, planes, stride, f);
                 uint32_t o[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -241,8 +244,8 @@ prefill_qkv_kernel(QkvRun a) {
                 }
                 val = make_uint4(o[0], o[1], o[2], o[3]);
                 *reinterpret_cast<uint4*>(a.v_out + off) = val;
-            } else if (kp >= a.first_visible && kp < a.position) {
-                const U4a4 t = *reinterpret_cast<const U4a4*>(a.ring_v + size_t(kp & a.ring_mask) * width + kvh * HD + 8 * d8);
+            } else if (kp >= a.first_visible && kp < position) {
+                const U4a4 t = *reinterpret_cast<const U4a4*>(ring_v + size_t(kp & a.ring_mask) * width + kvh * HD + 8 * d8);
                 val = make_uint4(t.x, t.y, t.z, t.w);
             }
             *reinterpret_cast<uint4*>(&tile[token][8 * d8]) = val;
@@ -272,12 +275,10 @@ int prefill_joint(hipStream_t s, const float* x, uint32_t planes, const float* g
     const uint32_t threads = row_threads(width);
     const uint64_t copies = run.run_k ? uint64_t(rows - run.first_row) * run.row_vec : 0;
     const dim3 grid(rows + static_cast<uint32_t>((copies + threads - 1) / threads));
-    if (planes > 8 && threads <= 512)
-        launch(prefill_joint_kernel<16, 512>, grid, dim3(threads), 0, s, x, planes, size_t(rows) * width, gamma_post, residual, out_residual,
-               gamma_next, out_norm, image, rows, width, eps, run, status);
-    else
-        launch(prefill_joint_kernel<8, 1024>, grid, dim3(threads), 0, s, x, planes, size_t(rows) * width, gamma_post, residual, out_residual,
-               gamma_next, out_norm, image, rows, width, eps, run, status);
+#define GUFFIN_JOINT(...) launch((prefill_joint_kernel<__VA_ARGS__>), grid, dim3(threads), 0, s, x, residual, gamma_post, gamma_next, size_t(rows) * width, \
+                                 planes, width, rows, eps, out_residual, out_norm, image, run, status)
+    if (planes > 8 && threads <= 512) GUFFIN_JOINT(16, 512); else GUFFIN_JOINT(8, 1024);
+#undef GUFFIN_JOINT
     return check_launch("prefill_joint");
 }
 
@@ -288,7 +289,8 @@ int prefill_geglu(hipStream_t s, const float* gate, const float* up, uint32_t pl
 
 int prefill_qkv(hipStream_t s, QkvRun a) {
     a.head_groups = (a.rows * (a.q_heads + a.kv_heads) + kQkvThreads / 64 - 1) / (kQkvThreads / 64);
-    launch(prefill_qkv_kernel, dim3(a.head_groups + (a.T / 32) * a.kv_heads), dim3(kQkvThreads), 0, s, a);
+    launch(prefill_qkv_kernel, dim3(a.head_groups + (a.T / 32) * a.kv_heads), dim3(kQkvThreads), 0, s, a.q_planes,
+           a.k_planes, a.v_planes, a.ring_v, a.rows, a.head_groups, a.planes, a.kv_heads, a.position, a.base32, a);
     return check_launch("prefill_qkv");
 }
 
