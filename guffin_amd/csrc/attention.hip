@@ -150,9 +150,10 @@ __global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_parti
     const uint32_t part = blockIdx.x, kvh = blockIdx.y;
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     constexpr uint32_t group = GROUP;
-    const uint32_t partitions = cut >> 16;
+    // (a field at its largest value: what it cannot hold stands in the struct)
+    const uint32_t partitions = cut >> 16 == 0xFFFFu ? a.partitions : cut >> 16;
     const uint32_t ring_mask = static_cast<uint32_t>((uint64_t{1} << ((cut >> 10) & 63u)) - 1);
-    const uint32_t kv_heads = form & 0xFFFFu, planes = (form >> 16) & 0x7FFFu, q_heads = kv_heads * GROUP;
+    const uint32_t kv_heads = form & 0xFFFFu, planes = ((form >> 16) & 0x7FFFu) == 0x7FFFu ? a.planes : (form >> 16) & 0x7FFFu, q_heads = kv_heads * GROUP;
     const bool scheduled = form >> 31;   // the host knows the rows' token lists
     const uint32_t row_stride = kv_heads * HD;  // in halves
 
@@ -512,7 +513,7 @@ int launch_partial(hipStream_t s, const AttnArgs& a) {
     constexpr int NQ = ROWS * GROUP;
     constexpr int kAW = attention_waves(NQ);
     const bool fused = a.q_raw != nullptr;
-    if (a.partitions > 0xFFFFu || a.kv_heads > 0xFFFFu || a.planes > 0x7FFFu) return fail(GUFFIN_E_SHAPE, "attention: more partitions, KV heads or planes than a launch takes");
+    if (a.kv_heads > 0xFFFFu) return fail(GUFFIN_E_SHAPE, "attention_decode: more KV heads than a grid has rows");
     uint32_t first = 0xFFFFFFFFu, end = 0;   // of the rows' token lists together, where they are known here
     for (int r = 0; r < ROWS && a.inline_schedule; ++r)
         if (a.sched[r][1]) { first = std::min(first, a.sched[r][0]); end = std::max(end, a.sched[r][0] + a.sched[r][1]); }
@@ -520,8 +521,8 @@ int launch_partial(hipStream_t s, const AttnArgs& a) {
     const uint32_t ring = end - first;
     uint32_t cap = 0;
     while (cap < 32 && (a.ring_mask >> cap)) ++cap;
-    const uint32_t cut = a.tp / 16 | a.span / 16 << 5 | cap << 10 | a.partitions << 16;
-    const uint32_t form = a.kv_heads | a.planes << 16 | a.inline_schedule << 31;
+    const uint32_t cut = a.tp / 16 | a.span / 16 << 5 | cap << 10 | std::min(a.partitions, 0xFFFFu) << 16;
+    const uint32_t form = a.kv_heads | std::min(a.planes, 0x7FFFu) << 16 | a.inline_schedule << 31;
     const size_t lds = (size_t(NQ) * a.span + size_t(kAW) * NQ * 256 + (fused ? size_t(NQ) * 256 : 0)) * sizeof(float);
     if constexpr (kAW * NQ * 256 * sizeof(float) >= 64 * 1024) {   // more than a launch gets unasked, allowed once per kernel
         static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_partial_kernel<ROWS, GROUP, 256, true>),
