@@ -13,6 +13,7 @@
 // caller can capture a whole step into a HIP graph.
 #include <cstddef>
 #include "common.hpp"
+#include "embed.hpp"
 #include "resident.hpp"
 #include "selection_request.hpp"
 #include "receipt.hpp"
@@ -161,30 +162,89 @@ void row_schedule(const guffin_model_desc& m, uint32_t layer, uint32_t position,
 // positions, ancestors, the per-layer attention schedule of `rows` contiguous rows and the two
 // rotation tables (local and global frequency base) of the pass.  depths: byte r is row r's distance from `position`
 // (r itself for contiguous rows; a tree's schedule travels with its launches, it asks for no layers here)
-__global__ void stage_rows_kernel(uint32_t* positions, uint32_t* ancestors, uint32_t* schedule, uint32_t rows,
-                                  uint32_t position, uint32_t depths, uint32_t layers, uint32_t window, uint32_t global_period,
-                                  float2* rope_local, float2* rope_global, uint32_t rope_dim, float local_base,
-                                  float global_base, float global_scale, uint32_t* sync, uint32_t sync_words) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < sync_words) sync[i] = 0u;   // barrier counters of the resident pass start at zero
-    const uint32_t half = rope_dim / 2;
-    auto at = [&](uint32_t row) { return position + ((depths >> (8 * row)) & 255u); };
+struct Staging {
+    uint32_t *positions, *ancestors, *schedule;
+    uint32_t rows, position, depths, layers, window, global_period;
+    float2 *rope_local, *rope_global;
+    uint32_t rope_dim;
+    float local_base, global_base, global_scale;
+    uint32_t* sync; uint32_t sync_words;
+};
+// item i of them
+__device__ __forceinline__ void stage_item(const Staging& p, uint32_t i) {
+    if (i < p.sync_words) p.sync[i] = 0u;   // barrier counters of the resident pass start at zero
+    const uint32_t half = p.rope_dim / 2, rows = p.rows;
+    auto at = [&](uint32_t row) { return p.position + ((p.depths >> (8 * row)) & 255u); };
     if (i < rows * half) {
         float c, s;
-        if (global_period > 1) {  // a model without local blocks has no local base
-            rope_sincos(at(i / half), i % half, rope_dim, local_base, 1.0f, c, s);
-            rope_local[i] = make_float2(c, s);
+        if (p.global_period > 1) {  // a model without local blocks has no local base
+            rope_sincos(at(i / half), i % half, p.rope_dim, p.local_base, 1.0f, c, s);
+            p.rope_local[i] = make_float2(c, s);
         }
-        rope_sincos(at(i / half), i % half, rope_dim, global_base, global_scale, c, s);
-        rope_global[i] = make_float2(c, s);
+        rope_sincos(at(i / half), i % half, p.rope_dim, p.global_base, p.global_scale, c, s);
+        p.rope_global[i] = make_float2(c, s);
     }
-    if (i < rows) { positions[i] = at(i); ancestors[i] = i; }
-    if (i >= layers * rows) return;
+    if (i < rows) { p.positions[i] = at(i); p.ancestors[i] = i; }
+    if (i >= p.layers * rows) return;
     const uint32_t layer = i / rows, row = i % rows;
     uint32_t words[4];
-    row_schedule_words(layer_is_local(global_period, layer), window, position, row, words);
-    uint32_t* s = schedule + 4 * i;
+    row_schedule_words(layer_is_local(p.global_period, layer), p.window, p.position, row, words);
+    uint32_t* s = p.schedule + 4 * i;
     s[0] = words[0]; s[1] = words[1]; s[2] = words[2]; s[3] = words[3];
+}
+__global__ void __launch_bounds__(64) stage_rows_kernel(const Staging p) { stage_item(p, blockIdx.x * 64 + threadIdx.x); }
+
+// What a pass starts with, in one launch: workgroups [0, rows) look a row up, scaled (x), and leave it normalised with its
+// receipt (u); the others stage.  Three launches of 4.8 us, each its boundary and a chain of two or three trips, are one of
+// 4.6 us (640 columns of Q8_0) or 7.5 (3840 of Q6_K).  Arithmetic and order are those of embed_kernel and rms_norm_kernel (ops.hip).  block: `threads`.
+template <int DTYPE>
+__global__ void __launch_bounds__(1024)
+enter_rows_kernel(const uint32_t* __restrict__ tokens, const uint8_t* __restrict__ w, const float* __restrict__ gamma, uint32_t width, float scale,
+                  uint32_t vocab, float eps, uint32_t rows, uint32_t threads, float* __restrict__ x, float* __restrict__ u, float* __restrict__ u_sums,
+                  uint32_t* __restrict__ status, const Staging staging) {
+    if (blockIdx.x >= rows) {
+        stage_item(staging, (blockIdx.x - rows) * threads + threadIdx.x);
+        return;
+    }
+    extern __shared__ float row[];   // [width]
+    __shared__ float sums[16];
+    const uint32_t r = blockIdx.x;
+    uint32_t token = tokens[r];
+    if (token >= vocab) {
+        if (threadIdx.x == 0 && status) atomicOr(status, GUFFIN_STATUS_BAD_TOKEN);
+        token = 0;
+    }
+    const uint8_t* from = embed_row<DTYPE>(w, token, width);
+    bool bad = false;
+    float ss = 0.f;
+    for (uint32_t c0 = threadIdx.x; c0 < width; c0 += 4 * threads) {
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = c0 + k * threads < width ? __fmul_rn(embed_element<DTYPE>(from, c0 + k * threads), scale) : 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (c0 + k * threads < width) {
+                bad |= !isfinite(v[k]);
+                row[c0 + k * threads] = v[k];
+                x[size_t(r) * width + c0 + k * threads] = v[k];
+                ss = fmaf(v[k], v[k], ss);
+            }
+    }
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = ss;
+    lds_barrier();
+    float total = 0.f;
+    for (uint32_t i = 0; i < threads / 64; ++i) total += sums[i];
+    const float inv = 1.0f / sqrtf(total / static_cast<float>(width) + eps);
+    for (uint32_t c = threadIdx.x; c < width; c += threads) {
+        const float v = row[c] * inv * gamma[c];
+        bad |= !isfinite(v);
+        row[c] = v;
+        u[size_t(r) * width + c] = v;
+    }
+    if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
+    lds_barrier();
+    emit_receipt(row, 0, width, r, rows, width, u_sums, threadIdx.x, threads);
 }
 
 int validate_model(const guffin_model_desc* m) {
@@ -262,14 +322,29 @@ int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t*
         depths = 0;
         for (uint32_t r = 0; r < rows; ++r) depths |= tree->depth[r] << (8 * r);
     }
-    launch(stage_rows_kernel, dim3((n_stage + 63) / 64), dim3(64), 0, stream, s.positions, s.ancestors,
-                       s.schedule, rows, position, depths, tree ? 0u : m.layer_count, m.sliding_window, m.global_period,
-                       reinterpret_cast<float2*>(s.rope_local), reinterpret_cast<float2*>(s.rope_global), m.head_dim,
-                       m.local_base, m.global_base, m.global_scale, s.sync, sync_words);
-    GUFFIN_TRY(check_launch("stage_rows"));
-    GUFFIN_TRY(guffin_hip_embed(st, m.embed_dtype, m.embed_rows, tokens, s.x, rows, H,
-                                std::sqrt(static_cast<float>(H)), m.vocab, status));
-    GUFFIN_TRY(guffin_hip_rms_norm(st, s.x, 1, 0, m.layers[0].norm[0], nullptr, s.u, s.us, rows, H, m.eps, status));
+    const Staging staging {s.positions, s.ancestors, s.schedule, rows, position, depths, tree ? 0u : m.layer_count, m.sliding_window,
+                           m.global_period, reinterpret_cast<float2*>(s.rope_local), reinterpret_cast<float2*>(s.rope_global), m.head_dim,
+                           m.local_base, m.global_base, m.global_scale, s.sync, sync_words};
+    const float scale = std::sqrt(static_cast<float>(H));
+    const float* gamma = m.layers[0].norm[0];
+    const uint32_t format = static_cast<uint32_t>(m.embed_dtype);
+    // the general operators take what the one launch does not (a row beyond 64 KB of LDS) and refuse what nothing takes
+    if (tokens && gamma && format <= uint32_t(GUFFIN_Q6_K) && H % (format == GUFFIN_Q8_0 ? 32u : 256u) == 0 && H <= 16128 && m.vocab != 0 && m.eps > 0.f
+        && ((reinterpret_cast<uintptr_t>(m.embed_rows) & 1u) | (reinterpret_cast<uintptr_t>(gamma) & 3u)) == 0) {
+        const uint32_t threads = std::min((H / 4 + 63) / 64 * 64, 1024u);
+        const dim3 grid(rows + (n_stage + threads - 1) / threads), block(threads);
+        const uint8_t* w = static_cast<const uint8_t*>(m.embed_rows);
+#define GUFFIN_ENTER(D_) launch(enter_rows_kernel<D_>, grid, block, H * 4, stream, tokens, w, gamma, H, scale, m.vocab, m.eps, rows, threads, s.x, s.u, s.us, \
+                                status, staging)
+        if (format == GUFFIN_Q8_0) GUFFIN_ENTER(GUFFIN_Q8_0); else if (format == GUFFIN_Q4_K) GUFFIN_ENTER(GUFFIN_Q4_K); else GUFFIN_ENTER(GUFFIN_Q6_K);
+#undef GUFFIN_ENTER
+        GUFFIN_TRY(check_launch("enter_rows"));
+    } else {
+        launch(stage_rows_kernel, dim3((n_stage + 63) / 64), dim3(64), 0, stream, staging);
+        GUFFIN_TRY(check_launch("stage_rows"));
+        GUFFIN_TRY(guffin_hip_embed(st, m.embed_dtype, m.embed_rows, tokens, s.x, rows, H, scale, m.vocab, status));
+        GUFFIN_TRY(guffin_hip_rms_norm(st, s.x, 1, 0, gamma, nullptr, s.u, s.us, rows, H, m.eps, status));
+    }
     if (resident && drafter_pass_fits(m))
         return drafter_pass(stream, m, rows, {s.exchange, s.sync, s.rope_local, s.rope_global, s.schedule, s.ancestors, priv_k, priv_v,
                                               s.x, s.u, out_hidden, out_hidden_sums, status});
