@@ -7,7 +7,7 @@
 // 16x16x32 instruction, whose 16 rows hold the 8 variants twice: lane (j, g) has the sums of rows 2 (g % 2) and + 1, columns
 // 32 (g / 2) + j and + 16.
 // Blocks of a 12B-shaped stack, four rows, with the operand staged in LDS for the 16x16x32 form / now / two launches of two rows
-// (us): q/k/v 8.7 / 8.4 / 14.3, o 4.8 / 5.7 / 9.1, gate + up 19.3 / 17.7 / 29.8, down 15.1 / 12.2 / 21.5.  (The block's multipliers
+// (us): q/k/v 8.7 / 8.4 / 14.3, o 4.8 / 5.7 / 9.1, gate + up 19.3 / 17.2 / 29.8, down 15.1 / 12.2 / 21.5.  (The block's multipliers
 // and sums brought to scalar registers ahead of the tile, which 64 to 96 words do not fit: down 14.1, q/k/v 11.2.)
 // Three rows leave the last pair of variants zero and its row unwritten.
 #include "common.hpp"
