@@ -140,7 +140,8 @@ gateup_wide_kernel(const uint8_t* __restrict__ gate_tiles, const uint8_t* __rest
         vals[i] = v;
     }
     lds_barrier();   // h is on its way out and nobody here reads it
-    if (wave < rows) emit_receipt(vals + wave * 64, blockIdx.x * kTileCols, kTileCols, wave, rows, F, h_receipt, lane, 64);
+    // a wave a row; a tile of one k-slice has two waves for up to four rows
+    for (uint32_t r = wave; r < rows; r += 2 * W) emit_receipt(vals + r * 64, blockIdx.x * kTileCols, kTileCols, r, rows, F, h_receipt, lane, 64);
 }
 
 __global__ void wide_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, uint32_t planes, uint32_t count) {

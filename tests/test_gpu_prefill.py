@@ -445,7 +445,7 @@ def test_prefill_rows_agree_with_decode_at_row_tile_edges(hip, kind, rows, posit
 
 @pytest.mark.parametrize("position", [0, 20, 95, 125, 200])
 @pytest.mark.parametrize("rows", [1, 2, 3, 4])
-@pytest.mark.parametrize("kind", ["target", "mixed", "drafter"])
+@pytest.mark.parametrize("kind", ["target", "mixed", "drafter", "one_slice"])
 def test_the_shortest_runs_agree_with_a_longer_one(hip, kind, rows, position):
     """Runs of up to four rows take the verify pass' products where the model allows: their hidden rows and ring rows are those
     of the first rows of a five-row run through the tiled GEMMs (2e-4 of the row RMS: fp32 sums in another order, and fp16 K/V
@@ -457,6 +457,8 @@ def test_the_shortest_runs_agree_with_a_longer_one(hip, kind, rows, position):
     shape = replace(base, layers=6, vocab=2048, ring_global=2048, ring_local=128, sliding_window=96)
     if kind == "mixed":
         shape = replace(shape, layer_dtypes=tuple(shape.dtypes if l % 2 == 0 else tuple(1 for _ in shape.dtypes) for l in range(6)))
+    elif kind == "one_slice":   # one block of K in gate + up
+        shape = replace(shape, hidden=256, ffn=512, q_heads=4, kv_heads=2)
     host = model.HostModel(shape, seed=31, position=position)
     short, long = model.DeviceModel.from_host(host), model.DeviceModel.from_host(host)
     tokens = dev(np.random.default_rng(23).integers(0, shape.vocab, 5).astype(np.int32))

@@ -258,7 +258,7 @@ def test_three_row_tree_against_the_oracle_and_every_path(hip, gfo):
 
 @pytest.mark.parametrize("position", [0, 5, 1023])
 @pytest.mark.parametrize("parents", [(None, 0, 0), (None, 0, 1, 0), (None, 0, 1, 2)])
-@pytest.mark.parametrize("kind", ["12b", "mixed", "q8_0", "one_head"])
+@pytest.mark.parametrize("kind", ["12b", "mixed", "q8_0", "one_head", "one_slice"])
 def test_a_tree_in_one_pass_equals_its_chains(hip, kind, parents, position):
     """Trees of 3 and 4 rows run as one pass over the wide products (Q4_K, Q6_K, both in a launch, Q8_0; ragged column groups and
     K slices) and the attention of 3 and 4 rows.  Every row's path from the root, taken as a chain of one-row passes over rings that
@@ -273,6 +273,8 @@ def test_a_tree_in_one_pass_equals_its_chains(hip, kind, parents, position):
         shape = replace(shape, hidden=640, ffn=1088, q_heads=4, kv_heads=2, dtypes=(synth.Q8_0,) * 7, embed_dtype=synth.Q8_0)
     elif kind == "one_head":   # one query head per KV head
         shape = replace(shape, hidden=512, ffn=768, q_heads=4, kv_heads=4)
+    elif kind == "one_slice":   # one block of K: gate + up in two waves, for three and four rows
+        shape = replace(shape, hidden=256, ffn=512, q_heads=4, kv_heads=2)
     host = model.HostModel(shape, seed=9, position=position, untied_head=True)
     target = model.DeviceModel.from_host(host)
     ticket = model.VerifyTicket(target, position + 4)
