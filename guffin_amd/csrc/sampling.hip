@@ -694,7 +694,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
             const uint64_t mine = sc.sorted[t];
             below = __fsub_rn(key_score(mine), key_score(sc.sorted[0]));
             out.token[t] = key_token(mine);
-            w = exp(static_cast<double>(below));
+            w = opt.temperature == 0.f ? 1.0 : exp(static_cast<double>(below));   // greedy: one, also where the penalty made the best infinite
         }
         sc.w[t] = w;
     }

@@ -77,6 +77,18 @@ def greedy_cases():
     return out
 
 
+def greedy_overflow_cases():
+    """A greedy target's law is its first candidate with weight one (part of src/engine/sampling.cpp:394-499), also where the repetition
+    penalty takes logits beyond the float range: +inf ahead of a finite one, or -inf for all."""
+    out = []
+    for proposal in (3, 7):
+        for row, history, penalty in (([(3, 3e38), (7, 0.0), (3, 3e38)], [3], 0.5), ([(3, 3e38), (7, 3e38)], [3, 7], 0.25),
+                                      ([(3, -3e38), (7, -3e38)], [3, 7], 2.0)):
+            out.append(dict(rows=[row] * 2, history=[history] * 2, law=[(proposal, TOTAL)], proposal=proposal,
+                            options=(0.0, 2, 1.0, 0.0, penalty), draws=(0.5, 0.5, 0.5), want=(int(proposal == 3), 3)))
+    return out
+
+
 def unit_bin_cases():
     """:550-578: 256 target tokens of equal weight against one-word q bins (acceptance 1, all 256 in the residual,
     total 1 - 256 / 2^32), and a 2^32-mass delta (acceptance 1, no residual)."""

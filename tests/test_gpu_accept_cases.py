@@ -57,10 +57,10 @@ def same(got, want):
     assert int(got["residual_count"]) == want.residual_count
 
 
-@pytest.mark.parametrize("family", ["transforms", "greedy", "unit_bins", "rollback"])
+@pytest.mark.parametrize("family", ["transforms", "greedy", "greedy_overflow", "unit_bins", "rollback"])
 def test_reference_cases_equal_the_oracle(hip, gfo, family):
-    todo = {"transforms": cases.transform_cases, "greedy": cases.greedy_cases, "unit_bins": cases.unit_bin_cases,
-            "rollback": cases.rollback_cases}[family]()
+    todo = {"transforms": cases.transform_cases, "greedy": cases.greedy_cases, "greedy_overflow": cases.greedy_overflow_cases,
+            "unit_bins": cases.unit_bin_cases, "rollback": cases.rollback_cases}[family]()
     for case in todo:
         rc, want = oracle_run(gfo, case)
         got, status = device_run(hip, case)

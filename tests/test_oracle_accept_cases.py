@@ -20,10 +20,10 @@ def run(gfo, case):
                                    ua, ur, un)
 
 
-@pytest.mark.parametrize("family", ["transforms", "greedy", "unit_bins", "rollback"])
+@pytest.mark.parametrize("family", ["transforms", "greedy", "greedy_overflow", "unit_bins", "rollback"])
 def test_reference_cases_decide_as_the_reference_expects(gfo, family):
-    todo = {"transforms": cases.transform_cases, "greedy": cases.greedy_cases, "unit_bins": cases.unit_bin_cases,
-            "rollback": cases.rollback_cases}[family]()
+    todo = {"transforms": cases.transform_cases, "greedy": cases.greedy_cases, "greedy_overflow": cases.greedy_overflow_cases,
+            "unit_bins": cases.unit_bin_cases, "rollback": cases.rollback_cases}[family]()
     accepted = 0
     for case in todo:
         rc, got = run(gfo, case)
