@@ -300,26 +300,29 @@ topk_merge_kernel(const float* __restrict__ logits, const uint64_t* __restrict__
 // maximum is at or below the retain-th largest logit of the row, so only logits at or above it can be
 // selected, and on anything but massively tied rows they are few more than `retain`.  Two launches:
 //   segment_max_kernel       the ordered score bits of every segment's maximum; clears the row's counters
-//   threshold_select_kernel  (`sure` != 0: the best `sure` logits and every tie with the last of them are all the caller
-//                            needs, and as many of the following, up to `retain`, as come with the bound for those.)  Every workgroup finds the bound for itself (a radix select over at most 1024
+//   threshold_select_kernel  every workgroup finds the bound for itself (a radix select over at most 1024
 //                            words that stops as soon as few maxima lie between it and the exact one),
 //                            collects the keys of its 4096 logits that reach it, and the workgroup that
 //                            finishes last sorts all of them and writes the row
-// What bounds the second is the chain of trips to memory behind one another (the workgroups sit on different
+// A caller that needs the best `sure` logits and every tie with the last of them, and as many of the following
+// (up to `retain`) as come with these, passes `sure` != 0: the bound is then the one for `sure`.
+// What bounds the second launch is the chain of trips to memory behind one another (the workgroups sit on different
 // L2s, so what they exchange moves with device-scope accesses).  A workgroup therefore has places of its own
 // for kSlots keys and its count, stored without asking anybody; only what does not fit goes through a
 // reservation in the row's common list, and the last workgroup asks for counts and places at once.  Its
 // logits lie 64 apart from its neighbours', so that a run of equal or large ones is dealt to all.  Every
 // workgroup waits for its own stores before it counts itself done, and nobody waits for anybody: the last
-// arrival is whoever draws the last ticket.  A row whose common list overflows, or with more than kCollectCap
-// keys, is selected exactly, and slowly, by a radix select over the whole row in that workgroup.
+// arrival is whoever draws the last ticket.  Up to kCollectCap keys of a row are sorted in LDS, however they
+// lie: the common list holds what the places of a single collector leave of that many.  A row with more is
+// selected exactly, and slowly, by a radix select over the whole row in that workgroup.
 // 262144 logits: 64 of two rows 9.5 us (10.6 with an exact bound and every key through one reservation), what a compact law
-// of 64 needs of one row 9.5 (15.4 with its best 257 in order).
+// of 64 needs of one row 9.5 (15.4 with its best 257 in order).  Ties, both launches and the call: 300 to 2000 keys 18 to 29 us,
+// beyond 2048 keys 1015.
 constexpr uint32_t kSeg = 256, kMaxSegs = 1024, kCollectTile = 4096, kCollectCap = 2048;
-constexpr uint32_t kMaxCollectors = kMaxSegs * kSeg / kCollectTile, kSlots = 16;
+constexpr uint32_t kMaxCollectors = kMaxSegs * kSeg / kCollectTile, kSlots = 16, kCommonCap = kCollectCap - kSlots;
 // segment maxima; common list's length, workgroups done, pad; the workgroups' counts, their places, the common list
-constexpr uint32_t kThresholdRowWords = kMaxSegs + 4 + 2 * kCollectCap;
-constexpr uint32_t kCommonCap = kCollectCap - kMaxCollectors / 2 - kMaxCollectors * kSlots;
+constexpr uint32_t kThresholdRowWords = kMaxSegs + 4 + kMaxCollectors + 2 * (kMaxCollectors * kSlots + kCommonCap);
+static_assert((kMaxSegs + 4 + kMaxCollectors) % 2 == 0 && kThresholdRowWords % 2 == 0, "keys on 8 bytes");
 static_assert(kMaxCollectors == 64, "a wave scans the workgroups' counts");
 
 __device__ __forceinline__ uint32_t ordered_bits(float v) {
@@ -467,7 +470,7 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t* __restrict__
     const uint32_t n = __builtin_amdgcn_readlane(all, 63), placed = __builtin_amdgcn_readlane(upto, 63);
     const uint32_t own_kept = __shfl(kept, owner, kWave), own_upto = __shfl(upto, owner, kWave);
     static_assert(kMaxCollectors * kSlots == 1024, "a place per thread");
-    if (n <= kCollectCap && n - placed <= kCommonCap) {
+    if (n <= kCollectCap) {
         if (tid % kSlots < own_kept) sel[own_upto - own_kept + tid % kSlots] = place;
         for (uint32_t i = tid; i < n - placed; i += 1024) sel[placed + i] = shared_load(common + i);
         if (n <= 512) {

@@ -1,5 +1,5 @@
-"""Selection against a bound, where its stages change over: keys past a collector's own places, past the row's common list
-(992 keys) and past what is sorted in LDS (2048), ties across the last place, zeros of both signs, and results in memory that
+"""Selection against a bound, where its stages change over: keys past a collector's own places, past what is ranked (512) and
+past what is sorted in LDS (2048), ties across the last place, zeros of both signs, and results in memory that
 held something else.  The order (logit descending, token ascending) is exact, so the oracle is a stable sort on the host."""
 import numpy as np
 import pytest
@@ -35,7 +35,7 @@ def rows_of(kind, vocab, rng):
 
 @pytest.mark.parametrize("vocab", [32768, 131585, 262144])
 @pytest.mark.parametrize("retain", [1, 17, 64])
-@pytest.mark.parametrize("kind", ["normal", "narrow", "zeros", "run15", "run300", "run1100", "run2049", "spread1023", "spread1100", "spread2500"])
+@pytest.mark.parametrize("kind", ["normal", "narrow", "zeros", "run15", "run300", "run1100", "run1500", "run1900", "run2049", "spread1023", "spread1100", "spread2030", "spread2500"])
 def test_selection_is_a_stable_sort(kind, retain, vocab):
     x = rows_of(kind, vocab, np.random.default_rng(retain + vocab))
     junk = torch.full((1 << 20,), 0x5A, dtype=torch.uint8, device="cuda")   # what the next buffers may be cut from
@@ -50,6 +50,25 @@ def test_selection_is_a_stable_sort(kind, retain, vocab):
         assert np.array_equal(values["token"][:retain], want.astype(np.uint32))
         assert np.array_equal(values["logit"][:retain].view(np.uint32), x[r][want].view(np.uint32))   # a zero's sign too
         assert not values["token"][retain:].any() and not values["logit"][retain:].view(np.uint32).any()
+
+
+@pytest.mark.parametrize("kind", ["run1500", "run1900", "spread2030"])
+def test_ties_up_to_what_lds_sorts_cost_no_walk_over_the_row(kind):
+    """Up to 2048 keys are sorted in LDS wherever they lie.  The walk that selects from more passes over the whole row eight times
+    in one workgroup, 35 times the whole call's time of 1000 ties (1015 us against 28); four times is between them."""
+    def time_of(kind):
+        x = torch.from_numpy(rows_of(kind, 262144, np.random.default_rng(5))).cuda()
+        best = float("inf")
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                hip.select_candidates(x, 64)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+    assert time_of(kind) <= 4 * time_of("run1000")
 
 
 @pytest.mark.parametrize("top_k", [1, 5, 64])
