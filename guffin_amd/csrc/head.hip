@@ -84,12 +84,13 @@ struct Candidates {  // layout of one row of the result (sampling.hpp:57-61 plus
 };
 
 // Adds one to hist[bin] for every lane with `valid`; lanes of a wave that hit the same bin are
-// counted with one atomic (keys cluster in a few bins, and same-address LDS atomics serialise).
+// counted with one atomic (keys cluster in a few bins, and same-address LDS atomics serialise).  (The leader's bin read into a
+// scalar register instead: 9.5 us for the 8.8 of threshold_select_kernel, 1018 for the 920 of its walk over a whole row.)
 __device__ __forceinline__ void hist_add(uint32_t* hist, bool valid, uint32_t bin, uint32_t lane) {
     uint64_t todo = __ballot(valid);
     for (int it = 0; it < 8 && todo; ++it) {
         const int leader = __ffsll(static_cast<long long>(todo)) - 1;
-        const uint32_t b0 = __builtin_amdgcn_readlane(bin, leader);
+        const uint32_t b0 = __shfl(bin, leader, kWave);
         const uint64_t same = __ballot(valid && bin == b0) & todo;
         if (lane == uint32_t(leader)) atomicAdd(&hist[b0], static_cast<uint32_t>(__popcll(same)));
         todo &= ~same;
@@ -315,9 +316,9 @@ topk_merge_kernel(const float* __restrict__ logits, const uint64_t* __restrict__
 // arrival is whoever draws the last ticket.  Up to kCollectCap keys of a row are sorted in LDS, however they
 // lie: the common list holds what the places of a single collector leave of that many.  A row with more is
 // selected exactly, and slowly, by a radix select over the whole row in that workgroup.
-// 262144 logits: 64 of two rows 9.5 us (10.6 with an exact bound and every key through one reservation), what a compact law
-// of 64 needs of one row 9.5 (15.4 with its best 257 in order).  Ties, both launches and the call: 300 to 2000 keys 18 to 29 us,
-// beyond 2048 keys 1015.
+// 262144 logits: 64 of two rows 8.8 us (10.6 with an exact bound and every key through one reservation), what a compact law
+// of 64 needs of one row 8.8 (15.4 with its best 257 in order).  Ties, both launches and the call: 300 to 2000 keys 18 to 29 us,
+// beyond 2048 keys 920.
 constexpr uint32_t kSeg = 256, kMaxSegs = 1024, kCollectTile = 4096, kCollectCap = 2048;
 constexpr uint32_t kMaxCollectors = kMaxSegs * kSeg / kCollectTile, kSlots = 16, kCommonCap = kCollectCap - kSlots;
 // segment maxima; common list's length, workgroups done, pad; the workgroups' counts, their places, the common list
