@@ -524,16 +524,6 @@ int launch_partial(hipStream_t s, const AttnArgs& a) {
     const uint32_t cut = a.tp / 16 | a.span / 16 << 5 | cap << 10 | std::min(a.partitions, 0xFFFFu) << 16;
     const uint32_t form = a.kv_heads | std::min(a.planes, 0x7FFFu) << 16 | a.inline_schedule << 31;
     const size_t lds = (size_t(NQ) * a.span + size_t(kAW) * NQ * 256 + (fused ? size_t(NQ) * 256 : 0)) * sizeof(float);
-    if constexpr (kAW * NQ * 256 * sizeof(float) >= 64 * 1024) {   // more than a launch gets unasked, allowed once per kernel
-        static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_partial_kernel<ROWS, GROUP, 256, true>),
-                                                              hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-        if (allowed != hipSuccess || lds > 96 * 1024) return fail(GUFFIN_E_HIP, "attention_partial: could not raise the dynamic LDS limit");
-    }
-    if constexpr (kAW * NQ * 256 * sizeof(float) >= 64 * 1024 && ROWS <= 2) {
-        static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_partial_kernel<ROWS, GROUP, 256, false>),
-                                                              hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-        if (allowed != hipSuccess) return fail(GUFFIN_E_HIP, "attention_partial: could not raise the dynamic LDS limit");
-    }
     if (fused || ROWS > 2)
         launch((attn_partial_kernel<ROWS, GROUP, 256, true>), dim3(a.partitions, a.kv_heads), dim3(64 * kAW), lds, s, a.ring_k, a.q_raw, a.q_norm,
                a.rope, a.q_stride, first, ring, cut, form, a);
@@ -544,6 +534,14 @@ int launch_partial(hipStream_t s, const AttnArgs& a) {
 }
 
 }  // namespace
+
+// Eight queries take 73 to 81 KB a workgroup.
+int attention_init() {
+    constexpr uint32_t kLds = 96 * 1024;
+    const bool allowed = allow_lds(attn_partial_kernel<4, 2, 256, true>, kLds) && allow_lds(attn_partial_kernel<2, 4, 256, true>, kLds)
+        && allow_lds(attn_partial_kernel<2, 4, 256, false>, kLds);
+    return allowed ? 0 : -1;
+}
 }  // namespace guffin
 
 using namespace guffin;

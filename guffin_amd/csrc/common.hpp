@@ -15,6 +15,13 @@ void set_last_error(const char* message);
 int fail(int code, const char* message);
 int check_launch(const char* what);
 
+// Lets `kernel` ask for more than 64 KB of dynamic LDS on the current device.  The permission is a device's own, so this runs in
+// the init functions that guffin_hip_init calls, once per device, and nowhere else.
+template <typename Kernel>
+inline bool allow_lds(Kernel* kernel, uint32_t bytes) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)) == hipSuccess;
+}
+
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 // Layer policy of src/engine/model.cpp:607-610: with a period above one, every layer but the last of

@@ -31,6 +31,8 @@ int gemv_init(int cu_count);
 int ops_init(int cu_count);
 int gemv_packed_init(int device, int cu_count);
 int head_init();
+int attention_init();
+int prefill_attention_init();
 
 }  // namespace guffin
 
@@ -53,9 +55,9 @@ extern "C" int guffin_hip_init(int device) {
         std::snprintf(buf, sizeof(buf), "init: code object is gfx950 only, device is %s", prop.gcnArchName);
         return fail(GUFFIN_E_HIP, buf);
     }
-    if (gemv_init(prop.multiProcessorCount) != 0 || ops_init(prop.multiProcessorCount) != 0 || head_init() != 0)
+    if (gemv_init(prop.multiProcessorCount) != 0 || ops_init(prop.multiProcessorCount) != 0 || head_init() != 0
+        || attention_init() != 0 || prefill_attention_init() != 0 || resident_init(prop.multiProcessorCount) != 0)
         return fail(GUFFIN_E_HIP, "init: could not raise a kernel's dynamic LDS limit");
-    resident_init(prop.multiProcessorCount);
     if (gemv_packed_init(device, prop.multiProcessorCount) != 0)
         return fail(GUFFIN_E_HIP, "init: could not take the address of the static scratch array on this device");
     return GUFFIN_OK;

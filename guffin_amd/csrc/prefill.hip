@@ -677,12 +677,6 @@ AttentionCut attention_cut(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_
     // parts 16.4 us, in nine 14.4; a second part costs the launch that merges them, more than a second round)
     return {1, std::max(1u, std::min(2 * cus / ones, T < 256 ? 1 : (T + 127) / 128))};
 }
-// more than 64 KB of LDS a workgroup has to be allowed once per kernel
-int allow_attention_lds() {
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_attention_mfma_kernel<1>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, attention_lds(1));
-    return allowed == hipSuccess ? GUFFIN_OK : fail(GUFFIN_E_HIP, "prefill_attention: could not raise the dynamic LDS limit");
-}
 uint64_t transposed_bytes(uint32_t T, uint32_t kv_heads) { return (uint64_t(kv_heads) * 256 * T * 2 + 255) & ~uint64_t{255}; }
 }  // namespace
 
@@ -700,6 +694,8 @@ extern "C" uint64_t guffin_hip_prefill_attention_workspace_bytes(uint32_t rows, 
 }
 
 namespace guffin {
+int prefill_attention_init() { return allow_lds(prefill_attention_mfma_kernel<1>, attention_lds(1)) ? 0 : -1; }
+
 bool prefill_attention_on_matrix_core(const void* q, const void* ring_k, const void* ring_v, const void* run_k, const void* run_v,
                                       uint32_t q_heads, uint32_t kv_heads) {
     const uint32_t group = q_heads / kv_heads;
@@ -723,7 +719,6 @@ int prefill_attention_run(hipStream_t s, const float* q, const void* ring_k, con
     float* states = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + transposed_bytes(vs.T, kv_heads));
     const AttentionOut to {out, image, states, states + size_t(parts) * rows * q_heads * 256};
     const uint32_t lds = attention_lds(nt);
-    if (int rc = allow_attention_lds()) return rc;
     const dim3 grid((rows * group + 16 * nt - 1) / (16 * nt), kv_heads, parts);
     const uint32_t form = kv_heads | (shift << 16) | (parts << 18);   // at most two parts a compute unit
 #define GUFFIN_PA(NT_) launch(prefill_attention_mfma_kernel<NT_>, grid, dim3(256), lds, s, q, static_cast<const uint16_t*>(ring_k), \

@@ -944,11 +944,6 @@ int g_device_cus = 0;          // CU count of the device guffin_hip_init saw (0:
 bool g_resident_off = false;   // a pass gave up a wait: the automatic mode uses one launch per operator from then on
 }  // namespace
 
-int resident_init(int cu_count) {
-    g_device_cus = cu_count;
-    return 0;
-}
-
 void resident_note_status(uint32_t status_word) {
     if (status_word & GUFFIN_STATUS_SYNC) g_resident_off = true;
 }
@@ -1054,16 +1049,20 @@ uint32_t resident_sync_words(const guffin_model_desc& m) {
     return ((m.layer_count + kResidentLayers - 1) / kResidentLayers) * kSyncWords;
 }
 
+template <int R, int G>
+static bool allow_resident() {
+    return allow_lds(resident_blocks_kernel<R, G, false>, 140 * 1024) && allow_lds(resident_blocks_kernel<R, G, true>, 140 * 1024);
+}
+int resident_init(int cu_count) {
+    g_device_cus = cu_count;
+    const bool allowed = allow_resident<1, 1>() && allow_resident<1, 2>() && allow_resident<1, 4>() && allow_resident<2, 1>()
+        && allow_resident<2, 2>() && allow_resident<2, 4>();
+    return allowed ? 0 : -1;
+}
+
 template <int R, int G, bool KQ>
 static int launch_resident(hipStream_t stream, const RArgs& args, uint32_t lds) {
-    static bool raised = false;
-    auto* kernel = resident_blocks_kernel<R, G, KQ>;
-    if (!raised) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 140 * 1024) != hipSuccess)
-            return fail(GUFFIN_E_HIP, "resident forward: could not raise the dynamic LDS limit");
-        raised = true;
-    }
-    launch(kernel, dim3(kGrid), dim3(kThreads), lds, stream, args);
+    launch((resident_blocks_kernel<R, G, KQ>), dim3(kGrid), dim3(kThreads), lds, stream, args);
     return check_launch("resident_blocks");
 }
 
