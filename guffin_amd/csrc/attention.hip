@@ -116,11 +116,11 @@ __device__ __forceinline__ float dot2(float acc, uint32_t packed_half2, float a,
     return fmaf(static_cast<float>(h.y), b, acc);
 }
 
-// waves of a partition's workgroup: two per SIMD.  With eight the queries and the private rows' key / value are
-// prepared by different waves, and a 32-token partition is one round of keys and two of values per wave.
-// (Sixteen queries keep four waves: their per-wave output slots would take all of the LDS otherwise.  Eight take 73-81 KB, for
-// one workgroup on a compute unit as it is; with four waves a local layer of four rows took 15.4 us instead of 9.4.)
-constexpr int attention_waves(int queries) { return queries <= 8 ? 8 : 4; }
+// waves of a partition's workgroup: two per SIMD.  The queries and the private rows' key / value are prepared by
+// different waves, and a 32-token partition is one round of keys and two of values per wave.  (Eight queries take
+// 73-81 KB of LDS, for one workgroup on a compute unit as it is; with four waves a local layer of four rows took 15.4 us
+// instead of 9.4.)
+constexpr int kAW = 8;
 
 // Where a dimension lies among the 256 floats of a query in LDS: a lane reads dimensions 8 seg .. 8 seg + 7 of each half of the
 // row in four pieces of 16 bytes, and a piece of 16 lanes is 256 bytes without a gap (in the row's own order, every other 16
@@ -131,14 +131,15 @@ __device__ __forceinline__ uint32_t query_place(uint32_t d) {
 }
 
 template <int ROWS, int GROUP, int HD, bool FUSED>
-__global__ void __launch_bounds__(64 * attention_waves(ROWS * GROUP)) attn_partial_kernel(const uint16_t* __restrict__ ring_k, const float* __restrict__ q_raw, const float* __restrict__ q_norm,
-                                                                                const float2* __restrict__ rope, size_t q_stride, uint32_t host_first,
-                                                                                uint32_t host_ring, uint32_t cut, uint32_t form, AttnArgs a) {
+__global__ void __launch_bounds__(64 * kAW)
+attn_partial_kernel(const uint16_t* __restrict__ ring_k, const float* __restrict__ q_raw, const float* __restrict__ q_norm,
+                    const float2* __restrict__ rope, size_t q_stride, uint32_t host_first, uint32_t host_ring, uint32_t cut,
+                    uint32_t form, AttnArgs a) {
     // What the first requests need comes in words of its own, in registers when a wave starts (see the kernels of
     // gemv_packed.hip); the struct is a trip away.
     static_assert(HD == 256, "head dimension 256 (16 lanes x 16 dims)");
     constexpr int NQ = ROWS * GROUP;
-    constexpr int kAW = attention_waves(NQ);
+    static_assert(NQ <= kAW, "a wave's output slots for every query fit the LDS");
     const uint32_t tp = 16 * (cut & 31u), span = 16 * ((cut >> 5) & 31u);
     extern __shared__ float lds[];
     float* sc = lds;                          // [NQ][tp] scores, then probabilities
@@ -511,7 +512,6 @@ attn_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ 
 template <int ROWS, int GROUP>
 int launch_partial(hipStream_t s, const AttnArgs& a) {
     constexpr int NQ = ROWS * GROUP;
-    constexpr int kAW = attention_waves(NQ);
     const bool fused = a.q_raw != nullptr;
     if (a.kv_heads > 0xFFFFu) return fail(GUFFIN_E_SHAPE, "attention_decode: more KV heads than a grid has rows");
     uint32_t first = 0xFFFFFFFFu, end = 0;   // of the rows' token lists together, where they are known here

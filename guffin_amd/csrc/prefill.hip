@@ -417,13 +417,13 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         for (uint32_t w = 0; w < 4; ++w) {
             __syncthreads();
             if (wave != w) continue;
-    #pragma unroll
+#pragma unroll
             for (int g = 0; g < NT; ++g)
-    #pragma unroll
+#pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     float* slots = ob + (g * 64 + r) * 64 + lane;   // [dt][4][64]
                     if (w == 0) {
-    #pragma unroll
+#pragma unroll
                         for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r];
                         continue;
                     }
@@ -432,16 +432,16 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
                     const float mine = m[g][r] == -INFINITY ? 0.f : exp_of(m[g][r] - M), theirs = mo == -INFINITY ? 0.f : exp_of(mo - M);
                     l[g][r] = l[g][r] * mine + lo_ * theirs;
                     m[g][r] = M;
-    #pragma unroll
+#pragma unroll
                     for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r] * mine + slots[dt * 256] * theirs;
                 }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             if (j == 0) {
-    #pragma unroll
+#pragma unroll
                 for (int g = 0; g < NT; ++g)
-    #pragma unroll
+#pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         ml[(g * 16 + 4 * lg + r) * 2] = m[g][r];
                         ml[(g * 16 + 4 * lg + r) * 2 + 1] = l[g][r];
