@@ -31,7 +31,17 @@ def rel_rms(got, want):
 
 
 CASES = [("drafter", 3, 1, 700), ("drafter", 7, 2, 5), ("drafter", 2, 1, 0), ("drafter", 6, 1, 4000),
-         ("target", 2, 2, 1500), ("target", 7, 2, 40), ("target", 2, 1, 0), ("target", 6, 2, 2046)]
+         ("target", 2, 2, 1500), ("target", 7, 2, 40), ("target", 2, 1, 0), ("target", 6, 2, 2046),
+         # one KV head outside what drafter_pass.hip covers (the "drafter" cases above are its): wider Q8_0 blocks, K-quants
+         ("wide", 3, 1, 700), ("wide", 7, 2, 5), ("wide", 2, 1, 0), ("wide", 6, 1, 4000), ("wide", 7, 2, 1400),
+         ("kquant", 2, 1, 0), ("kquant", 7, 2, 700), ("kquant", 3, 2, 1500), ("kquant", 6, 1, 2046)]
+
+
+def one_head(kind, layers, ring_global):
+    from guffin_amd import model
+    if kind == "wide":
+        return replace(model.GEMMA3_270M, layers=layers, vocab=4096, ring_global=ring_global, hidden=768, ffn=2304)
+    return replace(model.GEMMA3_12B, layers=layers, vocab=2048, ring_global=ring_global, hidden=1024, ffn=2048, q_heads=4, kv_heads=1)
 
 
 @pytest.mark.parametrize("kind,layers,rows,position", CASES)
@@ -40,6 +50,8 @@ def test_resident_pass_equals_the_per_operator_pass(hip, gfo, kind, layers, rows
     from guffin_amd import model
     if kind == "drafter":
         shape = replace(model.GEMMA3_270M, layers=layers, vocab=4096, ring_global=4096)
+    elif kind in ("wide", "kquant"):
+        shape = one_head(kind, layers, 4096)
     else:
         shape = replace(model.GEMMA3_12B, layers=layers, vocab=2048, ring_global=2048)
     host = model.HostModel(shape, seed=3 + layers, position=position)
@@ -69,10 +81,11 @@ def test_resident_pass_equals_the_per_operator_pass(hip, gfo, kind, layers, rows
     assert rel_rms(got[0].cpu().numpy(), oracle) <= 1e-3
 
 
-def test_a_wait_that_gives_up_raises_the_status_bit_and_the_launch_ends(hip):
+@pytest.mark.parametrize("kind", ["drafter", "wide"])
+def test_a_wait_that_gives_up_raises_the_status_bit_and_the_launch_ends(hip, kind):
     import torch
     from guffin_amd import model
-    shape = replace(model.GEMMA3_270M, layers=2, vocab=4096, ring_global=1024)
+    shape = one_head(kind, 2, 1024) if kind == "wide" else replace(model.GEMMA3_270M, layers=2, vocab=4096, ring_global=1024)
     devm = model.DeviceModel.from_host(model.HostModel(shape, seed=9, position=100))
     tokens = torch.tensor([5], dtype=torch.int32, device="cuda")
     hip.set_forward_mode(2)

@@ -1,6 +1,8 @@
 """Selection against a bound, where its stages change over: keys past a collector's own places, past what is ranked (512) and
 past what is sorted in LDS (2048), ties across the last place, zeros of both signs, and results in memory that
 held something else.  The order (logit descending, token ascending) is exact, so the oracle is a stable sort on the host."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -90,3 +92,51 @@ def test_the_law_holds_every_tie_with_the_last_place(ties, top_k):
         assert np.array_equal(law["ids"][:n], np.sort(np.flatnonzero(x >= x[order[top_k - 1]])).astype(np.uint32))
         assert int(law["cdf"][0]) == 0 and int(law["cdf"][n]) == 1 << 32
         assert not law["ids"][n:].any() and not law["cdf"][n + 1:].any()
+
+
+def dirty(nbytes):
+    return torch.full((nbytes,), 0x5A, dtype=torch.uint8, device="cuda")
+
+
+@pytest.mark.parametrize("vocab", [64, 5000, 32768, 262144])   # sorted tiles (two merges), then a bound
+@pytest.mark.parametrize("retain", [1, 64])
+def test_fresh_selection_clears_what_it_does_not_write(vocab, retain):
+    """Memory that held something else: status starts from 0, and every unused word of a row's record is zero."""
+    x = np.random.default_rng(vocab).standard_normal((2, vocab)).astype(np.float32)
+    logits, lib = torch.from_numpy(x).cuda(), hip.lib()
+    result, status = dirty(2 * hip.candidates_dtype.itemsize), dirty(8)
+    workspace = dirty(int(lib.guffin_hip_select_workspace_bytes(2, vocab, retain)))
+    history, counts = torch.tensor([[7] + [0] * 63, [0] * 64], dtype=torch.int32, device="cuda"), torch.tensor([1, 0], dtype=torch.int32, device="cuda")
+    hip.check(lib.guffin_hip_select_candidates_fresh(hip._stream(), hip._p(logits), 2, vocab, retain, hip._p(history), hip._p(counts),
+                                                     hip._p(workspace), hip._p(result), hip._p(status)))
+    got = hip.candidates_to_numpy(result)
+    assert status.view(torch.int32).cpu().tolist() == [0, 0]
+    for r, extra in ((0, [7]), (1, [])):
+        values, used = got[r]["values"], retain + len(extra)
+        want = np.argsort(-x[r], kind="stable")[:retain].tolist() + extra
+        assert (int(got[r]["count"]), int(got[r]["status"])) == (used, 0)
+        assert values["token"][:used].tolist() == want
+        assert not values["token"][used:].any() and not values["logit"][used:].view(np.uint32).any()
+
+
+@pytest.mark.parametrize("ties", [0, 300])   # a law of top_k, and one that more ties than it holds refuse
+@pytest.mark.parametrize("vocab", [5000, 262144])
+def test_a_fresh_law_clears_what_it_does_not_write(vocab, ties):
+    x = np.random.default_rng(ties).standard_normal(vocab).astype(np.float32)
+    order = np.argsort(-x, kind="stable")
+    x[order[4:5 + ties]] = x[order[4]]
+    logits, lib = torch.from_numpy(x).cuda(), hip.lib()
+    options = hip.SamplerOptions(1.0, 5, 1.0, 0.0, 1.0)
+    law, proposal, status = dirty(hip.law_dtype.itemsize), dirty(4), dirty(4)
+    workspace = dirty(int(lib.guffin_hip_draft_law_workspace_bytes(vocab)))
+    hip.check(lib.guffin_hip_draft_law_fresh(hip._stream(), hip._p(logits), vocab, C.byref(options), C.c_uint64(3), C.c_uint64(1), None,
+                                             hip._p(workspace), hip._p(law), hip._p(proposal), hip._p(status)))
+    got = law.cpu().numpy().view(hip.law_dtype)[0]
+    n = 0 if ties else 5
+    assert (int(got["count"]), int(got["pad"])) == (n, 0)
+    assert not got["ids"][n:].any() and not got["cdf"][(n + 1 if n else 0):].any()
+    status = int(status.view(torch.int32).item())
+    if ties:
+        assert status == 48 and proposal.view(torch.int32).item() == -1   # refused, more than fit, and nothing else
+    else:
+        assert status == 0 and proposal.view(torch.int32).item() in order[:5].tolist()
