@@ -927,14 +927,17 @@ __global__ void __launch_bounds__(kThreads) drafter_blocks_kernel(const DArgs a)
 
 }  // namespace
 
-// Widths whose tiles a workgroup's waves hold: three blocks of the hidden width a worker, a gate / up pair a workgroup.
+// Widths whose tiles a workgroup's waves hold: three blocks of the hidden width a worker, a gate / up pair a workgroup.  Heads are
+// normalised here always: a model without head norms (null gammas) is the general resident pass's.
 bool drafter_pass_fits(const guffin_model_desc& m) {
     if (m.kv_heads != 1 || m.head_dim != kHd || (m.q_heads != 1 && m.q_heads != 2 && m.q_heads != 4)) return false;
     if (uint64_t(std::max(m.ring_local, m.ring_global)) * 2 * kHd >= (uint64_t(1) << 31)) return false;   // 32-bit offsets into a ring
     if (m.hidden % 64 || m.hidden > kMaxWidth || m.ffn % 64 || m.ffn > kMaxFfn) return false;
-    for (uint32_t l = 0; l < m.layer_count; ++l)
+    for (uint32_t l = 0; l < m.layer_count; ++l) {
+        if (!m.layers[l].norm[1] || !m.layers[l].norm[2]) return false;
         for (int i = 0; i < 7; ++i)
             if (m.layers[l].dtype[i] != GUFFIN_Q8_0) return false;
+    }
     return true;
 }
 

@@ -90,3 +90,25 @@ def test_a_row_keeps_a_nan_and_says_so(hip):
         assert not bool(torch.isfinite(out[0]).any())
     hip.set_forward_mode(0)
     assert words[0] != 0 and words[0] == words[1]
+
+
+@pytest.mark.parametrize("rows", [1, 2])
+def test_a_model_without_head_norms(hip, rows):
+    """Null gammas leave the head norms out, also on the widths of the drafter's own pass."""
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=2, vocab=1024, ring_global=1024, global_period=2)
+    devm = model.DeviceModel.from_host(model.HostModel(shape, seed=4, position=300))
+    tokens = torch.tensor([17, 999][:rows], dtype=torch.int32, device="cuda")
+    normed = devm.forward(tokens, 300)[0].cpu().numpy()
+    for l in range(shape.layers):
+        devm.layers[l].norm[1] = devm.layers[l].norm[2] = None
+    out = []
+    for mode in (1, 0):
+        hip.set_forward_mode(mode)
+        got = devm.forward(tokens, 300)
+        torch.cuda.synchronize()
+        assert int(got[4].item()) == 0
+        out.append(got[0].cpu().numpy())
+    hip.set_forward_mode(0)
+    assert rel_rms(out[1], out[0]) <= 1e-4 and rel_rms(out[0], normed) > 1e-2
