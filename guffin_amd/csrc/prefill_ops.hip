@@ -190,7 +190,11 @@ prefill_qkv_kernel(const float* __restrict__ q_planes, const float* __restrict__
         const float* gamma = is_q ? a.q_norm : a.k_norm;
         // lane: columns 2 lane, 2 lane + 1 of either half, the pairs that rotate together
         const float4 rot = reinterpret_cast<const float4*>(a.rope_table)[size_t(r) * (HD / 4) + lane];   // cos, sin of two pairs
-        const float2 g0 = make_float2(gamma[2 * lane], gamma[2 * lane + 1]), g1 = make_float2(gamma[HD / 2 + 2 * lane], gamma[HD / 2 + 2 * lane + 1]);
+        float2 g0 = make_float2(1.f, 1.f), g1 = g0;   // null: no head norm
+        if (gamma) {
+            g0 = make_float2(gamma[2 * lane], gamma[2 * lane + 1]);
+            g1 = make_float2(gamma[HD / 2 + 2 * lane], gamma[HD / 2 + 2 * lane + 1]);
+        }
         float v[4];
         for (uint32_t s0 = 0; s0 < planes; s0 += 8) {
             float2 x[8], y[8];
@@ -208,7 +212,7 @@ prefill_qkv_kernel(const float* __restrict__ q_planes, const float* __restrict__
                 }
         }
         float ss = fmaf(v[0], v[0], fmaf(v[1], v[1], fmaf(v[2], v[2], v[3] * v[3])));
-        const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(HD) + a.eps);
+        const float normed = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(HD) + a.eps), inv = gamma ? normed : 1.f;
         v[0] = v[0] * inv * g0.x; v[1] = v[1] * inv * g0.y; v[2] = v[2] * inv * g1.x; v[3] = v[3] * inv * g1.y;
         const float o0 = __fsub_rn(__fmul_rn(v[0], rot.x), __fmul_rn(v[2], rot.y)), o1 = __fsub_rn(__fmul_rn(v[1], rot.z), __fmul_rn(v[3], rot.w));
         const float o2 = __fadd_rn(__fmul_rn(v[0], rot.y), __fmul_rn(v[2], rot.x)), o3 = __fadd_rn(__fmul_rn(v[1], rot.w), __fmul_rn(v[3], rot.z));

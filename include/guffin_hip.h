@@ -414,7 +414,7 @@ int guffin_hip_step_draws(uint64_t seed, uint64_t step, void* out_draws_host);
 typedef struct guffin_layer_desc {
     int32_t dtype[7];          /* q, k, v, o, gate, up, down */
     const void* tiles[7];
-    const float* norm[6];      /* attn_norm, q_norm, k_norm, post_attention_norm, ffn_norm, post_ffw_norm */
+    const float* norm[6];      /* attn_norm, q_norm, k_norm, post_attention_norm, ffn_norm, post_ffw_norm; q_norm, k_norm NULL: no head norm */
     void* ring_k; void* ring_v; /* fp16 [ring capacity][kv_heads * head_dim] */
 } guffin_layer_desc;
 

@@ -480,3 +480,25 @@ def test_the_shortest_runs_agree_with_a_longer_one(hip, kind, rows, position):
                 assert float((mine[s] == other[s]).float().mean()) >= 0.95
             rest = [s for s in range(cap) if s not in theirs]
             assert torch.equal(mine[rest], other[rest])   # nothing else moves
+
+
+@pytest.mark.parametrize("q_norm,k_norm", [(False, False), (True, False), (False, True)])
+def test_a_run_without_head_norms(hip, q_norm, k_norm):
+    """Null gammas leave the head norms out: the last of twenty rows against the decode pass of its token over the same rings (bound
+    as at the edges of row tiles)."""
+    import torch
+    from dataclasses import replace
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_12B, layers=2, vocab=2048, ring_global=256, ring_local=128, sliding_window=96)
+    devm = model.DeviceModel.from_host(model.HostModel(shape, seed=25, position=40))
+    for l in range(shape.layers):
+        for i, on in ((1, q_norm), (2, k_norm)):
+            if not on:
+                devm.layers[l].norm[i] = None
+    tokens = dev(np.random.default_rng(20).integers(0, shape.vocab, 20).astype(np.int32))
+    hidden, status = devm.prefill(tokens, 40)
+    one, _, _, _, st = devm.forward(tokens[19:].contiguous(), 59)
+    torch.cuda.synchronize()
+    assert int(status.item()) == 0 and int(st.item()) == 0
+    want = one.cpu().numpy().astype(np.float64)[0]
+    assert np.max(np.abs(hidden[19].cpu().numpy() - want)) <= 2e-4 * np.sqrt((want ** 2).mean())
