@@ -25,8 +25,8 @@
 //   * Attention: a wave a query (four waves are one a SIMD: eight would share the issue slots), a token per 16 lanes with a
 //     running softmax of their own, merged over lanes by register swaps; a list's first 20 tokens lie in LDS before the phase.
 //
-// 270M-shaped model, one row at position 150 / 600 / 4096: 299 / 303 / 356 us; two rows: 394 / 415 / 463.  (resident_blocks_kernel,
-// three launches: 606 / 621 / 652 and 777 / 816 / 888.)  rms error of the hidden row against 64 bits, one block, where no K/V
+// 270M-shaped model, whole pass, one row at position 150 / 4096: 293 / 360 us; two rows: 395 / 464.  (resident_blocks_kernel, three
+// launches: 606 / 652 and 777 / 888; one launch per operator: 559 / 581 and 609 / 653.)  rms error of the hidden row against 64 bits, one block, where no K/V
 // rounding falls the other way: 5.3-8e-8, as before.
 #include "common.hpp"
 #include "receipt.hpp"

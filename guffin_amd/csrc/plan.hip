@@ -311,8 +311,8 @@ int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t*
     void* st = stream;
     const uint32_t H = m.hidden, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
     const float attn_scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
-    // the resident pass is the default where it is the faster one: models with a single KV head (the drafter's
-    // small blocks); it can be forced for any model it covers, for runs of rows: a tree always goes one launch per operator
+    // the resident passes are the default for models with a single KV head (resident_chosen has the figures) and can be forced for any
+    // model they cover, for runs of rows: a tree always goes one launch per operator
     const bool resident = s.exchange != nullptr && resident_chosen(m, rows) && !tree;
     if (g_forward_mode == 2 && !resident && !tree) return fail(GUFFIN_E_SHAPE, "forward: the resident pass does not cover this model");
     const uint32_t sync_words = resident ? s.sync_words : 0u;
