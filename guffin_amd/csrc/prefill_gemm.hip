@@ -22,6 +22,13 @@
 // A workgroup is four waves on the same R * 16 rows and four neighbouring column tiles.  The A operand of a 64-element
 // chunk goes from memory to LDS without passing registers, two chunks ahead in three rotating buffers, one barrier per
 // chunk; weights are private to a wave and requested half a block ahead.
+//
+// What bounds it: the instructions that form B.  A loop of one matrix and V vector instructions takes, with two waves a SIMD,
+// 10 + 4.3 V cycles for V >= 2 (17 for the matrix instruction alone, 22.9 with three beside it), in whatever order they stand; a
+// block of four row tiles is 272 (Q6_K 384) of the one and 780 (920) of the other and takes 6900 of the 6100 cycles that makes.  So
+// scales are widened for two column groups at once, Q6_K's quants put together as bytes, operands change places instead of being
+// copied, and addresses are immediates.  us before / after: 2048 rows gate + up 855 / 839, down (Q6_K) 571 / 552, q/k/v 250 / 243, o 121 /
+// 119; 333 rows 180 / 174, 129 / 119, 64.7 / 61.0, 29.1 / 28.4; 37 rows 31.9 / 30.7, 26.9 / 25.1, 14.8 / 13.9, 10.2 / 9.8.
 #include "common.hpp"
 #include "prefill_image.hpp"
 #include "prefill_run.hpp"
@@ -65,6 +72,9 @@ __device__ __forceinline__ half8_t as_half8(uint32_t a, uint32_t b, uint32_t c, 
 __device__ __forceinline__ half2_t h2(uint32_t v) { return __builtin_bit_cast(half2_t, v); }
 __device__ __forceinline__ uint32_t u2(half2_t v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ half2_t splat(float f) { const _Float16 h = static_cast<_Float16>(f); return half2_t{h, h}; }
+// one half for both places: a modifier of the packed instruction that takes it
+template <int I>
+__device__ __forceinline__ half2_t both(half2_t v) { return __builtin_shufflevector(v, v, I, I); }
 
 // two bytes of w under the bias 1024, which comes off exactly, as a pair of halves; sel: their
 // places with 0x04 (the bias byte) in between
@@ -75,6 +85,8 @@ __device__ __forceinline__ uint32_t bytes_as_halves(uint32_t w, uint32_t sel, fl
 // (w & mask) | c is one instruction if it needs no literal (it takes none) and at most one scalar register: the mask is kept
 // in a scalar, c in a vector register.  (Empty asm statements pin them; the instruction itself is the compiler's, whose
 // hazard handling around matrix instructions does not look into an asm statement.)
+// the bytes of a pair of groups' scale word that belong to the first (second) group, under a bias byte each
+constexpr uint32_t pair_bytes(int second) { return second ? 0x04030402u : 0x04010400u; }
 __device__ __forceinline__ uint32_t scalar(uint32_t v) { asm("" : "+s"(v)); return v; }
 __device__ __forceinline__ uint32_t and_or(uint32_t w, uint32_t mask, uint32_t c) { return (w & mask) | c; }
 // a value the compiler takes as it is (it would turn two of the above into two ands and an or3)
@@ -101,9 +113,11 @@ __device__ __forceinline__ uint32_t ld4(__amdgpu_buffer_rsrc_t r, uint32_t lane_
     return __builtin_amdgcn_raw_buffer_load_b32(r, static_cast<int>(lane_off), static_cast<int>(uniform_off), 0);
 }
 // 64 lanes x 16 (4) bytes straight into LDS at `to` (+ 16 (4) per lane)
+// (and AT further on both sides: an immediate of the instruction)
+template <int AT = 0>
 __device__ __forceinline__ void to_lds16(__amdgpu_buffer_rsrc_t r, uint8_t* to, uint32_t lane_off, uint32_t uniform_off) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)to, 16, static_cast<int>(lane_off),
-                                             static_cast<int>(uniform_off), 0, 0);
+                                             static_cast<int>(uniform_off), AT, 0);
 }
 __device__ __forceinline__ void to_lds4(__amdgpu_buffer_rsrc_t r, uint8_t* to, uint32_t lane_off, uint32_t uniform_off) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)to, 4, static_cast<int>(lane_off),
@@ -157,8 +171,10 @@ struct Feed {
         const uint32_t c = chunk < last ? chunk : last;   // past the end: the last chunk again, never read
         const uint32_t from = base + (2 * c + (wv >> 1)) * group_stride;
         uint8_t* to = stage + buffer * Stage<R>::kChunk + (wv >> 1) * (2048 * R) + (wv & 1) * (1024 * R);
-#pragma unroll
-        for (int i = 0; i < R; ++i) to_lds16(img, to + 1024 * i, lane16, from + 1024 * i);
+        to_lds16<0>(img, to, lane16, from);
+        if constexpr (R > 1) to_lds16<1024>(img, to, lane16, from);
+        if constexpr (R > 2) to_lds16<2048>(img, to, lane16, from);
+        if constexpr (R > 3) to_lds16<3072>(img, to, lane16, from);
     }
 };
 
@@ -191,18 +207,20 @@ __device__ __forceinline__ uint32_t lane_again() {
 template <int G, int P>
 __device__ __forceinline__ void q4_operands(const uint4 (&q)[4], const uint32_t (&scw)[4], half8_t (&b)[4]) {
     constexpr bool HIGH = G & 1;
-    constexpr int BYTE = G & 3, WORD = (G >> 1) & 1;
+    constexpr int WORD = (G >> 1) & 1;
     // the quant under a bias whose last place is the quant's: 1024 + q, or 64 + q where the high nibbles stay in bits 4-7
     const uint32_t bias = vector_bias(HIGH ? 0x54005400u : 0x64006400u), mask = scalar(HIGH ? 0x00F000F0u : 0x000F000Fu);
-#pragma unroll
-    for (int cg = 2 * P; cg < 2 * P + 2; ++cg) {
-        // the scale byte under the bias: 1024 + sc in both halves, then sc and -bias sc (all exact in fp16)
-        const half2_t sc = h2(__builtin_amdgcn_perm(0x64646464u, scw[cg], 0x04000400u | (BYTE << 16) | BYTE)) - splat(1024.f);
-        const half2_t off = sc * splat(HIGH ? -64.f : -1024.f);
-        const uint32_t w0 = WORD ? q[cg].z : q[cg].x, w1 = WORD ? q[cg].w : q[cg].y;
-        auto piece = [&](uint32_t w) { return u2(__builtin_elementwise_fma(h2(and_or(w, mask, bias)), sc, off)); };
-        b[cg] = as_half8(piece(w0), piece(w0 >> 8), piece(w1), piece(w1 >> 8));
-    }
+    // both column groups' scales under the bias: 1024 + sc, then sc and -bias sc (all exact in fp16)
+    const half2_t sc = h2(__builtin_amdgcn_perm(0x64646464u, scw[2 * P + WORD], pair_bytes(G & 1))) - splat(1024.f);
+    const half2_t off = sc * splat(HIGH ? -64.f : -1024.f);
+    auto column = [&]<int I>() {
+        const uint4 v = q[2 * P + I];
+        const uint32_t w0 = WORD ? v.z : v.x, w1 = WORD ? v.w : v.y;
+        auto piece = [&](uint32_t w) { return u2(__builtin_elementwise_fma(h2(and_or(w, mask, bias)), both<I>(sc), both<I>(off))); };
+        b[2 * P + I] = as_half8(piece(w0), piece(w0 >> 8), piece(w1), piece(w1 >> 8));
+    };
+    column.template operator()<0>();
+    column.template operator()<1>();
 }
 
 template <int R, bool FIRST, int C0 = 0, int C1 = 4>
@@ -222,11 +240,11 @@ template <int R>
 __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint8_t* stage, const uint8_t* tile_base,
                                         uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q4_K);
-    constexpr int V = (30 + 4 * R - 1) / (4 * R);   // vector instructions behind each matrix instruction
+    constexpr int V = (26 + 4 * R - 1) / (4 * R);   // vector instructions behind each matrix instruction
     // Up to three row tiles the fold is woven in as well: a tile's beside the next tile's products, the last one's beside the
     // second half's first products.  Four leave no registers for that (2048 x 3840 x 15360: 446 us against 440 by itself).
     constexpr bool WOVEN = R < 4;
-    constexpr int VA = (30 + 32 * (R - 1) + 4 * R - 1) / (4 * R), VB = (62 + 4 * R - 1) / (4 * R);
+    constexpr int VA = (26 + 32 * (R - 1) + 4 * R - 1) / (4 * R), VB = (58 + 4 * R - 1) / (4 * R);
     using S = Stage<R>;
     const uint32_t wv = feed.wv;
     uint32_t lane = lane_again(), j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
@@ -234,7 +252,7 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
     uint8_t* const heads = stage + S::kHead + wv * 1280;
     uint4 q[2][4];
     uint32_t sc[4];
-    half8_t hi[R], lo[R], b[4], bn[4];
+    half8_t hi[R], lo[R], operands[2][4];   // B of a group and of the next, by turns
     float4_t D[4][R];
     auto ask_half = [&](uint32_t blk, int h, uint4 (&to)[4]) {
 #pragma unroll
@@ -246,11 +264,18 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
         if (wv < 2) to_lds16(feed.img, stage + S::kSums + 1024 * wv, lane16, static_cast<uint32_t>(L.sums_off) + (blk * (L.mpad / 16) + rt0) * 512 + 1024 * wv);
         else if (wv == 2) to_lds4(feed.img, stage + S::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (blk * L.mpad + rt0 * 16) * 4);
     };
+    // a word holds the scales of two column groups for two groups of the half: [column pair][groups 0, 1 | 2, 3]
     auto scales = [&](uint32_t blk, int half) {
+        uint32_t four[4];   // a column's four groups
 #pragma unroll
         for (int cg = 0; cg < 4; ++cg) {
             const uint32_t* h = reinterpret_cast<const uint32_t*>(heads + (blk & 1) * 5120 + 256 * cg + j * 16);
-            sc[cg] = half ? (h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u) : h[1] & 0x3F3F3F3Fu;
+            four[cg] = half ? (h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u) : h[1] & 0x3F3F3F3Fu;
+        }
+#pragma unroll
+        for (int p = 0; p < 4; p += 2) {
+            sc[p] = __builtin_amdgcn_perm(four[p + 1], four[p], 0x05010400u);
+            sc[p + 1] = __builtin_amdgcn_perm(four[p + 1], four[p], 0x07030602u);
         }
     };
     ask_half(b0, 0, q[0]);
@@ -264,8 +289,8 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
     arrive<2 * R>();
     scales(b0, 0);
     read_half<R>(stage, 1, lane16, lo);
-    q4_operands<0, 0>(q[0], sc, b);
-    q4_operands<0, 1>(q[0], sc, b);
+    q4_operands<0, 0>(q[0], sc, operands[0]);
+    q4_operands<0, 1>(q[0], sc, operands[0]);
     uint32_t rd = 0;   // the buffer of the chunk in work
     for (uint32_t blk = b0; blk < b1; ++blk) {
         if constexpr (!WOVEN) { lane = lane_again(); j = lane & 15; lg = lane >> 4; lane16 = feed.lane16 = lane * 16; }   // no register to keep addresses in
@@ -284,6 +309,7 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
                 for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(dh[cg] * mult[i], D[cg][r][i], acc[cg][r][i]);
         };
         auto group = [&]<int G>() {
+            half8_t (&b)[4] = operands[G & 1], (&bn)[4] = operands[(G + 1) & 1];
             const uint8_t* now = stage + rd * S::kChunk + (G & 1) * (2048 * R);
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (G == 3) scales(blk, 1);
@@ -331,8 +357,6 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
                 products<R, false>(hi, b, D);
                 weave<4 * R, V, R>();
             }
-#pragma unroll
-            for (int cg = 0; cg < 4; ++cg) b[cg] = bn[cg];
         };
         group.template operator()<0>();
         group.template operator()<1>();
@@ -376,34 +400,35 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
 }
 
 // ---- Q6_K ------------------------------------------------------------------------------------------------
-// Group QD (0..3) of a half block: the quants q - 32 of column groups C0 .. C1 - 1 as halves
+// Group QD (0..3) of a half block: the quants q - 32 of column groups C0 .. C1 - 1 as halves.  Put together as bytes, four at
+// a time, and widened under the bias: 14.5 instructions for a column group's eight quants instead of 18.5 on pairs of halves.
 template <int QD, int C0 = 0, int C1 = 4>
 __device__ __forceinline__ void q6_quants(const uint4 (&ql)[4], const uint2 (&qh)[4], half8_t (&q)[4]) {
-    const uint32_t bias = vector_bias(), low = scalar(0x000F000Fu), high = scalar(0x00300030u);
+    const uint32_t low = scalar(0x0F0F0F0Fu), high = scalar(0x30303030u);
 #pragma unroll
     for (int cg = C0; cg < C1; ++cg) {
         const uint32_t w[2] = {(QD & 1) ? ql[cg].z : ql[cg].x, (QD & 1) ? ql[cg].w : ql[cg].y};
         const uint32_t h[2] = {qh[cg].x, qh[cg].y};
         uint32_t o[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            constexpr int ls = QD >= 2 ? 4 : 0, up = 4 - 2 * QD;   // the two high bits go to bits 4-5
-            const int sh = 8 * (k & 1) - up;
-            const uint32_t wk = w[k >> 1] >> (ls + 8 * (k & 1));
-            const uint32_t hk = sh >= 0 ? h[k >> 1] >> (sh >= 0 ? sh : 0) : h[k >> 1] << (sh < 0 ? -sh : 0);
-            o[k] = u2(h2(and_or(wk, low, kept(and_or(hk, high, bias)))) - splat(1056.f));
+        for (int k = 0; k < 2; ++k) {
+            constexpr int up = 4 - 2 * QD;   // the two high bits go to bits 4-5
+            const uint32_t wk = QD >= 2 ? w[k] >> 4 : w[k];
+            const uint32_t hk = up >= 0 ? h[k] << (up >= 0 ? up : 0) : h[k] >> (up < 0 ? -up : 0);
+            const uint32_t bytes = and_or(wk, low, kept(hk & high));
+            o[2 * k] = bytes_as_halves(bytes, 0x04020400u, 1056.f);
+            o[2 * k + 1] = bytes_as_halves(bytes, 0x04030401u, 1056.f);
         }
         q[cg] = as_half8(o[0], o[1], o[2], o[3]);
     }
 }
-// times the lane's scale (a scale covers 16 elements; sel picks the lane's byte of the group's pair, int8 + 128 under the
-// bias): q becomes the nearest half of the product, rest what that rounding left
+// times the lane's scale (a scale covers 16 elements; a word holds those of two column groups for two groups, int8 + 128): q
+// becomes the nearest half of the product, rest what that rounding left
 template <int QD, int C0 = 0, int C1 = 4>
-__device__ __forceinline__ void q6_scaled(const uint2 (&sc)[4], uint32_t sel, half8_t (&q)[4], half8_t (&rest)[4]) {
-#pragma unroll
-    for (int cg = C0; cg < C1; ++cg) {
-        const half2_t s = h2(__builtin_amdgcn_perm(0x64646464u, (QD >> 1) ? sc[cg].y : sc[cg].x, sel + (QD & 1) * 0x00020002u)) - splat(1152.f);
-        const uint4 v = __builtin_bit_cast(uint4, q[cg]);
+__device__ __forceinline__ void q6_scaled(const uint32_t (&scw)[4], half8_t (&q)[4], half8_t (&rest)[4]) {
+    auto column = [&]<int CG>(half2_t pair) {
+        const half2_t s = both<CG & 1>(pair);
+        const uint4 v = __builtin_bit_cast(uint4, q[CG]);
         const uint32_t x[4] = {v.x, v.y, v.z, v.w};
         uint32_t p[4], r[4];
 #pragma unroll
@@ -412,8 +437,24 @@ __device__ __forceinline__ void q6_scaled(const uint2 (&sc)[4], uint32_t sel, ha
             p[k] = u2(prod);
             r[k] = u2(__builtin_elementwise_fma(s, h2(x[k]), -prod));
         }
-        q[cg] = as_half8(p[0], p[1], p[2], p[3]);
-        rest[cg] = as_half8(r[0], r[1], r[2], r[3]);
+        q[CG] = as_half8(p[0], p[1], p[2], p[3]);
+        rest[CG] = as_half8(r[0], r[1], r[2], r[3]);
+    };
+    auto two = [&]<int P>() {
+        const half2_t pair = h2(__builtin_amdgcn_perm(0x64646464u, scw[2 * P + (QD >> 1)], pair_bytes(QD & 1))) - splat(1152.f);
+        column.template operator()<2 * P>(pair);
+        column.template operator()<2 * P + 1>(pair);
+    };
+    if constexpr (C0 == 0) two.template operator()<0>();
+    if constexpr (C1 == 4) two.template operator()<1>();
+}
+// a half block's scale words from the waves' headers: lanes of k-slices 0, 1 take a group's first scale, of 2, 3 its second
+__device__ __forceinline__ void q6_scale_words(const uint8_t* head, int half, uint32_t j, uint32_t sel, uint32_t (&sc)[4]) {
+#pragma unroll
+    for (int p = 0; p < 4; p += 2) {
+        const uint2_t a = from_lds8(head + 256 * p + j * 16 + 8 * half), b = from_lds8(head + 256 * p + 256 + j * 16 + 8 * half);
+        sc[p] = __builtin_amdgcn_perm(b.x, a.x, sel) ^ 0x80808080u;   // int8 -> + 128
+        sc[p + 1] = __builtin_amdgcn_perm(b.y, a.y, sel) ^ 0x80808080u;
     }
 }
 
@@ -424,34 +465,29 @@ template <int R>
 __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& feed, uint8_t* stage, const uint8_t* tile_base,
                                         uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q6_K);
-    constexpr int V0 = (96 + 4 * R - 1) / (4 * R), V1 = (48 + 4 * R - 1) / (4 * R);
+    constexpr int V0 = (60 + 4 * R - 1) / (4 * R), V1 = (38 + 4 * R - 1) / (4 * R);
     using S = Stage<R>;
     const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
     const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
-    const uint32_t sel = lane >= 32 ? 0x04010401u : 0x04000400u;
+    const uint32_t sel = lane >= 32 ? 0x07030501u : 0x06020400u;
     uint8_t* const heads = stage + S::kHead + wv * 1280;
     uint4 ql[2][4];
-    uint2 qh[2][4], sc[4];
-    half8_t hi[R], lo[R], b[4], bn[4], rest[4];
+    uint2 qh[2][4];
+    uint32_t sc[4];
+    half8_t hi[R], lo[R], operands[2][4], rest[4];
     float4_t D[4][R];
     auto ask_half = [&](uint32_t blk, int h) {
 #pragma unroll
         for (int cg = 0; cg < 4; ++cg) {
-            ql[h][cg] = ld16(tile, lane16, blk * TB + 2048 * cg + 1024 * h);
-            qh[h][cg] = ld8(tile, lane16 + 8 * h, blk * TB + 8192 + 1024 * cg);
+            ql[h][cg] = ld16(tile, lane16 + 2048 * (cg & 1) + 1024 * h, blk * TB + 4096 * (cg >> 1));
+            qh[h][cg] = ld8(tile, lane16 + 8 * h + 1024 * (cg & 3), blk * TB + 8192);
         }
     };
     auto ask_head = [&](uint32_t blk) {   // the 16 scales of every column, then the columns' d (read beyond the tile: zeros)
         to_lds16(tile, heads + (blk & 1) * 5120, lane16, blk * TB + 12288);
         to_lds4(tile, heads + (blk & 1) * 5120 + 1024, lane < 32 ? lane * 4 : 0, blk * TB + 13312);
     };
-    auto scales = [&](uint32_t blk, int half) {
-#pragma unroll
-        for (int cg = 0; cg < 4; ++cg) {
-            const uint2_t v = from_lds8(heads + (blk & 1) * 5120 + 256 * cg + j * 16 + 8 * half);
-            sc[cg] = make_uint2(v.x ^ 0x80808080u, v.y ^ 0x80808080u);   // int8 -> + 128
-        }
-    };
+    auto scales = [&](uint32_t blk, int half) { q6_scale_words(heads + (blk & 1) * 5120, half, j, sel, sc); };
     ask_half(b0, 0);
     ask_head(b0);
     feed.ask(4 * b0, 0);
@@ -463,13 +499,14 @@ __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& fee
     arrive<2 * R>();
     scales(b0, 0);
     read_half<R>(stage, 0, lane16, hi);
-    q6_quants<0>(ql[0], qh[0], b);
-    q6_scaled<0>(sc, sel, b, rest);
+    q6_quants<0>(ql[0], qh[0], operands[0]);
+    q6_scaled<0>(sc, operands[0], rest);
     uint32_t rd = 0;
     for (uint32_t blk = b0; blk < b1; ++blk) {
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
         auto group = [&]<int G>() {
             constexpr int H = ((G + 1) & 7) >> 2, QD = (G + 1) & 3;   // the next group's half block and place
+            half8_t (&b)[4] = operands[G & 1], (&bn)[4] = operands[(G + 1) & 1];
             const uint8_t* now = stage + rd * S::kChunk + (G & 1) * (2048 * R);
             __builtin_amdgcn_sched_barrier(0);
             read_half<R>(now, 1, lane16, lo);
@@ -478,7 +515,7 @@ __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& fee
             weave<4 * R, V0, R>();
             if constexpr (G == 3) scales(blk, 1);
             if constexpr (G == 7) scales(next, 0);
-            q6_scaled<QD>(sc, sel, bn, rest);
+            q6_scaled<QD>(sc, bn, rest);
             products<R, false>(hi, b, D);
             weave<4 * R, V1, 0>();
             if constexpr (G & 1) {
@@ -496,8 +533,6 @@ __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& fee
             read_half<R>(stage + rd * S::kChunk + ((G + 1) & 1) * (2048 * R), 0, lane16, hi);
             products<R, false>(lo, b, D);
             __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int cg = 0; cg < 4; ++cg) b[cg] = bn[cg];
         };
         group.template operator()<0>();
         group.template operator()<1>();
@@ -527,35 +562,31 @@ __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& fee
 // the compiler's order, and the second wave of the SIMD to fill the gaps (the woven form spills: 2048 x 15360 x 3840 takes
 // 772 us instead of 614).  The workgroup meets at a chunk's start; the chunk after the next is asked for there.
 template <int R>
-__device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, const Feed<R>& feed, uint8_t* stage, const uint8_t* tile_base,
+__device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed, uint8_t* stage, const uint8_t* tile_base,
                                              uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q6_K);
     using S = Stage<R>;
-    const uint32_t lane = lane_again(), wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
+    const uint32_t wv = feed.wv;
+    uint32_t lane = lane_again(), j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
     const __amdgpu_buffer_rsrc_t tile = make_resource(tile_base, b1 * TB);
-    const uint32_t sel = lane >= 32 ? 0x04010401u : 0x04000400u;
+    uint32_t sel = lane >= 32 ? 0x07030501u : 0x06020400u;
     uint8_t* const heads = stage + S::kHead + wv * 1280;
     uint4 ql[2][4];
-    uint2 qh[2][4], sc[4];
+    uint2 qh[2][4];
+    uint32_t sc[4];
     float4_t D[4][R];
     auto ask_half = [&](uint32_t blk, int h) {
 #pragma unroll
         for (int cg = 0; cg < 4; ++cg) {
-            ql[h][cg] = ld16(tile, lane16, blk * TB + 2048 * cg + 1024 * h);
-            qh[h][cg] = ld8(tile, lane16 + 8 * h, blk * TB + 8192 + 1024 * cg);
+            ql[h][cg] = ld16(tile, lane16 + 2048 * (cg & 1) + 1024 * h, blk * TB + 4096 * (cg >> 1));
+            qh[h][cg] = ld8(tile, lane16 + 8 * h + 1024 * (cg & 3), blk * TB + 8192);
         }
     };
     auto ask_head = [&](uint32_t blk) {
         to_lds16(tile, heads + (blk & 1) * 5120, lane16, blk * TB + 12288);
         to_lds4(tile, heads + (blk & 1) * 5120 + 1024, lane < 32 ? lane * 4 : 0, blk * TB + 13312);
     };
-    auto scales = [&](uint32_t blk, int half) {
-#pragma unroll
-        for (int cg = 0; cg < 4; ++cg) {
-            const uint2_t v = from_lds8(heads + (blk & 1) * 5120 + 256 * cg + j * 16 + 8 * half);
-            sc[cg] = make_uint2(v.x ^ 0x80808080u, v.y ^ 0x80808080u);
-        }
-    };
+    auto scales = [&](uint32_t blk, int half) { q6_scale_words(heads + (blk & 1) * 5120, half, j, sel, sc); };
     ask_half(b0, 0);
     ask_head(b0);
     feed.ask(4 * b0, 0);
@@ -563,6 +594,8 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, const Feed<R>
     feed.ask(4 * b0 + 1, 1);
     uint32_t rd = 0, wr = 2;
     for (uint32_t blk = b0; blk < b1; ++blk) {
+        lane = lane_again(); j = lane & 15; lg = lane >> 4; lane16 = feed.lane16 = lane * 16;   // no register to keep addresses in
+        sel = lane >= 32 ? 0x07030501u : 0x06020400u;
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;
         auto group = [&]<int G>() {
             constexpr int H = G >> 2, QD = G & 3;
@@ -583,12 +616,13 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, const Feed<R>
             read_half<R>(from, 1, lane16, lo);
             auto pair = [&]<int C>() {
                 q6_quants<QD, C, C + 2>(ql[H], qh[H], b);
-                q6_scaled<QD, C, C + 2>(sc, sel, b, rest);
+                q6_scaled<QD, C, C + 2>(sc, b, rest);
                 products<R, G == 0, C, C + 2>(hi, b, D);
                 products<R, false, C, C + 2>(lo, b, D);
                 products<R, false, C, C + 2>(hi, rest, D);
             };
             pair.template operator()<0>();
+            __builtin_amdgcn_sched_barrier(0);
             pair.template operator()<2>();
             if constexpr (G & 1) { rd = rd == 2 ? 0 : rd + 1; wr = wr == 2 ? 0 : wr + 1; }
         };
@@ -637,34 +671,35 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
     feed.base = rt0 * 2048 + (wv & 1) * (1024 * R);
     feed.wv = wv;
     feed.last = 4 * b1 - 1;
-    float acc[4][R][4];
+    // a whole form per format: what they share would have to lie in the same registers for both
+    auto run = [&](auto walk, uint32_t bytes) {
+        float acc[4][R][4];
 #pragma unroll
-    for (int cg = 0; cg < 4; ++cg)
+        for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[cg][r][i] = 0.f;
+        walk(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * bytes), rt0, b0, b1, acc);
+        // the chunks asked for past the end are still on their way into this workgroup's LDS
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (!valid) return;
+        const uint32_t N = seg.columns * kCols;
+        float* y = seg.y + blockIdx.z * (uint64_t(M) * N);
+        const uint32_t at = lane_again(), col = tile_index * kCols + (at & 15), row0 = rt0 * 16 + 4 * (at >> 4);
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[cg][r][i] = 0.f;
-    if (KINDS == 1 || (KINDS == 3 && seg.dtype == GUFFIN_Q4_K))
-        q4_walk<R>(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q4_K)), rt0, b0, b1, acc);
-    else if constexpr (R == 4)
-        q6_walk_wide<R>(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q6_K)), rt0, b0, b1, acc);
-    else
-        q6_walk<R>(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * block_bytes(GUFFIN_Q6_K)), rt0, b0, b1, acc);
-    // the chunks asked for past the end are still on their way into this workgroup's LDS
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (!valid) return;
-    const uint32_t N = seg.columns * kCols;
-    float* y = seg.y + blockIdx.z * (uint64_t(M) * N);
-    const uint32_t at = lane_again(), col = tile_index * kCols + (at & 15), row0 = rt0 * 16 + 4 * (at >> 4);
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t row = row0 + 16 * r + i;
+                if (row < M)
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t row = row0 + 16 * r + i;
-            if (row < M)
-#pragma unroll
-                for (int cg = 0; cg < 4; ++cg) y[size_t(row) * N + col + 16 * cg] = acc[cg][r][i];
-        }
+                    for (int cg = 0; cg < 4; ++cg) y[size_t(row) * N + col + 16 * cg] = acc[cg][r][i];
+            }
+    };
+    if (KINDS == 1 || (KINDS == 3 && seg.dtype == GUFFIN_Q4_K)) run(q4_walk<R>, block_bytes(GUFFIN_Q4_K));
+    else if constexpr (KINDS != 1 && R == 4) run(q6_walk_wide<R>, block_bytes(GUFFIN_Q6_K));
+    else if constexpr (KINDS != 1) run(q6_walk<R>, block_bytes(GUFFIN_Q6_K));
 }
 
 // ---- Q8_0 ------------------------------------------------------------------------------------------------
