@@ -52,6 +52,15 @@ int resident_launch(hipStream_t stream, const guffin_model_desc& m, uint32_t row
                     const void* u_receipt_in, float* x_out, float* u_out, void* u_receipt_out, uint32_t max_ring_tokens,
                     uint32_t* status);
 
+// Up to kRunRows contiguous rows of a model that the drafter's pass covers (plan.hip): every row's final state to row_states (or null),
+// the last one's with its receipt to last_state / last_receipt as well.  scratch: forward_run_bytes, 256-byte aligned; priv_k,
+// priv_v: [block][rows][kv width].  A row's results are those of a pass by itself, bit for bit.
+constexpr uint32_t kRunRows = 8;          // XCDs of the part
+bool forward_run_chosen(const guffin_model_desc& m);
+uint64_t forward_run_bytes(const guffin_model_desc& m);
+int forward_run(hipStream_t stream, const guffin_model_desc& m, const uint32_t* tokens, uint32_t rows, uint32_t position, void* scratch,
+                void* priv_k, void* priv_v, float* row_states, float* last_state, float* last_receipt, uint32_t* status);
+
 // ---- streaming products of 3 and 4 rows (gemv_wide.hip) -------------------------------------------------------
 constexpr uint32_t kWideRows = 4;
 // The work split of a streaming product over `tiles` column tiles of `nblk` blocks (gemv_packed.hip): blocks per wave, waves per

@@ -75,10 +75,10 @@ Buffers carve(const guffin_model_desc& m, uint32_t arena, void* workspace, uint6
     Carve c {static_cast<uint8_t*>(workspace), 0};
     Buffers b {};
     const uint64_t kvw = uint64_t(m.kv_heads) * m.head_dim;
-    b.forward_bytes = guffin_hip_forward_scratch_bytes(&m, 2, m.ring_global - 2);
+    b.forward_bytes = std::max(guffin_hip_forward_scratch_bytes(&m, 2, m.ring_global - 2), forward_run_bytes(m));
     b.forward = c.take<uint8_t>(b.forward_bytes);
-    b.priv_k = c.take<uint16_t>(uint64_t(m.layer_count) * 2 * kvw);
-    b.priv_v = c.take<uint16_t>(uint64_t(m.layer_count) * 2 * kvw);
+    b.priv_k = c.take<uint16_t>(uint64_t(m.layer_count) * kRunRows * kvw);
+    b.priv_v = c.take<uint16_t>(uint64_t(m.layer_count) * kRunRows * kvw);
     b.backup_k = c.take<uint16_t>(uint64_t(m.layer_count) * arena * kvw);
     b.backup_v = c.take<uint16_t>(uint64_t(m.layer_count) * arena * kvw);
     b.hidden = c.take<float>(2 * uint64_t(m.hidden));
@@ -119,16 +119,22 @@ int move_rows(hipStream_t s, const guffin_draft_plan* p, const Buffers& b, uint3
     return kv_move_rows(s, *p->model, save ? KvMove::Save : KvMove::Restore, b.backup_k, b.backup_v, p->transaction_arena, first, end - first);
 }
 
-// one pass of the token at `token` (device memory) at the materialized frontier, published to the rings
-int forward(hipStream_t s, guffin_draft_plan* p, const Buffers& b, const uint32_t* token) {
+// one pass of the `rows` tokens from `token` on (device memory) at the materialized frontier, published to the rings
+int forward(hipStream_t s, guffin_draft_plan* p, const Buffers& b, const uint32_t* token, uint32_t rows) {
     const guffin_model_desc& m = *p->model;
     const uint32_t at = p->materialized;
-    GUFFIN_TRY(guffin_hip_forward_rows(s, &m, token, 1, at, b.forward, b.forward_bytes, b.priv_k, b.priv_v, b.hidden,
-                                       b.hidden_sums, b.status));
     // a transaction keeps the rows' final normalised states by their place in it
     float* kept = p->transaction_active ? b.txn_hidden + uint64_t(at - p->checkpoint_materialized) * m.hidden : nullptr;
-    GUFFIN_TRY(commit_rows_keeping(s, m, b.priv_k, b.priv_v, b.ring_k_table, b.ring_v_table, nullptr, at, 1, b.hidden, kept));
-    p->materialized = at + 1;
+    if (forward_run_chosen(m)) {
+        GUFFIN_TRY(forward_run(s, m, token, rows, at, b.forward, b.priv_k, b.priv_v, kept, b.hidden, b.hidden_sums, b.status));
+        GUFFIN_TRY(commit_rows_keeping(s, m, b.priv_k, b.priv_v, b.ring_k_table, b.ring_v_table, nullptr, at, rows, nullptr, nullptr));
+    } else {
+        GUFFIN_TRY(guffin_hip_forward_rows(s, &m, token, 1, at, b.forward, b.forward_bytes, b.priv_k, b.priv_v, b.hidden,
+                                           b.hidden_sums, b.status));
+        GUFFIN_TRY(commit_rows_keeping(s, m, b.priv_k, b.priv_v, b.ring_k_table, b.ring_v_table, nullptr, at, 1, b.hidden, kept));
+        rows = 1;
+    }
+    p->materialized = at + rows;
     p->last_rows = 1;
     p->logits_valid = 0;
     p->hidden_valid = 1;
@@ -216,9 +222,10 @@ int run_batch(hipStream_t s, guffin_draft_plan* p, const Buffers& b, uint32_t ro
     }
 }
 
-// host tokens through the blocks one row per pass, a pending token first: a token's rows and logits then do
-// not depend on how the caller grouped its appends (a two-row pass sums attention partitions and norms in
-// another order than two one-row passes), which is what lets a commit be compared with a replay bit for bit
+// host tokens through the blocks, a pending token first: a token's rows and logits do not depend on how the caller grouped its
+// appends, which is what lets a commit be compared with a replay bit for bit.  The drafter's pass takes eight at a time, an XCD a
+// row, each summed as by itself; any other form goes one row per pass (a two-row pass of those sums attention partitions and norms
+// in another order than two one-row passes)
 int ingest(hipStream_t s, guffin_draft_plan* p, const Buffers& b, const uint32_t* tokens, uint32_t count, const char* what) {
     std::vector<uint32_t> input;
     if (p->has_pending) input.push_back(p->pending_token);
@@ -228,7 +235,10 @@ int ingest(hipStream_t s, guffin_draft_plan* p, const Buffers& b, const uint32_t
         if (hipMemcpyWithStream(b.staging->tokens, input.data() + i0, n * 4, hipMemcpyHostToDevice, s) != hipSuccess)
             return poison(p, GUFFIN_E_HIP, "draft_plan: token upload failed");
         GUFFIN_TRY(run_batch(s, p, b, n, what, [&](bool) {
-            for (uint32_t i = 0; i < n; ++i) GUFFIN_TRY(forward(s, p, b, b.staging->tokens + i));
+            for (const uint32_t first = p->materialized; p->materialized - first < n;) {
+                const uint32_t done = p->materialized - first;
+                GUFFIN_TRY(forward(s, p, b, b.staging->tokens + done, std::min(n - done, kRunRows)));
+            }
             return int(GUFFIN_OK);
         }));
     }
@@ -461,7 +471,7 @@ extern "C" int guffin_hip_draft_plan_propose(void* stream, guffin_draft_plan* pl
     const bool compact = opt.temperature > 0.f && std::isfinite(opt.temperature) && opt.top_k >= 1 && opt.top_k <= 64 && opt.top_p > 0.f
                       && opt.top_p <= 1.f && opt.min_p >= 0.f && opt.min_p <= 1.f;
     GUFFIN_TRY(run_batch(s, plan, b, horizon - 1 + (pending ? 1u : 0u), "draft_plan_propose: a pass or a law raised the device status", [&](bool full_laws) {
-        if (pending) GUFFIN_TRY(forward(s, plan, b, b.staging->tokens));
+        if (pending) GUFFIN_TRY(forward(s, plan, b, b.staging->tokens, 1));
         for (uint32_t i = 0; i < horizon; ++i) {
             GUFFIN_TRY(ensure_logits(s, plan, b));
             const float* logits = b.logits + uint64_t(plan->last_rows - 1) * m.vocab;
@@ -476,7 +486,7 @@ extern "C" int guffin_hip_draft_plan_propose(void* stream, guffin_draft_plan* pl
             else
                 GUFFIN_TRY(guffin_hip_draft_law_any(s, logits, m.vocab, &law_options, 0, 0, b.staging->draws + i, b.law_ws, b.law, b.cdf,
                                                     token, b.status));
-            if (i + 1 < horizon) GUFFIN_TRY(forward(s, plan, b, token));
+            if (i + 1 < horizon) GUFFIN_TRY(forward(s, plan, b, token, 1));
         }
         return int(GUFFIN_OK);
     }));

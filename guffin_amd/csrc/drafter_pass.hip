@@ -1,5 +1,5 @@
-// The block graph of a decode pass (one or two rows) of a narrow Q8_0 model with one KV head -- the drafter -- as one launch of
-// up to 24 blocks on the 32 CUs of one XCD.
+// The block graph of a decode pass of a narrow Q8_0 model with one KV head -- the drafter -- as one launch of up to 24 blocks, up to
+// eight contiguous rows side by side: a row on the 32 CUs of an XCD each.
 //
 // Operator order per block: the drafter's forward (src/engine/gemma3_draft.mm:888-972).  The placement and the bounded waits are
 // those of resident.hip; as there, workgroups hand over through the XCD's L2: plain stores, a counter, reads past the L1.
@@ -25,9 +25,14 @@
 //   * Attention: a wave a query (four waves are one a SIMD: eight would share the issue slots), a token per 16 lanes with a
 //     running softmax of their own, merged over lanes by register swaps; a list's first 20 tokens lie in LDS before the phase.
 //
-// 270M-shaped model, whole pass, one row at position 150 / 4096: 293 / 360 us; two rows: 395 / 464.  (resident_blocks_kernel, three
-// launches: 606 / 652 and 777 / 888; one launch per operator: 559 / 581 and 609 / 653.)  rms error of the hidden row against 64 bits, one block, where no K/V
-// rounding falls the other way: 5.3-8e-8, as before.
+//   * Rows depend on each other through keys and values alone.  A row writes its own past its L2, raises a flag for the block, and
+//     the workgroups whose part of the list holds an earlier row's wait for that row's flag and take them over into LDS -- the last
+//     wave, which has no weights under way, while the others prepare the queries.  Every row is one hand-over behind the row before
+//     from the first block on, so the wait is short after that; and a row's operations are those of a pass by itself.
+//
+// 270M-shaped model, whole pass at position 150 / 4096: one row 299 / 351 us, two rows 316 / 368 (in one XCD, sharing the weights: 402 / 471),
+// eight rows 361 at 150.  (resident_blocks_kernel, three launches: one row 606 / 652, two 777 / 888; one launch per operator: 559 / 581 and 609 / 653.)
+// rms error of the hidden row against 64 bits, one block, where no K/V rounding falls the other way: 5.3-8e-8.
 #include "common.hpp"
 #include "receipt.hpp"
 #include "resident.hpp"
@@ -47,8 +52,9 @@ constexpr int kOwn = 3, kOwnO = 2, kOwnDown = 4;          // blocks per worker: 
 constexpr uint32_t kTile = 64 * 34;       // a wave tile of one Q8_0 block (gemv_packed.hip has the layout)
 constexpr uint32_t kChunk = 20;           // tokens whose keys and values lie in LDS (a window of 512: 17 a workgroup)
 
-constexpr uint32_t kSyncStride = 64;      // words between the counters of consecutive launches
+constexpr uint32_t kLine = 64;            // words between the counters of two rows
 constexpr uint32_t kLayers = 24;          // blocks per launch (their pointers travel as kernel arguments)
+constexpr uint32_t kFlagsAt = kRunRows * kLine, kSyncWords = kFlagsAt + kLayers * kRunRows;
 
 struct DLayer {
     const uint8_t* tiles[7];                 // q k v o gate up down
@@ -58,15 +64,17 @@ struct DLayer {
 };
 struct DArgs {
     DLayer layer[kLayers];
-    uint32_t layers, H, F;
+    uint32_t layers, rows, H, F;
     float eps, scale;
-    uint8_t* exchange;                       // the hand-over buffers; offsets of its regions, all of them
+    uint8_t* exchange;                       // a row's hand-over buffers; offsets of its regions, all of them
     uint32_t qkv_at, out_at, ml_at, o_at, d_at, h_at, exchange_bytes;
-    uint32_t* sync;                          // one cleared counter
+    uint32_t* sync;                          // cleared: a line with a counter for each row, then the rows' flags, block by block
     const float *x_in, *u_in;
-    float *x_out, *u_out; void* u_receipt_out;   // written after the last block
+    float *x_out, *u_out;                    // written after the last block; u_last, the receipt: the launch with the output norm alone
+    float* u_last;                           // the last row's final state, or null
+    void* u_receipt_out; uint32_t receipt_rows;  // of all rows, or (1) of the last one
     const float2 *rope_local, *rope_global;
-    const uint32_t *schedule, *ancestors;    // of the launch's first block on
+    const uint32_t* schedule;                // of the launch's first block on
     uint16_t *priv_k, *priv_v;               // [block][row][256], of the launch's first block on
     uint32_t* status;
     uint32_t spin_limit;
@@ -79,19 +87,18 @@ typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
 typedef int i4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
-template <int R>
 struct Shared {
-    float red[kWorkers][2][R][64];                 // the workers' column sums (gate and up)
-    float sums[2][R][kWaves];                      // their parts of a row's two sums of squares
-    float2 rope[2][R][kHd / 2];                    // local, global
-    uint32_t opnd[kWorkers][R][128];               // a worker's operand: an element's four digits a word
-    float mult[kWorkers][R][4];
+    float red[kWorkers][2][64];                    // the workers' column sums (gate and up)
+    float sums[2][kWaves];                         // their parts of the row's two sums of squares
+    float2 rope[2][kHd / 2];                       // local, global
+    uint32_t opnd[kWorkers][128];                  // a worker's operand: an element's four digits a word
+    float mult[kWorkers][4];
     float head[kWaves][kHd];                       // a wave's query (then its output, where several waves share a query)
     float2 ml[kWaves];
     uint16_t k_s[kChunk][kHd], v_s[kChunk][kHd];   // ring rows of a chunk of this workgroup's tokens
-    uint16_t kp_s[R][kHd], vp_s[R][kHd];           // the private rows among them
-    float weight[kWorkers][R][kGroups];            // a worker's partition weights, those of lane group g at 8 g ..
-    uint32_t schedule[kLayers][R][4];      // first ring position, ring count, private rows attended (a bit each)
+    uint16_t kp_s[kRunRows][kHd], vp_s[kRunRows][kHd];   // the private rows among them
+    float weight[kWorkers][kGroups];               // a worker's partition weights, those of lane group g at 8 g ..
+    uint32_t schedule[kLayers][4];                 // first ring position, ring count, first private row, private rows (this one the last)
     uint32_t dead;
 };
 
@@ -185,34 +192,28 @@ __device__ __forceinline__ float digit_value(const i4_t D) {
     return fmaf(static_cast<float>(D[3]), 16777216.f, f);
 }
 // elements 4 STEP .. 4 STEP + 3 of every block: the chains of the blocks side by side
-template <int STEP, int N, int R, int V, int I = 0>
-__device__ __forceinline__ void step(const Tile (&t)[N], const int (&a)[R][V], i4_t (&D)[N][R]) {
+template <int STEP, int N, int V, int I = 0>
+__device__ __forceinline__ void step(const Tile (&t)[N], const int (&a)[V], i4_t (&D)[N]) {
     if constexpr (I < N) {
         const int w = static_cast<int>((STEP & 1) ? t[I].q[STEP >> 1].y : t[I].q[STEP >> 1].x);
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            D[I][r] = __builtin_amdgcn_mfma_i32_4x4x4i8(a[r][I >> 1], w, STEP == 0 ? i4_t{0, 0, 0, 0} : D[I][r], 4, 8 * (I & 1) + STEP, 0);
-        step<STEP, N, R, V, I + 1>(t, a, D);
+        D[I] = __builtin_amdgcn_mfma_i32_4x4x4i8(a[I >> 1], w, STEP == 0 ? i4_t{0, 0, 0, 0} : D[I], 4, 8 * (I & 1) + STEP, 0);
+        step<STEP, N, V, I + 1>(t, a, D);
     }
 }
-template <int N, int R, int V, int STEP = 0>
-__device__ __forceinline__ void steps(const Tile (&t)[N], const int (&a)[R][V], i4_t (&D)[N][R]) {
-    if constexpr (STEP < 8) { step<STEP>(t, a, D); steps<N, R, V, STEP + 1>(t, a, D); }
+template <int N, int V, int STEP = 0>
+__device__ __forceinline__ void steps(const Tile (&t)[N], const int (&a)[V], i4_t (&D)[N]) {
+    if constexpr (STEP < 8) { step<STEP>(t, a, D); steps<N, V, STEP + 1>(t, a, D); }
 }
 // this lane's column over the wave's `count` blocks, in block order
-template <int N, int R>
-__device__ __forceinline__ void fold(const Tile (&t)[N], uint32_t count, const i4_t (&D)[N][R], const float (*mult)[4], float (&acc)[R]) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+template <int N>
+__device__ __forceinline__ float fold(const Tile (&t)[N], uint32_t count, const i4_t (&D)[N], const float (&mult)[4]) {
+    float acc = 0.f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-        const float d = h2f(t[i].d);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const float sum = fmaf(d * mult[r][i], digit_value(D[i][r]), acc[r]);
-            acc[r] = uint32_t(i) < count ? sum : acc[r];
-        }
+        const float sum = fmaf(h2f(t[i].d) * mult[i], digit_value(D[i]), acc);
+        acc = uint32_t(i) < count ? sum : acc;
     }
+    return acc;
 }
 
 // how `total` items are dealt to `ways`: the first ones get one more
@@ -223,23 +224,14 @@ __device__ __forceinline__ Share share_of(uint32_t total, uint32_t ways, uint32_
 }
 
 // ---- attention -------------------------------------------------------------------------------------------
-// The tokens of a block's rows (union of the rows' ring ranges, then the private rows) and this workgroup's part of them.
-template <int R>
-struct Tokens { uint32_t u_first, n_ring, t0, t1, mask, first[R], end[R], attends[R]; };
+// The tokens of a block's row (ring rows, then private rows of the launch's rows up to this one) and this workgroup's part of them.
+struct Tokens { uint32_t first, n_ring, priv_first, priv_count, t0, t1, mask; };
 
-template <int R>
-__device__ __forceinline__ Tokens<R> tokens_of(const Shared<R>& sh, uint32_t l, uint32_t mask, uint32_t slot) {
-    Tokens<R> t;
-    uint32_t first = 0xFFFFFFFFu, end = 0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const uint32_t f = uniform(sh.schedule[l][r][0]), n = uniform(sh.schedule[l][r][1]);
-        t.first[r] = f; t.end[r] = f + n; t.attends[r] = uniform(sh.schedule[l][r][2]);
-        if (n) { first = min(first, f); end = max(end, f + n); }
-    }
-    t.u_first = end ? first : 0u;
-    t.n_ring = end ? end - first : 0u;
-    const uint32_t total = t.n_ring + R, per = (total + kGroups - 1) / kGroups;
+__device__ __forceinline__ Tokens tokens_of(const Shared& sh, uint32_t l, uint32_t mask, uint32_t slot) {
+    Tokens t;
+    t.first = uniform(sh.schedule[l][0]); t.n_ring = uniform(sh.schedule[l][1]);
+    t.priv_first = uniform(sh.schedule[l][2]); t.priv_count = uniform(sh.schedule[l][3]);
+    const uint32_t total = t.n_ring + t.priv_count, per = (total + kGroups - 1) / kGroups;
     t.t0 = min(slot * per, total); t.t1 = min(t.t0 + per, total);
     t.mask = mask;
     return t;
@@ -248,20 +240,18 @@ __device__ __forceinline__ Tokens<R> tokens_of(const Shared<R>& sh, uint32_t l, 
 // A worker's share of a chunk: up to three of its 20 pairs of rows (ten of keys, ten of values), half a wave a row.  Asked for
 // through a buffer resource: lanes past the last token ask beyond its end, which reads zeros and touches no memory.
 struct Rows { uint4 v[3]; };
-template <int R>
-__device__ __forceinline__ void ask_rows(Rows& to, const uint16_t* ring_k, const uint16_t* ring_v, const Tokens<R>& t, uint32_t chunk, uint32_t wave, uint32_t lane) {
+__device__ __forceinline__ void ask_rows(Rows& to, const uint16_t* ring_k, const uint16_t* ring_v, const Tokens& t, uint32_t chunk, uint32_t wave, uint32_t lane) {
 #pragma unroll
     for (uint32_t i = 0; i < 3; ++i) {
         const uint32_t pair = wave + kWorkers * i, row = 2 * (pair % (kChunk / 2)) + (lane >> 5), token = chunk + row;
         const __amdgpu_buffer_rsrc_t ring = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pair < kChunk / 2 ? ring_k : ring_v), 0,
                                                                               static_cast<int>((t.mask + 1) * (2 * kHd)), 0x00020000);
         const bool there = pair < kChunk && token < t.t1 && token < t.n_ring;
-        const int at = there ? static_cast<int>(((t.u_first + token) & t.mask) * (2 * kHd) + 16 * (lane & 31u)) : -1024;
+        const int at = there ? static_cast<int>(((t.first + token) & t.mask) * (2 * kHd) + 16 * (lane & 31u)) : -1024;
         to.v[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ring, at, 0, 0));
     }
 }
-template <int R>
-__device__ __forceinline__ void put_rows(Shared<R>& sh, const Rows& from, uint32_t wave, uint32_t lane) {
+__device__ __forceinline__ void put_rows(Shared& sh, const Rows& from, uint32_t wave, uint32_t lane) {
 #pragma unroll
     for (uint32_t i = 0; i < 3; ++i) {
         const uint32_t pair = wave + kWorkers * i, row = 2 * (pair % (kChunk / 2)) + (lane >> 5);
@@ -291,19 +281,16 @@ __device__ __forceinline__ void norm_rotate(float (&v)[4], const HeadNorm& gamma
     }
 }
 
-template <int R, int G>
+template <int G>
 struct Pass {
-    static constexpr int NQ = R * G;
     static constexpr uint32_t CW = (G + 2) * kHd, TA = 4 * G + 8;
-    // Four or eight waves attend, a query each (two or four of them, where there are fewer queries): four are one a SIMD, and
-    // eight would share its issue slots.
-    static constexpr uint32_t WPQ = NQ < 4 ? 4 / NQ : 1, ATTENDING = WPQ * NQ;
+    // Four waves attend, WPQ of them a query: one a SIMD (eight would share its issue slots).  Two more prepare the row's key and value.
+    static constexpr uint32_t WPQ = 4 / G, ATTENDING = 4, PREPARING = 4;
     static constexpr uint32_t STEP = 4 * WPQ;                                  // tokens of a round
-    static constexpr uint32_t PREPARING = ATTENDING + 2 * R <= kWorkers ? ATTENDING : 0;   // first wave of those that prepare private rows
     const DArgs& a;
-    Shared<R>& sh;
+    Shared& sh;
     uint32_t lane;
-    const uint32_t wave, slot;
+    const uint32_t wave, slot, row;
     uint32_t generation = 0;
     __amdgpu_buffer_rsrc_t exchange;
 
@@ -327,98 +314,140 @@ struct Pass {
 
     __device__ __forceinline__ void enter() { lane = opaque(lane); }   // or every address that depends on the lane alone is kept in a register over the loop
     __device__ __forceinline__ void stamp(uint32_t l, uint32_t phase) const {
-        if (a.stamps && slot == 0 && lane == 0) a.stamps[l * 16 + phase] = wall_clock64();
+        if (a.stamps && row == 0 && slot == 0 && lane == 0) a.stamps[l * 16 + phase] = wall_clock64();
     }
 
+    __device__ __forceinline__ void give_up() const { sh.dead = 1u; atomicOr(a.status, GUFFIN_STATUS_SYNC); }
     // The last wave: its stores are in the L2, then the arrival, then the wait for the other workgroups.  A wait that gives up
     // raises the status bit, and the workgroup waits no more for the rest of the launch.
     __device__ __forceinline__ void arrive_and_wait() {
         __builtin_amdgcn_s_waitcnt(0);
         generation += 1;
         if (lane == 0 && !sh.dead) {
-            __hip_atomic_fetch_add(a.sync, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            uint32_t* counter = a.sync + row * kLine;
+            __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             const uint32_t target = kGroups * generation;
             uint32_t spins = 0;
-            while (__hip_atomic_load(a.sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-                if (++spins > a.spin_limit) {
-                    sh.dead = 1u;
-                    atomicOr(a.status, GUFFIN_STATUS_SYNC);
-                    break;
-                }
-            }
+            while (__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)
+                if (++spins > a.spin_limit) { give_up(); break; }
         }
         asm volatile("" ::: "memory");
     }
-    __device__ __forceinline__ float workers_sum(int matrix, int r) const {
-        float s = sh.red[0][matrix][r][lane];
+    __device__ __forceinline__ float workers_sum(int matrix) const {
+        float s = sh.red[0][matrix][lane];
 #pragma unroll
-        for (uint32_t w = 1; w < kWorkers; ++w) s += sh.red[w][matrix][r][lane];
+        for (uint32_t w = 1; w < kWorkers; ++w) s += sh.red[w][matrix][lane];
         return s;
+    }
+
+    // ---- rows of the same launch: the last wave hands keys and values on, 16 bytes a lane, keys in the lower half of the wave ----
+    using Words = uint32_t __attribute__((ext_vector_type(4)));
+    __device__ __forceinline__ uint16_t* private_rows(uint32_t l, uint32_t r) const {
+        return ((lane < 32 ? a.priv_k : a.priv_v) + (size_t(l) * a.rows + r) * kHd) + 8 * (lane & 31u);
+    }
+    __device__ __forceinline__ uint16_t* staged(uint32_t i) const { return (lane < 32 ? sh.kp_s[i] : sh.vp_s[i]) + 8 * (lane & 31u); }
+    // this row's, for the XCDs of later rows: past this L2 (sc1), then the flag
+    __device__ __forceinline__ void hand_on(uint32_t l, uint32_t i) const {
+        const uint2* from = reinterpret_cast<const uint2*>(staged(i));
+        unsigned long long* to = reinterpret_cast<unsigned long long*>(private_rows(l, row));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint2 w = from[h];
+            __hip_atomic_store(to + h, w.x | static_cast<unsigned long long>(w.y) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __builtin_amdgcn_s_waitcnt(0);
+        asm volatile("" ::: "memory");
+        if (lane == 0) __hip_atomic_store(a.sync + kFlagsAt + l * kRunRows + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // those of the private rows [from, to), counted from the first one attended, into their places in LDS
+    __device__ __forceinline__ void take_over(uint32_t l, const Tokens& t, uint32_t from, uint32_t to) const {
+        if (lane >= from && lane < to && !sh.dead) {
+            const uint32_t* flag = a.sync + kFlagsAt + l * kRunRows + t.priv_first + lane;
+            uint32_t spins = 0;
+            while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+                if (++spins > a.spin_limit) { give_up(); break; }
+        }
+        asm volatile("" ::: "memory");
+        for (uint32_t i0 = from; i0 < to; i0 += 4) {
+            unsigned long long w[4][2];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {   // past the last one the last again, unused
+                const unsigned long long* p = reinterpret_cast<const unsigned long long*>(private_rows(l, t.priv_first + min(i0 + i, to - 1)));
+                w[i][0] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                w[i][1] = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i)
+                if (i0 + i < to) {
+                    unsigned long long* p = reinterpret_cast<unsigned long long*>(staged(i0 + i));
+                    p[0] = w[i][0]; p[1] = w[i][1];
+                }
+        }
     }
 
     // What a wave's part in a block's attention needs and does not depend on the pass, asked for a phase ahead.
     __device__ __forceinline__ HeadNorm ask_gamma(const DLayer& L) const {
-        const bool key = PREPARING >= ATTENDING && wave >= PREPARING && wave < PREPARING + 2 * R;
-        return load_head_norm(L.weights[key ? 5 : 4], lane);
+        return load_head_norm(L.weights[wave == PREPARING ? 5 : 4], lane);
     }
 
-    // Every query of the rows against this workgroup's tokens.  The first chunk's rows lie in LDS, `rows` holds this worker's share
+    // Every query of the row against this workgroup's tokens.  The first chunk's rows lie in LDS, `rows` holds this worker's share
     // of the second one; a token per 16 lanes, lane s of them with dimensions 8s .. 8s+7 and 128 + 8s .. 128 + 8s + 7.
     template <typename First, typename Second>
-    __device__ __forceinline__ void attend(uint32_t l, const DLayer& L, const Tokens<R>& t, const HeadNorm& gamma, Rows& rows, First first_request, Second second_request) {
+    __device__ __forceinline__ void attend(uint32_t l, const DLayer& L, const Tokens& t, const HeadNorm& gamma, Rows& rows, First first_request, Second second_request) {
         constexpr uint32_t ROUNDS = (kChunk + STEP - 1) / STEP;
-        const uint32_t query = wave / WPQ, r = R > 1 ? query / G : 0, s16 = lane & 15u;
-        const float2* rope = sh.rope[L.local ? 0 : 1][0];
-        // the private rows' keys and values are the work of the workgroup whose tokens they are, a wave each
-        const bool owner = t.t1 > t.n_ring && t.t1 > t.t0;
-        const uint32_t pr = (wave - PREPARING) >> 1;
-        const bool prepares = owner && wave >= PREPARING && wave < PREPARING + 2 * R && t.n_ring + pr >= t.t0 && t.n_ring + pr < t.t1;
-        const bool is_key = ((wave - PREPARING) & 1u) == 0;
-        float2 v0 = make_float2(0.f, 0.f), v1 = v0, p0 = v0, p1 = v0;
-        HeadNorm key_gamma = gamma;
-        if (wave < ATTENDING) {
-            const uint32_t own = r * CW + (query % G) * kHd + 2 * lane;
-            v0 = ld2(a.qkv_at, own); v1 = ld2(a.qkv_at, own + 128);
-        }
-        if (prepares) {
-            const uint32_t src = pr * CW + (is_key ? G : G + 1) * kHd + 2 * lane;
-            p0 = ld2(a.qkv_at, src); p1 = ld2(a.qkv_at, src + 128);
-            if (PREPARING < ATTENDING && is_key) key_gamma = load_head_norm(L.weights[5], lane);
+        const uint32_t query = wave / WPQ, s16 = lane & 15u;
+        const float2* rope = sh.rope[L.local ? 0 : 1];
+        // private rows among this workgroup's tokens: this row's key and value are prepared here, a wave each, earlier rows' come
+        // from their XCDs
+        const uint32_t own = t.priv_count - 1, priv_from = max(t.t0, t.n_ring) - t.n_ring, priv_to = max(t.t1, t.n_ring) - t.n_ring;
+        const bool owner = priv_from <= own && own < priv_to, peers = min(priv_to, own) > priv_from;
+        const bool prepares = owner && wave >= PREPARING && wave < PREPARING + 2, is_key = wave == PREPARING;
+        float2 v0 = make_float2(0.f, 0.f), v1 = v0;
+        if (wave < ATTENDING || prepares) {
+            const uint32_t src = (wave < ATTENDING ? query : is_key ? G : G + 1) * kHd + 2 * lane;
+            v0 = ld2(a.qkv_at, src); v1 = ld2(a.qkv_at, src + 128);
         }
         arrived();
         first_request();
         float* q_s = sh.head[wave];
+        float v[4] = {v0.x, v0.y, v1.x, v1.y};
         if (wave < ATTENDING) {
-            float v[4] = {v0.x, v0.y, v1.x, v1.y};
-            norm_rotate(v, gamma, rope + r * (kHd / 2), a.eps, lane);
+            norm_rotate(v, gamma, rope, a.eps, lane);
             *reinterpret_cast<float2*>(q_s + 2 * lane) = make_float2(v[0] * a.scale, v[1] * a.scale);
             *reinterpret_cast<float2*>(q_s + 128 + 2 * lane) = make_float2(v[2] * a.scale, v[3] * a.scale);
         }
         if (prepares) {
-            float pv[4] = {p0.x, p0.y, p1.x, p1.y};
-            if (is_key) norm_rotate(pv, key_gamma, rope + pr * (kHd / 2), a.eps, lane);
+            if (is_key) norm_rotate(v, gamma, rope, a.eps, lane);
+            const bool passed_on = row + 1 < a.rows;   // the last wave's to store
             bool bad = false;
             uint32_t bits[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const _Float16 hv = static_cast<_Float16>(pv[k]);
+                const _Float16 hv = static_cast<_Float16>(v[k]);
                 bad |= !isfinite(static_cast<float>(hv));
                 bits[k] = __builtin_bit_cast(uint16_t, hv);
             }
-            uint16_t* to = (is_key ? sh.kp_s : sh.vp_s)[pr];
-            uint16_t* out = (is_key ? a.priv_k : a.priv_v) + (size_t(l) * R + pr) * kHd;
+            uint16_t* to = (is_key ? sh.kp_s : sh.vp_s)[own];
+            uint16_t* out = (is_key ? a.priv_k : a.priv_v) + (size_t(l) * a.rows + row) * kHd;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const uint32_t d = (k >> 1) * 128 + 2 * lane + (k & 1);
                 to[d] = static_cast<uint16_t>(bits[k]);
-                out[d] = static_cast<uint16_t>(bits[k]);
+                if (!passed_on) out[d] = static_cast<uint16_t>(bits[k]);
             }
             if (bad) atomicOr(a.status, GUFFIN_STATUS_KV_NONFINITE);
         }
-        if (owner) meet(); else own_lds();
+        if (owner) {
+            meet();
+            if (wave == kWorkers && row + 1 < a.rows) hand_on(l, own);
+        }
+        if (peers) {
+            if (wave == kWorkers) take_over(l, t, priv_from, min(priv_to, own));
+            meet();
+        }
+        if (!owner && !peers) own_lds();
         second_request();
         f4_t q[4];
-        const uint32_t first = t.first[R > 1 && r ? R - 1 : 0], end = t.end[R > 1 && r ? R - 1 : 0], attends = t.attends[R > 1 && r ? R - 1 : 0];
         float m = -INFINITY, sum = 0.f, acc[16];
         if (wave < ATTENDING) {
 #pragma unroll
@@ -433,7 +462,7 @@ struct Pass {
                 float s[ROUNDS];
                 // a token's row: a private one, or the chunk's (past the last token zeros, or what the chunk before left)
                 auto row_at = [&](uint32_t at, const uint16_t (*ring)[kHd], const uint16_t (*priv)[kHd]) {
-                    return (owner && chunk + at >= t.n_ring && chunk + at < t.t1 ? priv[chunk + at - t.n_ring] : ring[min(at, kChunk - 1)]) + 8 * s16;
+                    return (chunk + at >= t.n_ring && chunk + at < t.t1 ? priv[chunk + at - t.n_ring] : ring[min(at, kChunk - 1)]) + 8 * s16;
                 };
 #pragma unroll
                 for (uint32_t u = 0; u < ROUNDS; ++u) {
@@ -455,9 +484,7 @@ struct Pass {
                             }
                         }
                         const float dot = row16_sum(d[0] + d[1]);
-                        const uint32_t pos = t.u_first + token;
-                        const bool valid = token < chunk_end && (token >= t.n_ring ? ((attends >> (token - t.n_ring)) & 1u) != 0 : (pos >= first && pos < end));
-                        s[u] = valid ? dot : -INFINITY;
+                        s[u] = token < chunk_end ? dot : -INFINITY;
                     }
                 }
                 float top = m;
@@ -497,8 +524,8 @@ struct Pass {
             if (chunk + kChunk < t.t1) {   // a longer list: the next chunk takes this one's place
                 meet();
                 if (wave < kWorkers) {
-                    put_rows<R>(sh, rows, wave, lane);
-                    ask_rows<R>(rows, L.ring_k, L.ring_v, t, chunk + 2 * kChunk, wave, lane);
+                    put_rows(sh, rows, wave, lane);
+                    ask_rows(rows, L.ring_k, L.ring_v, t, chunk + 2 * kChunk, wave, lane);
                 }
                 meet();
             }
@@ -521,8 +548,8 @@ struct Pass {
         }
         const uint32_t at = (lane >> 5) * 128 + 8 * s16 + ((lane >> 4) & 1u) * 4;
         if constexpr (WPQ == 1) {
-            st4(a.out_at, (slot * NQ + query) * kHd + at, o);
-            if (lane == 0) st2(a.ml_at, (slot * NQ + query) * 2, make_float2(top, sum));
+            st4(a.out_at, (slot * G + query) * kHd + at, o);
+            if (lane == 0) st2(a.ml_at, (slot * G + query) * 2, make_float2(top, sum));
             arrived();
         } else {
             own_lds();   // the query has been read
@@ -534,7 +561,7 @@ struct Pass {
     // the last wave, where several share a query: the queries' outputs over this workgroup's tokens
     __device__ __forceinline__ void publish_attention() {
 #pragma unroll
-        for (int n = 0; n < NQ; ++n) {
+        for (int n = 0; n < G; ++n) {
             float top = sh.ml[n * WPQ].x;
 #pragma unroll
             for (uint32_t j = 1; j < WPQ; ++j) top = fmaxf(top, sh.ml[n * WPQ + j].x);
@@ -550,79 +577,65 @@ struct Pass {
                 for (int i = 0; i < 4; ++i) o[i] = fmaf(oj[i], f, o[i]);
                 sum = fmaf(mj.y, f, sum);
             }
-            st4(a.out_at, (slot * NQ + n) * kHd + 4 * lane, o);
-            if (lane == 0) st2(a.ml_at, (slot * NQ + n) * 2, make_float2(top, sum));
+            st4(a.out_at, (slot * G + n) * kHd + 4 * lane, o);
+            if (lane == 0) st2(a.ml_at, (slot * G + n) * 2, make_float2(top, sum));
         }
     }
 
     // A worker's quads of a row: those of its own blocks, one a lane.
     struct Own { Share blocks; bool on; uint32_t at; };
-    // The last of a row's sum of squares, over the workers' parts.  Every wave meets here.
-    __device__ __forceinline__ float row_total(int which, int r) const {
-        const f4_t lo = *reinterpret_cast<const f4_t*>(&sh.sums[which][r][0]), hi = *reinterpret_cast<const f4_t*>(&sh.sums[which][r][4]);
+    // The last of the row's sum of squares, over the workers' parts.  Every wave meets here.
+    __device__ __forceinline__ float row_total(int which) const {
+        const f4_t lo = *reinterpret_cast<const f4_t*>(&sh.sums[which][0]), hi = *reinterpret_cast<const f4_t*>(&sh.sums[which][4]);
         return ((lo.x + lo.y) + (lo.z + lo.w)) + ((hi.x + hi.y) + hi.z);
     }
     // x = x + rms(planes, post); the operand of this worker's blocks from rms(x, next).  Two meetings.
     // outputs: also written to memory (the state after the last block of the launch).
     template <typename First, typename Second, typename Third>
-    __device__ __forceinline__ void norm_pair(uint32_t planes, const f4_t& post, const f4_t& next, f4_t (&x)[R], const Own& own,
+    __device__ __forceinline__ void norm_pair(uint32_t planes, const f4_t& post, const f4_t& next, f4_t& x, const Own& own,
                                               bool outputs, First first_request, Second second_request, Third third_request) {
         const uint32_t H = a.H;
-        f4_t v[R], p1[R], p2[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            v[r] = ld4(planes, r * H + own.at);
-            p1[r] = ld4(planes, (R + r) * H + own.at);
-            p2[r] = ld4(planes, (2 * R + r) * H + own.at);
-        }
+        f4_t v = ld4(planes, own.at);
+        const f4_t p1 = ld4(planes, H + own.at), p2 = ld4(planes, 2 * H + own.at);
         arrived();
         first_request();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            v[r] = v[r] + p1[r] + p2[r];
-            float ss = (v[r].x * v[r].x + v[r].y * v[r].y) + (v[r].z * v[r].z + v[r].w * v[r].w);
-            ss = swap16_sum(row16_sum(own.on ? ss : 0.f));   // 24 lanes at most
-            if (lane == 0) sh.sums[0][r][wave] = ss;
-        }
+        v = v + p1 + p2;
+        float ss = (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+        ss = swap16_sum(row16_sum(own.on ? ss : 0.f));   // 24 lanes at most
+        if (lane == 0) sh.sums[0][wave] = ss;
         meet();
         second_request();
         bool bad = false;
+        float inv = 1.0f / sqrtf(row_total(0) / static_cast<float>(H) + a.eps);
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const float inv = 1.0f / sqrtf(row_total(0, r) / static_cast<float>(H) + a.eps);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                x[r][i] = v[r][i] * inv * post[i] + x[r][i];
-                bad |= !isfinite(x[r][i]);
-            }
-            float ss = (x[r].x * x[r].x + x[r].y * x[r].y) + (x[r].z * x[r].z + x[r].w * x[r].w);
-            ss = swap16_sum(row16_sum(own.on ? ss : 0.f));
-            if (lane == 0) sh.sums[1][r][wave] = ss;
+        for (int i = 0; i < 4; ++i) {
+            x[i] = v[i] * inv * post[i] + x[i];
+            bad |= !isfinite(x[i]);
         }
+        ss = (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w);
+        ss = swap16_sum(row16_sum(own.on ? ss : 0.f));
+        if (lane == 0) sh.sums[1][wave] = ss;
         meet();
         third_request();
+        inv = 1.0f / sqrtf(row_total(1) / static_cast<float>(H) + a.eps);
+        f4_t u;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const float inv = 1.0f / sqrtf(row_total(1, r) / static_cast<float>(H) + a.eps);
-            f4_t u;
+        for (int i = 0; i < 4; ++i) u[i] = x[i] * inv * next[i];
+        put_quad(u, lane, own.on, sh.opnd[wave], sh.mult[wave]);
+        if (outputs) {
+            float* part = sh.head[wave];   // attention is over: room for the wave's part of the row
+            if (own.on) {
+                *reinterpret_cast<f4_t*>(a.x_out + size_t(row) * H + own.at) = x;
+                *reinterpret_cast<f4_t*>(a.u_out + size_t(row) * H + own.at) = u;
+                if (a.u_last && row + 1 == a.rows) *reinterpret_cast<f4_t*>(a.u_last + own.at) = u;
+                *reinterpret_cast<f4_t*>(part + 4 * lane) = u;
+            }
+            own_lds();
+            if (a.u_receipt_out && (a.receipt_rows > 1 || row + 1 == a.rows) && lane < 4 * own.blocks.count) {
+                float y[8];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[i] = x[r][i] * inv * next[i];
-            put_quad(u, lane, own.on, sh.opnd[wave][r], sh.mult[wave][r]);
-            if (outputs) {
-                float* row = sh.head[wave];   // attention is over: room for the wave's part of the row
-                if (own.on) {
-                    *reinterpret_cast<f4_t*>(a.x_out + size_t(r) * H + own.at) = x[r];
-                    *reinterpret_cast<f4_t*>(a.u_out + size_t(r) * H + own.at) = u;
-                    *reinterpret_cast<f4_t*>(row + 4 * lane) = u;
-                }
-                own_lds();
-                if (a.u_receipt_out && lane < 4 * own.blocks.count) {
-                    float y[8];
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) y[i] = row[8 * lane + i];
-                    emit_receipt_values(y, 32 * own.blocks.first, lane, r, R, H, a.u_receipt_out);
-                }
-                own_lds();
+                for (int i = 0; i < 8; ++i) y[i] = part[8 * lane + i];
+                emit_receipt_values(y, 32 * own.blocks.first, lane, a.receipt_rows > 1 ? row : 0u, a.receipt_rows, H, a.u_receipt_out);
             }
         }
         if (bad && own.on) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
@@ -635,14 +648,12 @@ struct Pass {
         for (uint32_t l = 0; l < a.layers; ++l) {
             const DLayer& L = a.layer[l];
             enter();
-            const Tokens<R> t = tokens_of<R>(sh, l, L.ring_mask, slot);
+            const Tokens t = tokens_of(sh, l, L.ring_mask, slot);
             Rows none;
             const HeadNorm gamma = ask_gamma(L);
             stamp(l, 0);
             meet();
-            if (slot < TA)
-#pragma unroll
-                for (int r = 0; r < R; ++r) st(a.qkv_at, r * CW + slot * 64 + lane, workers_sum(0, r));
+            if (slot < TA) st(a.qkv_at, slot * 64 + lane, workers_sum(0));
             arrive_and_wait();
             stamp(l, 1);
             meet();
@@ -655,9 +666,7 @@ struct Pass {
             // o-projection
             meet();
             stamp(l, 3);
-            if (part < kParts)
-#pragma unroll
-                for (int r = 0; r < R; ++r) st(a.o_at, (part * R + r) * a.H + column, workers_sum(0, r));
+            if (part < kParts) st(a.o_at, part * a.H + column, workers_sum(0));
             arrive_and_wait();
             stamp(l, 4);
             meet();
@@ -666,17 +675,13 @@ struct Pass {
             meet();
             meet();
             stamp(l, 5);
-            if (slot < a.F / 64)
-#pragma unroll
-                for (int r = 0; r < R; ++r) st(a.h_at, r * a.F + slot * 64 + lane, geglu_value(workers_sum(0, r), workers_sum(1, r)));
+            if (slot < a.F / 64) st(a.h_at, slot * 64 + lane, geglu_value(workers_sum(0), workers_sum(1)));
             arrive_and_wait();
             stamp(l, 6);
             meet();
             // down
             meet();
-            if (part < kParts)
-#pragma unroll
-                for (int r = 0; r < R; ++r) st(a.d_at, (part * R + r) * a.H + column, workers_sum(0, r));
+            if (part < kParts) st(a.d_at, part * a.H + column, workers_sum(0));
             arrive_and_wait();
             stamp(l, 7);
             meet();
@@ -715,7 +720,7 @@ struct Pass {
         // workgroup, which one XCD takes 1.1 to 2 us to fetch (1.3 TB/s); in front of a phase's products that is what the products
         // wait for, behind them what the last wave's store and poll do.
         Tile tq[kOwn], to[kOwnO], tg[kOwn], tu[kOwn], td[kOwnDown];
-        f4_t post, next, x[R];
+        f4_t post, next, x;
         Rows rows;
         HeadNorm gamma;
         auto ask_q = [&](const DLayer& from, int i) { ask_tile(tq[i], from.tiles[qm] + q_at, i, own.blocks.count, lane); };
@@ -730,46 +735,36 @@ struct Pass {
             for (int i = 0; i < kOwnO; ++i) ask_o(L, i);
             for (int i = 0; i < kOwn; ++i) ask_gate(L, i);
             for (int i = 0; i < 1; ++i) ask_up(L, i);
-            const Tokens<R> t = tokens_of<R>(sh, 0, L.ring_mask, slot);
-            ask_rows<R>(rows, L.ring_k, L.ring_v, t, t.t0, wave, lane);
+            const Tokens t = tokens_of(sh, 0, L.ring_mask, slot);
+            ask_rows(rows, L.ring_k, L.ring_v, t, t.t0, wave, lane);
             gamma = ask_gamma(L);
         }
         auto norm_weights = [&](const float* p, const float* n) {
             const float4 vp = ldf4_a4(p + own.at), vn = ldf4_a4(n + own.at);
             post = f4_t{vp.x, vp.y, vp.z, vp.w}; next = f4_t{vn.x, vn.y, vn.z, vn.w};
         };
-        // the rows and the operand that the launch starts from
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            x[r] = *reinterpret_cast<const f4_t*>(a.x_in + size_t(r) * H + own.at);
-            const f4_t u = *reinterpret_cast<const f4_t*>(a.u_in + size_t(r) * H + own.at);
-            put_quad(u, lane, own.on, sh.opnd[wave][r], sh.mult[wave][r]);
-        }
+        // the row and the operand that the launch starts from
+        x = *reinterpret_cast<const f4_t*>(a.x_in + size_t(row) * H + own.at);
+        put_quad(*reinterpret_cast<const f4_t*>(a.u_in + size_t(row) * H + own.at), lane, own.on, sh.opnd[wave], sh.mult[wave]);
         own_lds();
-        auto publish = [&](const float (&acc)[R], int matrix) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) sh.red[wave][matrix][r][lane] = acc[r];
-        };
+        auto publish = [&](float acc, int matrix) { sh.red[wave][matrix][lane] = acc; };
         for (uint32_t l = 0; l < a.layers; ++l) {
             const DLayer& L = a.layer[l];
             const uint32_t ln = l + 1 < a.layers ? l + 1 : l;   // past the last block: this one's again, unused
             const DLayer& N = a.layer[ln];
             enter();
-            float acc[R];
             // ---- q, k, v -----------------------------------------------------------------------------------
             {
-                int op[R][2];
-                i4_t D[kOwn][R];
-#pragma unroll
-                for (int r = 0; r < R; ++r) read_operand(op[r], sh.opnd[wave][r], lane);
+                int op[2];
+                i4_t D[kOwn];
+                read_operand(op, sh.opnd[wave], lane);
                 steps(tq, op, D);
-                fold(tq, own.blocks.count, D, sh.mult[wave], acc);
-                publish(acc, 0);
+                publish(fold(tq, own.blocks.count, D, sh.mult[wave]), 0);
             }
-            put_rows<R>(sh, rows, wave, lane);
+            put_rows(sh, rows, wave, lane);
             meet();
-            const Tokens<R> t = tokens_of<R>(sh, l, L.ring_mask, slot);
-            if (t.t0 + kChunk < t.t1) ask_rows<R>(rows, L.ring_k, L.ring_v, t, t.t0 + kChunk, wave, lane);
+            const Tokens t = tokens_of(sh, l, L.ring_mask, slot);
+            if (t.t0 + kChunk < t.t1) ask_rows(rows, L.ring_k, L.ring_v, t, t.t0 + kChunk, wave, lane);
             meet();
             // ---- attention ---------------------------------------------------------------------------------
             attend(l, L, t, gamma, rows, [&] { ask_up(L, 1); }, [&] { ask_up(L, 2); });
@@ -781,124 +776,102 @@ struct Pass {
             {
                 // 16 lanes hold the 64 elements, four each; lane group g the partitions 4 i + g
                 const uint32_t head = (64 * o_pair) / kHd, dim = (64 * o_pair) % kHd, g = lane >> 4, s16 = lane & 15u;
-                f4_t pv[R][kGroups / 4];
-                float2 ml[R];
+                f4_t pv[kGroups / 4];
+                const float2 ml = ld2(a.ml_at, ((lane & 31u) * G + head) * 2);
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const uint32_t n = r * G + head;
-                    ml[r] = ld2(a.ml_at, ((lane & 31u) * NQ + n) * 2);
-#pragma unroll
-                    for (uint32_t i = 0; i < kGroups / 4; ++i)
-                        pv[r][i] = ld4(a.out_at + (4 * i * NQ * kHd + n * kHd + dim) * 4, g * (NQ * kHd) + 4 * s16);
-                }
+                for (uint32_t i = 0; i < kGroups / 4; ++i)
+                    pv[i] = ld4(a.out_at + (4 * i * G * kHd + head * kHd + dim) * 4, g * (G * kHd) + 4 * s16);
                 arrived();
                 ask_down(L, 2);
                 norm_weights(L.weights[0], L.weights[1]);
-                float den[R];
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    float top = ml[r].y > 0.f ? ml[r].x : -INFINITY;
-                    top = swap16_max(row16_max(top));
-                    const float w = ml[r].y > 0.f ? expf(ml[r].x - top) : 0.f;
-                    den[r] = swap16_sum(row16_sum(w * ml[r].y));
-                    if (lane < kGroups) sh.weight[wave][r][8 * (lane & 3u) + (lane >> 2)] = w;
-                }
+                float top = ml.y > 0.f ? ml.x : -INFINITY;
+                top = swap16_max(row16_max(top));
+                const float w = ml.y > 0.f ? expf(ml.x - top) : 0.f;
+                const float den = swap16_sum(row16_sum(w * ml.y));
+                if (lane < kGroups) sh.weight[wave][8 * (lane & 3u) + (lane >> 2)] = w;
                 own_lds();
-                bool bad = false;
+                const f4_t w0 = *reinterpret_cast<const f4_t*>(&sh.weight[wave][8 * g]), w1 = *reinterpret_cast<const f4_t*>(&sh.weight[wave][8 * g + 4]);
+                f4_t e = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const f4_t w0 = *reinterpret_cast<const f4_t*>(&sh.weight[wave][r][8 * g]), w1 = *reinterpret_cast<const f4_t*>(&sh.weight[wave][r][8 * g + 4]);
-                    f4_t e = {0.f, 0.f, 0.f, 0.f};
+                for (uint32_t i = 0; i < kGroups / 4; ++i)
 #pragma unroll
-                    for (uint32_t i = 0; i < kGroups / 4; ++i)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) e[j] = fmaf(i < 4 ? w0[i & 3] : w1[i & 3], pv[r][i][j], e[j]);
-                    // element 4 s16 + g is left in this lane
-                    const u2_t x = __builtin_amdgcn_permlane32_swap(__float_as_uint(e.x), __float_as_uint(e.z), false, false);
-                    const u2_t y = __builtin_amdgcn_permlane32_swap(__float_as_uint(e.y), __float_as_uint(e.w), false, false);
-                    const u2_t z = __builtin_amdgcn_permlane16_swap(__float_as_uint(__uint_as_float(x.x) + __uint_as_float(x.y)),
-                                                                    __float_as_uint(__uint_as_float(y.x) + __uint_as_float(y.y)), false, false);
-                    const float v = (__uint_as_float(z.x) + __uint_as_float(z.y)) / den[r];
-                    bad |= o_on && !isfinite(v);
-                    uint32_t m = magnitude(v);
-                    m = max(m, lane_cross_u32<0xB1, 0xF>(m));
-                    m = max(m, lane_cross_u32<0x4E, 0xF>(m));
-                    m = max(m, lane_cross_u32<0x141, 0xF>(m));
-                    const u2_t m16 = __builtin_amdgcn_permlane16_swap(m, m, false, false);
-                    m = max(m16.x, m16.y);
-                    const u2_t m32 = __builtin_amdgcn_permlane32_swap(m, m, false, false);
-                    const GroupScale scale = group_scale(max(m32.x, m32.y));
-                    sh.opnd[wave][r][4 * s16 + g] = digits(v, scale.scale);
-                    if ((lane & 0x37u) == 0) sh.mult[wave][r][s16 >> 3] = scale.mult;
-                }
-                if (bad) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
+                    for (int j = 0; j < 4; ++j) e[j] = fmaf(i < 4 ? w0[i & 3] : w1[i & 3], pv[i][j], e[j]);
+                // element 4 s16 + g is left in this lane
+                const u2_t ex = __builtin_amdgcn_permlane32_swap(__float_as_uint(e.x), __float_as_uint(e.z), false, false);
+                const u2_t ey = __builtin_amdgcn_permlane32_swap(__float_as_uint(e.y), __float_as_uint(e.w), false, false);
+                const u2_t ez = __builtin_amdgcn_permlane16_swap(__float_as_uint(__uint_as_float(ex.x) + __uint_as_float(ex.y)),
+                                                                 __float_as_uint(__uint_as_float(ey.x) + __uint_as_float(ey.y)), false, false);
+                const float v = (__uint_as_float(ez.x) + __uint_as_float(ez.y)) / den;
+                uint32_t m = magnitude(v);
+                m = max(m, lane_cross_u32<0xB1, 0xF>(m));
+                m = max(m, lane_cross_u32<0x4E, 0xF>(m));
+                m = max(m, lane_cross_u32<0x141, 0xF>(m));
+                const u2_t m16 = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+                m = max(m16.x, m16.y);
+                const u2_t m32 = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+                const GroupScale scale = group_scale(max(m32.x, m32.y));
+                sh.opnd[wave][4 * s16 + g] = digits(v, scale.scale);
+                if ((lane & 0x37u) == 0) sh.mult[wave][s16 >> 3] = scale.mult;
+                if (o_on && !isfinite(v)) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
                 ask_down(L, 3);
                 own_lds();
-                int op[R][1];
-                i4_t D[kOwnO][R];
-#pragma unroll
-                for (int r = 0; r < R; ++r) read_operand(op[r], sh.opnd[wave][r], lane);
+                int op[1];
+                i4_t D[kOwnO];
+                read_operand(op, sh.opnd[wave], lane);
                 steps(to, op, D);
-                fold(to, o_on ? 2u : 0u, D, sh.mult[wave], acc);
-                publish(acc, 0);
+                publish(fold(to, o_on ? 2u : 0u, D, sh.mult[wave]), 0);
             }
             meet();
             meet();
             // ---- x1 = x + rms(o, post_attention_norm); rms(x1, ffn_norm); gate and up ---------------------
             norm_pair(a.o_at, post, next, x, own, false, [&] { ask_o(N, 0); ask_o(N, 1); }, [] {}, [] {});
             {
-                int op[R][2];
-                i4_t D[kOwn][R], E[kOwn][R];
-#pragma unroll
-                for (int r = 0; r < R; ++r) read_operand(op[r], sh.opnd[wave][r], lane);
+                int op[2];
+                i4_t D[kOwn], E[kOwn];
+                read_operand(op, sh.opnd[wave], lane);
                 steps(tg, op, D);
                 steps(tu, op, E);
-                fold(tg, own.blocks.count, D, sh.mult[wave], acc);
-                publish(acc, 0);
-                fold(tu, own.blocks.count, E, sh.mult[wave], acc);
-                publish(acc, 1);
+                publish(fold(tg, own.blocks.count, D, sh.mult[wave]), 0);
+                publish(fold(tu, own.blocks.count, E, sh.mult[wave]), 1);
             }
             meet();
             meet();
             // ---- down --------------------------------------------------------------------------------------
             {
-                f4_t hv[R];
                 const uint32_t at = 32 * d_first + 4 * min(lane, 8 * max(d_own.count, 1u) - 1);
-#pragma unroll
-                for (int r = 0; r < R; ++r) hv[r] = ld4(a.h_at, r * F + at);
+                const f4_t hv = ld4(a.h_at, at);
                 arrived();
                 ask_q(N, 0);
                 ask_q(N, 1);
                 ask_q(N, 2);
                 norm_weights(L.weights[2], L.weights[3]);
-#pragma unroll
-                for (int r = 0; r < R; ++r) put_quad(hv[r], lane, lane < 8 * d_own.count, sh.opnd[wave][r], sh.mult[wave][r]);
+                put_quad(hv, lane, lane < 8 * d_own.count, sh.opnd[wave], sh.mult[wave]);
                 ask_gate(N, 0);
                 own_lds();
-                int op[R][2];
-                i4_t D[kOwnDown][R];
-#pragma unroll
-                for (int r = 0; r < R; ++r) read_operand(op[r], sh.opnd[wave][r], lane);
+                int op[2];
+                i4_t D[kOwnDown];
+                read_operand(op, sh.opnd[wave], lane);
                 steps(td, op, D);
-                fold(td, d_own.count, D, sh.mult[wave], acc);
-                publish(acc, 0);
+                publish(fold(td, d_own.count, D, sh.mult[wave]), 0);
             }
             meet();
-            const Tokens<R> tn = tokens_of<R>(sh, ln, N.ring_mask, slot);
+            const Tokens tn = tokens_of(sh, ln, N.ring_mask, slot);
             meet();
             // ---- x = x1 + rms(down, post_ffw_norm); rms(x, next block's attn_norm or the output norm) -----
             norm_pair(a.d_at, post, next, x, own, l + 1 == a.layers && slot == 0, [&] { ask_gate(N, 1); },
-                      [&] { ask_gate(N, 2); ask_rows<R>(rows, N.ring_k, N.ring_v, tn, tn.t0, wave, lane); gamma = ask_gamma(N); }, [&] { ask_up(N, 0); });
+                      [&] { ask_gate(N, 2); ask_rows(rows, N.ring_k, N.ring_v, tn, tn.t0, wave, lane); gamma = ask_gamma(N); }, [&] { ask_up(N, 0); });
         }
     }
 };
 
-template <int R, int G>
+template <int G>
 __global__ void __launch_bounds__(kThreads) drafter_blocks_kernel(const DArgs a) {
-    __shared__ __attribute__((aligned(256))) Shared<R> sh;
-    if (xcc_id() != 0) return;   // the model has one KV head: the other XCDs leave at once
+    __shared__ __attribute__((aligned(256))) Shared sh;
+    const uint32_t row = uniform(xcc_id());   // the model has one KV head: a row an XCD
+    if (row >= a.rows) return;
     const uint32_t lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-    Pass<R, G> pass {a, sh, lane, wave, blockIdx.x / 8, 0, __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, static_cast<int>(a.exchange_bytes), 0x00020000)};
+    Pass<G> pass {a, sh, lane, wave, blockIdx.x / 8, row, 0,
+                  __builtin_amdgcn_make_buffer_rsrc(a.exchange + size_t(row) * a.exchange_bytes, 0, static_cast<int>(a.exchange_bytes), 0x00020000)};
     // The arguments' lines, once, all at a time: they come from far, and a block's pointers otherwise cost a wait at each first use.
     {
         uint64_t seen = 0;
@@ -909,17 +882,9 @@ __global__ void __launch_bounds__(kThreads) drafter_blocks_kernel(const DArgs a)
     }
     // the rotations and the schedules
     if (threadIdx.x == 0) sh.dead = 0;
-    for (uint32_t i = threadIdx.x; i < 2 * R * (kHd / 2); i += kThreads) {
-        const uint32_t at = i % (R * (kHd / 2));
-        (&sh.rope[0][0][0])[i] = i < R * (kHd / 2) ? a.rope_local[at] : a.rope_global[at];
-    }
-    for (uint32_t i = threadIdx.x; i < a.layers * R; i += kThreads) {
-        const uint32_t* s = a.schedule + 4 * i;
-        uint32_t attends = 0;
-        for (uint32_t k = 0; k < s[3]; ++k) attends |= 1u << a.ancestors[s[2] + k];
-        uint32_t* to = sh.schedule[i / R][i % R];
-        to[0] = s[0]; to[1] = s[1]; to[2] = attends;
-    }
+    for (uint32_t i = threadIdx.x; i < 2 * (kHd / 2); i += kThreads)
+        (&sh.rope[0][0])[i] = (i < kHd / 2 ? a.rope_local : a.rope_global)[row * (kHd / 2) + i % (kHd / 2)];
+    for (uint32_t i = threadIdx.x; i < 4 * a.layers; i += kThreads) sh.schedule[i / 4][i % 4] = a.schedule[4 * (i / 4 * a.rows + row) + i % 4];
     __syncthreads();
     if (wave == kWorkers) pass.publisher();
     else pass.worker();
@@ -941,27 +906,36 @@ bool drafter_pass_fits(const guffin_model_desc& m) {
     return true;
 }
 
-int drafter_pass(hipStream_t stream, const guffin_model_desc& m, uint32_t rows, const DrafterPass& p) {
-    DArgs a {};
-    a.H = m.hidden; a.F = m.ffn; a.eps = m.eps; a.scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
-    a.exchange = p.exchange;
-    const uint32_t NQ = rows * m.q_heads;
+// where the regions of a row's exchange buffers start; they start on cache lines of their own
+static uint32_t lay_out(const guffin_model_desc& m, DArgs& a) {
     uint32_t used = 0;
-    auto take = [&](uint32_t floats) {   // regions start on cache lines of their own
+    auto take = [&](uint32_t floats) {
         const uint32_t at = used;
         used += (floats * 4 + 255) & ~255u;
         return at;
     };
-    a.qkv_at = take(rows * (m.q_heads + 2) * kHd);
-    a.out_at = take(kGroups * NQ * kHd);
-    a.ml_at = take(kGroups * NQ * 2);
-    a.o_at = take(kParts * rows * m.hidden);
-    a.d_at = take(kParts * rows * m.hidden);
-    a.h_at = take(rows * m.ffn);
-    a.exchange_bytes = used;
-    if (used > resident_scratch_bytes(m, rows)) return fail(GUFFIN_E_CAPACITY, "drafter pass: exchange buffers");
+    a.qkv_at = take((m.q_heads + 2) * kHd);
+    a.out_at = take(kGroups * m.q_heads * kHd);
+    a.ml_at = take(kGroups * m.q_heads * 2);
+    a.o_at = take(kParts * m.hidden);
+    a.d_at = take(kParts * m.hidden);
+    a.h_at = take(m.ffn);
+    return used;
+}
+uint64_t drafter_pass_bytes(const guffin_model_desc& m, uint32_t rows) {
+    DArgs a {};
+    return uint64_t(rows) * lay_out(m, a);
+}
+uint32_t drafter_pass_sync_words(const guffin_model_desc& m) { return (m.layer_count + kLayers - 1) / kLayers * kSyncWords; }
+
+int drafter_pass(hipStream_t stream, const guffin_model_desc& m, uint32_t rows, const DrafterPass& p) {
+    if (rows < 1 || rows > kRunRows) return fail(GUFFIN_E_SHAPE, "drafter pass: rows");
+    DArgs a {};
+    a.rows = rows; a.H = m.hidden; a.F = m.ffn; a.eps = m.eps; a.scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
+    a.exchange = p.exchange;
+    a.exchange_bytes = lay_out(m, a);
     a.rope_local = reinterpret_cast<const float2*>(p.rope_local); a.rope_global = reinterpret_cast<const float2*>(p.rope_global);
-    a.ancestors = p.ancestors; a.status = p.status; a.spin_limit = g_spin_limit;
+    a.status = p.status; a.spin_limit = g_spin_limit;
     for (uint32_t first = 0, n = 0; first < m.layer_count; first += kLayers, ++n) {
         a.layers = std::min(kLayers, m.layer_count - first);
         for (uint32_t i = 0; i < a.layers; ++i) {
@@ -977,21 +951,20 @@ int drafter_pass(hipStream_t stream, const guffin_model_desc& m, uint32_t rows, 
             d.ring_mask = (d.local ? m.ring_local : m.ring_global) - 1;
         }
         const bool last = first + a.layers == m.layer_count;
-        a.sync = p.sync + n * kSyncStride;
+        a.sync = p.sync + n * kSyncWords;
         a.schedule = p.schedule + size_t(first) * rows * 4;
         a.priv_k = static_cast<uint16_t*>(p.priv_k) + size_t(first) * rows * kHd;
         a.priv_v = static_cast<uint16_t*>(p.priv_v) + size_t(first) * rows * kHd;
         a.x_in = p.x; a.u_in = p.u; a.x_out = p.x;
         a.u_out = last ? p.out_hidden : p.u;
+        a.u_last = last ? p.last_hidden : nullptr;
         a.u_receipt_out = last ? p.out_sums : nullptr;
+        a.receipt_rows = p.receipt_rows;
         a.stamps = g_resident_stamps ? g_resident_stamps + size_t(first) * 16 : nullptr;
-        switch (rows * 10 + m.q_heads) {
-            case 11: launch(drafter_blocks_kernel<1, 1>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
-            case 12: launch(drafter_blocks_kernel<1, 2>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
-            case 14: launch(drafter_blocks_kernel<1, 4>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
-            case 21: launch(drafter_blocks_kernel<2, 1>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
-            case 22: launch(drafter_blocks_kernel<2, 2>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
-            case 24: launch(drafter_blocks_kernel<2, 4>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+        switch (m.q_heads) {
+            case 1: launch(drafter_blocks_kernel<1>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+            case 2: launch(drafter_blocks_kernel<2>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
+            case 4: launch(drafter_blocks_kernel<4>, dim3(kGrid), dim3(kThreads), 0, stream, a); break;
             default: return fail(GUFFIN_E_SHAPE, "drafter pass: unsupported head grouping");
         }
         if (int rc = check_launch("drafter_blocks")) return rc;

@@ -164,7 +164,9 @@ void row_schedule(const guffin_model_desc& m, uint32_t layer, uint32_t position,
 // (r itself for contiguous rows; a tree's schedule travels with its launches, it asks for no layers here)
 struct Staging {
     uint32_t *positions, *ancestors, *schedule;
-    uint32_t rows, position, depths, layers, window, global_period;
+    uint32_t rows, position;
+    uint64_t depths;
+    uint32_t layers, window, global_period;
     float2 *rope_local, *rope_global;
     uint32_t rope_dim;
     float local_base, global_base, global_scale;
@@ -174,7 +176,7 @@ struct Staging {
 __device__ __forceinline__ void stage_item(const Staging& p, uint32_t i) {
     if (i < p.sync_words) p.sync[i] = 0u;   // barrier counters of the resident pass start at zero
     const uint32_t half = p.rope_dim / 2, rows = p.rows;
-    auto at = [&](uint32_t row) { return p.position + ((p.depths >> (8 * row)) & 255u); };
+    auto at = [&](uint32_t row) { return p.position + uint32_t((p.depths >> (8 * row)) & 255u); };
     if (i < rows * half) {
         float c, s;
         if (p.global_period > 1) {  // a model without local blocks has no local base
@@ -243,6 +245,7 @@ enter_rows_kernel(const uint32_t* __restrict__ tokens, const uint8_t* __restrict
         u[size_t(r) * width + c] = v;
     }
     if (bad && status) atomicOr(status, GUFFIN_STATUS_NONFINITE);
+    if (!u_sums) return;   // the drafter's pass forms its own operand
     lds_barrier();
     emit_receipt(row, 0, width, r, rows, width, u_sums, threadIdx.x, threads);
 }
@@ -305,22 +308,16 @@ int block_tail(void* st, const guffin_model_desc& m, uint32_t l, const Scratch& 
 // below `position` (through its window) and the rows of ancestors[r], a bit each, itself among them
 struct TreeRows { uint32_t depth[kWideRows], ancestors[kWideRows]; };
 
-int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t* tokens, uint32_t rows,
-                 uint32_t position, const Scratch& s, void* priv_k, void* priv_v, float* out_hidden,
-                 float* out_hidden_sums, uint32_t* status, const TreeRows* tree = nullptr) {
+// What a pass starts from: the rows' embeddings (s.x), their first norm (s.u, its receipt in s.us unless that is null), the staging.
+int enter_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t* tokens, uint32_t rows, uint32_t position, const Scratch& s,
+               uint32_t sync_words, uint32_t* status, const TreeRows* tree = nullptr) {
     void* st = stream;
-    const uint32_t H = m.hidden, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
-    const float attn_scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
-    // the resident passes are the default for models with a single KV head (resident_chosen has the figures) and can be forced for any
-    // model they cover, for runs of rows: a tree always goes one launch per operator
-    const bool resident = s.exchange != nullptr && resident_chosen(m, rows) && !tree;
-    if (g_forward_mode == 2 && !resident && !tree) return fail(GUFFIN_E_SHAPE, "forward: the resident pass does not cover this model");
-    const uint32_t sync_words = resident ? s.sync_words : 0u;
+    const uint32_t H = m.hidden;
     const uint32_t n_stage = std::max({m.layer_count * rows, rows * (m.head_dim / 2), sync_words});
-    uint32_t depths = 0x03020100u;
+    uint64_t depths = 0x0706050403020100u;
     if (tree) {
         depths = 0;
-        for (uint32_t r = 0; r < rows; ++r) depths |= tree->depth[r] << (8 * r);
+        for (uint32_t r = 0; r < rows; ++r) depths |= uint64_t(tree->depth[r]) << (8 * r);
     }
     const Staging staging {s.positions, s.ancestors, s.schedule, rows, position, depths, tree ? 0u : m.layer_count, m.sliding_window,
                            m.global_period, reinterpret_cast<float2*>(s.rope_local), reinterpret_cast<float2*>(s.rope_global), m.head_dim,
@@ -338,16 +335,34 @@ int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t*
                                 status, staging)
         if (format == GUFFIN_Q8_0) GUFFIN_ENTER(GUFFIN_Q8_0); else if (format == GUFFIN_Q4_K) GUFFIN_ENTER(GUFFIN_Q4_K); else GUFFIN_ENTER(GUFFIN_Q6_K);
 #undef GUFFIN_ENTER
-        GUFFIN_TRY(check_launch("enter_rows"));
-    } else {
-        launch(stage_rows_kernel, dim3((n_stage + 63) / 64), dim3(64), 0, stream, staging);
-        GUFFIN_TRY(check_launch("stage_rows"));
-        GUFFIN_TRY(guffin_hip_embed(st, m.embed_dtype, m.embed_rows, tokens, s.x, rows, H, scale, m.vocab, status));
-        GUFFIN_TRY(guffin_hip_rms_norm(st, s.x, 1, 0, gamma, nullptr, s.u, s.us, rows, H, m.eps, status));
+        return check_launch("enter_rows");
     }
-    if (resident && drafter_pass_fits(m))
-        return drafter_pass(stream, m, rows, {s.exchange, s.sync, s.rope_local, s.rope_global, s.schedule, s.ancestors, priv_k, priv_v,
-                                              s.x, s.u, out_hidden, out_hidden_sums, status});
+    launch(stage_rows_kernel, dim3((n_stage + 63) / 64), dim3(64), 0, stream, staging);
+    GUFFIN_TRY(check_launch("stage_rows"));
+    GUFFIN_TRY(guffin_hip_embed(st, m.embed_dtype, m.embed_rows, tokens, s.x, rows, H, scale, m.vocab, status));
+    return guffin_hip_rms_norm(st, s.x, 1, 0, gamma, nullptr, s.u, s.us, rows, H, m.eps, status);
+}
+
+int forward_rows(hipStream_t stream, const guffin_model_desc& m, const uint32_t* tokens, uint32_t rows,
+                 uint32_t position, const Scratch& s, void* priv_k, void* priv_v, float* out_hidden,
+                 float* out_hidden_sums, uint32_t* status, const TreeRows* tree = nullptr) {
+    void* st = stream;
+    const uint32_t H = m.hidden, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;
+    const float attn_scale = 1.0f / std::sqrt(static_cast<float>(m.head_dim));
+    // the resident passes are the default for models with a single KV head (resident_chosen has the figures) and can be forced for any
+    // model they cover, for runs of rows: a tree always goes one launch per operator
+    const bool resident = s.exchange != nullptr && resident_chosen(m, rows) && !tree;
+    if (g_forward_mode == 2 && !resident && !tree) return fail(GUFFIN_E_SHAPE, "forward: the resident pass does not cover this model");
+    if (resident && drafter_pass_fits(m)) {
+        if (drafter_pass_bytes(m, rows) > resident_scratch_bytes(m, rows) || drafter_pass_sync_words(m) > s.sync_words)
+            return fail(GUFFIN_E_CAPACITY, "forward: the drafter pass' exchange buffers");
+        Scratch entered = s;
+        entered.us = nullptr;
+        GUFFIN_TRY(enter_rows(stream, m, tokens, rows, position, entered, drafter_pass_sync_words(m), status));
+        return drafter_pass(stream, m, rows, {s.exchange, s.sync, s.rope_local, s.rope_global, s.schedule, priv_k, priv_v,
+                                              s.x, s.u, out_hidden, nullptr, out_hidden_sums, rows, status});
+    }
+    GUFFIN_TRY(enter_rows(stream, m, tokens, rows, position, s, resident ? s.sync_words : 0u, status, tree));
     if (resident) {
         // groups of blocks, each one launch whose workgroups stay on the chip; the residual rows and the
         // normalised rows' receipt pass from launch to launch through s.x / s.us
@@ -499,6 +514,39 @@ extern "C" int guffin_hip_forward_rows(void* stream, const guffin_model_desc* mo
     if (s.bytes > scratch_bytes) return fail(GUFFIN_E_CAPACITY, "forward_rows: scratch arena too small");
     return forward_rows(as_stream(stream), *model, tokens, rows, position, s, priv_k, priv_v, out_hidden,
                         out_hidden_sums, status);
+}
+
+// ---- contiguous rows of the drafter's pass, an XCD each ------------------------------------------
+bool guffin::forward_run_chosen(const guffin_model_desc& m) { return resident_chosen(m, 1) && drafter_pass_fits(m); }
+
+static Scratch run_layout(const guffin_model_desc& m, uint8_t* base) {
+    Arena ar {base, 0, 0};
+    Scratch s {};
+    s.x = ar.take<float>(uint64_t(kRunRows) * m.hidden);
+    s.u = ar.take<float>(uint64_t(kRunRows) * m.hidden);
+    s.h = ar.take<float>(uint64_t(kRunRows) * m.hidden);   // the final states, where the caller does not keep them
+    s.rope_local = ar.take<float>(uint64_t(kRunRows) * m.head_dim);
+    s.rope_global = ar.take<float>(uint64_t(kRunRows) * m.head_dim);
+    s.positions = ar.take<uint32_t>(kRunRows);
+    s.ancestors = ar.take<uint32_t>(kRunRows);
+    s.schedule = ar.take<uint32_t>(uint64_t(m.layer_count) * kRunRows * 4);
+    s.exchange = ar.take<uint8_t>(drafter_pass_bytes(m, kRunRows));
+    s.sync_words = drafter_pass_sync_words(m);
+    s.sync = ar.take<uint32_t>(s.sync_words);
+    s.bytes = (ar.used + 255) & ~uint64_t{255};
+    return s;
+}
+
+uint64_t guffin::forward_run_bytes(const guffin_model_desc& m) { return drafter_pass_fits(m) ? run_layout(m, nullptr).bytes : 0; }
+
+int guffin::forward_run(hipStream_t stream, const guffin_model_desc& m, const uint32_t* tokens, uint32_t rows, uint32_t position, void* scratch,
+                        void* priv_k, void* priv_v, float* row_states, float* last_state, float* last_receipt, uint32_t* status) {
+    GUFFIN_TRY(validate_model(&m));
+    GUFFIN_TRY(check_ring_capacity(m, position, rows, "forward_run: the rows do not fit the KV rings"));
+    Scratch s = run_layout(m, static_cast<uint8_t*>(scratch));
+    GUFFIN_TRY(enter_rows(stream, m, tokens, rows, position, s, s.sync_words, status));
+    return drafter_pass(stream, m, rows, {s.exchange, s.sync, s.rope_local, s.rope_global, s.schedule, priv_k, priv_v, s.x, s.u,
+                                          row_states ? row_states : s.h, last_state, last_receipt, 1, status});
 }
 
 // ---- a whole verify tree in one pass -----------------------------------------------------------

@@ -72,6 +72,43 @@ def test_the_pass_equals_the_per_operator_pass(hip, gfo, heads, hidden, ffn, lay
     assert rel_rms(got[0].cpu().numpy(), oracle) <= 1e-3
 
 
+# heads, hidden, ffn, layers, window, first position, runs: rows of a launch that attend each other's keys from the first token on,
+# across a window's start (also one shorter than a run), in lists of several chunks a workgroup, over more blocks than a launch takes
+RUNS = [(4, 640, 2048, 2, 512, 0, (8, 8, 8)), (4, 640, 2048, 2, 512, 505, (8, 3, 24)), (4, 640, 2048, 3, 512, 1276, (2, 8, 7)),
+        (2, 640, 2048, 2, 512, 25, (8, 8)), (1, 64, 256, 2, 512, 60, (5, 8)), (4, 64, 256, 26, 512, 15, (8, 4)), (4, 64, 256, 2, 5, 2, (8, 9))]
+
+
+@pytest.mark.parametrize("heads,hidden,ffn,layers,window,start,runs", RUNS)
+def test_rows_of_a_run_equal_passes_of_one_row(hip, heads, hidden, ffn, layers, window, start, runs):
+    """Each row is summed as by itself: hidden rows, K/V rows and logits to the last bit, also behind a window and for rows whose
+    neighbours lie in several workgroups' parts of the list."""
+    import random
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=layers, vocab=1024, ring_global=2048, q_heads=heads, hidden=hidden, ffn=ffn, global_period=2,
+                    sliding_window=window)
+    devs = [model.DeviceModel.random(shape, seed=layers + heads, position=0) for _ in range(2)]
+    plans = [model.DraftPlan(d) for d in devs]
+    tokens = [random.Random(start).randrange(2, 1024) for _ in range(start + sum(runs))]
+    print("runs", heads, hidden, ffn, layers, window, start, runs, flush=True)
+    at = start
+    for plan in plans:
+        if start:
+            plan.append(tokens[:start])
+    for n in runs:
+        plans[0].append(tokens[at:at + n])
+        for t in tokens[at:at + n]:
+            plans[1].append([t])
+        at += n
+        assert np.array_equal(plans[0].read_logits(), plans[1].read_logits())
+        for a, b in zip(devs[0].ring_k + devs[0].ring_v, devs[1].ring_k + devs[1].ring_v):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    pair = torch.tensor(tokens[:2], dtype=torch.int32, device="cuda")
+    both = devs[0].forward(pair, at)
+    first = devs[0].forward(pair[:1].contiguous(), at)
+    assert torch.equal(both[0][0], first[0][0]) and torch.equal(both[2][:, 0], first[2][:, 0])
+
+
 def test_a_row_keeps_a_nan_and_says_so(hip):
     """A non-finite row in a ring's values reaches the hidden row and the status word, as in the per-operator pass: an operand
     group with a NaN has no fixed-point digits, its multiplier carries the NaN instead."""
