@@ -196,7 +196,7 @@ constexpr uint32_t attention_lds(uint32_t nt) {
     return nt == 1 ? 4 * 16384 + 5 * 16 * 2 * 4 : nt * (16384 + 4 * 16 * 32 * 4 + 16 * 2 * 4);
 }
 
-// grid (ceil(rows * group / (16 NT)), kv_heads, parts), 4 waves.  A workgroup serves 16 NT (row, head) pairs of one KV head
+// grid (kv_heads * ceil(rows * group / (16 NT)), 1, parts), 4 waves.  A workgroup serves 16 NT (row, head) pairs of one KV head
 // -- the group's heads of 16 NT / group consecutive rows, as NT A tiles of 16 pairs -- and one part of the key range.  Each
 // wave walks its own 32-token tiles (tile index = wave mod 4) with its own online softmax state and its own output
 // accumulators; the four states are merged at the end.  A run of few rows is cut into parts so that the chip is full; their
@@ -223,7 +223,8 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
     const uint32_t j = lane & 15, lg = lane >> 4;
     float* pt = reinterpret_cast<float*>(lds + NT * 16384) + wave * (kPairs * 32);   // [NT][16 pairs][32 tokens]
     float* ml = reinterpret_cast<float*>(lds + NT * 16384 + 4 * kPairs * 32 * 4);    // [pairs][2] for the merge
-    const uint32_t kvh = blockIdx.y, r0 = blockIdx.x * (kPairs >> group_shift), group = 1u << group_shift;
+    const uint32_t kvh = blockIdx.x % kv_heads, group = 1u << group_shift;
+    const uint32_t r0 = ((((rows << group_shift) + kPairs - 1) / kPairs) - 1 - blockIdx.x / kv_heads) * (kPairs >> group_shift);
     const size_t row_stride = size_t(kv_heads) * HD;
     const uint32_t last_row = min(r0 + (kPairs >> group_shift), rows) - 1;
     const uint32_t hi_pos = position + last_row;
@@ -719,7 +720,7 @@ int prefill_attention_run(hipStream_t s, const float* q, const void* ring_k, con
     float* states = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + transposed_bytes(vs.T, kv_heads));
     const AttentionOut to {out, image, states, states + size_t(parts) * rows * q_heads * 256};
     const uint32_t lds = attention_lds(nt);
-    const dim3 grid((rows * group + 16 * nt - 1) / (16 * nt), kv_heads, parts);
+    const dim3 grid((rows * group + 16 * nt - 1) / (16 * nt) * kv_heads, 1, parts);
     const uint32_t form = kv_heads | (shift << 16) | (parts << 18);   // at most two parts a compute unit
 #define GUFFIN_PA(NT_) launch(prefill_attention_mfma_kernel<NT_>, grid, dim3(256), lds, s, q, static_cast<const uint16_t*>(ring_k), \
                               static_cast<const uint16_t*>(run_k), static_cast<const uint16_t*>(workspace), rows, position, window, ring_mask, \

@@ -151,6 +151,20 @@ __device__ __forceinline__ GemmSegment segment_of(uint32_t group, const uint8_t*
     return {t2, y2, n2, form >> 24, 4 * (group - g2)};
 }
 
+// Where a workgroup works: row chunk, column group of 256 over all segments, k-slice (past the last one: nothing to do).
+constexpr uint32_t kSliceBits = 5;   // of `form`; above them, up to its matrices' formats: 0, or 1 + log2(row_ways)
+struct GemmPlace { uint32_t chunk, group, slice; };
+template <int R>
+__device__ __forceinline__ GemmPlace place_of(uint32_t M, uint32_t n0, uint32_t n1, uint32_t n2, uint32_t form) {
+    const uint32_t cut = (form >> kSliceBits) & 7u;
+    if (cut == 0) return {blockIdx.x, blockIdx.y, blockIdx.z};
+    const uint32_t chunks = (M + 16 * R - 1) / (16 * R), groups = (n0 + 3) / 4 + (n1 + 3) / 4 + (n2 + 3) / 4;
+    const uint32_t lc = cut - 1, ways = 1u << lc, own = (chunks + ways - 1) >> lc;
+    const uint32_t x = blockIdx.x & 7u, k = blockIdx.x >> 3, turn = k / own;
+    const uint32_t chunk = (x & (ways - 1)) + ways * (k - turn * own), unit = (x >> lc) + (8u >> lc) * turn, slice = unit / groups;
+    return {chunk, unit - slice * groups, chunk < chunks ? slice : ~0u};
+}
+
 // what the workgroup keeps in LDS, R row tiles of 16
 template <int R>
 struct Stage {
@@ -649,8 +663,8 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
     }
 }
 
-// grid (row chunks, column groups of 256 over all segments, k-slices), 256 threads.  Consecutive workgroups walk the
-// rows, so that an XCD's L2 keeps its share of the image.
+// grid (row chunks, column groups of 256 over all segments, k-slices), so that an XCD's L2 keeps its share of the image, or as
+// row_ways has it; 256 threads.
 template <int R, int KINDS>
 __global__ void __launch_bounds__(256, 2)
 prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const uint8_t* __restrict__ blob,
@@ -659,10 +673,13 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
     __shared__ __attribute__((aligned(16))) uint8_t stage[Stage<R>::kBytes];
     const ImageLayout L = image_layout(M, K);
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const GemmSegment seg = segment_of(blockIdx.y, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
-    const uint32_t tile_index = seg.first + wv, nblk = K / 256, rt0 = blockIdx.x * R, slices = form & 0xFFu;
+    const GemmPlace at = place_of<R>(M, n0, n1, n2, form);
+    const uint32_t slices = form & ((1u << kSliceBits) - 1);
+    if (at.slice >= slices) return;
+    const GemmSegment seg = segment_of(at.group, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
+    const uint32_t tile_index = seg.first + wv, nblk = K / 256, rt0 = at.chunk * R;
     const bool valid = tile_index < seg.columns;   // a wave past the last tile works on tile 0 and stores nothing
-    const uint32_t b0 = blockIdx.z * nblk / slices, b1 = (blockIdx.z + 1) * nblk / slices;
+    const uint32_t b0 = at.slice * nblk / slices, b1 = (at.slice + 1) * nblk / slices;
     Feed<R> feed;
     feed.img = make_resource(blob, static_cast<uint32_t>(L.bytes));
     feed.stage = stage;
@@ -685,8 +702,8 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (!valid) return;
         const uint32_t N = seg.columns * kCols;
-        float* y = seg.y + blockIdx.z * (uint64_t(M) * N);
-        const uint32_t at = lane_again(), col = tile_index * kCols + (at & 15), row0 = rt0 * 16 + 4 * (at >> 4);
+        float* y = seg.y + at.slice * (uint64_t(M) * N);
+        const uint32_t lane = lane_again(), col = tile_index * kCols + (lane & 15), row0 = rt0 * 16 + 4 * (lane >> 4);
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -714,10 +731,13 @@ prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict
     __shared__ __attribute__((aligned(16))) uint8_t stage[3 * kSlot];
     const ImageLayout L = image_layout(M, K);
     const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, lg = lane >> 4;
-    const GemmSegment seg = segment_of(blockIdx.y, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
-    const uint32_t tile_index = seg.first + wv, nblk = K / 32, rt0 = blockIdx.x * R, slices = form & 0xFFu;
+    const GemmPlace at = place_of<R>(M, n0, n1, n2, form);
+    const uint32_t slices = form & ((1u << kSliceBits) - 1);
+    if (at.slice >= slices) return;
+    const GemmSegment seg = segment_of(at.group, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
+    const uint32_t tile_index = seg.first + wv, nblk = K / 32, rt0 = at.chunk * R;
     const bool valid = tile_index < seg.columns;
-    const uint32_t chunks = (nblk + 1) / 2, c0 = blockIdx.z * chunks / slices, c1 = (blockIdx.z + 1) * chunks / slices;
+    const uint32_t chunks = (nblk + 1) / 2, c0 = at.slice * chunks / slices, c1 = (at.slice + 1) * chunks / slices;
     const __amdgpu_buffer_rsrc_t img = make_resource(blob, static_cast<uint32_t>(L.bytes));
     const __amdgpu_buffer_rsrc_t tile = make_resource(seg.tiles + size_t(valid ? tile_index : 0) * nblk * TB, nblk * TB);
     const uint32_t lane16 = lane * 16, group_stride = (L.mpad / 16) * 2048, shift = L.span == 256 ? 3 : 0;
@@ -803,7 +823,7 @@ prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!valid) return;
     const uint32_t N = seg.columns * kCols;
-    float* y = seg.y + blockIdx.z * (uint64_t(M) * N);
+    float* y = seg.y + at.slice * (uint64_t(M) * N);
     const uint32_t col = tile_index * kCols + j, row0 = rt0 * 16 + 4 * lg;
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -816,9 +836,17 @@ prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict
         }
 }
 
+// How many ways the XCDs cut the row chunks of a launch between them, the column groups being dealt over the others; 0: the grid's
+// own order.  Consecutive workgroups go to different XCDs, so where the rows run fastest the workgroups that share weights sit in
+// different L2s: all of them fetch all weights.  Good where a whole image does not fit an L2 and each keeps its share of it;
+// with few chunks the weights are what is worth keeping.  A pass of the 12B shapes, us, grid's order / one way / two ways: 160 rows 12207 / 11861 /
+// 13439, 333 21035 / 20486 / 20563, 448 25888 / 25270 / 24869, 640 34744 / 35441 / 33996, 704 38435 / 40628 / 39683, 2048 100656 / 104727 /
+// 102185.  The drafter's weights are small beside its image: 333 rows 1302 / 1417 / 1375.
+uint32_t row_ways(uint32_t chunks, bool q8) { return q8 || chunks < 2 || chunks > 10 ? 0 : chunks <= 6 ? 1 : 2; }
+
 int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M, uint32_t K,
                 uint32_t slices, uint32_t R) {
-    if (count > 3 || slices > 255) return fail(GUFFIN_E_SHAPE, "prefill_gemm: at most three matrices and 255 slices");
+    if (count > 3 || slices >= 1u << kSliceBits) return fail(GUFFIN_E_SHAPE, "prefill_gemm: at most three matrices and 31 slices");
     GemmArgs a {};
     a.blob = image; a.M = M; a.K = K; a.form = slices;
     uint32_t groups = 0, kinds = 0;
@@ -829,7 +857,13 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
         groups += (a.columns[i] + 3) / 4;
         kinds |= m[i].dtype == GUFFIN_Q4_K ? 1u : m[i].dtype == GUFFIN_Q6_K ? 2u : 4u;
     }
-    const dim3 grid((M + 16 * R - 1) / (16 * R), groups, slices), block(256);
+    const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
+    dim3 grid(chunks, groups, slices), block(256);
+    if (const uint32_t ways = row_ways(chunks, kinds == 4u)) {
+        const uint32_t units = groups * slices, others = 8 / ways;
+        a.form |= (ways == 1 ? 1u : 2u) << kSliceBits;
+        grid = dim3(8 * ((chunks + ways - 1) / ways) * ((units + others - 1) / others));
+    }
 #define GUFFIN_PG_ARGS a.tiles[0], a.tiles[1], a.tiles[2], a.blob, a.M, a.K, a.columns[0], a.columns[1], a.columns[2], a.form, a.y[0], a.y[1], a.y[2]
 #define GUFFIN_PG(R_) \
     do { \

@@ -64,12 +64,19 @@ __device__ __forceinline__ void store8_words(float* p, const float (&v)[8]) {
     *reinterpret_cast<F4a4*>(p + 4) = F4a4 {v[4], v[5], v[6], v[7]};
 }
 
+// The row of a workgroup.  Eight rows of a record's k-slice share a 128-byte line of the image, and consecutive workgroups go to
+// different XCDs: the eight go to one, whose L2 puts the line together.
+__device__ __forceinline__ uint32_t row_of(uint32_t b, uint32_t rows) {
+    const uint32_t x = b & 7u, k = b >> 3;
+    return b < (rows & ~63u) ? (k & ~7u) * 8 + x * 8 + (k & 7u) : b;
+}
+
 // one workgroup per row, a thread owns 8 consecutive columns
 __global__ void __launch_bounds__(1024)
 prefill_norm_kernel(const float* __restrict__ x, const float* __restrict__ gamma, uint8_t* __restrict__ image, uint32_t rows,
                     uint32_t width, float eps, uint32_t* __restrict__ status) {
     __shared__ float scratch[16];
-    const uint32_t r = blockIdx.x, t = threadIdx.x;
+    const uint32_t r = row_of(blockIdx.x, rows), t = threadIdx.x;
     const bool active = t < width / 8;
     float v[8] = {}, g[8] = {};
     if (active) { load8(x + size_t(r) * width + 8 * t, v); load8_words(gamma + 8 * t, g); }
@@ -103,7 +110,7 @@ prefill_joint_kernel(const float* __restrict__ x, const float* __restrict__ resi
         return;
     }
     __shared__ float scratch[2][16];
-    const uint32_t r = blockIdx.x, t = threadIdx.x;
+    const uint32_t r = row_of(blockIdx.x, rows), t = threadIdx.x;
     const bool active = t < width / 8;
     const size_t at = size_t(r) * width + 8 * t;
     float v[8] = {}, gp[8] = {}, gn[8] = {}, res[8] = {};

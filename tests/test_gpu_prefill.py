@@ -85,6 +85,24 @@ def test_prefill_gemm_sums_against_64_bits(hip, rows):
     assert float(((y - want).pow(2).mean() / want.pow(2).mean()).sqrt()) <= 1.6e-7
 
 
+@pytest.mark.parametrize("dtype,N", [(1, 64), (1, 64 * 33), (2, 64 * 5), (2, 64 * 36)])
+@pytest.mark.parametrize("M", [65, 97, 385, 449, 577, 640, 641, 705])
+def test_prefill_gemm_wherever_its_workgroups_go(hip, dtype, N, M):
+    """Row chunks dealt to the XCDs in two, one and (one chunk more than that takes) the grid's order, with fewer column groups than
+    XCDs and numbers of them that eight does not divide: every element, against 64 bits.  The rms error of such sums is 1.6e-7
+    (Q4_K) and 2.3e-7 (Q6_K) of the result's; a workgroup that worked on another's place, or on none, is off by the result itself."""
+    import torch
+    K = 512
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N)
+    w = dev(synth.make_weight(dtype, K, N, seed=9 + dtype))
+    x = torch.randn((M, K), device="cuda", generator=gen)
+    want = x.double() @ hip.dequant(dtype, w, N * K // 256).view(N, K).double().T.contiguous()
+    y = hip.prefill_gemm(dtype, hip.repack(dtype, w, K, N), hip.prefill_pack(x), M, K, N).double()
+    assert float(((y - want).pow(2).mean() / want.pow(2).mean()).sqrt()) <= 4e-7
+    assert float((y - want).abs().max() / want.pow(2).mean().sqrt()) <= 1e-5
+
+
 def test_prefill_gemm_down_projection_shape(hip, gfo):
     """Q6_K at the down projection's K = 15360 (60 blocks per column, the longest chain of LDS
     stages and weight prefetches) with an odd number of column tiles and rows in every row group."""
