@@ -196,7 +196,9 @@ constexpr uint32_t attention_lds(uint32_t nt) {
     return nt == 1 ? 4 * 16384 + 5 * 16 * 2 * 4 : nt * (16384 + 4 * 16 * 32 * 4 + 16 * 2 * 4);
 }
 
-// grid (kv_heads * ceil(rows * group / (16 NT)), 1, parts), 4 waves.  A workgroup serves 16 NT (row, head) pairs of one KV head
+// grid (kv_heads * ceil(rows * group / (16 NT)), 1, parts), 4 waves.  Heads run fastest and the last rows come first: consecutive
+// workgroups go to different XCDs, so with eight KV heads an L2 holds one head's keys and values, and the longest lists of a causal
+// block start first.  (Tiles fastest, first rows first: 2048 rows 162 us instead of 142, 333 rows 22.6 instead of 17.6.)  A workgroup serves 16 NT (row, head) pairs of one KV head
 // -- the group's heads of 16 NT / group consecutive rows, as NT A tiles of 16 pairs -- and one part of the key range.  Each
 // wave walks its own 32-token tiles (tile index = wave mod 4) with its own online softmax state and its own output
 // accumulators; the four states are merged at the end.  A run of few rows is cut into parts so that the chip is full; their

@@ -65,7 +65,8 @@ __device__ __forceinline__ void store8_words(float* p, const float (&v)[8]) {
 }
 
 // The row of a workgroup.  Eight rows of a record's k-slice share a 128-byte line of the image, and consecutive workgroups go to
-// different XCDs: the eight go to one, whose L2 puts the line together.
+// different XCDs: the eight go to one, whose L2 puts the line together.  (2048 x 3840: the joints 44.7 -> 32.0 and 50.1 -> 35.1 us, the
+// first norm 34.4 -> 16.5; 333 rows 10.6 -> 10.0 and 10.3 -> 9.4.)
 __device__ __forceinline__ uint32_t row_of(uint32_t b, uint32_t rows) {
     const uint32_t x = b & 7u, k = b >> 3;
     return b < (rows & ~63u) ? (k & ~7u) * 8 + x * 8 + (k & 7u) : b;
