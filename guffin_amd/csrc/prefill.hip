@@ -118,7 +118,8 @@ prefill_attention_kernel(const float* __restrict__ q, const uint16_t* __restrict
 
 // ---- the same attention on the matrix core ------------------------------------------------
 // Values are contracted over tokens, so the B operand needs 8 consecutive tokens of one output
-// dimension: a small pass first writes V^T, [kv_heads][256][T] fp16, for the virtual tokens
+// dimension: a small pass first writes V^T, [kv_heads][T / 32][256][32] fp16 (a tile in one piece: with rows of T tokens an operand
+// took half of each of sixteen lines), for the virtual tokens
 // base32 .. base32 + T (T a multiple of 32; tokens outside [first_visible, end) are zero).
 __global__ void __launch_bounds__(256)
 transpose_values_kernel(const uint16_t* __restrict__ ring_v, const uint16_t* __restrict__ run_v,
@@ -144,7 +145,7 @@ transpose_values_kernel(const uint16_t* __restrict__ ring_v, const uint16_t* __r
     uint32_t w[16];
 #pragma unroll
     for (int t = 0; t < 16; ++t) w[t] = uint32_t(tile[2 * t][dim]) | (uint32_t(tile[2 * t + 1][dim]) << 16);
-    uint4* dst = reinterpret_cast<uint4*>(vt + (size_t(kvh) * HD + dim) * T + v0);
+    uint4* dst = reinterpret_cast<uint4*>(vt + size_t(kvh) * HD * T + (size_t(v0) * HD + dim * 32));
 #pragma unroll
     for (int i = 0; i < 4; ++i) dst[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
 }
@@ -190,11 +191,9 @@ __device__ __forceinline__ void emit_attention(const AttentionOut& to, const flo
     }
 }
 
-// whether the merge of a workgroup's waves has room for all of their outputs, and its LDS
-template <int NT> constexpr bool kMergeAtOnce = NT == 1;
-constexpr uint32_t attention_lds(uint32_t nt) {
-    return nt == 1 ? 4 * 16384 + 5 * 16 * 2 * 4 : nt * (16384 + 4 * 16 * 32 * 4 + 16 * 2 * 4);
-}
+// a workgroup's LDS: four waves' outputs of an A tile, their states and the merged ones (queries and probabilities take less)
+constexpr uint32_t attention_lds(uint32_t nt) { return 4 * 16384 + 5 * nt * 16 * 2 * 4; }
+static_assert(attention_lds(2) >= 2 * (16384 + 4 * 16 * 32 * 4));
 
 // grid (kv_heads * ceil(rows * group / (16 NT)), 1, parts), 4 waves.  Heads run fastest and the last rows come first: consecutive
 // workgroups go to different XCDs, so with eight KV heads an L2 holds one head's keys and values, and the longest lists of a causal
@@ -219,12 +218,11 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
     constexpr int HD = 256;
     constexpr uint32_t kPairs = 16 * NT;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    // [NT][8 k-steps][hi, lo][64 lanes] 16-byte query operands, later the merge buffer
+    // [NT][8 k-steps][hi, lo][64 lanes] 16-byte query operands
     uint8_t* qa = lds;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 15, lg = lane >> 4;
     float* pt = reinterpret_cast<float*>(lds + NT * 16384) + wave * (kPairs * 32);   // [NT][16 pairs][32 tokens]
-    float* ml = reinterpret_cast<float*>(lds + NT * 16384 + 4 * kPairs * 32 * 4);    // [pairs][2] for the merge
     const uint32_t kvh = blockIdx.x % kv_heads, group = 1u << group_shift;
     const uint32_t r0 = ((((rows << group_shift) + kPairs - 1) / kPairs) - 1 - blockIdx.x / kv_heads) * (kPairs >> group_shift);
     const size_t row_stride = size_t(kv_heads) * HD;
@@ -246,13 +244,21 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         }
     };
     uint4 kb[2][8];
-    // one A tile leaves registers for the next keys beside the values: the first ones travel while the queries are staged
-    if constexpr (NT == 1) ask_keys(min(begin + wave, tile_lo + tiles - 1), kb);
-    for (uint32_t idx = threadIdx.x; idx < kPairs * 32; idx += 256) {
-        const uint32_t m = idx / 32, c8 = idx % 32;
+    float4 qv[kPairs / 8][2];
+#pragma unroll
+    for (uint32_t i = 0; i < kPairs / 8; ++i) {
+        const uint32_t m = 8 * i + threadIdx.x / 32, c8 = threadIdx.x % 32;
         const uint32_t row = min(r0 + (m >> group_shift), rows - 1), head = kvh * group + (m & (group - 1));
         const float* src = q + (size_t(row) * q_heads + head) * HD + 8 * c8;
-        const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
+        qv[i][0] = *reinterpret_cast<const float4*>(src); qv[i][1] = *reinterpret_cast<const float4*>(src + 4);
+    }
+    asm volatile("" ::: "memory");   // the queries are asked for first: what is asked for before them arrives before them
+    // one A tile leaves registers for the next keys beside the values: the first ones travel while the queries are staged
+    if constexpr (NT == 1) ask_keys(min(begin + wave, tile_lo + tiles - 1), kb);
+#pragma unroll
+    for (uint32_t i = 0; i < kPairs / 8; ++i) {
+        const uint32_t m = 8 * i + threadIdx.x / 32, c8 = threadIdx.x % 32;
+        const float4 a = qv[i][0], b = qv[i][1];
         const float x[8] = {a.x * scale, a.y * scale, a.z * scale, a.w * scale, b.x * scale, b.y * scale, b.z * scale, b.w * scale};
         uint4 hi, lo;
         split_half8(x, hi, lo);
@@ -275,11 +281,11 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
     for (uint32_t ti = begin + wave; ti < end; ti += 4) {
         const uint32_t t0 = base32 + 32 * ti;
         if constexpr (NT > 1) ask_keys(ti, kb);
-        const uint16_t* vcol = vt + (size_t(kvh) * HD + j) * T + (t0 - base32) + 8 * lg;
+        const uint16_t* vcol = vt + size_t(kvh) * HD * T + size_t(ti) * (32 * HD) + 32 * j + 8 * lg;
         uint4 vb[VB];
         auto ask_values = [&](int first) {
 #pragma unroll
-            for (int i = 0; i < VB; ++i) vb[i] = *reinterpret_cast<const uint4*>(vcol + size_t(16 * (first + i)) * T);
+            for (int i = 0; i < VB; ++i) vb[i] = *reinterpret_cast<const uint4*>(vcol + 512 * (first + i));
         };
         if constexpr (NT == 1) ask_values(0);
         // A sum rounds at the size it has grown to: the hi halves of the first four steps are one chain; the other takes the lo
@@ -387,94 +393,63 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    // merge the four waves' states in wave order through LDS (the query operands are dead now)
-    float* ob = reinterpret_cast<float*>(qa);  // [(g * 16 + dt) * 4 + r][lane]
-    constexpr uint32_t kWaveSlots = NT * 4096;   // of one wave's outputs
-    if constexpr (kMergeAtOnce<NT>) {
-        // every wave's outputs have room: scaled to the common maximum by their own wave, summed by whoever stores them.  (One
-        // wave behind the other over the same slots, as below: three more passes over them.  With the values asked for ahead of the scores 12 rows at
-        // position 100 take 11.1 instead of 12.4 us, 37 at 1500 16.1 instead of 16.8.)
-        float* states = reinterpret_cast<float*>(lds + 4 * kWaveSlots * 4);   // [wave][pair][2]
-        ml = states + 4 * kPairs * 2;
-        __syncthreads();
-        if (j == 0)
+    // Merge the four waves' states through LDS, an A tile at a time: every wave's outputs, scaled to the common maximum by their own
+    // wave, have room together and are summed in wave order by whoever stores them.  (One wave behind the other over the same slots:
+    // three more passes over them,
+    // 14 us of a workgroup's 65 at 2048 rows instead of 9.)
+    float* ob = reinterpret_cast<float*>(lds);  // [wave][dt][4][64 lanes]; the query operands and the probabilities are dead now
+    constexpr uint32_t kWaveSlots = 4096;       // of one wave's outputs
+    float* states = reinterpret_cast<float*>(lds + 4 * kWaveSlots * 4);   // [wave][pair][2]
+    float* ml = states + 4 * kPairs * 2;        // [pair][2], merged
+    __syncthreads();
+    if (j == 0)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) *reinterpret_cast<float2*>(states + (wave * kPairs + 4 * lg + r) * 2) = make_float2(m[0][r], l[0][r]);
-        __syncthreads();
+        for (int g = 0; g < NT; ++g)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                *reinterpret_cast<float2*>(states + (wave * kPairs + 16 * g + 4 * lg + r) * 2) = make_float2(m[g][r], l[g][r]);
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < NT; ++g) {
+        if (g > 0) __syncthreads();   // the tile before has been read
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+            const uint32_t pair = 16 * g + 4 * lg + r;
             float2 st[4];
 #pragma unroll
-            for (int w = 0; w < 4; ++w) st[w] = *reinterpret_cast<const float2*>(states + (w * kPairs + 4 * lg + r) * 2);
+            for (int w = 0; w < 4; ++w) st[w] = *reinterpret_cast<const float2*>(states + (w * kPairs + pair) * 2);
             const float M = fmaxf(fmaxf(st[0].x, st[1].x), fmaxf(st[2].x, st[3].x));
             float den = 0.f;
 #pragma unroll
             for (int w = 0; w < 4; ++w) den += st[w].x == -INFINITY ? 0.f : st[w].y * exp_of(st[w].x - M);
-            const float mine = m[0][r] == -INFINITY ? 0.f : exp_of(m[0][r] - M);
+            const float mine = m[g][r] == -INFINITY ? 0.f : exp_of(m[g][r] - M);
             float* slots = ob + wave * kWaveSlots + r * 64 + lane;
 #pragma unroll
-            for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[0][dt][r] * mine;
-            if (wave == 0 && j == 0) *reinterpret_cast<float2*>(ml + (4 * lg + r) * 2) = make_float2(M, den);
+            for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r] * mine;
+            if (wave == 0 && j == 0) *reinterpret_cast<float2*>(ml + pair * 2) = make_float2(M, den);
         }
-    } else {
-        for (uint32_t w = 0; w < 4; ++w) {
-            __syncthreads();
-            if (wave != w) continue;
+        __syncthreads();
+#pragma unroll 1
+        for (uint32_t n = 0; n < 2; ++n) {   // 32 consecutive lanes: one (row, head)
+            const uint32_t i = 8 * n + threadIdx.x / 32, c8 = threadIdx.x % 32, p = 16 * g + i;
+            const uint32_t row = r0 + (p >> group_shift), head = kvh * group + (p & (group - 1));
+            if (row >= rows) continue;
+            const float* src = ob + (((c8 >> 1) * 4 + (i & 3)) * 64 + 8 * (c8 & 1) + 16 * (i >> 2));
+            float v[8];
 #pragma unroll
-            for (int g = 0; g < NT; ++g)
+            for (int k = 0; k < 8; ++k) v[k] = src[k] + (src[kWaveSlots + k] + src[2 * kWaveSlots + k] + src[3 * kWaveSlots + k]);
+            if (parts == 1) {
+                const float den = ml[p * 2 + 1] * kProbScale;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float* slots = ob + (g * 64 + r) * 64 + lane;   // [dt][4][64]
-                    if (w == 0) {
+                for (int k = 0; k < 8; ++k) v[k] /= den;
+                emit_attention(to, v, row, rows, head, q_heads, c8);
+            } else {
+                const size_t at = (size_t(blockIdx.z) * rows + row) * q_heads + head;
+                float* dst = to.part_o + at * HD + 8 * c8;
 #pragma unroll
-                        for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r];
-                        continue;
-                    }
-                    const float mo = ml[(g * 16 + 4 * lg + r) * 2], lo_ = ml[(g * 16 + 4 * lg + r) * 2 + 1];
-                    const float M = fmaxf(m[g][r], mo);
-                    const float mine = m[g][r] == -INFINITY ? 0.f : exp_of(m[g][r] - M), theirs = mo == -INFINITY ? 0.f : exp_of(mo - M);
-                    l[g][r] = l[g][r] * mine + lo_ * theirs;
-                    m[g][r] = M;
-#pragma unroll
-                    for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r] * mine + slots[dt * 256] * theirs;
-                }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (j == 0) {
-#pragma unroll
-                for (int g = 0; g < NT; ++g)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        ml[(g * 16 + 4 * lg + r) * 2] = m[g][r];
-                        ml[(g * 16 + 4 * lg + r) * 2 + 1] = l[g][r];
-                    }
+                for (int k = 0; k < 8; ++k) dst[k] = v[k];
+                if (c8 == 0) { to.part_ml[2 * at] = ml[p * 2]; to.part_ml[2 * at + 1] = ml[p * 2 + 1]; }
             }
-        }
-    }
-    __syncthreads();
-    for (uint32_t idx = threadIdx.x; idx < kPairs * 32; idx += 256) {   // 32 consecutive lanes: one (row, head)
-        const uint32_t p = idx / 32, c8 = idx % 32, i = p & 15;
-        const uint32_t row = r0 + (p >> group_shift), head = kvh * group + (p & (group - 1));
-        if (row >= rows) continue;
-        const float* src = ob + ((((p >> 4) * 16 + (c8 >> 1)) * 4 + (i & 3)) * 64 + 8 * (c8 & 1) + 16 * (i >> 2));
-        float v[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            v[k] = src[k];
-            if constexpr (kMergeAtOnce<NT>) v[k] += src[kWaveSlots + k] + src[2 * kWaveSlots + k] + src[3 * kWaveSlots + k];
-        }
-        if (parts == 1) {
-            const float den = ml[p * 2 + 1] * kProbScale;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] /= den;
-            emit_attention(to, v, row, rows, head, q_heads, c8);
-        } else {
-            const size_t at = (size_t(blockIdx.z) * rows + row) * q_heads + head;
-            float* dst = to.part_o + at * HD + 8 * c8;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) dst[k] = v[k];
-            if (c8 == 0) { to.part_ml[2 * at] = ml[p * 2]; to.part_ml[2 * at + 1] = ml[p * 2 + 1]; }
         }
     }
 }
@@ -697,7 +672,9 @@ extern "C" uint64_t guffin_hip_prefill_attention_workspace_bytes(uint32_t rows, 
 }
 
 namespace guffin {
-int prefill_attention_init() { return allow_lds(prefill_attention_mfma_kernel<1>, attention_lds(1)) ? 0 : -1; }
+int prefill_attention_init() {
+    return allow_lds(prefill_attention_mfma_kernel<1>, attention_lds(1)) && allow_lds(prefill_attention_mfma_kernel<2>, attention_lds(2)) ? 0 : -1;
+}
 
 bool prefill_attention_on_matrix_core(const void* q, const void* ring_k, const void* ring_v, const void* run_k, const void* run_v,
                                       uint32_t q_heads, uint32_t kv_heads) {

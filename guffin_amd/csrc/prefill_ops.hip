@@ -267,7 +267,7 @@ prefill_qkv_kernel(const float* __restrict__ q_planes, const float* __restrict__
         uint32_t o[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) o[t] = uint32_t(tile[t0 + 2 * t][dim]) | (uint32_t(tile[t0 + 2 * t + 1][dim]) << 16);
-        *reinterpret_cast<uint4*>(a.vt + (size_t(kvh) * HD + dim) * a.T + v0 + t0) = make_uint4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<uint4*>(a.vt + size_t(kvh) * HD * a.T + size_t(v0) * HD + 32 * dim + t0) = make_uint4(o[0], o[1], o[2], o[3]);
     }
     if (bad && a.status) atomicOr(a.status, GUFFIN_STATUS_KV_NONFINITE);
 }

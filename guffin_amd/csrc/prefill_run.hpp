@@ -41,7 +41,7 @@ struct QkvRun {
     const float *q_planes, *k_planes, *v_planes;   // planes of [rows][heads * 256]
     const float *q_norm, *k_norm, *rope_table;     // table [rows][128] of cos, sin
     float* q_out; uint16_t *k_out, *v_out;         // [rows][heads * 256]
-    const uint16_t* ring_v; uint16_t* vt;          // vt [kv_heads][256][T]
+    const uint16_t* ring_v; uint16_t* vt;          // vt [kv_heads][T / 32][256][32]
     uint32_t planes, rows, q_heads, kv_heads, position, ring_mask, first_visible, base32, T, head_groups;
     float eps;
     uint32_t* status;
