@@ -11,6 +11,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 HSACO = os.path.join(HERE, "hsaco")
 LIB = os.path.join(HERE, "libguffin_hip.so")
+OPERATORS = os.path.join(HERE, "_operators.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 READELF = os.environ.get("LLVM_READELF", "/opt/rocm/llvm/bin/llvm-readelf")
 FLAGS = [
@@ -80,6 +81,24 @@ def kernarg_rows(code_object):
     return rows
 
 
+def _operators():
+    """The native forms of the small operators for Python: host code against torch's headers, bound to the library at run time."""
+    import sysconfig
+
+    import torch
+    base = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
+           *("-isystem" + d for d in (base + "/include", base + "/include/torch/csrc/api/include", "/opt/rocm/include",
+                                      sysconfig.get_paths()["include"])),
+           os.path.join(CSRC, "python", "operators.cpp"), "-o", OPERATORS, "-L" + base + "/lib", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for operators.cpp:\n" + r.stderr)
+    return r.stderr
+
+
 def build(verbose=False):
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(HSACO, exist_ok=True)
@@ -88,7 +107,9 @@ def build(verbose=False):
     with concurrent.futures.ThreadPoolExecutor(max_workers=8) as pool:
         objects = pool.map(_compile, sources)
         code_objects = pool.map(_code_object, device_sources)
+        operators = pool.submit(_operators)
         results = list(objects)
+        operators.result()
         code_objects = list(code_objects)
     objs = [o for o, _ in results]
     if verbose:

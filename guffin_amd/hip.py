@@ -72,6 +72,25 @@ class _Calls:
 _calls = _Calls()
 
 
+class _Operators:
+    """The native forms of the small operators (csrc/python/operators.cpp), bound to the library's entry points on first use.  A
+    call returns None where its arguments are not the usual ones: the function it stands in then goes on by itself."""
+
+    ENTRY_POINTS = ("receipt_bytes", "group_sums", "gemv_packed_slices", "gemv_packed", "repack", "select_workspace_bytes",
+                    "select_candidates_fresh", "draft_law_workspace_bytes", "draft_law_fresh", "spec_accept")
+
+    def __getattr__(self, name):
+        from . import _operators as native   # built beside the library; no fallback if it is missing
+        native.bind(*(C.cast(getattr(lib(), "guffin_hip_" + e), C.c_void_p).value for e in self.ENTRY_POINTS),
+                    _candidates_bytes, _law_bytes, result_dtype.itemsize, check)
+        for f in ("group_sums", "gemv_packed", "repack", "select_candidates", "draft_law", "spec_accept"):
+            setattr(self, f, getattr(native, f))
+        return self.__dict__[name]
+
+
+_ops = _Operators()
+
+
 def _raw_stream():
     return _current_stream(torch.cuda.current_device())
 
@@ -189,6 +208,9 @@ def packed_bytes(dtype, K, N):
 
 
 def repack(dtype, canonical, K, N):
+    tiles = _ops.repack(dtype, canonical, K, N)
+    if tiles is not None:
+        return tiles
     tiles = torch.empty_like(canonical)
     check(_calls.guffin_hip_repack(_raw_stream(), dtype, canonical.data_ptr(), tiles.data_ptr(), K, N))
     return tiles
@@ -231,6 +253,10 @@ def receipt_parts(sums, rows, K):
 
 def group_sums(x, out=None):
     """Activation receipt of x (sums, multipliers, matrix-core image); returns its sums view."""
+    if out is None:
+        out = _ops.group_sums(x)
+        if out is not None:
+            return out
     rows, K = x.shape
     if out is None:
         out = _receipt(rows, K, x.device)
@@ -244,6 +270,10 @@ def gemv_packed_slices(dtype, K, N):
 
 
 def gemv_packed(dtype, tiles, x, xsums, N, partials=None, out=None, reduce=True):
+    if partials is None and out is None and reduce:
+        y = _ops.gemv_packed(dtype, tiles, x, xsums, N)
+        if y is not None:
+            return y
     rows, K = x.shape
     if partials is None or (reduce and out is None):
         # a single plane is the result itself; several and their sum are one allocation
@@ -471,6 +501,10 @@ def _draft_law_workspace_bytes(vocab):
 
 
 def select_candidates(logits, retain, history=None, history_count=None, status=None, result=None):
+    if history is None and history_count is None and status is None and result is None:
+        both = _ops.select_candidates(logits, retain)
+        if both is not None:
+            return both
     rows, vocab = logits.shape
     ws = torch.empty(_select_workspace_bytes(rows, vocab, retain), dtype=torch.uint8, device="cuda")
     call = _calls.guffin_hip_select_candidates
@@ -540,6 +574,10 @@ def argmax(logits, status=None):
 
 
 def draft_law(logits, options, seed=0, step=0, draws=None, law=None, proposal=None, status=None, workspace=None):
+    if draws is None and law is None and proposal is None and status is None and workspace is None:
+        made = _ops.draft_law(logits, options, seed, step)
+        if made is not None:
+            return made
     vocab = logits.numel()
     if workspace is None:
         workspace = torch.empty(_draft_law_workspace_bytes(vocab), dtype=torch.uint8, device="cuda")
@@ -661,6 +699,10 @@ def spec_accept_history(cands, law, history, history_count, proposal, options, s
 
 
 def spec_accept(cands, law, proposal, options, seed=0, step=0, draws=None, result=None, status=None):
+    if draws is None and result is None:
+        decision = _ops.spec_accept(cands, law, proposal, options, seed, step, status)
+        if decision is not None:
+            return decision
     if result is None:
         result = torch.empty(result_dtype.itemsize, dtype=torch.uint8, device="cuda")   # the kernel writes every word
     check(_calls.guffin_hip_spec_accept(_raw_stream(), cands.data_ptr(), law.data_ptr(), proposal.data_ptr(), C.byref(options), seed, step,
