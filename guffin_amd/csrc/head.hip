@@ -16,6 +16,7 @@
 // A global top-R entry is necessarily a top-R entry of its own tile, so the two stages lose
 // nothing.
 #include "common.hpp"
+#include "law.hpp"
 #include "selection_request.hpp"
 
 #include <cstddef>
@@ -320,6 +321,12 @@ topk_merge_kernel(const float* __restrict__ logits, const uint64_t* __restrict__
 // of 64 needs of one row 8.8 (15.4 with its best 257 in order).  Ties, both launches and the call: 300 to 2000 keys 18 to 29 us,
 // beyond 2048 keys 920.
 constexpr uint32_t kSeg = 256, kMaxSegs = 1024, kCollectTile = 4096, kCollectCap = 2048;
+struct Nothing {};
+// large vocabularies, where the segment maxima give a bound for the best `keep` logits
+bool by_threshold(uint32_t vocab, uint32_t keep) {
+    const uint32_t segs = (vocab + kSeg - 1) / kSeg;
+    return segs <= kMaxSegs && segs >= 2 * keep;
+}
 constexpr uint32_t kMaxCollectors = kMaxSegs * kSeg / kCollectTile, kSlots = 16, kCommonCap = kCollectCap - kSlots;
 // segment maxima; common list's length, workgroups done, pad; the workgroups' counts, their places, the common list
 constexpr uint32_t kThresholdRowWords = kMaxSegs + 4 + kMaxCollectors + 2 * (kMaxCollectors * kSlots + kCommonCap);
@@ -377,11 +384,12 @@ __device__ __forceinline__ T shared_load(const T* p) { return __hip_atomic_load(
 template <typename T>
 __device__ __forceinline__ void shared_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
+template <bool LAW>
 __global__ void __launch_bounds__(1024)
 threshold_select_kernel(const float* __restrict__ logits, uint32_t* __restrict__ ws, uint32_t vocab, uint32_t segs, uint32_t retain_cap,
                         uint32_t sure, float divisor, uint32_t row_stride, const uint32_t* __restrict__ history_count,
                         const uint32_t* __restrict__ row_retain, const uint32_t* __restrict__ history, uint32_t history_stride,
-                        Candidates* __restrict__ result, uint32_t* __restrict__ status, bool suppressed_ok, bool whole) {
+                        Candidates* __restrict__ result, uint32_t* __restrict__ status, bool suppressed_ok, bool whole, std::conditional_t<LAW, LawCall, Nothing> law) {
     __shared__ uint32_t hist[256];
     __shared__ uint64_t sel[kCollectCap];
     __shared__ uint64_t keys[512];
@@ -525,7 +533,18 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t* __restrict__
             keys[rank] = k;
         }
     }
-    emit_candidates(keys, retain, row, logits, vocab, divisor, history, hc, history_stride, raised, whole, result, status);
+    if constexpr (LAW) {
+        __syncthreads();
+        if (tid >= 256) return;   // a law is four waves' work: the meetings are theirs from here on
+        auto logit_of = [&](uint32_t i) {   // as emit_candidates has it
+            const float v = key_logit(keys[i]);
+            return v < 0.f || v > 0.f ? v : lr[key_token(keys[i])] / divisor;
+        };
+        const bool mine_too = tid < retain;
+        compact_law(law, retain, raised, mine_too ? key_token(keys[tid]) : 0u, mine_too ? logit_of(tid) : 0.f, retain > 256 ? logit_of(256) : 0.f);
+    } else {
+        emit_candidates(keys, retain, row, logits, vocab, divisor, history, hc, history_stride, raised, whole, result, status);
+    }
 }
 
 __global__ void clear_words_kernel(uint32_t* words, uint32_t n) {
@@ -665,14 +684,14 @@ int guffin::select_candidates_scaled(hipStream_t s, const float* logits, uint32_
     const uint32_t keep = retain < vocab ? retain : vocab;
     const uint32_t tiles = (vocab + kTile - 1) / kTile;
     const uint32_t segs = (vocab + kSeg - 1) / kSeg;
-    if (segs <= kMaxSegs && segs >= 2 * keep) {   // large vocabulary: a bound from the segment maxima, then one pass
+    if (by_threshold(vocab, keep)) {   // large vocabulary: a bound from the segment maxima, then one pass
         uint32_t* words = static_cast<uint32_t*>(workspace);
         launch(segment_max_kernel, dim3((segs + 3) / 4, rows), dim3(256), 0, s, logits, vocab, segs, divisor, words,
                fresh ? status : nullptr);
         if (int rc = check_launch("select_candidates(segment maxima)")) return rc;
-        launch(threshold_select_kernel, dim3((vocab + kCollectTile - 1) / kCollectTile, rows), dim3(1024), 0, s,
+        launch(threshold_select_kernel<false>, dim3((vocab + kCollectTile - 1) / kCollectTile, rows), dim3(1024), 0, s,
                            logits, words, vocab, segs, keep, sure, divisor, row_stride, history_count, row_retain, history,
-                           row_stride == 1 ? 64u : row_stride, static_cast<Candidates*>(result), status, suppressed_ok, fresh);
+                           row_stride == 1 ? 64u : row_stride, static_cast<Candidates*>(result), status, suppressed_ok, fresh, Nothing {});
         return check_launch("select_candidates(threshold)");
     }
     if (fresh) launch(clear_words_kernel, dim3((rows + 63) / 64), dim3(64), 0, s, status, rows);
@@ -688,6 +707,24 @@ int guffin::select_candidates_scaled(hipStream_t s, const float* logits, uint32_
                            keep, divisor, history, history_count, row_retain, row_stride, row_stride == 1 ? 64u : row_stride,
                            fresh, static_cast<Candidates*>(result), status);
     return check_launch("select_candidates(merge)");
+}
+
+// A law is decided where its selection ends: the workgroup that sorts a row's keys goes on with them, and the record, its trip and a
+// launch fall away (one row of 262144, 64 kept: 9.0 + 7.1 us and the boundary between them are 15.7; with all sixteen waves in the law's
+// meetings 16.7).  Other vocabularies are selected by tiles, their law a launch of its own.
+bool guffin::selection_makes_laws(uint32_t vocab, uint32_t retain) { return vocab >= retain && by_threshold(vocab, retain); }
+
+int guffin::select_law(hipStream_t s, const float* logits, uint32_t vocab, uint32_t retain, uint32_t sure, void* workspace, const LawCall& law,
+                       bool suppressed_ok) {
+    if (reinterpret_cast<uintptr_t>(workspace) & 7u) return fail(GUFFIN_E_ALIGN, "select_candidates: workspace must be 8-byte aligned");
+    const uint32_t segs = (vocab + kSeg - 1) / kSeg;
+    const float divisor = law.opt.temperature;
+    uint32_t* words = static_cast<uint32_t*>(workspace);
+    launch(segment_max_kernel, dim3((segs + 3) / 4, 1), dim3(256), 0, s, logits, vocab, segs, divisor, words, law.whole ? law.status : nullptr);
+    if (int rc = check_launch("draft_law(segment maxima)")) return rc;
+    launch(threshold_select_kernel<true>, dim3((vocab + kCollectTile - 1) / kCollectTile, 1), dim3(1024), 0, s, logits, words, vocab, segs, retain,
+           sure, divisor, 1u, nullptr, nullptr, nullptr, 64u, nullptr, law.status, suppressed_ok, law.whole != 0, law);
+    return check_launch("draft_law(threshold)");
 }
 
 extern "C" int guffin_hip_input_validation(void* stream, const uint32_t* actual, const uint32_t* expected, uint32_t rows,
