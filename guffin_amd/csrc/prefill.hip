@@ -191,24 +191,24 @@ __device__ __forceinline__ void emit_attention(const AttentionOut& to, const flo
     }
 }
 
-// a workgroup's LDS: four waves' outputs of an A tile, their states and the merged ones (queries and probabilities take less)
-constexpr uint32_t attention_lds(uint32_t nt) { return 4 * 16384 + 5 * nt * 16 * 2 * 4; }
-static_assert(attention_lds(2) >= 2 * (16384 + 4 * 16 * 32 * 4));
+// a workgroup's LDS: its waves' outputs of an A tile, their states and the merged ones (queries and probabilities take less)
+constexpr uint32_t attention_lds(uint32_t nt, uint32_t waves) { return waves * 16384 + (waves + 1) * nt * 16 * 2 * 4; }
+static_assert(attention_lds(2, 4) >= 2 * (16384 + 4 * 16 * 32 * 4));
 
-// grid (kv_heads * ceil(rows * group / (16 NT)), 1, parts), 4 waves.  Heads run fastest and the last rows come first: consecutive
+// grid (kv_heads * ceil(rows * group / (16 NT)), 1, parts), W waves.  Heads run fastest and the last rows come first: consecutive
 // workgroups go to different XCDs, so with eight KV heads an L2 holds one head's keys and values, and the longest lists of a causal
 // block start first.  (Tiles fastest, first rows first: 2048 rows 162 us instead of 142, 333 rows 22.6 instead of 17.6.)  A workgroup serves 16 NT (row, head) pairs of one KV head
 // -- the group's heads of 16 NT / group consecutive rows, as NT A tiles of 16 pairs -- and one part of the key range.  Each
-// wave walks its own 32-token tiles (tile index = wave mod 4) with its own online softmax state and its own output
-// accumulators; the four states are merged at the end.  A run of few rows is cut into parts so that the chip is full; their
+// wave walks its own 32-token tiles (tile index = wave mod W) with its own online softmax state and its own output
+// accumulators; the states are merged at the end.  A run of few rows is cut into parts so that the chip is full; their
 // states are merged by prefill_attention_merge_kernel.
 //   scores   S = Q K^T: queries (scaled, fp16 hi + lo, staged once in LDS in operand order) as A,
 //            keys straight from their fp16 rows as B (a lane reads 8 dims of one key per MFMA)
 //   softmax  a tile that every row sees whole needs no masks, and the accumulators are rescaled only where a maximum moved
 //   values   O += P V: probabilities times 2^10 as fp16 hi + lo through a wave-private LDS
 //            transpose as A, V^T rows as B
-template <int NT>
-__global__ void __launch_bounds__(256, 2)
+template <int NT, int W>
+__global__ void __launch_bounds__(64 * W, W == 4 ? 2 : 1)
 prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __restrict__ ring_k,
                               const uint16_t* __restrict__ run_k, const uint16_t* __restrict__ vt,
                               uint32_t rows, uint32_t position, uint32_t window, uint32_t ring_mask, uint32_t base32, uint32_t form,
@@ -244,10 +244,11 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         }
     };
     uint4 kb[2][8];
-    float4 qv[kPairs / 8][2];
+    constexpr uint32_t kStep = 2 * W;   // pairs staged (or stored) at a time
+    float4 qv[kPairs / kStep][2];
 #pragma unroll
-    for (uint32_t i = 0; i < kPairs / 8; ++i) {
-        const uint32_t m = 8 * i + threadIdx.x / 32, c8 = threadIdx.x % 32;
+    for (uint32_t i = 0; i < kPairs / kStep; ++i) {
+        const uint32_t m = kStep * i + threadIdx.x / 32, c8 = threadIdx.x % 32;
         const uint32_t row = min(r0 + (m >> group_shift), rows - 1), head = kvh * group + (m & (group - 1));
         const float* src = q + (size_t(row) * q_heads + head) * HD + 8 * c8;
         qv[i][0] = *reinterpret_cast<const float4*>(src); qv[i][1] = *reinterpret_cast<const float4*>(src + 4);
@@ -256,8 +257,8 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
     // one A tile leaves registers for the next keys beside the values: the first ones travel while the queries are staged
     if constexpr (NT == 1) ask_keys(min(begin + wave, tile_lo + tiles - 1), kb);
 #pragma unroll
-    for (uint32_t i = 0; i < kPairs / 8; ++i) {
-        const uint32_t m = 8 * i + threadIdx.x / 32, c8 = threadIdx.x % 32;
+    for (uint32_t i = 0; i < kPairs / kStep; ++i) {
+        const uint32_t m = kStep * i + threadIdx.x / 32, c8 = threadIdx.x % 32;
         const float4 a = qv[i][0], b = qv[i][1];
         const float x[8] = {a.x * scale, a.y * scale, a.z * scale, a.w * scale, b.x * scale, b.y * scale, b.z * scale, b.w * scale};
         uint4 hi, lo;
@@ -278,7 +279,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         for (int dt = 0; dt < 16; ++dt) O[g][dt] = float4_t{0.f, 0.f, 0.f, 0.f};
     }
     constexpr int VB = NT > 1 ? 8 : 16;   // one A tile: all values of a tile in registers, asked for ahead of the scores
-    for (uint32_t ti = begin + wave; ti < end; ti += 4) {
+    for (uint32_t ti = begin + wave; ti < end; ti += W) {
         const uint32_t t0 = base32 + 32 * ti;
         if constexpr (NT > 1) ask_keys(ti, kb);
         const uint16_t* vcol = vt + size_t(kvh) * HD * T + size_t(ti) * (32 * HD) + 32 * j + 8 * lg;
@@ -381,7 +382,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
                         O[g][first + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[g][half], __builtin_bit_cast(half8_t, vb[i]), O[g][first + i], 0, 0, 0);
         };
         if constexpr (NT == 1) {
-            if (ti + 4 < end) ask_keys(ti + 4, kb);
+            if (ti + W < end) ask_keys(ti + W, kb);
             values(0);
         } else {
             values(0);
@@ -393,14 +394,14 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    // Merge the four waves' states through LDS, an A tile at a time: every wave's outputs, scaled to the common maximum by their own
+    // Merge the waves' states through LDS, an A tile at a time: every wave's outputs, scaled to the common maximum by their own
     // wave, have room together and are summed in wave order by whoever stores them.  (One wave behind the other over the same slots:
     // three more passes over them,
     // 14 us of a workgroup's 65 at 2048 rows instead of 9.)
     float* ob = reinterpret_cast<float*>(lds);  // [wave][dt][4][64 lanes]; the query operands and the probabilities are dead now
     constexpr uint32_t kWaveSlots = 4096;       // of one wave's outputs
-    float* states = reinterpret_cast<float*>(lds + 4 * kWaveSlots * 4);   // [wave][pair][2]
-    float* ml = states + 4 * kPairs * 2;        // [pair][2], merged
+    float* states = reinterpret_cast<float*>(lds + W * kWaveSlots * 4);   // [wave][pair][2]
+    float* ml = states + W * kPairs * 2;        // [pair][2], merged
     __syncthreads();
     if (j == 0)
 #pragma unroll
@@ -415,13 +416,15 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t pair = 16 * g + 4 * lg + r;
-            float2 st[4];
+            float2 st[W];
 #pragma unroll
-            for (int w = 0; w < 4; ++w) st[w] = *reinterpret_cast<const float2*>(states + (w * kPairs + pair) * 2);
-            const float M = fmaxf(fmaxf(st[0].x, st[1].x), fmaxf(st[2].x, st[3].x));
+            for (int w = 0; w < W; ++w) st[w] = *reinterpret_cast<const float2*>(states + (w * kPairs + pair) * 2);
+            float M = st[0].x;
+#pragma unroll
+            for (int w = 1; w < W; ++w) M = fmaxf(M, st[w].x);
             float den = 0.f;
 #pragma unroll
-            for (int w = 0; w < 4; ++w) den += st[w].x == -INFINITY ? 0.f : st[w].y * exp_of(st[w].x - M);
+            for (int w = 0; w < W; ++w) den += st[w].x == -INFINITY ? 0.f : st[w].y * exp_of(st[w].x - M);
             const float mine = m[g][r] == -INFINITY ? 0.f : exp_of(m[g][r] - M);
             float* slots = ob + wave * kWaveSlots + r * 64 + lane;
 #pragma unroll
@@ -430,14 +433,19 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
         }
         __syncthreads();
 #pragma unroll 1
-        for (uint32_t n = 0; n < 2; ++n) {   // 32 consecutive lanes: one (row, head)
-            const uint32_t i = 8 * n + threadIdx.x / 32, c8 = threadIdx.x % 32, p = 16 * g + i;
+        for (uint32_t n = 0; n < 16 / kStep; ++n) {   // 32 consecutive lanes: one (row, head)
+            const uint32_t i = kStep * n + threadIdx.x / 32, c8 = threadIdx.x % 32, p = 16 * g + i;
             const uint32_t row = r0 + (p >> group_shift), head = kvh * group + (p & (group - 1));
             if (row >= rows) continue;
             const float* src = ob + (((c8 >> 1) * 4 + (i & 3)) * 64 + 8 * (c8 & 1) + 16 * (i >> 2));
             float v[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = src[k] + (src[kWaveSlots + k] + src[2 * kWaveSlots + k] + src[3 * kWaveSlots + k]);
+            for (int k = 0; k < 8; ++k) {
+                float more = src[kWaveSlots + k];
+#pragma unroll
+                for (uint32_t w = 2; w < W; ++w) more += src[w * kWaveSlots + k];
+                v[k] = src[k] + more;
+            }
             if (parts == 1) {
                 const float den = ml[p * 2 + 1] * kProbScale;
 #pragma unroll
@@ -643,17 +651,20 @@ extern "C" int guffin_hip_publish_run(void* stream, const void* run_k, const voi
 }
 
 namespace {
-// A tiles of a workgroup and parts of the key range.  Two tiles read a key and a value row once for twice the queries, so they
+// A tiles and waves of a workgroup, parts of the key range.  Two tiles read a key and a value row once for twice the queries, so they
 // stay while they leave a workgroup per compute unit; a short run takes single tiles (half the accumulators, half the merge)
 // and parts: two workgroups per compute unit, every wave of a part with a tile of its own.
-struct AttentionCut { uint32_t tiles, parts; };
+struct AttentionCut { uint32_t tiles, parts, waves; };
 AttentionCut attention_cut(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_t group) {
     const uint32_t pairs = rows * group, twos = (pairs + 31) / 32 * kv_heads, ones = (pairs + 15) / 16 * kv_heads;
     const uint32_t cus = compute_units();
-    if (twos >= cus) return {2, 1};
+    if (twos >= cus) return {2, 1, 4};
     // (one tile more than a wave each would be a second round for one of them: 37 rows behind 1500 tokens, 34 tiles in eight
     // parts 16.4 us, in nine 14.4; a second part costs the launch that merges them, more than a second round)
-    return {1, std::max(1u, std::min(2 * cus / ones, T < 256 ? 1 : (T + 127) / 128))};
+    const uint32_t parts = std::max(1u, std::min(2 * cus / ones, T < 256 ? 1 : (T + 127) / 128));
+    // Two parts are eight waves of one workgroup, which merges them itself: 1000 rows of the drafter 2025 -> 1934 us a pass, 256 of the 12B
+    // shapes 15442 -> 15107.  More parts in half as many such workgroups: 12 rows behind 1500 tokens 4659 -> 4793, 96 8516 -> 9083.
+    return parts == 2 ? AttentionCut {1, 1, 8} : AttentionCut {1, parts, 4};
 }
 uint64_t transposed_bytes(uint32_t T, uint32_t kv_heads) { return (uint64_t(kv_heads) * 256 * T * 2 + 255) & ~uint64_t{255}; }
 }  // namespace
@@ -673,7 +684,8 @@ extern "C" uint64_t guffin_hip_prefill_attention_workspace_bytes(uint32_t rows, 
 
 namespace guffin {
 int prefill_attention_init() {
-    return allow_lds(prefill_attention_mfma_kernel<1>, attention_lds(1)) && allow_lds(prefill_attention_mfma_kernel<2>, attention_lds(2)) ? 0 : -1;
+    return allow_lds(prefill_attention_mfma_kernel<1, 4>, attention_lds(1, 4)) && allow_lds(prefill_attention_mfma_kernel<1, 8>, attention_lds(1, 8))
+        && allow_lds(prefill_attention_mfma_kernel<2, 4>, attention_lds(2, 4)) ? 0 : -1;
 }
 
 bool prefill_attention_on_matrix_core(const void* q, const void* ring_k, const void* ring_v, const void* run_k, const void* run_v,
@@ -694,17 +706,17 @@ int prefill_attention_run(hipStream_t s, const float* q, const void* ring_k, con
                           void* workspace) {
     const ValueSpan vs = value_span(rows, position, window);
     const uint32_t group = q_heads / kv_heads, shift = group == 1 ? 0 : group == 2 ? 1 : 2;
-    const auto [nt, parts] = attention_cut(rows, vs.T, kv_heads, group);
+    const auto [nt, parts, waves] = attention_cut(rows, vs.T, kv_heads, group);
     if (kv_heads > 0xFFFFu) return fail(GUFFIN_E_SHAPE, "prefill_attention: more KV heads than a grid has rows");
     float* states = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + transposed_bytes(vs.T, kv_heads));
     const AttentionOut to {out, image, states, states + size_t(parts) * rows * q_heads * 256};
-    const uint32_t lds = attention_lds(nt);
+    const uint32_t lds = attention_lds(nt, waves);
     const dim3 grid((rows * group + 16 * nt - 1) / (16 * nt) * kv_heads, 1, parts);
     const uint32_t form = kv_heads | (shift << 16) | (parts << 18);   // at most two parts a compute unit
-#define GUFFIN_PA(NT_) launch(prefill_attention_mfma_kernel<NT_>, grid, dim3(256), lds, s, q, static_cast<const uint16_t*>(ring_k), \
+#define GUFFIN_PA(NT_, W_) launch((prefill_attention_mfma_kernel<NT_, W_>), grid, dim3(64 * W_), lds, s, q, static_cast<const uint16_t*>(ring_k), \
                               static_cast<const uint16_t*>(run_k), static_cast<const uint16_t*>(workspace), rows, position, window, ring_mask, \
                               vs.base32, form, scale, vs.T, to)
-    if (nt == 1) GUFFIN_PA(1); else GUFFIN_PA(2);
+    if (nt == 2) GUFFIN_PA(2, 4); else if (waves == 8) GUFFIN_PA(1, 8); else GUFFIN_PA(1, 4);
 #undef GUFFIN_PA
     if (int rc = check_launch("prefill_attention_mfma")) return rc;
     if (parts == 1) return GUFFIN_OK;

@@ -361,6 +361,25 @@ def test_prefill_attention_scores_are_as_close_as_plain_fp32(hip, q_heads, kv_he
     assert rms[0] <= (1.0 if q_heads == 4 * kv_heads else 1.25) * rms[1], rms
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,rows,position,window,cap", [
+    (4, 1, 690, 5, 512, 512), (4, 1, 1024, 0, 512, 512), (8, 8, 350, 40, 0, 512), (16, 8, 172, 100, 64, 128), (16, 8, 256, 0, 0, 16),
+    (2, 1, 1399, 0, 256, 256), (16, 8, 257, 20, 0, 64)])
+def test_prefill_attention_where_a_workgroup_takes_both_parts(hip, q_heads, kv_heads, rows, position, window, cap):
+    """Runs that would be cut into two parts go through workgroups of eight waves, which merge their states: one tile a wave and
+    none (a window of 64), the largest and smallest such runs, ragged rows, and the next longer run.  As close as any (2e-6)."""
+    import torch
+    hd = 256
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows)
+    rand = lambda *shape: torch.randn(shape, device="cuda", generator=gen)
+    q = rand(rows, q_heads * hd)
+    ring_k, ring_v = rand(cap, kv_heads * hd).half(), rand(cap, kv_heads * hd).half()
+    run_k, run_v = rand(rows, kv_heads * hd).half(), rand(rows, kv_heads * hd).half()
+    got = hip.prefill_attention(q, ring_k, ring_v, run_k, run_v, position, window, cap - 1, q_heads, kv_heads, hd, 0.0625, matrix_core=True)
+    want = double_attention(q, ring_k, ring_v, run_k, run_v, position, window, cap - 1, q_heads, kv_heads, 0.0625)
+    assert float((got.double() - want).abs().max()) <= 2e-6 * max(1.0, float(want.abs().max()))
+
+
 def test_prefill_attention_takes_queries_up_to_the_range_of_a_half(hip):
     """A query element of 60 000 after the scale (a half holds 65 504) against keys small enough for ordinary scores."""
     import torch
