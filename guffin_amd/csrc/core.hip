@@ -33,6 +33,7 @@ int gemv_packed_init(int device, int cu_count);
 int head_init();
 int attention_init();
 int prefill_attention_init();
+int prefill_gemm_init();
 
 }  // namespace guffin
 
@@ -56,7 +57,7 @@ extern "C" int guffin_hip_init(int device) {
         return fail(GUFFIN_E_HIP, buf);
     }
     if (gemv_init(prop.multiProcessorCount) != 0 || ops_init(prop.multiProcessorCount) != 0 || head_init() != 0
-        || attention_init() != 0 || prefill_attention_init() != 0 || resident_init(prop.multiProcessorCount) != 0)
+        || attention_init() != 0 || prefill_attention_init() != 0 || prefill_gemm_init() != 0 || resident_init(prop.multiProcessorCount) != 0)
         return fail(GUFFIN_E_HIP, "init: could not raise a kernel's dynamic LDS limit");
     if (gemv_packed_init(device, prop.multiProcessorCount) != 0)
         return fail(GUFFIN_E_HIP, "init: could not take the address of the static scratch array on this device");

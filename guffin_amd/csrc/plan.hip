@@ -742,6 +742,9 @@ class PrefillLaunches {
     std::vector<Set> sets_;
 };
 
+// floats of an operand image in front of something else
+uint64_t gated_floats(uint32_t rows, uint32_t F) { return (guffin_hip_prefill_image_bytes(rows, F) / 4 + 63) & ~uint64_t{63}; }
+
 PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, uint8_t* base) {
     Arena ar {base, 0, 0};
     const uint64_t H = m.hidden, QW = uint64_t(m.q_heads) * m.head_dim, KW = uint64_t(m.kv_heads) * m.head_dim;
@@ -758,6 +761,9 @@ PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, uint8_t
             for (uint32_t i = 0; i < g.count; ++i) width += g.m[i].N;
             planes = std::max(planes, uint64_t(g.split.slices) * rows * width);
         }
+        // the gated operand lies ahead of the planes of the product that reads it
+        if (prefill_gateup_tiles(m.layers[l].dtype[4], m.layers[l].dtype[5], rows, m.hidden, m.ffn))
+            planes = std::max(planes, gated_floats(rows, m.ffn) + uint64_t(launches(l, kGemmDown).split.slices) * rows * m.hidden);
     }
     s.planes = ar.take<float>(planes);
     s.rope_local = ar.take<float>(uint64_t(rows) * m.head_dim);
@@ -852,14 +858,14 @@ extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* mo
         GUFFIN_TRY(guffin_hip_prefill_pack(stream, s.u, s.image, rows, H));
     }
     // residual + rms(the planes), then the next norm, as the next GEMM's operand or (at the end) the output rows
-    auto joint = [&](uint32_t planes, const float* gamma_post, const float* residual, float* out_residual, const float* gamma_next,
+    auto joint = [&](const float* from, uint32_t planes, const float* gamma_post, const float* residual, float* out_residual, const float* gamma_next,
                      float* out, const RunRows& run) {
         if (fits)
-            return prefill_joint(hs, s.planes, planes, gamma_post, residual, out_residual, gamma_next, out, out ? nullptr : s.image, rows, H,
+            return prefill_joint(hs, from, planes, gamma_post, residual, out_residual, gamma_next, out, out ? nullptr : s.image, rows, H,
                                  m.eps, run, status);
         if (run.run_k)
             GUFFIN_TRY(guffin_hip_publish_run(stream, run.run_k, run.run_v, run.ring_k, run.ring_v, rows, position, run.ring_mask, KW));
-        GUFFIN_TRY(guffin_hip_rms_norm_add_norm(stream, s.planes, planes, uint64_t(rows) * H, gamma_post, residual, out_residual, gamma_next,
+        GUFFIN_TRY(guffin_hip_rms_norm_add_norm(stream, from, planes, uint64_t(rows) * H, gamma_post, residual, out_residual, gamma_next,
                                                 out ? out : s.u, nullptr, rows, H, m.eps, status));
         return out ? GUFFIN_OK : guffin_hip_prefill_pack(stream, s.u, s.image, rows, H);
     };
@@ -899,13 +905,20 @@ extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* mo
         float* const one[1] = {s.planes};
         GUFFIN_TRY(gemm(kGemmO, one));
         const RunRows run {s.run_k, s.run_v, L.ring_k, L.ring_v, rows > ring_mask + 1 ? rows - (ring_mask + 1) : 0u, position, ring_mask, KW / 8};
-        GUFFIN_TRY(joint(g[kGemmO].split.slices, L.norm[3], s.x, s.x1, L.norm[4], nullptr, run));
+        GUFFIN_TRY(joint(s.planes, g[kGemmO].split.slices, L.norm[3], s.x, s.x1, L.norm[4], nullptr, run));
+        const uint32_t gated = prefill_gateup_tiles(L.dtype[4], L.dtype[5], rows, H, m.ffn);
+        uint8_t* const operand = gated ? reinterpret_cast<uint8_t*>(s.planes) : s.image;
+        float* const down[1] = {gated ? s.planes + gated_floats(rows, m.ffn) : s.planes};
         float* const gu[2] = {s.planes, s.planes + uint64_t(g[kGemmGateUp].split.slices) * rows * m.ffn};
-        GUFFIN_TRY(gemm(kGemmGateUp, gu));
-        GUFFIN_TRY(prefill_geglu(hs, gu[0], gu[1], g[kGemmGateUp].split.slices, s.image, rows, m.ffn));
-        GUFFIN_TRY(gemm(kGemmDown, one));
+        if (gated) {
+            GUFFIN_TRY(prefill_gateup(hs, L.tiles[4], L.tiles[5], s.image, rows, H, m.ffn, gated, operand));
+        } else {
+            GUFFIN_TRY(gemm(kGemmGateUp, gu));
+            GUFFIN_TRY(prefill_geglu(hs, gu[0], gu[1], g[kGemmGateUp].split.slices, operand, rows, m.ffn));
+        }
+        GUFFIN_TRY(prefill_gemm_planes(hs, g[kGemmDown].m, 1, operand, down, rows, m.ffn, g[kGemmDown].split));
         const bool last = l + 1 == m.layer_count;
-        GUFFIN_TRY(joint(g[kGemmDown].split.slices, L.norm[5], s.x1, s.x, last ? m.out_norm : m.layers[l + 1].norm[0],
+        GUFFIN_TRY(joint(down[0], g[kGemmDown].split.slices, L.norm[5], s.x1, s.x, last ? m.out_norm : m.layers[l + 1].norm[0],
                          last ? out_hidden : nullptr, RunRows {}));
     }
     return GUFFIN_OK;

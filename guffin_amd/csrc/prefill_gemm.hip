@@ -32,6 +32,7 @@
 #include "common.hpp"
 #include "prefill_image.hpp"
 #include "prefill_run.hpp"
+#include "receipt.hpp"
 
 #include <algorithm>
 
@@ -720,34 +721,26 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
 }
 
 // ---- Q8_0 ------------------------------------------------------------------------------------------------
-// The same workgroup and stages; a 32-element block is one group, so its d and the span's multiplier are applied after
-// the two matrix instructions (hi, lo) of a tile.  grid as above, k-slices in chunks of two blocks.
+// The same stages; a 32-element block is one group, so its d and the span's multiplier are applied after the two matrix
+// instructions (hi, lo) of a tile.  Chunks [c0, c1) of two blocks; WAVES share the chunk's records, the waves of a pair (wv, wv + 4) by turns.
 template <int R>
-__global__ void __launch_bounds__(256, 2)
-prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const uint8_t* __restrict__ blob,
-                    uint32_t M, uint32_t K, uint32_t n0, uint32_t n1, uint32_t n2, uint32_t form, float* __restrict__ y0,
-                    float* __restrict__ y1, float* __restrict__ y2) {
-    constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q8_0), kSlot = Stage<R>::kChunk + 512;   // chunk, its two groups' multipliers
-    __shared__ __attribute__((aligned(16))) uint8_t stage[3 * kSlot];
-    const ImageLayout L = image_layout(M, K);
-    const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, lg = lane >> 4;
-    const GemmPlace at = place_of<R>(M, n0, n1, n2, form);
-    const uint32_t slices = form & ((1u << kSliceBits) - 1);
-    if (at.slice >= slices) return;
-    const GemmSegment seg = segment_of(at.group, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
-    const uint32_t tile_index = seg.first + wv, nblk = K / 32, rt0 = at.chunk * R;
-    const bool valid = tile_index < seg.columns;
-    const uint32_t chunks = (nblk + 1) / 2, c0 = at.slice * chunks / slices, c1 = (at.slice + 1) * chunks / slices;
-    const __amdgpu_buffer_rsrc_t img = make_resource(blob, static_cast<uint32_t>(L.bytes));
-    const __amdgpu_buffer_rsrc_t tile = make_resource(seg.tiles + size_t(valid ? tile_index : 0) * nblk * TB, nblk * TB);
-    const uint32_t lane16 = lane * 16, group_stride = (L.mpad / 16) * 2048, shift = L.span == 256 ? 3 : 0;
-    const uint32_t base = rt0 * 2048 + (wv & 1) * (1024 * R), mult_off = static_cast<uint32_t>(L.mult_off) + rt0 * 64;
+constexpr uint32_t kQ8Slot = Stage<R>::kChunk + 512;   // chunk, its two groups' multipliers
+template <int R, int WAVES>
+__device__ __forceinline__ void q8_walk(const ImageLayout& L, __amdgpu_buffer_rsrc_t img, __amdgpu_buffer_rsrc_t tile, uint8_t* stage, uint32_t lane,
+                                        uint32_t wv, uint32_t rt0, uint32_t nblk, uint32_t c0, uint32_t c1, float (&acc)[4][R][4]) {
+    constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q8_0), kSlot = kQ8Slot<R>;
+    constexpr int kOwn = WAVES == 4 ? R : R / 2;   // records that every wave asks for at least
+    const uint32_t j = lane & 15, lg = lane >> 4;
+    const uint32_t lane16 = lane * 16, group_stride = (L.mpad / 16) * 2048, shift = L.span == 256 ? 3 : 0, quarter = wv & 3;
+    const uint32_t base = rt0 * 2048 + (quarter & 1) * (1024 * R), mult_off = static_cast<uint32_t>(L.mult_off) + rt0 * 64;
     auto ask = [&](uint32_t chunk, uint32_t buffer) {
         const uint32_t c = chunk < c1 ? chunk : c1 - 1;
         uint8_t* to = stage + buffer * kSlot;
 #pragma unroll
         for (int i = 0; i < R; ++i)
-            to_lds16(img, to + (wv >> 1) * (2048 * R) + (wv & 1) * (1024 * R) + 1024 * i, lane16, base + min(2 * c + (wv >> 1), nblk - 1) * group_stride + 1024 * i);
+            if (WAVES == 4 || uint32_t(i & 1) == wv >> 2)
+                to_lds16(img, to + (quarter >> 1) * (2048 * R) + (quarter & 1) * (1024 * R) + 1024 * i, lane16,
+                         base + min(2 * c + (quarter >> 1), nblk - 1) * group_stride + 1024 * i);
         if (wv < 2) to_lds4(img, to + Stage<R>::kChunk + 256 * wv, lane * 4, mult_off + (min(2 * c + wv, nblk - 1) >> shift) * L.mpad * 4);
     };
     uint4 q[2][2][2];       // [buffer][group][piece]
@@ -762,7 +755,6 @@ prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict
             for (int cg = 0; cg < 4; ++cg) dw[to][h][cg] = ld4(tile, (j >> 1) * 4, at + 2048 + 32 * cg);
         }
     };
-    float acc[4][R][4];
 #pragma unroll
     for (int cg = 0; cg < 4; ++cg)
 #pragma unroll
@@ -775,7 +767,7 @@ prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict
     ask(c0 + 1, 1);
     uint32_t rd = 0, wr = 2;
     auto chunk = [&](uint32_t c, int now) {
-        arrive<R>();
+        arrive<kOwn>();
         ask_weights(c + 1, now ^ 1);
         ask(c + 2, wr);
         const uint8_t* from = stage + rd * kSlot;
@@ -820,10 +812,32 @@ prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict
         chunk(c, 0);
         if (c + 1 < c1) chunk(c + 1, 1);
     }
+    // the chunks asked for past the end are still on their way into this workgroup's LDS
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// grid as prefill_gemm_kernel's, k-slices in chunks of two blocks.
+template <int R>
+__global__ void __launch_bounds__(256, 2)
+prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const uint8_t* __restrict__ blob,
+                    uint32_t M, uint32_t K, uint32_t n0, uint32_t n1, uint32_t n2, uint32_t form, float* __restrict__ y0,
+                    float* __restrict__ y1, float* __restrict__ y2) {
+    constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q8_0);
+    __shared__ __attribute__((aligned(16))) uint8_t stage[3 * kQ8Slot<R>];
+    const ImageLayout L = image_layout(M, K);
+    const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, lg = lane >> 4;
+    const uint32_t slices = form & ((1u << kSliceBits) - 1);
+    const GemmSegment seg = segment_of(blockIdx.y, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
+    const uint32_t tile_index = seg.first + wv, nblk = K / 32, rt0 = blockIdx.x * R;
+    const bool valid = tile_index < seg.columns;
+    const uint32_t chunks = (nblk + 1) / 2, c0 = blockIdx.z * chunks / slices, c1 = (blockIdx.z + 1) * chunks / slices;
+    const __amdgpu_buffer_rsrc_t img = make_resource(blob, static_cast<uint32_t>(L.bytes));
+    const __amdgpu_buffer_rsrc_t tile = make_resource(seg.tiles + size_t(valid ? tile_index : 0) * nblk * TB, nblk * TB);
+    float acc[4][R][4];
+    q8_walk<R, 4>(L, img, tile, stage, lane, wv, rt0, nblk, c0, c1, acc);
     if (!valid) return;
     const uint32_t N = seg.columns * kCols;
-    float* y = seg.y + at.slice * (uint64_t(M) * N);
+    float* y = seg.y + blockIdx.z * (uint64_t(M) * N);
     const uint32_t col = tile_index * kCols + j, row0 = rt0 * 16 + 4 * lg;
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -834,6 +848,94 @@ prefill_gemm_q8_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict
 #pragma unroll
                 for (int cg = 0; cg < 4; ++cg) y[size_t(row) * N + col + 16 * cg] = acc[cg][r][i];
         }
+}
+
+// Gate, up and GeGLU: the next GEMM's operand straight from the products.  grid (row chunks, F / 256), eight waves: four gate tiles and the four
+// up tiles of the same columns, 256 of them -- one span of the operand.  A gate wave takes the first 32 columns of the tile pair over, its
+// up wave the others; values go through LDS from a column a lane to eight columns a lane, and the span's largest from wave to wave.
+// Bound by its first trips and the twenty vector instructions a column group costs (as above); 1000 rows of the drafter: 20.0 + 7.2 us as
+// two launches.
+template <int R>
+struct GatedStage {
+    static constexpr uint32_t kSwap = 8 * R * 2048;                           // half an accumulator of every wave
+    static constexpr uint32_t kPitch = 36, kTurn = 8 * 16 * R * kPitch * 4;    // rows of 32 columns of every wave
+    static constexpr uint32_t kWalk = 3 * kQ8Slot<R>;
+    static constexpr uint32_t kMost = kTurn > kSwap ? (kTurn > kWalk ? kTurn : kWalk) : (kSwap > kWalk ? kSwap : kWalk);
+    static constexpr uint32_t kBytes = kMost + 8 * 16 * R * 4;                 // and its rows' largest
+};
+template <int R>
+__global__ void __launch_bounds__(512)
+prefill_gateup_q8_kernel(const uint8_t* __restrict__ gate, const uint8_t* __restrict__ up, const uint8_t* __restrict__ blob, uint32_t M, uint32_t K,
+                         uint32_t F, uint8_t* __restrict__ out) {
+    constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q8_0);
+    using G = GatedStage<R>;
+    extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
+    const ImageLayout L = image_layout(M, K), O = image_layout(M, F);
+    const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, lg = lane >> 4;
+    const uint32_t pair = wv & 3, nblk = K / 32, rt0 = blockIdx.x * R;
+    const bool is_up = wv >= 4;
+    const __amdgpu_buffer_rsrc_t img = make_resource(blob, static_cast<uint32_t>(L.bytes));
+    const __amdgpu_buffer_rsrc_t tile = make_resource((is_up ? up : gate) + size_t(4 * blockIdx.y + pair) * nblk * TB, nblk * TB);
+    float acc[4][R][4];
+    q8_walk<R, 8>(L, img, tile, stage, lane, wv, rt0, nblk, 0, (nblk + 1) / 2, acc);
+    __syncthreads();
+    // the other half of the tile pair's products
+    float4_t* swap = reinterpret_cast<float4_t*>(stage);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float(&give)[4] = acc[is_up ? c : 2 + c][r];
+            swap[((wv * 2 + c) * R + r) * 64 + lane] = float4_t{give[0], give[1], give[2], give[3]};
+        }
+    __syncthreads();
+    float h[2][R][4];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float4_t other = swap[(((wv ^ 4) * 2 + c) * R + r) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float own = is_up ? acc[2 + c][r][i] : acc[c][r][i];
+                h[c][r][i] = is_up ? geglu_value(other[i], own) : geglu_value(own, other[i]);
+            }
+        }
+    __syncthreads();
+    float* turn = reinterpret_cast<float*>(stage) + wv * (16 * R * G::kPitch);   // this wave's [row][32 columns]
+    float* largest = reinterpret_cast<float*>(stage + G::kMost);                 // [wave][row]
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) turn[(16 * r + 4 * lg + i) * G::kPitch + 16 * c + j] = h[c][r][i];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own
+    // lane (row j, k-slice lg) of a record
+    float v[R][8];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float* from = turn + (16 * r + j) * G::kPitch + 8 * lg;
+        const float4_t a = *reinterpret_cast<const float4_t*>(from), b = *reinterpret_cast<const float4_t*>(from + 4);
+        float m = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) { v[r][k] = k < 4 ? a[k & 3] : b[k & 3]; m = fmaxf(m, fabsf(v[r][k])); }
+        m = fmaxf(m, __shfl_xor(m, 16, kWave));
+        m = fmaxf(m, __shfl_xor(m, 32, kWave));
+        if (lg == 0) largest[wv * (16 * R) + 16 * r + j] = m;
+    }
+    __syncthreads();
+    const uint32_t group = 8 * blockIdx.y + 2 * pair + (is_up ? 1u : 0u);   // of 32 columns
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        float m = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) m = fmaxf(m, largest[w * (16 * R) + 16 * r + j]);
+        const uint32_t row = 16 * (rt0 + r) + j;
+        if (row >= M) continue;
+        emit_image_record(v[r], m, group, lg, row, O, out);
+        if (wv == 0 && lg == 0) reinterpret_cast<float*>(out + O.mult_off)[size_t(blockIdx.y) * O.mpad + row] = image_multiplier(m);
+    }
 }
 
 // How many ways the XCDs cut the row chunks of a launch between them, the column groups being dealt over the others; 0: the grid's
@@ -918,6 +1020,33 @@ PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint3
 }
 
 }  // namespace
+
+int prefill_gemm_init() { return allow_lds(prefill_gateup_q8_kernel<4>, GatedStage<4>::kBytes) ? 0 : -1; }
+
+// The fewest row tiles a workgroup with which every workgroup has a compute unit, as long as more than half of them have work: a
+// launch, a write and a read of both products less.  A pass of the drafter (640 x 2048, 18 blocks), us, as two launches / so: 270 rows 1256 /
+// 1214, 512 1523 / 1461, 1024 2009 / 1896, 1536 2624 / 2491, 2048 3035 / 2905; fewer rows leave the chip idle (240: 1182 / 1185; 64: 912 /
+// 979), two row tiles where one is enough cost more (512: 1556).  Wider models form B too often so: 768 x 2304 1923 / 1855 at 700 rows, but
+// 1024 x 4096 1708 / 1762 at 300 and 2048 x 8192 1800 / 2003 at 100.
+uint32_t prefill_gateup_tiles(int gate_dtype, int up_dtype, uint32_t rows, uint32_t K, uint32_t F) {
+    if (gate_dtype != GUFFIN_Q8_0 || up_dtype != GUFFIN_Q8_0 || F % 256 != 0 || K > 768) return 0;
+    const uint32_t cus = compute_units();
+    for (uint32_t R = 1; R <= 4; ++R)
+        if ((rows + 16 * R - 1) / (16 * R) * (F / 256) <= cus) return R > 1 || (rows + 15) / 16 * (F / 256) > cus / 2 ? R : 0;
+    return 0;
+}
+
+int prefill_gateup(hipStream_t s, const void* gate, const void* up, const uint8_t* image, uint32_t M, uint32_t K, uint32_t F, uint32_t R, uint8_t* out) {
+    if (K % 32 != 0 || F % 256 != 0) return fail(GUFFIN_E_SHAPE, "prefill_gateup: need K % 32 == 0 and F % 256 == 0");
+    if ((reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up)) & 15u) return fail(GUFFIN_E_ALIGN, "prefill_gateup: tiles need 16-byte alignment");
+    if (image_layout(M, K).bytes >= (size_t(1) << 31)) return fail(GUFFIN_E_SHAPE, "prefill_gateup: the image of M x K exceeds 2 GiB, split the rows");
+    const dim3 grid((M + 16 * R - 1) / (16 * R), F / 256), block(512);
+    const uint8_t *g = static_cast<const uint8_t*>(gate), *u = static_cast<const uint8_t*>(up);
+#define GUFFIN_PG(R_) launch(prefill_gateup_q8_kernel<R_>, grid, block, GatedStage<R_>::kBytes, s, g, u, image, M, K, F, out)
+    if (R == 1) GUFFIN_PG(1); else if (R == 2) GUFFIN_PG(2); else if (R == 3) GUFFIN_PG(3); else GUFFIN_PG(4);
+#undef GUFFIN_PG
+    return check_launch("prefill_gateup");
+}
 
 PrefillSplit prefill_split(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K) { return split_for(m, count, M, K, 16); }
 

@@ -33,6 +33,50 @@ __host__ __device__ inline ImageLayout image_layout(uint32_t M, uint32_t K) {
     return L;
 }
 
+// biased exponent of a span's largest, clamped so that both scale factors are normal floats; the span's multiplier
+__device__ __forceinline__ uint32_t image_exponent(float largest) {
+    const uint32_t eb = __float_as_uint(largest) >> 23;
+    return eb < 15u ? 15u : eb > 244u ? 244u : eb;
+}
+__device__ __forceinline__ float image_multiplier(float largest) { return __uint_as_float((image_exponent(largest) - 14u) << 23); }
+
+// A record's share of a lane: elements 8s .. 8s+7 of 32-group g of a row whose span of 256 holds `largest`.  The lanes (row, 0 .. 3) of
+// a row, 16 apart, run it together.
+__device__ __forceinline__ void emit_image_record(const float (&v)[8], float largest, uint32_t g, uint32_t s, uint32_t row, const ImageLayout& L, uint8_t* blob) {
+    constexpr int order[8] = {0, 2, 1, 3, 4, 6, 5, 7};
+    const float inv = __uint_as_float((268u - image_exponent(largest)) << 23);
+    float sum = v[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) sum += v[i];
+    sum += __shfl_xor(sum, 16, kWave);
+    sum += __shfl_xor(sum, 32, kWave);
+    const uint32_t tile = row >> 4, i16 = row & 15u;
+    if (s == 0) {
+        const float sv = sum * (inv * 0.03125f);   // |sum| <= 32 times the span's largest
+        const _Float16 h = static_cast<_Float16>(sv), l = static_cast<_Float16>(sv - static_cast<float>(h));
+        uint8_t* rec = blob + L.sums_off + (size_t(g >> 3) * (L.mpad / 16) + tile) * 512 + i16 * 16 + order[g & 7u] * 2;
+        *reinterpret_cast<uint16_t*>(rec) = __builtin_bit_cast(uint16_t, h);
+        *reinterpret_cast<uint16_t*>(rec + 256) = __builtin_bit_cast(uint16_t, l);
+    }
+    uint32_t hi[4], lo[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        uint32_t hw = 0, lw = 0;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const float xv = v[order[2 * p + q]] * inv;
+            const _Float16 h = static_cast<_Float16>(xv);
+            const _Float16 l = static_cast<_Float16>(xv - static_cast<float>(h));
+            hw |= uint32_t(__builtin_bit_cast(uint16_t, h)) << (16 * q);
+            lw |= uint32_t(__builtin_bit_cast(uint16_t, l)) << (16 * q);
+        }
+        hi[p] = hw; lo[p] = lw;
+    }
+    uint8_t* base = blob + (size_t(g) * (L.mpad / 16) + tile) * 2048 + (i16 + 16 * s) * 16;
+    *reinterpret_cast<uint4*>(base) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    *reinterpret_cast<uint4*>(base + 1024) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+}
+
 // Elements 8t .. 8t+7 of row `row` (t counts along K).  The lanes of a span (32 or 4 consecutive t in consecutive,
 // aligned lanes) must run it together.  records: where a workgroup that holds 8 rows of eight groups collects their pieces of the
 // records (16 KB of LDS) instead of writing 16 bytes at a time to lines that it shares with other rows.

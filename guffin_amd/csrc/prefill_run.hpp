@@ -14,6 +14,11 @@ PrefillSplit prefill_split(const PrefillMatrix* m, uint32_t count, uint32_t M, u
 int prefill_gemm_planes(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M,
                         uint32_t K, PrefillSplit split);
 
+// gate, up and GeGLU of a Q8_0 block as one launch: out is the down projection's operand (not the memory of image)
+// row_tiles: of a workgroup; prefill_gateup_tiles has them, 0: the launches apart
+uint32_t prefill_gateup_tiles(int gate_dtype, int up_dtype, uint32_t rows, uint32_t K, uint32_t F);
+int prefill_gateup(hipStream_t s, const void* gate, const void* up, const uint8_t* image, uint32_t M, uint32_t K, uint32_t F, uint32_t row_tiles, uint8_t* out);
+
 // ---- attention (prefill.hip) -----------------------------------------------------------------
 struct ValueSpan { uint32_t first_visible, base32, T; };
 // virtual tokens whose values a run of `rows` rows at `position` can see, padded to whole 32-token tiles

@@ -480,6 +480,32 @@ def test_prefill_rows_agree_with_decode_at_row_tile_edges(hip, kind, rows, posit
         assert float((devm.ring_k[l][slot] == pk[l, 0]).float().mean()) >= 0.95 and float((devm.ring_v[l][slot] == pv[l, 0]).float().mean()) >= 0.95
 
 
+@pytest.mark.parametrize("hidden,ffn,rows", [(640, 2048, 256), (640, 2048, 257), (640, 2048, 512), (640, 2048, 513), (640, 2048, 1025),
+                                             (640, 2048, 1537), (640, 2048, 2047), (640, 2048, 2049), (768, 2304, 250), (64, 256, 2065),
+                                             (64, 256, 4100), (768, 1024, 555)])
+def test_a_run_s_gated_product_is_that_of_shorter_runs(hip, hidden, ffn, rows):
+    """Gate, up and GeGLU as one launch, with each number of row tiles, at its edges and one row past them, against the same tokens
+    as runs of at most 100 rows, which take the launches apart (of models this narrow: fewer than half the workgroups).  The bound is
+    that of runs against decoding: the same products in another order, 1e-4 of the row's rms."""
+    import random
+    from dataclasses import replace
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, hidden=hidden, ffn=ffn, layers=1, vocab=1024, ring_global=8192, ring_local=8192)
+    tokens = torch.tensor([random.Random(i).randrange(2, 1024) for i in range(rows)], dtype=torch.int32, device="cuda")
+    whole, cut = (model.DeviceModel.random(shape, seed=hidden, position=0) for _ in range(2))
+    hidden_rows, status = whole.prefill(tokens, 0)
+    parts = []
+    for at in range(0, rows, 100):
+        part, part_status = cut.prefill(tokens[at:at + 100].contiguous(), at)
+        assert int(part_status.item()) == 0
+        parts.append(part)
+    assert int(status.item()) == 0
+    want = torch.cat(parts).double()
+    scale = want.pow(2).mean(1, keepdim=True).sqrt()
+    assert float(((hidden_rows.double() - want).abs() / scale).max()) <= 1e-4
+
+
 @pytest.mark.parametrize("position", [0, 20, 95, 125, 200])
 @pytest.mark.parametrize("rows", [1, 2, 3, 4])
 @pytest.mark.parametrize("kind", ["target", "mixed", "drafter", "one_slice"])
