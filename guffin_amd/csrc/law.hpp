@@ -104,6 +104,13 @@ __device__ __forceinline__ T ordered_sums(const T* __restrict__ v, uint32_t n, T
     return sum;
 }
 
+// The smallest index of `hit` threads into *to (LDS): a wave finds its own and one lane enters it.  (Every hit's atomicMin on the one word is
+// served lane by lane: 2.0 us of a law's 6.7 for 200 of them, 1.8 of an acceptance's 11.8.)
+__device__ __forceinline__ void note_first(bool hit, uint32_t index, uint32_t* to) {
+    const uint64_t hits = __ballot(hit);
+    if (hits && (threadIdx.x & 63u) == 0) atomicMin(to, index + static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(hits))) - 1u);
+}
+
 // Sort of the first n keys in LDS by rank, n at most the workgroup's size: every thread counts the keys that go
 // before its own (all lanes read the same word: a broadcast) and drops its key at that place.  Three barriers
 // instead of the bitonic network's one per stage (28 for 128 keys, 45 for 512).
@@ -145,7 +152,7 @@ __device__ __forceinline__ void compact_law(const LawCall& call, uint32_t avail,
     const float cutoff = usable ? score[k - 1] : 0.f, first_logit = usable ? score[0] : 0.f;
     // entries are sorted by (score desc, token asc): the support is a prefix, its length the first
     // entry that is below the cutoff or -inf
-    if (!(t < avail && !(my_logit < cutoff) && my_logit != -INFINITY)) atomicMin(&s_first, t);
+    note_first(!(t < avail && !(my_logit < cutoff) && my_logit != -INFINITY), t, &s_first);
     __syncthreads();
     if (t == 0) {
         uint32_t st = 0, n = 0;

@@ -491,8 +491,8 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
     // entries (the first always) whose weight is at least min_p
     if (count) {
         const double total = out.run[count - 1];
-        if (t + 1 < count && !(out.run[t] / total < static_cast<double>(opt.top_p))) atomicMin(&sc.kept, t + 1);
-        if (opt.min_p > 0.f && t >= 1 && t < count && !(sc.w[t] >= static_cast<double>(opt.min_p))) atomicMin(&sc.cut, t);
+        note_first(t + 1 < count && !(out.run[t] / total < static_cast<double>(opt.top_p)), t + 1, &sc.kept);
+        if (opt.min_p > 0.f) note_first(t >= 1 && t < count && !(sc.w[t] >= static_cast<double>(opt.min_p)), t, &sc.cut);
     }
     __syncthreads();
     count = sc.kept < sc.cut ? sc.kept : sc.cut;
@@ -581,12 +581,12 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
         if (accepted) {
             const Prepared& after = prepared[1];
             if (scratch[1].err) code = scratch[1].err - 100;
-            else if (t < after.count && d.u_next * after.total < after.run[t]) atomicMin(&sc.pick, t);
+            else note_first(t < after.count && d.u_next * after.total < after.run[t], t, &sc.pick);
         } else {
             if (!total_usable(excess, residual_total) || !total_holds(sc.compensated[excess - 1], residual_total, excess)) code = -26;
-            else if (t < excess) {
-                if (!weight_usable(residual.weight[t], residual_total)) sc.flag = 1;
-                if (d.u_residual * residual_total < residual.run[t]) atomicMin(&sc.pick, t);
+            else {
+                if (t < excess && !weight_usable(residual.weight[t], residual_total)) sc.flag = 1;
+                note_first(t < excess && d.u_residual * residual_total < residual.run[t], t, &sc.pick);
             }
         }
     }
