@@ -981,24 +981,33 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
 }
 
 // Time of a launch by a model of the chip, in microseconds: `start` from the launch to the first product and from the last one
-// to the end, then every compute unit works off its share of the workgroups at `unit` per slice unit -- 256 elements
-// of K, 64 for Q8_0 --, and a plane costs a write here and a read in the next operator.  Constants fitted to sweeps
-// over 4 to 1000 rows of both models' shapes.  Against the best pair of a sweep of 5 to 2048 rows, planes counted: the 12B
-// shapes' launches 1 % longer on the mean, 12 % at most (64 rows); the drafter's, 4 to 30 us of them, 5 % and 45 %.
-constexpr float kStart[4] = {5.0f, 6.2f, 7.5f, 8.5f};
-constexpr float kUnit[3][4] = {{0.6f, 0.82f, 1.0f, 1.35f}, {2.3f, 2.7f, 3.2f, 3.8f}, {2.8f, 3.3f, 4.0f, 4.8f}};   // Q8_0, Q4_K, Q6_K
-constexpr float kPlaneBytesPerUs = 5.0e6f;
+// to the end, then every compute unit works off its share of the workgroups, each `workgroup` of its own and `unit` per slice unit -- 256
+// elements of K, 64 for Q8_0 --, one workgroup by itself on a compute unit `alone` of that (it leaves gaps that a second one fills); a plane
+// costs a write here and a read in the next operator.  Constants fitted to sweeps over 4 to 1000 rows of both models' shapes.
+//
+// K-quant launches of up to kShortRun rows have a set of their own, fitted to whole passes over every pair of 5 to 150 rows after the
+// kernels had lost a tenth of their instructions: what a workgroup costs by itself now counts, and one workgroup a compute unit beats
+// twice as many half as long (gate + up of 64 rows: two slices, not three).  A pass of the 12B shapes, us, by the other set / by this one: 5 rows
+// 4536 / 4487, 20 rows 5034 / 4982, 37 rows 6411 / 6167, 55 rows 7378 / 6922, 64 rows 6920 / 6382, 128 rows 9570 / 9331, 96 rows
+// 8027 / 8078.  Past the line it finds nothing in most runs and loses some: 200 rows 14528 / 14638, 512 rows 26588 / 26793.  A product of one
+// to sixteen slices is 1.30-1.53e-7 (Q4_K, K = 3840 and 4096) and 1.72-2.15e-7 (Q6_K) of its rms from 64 bits, the most with one, as in long runs.
+struct SplitCosts { float start[4], unit[3][4], alone[4], workgroup, plane_bytes; };   // unit: Q8_0, Q4_K, Q6_K
+constexpr uint32_t kShortRun = 192;
+constexpr SplitCosts kShort = {{4.6f, 6.7f, 8.2f, 9.3f}, {{}, {2.27f, 2.61f, 3.19f, 4.08f}, {2.92f, 3.62f, 4.73f, 5.61f}}, {1.21f, 1.19f, 1.17f, 1.11f}, 5.1f, 14.4e6f};
+constexpr SplitCosts kLong = {{5.0f, 6.2f, 7.5f, 8.5f}, {{0.6f, 0.82f, 1.0f, 1.35f}, {2.3f, 2.7f, 3.2f, 3.8f}, {2.8f, 3.3f, 4.0f, 4.8f}},
+                              {1.22f, 1.22f, 1.22f, 1.22f}, 0.0f, 5.0e6f};
 
 PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K, uint32_t most) {
     uint32_t groups = 0, width = 0;
     float unit[4] = {};   // of a workgroup, the mean over the launch
     bool q8 = false;
+    for (uint32_t i = 0; i < count; ++i) q8 |= m[i].dtype == GUFFIN_Q8_0;
+    const SplitCosts& costs = q8 || M > kShortRun ? kLong : kShort;
     for (uint32_t i = 0; i < count; ++i) {
         const uint32_t n = (m[i].N / kCols + 3) / 4;
         groups += n;
         width += m[i].N;
-        q8 |= m[i].dtype == GUFFIN_Q8_0;
-        for (int r = 0; r < 4; ++r) unit[r] += float(n) * kUnit[m[i].dtype][r];
+        for (int r = 0; r < 4; ++r) unit[r] += float(n) * costs.unit[m[i].dtype][r];
     }
     const uint32_t units = q8 ? (K + 63) / 64 : K / 256;   // what a slice is made of
     const uint32_t cus = compute_units();
@@ -1008,11 +1017,10 @@ PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint3
         const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
         for (uint32_t S = 1; S <= std::max(1u, std::min(units, most)); ++S) {
             const uint32_t n = chunks * groups * S;
-            // one workgroup per compute unit leaves gaps that a second one fills; the last, partly filled turn overlaps the
-            // one before it: half of it counts
-            const float turns = std::max(1.22f, 0.5f * (float((n + cus - 1) / cus) + float(n) / float(cus)));
-            const float cost = kStart[R - 1] + turns * float((units + S - 1) / S) * unit[R - 1] / float(groups)
-                + float(S) * 8.0f * float(M) * float(width) / kPlaneBytesPerUs;
+            // the last, partly filled turn overlaps the one before it: half of it counts
+            const float turns = std::max(costs.alone[R - 1], 0.5f * (float((n + cus - 1) / cus) + float(n) / float(cus)));
+            const float cost = costs.start[R - 1] + turns * (costs.workgroup + float((units + S - 1) / S) * unit[R - 1] / float(groups))
+                + float(S) * 8.0f * float(M) * float(width) / costs.plane_bytes;
             if ((R == 1 && S == 1) || cost < least) { best = {R, S}; least = cost; }
         }
     }

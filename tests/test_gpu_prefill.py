@@ -480,6 +480,34 @@ def test_prefill_rows_agree_with_decode_at_row_tile_edges(hip, kind, rows, posit
         assert float((devm.ring_k[l][slot] == pk[l, 0]).float().mean()) >= 0.95 and float((devm.ring_v[l][slot] == pv[l, 0]).float().mean()) >= 0.95
 
 
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("rows", [5, 31, 37, 48, 49, 64, 65, 96, 112, 128, 192, 193])
+def test_a_short_run_s_splits_are_those_of_shorter_runs(hip, rows, mixed):
+    """A block of the 12B shapes, whose products a run of up to 192 rows cuts into other slices and row tiles than a longer one, on
+    both sides of that line and at the edges of row tiles, against the same tokens as runs of at most four, which the verify pass'
+    streaming products take.  The bar is that of runs against decoding: fp32 sums of exact products in another order, and fp16 K/V
+    rows that may round the other way."""
+    import random
+    from dataclasses import replace
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_12B, layers=1, vocab=1024, ring_global=512, ring_local=512, sliding_window=256)
+    if mixed:
+        shape = replace(shape, layer_dtypes=((synth.Q4_K,) * 7,))
+    tokens = torch.tensor([random.Random(i).randrange(2, 1024) for i in range(rows)], dtype=torch.int32, device="cuda")
+    whole, cut = (model.DeviceModel.random(shape, seed=7, position=0) for _ in range(2))
+    hidden_rows, status = whole.prefill(tokens, 0)
+    parts = []
+    for at in range(0, rows, 4):
+        part, part_status = cut.prefill(tokens[at:at + 4].contiguous(), at)
+        assert int(part_status.item()) == 0
+        parts.append(part)
+    assert int(status.item()) == 0
+    want = torch.cat(parts).double()
+    scale = want.pow(2).mean(1, keepdim=True).sqrt()
+    assert float(((hidden_rows.double() - want).abs() / scale).max()) <= 2e-4
+
+
 @pytest.mark.parametrize("hidden,ffn,rows", [(640, 2048, 256), (640, 2048, 257), (640, 2048, 512), (640, 2048, 513), (640, 2048, 1025),
                                              (640, 2048, 1537), (640, 2048, 2047), (640, 2048, 2049), (768, 2304, 250), (64, 256, 2065),
                                              (64, 256, 4100), (768, 1024, 555)])
