@@ -1010,6 +1010,10 @@ PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint3
         for (int r = 0; r < 4; ++r) unit[r] += float(n) * costs.unit[m[i].dtype][r];
     }
     const uint32_t units = q8 ? (K + 63) / 64 : K / 256;   // what a slice is made of
+    // A Q8_0 slice has two units at least: a single one is a workgroup's first trips and little else, and leaves twice the planes (q/k/v of the
+    // 640-wide drafter: ten, which the next operator asks for in two goes).  A pass, us, with slices of one unit / so: 16 rows 786 / 756, 30 rows
+    // 836 / 795, 48 rows 884 / 838, 57 rows 989 / 930; from 64 rows on, where the model cuts less, 865 / 852 and 0.3-0.9 % less.
+    if (q8) most = std::min(most, units / 2);
     const uint32_t cus = compute_units();
     PrefillSplit best {1, 1};
     float least = 0.f;

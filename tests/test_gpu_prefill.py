@@ -480,6 +480,12 @@ def test_prefill_rows_agree_with_decode_at_row_tile_edges(hip, kind, rows, posit
         assert float((devm.ring_k[l][slot] == pk[l, 0]).float().mean()) >= 0.95 and float((devm.ring_v[l][slot] == pv[l, 0]).float().mean()) >= 0.95
 
 
+@pytest.mark.parametrize("rows,position", [(16, 0), (48, 90), (64, 0)])
+def test_short_drafter_runs_agree_with_decode(hip, rows, position):
+    """As at the edges of row tiles, where a Q8_0 slice has two units of K and more."""
+    test_prefill_rows_agree_with_decode_at_row_tile_edges(hip, "drafter", rows, position)
+
+
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("rows", [5, 31, 37, 48, 49, 64, 65, 96, 112, 128, 192, 193])
 def test_a_short_run_s_splits_are_those_of_shorter_runs(hip, rows, mixed):
