@@ -251,9 +251,12 @@ __device__ __forceinline__ void products(const half8_t (&a)[R], const half8_t (&
 // next region's A operands come from LDS and the next group's B operands are formed, so a wave by itself keeps the matrix
 // pipe and the vector pipe busy together.  A chunk's last lo half is in registers when its last region starts: there the
 // workgroup meets, the next chunk has arrived and the one after the next but one is asked for in place of the old.
-template <int R>
+// HALVES: the sums start anew at block `mid`, the first half's wait in LDS (`kept_sums`, [4 R][256 threads]): a slice of twice the length
+// rounds as two slices, and the planes, the workgroups' first trips and the next operator's reads are those of one.
+constexpr uint32_t kKeptStride = 256;   // of a thread's quads: the workgroup's
+template <int R, bool HALVES>
 __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint8_t* stage, const uint8_t* tile_base,
-                                        uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
+                                        uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4], uint32_t mid, float4_t* kept_sums) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q4_K);
     constexpr int V = (26 + 4 * R - 1) / (4 * R);   // vector instructions behind each matrix instruction
     // Up to three row tiles the fold is woven in as well: a tile's beside the next tile's products, the last one's beside the
@@ -310,6 +313,19 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
     for (uint32_t blk = b0; blk < b1; ++blk) {
         if constexpr (!WOVEN) { lane = lane_again(); j = lane & 15; lg = lane >> 4; lane16 = feed.lane16 = lane * 16; }   // no register to keep addresses in
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
+        if constexpr (HALVES) {
+            if (blk == mid) {
+                float4_t* to = kept_sums + wv * 64 + lane_again();
+#pragma unroll
+                for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        float(&sum)[4] = acc[cg][r];
+                        to[(cg * R + r) * kKeptStride] = float4_t{sum[0], sum[1], sum[2], sum[3]};
+                        sum[0] = sum[1] = sum[2] = sum[3] = 0.f;
+                    }
+            }
+        }
         float dh[4];   // the first half's sums leave their chain for acc (no bias term yet)
         auto fold_scales = [&] {
 #pragma unroll
@@ -666,7 +682,7 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
 
 // grid (row chunks, column groups of 256 over all segments, k-slices), so that an XCD's L2 keeps its share of the image, or as
 // row_ways has it; 256 threads.
-template <int R, int KINDS>
+template <int R, int KINDS, bool HALVES = false>
 __global__ void __launch_bounds__(256, 2)
 prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const uint8_t* __restrict__ blob,
                     uint32_t M, uint32_t K, uint32_t n0, uint32_t n1, uint32_t n2, uint32_t form, float* __restrict__ y0,
@@ -689,6 +705,7 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
     feed.base = rt0 * 2048 + (wv & 1) * (1024 * R);
     feed.wv = wv;
     feed.last = 4 * b1 - 1;
+    extern __shared__ float4_t first_sums[];   // HALVES: [4 R][256 threads]
     // a whole form per format: what they share would have to lie in the same registers for both
     auto run = [&](auto walk, uint32_t bytes) {
         float acc[4][R][4];
@@ -699,6 +716,17 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[cg][r][i] = 0.f;
         walk(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * bytes), rt0, b0, b1, acc);
+        if constexpr (HALVES) {
+            const float4_t* from = first_sums + wv * 64 + lane_again();
+#pragma unroll
+            for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float4_t first = from[(cg * R + r) * kKeptStride];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[cg][r][i] = first[i] + acc[cg][r][i];
+                }
+        }
         // the chunks asked for past the end are still on their way into this workgroup's LDS
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (!valid) return;
@@ -715,7 +743,8 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
                     for (int cg = 0; cg < 4; ++cg) y[size_t(row) * N + col + 16 * cg] = acc[cg][r][i];
             }
     };
-    if (KINDS == 1 || (KINDS == 3 && seg.dtype == GUFFIN_Q4_K)) run(q4_walk<R>, block_bytes(GUFFIN_Q4_K));
+    auto q4 = [&](auto&&... args) { q4_walk<R, HALVES>(args..., (2 * at.slice + 1) * nblk / (2 * slices), first_sums); };
+    if (KINDS == 1 || (KINDS == 3 && seg.dtype == GUFFIN_Q4_K)) run(q4, block_bytes(GUFFIN_Q4_K));
     else if constexpr (KINDS != 1 && R == 4) run(q6_walk_wide<R>, block_bytes(GUFFIN_Q6_K));
     else if constexpr (KINDS != 1) run(q6_walk<R>, block_bytes(GUFFIN_Q6_K));
 }
@@ -946,8 +975,9 @@ prefill_gateup_q8_kernel(const uint8_t* __restrict__ gate, const uint8_t* __rest
 // 102185.  The drafter's weights are small beside its image: 333 rows 1302 / 1417 / 1375.
 uint32_t row_ways(uint32_t chunks, bool q8) { return q8 || chunks < 2 || chunks > 10 ? 0 : chunks <= 6 ? 1 : 2; }
 
+constexpr uint32_t kept_bytes(uint32_t R) { return 4 * R * kKeptStride * sizeof(float4_t); }
 int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M, uint32_t K,
-                uint32_t slices, uint32_t R) {
+                uint32_t slices, uint32_t R, bool halves) {
     if (count > 3 || slices >= 1u << kSliceBits) return fail(GUFFIN_E_SHAPE, "prefill_gemm: at most three matrices and 31 slices");
     GemmArgs a {};
     a.blob = image; a.M = M; a.K = K; a.form = slices;
@@ -959,6 +989,7 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
         groups += (a.columns[i] + 3) / 4;
         kinds |= m[i].dtype == GUFFIN_Q4_K ? 1u : m[i].dtype == GUFFIN_Q6_K ? 2u : 4u;
     }
+    if (halves && (kinds != 1 || 2 * slices > K / 256)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: a slice in halves is two blocks of Q4_K at least");
     const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
     dim3 grid(chunks, groups, slices), block(256);
     if (const uint32_t ways = row_ways(chunks, kinds == 4u)) {
@@ -969,7 +1000,8 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
 #define GUFFIN_PG_ARGS a.tiles[0], a.tiles[1], a.tiles[2], a.blob, a.M, a.K, a.columns[0], a.columns[1], a.columns[2], a.form, a.y[0], a.y[1], a.y[2]
 #define GUFFIN_PG(R_) \
     do { \
-        if (kinds == 1) launch(prefill_gemm_kernel<R_, 1>, grid, block, 0, s, GUFFIN_PG_ARGS); \
+        if (halves) launch((prefill_gemm_kernel<R_, 1, true>), grid, block, kept_bytes(R_), s, GUFFIN_PG_ARGS); \
+        else if (kinds == 1) launch(prefill_gemm_kernel<R_, 1>, grid, block, 0, s, GUFFIN_PG_ARGS); \
         else if (kinds == 2) launch(prefill_gemm_kernel<R_, 2>, grid, block, 0, s, GUFFIN_PG_ARGS); \
         else if (kinds == 3) launch(prefill_gemm_kernel<R_, 3>, grid, block, 0, s, GUFFIN_PG_ARGS); \
         else launch(prefill_gemm_q8_kernel<R_>, grid, block, 0, s, GUFFIN_PG_ARGS); \
@@ -986,54 +1018,97 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
 // costs a write here and a read in the next operator.  Constants fitted to sweeps over 4 to 1000 rows of both models' shapes.
 //
 // K-quant launches of up to kShortRun rows have a set of their own, fitted to whole passes over every pair of 5 to 150 rows after the
-// kernels had lost a tenth of their instructions: what a workgroup costs by itself now counts, and one workgroup a compute unit beats
-// twice as many half as long (gate + up of 64 rows: two slices, not three).  A pass of the 12B shapes, us, by the other set / by this one: 5 rows
-// 4536 / 4487, 20 rows 5034 / 4982, 37 rows 6411 / 6167, 55 rows 7378 / 6922, 64 rows 6920 / 6382, 128 rows 9570 / 9331, 96 rows
-// 8027 / 8078.  Past the line it finds nothing in most runs and loses some: 200 rows 14528 / 14638, 512 rows 26588 / 26793.  A product of one
-// to sixteen slices is 1.30-1.53e-7 (Q4_K, K = 3840 and 4096) and 1.72-2.15e-7 (Q6_K) of its rms from 64 bits, the most with one, as in long runs.
+// kernels had lost a tenth of their instructions: what a workgroup costs by itself counts there, and one workgroup a compute unit beats twice as
+// many half as long.  It chooses among the cuts whose sums round no more than those of the other set's cut, see rounding().  A pass of the 12B
+// shapes, us, by the other set / so: 5 rows 4568 / 4550, 20 rows 5430 / 5374, 37 rows 6429 / 6293, 55 rows 7430 / 7137, 64 rows 7701 / 7302, 100 rows
+// 10453 / 10121, 128 rows 10671 / 10406; what planes cost differs from machine to machine, on another one 37 rows 6198 / 6215, 64 rows 7381 / 7131, 100
+// rows 9901 / 9909.  Past the line it finds nothing in most runs and loses some: 200 rows 14528 / 14638, 512 rows 26588 / 26793.
 struct SplitCosts { float start[4], unit[3][4], alone[4], workgroup, plane_bytes; };   // unit: Q8_0, Q4_K, Q6_K
-constexpr uint32_t kShortRun = 192;
+constexpr uint32_t kShortRun = 192;   // whole row tiles
 constexpr SplitCosts kShort = {{4.6f, 6.7f, 8.2f, 9.3f}, {{}, {2.27f, 2.61f, 3.19f, 4.08f}, {2.92f, 3.62f, 4.73f, 5.61f}}, {1.21f, 1.19f, 1.17f, 1.11f}, 5.1f, 14.4e6f};
 constexpr SplitCosts kLong = {{5.0f, 6.2f, 7.5f, 8.5f}, {{0.6f, 0.82f, 1.0f, 1.35f}, {2.3f, 2.7f, 3.2f, 3.8f}, {2.8f, 3.3f, 4.0f, 4.8f}},
                               {1.22f, 1.22f, 1.22f, 1.22f}, 0.0f, 5.0e6f};
 
-PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K, uint32_t most) {
-    uint32_t groups = 0, width = 0;
-    float unit[4] = {};   // of a workgroup, the mean over the launch
-    bool q8 = false;
-    for (uint32_t i = 0; i < count; ++i) q8 |= m[i].dtype == GUFFIN_Q8_0;
-    const SplitCosts& costs = q8 || M > kShortRun ? kLong : kShort;
+// The part of a sum's squared error that its cut decides: an addition rounds at the size its chain has reached, so a chain of
+// units / S blocks (half as many in halves) counts by its length and the one over S planes by its own, weighted by what a block's other
+// roundings leave of it.  rms error from 64 bits, 1e-7 of the result's rms, of 1, 2, 4, 8 and all slices: Q4_K, K = 3840 1.52, 1.38, 1.33, 1.33,
+// 1.40, K = 15360 2.30, 1.85, 1.59, 1.49, (16) 1.50; Q6_K, K = 3840 1.79, 1.74, 1.73, 1.75, 1.82, K = 15360 2.17, 1.96, 1.85, 1.82, (16)
+// 1.86; Q4_K in halves, 1, 2 and 4 slices: K = 3840 1.38, 1.33, 1.32, K = 15360 1.86, 1.59, 1.47.
+constexpr float kPlaneRounding[3] = {0.f, 0.54f, 1.2f};
+constexpr float rounding(uint32_t units, uint32_t S, uint32_t halves, float plane) { return float(units) / float(S << halves) + plane * float(S + halves); }
+
+constexpr float kHalvesCost = 0.04f;   // us a row tile: through LDS and back (fitted: 17 to 32 rows keep four slices of gate + up, 20 rows 5169 us instead of 5290)
+struct SplitShape { uint32_t units, groups, width, most; bool q8; float unit[4]; };   // units: what a slice is made of; unit: of a workgroup, the mean over the launch
+SplitShape split_shape(const PrefillMatrix* m, uint32_t count, uint32_t K, uint32_t most, const SplitCosts& costs) {
+    SplitShape s {};
     for (uint32_t i = 0; i < count; ++i) {
         const uint32_t n = (m[i].N / kCols + 3) / 4;
-        groups += n;
-        width += m[i].N;
-        for (int r = 0; r < 4; ++r) unit[r] += float(n) * costs.unit[m[i].dtype][r];
+        s.q8 |= m[i].dtype == GUFFIN_Q8_0;
+        s.groups += n;
+        s.width += m[i].N;
+        for (int r = 0; r < 4; ++r) s.unit[r] += float(n) * costs.unit[m[i].dtype][r];
     }
-    const uint32_t units = q8 ? (K + 63) / 64 : K / 256;   // what a slice is made of
+    s.units = s.q8 ? (K + 63) / 64 : K / 256;
     // A Q8_0 slice has two units at least: a single one is a workgroup's first trips and little else, and leaves twice the planes (q/k/v of the
     // 640-wide drafter: ten, which the next operator asks for in two goes).  A pass, us, with slices of one unit / so: 16 rows 786 / 756, 30 rows
     // 836 / 795, 48 rows 884 / 838, 57 rows 989 / 930; from 64 rows on, where the model cuts less, 865 / 852 and 0.3-0.9 % less.
-    if (q8) most = std::min(most, units / 2);
+    s.most = std::max(1u, std::min(most, s.q8 ? s.units / 2 : s.units));
+    return s;
+}
+
+template <typename Allowed>
+PrefillSplit cheapest_split(const SplitShape& s, const SplitCosts& costs, uint32_t M, Allowed allowed, uint32_t most_halves = 0) {
     const uint32_t cus = compute_units();
-    PrefillSplit best {1, 1};
+    const float plane = 8.0f * float(M) * float(s.width) / costs.plane_bytes;
+    PrefillSplit best {};
     float least = 0.f;
     for (uint32_t R = 1; R <= 4; ++R) {
         const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
-        for (uint32_t S = 1; S <= std::max(1u, std::min(units, most)); ++S) {
-            const uint32_t n = chunks * groups * S;
-            // the last, partly filled turn overlaps the one before it: half of it counts
-            const float turns = std::max(costs.alone[R - 1], 0.5f * (float((n + cus - 1) / cus) + float(n) / float(cus)));
-            const float cost = costs.start[R - 1] + turns * (costs.workgroup + float((units + S - 1) / S) * unit[R - 1] / float(groups))
-                + float(S) * 8.0f * float(M) * float(width) / costs.plane_bytes;
-            if ((R == 1 && S == 1) || cost < least) { best = {R, S}; least = cost; }
+        for (uint32_t S = 1; S <= s.most; ++S) {
+            const float fixed = costs.start[R - 1] + float(S) * plane;
+            if (best.slices && fixed >= least) break;   // grows with S
+            for (uint32_t halves = 0; halves <= most_halves; ++halves) {
+                if (!allowed(R, S, halves)) continue;
+                const uint32_t n = chunks * s.groups * S;
+                // the last, partly filled turn overlaps the one before it: half of it counts
+                const float turns = std::max(costs.alone[R - 1], 0.5f * (float((n + cus - 1) / cus) + float(n) / float(cus)));
+                const float cost = fixed + turns * (costs.workgroup + float(halves) * kHalvesCost * float(R)
+                                                    + float((s.units + S - 1) / S) * s.unit[R - 1] / float(s.groups));
+                if (!best.slices || cost < least) { best = {R, S, halves}; least = cost; }
+            }
         }
     }
     return best;
 }
 
+PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K, uint32_t most) {
+    const SplitShape shape = split_shape(m, count, K, most, kLong);
+    auto any = [](uint32_t, uint32_t, uint32_t) { return true; };
+    if (shape.q8 || M > kShortRun) return cheapest_split(shape, kLong, M, any);
+    // one cut for all runs of as many row tiles, by the costs in their middle: it holds against the other set's for the shortest and the longest
+    const uint32_t last = (M + 15) & ~15u;
+    const PrefillSplit bar[2] = {cheapest_split(shape, kLong, last - 15, any), cheapest_split(shape, kLong, last, any)};
+    bool q4 = true;
+    for (uint32_t i = 0; i < count; ++i) q4 &= m[i].dtype == GUFFIN_Q4_K;
+    // (Q6_K in four row tiles adds up in another order, 1 % further off: q6_walk_wide)
+    const uint32_t tallest = q4 || (bar[0].row_tiles == 4 && bar[1].row_tiles == 4) ? 4 : 3;
+    auto close = [&](uint32_t R, uint32_t S, uint32_t halves) {
+        if (R > tallest || (halves && 2 * S > shape.units)) return false;
+        for (uint32_t i = 0; i < count; ++i)
+            for (const PrefillSplit& b : bar)
+                if (rounding(shape.units, S, halves, kPlaneRounding[m[i].dtype]) > rounding(shape.units, b.slices, 0, kPlaneRounding[m[i].dtype])) return false;
+        return true;
+    };
+    const PrefillSplit best = cheapest_split(split_shape(m, count, K, most, kShort), kShort, last - 8, close, q4 && most > 1 ? 1u : 0u);
+    return best.slices ? best : bar[1];
+}
+
 }  // namespace
 
-int prefill_gemm_init() { return allow_lds(prefill_gateup_q8_kernel<4>, GatedStage<4>::kBytes) ? 0 : -1; }
+int prefill_gemm_init() {
+    return allow_lds(prefill_gateup_q8_kernel<4>, GatedStage<4>::kBytes) && allow_lds((prefill_gemm_kernel<2, 1, true>), kept_bytes(2))
+        && allow_lds((prefill_gemm_kernel<3, 1, true>), kept_bytes(3)) && allow_lds((prefill_gemm_kernel<4, 1, true>), kept_bytes(4)) ? 0 : -1;
+}
 
 // The fewest row tiles a workgroup with which every workgroup has a compute unit, as long as more than half of them have work: a
 // launch, a write and a read of both products less.  A pass of the drafter (640 x 2048, 18 blocks), us, as two launches / so: 270 rows 1256 /
@@ -1060,7 +1135,8 @@ int prefill_gateup(hipStream_t s, const void* gate, const void* up, const uint8_
     return check_launch("prefill_gateup");
 }
 
-PrefillSplit prefill_split(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K) { return split_for(m, count, M, K, 16); }
+constexpr uint32_t kMostSlices = 16;
+PrefillSplit prefill_split(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K) { return split_for(m, count, M, K, kMostSlices); }
 
 int prefill_gemm_planes(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M,
                         uint32_t K, PrefillSplit split) {
@@ -1076,7 +1152,7 @@ int prefill_gemm_planes(hipStream_t s, const PrefillMatrix* m, uint32_t count, c
             if (int rc = prefill_gemm_planes(s, m + i, 1, image, y + i, M, K, split)) return rc;
         return GUFFIN_OK;
     }
-    return gemm_launch(s, m, count, image, y, M, K, split.slices, split.row_tiles);
+    return gemm_launch(s, m, count, image, y, M, K, split.slices, split.row_tiles, split.halves);
 }
 }  // namespace guffin
 
@@ -1108,5 +1184,5 @@ extern "C" int guffin_hip_prefill_gemm(void* stream, int dtype, const void* tile
     // the kernels address the image with 32-bit offsets
     if (image_layout(M, K).bytes >= (size_t(1) << 31)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: the image of M x K exceeds 2 GiB, split the rows");
     const PrefillMatrix m {dtype, tiles, N};
-    return gemm_launch(as_stream(stream), &m, 1, static_cast<const uint8_t*>(image), &y, M, K, 1, split_for(&m, 1, M, K, 1).row_tiles);
+    return gemm_launch(as_stream(stream), &m, 1, static_cast<const uint8_t*>(image), &y, M, K, 1, split_for(&m, 1, M, K, 1).row_tiles, false);
 }

@@ -6,8 +6,9 @@ namespace guffin {
 
 // ---- GEMM (prefill_gemm.hip) ---------------------------------------------------------------
 struct PrefillMatrix { int dtype; const void* tiles; uint32_t N; };
-// rows per workgroup in tiles of 16, and k-slices: every slice leaves a plane of partial sums
-struct PrefillSplit { uint32_t row_tiles, slices; };
+// rows per workgroup in tiles of 16, and k-slices: every slice leaves a plane of partial sums; halves (Q4_K alone): a workgroup adds up its
+// slice as two
+struct PrefillSplit { uint32_t row_tiles, slices, halves; };
 // the split for `count` matrices (at most 3) over the same K that run as one launch
 PrefillSplit prefill_split(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K);
 // y[i]: split.slices planes of [M][N_i], one behind the other
@@ -30,7 +31,8 @@ inline ValueSpan value_span(uint32_t rows, uint32_t position, uint32_t window) {
 // The matrix-core path wants one, two or four query heads per KV head, and K/V rows and queries at 16-byte addresses.
 bool prefill_attention_on_matrix_core(const void* q, const void* ring_k, const void* ring_v, const void* run_k, const void* run_v,
                                       uint32_t q_heads, uint32_t kv_heads);
-// the largest workspace of a run of `rows` rows that sees at most T tokens
+// the workspace of a run of `rows` rows that sees at most T tokens; the largest of any run of up to `rows` rows
+uint64_t prefill_attention_bytes(uint32_t rows, uint32_t T, uint32_t q_heads, uint32_t kv_heads);
 uint64_t prefill_attention_most_bytes(uint32_t rows, uint32_t T, uint32_t q_heads, uint32_t kv_heads);
 // workspace: the transposed values of the span (already there) and room for the parts' states behind them; image: the
 // operand of the o projection

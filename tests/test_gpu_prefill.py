@@ -85,6 +85,47 @@ def test_prefill_gemm_sums_against_64_bits(hip, rows):
     assert float(((y - want).pow(2).mean() / want.pow(2).mean()).sqrt()) <= 1.6e-7
 
 
+@pytest.mark.parametrize("M,row_tiles", [(1, 1), (16, 1), (31, 2), (45, 3), (64, 4), (113, 4), (192, 3)])
+@pytest.mark.parametrize("K,slices", [(512, 1), (768, 1), (3840, 1), (3840, 2), (3840, 7), (4096, 8)])
+def test_a_slice_in_halves_is_the_sum_of_two_slices(hip, M, row_tiles, K, slices):
+    """Bit for bit: the same chains and the same addition, with odd and even numbers of blocks in a slice and a ragged group of columns."""
+    import torch
+    from prefill_cuts import Split, planes
+    N = 64 * 5
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + K)
+    tiles = hip.repack(1, dev(synth.make_weight(1, K, N, seed=K + slices)), K, N)
+    image = hip.prefill_pack(torch.randn((M, K), device="cuda", generator=gen))
+    whole = planes(1, tiles, image, M, K, N, Split(row_tiles, slices, 1))
+    parts = planes(1, tiles, image, M, K, N, Split(row_tiles, 2 * slices, 0))
+    assert torch.equal(whole, parts[0::2] + parts[1::2])
+
+
+@pytest.mark.parametrize("name,rows", [("gate_up", 24), ("gate_up", 37), ("gate_up", 55), ("gate_up", 64), ("gate_up", 100), ("gate_up", 144),
+                                       ("qkv4", 80), ("qkv4", 176), ("down4", 150), ("o", 20), ("o", 40), ("o", 104), ("down", 60)])
+def test_a_short_run_s_sums_are_as_close_as_in_the_long_runs_slices(hip, name, rows):
+    """rms error against 64 bits over 32 column tiles, in the planes' order.  1.005: the spread of such an estimate over two cuts of the same
+    products (some 1e5 of them)."""
+    import torch
+    from prefill_cuts import PRODUCTS, Split, bar, planes, split
+    K, parts = PRODUCTS[name]
+    dtype, N = parts[0][0], 64 * 32
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows)
+    w = dev(synth.make_weight(dtype, K, N, seed=rows))
+    x = torch.randn((rows, K), device="cuda", generator=gen)
+    want = x.double() @ hip.dequant(dtype, w, N * K // 256).view(N, K).double().T.contiguous()
+    tiles, image = hip.repack(dtype, w, K, N), hip.prefill_pack(x)
+    errors = []
+    for cut in (split(name, rows), Split(1, bar(name, rows), 0)):
+        y = planes(dtype, tiles, image, rows, K, N, cut)
+        total = y[0]
+        for plane in y[1:]:
+            total = total + plane
+        errors.append(float((total.double() - want).pow(2).mean().sqrt()))
+    assert errors[0] <= 1.005 * errors[1], errors
+
+
 @pytest.mark.parametrize("dtype,N", [(1, 64), (1, 64 * 33), (2, 64 * 5), (2, 64 * 36)])
 @pytest.mark.parametrize("M", [65, 97, 385, 449, 577, 640, 641, 705])
 def test_prefill_gemm_wherever_its_workgroups_go(hip, dtype, N, M):
