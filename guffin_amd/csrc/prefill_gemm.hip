@@ -1068,8 +1068,9 @@ PrefillSplit cheapest_split(const SplitShape& s, const SplitCosts& costs, uint32
             const float fixed = costs.start[R - 1] + float(S) * plane;
             if (best.slices && fixed >= least) break;   // grows with S
             for (uint32_t halves = 0; halves <= most_halves; ++halves) {
-                if (!allowed(R, S, halves)) continue;
                 const uint32_t n = chunks * s.groups * S;
+                // (halves: the sums that wait leave room for one workgroup of three or four row tiles a compute unit)
+                if (!allowed(R, S, halves) || (halves && n > cus)) continue;
                 // the last, partly filled turn overlaps the one before it: half of it counts
                 const float turns = std::max(costs.alone[R - 1], 0.5f * (float((n + cus - 1) / cus) + float(n) / float(cus)));
                 const float cost = fixed + turns * (costs.workgroup + float(halves) * kHalvesCost * float(R)
@@ -1093,7 +1094,7 @@ PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint3
     // (Q6_K in four row tiles adds up in another order, 1 % further off: q6_walk_wide)
     const uint32_t tallest = q4 || (bar[0].row_tiles == 4 && bar[1].row_tiles == 4) ? 4 : 3;
     auto close = [&](uint32_t R, uint32_t S, uint32_t halves) {
-        if (R > tallest || (halves && 2 * S > shape.units)) return false;
+        if (R > tallest || (halves && 2 * S > std::max(bar[0].slices, bar[1].slices))) return false;   // halves stand for two of its slices
         for (uint32_t i = 0; i < count; ++i)
             for (const PrefillSplit& b : bar)
                 if (rounding(shape.units, S, halves, kPlaneRounding[m[i].dtype]) > rounding(shape.units, b.slices, 0, kPlaneRounding[m[i].dtype])) return false;
