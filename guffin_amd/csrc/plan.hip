@@ -704,7 +704,10 @@ struct PrefillScratch {
 
 // the four GEMM launches of a block
 enum { kGemmQkv, kGemmO, kGemmGateUp, kGemmDown };
-struct PrefillLaunch { PrefillMatrix m[3]; uint32_t count, K; PrefillSplit split; };
+struct PrefillLaunch {
+    PrefillMatrix m[3]; uint32_t count, K; PrefillSplit split;
+    uint64_t width() const { uint64_t w = 0; for (uint32_t i = 0; i < count; ++i) w += m[i].N; return w; }
+};
 
 // A block's launches; their splits depend on its seven formats, of which a model has few sets: worked out once per set and call.
 class PrefillLaunches {
@@ -745,33 +748,70 @@ class PrefillLaunches {
 // floats of an operand image in front of something else
 uint64_t gated_floats(uint32_t rows, uint32_t F) { return (guffin_hip_prefill_image_bytes(rows, F) / 4 + 63) & ~uint64_t{63}; }
 
-PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, uint8_t* base) {
+// What the layout keeps whose size falls where a longer run is cut into fewer parts.
+struct PrefillPieces { uint64_t planes, attention; };   // floats; bytes
+
+// Whether an earlier block has block l's formats.
+bool formats_seen(const guffin_model_desc& m, uint32_t l) {
+    for (uint32_t e = 0; e < l; ++e)
+        if (std::memcmp(m.layers[e].dtype, m.layers[l].dtype, sizeof(m.layers[l].dtype)) == 0) return true;
+    return false;
+}
+
+// every token a row may see: at most a full ring plus the run, in whole 32-token tiles from an aligned start
+uint32_t prefill_span(const guffin_model_desc& m, uint32_t rows) { return (std::max(m.ring_global, m.sliding_window) + rows + 95) & ~31u; }
+
+PrefillPieces prefill_pieces(const guffin_model_desc& m, uint32_t rows) {
+    PrefillPieces p {};
+    PrefillLaunches launches(m, rows);
+    for (uint32_t l = 0; l < m.layer_count; ++l) {
+        for (int which = 0; which < 4; ++which) {
+            const PrefillLaunch g = launches(l, which);
+            p.planes = std::max(p.planes, uint64_t(g.split.slices) * rows * g.width());
+        }
+        // the gated operand lies ahead of the planes of the product that reads it
+        if (prefill_gateup_tiles(m.layers[l].dtype[4], m.layers[l].dtype[5], rows, m.hidden, m.ffn))
+            p.planes = std::max(p.planes, gated_floats(rows, m.ffn) + uint64_t(launches(l, kGemmDown).split.slices) * rows * m.hidden);
+    }
+    p.attention = prefill_attention_bytes(rows, prefill_span(m, rows), m.q_heads, m.kv_heads);
+    return p;
+}
+
+// The most of both that any run of up to `rows` rows keeps: an arena made for a chunk also takes the shorter last one.
+PrefillPieces prefill_most_pieces(const guffin_model_desc& m, uint32_t rows) {
+    PrefillPieces p = prefill_pieces(m, rows);
+    PrefillLaunches launches(m, rows);
+    for (uint32_t l = 0; l < m.layer_count; ++l) {
+        if (formats_seen(m, l)) continue;
+        for (int which = 0; which < 4; ++which) {
+            const PrefillLaunch g = launches(l, which);
+            const uint64_t width = g.width();
+            p.planes = std::max(p.planes, prefill_most_rows(g.m, g.count, rows, g.K, p.planes / width) * width);
+        }
+        // the gated operand of the longest run that has one, ahead of the most planes that any run has
+        for (uint32_t last = rows; last > 0; last = (last - 1) & ~15u)
+            if (prefill_gateup_tiles(m.layers[l].dtype[4], m.layers[l].dtype[5], last, m.hidden, m.ffn)) {
+                const PrefillLaunch g = launches(l, kGemmDown);
+                p.planes = std::max(p.planes, gated_floats(last, m.ffn) + prefill_most_rows(g.m, g.count, last, g.K, 0) * m.hidden);
+                break;
+            }
+    }
+    p.attention = prefill_attention_most_bytes(rows, prefill_span(m, rows), m.q_heads, m.kv_heads);
+    return p;
+}
+
+PrefillScratch prefill_layout(const guffin_model_desc& m, uint32_t rows, const PrefillPieces& pieces, uint8_t* base) {
     Arena ar {base, 0, 0};
     const uint64_t H = m.hidden, QW = uint64_t(m.q_heads) * m.head_dim, KW = uint64_t(m.kv_heads) * m.head_dim;
     PrefillScratch s {};
     s.x = ar.take<float>(rows * H); s.x1 = ar.take<float>(rows * H);
     s.u = ar.take<float>(H > kPrefillMaxWidth ? rows * H : 0);
     s.q = ar.take<float>(rows * QW); s.a = ar.take<float>(rows * QW);
-    uint64_t planes = 0;
-    PrefillLaunches launches(m, rows);
-    for (uint32_t l = 0; l < m.layer_count; ++l) {
-        for (int which = 0; which < 4; ++which) {
-            const PrefillLaunch g = launches(l, which);
-            uint64_t width = 0;
-            for (uint32_t i = 0; i < g.count; ++i) width += g.m[i].N;
-            planes = std::max(planes, uint64_t(g.split.slices) * rows * width);
-        }
-        // the gated operand lies ahead of the planes of the product that reads it
-        if (prefill_gateup_tiles(m.layers[l].dtype[4], m.layers[l].dtype[5], rows, m.hidden, m.ffn))
-            planes = std::max(planes, gated_floats(rows, m.ffn) + uint64_t(launches(l, kGemmDown).split.slices) * rows * m.hidden);
-    }
-    s.planes = ar.take<float>(planes);
+    s.planes = ar.take<float>(pieces.planes);
     s.rope_local = ar.take<float>(uint64_t(rows) * m.head_dim);
     s.rope_global = ar.take<float>(uint64_t(rows) * m.head_dim);
     s.run_k = ar.take<uint16_t>(rows * KW); s.run_v = ar.take<uint16_t>(rows * KW);
-    // every token a row may see: at most a full ring plus the run, in whole 32-token tiles from an aligned start
-    const uint32_t most = (std::max(m.ring_global, m.sliding_window) + rows + 95) & ~31u;
-    s.attn_ws = ar.take<uint8_t>(prefill_attention_most_bytes(rows, most, m.q_heads, m.kv_heads));
+    s.attn_ws = ar.take<uint8_t>(pieces.attention);
     const uint32_t widest = std::max({m.hidden, m.ffn, m.q_heads * m.head_dim});
     s.image = ar.take<uint8_t>(guffin_hip_prefill_image_bytes(rows, widest));
     s.positions = ar.take<uint32_t>(rows);
@@ -814,7 +854,12 @@ __global__ void fill_positions_kernel(uint32_t* positions, uint32_t rows, uint32
 
 extern "C" uint64_t guffin_hip_prefill_scratch_bytes(const guffin_model_desc* model, uint32_t rows) {
     if (!model || rows == 0 || guffin::validate_model(model)) return 0;
-    return guffin::prefill_layout(*model, rows, nullptr).bytes;
+    return guffin::prefill_layout(*model, rows, guffin::prefill_most_pieces(*model, rows), nullptr).bytes;
+}
+
+extern "C" uint64_t guffin_hip_prefill_run_bytes(const guffin_model_desc* model, uint32_t rows) {
+    if (!model || rows == 0 || guffin::validate_model(model)) return 0;
+    return guffin::prefill_layout(*model, rows, guffin::prefill_pieces(*model, rows), nullptr).bytes;
 }
 
 extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* model, const uint32_t* tokens,
@@ -827,7 +872,7 @@ extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* mo
     GUFFIN_TRY(check_ring_capacity(*model, position, rows, "prefill_rows: the rows do not fit the KV rings"));
     if (reinterpret_cast<uintptr_t>(scratch) & 255u) return fail(GUFFIN_E_ALIGN, "prefill_rows: scratch must be 256-byte aligned");
     const guffin_model_desc& m = *model;
-    const PrefillScratch s = prefill_layout(m, rows, static_cast<uint8_t*>(scratch));
+    const PrefillScratch s = prefill_layout(m, rows, prefill_pieces(m, rows), static_cast<uint8_t*>(scratch));
     if (s.bytes > scratch_bytes) return fail(GUFFIN_E_CAPACITY, "prefill_rows: scratch arena too small");
     hipStream_t hs = as_stream(stream);
     if (short_run_fits(m, rows)) {

@@ -667,18 +667,28 @@ AttentionCut attention_cut(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_
     return parts == 2 ? AttentionCut {1, 1, 8} : AttentionCut {1, parts, 4};
 }
 uint64_t transposed_bytes(uint32_t T, uint32_t kv_heads) { return (uint64_t(kv_heads) * 256 * T * 2 + 255) & ~uint64_t{255}; }
+uint64_t state_bytes(uint32_t parts, uint32_t rows, uint32_t heads) { return parts > 1 ? uint64_t(parts) * rows * heads * (256 + 2) * 4 : 0; }
+// The most bytes of states of any run of up to `rows` rows that sees at most T tokens.  Runs of as many single tiles are cut into as many
+// parts, the longest of them has the most rows; from a number of tiles on none is cut.
+uint64_t most_state_bytes(uint32_t rows, uint32_t T, uint32_t kv_heads, uint32_t group) {
+    uint64_t most = 0;
+    for (uint32_t tiles = 1; tiles * kv_heads <= 2 * compute_units(); ++tiles) {
+        const uint32_t last = std::min(rows, 16 * tiles / group);
+        if (last == 0) continue;   // one row takes more
+        most = std::max(most, state_bytes(attention_cut(last, T, kv_heads, group).parts, last, kv_heads * group));
+        if (last == rows) break;
+    }
+    return most;
+}
 }  // namespace
 
 extern "C" uint64_t guffin_hip_prefill_attention_workspace_bytes(uint32_t rows, uint32_t position, uint32_t window,
                                                                  uint32_t kv_heads, uint32_t head_dim) {
     if (rows == 0 || kv_heads == 0 || head_dim != 256) return 0;
-    // the values of all visible tokens transposed, then the parts' states (the query heads of a KV head are not known here: 4)
+    // the values of all visible tokens transposed, then the parts' states (the query heads of a KV head are not known here: 1, 2 or 4)
     const uint32_t T = value_span(rows, position, window).T;
     uint64_t states = 0;
-    for (uint32_t group = 1; group <= 4; group *= 2) {
-        const uint64_t parts = attention_cut(rows, T, kv_heads, group).parts;
-        if (parts > 1) states = std::max(states, parts * rows * kv_heads * group * (256 + 2) * 4);
-    }
+    for (uint32_t group = 1; group <= 4; group *= 2) states = std::max(states, most_state_bytes(rows, T, kv_heads, group));
     return transposed_bytes(T, kv_heads) + states;
 }
 
@@ -696,9 +706,11 @@ bool prefill_attention_on_matrix_core(const void* q, const void* ring_k, const v
              | reinterpret_cast<uintptr_t>(ring_v) | reinterpret_cast<uintptr_t>(run_v)) & 15u) == 0;
 }
 
+uint64_t prefill_attention_bytes(uint32_t rows, uint32_t T, uint32_t q_heads, uint32_t kv_heads) {
+    return transposed_bytes(T, kv_heads) + state_bytes(attention_cut(rows, T, kv_heads, q_heads / kv_heads).parts, rows, q_heads);
+}
 uint64_t prefill_attention_most_bytes(uint32_t rows, uint32_t T, uint32_t q_heads, uint32_t kv_heads) {
-    const uint64_t parts = attention_cut(rows, T, kv_heads, q_heads / kv_heads).parts;
-    return transposed_bytes(T, kv_heads) + (parts > 1 ? parts * rows * q_heads * (256 + 2) * 4 : 0);
+    return transposed_bytes(T, kv_heads) + most_state_bytes(rows, T, kv_heads, q_heads / kv_heads);
 }
 
 int prefill_attention_run(hipStream_t s, const float* q, const void* ring_k, const void* run_k, float* out, uint8_t* image, uint32_t rows,

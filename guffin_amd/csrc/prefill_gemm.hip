@@ -1139,6 +1139,14 @@ int prefill_gateup(hipStream_t s, const void* gate, const void* up, const uint8_
 constexpr uint32_t kMostSlices = 16;
 PrefillSplit prefill_split(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K) { return split_for(m, count, M, K, kMostSlices); }
 
+// Runs of as many row tiles differ in what a plane costs alone, so the shortest of them has the most slices and the longest the most rows.
+uint64_t prefill_most_rows(const PrefillMatrix* m, uint32_t count, uint32_t rows, uint32_t K, uint64_t least) {
+    const uint32_t most = split_shape(m, count, K, kMostSlices, kLong).most;
+    for (uint32_t last = rows; last > 0 && uint64_t(most) * last > least; last = (last - 1) & ~15u)
+        least = std::max(least, uint64_t(prefill_split(m, count, ((last - 1) & ~15u) + 1, K).slices) * last);
+    return least;
+}
+
 int prefill_gemm_planes(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M,
                         uint32_t K, PrefillSplit split) {
     bool q8 = false, k = false;

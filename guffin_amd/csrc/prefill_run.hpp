@@ -11,6 +11,8 @@ struct PrefillMatrix { int dtype; const void* tiles; uint32_t N; };
 struct PrefillSplit { uint32_t row_tiles, slices, halves; };
 // the split for `count` matrices (at most 3) over the same K that run as one launch
 PrefillSplit prefill_split(const PrefillMatrix* m, uint32_t count, uint32_t M, uint32_t K);
+// the most plane rows (slices times rows) that the launch keeps in any run of up to `rows` rows, or `least` if that is more
+uint64_t prefill_most_rows(const PrefillMatrix* m, uint32_t count, uint32_t rows, uint32_t K, uint64_t least);
 // y[i]: split.slices planes of [M][N_i], one behind the other
 int prefill_gemm_planes(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M,
                         uint32_t K, PrefillSplit split);

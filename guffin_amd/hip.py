@@ -59,6 +59,7 @@ class _Calls:
         "guffin_hip_forward_scratch_bytes": (Q, P, U, U),
         "guffin_hip_forward_rows": (I, P, P, P, U, U, P, Q, P, P, P, P, P),
         "guffin_hip_prefill_scratch_bytes": (Q, P, U),
+        "guffin_hip_prefill_run_bytes": (Q, P, U),
         "guffin_hip_prefill_rows": (I, P, P, P, U, U, P, Q, P, P),
         "guffin_hip_h1_step": (I, P, P, P, P, Q, P, P, P, P, P, P),
     }

@@ -378,7 +378,7 @@ class DeviceModel:
         """Ingests len(tokens) rows at `position` (rings are updated); returns the output-normed rows."""
         sh = self.shape
         rows = tokens.numel()
-        nbytes = hip._calls.guffin_hip_prefill_scratch_bytes(C.byref(self.desc), rows)
+        nbytes = hip._calls.guffin_hip_prefill_run_bytes(C.byref(self.desc), rows)
         if nbytes == 0:
             raise hip.GuffinError(-1, hip.lib().guffin_hip_last_error().decode())
         scratch = torch.empty(nbytes, dtype=torch.uint8, device="cuda")

@@ -513,8 +513,8 @@ int guffin_hip_prefill_gemm(void* stream, int dtype, const void* tiles, const vo
  * run_k / run_v [rows][kv_heads*head_dim]; window = 0 for global layers, else the sliding
  * window (the last `window` positions including the row's own).  q, out: [rows][q_heads*256].
  * workspace: guffin_hip_prefill_attention_workspace_bytes bytes (16-byte aligned) for the
- * transposed values and the partial results of the matrix-core path (q_heads / kv_heads 1, 2 or 4); NULL selects the
- * vector-unit kernel, which needs none. */
+ * transposed values and the partial results of the matrix-core path (q_heads / kv_heads 1, 2 or 4), enough for any run of up
+ * to `rows` rows there; NULL selects the vector-unit kernel, which needs none. */
 uint64_t guffin_hip_prefill_attention_workspace_bytes(uint32_t rows, uint32_t position, uint32_t window,
                                                       uint32_t kv_heads, uint32_t head_dim);
 int guffin_hip_prefill_attention(void* stream, const float* q, const void* ring_k, const void* ring_v,
@@ -538,8 +538,11 @@ int guffin_hip_kv_cache_copy(void* stream, const void* src_k, const void* src_v,
                              uint32_t row_width);
 /* The block graph of guffin_hip_forward_rows for any number of rows (prompt ingestion): same
  * operator order, matrix-core GEMMs, the run's K/V published to the rings layer by layer.
- * out_hidden [rows][hidden] holds the output-normed rows. */
+ * out_hidden [rows][hidden] holds the output-normed rows.  scratch: guffin_hip_prefill_scratch_bytes bytes take every run of up to
+ * `rows` rows (a shorter run may be cut into more parts and need more than a longer one); guffin_hip_prefill_run_bytes is what
+ * a run of exactly `rows` rows needs, for a caller that allocates for each. */
 uint64_t guffin_hip_prefill_scratch_bytes(const guffin_model_desc* model, uint32_t rows);
+uint64_t guffin_hip_prefill_run_bytes(const guffin_model_desc* model, uint32_t rows);
 int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* model, const uint32_t* tokens,
                             uint32_t rows, uint32_t position, void* scratch, uint64_t scratch_bytes,
                             float* out_hidden, uint32_t* status);

@@ -521,6 +521,25 @@ def test_prefill_rows_agree_with_decode_at_row_tile_edges(hip, kind, rows, posit
         assert float((devm.ring_k[l][slot] == pk[l, 0]).float().mean()) >= 0.95 and float((devm.ring_v[l][slot] == pv[l, 0]).float().mean()) >= 0.95
 
 
+@pytest.mark.parametrize("chunk,rows", [(785, 600), (785, 785), (132, 120)])
+def test_a_shorter_run_in_a_chunk_s_arena(hip, chunk, rows):
+    """The arena is the caller's, made once for its chunk size: the same bits as in one of the run's own."""
+    import ctypes as C
+    import torch
+    from dataclasses import replace
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M if chunk > 200 else model.GEMMA3_12B, layers=1, vocab=1024, ring_global=1024)
+    tokens = torch.arange(2, 2 + rows, dtype=torch.int32, device="cuda")
+    devm = model.DeviceModel.random(shape, seed=chunk, position=0)
+    want, status = devm.prefill(tokens, 0)
+    nbytes = hip._calls.guffin_hip_prefill_scratch_bytes(C.byref(devm.desc), chunk)
+    arena = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
+    got = torch.empty_like(want)
+    hip.check(hip._calls.guffin_hip_prefill_rows(hip._raw_stream(), C.byref(devm.desc), tokens.data_ptr(), rows, 0, arena.data_ptr(), nbytes,
+                                                 got.data_ptr(), status.data_ptr()))
+    assert torch.equal(got, want) and int(status.item()) == 0
+
+
 @pytest.mark.parametrize("rows,position", [(16, 0), (48, 90), (64, 0)])
 def test_short_drafter_runs_agree_with_decode(hip, rows, position):
     """As at the edges of row tiles, where a Q8_0 slice has two units of K and more."""
