@@ -25,7 +25,7 @@
 //   * Attention: a wave a query (four waves are one a SIMD: eight would share the issue slots), a token per 16 lanes with a
 //     running softmax of their own, merged over lanes by register swaps; a list's first 20 tokens lie in LDS before the phase.
 //
-//   * Rows depend on each other through keys and values alone.  A row writes its own past its L2, raises a flag for the block, and
+//   * Rows depend on each other through keys and values alone.  A row writes a copy of its own past its L2, raises a flag for the block, and
 //     the workgroups whose part of the list holds an earlier row's wait for that row's flag and take them over into LDS -- the last
 //     wave, which has no weights under way, while the others prepare the queries.  Every row is one hand-over behind the row before
 //     from the first block on, so the wait is short after that; and a row's operations are those of a pass by itself.
@@ -67,7 +67,7 @@ struct DArgs {
     uint32_t layers, rows, H, F;
     float eps, scale;
     uint8_t* exchange;                       // a row's hand-over buffers; offsets of its regions, all of them
-    uint32_t qkv_at, out_at, ml_at, o_at, d_at, h_at, exchange_bytes;
+    uint32_t qkv_at, out_at, ml_at, o_at, d_at, h_at, kv_at, exchange_bytes;
     uint32_t* sync;                          // cleared: a line with a counter for each row, then the rows' flags, block by block
     const float *x_in, *u_in;
     float *x_out, *u_out;                    // written after the last block; u_last, the receipt: the launch with the output norm alone
@@ -342,14 +342,15 @@ struct Pass {
 
     // ---- rows of the same launch: the last wave hands keys and values on, 16 bytes a lane, keys in the lower half of the wave ----
     using Words = uint32_t __attribute__((ext_vector_type(4)));
-    __device__ __forceinline__ uint16_t* private_rows(uint32_t l, uint32_t r) const {
-        return ((lane < 32 ? a.priv_k : a.priv_v) + (size_t(l) * a.rows + r) * kHd) + 8 * (lane & 31u);
+    // (a copy of its own per block: a row may be blocks ahead of its readers, and the caller's rows need not lie on 8 bytes)
+    __device__ __forceinline__ uint16_t* passed_on(uint32_t l, uint32_t r) const {
+        return reinterpret_cast<uint16_t*>(a.exchange + size_t(r) * a.exchange_bytes + a.kv_at) + (size_t(l) * 64 + lane) * 8;
     }
     __device__ __forceinline__ uint16_t* staged(uint32_t i) const { return (lane < 32 ? sh.kp_s[i] : sh.vp_s[i]) + 8 * (lane & 31u); }
     // this row's, for the XCDs of later rows: past this L2 (sc1), then the flag
     __device__ __forceinline__ void hand_on(uint32_t l, uint32_t i) const {
         const uint2* from = reinterpret_cast<const uint2*>(staged(i));
-        unsigned long long* to = reinterpret_cast<unsigned long long*>(private_rows(l, row));
+        unsigned long long* to = reinterpret_cast<unsigned long long*>(passed_on(l, row));
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const uint2 w = from[h];
@@ -372,7 +373,7 @@ struct Pass {
             unsigned long long w[4][2];
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {   // past the last one the last again, unused
-                const unsigned long long* p = reinterpret_cast<const unsigned long long*>(private_rows(l, t.priv_first + min(i0 + i, to - 1)));
+                const unsigned long long* p = reinterpret_cast<const unsigned long long*>(passed_on(l, t.priv_first + min(i0 + i, to - 1)));
                 w[i][0] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 w[i][1] = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -418,7 +419,6 @@ struct Pass {
         }
         if (prepares) {
             if (is_key) norm_rotate(v, gamma, rope, a.eps, lane);
-            const bool passed_on = row + 1 < a.rows;   // the last wave's to store
             bool bad = false;
             uint32_t bits[4];
 #pragma unroll
@@ -433,7 +433,7 @@ struct Pass {
             for (int k = 0; k < 4; ++k) {
                 const uint32_t d = (k >> 1) * 128 + 2 * lane + (k & 1);
                 to[d] = static_cast<uint16_t>(bits[k]);
-                if (!passed_on) out[d] = static_cast<uint16_t>(bits[k]);
+                out[d] = static_cast<uint16_t>(bits[k]);
             }
             if (bad) atomicOr(a.status, GUFFIN_STATUS_KV_NONFINITE);
         }
@@ -920,6 +920,7 @@ static uint32_t lay_out(const guffin_model_desc& m, DArgs& a) {
     a.o_at = take(kParts * m.hidden);
     a.d_at = take(kParts * m.hidden);
     a.h_at = take(m.ffn);
+    a.kv_at = take(std::min(m.layer_count, kLayers) * kHd);   // a key and a value a block, fp16
     return used;
 }
 uint64_t drafter_pass_bytes(const guffin_model_desc& m, uint32_t rows) {

@@ -109,6 +109,31 @@ def test_rows_of_a_run_equal_passes_of_one_row(hip, heads, hidden, ffn, layers, 
     assert torch.equal(both[0][0], first[0][0]) and torch.equal(both[2][:, 0], first[2][:, 0])
 
 
+@pytest.mark.parametrize("layers", [2, 26])
+@pytest.mark.parametrize("offset", [1, 2, 4])
+def test_private_rows_at_any_half(hip, layers, offset):
+    """Two rows side by side whose caller keeps its private rows `offset` halves behind an aligned address: the same bits."""
+    import ctypes as C
+    import torch
+    from guffin_amd import model
+    hip.set_forward_mode(0)
+    shape = replace(model.GEMMA3_270M, layers=layers, vocab=1024, ring_global=1024, hidden=64, ffn=256, global_period=2)
+    devm = model.DeviceModel.random(shape, seed=layers, position=40)
+    tokens = torch.tensor([17, 999], dtype=torch.int32, device="cuda")
+    want, _, pk, pv, status = devm.forward(tokens, 40)
+    words = pk.numel()
+    keys, values = (torch.zeros(words + 8, dtype=torch.float16, device="cuda") for _ in range(2))
+    nbytes = hip._calls.guffin_hip_forward_scratch_bytes(C.byref(devm.desc), 2, 40)
+    scratch, got = torch.empty(nbytes, dtype=torch.uint8, device="cuda"), torch.empty_like(want)
+    hip.check(hip._calls.guffin_hip_forward_rows(hip._raw_stream(), C.byref(devm.desc), tokens.data_ptr(), 2, 40, scratch.data_ptr(), nbytes,
+                                                 keys.data_ptr() + 2 * offset, values.data_ptr() + 2 * offset, got.data_ptr(), None, status.data_ptr()))
+    assert int(status.item()) == 0 and hip.lib().guffin_hip_resident_enabled() == 1
+    assert torch.equal(got, want)
+    for moved, own in ((keys, pk), (values, pv)):
+        assert torch.equal(moved[offset:offset + words].view(torch.int16), own.reshape(-1).view(torch.int16))
+        assert not moved[:offset].any() and not moved[offset + words:].any()
+
+
 def test_a_row_keeps_a_nan_and_says_so(hip):
     """A non-finite row in a ring's values reaches the hidden row and the status word, as in the per-operator pass: an operand
     group with a NaN has no fixed-point digits, its multiplier carries the NaN instead."""
