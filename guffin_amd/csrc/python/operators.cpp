@@ -36,7 +36,8 @@ constexpr Py_ssize_t kCount = sizeof(kNames) / sizeof(kNames[0]);
 static_assert(sizeof(Library) == kCount * sizeof(void*));
 Library g_lib;
 uint32_t g_candidates_bytes, g_law_bytes, g_result_bytes;
-PyObject* g_check;   // raises the library's error for a code
+PyObject* g_check;     // raises the library's error for a code
+PyObject* g_options;   // the class of a sampler's options
 
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
 at::TensorOptions on(const at::Device& device, at::ScalarType type) { return at::TensorOptions().dtype(type).device(device); }
@@ -58,15 +59,16 @@ bool wide(PyObject* o, uint64_t& to) {
     to = PyLong_AsUnsignedLongLongMask(o);
     return true;
 }
-// the bytes of a ctypes structure while it lives
-struct Bytes {
+// the bytes of a sampler's options (a ctypes structure; other objects with 20 bytes are not) while they live
+struct Options {
     Py_buffer view {};
     bool held = false;
-    explicit Bytes(PyObject* o) {
+    explicit Options(PyObject* o) {
+        if (reinterpret_cast<PyObject*>(Py_TYPE(o)) != g_options) return;
         held = PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) == 0;
         if (!held) PyErr_Clear();
     }
-    ~Bytes() { if (held) PyBuffer_Release(&view); }
+    ~Options() { if (held) PyBuffer_Release(&view); }
 };
 
 // the call without the interpreter's lock; false with an exception set where the library refuses it
@@ -90,7 +92,7 @@ bool done(Call call) {
 #define GUFFIN_LEAVE END_HANDLE_TH_ERRORS
 
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    if (n != kCount + 4) { PyErr_SetString(PyExc_TypeError, "bind: the entry points' addresses, three record sizes, the error function"); return nullptr; }
+    if (n != kCount + 5) { PyErr_SetString(PyExc_TypeError, "bind: the entry points' addresses, three record sizes, the error function, the options' class"); return nullptr; }
     void* at[kCount];
     for (Py_ssize_t i = 0; i < kCount; ++i) {
         at[i] = PyLong_AsVoidPtr(args[i]);
@@ -103,6 +105,8 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     std::memcpy(&g_lib, at, sizeof(g_lib));
     Py_INCREF(args[kCount + 3]);
     Py_XSETREF(g_check, args[kCount + 3]);
+    Py_INCREF(args[kCount + 4]);
+    Py_XSETREF(g_options, args[kCount + 4]);
     Py_RETURN_NONE;
 }
 
@@ -181,8 +185,8 @@ PyObject* draft_law(PyObject*, PyObject* const* args, Py_ssize_t n) {
     uint64_t seed, step;
     const at::Tensor* logits = n == 4 ? tensor(args[0]) : nullptr;
     if (!logits || !wide(args[2], seed) || !wide(args[3], step)) Py_RETURN_NONE;
-    const Bytes options(args[1]);
-    if (!options.held || options.view.len != 20) Py_RETURN_NONE;
+    const Options options(args[1]);
+    if (!options.held) Py_RETURN_NONE;
     const uint32_t vocab = static_cast<uint32_t>(logits->numel());
     const at::Device here(at::kCUDA);
     const at::Tensor ws = at::empty({static_cast<int64_t>(g_lib.draft_law_workspace_bytes(vocab))}, on(here, at::kByte));
@@ -202,8 +206,8 @@ PyObject* spec_accept(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 7 || !wide(args[4], seed) || !wide(args[5], step)) Py_RETURN_NONE;
     const at::Tensor *cands = tensor(args[0]), *law = tensor(args[1]), *proposal = tensor(args[2]), *status = args[6] == Py_None ? nullptr : tensor(args[6]);
     if (!cands || !law || !proposal || (args[6] != Py_None && !status)) Py_RETURN_NONE;
-    const Bytes options(args[3]);
-    if (!options.held || options.view.len != 20) Py_RETURN_NONE;
+    const Options options(args[3]);
+    if (!options.held) Py_RETURN_NONE;
     const at::Tensor result = at::empty({int64_t(g_result_bytes)}, on(at::Device(at::kCUDA), at::kByte));
     void *const s = stream(), *const r = result.data_ptr();
     auto* const st = status ? static_cast<uint32_t*>(status->data_ptr()) : nullptr;

@@ -83,7 +83,7 @@ class _Operators:
     def __getattr__(self, name):
         from . import _operators as native   # built beside the library; no fallback if it is missing
         native.bind(*(C.cast(getattr(lib(), "guffin_hip_" + e), C.c_void_p).value for e in self.ENTRY_POINTS),
-                    _candidates_bytes, _law_bytes, result_dtype.itemsize, check)
+                    _candidates_bytes, _law_bytes, result_dtype.itemsize, check, SamplerOptions)
         for f in ("group_sums", "gemv_packed", "repack", "select_candidates", "draft_law", "spec_accept"):
             setattr(self, f, getattr(native, f))
         return self.__dict__[name]

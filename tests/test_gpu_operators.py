@@ -73,3 +73,11 @@ def test_what_is_refused_stays_refused(hip):
     assert hip._ops.select_candidates(x, 2.0) is None
     with pytest.raises(AttributeError):
         hip.group_sums([1.0])
+    options = hip.SamplerOptions(1.0, 5, 0.95, 0.0, 1.0)
+    logits = torch.randn((2, 4096), device="cuda")
+    (cands, _), (law, proposal, _) = hip.select_candidates(logits, 5), hip.draft_law(logits[0], options)
+    for other in (bytes(options), bytearray(bytes(options)), np.frombuffer(bytes(options), np.uint8)):   # 20 bytes, no sampler's options
+        with pytest.raises(TypeError):
+            hip.draft_law(logits[0], other)
+        with pytest.raises(TypeError):
+            hip.spec_accept(cands, law, proposal, other)
