@@ -4,7 +4,9 @@ the HSA runtime and writes their dispatch packets itself."""
 import concurrent.futures
 import glob
 import os
+import shutil
 import subprocess
+import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -82,10 +84,18 @@ def kernarg_rows(code_object):
 
 
 def _operators():
-    """The native forms of the small operators for Python: host code against torch's headers, bound to the library at run time."""
+    """The native forms of the small operators for Python: host code against torch's headers, bound to the library at run time.  Without
+    torch or g++ there is nothing to build them for or with: the library stands by itself, and guffin_amd.hip says that they are missing."""
     import sysconfig
 
-    import torch
+    if os.path.exists(OPERATORS):
+        os.remove(OPERATORS)   # of another build
+    try:
+        import torch
+    except ImportError:
+        return "no torch: the operators for Python are not built"
+    if shutil.which("g++") is None:
+        return "no g++: the operators for Python are not built"
     base = os.path.dirname(torch.__file__)
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
@@ -96,10 +106,20 @@ def _operators():
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed for operators.cpp:\n" + r.stderr)
-    return r.stderr
+    return None
 
 
 def build(verbose=False):
+    with concurrent.futures.ThreadPoolExecutor(max_workers=1) as beside:
+        operators = beside.submit(_operators)
+        library = _library(verbose)
+        missing = operators.result()
+    if missing:
+        print(missing, file=sys.stderr)
+    return library
+
+
+def _library(verbose):
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(HSACO, exist_ok=True)
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "*.cpp")))  # .cpp: host only
@@ -107,9 +127,7 @@ def build(verbose=False):
     with concurrent.futures.ThreadPoolExecutor(max_workers=8) as pool:
         objects = pool.map(_compile, sources)
         code_objects = pool.map(_code_object, device_sources)
-        operators = pool.submit(_operators)
         results = list(objects)
-        operators.result()
         code_objects = list(code_objects)
     objs = [o for o, _ in results]
     if verbose:
