@@ -967,13 +967,22 @@ prefill_gateup_q8_kernel(const uint8_t* __restrict__ gate, const uint8_t* __rest
     }
 }
 
-// How many ways the XCDs cut the row chunks of a launch between them, the column groups being dealt over the others; 0: the grid's
-// own order.  Consecutive workgroups go to different XCDs, so where the rows run fastest the workgroups that share weights sit in
-// different L2s: all of them fetch all weights.  Good where a whole image does not fit an L2 and each keeps its share of it;
-// with few chunks the weights are what is worth keeping.  A pass of the 12B shapes, us, grid's order / one way / two ways: 160 rows 12207 / 11861 /
-// 13439, 333 21035 / 20486 / 20563, 448 25888 / 25270 / 24869, 640 34744 / 35441 / 33996, 704 38435 / 40628 / 39683, 2048 100656 / 104727 /
-// 102185.  The drafter's weights are small beside its image: 333 rows 1302 / 1417 / 1375.
-uint32_t row_ways(uint32_t chunks, bool q8) { return q8 || chunks < 2 || chunks > 10 ? 0 : chunks <= 6 ? 1 : 2; }
+// How many ways the XCDs cut the row chunks of a launch between them, the column groups of all slices (`units`) being dealt over the others;
+// 0: the grid's own order.  Consecutive workgroups go to different XCDs, so where the rows run fastest the workgroups that share weights sit in
+// different L2s and each fetches them, while an L2 keeps its share of the image; dealt, the workgroups of a unit share an L2 and the
+// weights are fetched once (one way) or twice.  The lines are by the number of chunks alone: as many XCDs fetch a weight as there are chunks, up to
+// eight.  Passes of the 12B shapes, us, grid's order / one way / two ways: 160 rows 12207 / 11861 / 13439, 333 21035 / 20486 / 20563, 448 25888 /
+// 25270 / 24869, 640 34744 / 35441 / 33996, 704 38435 / 40628 / 39683, 2048 100656 / 104727 / 102185.  Single launches of other widths, 288 / 448 /
+// 640 / 1024 rows, grid's order / so: K = 2048, N = 16384 Q4_K 49.4 / 46.2, 62.7 / 60.3, 91.2 / 88.6, the same; K = 8192, N = 2048 Q6_K 37.1 / 34.6, 47.2
+// / 42.7, the same, the same; K = 5120, N = 27648 182.9 / 173.8, 241.8 / 256.6 (seven chunks by fours leave XCDs uneven), 358.5 / 344.6, the same.
+// Not where the uneven shares take an XCD one more turn of two workgroups a compute unit: 288 rows of K = 13824, N = 5120, five chunks, 65
+// workgroups instead of 63, 93.9 / 119.2.  The drafter's weights are small beside its image: 333 rows 1302 / 1417 / 1375.
+uint32_t row_ways(uint32_t chunks, uint32_t units, bool q8) {
+    if (q8 || chunks < 2 || chunks > 10) return 0;
+    const uint32_t ways = chunks <= 6 ? 1 : 2, others = 8 / ways, turn = std::max(1u, 2 * compute_units() / 8);
+    const uint32_t dealt = (chunks + ways - 1) / ways * ((units + others - 1) / others), even = (chunks * units + 7) / 8;
+    return (dealt + turn - 1) / turn > (even + turn - 1) / turn ? 0 : ways;
+}
 
 constexpr uint32_t kept_bytes(uint32_t R) { return 4 * R * kKeptStride * sizeof(float4_t); }
 int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M, uint32_t K,
@@ -992,8 +1001,9 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
     if (halves && (kinds != 1 || 2 * slices > K / 256)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: a slice in halves is two blocks of Q4_K at least");
     const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
     dim3 grid(chunks, groups, slices), block(256);
-    if (const uint32_t ways = row_ways(chunks, kinds == 4u)) {
-        const uint32_t units = groups * slices, others = 8 / ways;
+    const uint32_t units = groups * slices;
+    if (const uint32_t ways = row_ways(chunks, units, kinds == 4u)) {
+        const uint32_t others = 8 / ways;
         a.form |= (ways == 1 ? 1u : 2u) << kSliceBits;
         grid = dim3(8 * ((chunks + ways - 1) / ways) * ((units + others - 1) / others));
     }
