@@ -42,11 +42,12 @@ def split(name, rows):
     return f(m, len(m), rows, K)
 
 
-def planes(dtype, tiles, image, M, K, N, cut):
-    """The product's planes, cut so, on the current stream."""
+def planes(parts, image, M, K, cut):
+    """The planes of each of `parts` ((format, tiles, N), one launch), cut so, on the current stream."""
     import torch
     f = hip.lib()._ZN6guffin19prefill_gemm_planesEP12ihipStream_tPKNS_13PrefillMatrixEjPKhPKPfjjNS_12PrefillSplitE
     f.argtypes, f.restype = [C.c_void_p, C.POINTER(Matrix), C.c_uint32, C.c_void_p, C.POINTER(C.c_void_p), C.c_uint32, C.c_uint32, Split], C.c_int
-    y = torch.full((cut.slices, M, N), float("nan"), device="cuda")
-    hip.check(f(hip._raw_stream(), C.byref(Matrix(dtype, tiles.data_ptr(), N)), 1, image.data_ptr(), (C.c_void_p * 1)(y.data_ptr()), M, K, cut))
+    y = [torch.full((cut.slices, M, N), float("nan"), device="cuda") for _, _, N in parts]
+    m = (Matrix * len(parts))(*[Matrix(dtype, tiles.data_ptr(), N) for dtype, tiles, N in parts])
+    hip.check(f(hip._raw_stream(), m, len(m), image.data_ptr(), (C.c_void_p * len(y))(*[p.data_ptr() for p in y]), M, K, cut))
     return y

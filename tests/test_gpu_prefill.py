@@ -96,8 +96,8 @@ def test_a_slice_in_halves_is_the_sum_of_two_slices(hip, M, row_tiles, K, slices
     gen.manual_seed(M + K)
     tiles = hip.repack(1, dev(synth.make_weight(1, K, N, seed=K + slices)), K, N)
     image = hip.prefill_pack(torch.randn((M, K), device="cuda", generator=gen))
-    whole = planes(1, tiles, image, M, K, N, Split(row_tiles, slices, 1))
-    parts = planes(1, tiles, image, M, K, N, Split(row_tiles, 2 * slices, 0))
+    whole, = planes([(1, tiles, N)], image, M, K, Split(row_tiles, slices, 1))
+    parts, = planes([(1, tiles, N)], image, M, K, Split(row_tiles, 2 * slices, 0))
     assert torch.equal(whole, parts[0::2] + parts[1::2])
 
 
@@ -118,7 +118,7 @@ def test_a_short_run_s_sums_are_as_close_as_in_the_long_runs_slices(hip, name, r
     tiles, image = hip.repack(dtype, w, K, N), hip.prefill_pack(x)
     errors = []
     for cut in (split(name, rows), Split(1, bar(name, rows), 0)):
-        y = planes(dtype, tiles, image, rows, K, N, cut)
+        y, = planes([(dtype, tiles, N)], image, rows, K, cut)
         total = y[0]
         for plane in y[1:]:
             total = total + plane
@@ -129,9 +129,10 @@ def test_a_short_run_s_sums_are_as_close_as_in_the_long_runs_slices(hip, name, r
 @pytest.mark.parametrize("dtype,N", [(1, 64), (1, 64 * 33), (2, 64 * 5), (2, 64 * 36)])
 @pytest.mark.parametrize("M", [65, 97, 385, 449, 577, 640, 641, 705])
 def test_prefill_gemm_wherever_its_workgroups_go(hip, dtype, N, M):
-    """Row chunks dealt to the XCDs in two, one and (one chunk more than that takes) the grid's order, with fewer column groups than
-    XCDs and numbers of them that eight does not divide: every element, against 64 bits.  The rms error of such sums is 1.6e-7
-    (Q4_K) and 2.3e-7 (Q6_K) of the result's; a workgroup that worked on another's place, or on none, is off by the result itself."""
+    """A product by itself, which is cut into chunks of one row tile mostly (two from 640 rows on of the wider ones): dealt to the XCDs at 65
+    and 97 rows, the grid's order beyond, with fewer column groups than XCDs and numbers of them that eight does not divide: every
+    element, against 64 bits.  The rms error of such sums is 1.6e-7 (Q4_K) and 2.3e-7 (Q6_K) of the result's; a workgroup that worked on
+    another's place, or on none, is off by the result itself."""
     import torch
     K = 512
     gen = torch.Generator(device="cuda")
@@ -142,6 +143,54 @@ def test_prefill_gemm_wherever_its_workgroups_go(hip, dtype, N, M):
     y = hip.prefill_gemm(dtype, hip.repack(dtype, w, K, N), hip.prefill_pack(x), M, K, N).double()
     assert float(((y - want).pow(2).mean() / want.pow(2).mean()).sqrt()) <= 4e-7
     assert float((y - want).abs().max() / want.pow(2).mean().sqrt()) <= 1e-5
+
+
+@pytest.mark.parametrize("columns", [((1, 64),), ((2, 64 * 33),), ((1, 64 * 16), (1, 64 * 5), (2, 64 * 9))])
+@pytest.mark.parametrize("slices", [1, 3, 5])
+@pytest.mark.parametrize("row_tiles", [1, 2, 3, 4])
+@pytest.mark.parametrize("chunks", [1, 2, 5, 6, 7, 8, 10, 11])
+def test_prefill_gemm_dealt_to_the_xcds(hip, chunks, row_tiles, slices, columns):
+    """Row chunks in the grid's order (one; eleven), dealt to the XCDs one way (two to six) and two ways (seven to ten), the last one ragged,
+    with each number of row tiles, column groups and slices that eight does or does not divide, one matrix and three formats' launches:
+    every element, against 64 bits, and no place that nobody worked on (the planes hold NaN before).  The rms error of such sums is
+    1.6e-7 (Q4_K) and 2.3e-7 (Q6_K) of the result's; a workgroup on another's place is off by the result itself."""
+    import torch
+    from prefill_cuts import Split, planes
+    K, M = 256 * 5, 16 * row_tiles * chunks - 3
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M)
+    x = torch.randn((M, K), device="cuda", generator=gen)
+    weights = [dev(synth.make_weight(dtype, K, N, seed=9 + i)) for i, (dtype, N) in enumerate(columns)]
+    parts = [(dtype, hip.repack(dtype, w, K, N), N) for w, (dtype, N) in zip(weights, columns)]
+    for w, (dtype, N), y in zip(weights, columns, planes(parts, hip.prefill_pack(x), M, K, Split(row_tiles, slices, 0))):
+        want = x.double() @ hip.dequant(dtype, w, N * K // 256).view(N, K).double().T.contiguous()
+        got = y.double().sum(0)
+        assert float(((got - want).pow(2).mean() / want.pow(2).mean()).sqrt()) <= 4e-7
+        assert float((got - want).abs().max() / want.pow(2).mean().sqrt()) <= 1e-5
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("rows", [257, 333, 448, 512, 577, 640])
+def test_dealt_runs_agree_with_shorter_ones(hip, rows, mixed):
+    """A block of the 12B shapes at runs whose launches are dealt to the XCDs in every way (looked at first), against the same tokens as
+    runs of at most 16 rows, which are not.  The bar is that of runs against decoding."""
+    import random
+    from dataclasses import replace
+    import torch
+    from guffin_amd import model
+    from prefill_cuts import split
+    seen = {-(-rows // (16 * split(name, rows).row_tiles)) for name in (("qkv4", "o", "gate_up", "down4") if mixed else ("qkv", "o", "gate_up", "down"))}
+    assert any(2 <= chunks <= 10 for chunks in seen), seen
+    shape = replace(model.GEMMA3_12B, layers=1, vocab=1024, ring_global=1024, ring_local=1024, sliding_window=256)
+    if mixed:
+        shape = replace(shape, layer_dtypes=((synth.Q4_K,) * 7,))
+    tokens = torch.tensor([random.Random(i).randrange(2, 1024) for i in range(rows)], dtype=torch.int32, device="cuda")
+    whole, cut = (model.DeviceModel.random(shape, seed=7, position=0) for _ in range(2))
+    hidden_rows, status = whole.prefill(tokens, 0)
+    want = torch.cat([cut.prefill(tokens[at:at + 16].contiguous(), at)[0] for at in range(0, rows, 16)]).double()
+    assert int(status.item()) == 0
+    scale = want.pow(2).mean(1, keepdim=True).sqrt()
+    assert float(((hidden_rows.double() - want).abs() / scale).max()) <= 2e-4
 
 
 def test_prefill_gemm_down_projection_shape(hip, gfo):
