@@ -1,4 +1,4 @@
-"""The drafter's pass on one XCD (drafter_pass.hip) at the edges of what it covers, against the launch-per-operator pass on the
+"""The drafter's pass, a row an XCD (drafter_pass.hip), at the edges of what it covers, against the launch-per-operator pass on the
 same model and rows and against the CPU oracle: head groupings (how many waves share a query), widths where workers have no
 blocks or the column tiles leave workgroups idle, token lists of one chunk of 20 a workgroup, of just more and of several,
 windows that begin inside a ring, more blocks than a launch takes.
@@ -81,10 +81,13 @@ RUNS = [(4, 640, 2048, 2, 512, 0, (8, 8, 8)), (4, 640, 2048, 2, 512, 505, (8, 3,
 @pytest.mark.parametrize("heads,hidden,ffn,layers,window,start,runs", RUNS)
 def test_rows_of_a_run_equal_passes_of_one_row(hip, heads, hidden, ffn, layers, window, start, runs):
     """Each row is summed as by itself: hidden rows, K/V rows and logits to the last bit, also behind a window and for rows whose
-    neighbours lie in several workgroups' parts of the list."""
+    neighbours lie in several workgroups' parts of the list.  A wait that gave up would switch both sides to one launch per operator, which
+    are equal too: it is looked at."""
     import random
     import torch
     from guffin_amd import model
+    hip.set_forward_mode(0)
+    side_by_side = hip.lib().guffin_hip_resident_enabled
     shape = replace(model.GEMMA3_270M, layers=layers, vocab=1024, ring_global=2048, q_heads=heads, hidden=hidden, ffn=ffn, global_period=2,
                     sliding_window=window)
     devs = [model.DeviceModel.random(shape, seed=layers + heads, position=0) for _ in range(2)]
@@ -97,6 +100,7 @@ def test_rows_of_a_run_equal_passes_of_one_row(hip, heads, hidden, ffn, layers, 
             plan.append(tokens[:start])
     for n in runs:
         plans[0].append(tokens[at:at + n])
+        assert side_by_side() == 1
         for t in tokens[at:at + n]:
             plans[1].append([t])
         at += n
@@ -107,6 +111,7 @@ def test_rows_of_a_run_equal_passes_of_one_row(hip, heads, hidden, ffn, layers, 
     both = devs[0].forward(pair, at)
     first = devs[0].forward(pair[:1].contiguous(), at)
     assert torch.equal(both[0][0], first[0][0]) and torch.equal(both[2][:, 0], first[2][:, 0])
+    assert int(both[4].item()) == 0 and int(first[4].item()) == 0 and side_by_side() == 1
 
 
 @pytest.mark.parametrize("layers", [2, 26])

@@ -470,6 +470,34 @@ def test_prefill_attention_where_a_workgroup_takes_both_parts(hip, q_heads, kv_h
     assert float((got.double() - want).abs().max()) <= 2e-6 * max(1.0, float(want.abs().max()))
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,rows,position,window,cap", [(4, 1, 690, 5, 512, 512), (16, 8, 172, 100, 64, 128), (16, 8, 37, 300, 0, 512)])
+def test_prefill_attention_keeps_a_nan_where_it_is(hip, q_heads, kv_heads, rows, position, window, cap):
+    """A query with a NaN: its own output alone, whatever wave or part of the list it goes through.  A key with one: the rows that see it, of its
+    head's group; all other outputs to the last bit what they are without.  (Two parts as one workgroup, and parts merged by a launch.)"""
+    import torch
+    hd, group = 256, q_heads // kv_heads
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows)
+    rand = lambda *shape: torch.randn(shape, device="cuda", generator=gen)
+    q = rand(rows, q_heads * hd)
+    ring_k, ring_v = rand(cap, kv_heads * hd).half(), rand(cap, kv_heads * hd).half()
+    run_k, run_v = rand(rows, kv_heads * hd).half(), rand(rows, kv_heads * hd).half()
+    attend = lambda q, k: hip.prefill_attention(q, ring_k, ring_v, k, run_v, position, window, cap - 1, q_heads, kv_heads, hd, 0.0625,
+                                                matrix_core=True).view(rows, q_heads, hd)
+    clean = attend(q, run_k)
+    row, head = rows // 2 + 1, q_heads - 1
+    bad = q.clone()
+    bad[row, head * hd + 7] = float("nan")
+    got, hit = attend(bad, run_k), torch.zeros((rows, q_heads), dtype=torch.bool, device="cuda")
+    hit[row, head] = True
+    assert bool(got[hit].isnan().all()) and torch.equal(got[~hit], clean[~hit])
+    keys = run_k.clone()
+    keys[row, (kv_heads - 1) * hd + 200] = float("nan")
+    got, hit = attend(q, keys), torch.zeros((rows, q_heads), dtype=torch.bool, device="cuda")
+    hit[row:row + window if window else rows, -group:] = True
+    assert bool(got[hit].isnan().all()) and torch.equal(got[~hit], clean[~hit])
+
+
 def test_prefill_attention_takes_queries_up_to_the_range_of_a_half(hip):
     """A query element of 60 000 after the scale (a half holds 65 504) against keys small enough for ordinary scores."""
     import torch
@@ -647,6 +675,38 @@ def test_a_run_s_gated_product_is_that_of_shorter_runs(hip, hidden, ffn, rows):
     want = torch.cat(parts).double()
     scale = want.pow(2).mean(1, keepdim=True).sqrt()
     assert float(((hidden_rows.double() - want).abs() / scale).max()) <= 1e-4
+
+
+@pytest.mark.parametrize("rows,bad", [(512, 488), (1025, 1000), (2047, 1992)])
+def test_a_row_that_is_no_number_in_the_gated_product(hip, rows, bad):
+    """A token whose embedding holds an infinity, late in a run that takes gate, up and GeGLU as one launch: the rows before it, eight of them in its
+    row tile, are the clean run's to the last bit, it and the rows that attend it hold no number and the status word says so, as in
+    runs of 96 rows.  (At position 24 its key starts a tile of 32, which the rows before it do not visit.)"""
+    import random
+    from dataclasses import replace
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=1, vocab=1024, ring_global=8192, ring_local=8192, sliding_window=512)
+    tokens = torch.tensor([random.Random(i).randrange(2, 1000) for i in range(24 + rows)], dtype=torch.int32, device="cuda")
+    first, tokens = tokens[:24].contiguous(), tokens[24:].contiguous()
+    devs = [model.DeviceModel.random(shape, seed=3, position=0) for _ in range(2)]
+    for d in devs:
+        d.prefill(first, 0)
+    clean, status = devs[0].prefill(tokens, 24)
+    assert int(status.item()) == 0 and bad % 16 == 8 and (24 + bad) % 32 == 0
+    for d in devs:
+        embed = next(t for t in d.keep if torch.is_tensor(t) and t.data_ptr() == d.desc.embed_rows)
+        at = 1001 * (shape.hidden // 32 * 34)
+        embed.view(-1).view(torch.uint8)[at:at + 2] = torch.tensor([0x00, 0x7C], dtype=torch.uint8, device="cuda")
+    tokens[bad] = 1001
+    whole, raised = devs[0].prefill(tokens, 24)
+    words = 0
+    for at in range(0, rows, 96):
+        part, word = devs[1].prefill(tokens[at:at + 96].contiguous(), 24 + at)
+        words |= int(word.item())
+        assert torch.equal(part.isfinite(), whole[at:at + 96].isfinite()), at
+    assert torch.equal(whole[:bad], clean[:bad]) and not bool(whole[bad:].isfinite().any())
+    assert int(raised.item()) == words != 0
 
 
 @pytest.mark.parametrize("position", [0, 20, 95, 125, 200])
