@@ -23,9 +23,9 @@
 // chunk goes from memory to LDS without passing registers, two chunks ahead in three rotating buffers, one barrier per
 // chunk; weights are private to a wave and requested half a block ahead.
 //
-// What bounds it: the instructions that form B.  A loop of one matrix and V vector instructions takes, with two waves a SIMD,
-// 10 + 4.3 V cycles for V >= 2 (17 for the matrix instruction alone, 22.9 with three beside it), in whatever order they stand; a
-// block of four row tiles is 272 (Q6_K 384) of the one and 780 (920) of the other and takes 6900 of the 6100 cycles that makes.  So
+// What bounds it: the instructions that form B.  A loop of one matrix and V packed vector instructions (sixteen independent chains of the one, eight
+// of the other, two waves a SIMD) takes 8.9, 10.2, 10.6, 12.2 and 13.6 ns of a SIMD for V = 0 to 4, 1.4 more for each further one; a
+// block of four row tiles is 272 (Q6_K 384) of the one and 780 (920) of the other, 3.2 (4.3) us by that, and takes 3.7 (4.9) at 2048 rows.  So
 // scales are widened for two column groups at once, Q6_K's quants put together as bytes, operands change places instead of being
 // copied, and addresses are immediates.  us before / after: 2048 rows gate + up 855 / 839, down (Q6_K) 571 / 552, q/k/v 250 / 243, o 121 /
 // 119; 333 rows 180 / 174, 129 / 119, 64.7 / 61.0, 29.1 / 28.4; 37 rows 31.9 / 30.7, 26.9 / 25.1, 14.8 / 13.9, 10.2 / 9.8.

@@ -598,7 +598,8 @@ int guffin_hip_h1_full_cdf(const guffin_h1_desc* desc, void* scratch, uint64_t**
  * proposals drafted at a frontier that a truncate or a shorter commit went back to.  transaction_rows is the
  * reference's constructor argument of that name (:648-657): how many positions one transaction may write, at
  * least the largest horizon + 2 = 25 and, rounded up to a power of two, at most the smallest ring; 0 = 32.
- * Tokens run through the decode path one row per pass, so a token's rows and logits do not
+ * Tokens run through the decode path, up to eight of them side by side in the drafter's own pass (each row summed as by itself), one
+ * row per pass for any other model; so a token's rows and logits do not
  * depend on how appends were grouped and a commit equals a replay bit for bit.  Every call returns when its device work is done; errors: GUFFIN_E_STATE for a call
  * the state does not admit (nested transaction, truncation of published rows, a second pending token, a
  * poisoned plan), GUFFIN_E_CAPACITY / GUFFIN_E_ARG raised before any state changes, GUFFIN_E_NUMERIC when a pass
