@@ -2,26 +2,33 @@
 // eight contiguous rows side by side: a row on the 32 CUs of an XCD each.
 //
 // Operator order per block: the drafter's forward (src/engine/gemma3_draft.mm:888-972).  The placement and the bounded waits are
-// those of resident.hip; as there, workgroups hand over through the XCD's L2: plain stores, a counter, reads past the L1.
+// those of resident.hip; as there, workgroups hand over through the XCD's L2: plain stores, reads past the L1.
 //
-// What bounds it: a chain of 18 x 5 phases, each a hand-over (1.05 us: a 256-byte store, its acknowledgement, arrival, poll) and
-// one to two microseconds of dependent steps; the weights alone (5.9 MB a block at the 1.3 TB/s that one XCD takes) would be 4.5
-// us a block.  So the design is about what lies between two hand-overs:
+// What bounds it: a chain of 18 x 5 phases, each a hand-over and one to two microseconds of dependent steps; the weights alone (5.9 MB
+// a block at the 1.3 TB/s that one XCD takes) would be 4.5 us of a block's 11.6.  So the design is about the hand-overs and what lies
+// between them:
 //
-//   * A wave works from its operand to its partial sums by itself.  It owns three blocks of the hidden width: it sums their
-//     planes, keeps their residual in registers and forms their operand (a norm pair needs the others for its two sums only, a
-//     meeting each); it merges just the attention outputs that its own two o-projection blocks want and loads just the GeGLU
-//     values of its own down blocks.
+//   * The words themselves are the message.  Every word of a set of exchange buffers is marked empty (kEmpty) by the workgroup that
+//     will write it; a reader looks at what it wants until nothing of it is empty.  So a hand-over is a store on its way and the trip
+//     of a look, instead of a store, its acknowledgement, an arrival at a counter, a look at that and then the trip for the words (1.05
+//     us and the trip).  Two sets by turns; when a set's words may be marked anew stands at publisher().
+//   * A wave works from its operand to its partial sums by itself.  It owns three blocks of the hidden width and forms their operand; it
+//     merges just the attention outputs that its own two o-projection blocks want and loads just the GeGLU values of its own down
+//     blocks.
+//   * The last wave takes a row's planes, has the residual in registers and makes both norms of a pair without a meeting: 10 quads'
+//     sums and two chains over its lanes.  (Shared by the workers, a meeting each: 0.2 us a pair more.)
 //   * Products are exact integers: the quants are int8 as they lie in the tile, an activation is four int8 digits of a 31-bit
 //     fixed-point number per group of 32, and v_mfma_i32_4x4x4_16b_i8 multiplies a column's four weights with the four digits
 //     of four elements: eight instructions a block, nothing to unpack, no bias to take off again, sums without rounding.  (The
 //     fp16 form of the other kernels: some 60 vector instructions a block, 22 bits of an activation.)
 //   * A wave's weights of a whole block of the model (15 tiles) have registers of their own and are asked for most of a block
-//     ahead, a few tiles behind each phase's own operands and never during a hand-over (which then takes 1.9 us).
+//     ahead, a few tiles behind each phase's own operands: spread evenly, as one XCD takes the 15 in half a block's time, and never
+//     right ahead of a wave's own look, which returns behind them.  (Seven of them between the down projection's look and the next
+//     q/k/v: 235 us a pass instead of 226.)
 //   * Weights are read through the caches' ordinary policy: non-temporal requests take 1200 cycles instead of 700 to come back
 //     (2176-byte tiles, one XCD), which is 47 us of a pass.
-//   * The eighth wave has no weights.  It adds the workers' partial sums, stores them, waits for that store alone, arrives
-//     and polls; so nobody's wait for a store or for the counter includes a weight request.
+//   * The eighth wave has no weights.  It adds the workers' partial sums and stores them; so its looks at the planes do not wait
+//     behind a weight request.
 //   * Attention: a wave a query (four waves are one a SIMD: eight would share the issue slots), a token per 16 lanes with a
 //     running softmax of their own, merged over lanes by register swaps; a list's first 20 tokens lie in LDS before the phase.
 //
@@ -30,9 +37,9 @@
 //     wave, which has no weights under way, while the others prepare the queries.  Every row is one hand-over behind the row before
 //     from the first block on, so the wait is short after that; and a row's operations are those of a pass by itself.
 //
-// 270M-shaped model, whole pass at position 150 / 4096: one row 299 / 351 us, two rows 316 / 368 (in one XCD, sharing the weights: 402 / 471),
-// eight rows 361 at 150.  (resident_blocks_kernel, three launches: one row 606 / 652, two 777 / 888; one launch per operator: 559 / 581 and 609 / 653.)
-// rms error of the hidden row against 64 bits, one block, where no K/V rounding falls the other way: 5.3-8e-8.
+// 270M-shaped model, whole pass at position 150 / 4096: one row 226 / 279 us (288 / 342 with acknowledged stores, a counter and norms shared by
+// the workers).  (resident_blocks_kernel, three launches: one row 606 / 652, two 777 / 888; one launch per operator: 559 / 581 and 609 / 653.)
+// rms error of the hidden row against 64 bits, one block, where no K/V rounding falls the other way: 6.2e-8 (6.5e-8 before).
 #include "common.hpp"
 #include "receipt.hpp"
 #include "resident.hpp"
@@ -52,6 +59,9 @@ constexpr int kOwn = 3, kOwnO = 2, kOwnDown = 4;          // blocks per worker: 
 constexpr uint32_t kTile = 64 * 34;       // a wave tile of one Q8_0 block (gemv_packed.hip has the layout)
 constexpr uint32_t kChunk = 20;           // tokens whose keys and values lie in LDS (a window of 512: 17 a workgroup)
 
+constexpr uint32_t kMl = 32;              // words between two workgroups' maxima and sums: a cache line each
+constexpr uint32_t kEmpty = 0xFFFFFFFFu;  // a word that nobody has handed over yet
+
 constexpr uint32_t kLine = 64;            // words between the counters of two rows
 constexpr uint32_t kLayers = 24;          // blocks per launch (their pointers travel as kernel arguments)
 constexpr uint32_t kFlagsAt = kRunRows * kLine, kSyncWords = kFlagsAt + kLayers * kRunRows;
@@ -66,8 +76,8 @@ struct DArgs {
     DLayer layer[kLayers];
     uint32_t layers, rows, H, F;
     float eps, scale;
-    uint8_t* exchange;                       // a row's hand-over buffers; offsets of its regions, all of them
-    uint32_t qkv_at, out_at, ml_at, o_at, d_at, h_at, kv_at, exchange_bytes;
+    uint8_t* exchange;                       // a row's hand-over buffers, two sets by turns; a set's regions, all of them
+    uint32_t qkv_at, out_at, ml_at, o_at, d_at, h_at, set_bytes, kv_at, exchange_bytes;
     uint32_t* sync;                          // cleared: a line with a counter for each row, then the rows' flags, block by block
     const float *x_in, *u_in;
     float *x_out, *u_out;                    // written after the last block; u_last, the receipt: the launch with the output norm alone
@@ -88,8 +98,8 @@ typedef int i4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 struct Shared {
-    float red[kWorkers][2][64];                    // the workers' column sums (gate and up)
-    float sums[2][kWaves];                         // their parts of the row's two sums of squares
+    float red[kWorkers][3][64];                    // the workers' column sums: q/k/v, o and gate, up, down
+    float u[kMaxWidth];                            // the normalised row that the next operand is made of
     float2 rope[2][kHd / 2];                       // local, global
     uint32_t opnd[kWorkers][128];                  // a worker's operand: an element's four digits a word
     float mult[kWorkers][4];
@@ -291,7 +301,7 @@ struct Pass {
     Shared& sh;
     uint32_t lane;
     const uint32_t wave, slot, row;
-    uint32_t generation = 0;
+    const float per_width;
     __amdgpu_buffer_rsrc_t exchange;
 
     // What another workgroup stored during this launch: past this CU's L1 (sc1), which nothing invalidates, from the L2.
@@ -302,15 +312,38 @@ struct Pass {
     __device__ __forceinline__ float2 ld2(uint32_t at, uint32_t floats) const {
         return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(exchange, static_cast<int>(4 * floats), static_cast<int>(at), kPast));
     }
-    __device__ __forceinline__ void st(uint32_t at, uint32_t floats, float v) const {
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
+    // (a NaN of every bit, which a weight could bring, goes as the usual one: the others would wait for it)
+    static __device__ __forceinline__ uint32_t sealed(float v) {
+        const uint32_t bits = __float_as_uint(v);
+        return bits == kEmpty ? 0x7FC00000u : bits;
     }
+    __device__ __forceinline__ void st_bits(uint32_t at, uint32_t floats, uint32_t v) const {
+        __builtin_amdgcn_raw_buffer_store_b32(v, exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
+    }
+    __device__ __forceinline__ void st(uint32_t at, uint32_t floats, float v) const { st_bits(at, floats, sealed(v)); }
     __device__ __forceinline__ void st2(uint32_t at, uint32_t floats, float2 v) const {
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2_t, v), exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
+        __builtin_amdgcn_raw_buffer_store_b64(u2_t{sealed(v.x), sealed(v.y)}, exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
+    }
+    __device__ __forceinline__ void st4_bits(uint32_t at, uint32_t floats, u4_t v) const {
+        __builtin_amdgcn_raw_buffer_store_b128(v, exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
     }
     __device__ __forceinline__ void st4(uint32_t at, uint32_t floats, f4_t v) const {
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, v), exchange, static_cast<int>(4 * floats), static_cast<int>(at), 0);
+        st4_bits(at, floats, u4_t{sealed(v.x), sealed(v.y), sealed(v.z), sealed(v.w)});
     }
+    // whether a word of these is still to come, for any lane
+    static __device__ __forceinline__ bool empty(float2 v) { return __any(max(__float_as_uint(v.x), __float_as_uint(v.y)) == kEmpty); }
+    static __device__ __forceinline__ bool empty(f4_t v) {
+        return __any(max(max(__float_as_uint(v.x), __float_as_uint(v.y)), max(__float_as_uint(v.z), __float_as_uint(v.w))) == kEmpty);
+    }
+    // after a look that found something missing: whether to look again
+    __device__ __forceinline__ bool again(uint32_t& looks) const {
+        asm volatile("" ::: "memory");
+        if (sh.dead) return false;
+        if (++looks <= a.spin_limit) return true;
+        if (lane == 0) give_up();
+        return false;
+    }
+    __device__ __forceinline__ uint32_t set_of(uint32_t l) const { return (l & 1u) * a.set_bytes; }
 
     __device__ __forceinline__ void enter() { lane = opaque(lane); }   // or every address that depends on the lane alone is kept in a register over the loop
     __device__ __forceinline__ void stamp(uint32_t l, uint32_t phase) const {
@@ -318,17 +351,15 @@ struct Pass {
     }
 
     __device__ __forceinline__ void give_up() const { sh.dead = 1u; atomicOr(a.status, GUFFIN_STATUS_SYNC); }
-    // The last wave: its stores are in the L2, then the arrival, then the wait for the other workgroups.  A wait that gives up
-    // raises the status bit, and the workgroup waits no more for the rest of the launch.
-    __device__ __forceinline__ void arrive_and_wait() {
+    // The last wave, once a launch: its stores (both sets marked empty) are in the L2, then the arrival, then the wait for the other
+    // workgroups.  A wait that gives up raises the status bit, and the workgroup waits no more for the rest of the launch.
+    __device__ __forceinline__ void arrive_and_wait() const {
         __builtin_amdgcn_s_waitcnt(0);
-        generation += 1;
         if (lane == 0 && !sh.dead) {
             uint32_t* counter = a.sync + row * kLine;
             __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            const uint32_t target = kGroups * generation;
             uint32_t spins = 0;
-            while (__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)
+            while (__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kGroups)
                 if (++spins > a.spin_limit) { give_up(); break; }
         }
         asm volatile("" ::: "memory");
@@ -405,10 +436,10 @@ struct Pass {
         const bool prepares = owner && wave >= PREPARING && wave < PREPARING + 2, is_key = wave == PREPARING;
         float2 v0 = make_float2(0.f, 0.f), v1 = v0;
         if (wave < ATTENDING || prepares) {
-            const uint32_t src = (wave < ATTENDING ? query : is_key ? G : G + 1) * kHd + 2 * lane;
-            v0 = ld2(a.qkv_at, src); v1 = ld2(a.qkv_at, src + 128);
+            const uint32_t src = (wave < ATTENDING ? query : is_key ? G : G + 1) * kHd + 2 * lane, from = set_of(l) + a.qkv_at;
+            uint32_t looks = 0;
+            do { v0 = ld2(from, src); v1 = ld2(from, src + 128); } while ((empty(v0) || empty(v1)) && again(looks));
         }
-        arrived();
         first_request();
         float* q_s = sh.head[wave];
         float v[4] = {v0.x, v0.y, v1.x, v1.y};
@@ -548,9 +579,8 @@ struct Pass {
         }
         const uint32_t at = (lane >> 5) * 128 + 8 * s16 + ((lane >> 4) & 1u) * 4;
         if constexpr (WPQ == 1) {
-            st4(a.out_at, (slot * G + query) * kHd + at, o);
-            if (lane == 0) st2(a.ml_at, (slot * G + query) * 2, make_float2(top, sum));
-            arrived();
+            st4(set_of(l) + a.out_at, (slot * G + query) * kHd + at, o);
+            if (lane == 0) st2(set_of(l) + a.ml_at, slot * kMl + query * 2, make_float2(top, sum));
         } else {
             own_lds();   // the query has been read
             *reinterpret_cast<f4_t*>(q_s + at) = o;
@@ -559,7 +589,7 @@ struct Pass {
     }
 
     // the last wave, where several share a query: the queries' outputs over this workgroup's tokens
-    __device__ __forceinline__ void publish_attention() {
+    __device__ __forceinline__ void publish_attention(uint32_t l) {
 #pragma unroll
         for (int n = 0; n < G; ++n) {
             float top = sh.ml[n * WPQ].x;
@@ -577,117 +607,177 @@ struct Pass {
                 for (int i = 0; i < 4; ++i) o[i] = fmaf(oj[i], f, o[i]);
                 sum = fmaf(mj.y, f, sum);
             }
-            st4(a.out_at, (slot * G + n) * kHd + 4 * lane, o);
-            if (lane == 0) st2(a.ml_at, (slot * G + n) * 2, make_float2(top, sum));
+            st4(set_of(l) + a.out_at, (slot * G + n) * kHd + 4 * lane, o);
+            if (lane == 0) st2(set_of(l) + a.ml_at, slot * kMl + n * 2, make_float2(top, sum));
         }
     }
 
     // A worker's quads of a row: those of its own blocks, one a lane.
     struct Own { Share blocks; bool on; uint32_t at; };
-    // The last of the row's sum of squares, over the workers' parts.  Every wave meets here.
-    __device__ __forceinline__ float row_total(int which) const {
-        const f4_t lo = *reinterpret_cast<const f4_t*>(&sh.sums[which][0]), hi = *reinterpret_cast<const f4_t*>(&sh.sums[which][4]);
-        return ((lo.x + lo.y) + (lo.z + lo.w)) + ((hi.x + hi.y) + hi.z);
+    // ---- the eighth wave -------------------------------------------------------------------------------------
+    // The row in this wave's registers, quads lane, lane + 64, lane + 128 of it (`mine`: the row has them).
+    static constexpr int kQuads = kMaxWidth / 256 + 1;
+    struct RowQuads { f4_t v[kQuads]; };
+    __device__ __forceinline__ bool mine(int i) const { return lane + 64 * i < a.H / 4; }
+    __device__ __forceinline__ uint32_t quad_at(int i) const { return 4 * min(lane + 64 * i, a.H / 4 - 1); }
+    __device__ __forceinline__ void ask_row(RowQuads& to, const float* p) const {
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) { const float4 t = ldf4_a4(p + quad_at(i)); to.v[i] = f4_t{t.x, t.y, t.z, t.w}; }
     }
-    // x = x + rms(planes, post); the operand of this worker's blocks from rms(x, next).  Two meetings.
-    // outputs: also written to memory (the state after the last block of the launch).
-    template <typename First, typename Second, typename Third>
-    __device__ __forceinline__ void norm_pair(uint32_t planes, const f4_t& post, const f4_t& next, f4_t& x, const Own& own,
-                                              bool outputs, First first_request, Second second_request, Third third_request) {
-        const uint32_t H = a.H;
-        f4_t v = ld4(planes, own.at);
-        const f4_t p1 = ld4(planes, H + own.at), p2 = ld4(planes, 2 * H + own.at);
-        arrived();
-        first_request();
-        v = v + p1 + p2;
-        float ss = (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
-        ss = swap16_sum(row16_sum(own.on ? ss : 0.f));   // 24 lanes at most
-        if (lane == 0) sh.sums[0][wave] = ss;
-        meet();
-        second_request();
-        bool bad = false;
-        float inv = 1.0f / sqrtf(row_total(0) / static_cast<float>(H) + a.eps);
+    // the sum of a projection's planes, once they are there
+    __device__ __forceinline__ RowQuads gather(uint32_t planes) const {
+        f4_t p[kQuads][kParts];
+        uint32_t missing = (1u << (kQuads * kParts)) - 1, looks = 0;
+        do {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            x[i] = v[i] * inv * post[i] + x[i];
-            bad |= !isfinite(x[i]);
+            for (int i = 0; i < kQuads; ++i)
+#pragma unroll
+                for (uint32_t k = 0; k < kParts; ++k)
+                    if (missing >> (kParts * i + k) & 1u) p[i][k] = ld4(planes, k * a.H + quad_at(i));
+            uint32_t left = 0;
+#pragma unroll
+            for (int i = 0; i < kQuads; ++i)
+#pragma unroll
+                for (uint32_t k = 0; k < kParts; ++k)
+                    if (empty(p[i][k])) left |= 1u << (kParts * i + k);
+            missing = left;
+        } while (missing && again(looks));
+        RowQuads r;
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) r.v[i] = p[i][0] + p[i][1] + p[i][2];
+        return r;
+    }
+    // 1 / rms of the row
+    __device__ __forceinline__ float inverse_rms(const RowQuads& r) const {
+        float ss[kQuads];
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) {
+            const f4_t& v = r.v[i];
+            ss[i] = mine(i) ? fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.y, v.y, v.x * v.x))) : 0.f;
         }
-        ss = (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w);
-        ss = swap16_sum(row16_sum(own.on ? ss : 0.f));
-        if (lane == 0) sh.sums[1][wave] = ss;
-        meet();
-        third_request();
-        inv = 1.0f / sqrtf(row_total(1) / static_cast<float>(H) + a.eps);
-        f4_t u;
+        float all = ss[0];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) u[i] = x[i] * inv * next[i];
-        put_quad(u, lane, own.on, sh.opnd[wave], sh.mult[wave]);
-        if (outputs) {
-            float* part = sh.head[wave];   // attention is over: room for the wave's part of the row
-            if (own.on) {
-                *reinterpret_cast<f4_t*>(a.x_out + size_t(row) * H + own.at) = x;
-                *reinterpret_cast<f4_t*>(a.u_out + size_t(row) * H + own.at) = u;
-                if (a.u_last && row + 1 == a.rows) *reinterpret_cast<f4_t*>(a.u_last + own.at) = u;
-                *reinterpret_cast<f4_t*>(part + 4 * lane) = u;
+        for (int i = 1; i < kQuads; ++i) all += ss[i];
+        const float mean = lanes_sum(all) * per_width + a.eps;
+        // the root's reciprocal and one step of Newton's: as close as a root and a division, in a third of their instructions
+        const float y = __builtin_amdgcn_rsqf(mean), better = fmaf(0.5f * y, fmaf(-(mean * y), y, 1.0f), y);
+        return mean == INFINITY ? 0.f : better;
+    }
+    // x = x + rms(v, post), then rms(x, next) for the workers.  outputs: also written to memory (the state after the launch's last block).
+    __device__ __forceinline__ void norm_pair(RowQuads v, const RowQuads& post, RowQuads next, RowQuads& x, bool outputs) const {
+        const uint32_t H = a.H;
+        float inv = inverse_rms(v);
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) v.v[i] *= post.v[i];
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x.v[i][k] = fmaf(v.v[i][k], inv, x.v[i][k]);
+        inv = inverse_rms(x);
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) next.v[i] *= x.v[i];
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) {
+            const f4_t u = next.v[i] * inv;
+            if (mine(i)) {
+                *reinterpret_cast<f4_t*>(sh.u + quad_at(i)) = u;
+                if (outputs) {
+                    const size_t at = size_t(row) * H + quad_at(i);
+                    *reinterpret_cast<f4_t*>(a.x_out + at) = x.v[i];
+                    *reinterpret_cast<f4_t*>(a.u_out + at) = u;
+                    if (a.u_last && row + 1 == a.rows) *reinterpret_cast<f4_t*>(a.u_last + quad_at(i)) = u;
+                }
             }
+        }
+        if (outputs && a.u_receipt_out && (a.receipt_rows > 1 || row + 1 == a.rows)) {
             own_lds();
-            if (a.u_receipt_out && (a.receipt_rows > 1 || row + 1 == a.rows) && lane < 4 * own.blocks.count) {
+            for (uint32_t t = lane; t < H / 8; t += 64) {
                 float y[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) y[i] = part[8 * lane + i];
-                emit_receipt_values(y, 32 * own.blocks.first, lane, a.receipt_rows > 1 ? row : 0u, a.receipt_rows, H, a.u_receipt_out);
+                for (int i = 0; i < 8; ++i) y[i] = sh.u[8 * t + i];
+                emit_receipt_values(y, 0, t, a.receipt_rows > 1 ? row : 0u, a.receipt_rows, H, a.u_receipt_out);
             }
         }
-        if (bad && own.on) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
-        own_lds();
+    }
+    __device__ __forceinline__ void check(const RowQuads& x) const {
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) bad |= mine(i) && !isfinite(x.v[i][k]);
+        if (bad) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
     }
 
-    // ---- the eighth wave -------------------------------------------------------------------------------------
     __device__ __forceinline__ void publisher() {
         const uint32_t tiles = a.H / 64, part = uniform(slot / tiles), column = (slot - part * tiles) * 64 + lane;
+        // this workgroup's words of a set: q/k/v and the attention's, the others'
+        auto mark_empty = [&](uint32_t set, bool attention, bool others) {
+            if (attention) {
+                if (slot < TA) st_bits(set + a.qkv_at, slot * 64 + lane, kEmpty);
+#pragma unroll
+                for (int n = 0; n < G; ++n) st4_bits(set + a.out_at, (slot * G + n) * kHd + 4 * lane, u4_t{kEmpty, kEmpty, kEmpty, kEmpty});
+                if (lane < kMl) st_bits(set + a.ml_at, slot * kMl + lane, kEmpty);
+            }
+            if (others) {
+                if (part < kParts) {
+                    st_bits(set + a.o_at, part * a.H + column, kEmpty);
+                    st_bits(set + a.d_at, part * a.H + column, kEmpty);
+                }
+                if (slot < a.F / 64) st_bits(set + a.h_at, slot * 64 + lane, kEmpty);
+            }
+        };
+        mark_empty(0, true, true);
+        mark_empty(a.set_bytes, true, true);
+        RowQuads x, post, next;
+        ask_row(x, a.x_in + size_t(row) * a.H);
         for (uint32_t l = 0; l < a.layers; ++l) {
             const DLayer& L = a.layer[l];
+            const uint32_t set = set_of(l);
             enter();
             const Tokens t = tokens_of(sh, l, L.ring_mask, slot);
             Rows none;
-            const HeadNorm gamma = ask_gamma(L);
+            const HeadNorm gamma {};
             stamp(l, 0);
             meet();
-            if (slot < TA) st(a.qkv_at, slot * 64 + lane, workers_sum(0));
-            arrive_and_wait();
+            if (slot < TA) st(set + a.qkv_at, slot * 64 + lane, workers_sum(0));
+            if (l == 0) { arrive_and_wait(); meet(); }
+            ask_row(post, L.weights[0]);
+            ask_row(next, L.weights[1]);
             stamp(l, 1);
-            meet();
             attend(l, L, t, gamma, none, [] {}, [] {});
             meet();
-            if constexpr (WPQ > 1) publish_attention();
-            arrive_and_wait();
+            if constexpr (WPQ > 1) publish_attention(l);
             stamp(l, 2);
-            meet();
-            // o-projection
+            // o-projection, norm pair
             meet();
             stamp(l, 3);
-            if (part < kParts) st(a.o_at, part * a.H + column, workers_sum(0));
-            arrive_and_wait();
+            if (part < kParts) st(set + a.o_at, part * a.H + column, workers_sum(0));
+            RowQuads v = gather(set + a.o_at);
             stamp(l, 4);
+            norm_pair(v, post, next, x, false);
             meet();
-            // norm pair, gate and up
-            meet();
-            meet();
+            check(x);
+            ask_row(post, L.weights[2]);
+            ask_row(next, L.weights[3]);
+            // gate and up
             meet();
             stamp(l, 5);
-            if (slot < a.F / 64) st(a.h_at, slot * 64 + lane, geglu_value(workers_sum(0), workers_sum(1)));
-            arrive_and_wait();
+            if (slot < a.F / 64) st(set + a.h_at, slot * 64 + lane, geglu_value(workers_sum(0), workers_sum(1)));
+            // Everybody has read what the block before left, and this block's q/k/v and attention (o says so, whose sums are all here).
+            // The next block's words are marked empty here, where they stay in the L2 until they are wanted; those of its first two phases
+            // were a block ago already: nobody knows there that this block's stores have been made, but the attention in between does.
+            mark_empty(set ^ a.set_bytes, true, true);
+            mark_empty(set, true, false);
             stamp(l, 6);
+            // down, norm pair
             meet();
-            // down
-            meet();
-            if (part < kParts) st(a.d_at, part * a.H + column, workers_sum(0));
-            arrive_and_wait();
+            arrived();
+            if (part < kParts) st(set + a.d_at, part * a.H + column, workers_sum(2));
+            v = gather(set + a.d_at);
             stamp(l, 7);
+            norm_pair(v, post, next, x, l + 1 == a.layers && slot == 0);
             meet();
-            // norm pair
-            meet();
-            meet();
+            check(x);
         }
     }
 
@@ -708,6 +798,7 @@ struct Pass {
         const uint32_t row_part = uniform(slot / tiles), part = row_part < kParts ? row_part : 0, tile = slot - row_part * tiles;
         const Share o_part = share_of(4 * G, kParts, part);
         const bool o_on = wave < o_part.count;
+        const bool merges = o_on && row_part < kParts;
         const uint32_t o_pair = uniform(o_part.first + (o_on ? wave : 0u));
         const uint32_t o_at = uniform((tile * (8 * G) + 2 * o_pair) * kTile);
         // gate and up: a tile pair a workgroup
@@ -720,7 +811,6 @@ struct Pass {
         // workgroup, which one XCD takes 1.1 to 2 us to fetch (1.3 TB/s); in front of a phase's products that is what the products
         // wait for, behind them what the last wave's store and poll do.
         Tile tq[kOwn], to[kOwnO], tg[kOwn], tu[kOwn], td[kOwnDown];
-        f4_t post, next, x;
         Rows rows;
         HeadNorm gamma;
         auto ask_q = [&](const DLayer& from, int i) { ask_tile(tq[i], from.tiles[qm] + q_at, i, own.blocks.count, lane); };
@@ -739,12 +829,7 @@ struct Pass {
             ask_rows(rows, L.ring_k, L.ring_v, t, t.t0, wave, lane);
             gamma = ask_gamma(L);
         }
-        auto norm_weights = [&](const float* p, const float* n) {
-            const float4 vp = ldf4_a4(p + own.at), vn = ldf4_a4(n + own.at);
-            post = f4_t{vp.x, vp.y, vp.z, vp.w}; next = f4_t{vn.x, vn.y, vn.z, vn.w};
-        };
-        // the row and the operand that the launch starts from
-        x = *reinterpret_cast<const f4_t*>(a.x_in + size_t(row) * H + own.at);
+        // the operand that the launch starts from
         put_quad(*reinterpret_cast<const f4_t*>(a.u_in + size_t(row) * H + own.at), lane, own.on, sh.opnd[wave], sh.mult[wave]);
         own_lds();
         auto publish = [&](float acc, int matrix) { sh.red[wave][matrix][lane] = acc; };
@@ -758,6 +843,10 @@ struct Pass {
                 int op[2];
                 i4_t D[kOwn];
                 read_operand(op, sh.opnd[wave], lane);
+                if (l != 0) {
+                    ask_gate(L, 2);
+                    ask_up(L, 0);
+                }
                 steps(tq, op, D);
                 publish(fold(tq, own.blocks.count, D, sh.mult[wave]), 0);
             }
@@ -765,25 +854,29 @@ struct Pass {
             meet();
             const Tokens t = tokens_of(sh, l, L.ring_mask, slot);
             if (t.t0 + kChunk < t.t1) ask_rows(rows, L.ring_k, L.ring_v, t, t.t0 + kChunk, wave, lane);
-            meet();
+            if (l == 0) meet();
             // ---- attention ---------------------------------------------------------------------------------
-            attend(l, L, t, gamma, rows, [&] { ask_up(L, 1); }, [&] { ask_up(L, 2); });
-            ask_down(L, 0);
-            ask_down(L, 1);
-            meet();
+            attend(l, L, t, gamma, rows, [&] { ask_q(N, 0); ask_q(N, 1); ask_q(N, 2); }, [&] { ask_up(L, 1); ask_up(L, 2); });
             meet();
             // ---- merge of the partitions for this wave's 64 elements, o-projection ------------------------
-            {
+            if (merges) {
                 // 16 lanes hold the 64 elements, four each; lane group g the partitions 4 i + g
                 const uint32_t head = (64 * o_pair) / kHd, dim = (64 * o_pair) % kHd, g = lane >> 4, s16 = lane & 15u;
                 f4_t pv[kGroups / 4];
-                const float2 ml = ld2(a.ml_at, ((lane & 31u) * G + head) * 2);
+                float2 ml;
+                // looked at until they are there, those that are missing only: all of them are 49 KB a workgroup
+                uint32_t missing = (2u << (kGroups / 4)) - 1, looks = 0;
+                do {
+                    if (missing >> (kGroups / 4)) ml = ld2(set_of(l) + a.ml_at, (lane & 31u) * kMl + head * 2);
 #pragma unroll
-                for (uint32_t i = 0; i < kGroups / 4; ++i)
-                    pv[i] = ld4(a.out_at + (4 * i * G * kHd + head * kHd + dim) * 4, g * (G * kHd) + 4 * s16);
-                arrived();
-                ask_down(L, 2);
-                norm_weights(L.weights[0], L.weights[1]);
+                    for (uint32_t i = 0; i < kGroups / 4; ++i)
+                        if (missing >> i & 1u) pv[i] = ld4(set_of(l) + a.out_at + (4 * i * G * kHd + head * kHd + dim) * 4, g * (G * kHd) + 4 * s16);
+                    uint32_t left = empty(ml) ? 1u << (kGroups / 4) : 0u;
+#pragma unroll
+                    for (uint32_t i = 0; i < kGroups / 4; ++i)
+                        if (empty(pv[i])) left |= 1u << i;
+                    missing = left;
+                } while (missing && again(looks));
                 float top = ml.y > 0.f ? ml.x : -INFINITY;
                 top = swap16_max(row16_max(top));
                 const float w = ml.y > 0.f ? expf(ml.x - top) : 0.f;
@@ -812,54 +905,64 @@ struct Pass {
                 const GroupScale scale = group_scale(max(m32.x, m32.y));
                 sh.opnd[wave][4 * s16 + g] = digits(v, scale.scale);
                 if ((lane & 0x37u) == 0) sh.mult[wave][s16 >> 3] = scale.mult;
-                if (o_on && !isfinite(v)) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
-                ask_down(L, 3);
                 own_lds();
                 int op[1];
                 i4_t D[kOwnO];
                 read_operand(op, sh.opnd[wave], lane);
+                ask_down(L, 0);
+                ask_down(L, 1);
+                ask_down(L, 2);
                 steps(to, op, D);
-                publish(fold(to, o_on ? 2u : 0u, D, sh.mult[wave]), 0);
+                publish(fold(to, 2u, D, sh.mult[wave]), 0);
+                if (!isfinite(v)) atomicOr(a.status, GUFFIN_STATUS_NONFINITE);
+            } else {
+                publish(0.f, 0);
+                ask_down(L, 0);
+                ask_down(L, 1);
+                ask_down(L, 2);
             }
             meet();
+            // ---- x1 = x + rms(o, post_attention_norm), u = rms(x1, ffn_norm) by the last wave; gate and up ------------
             meet();
-            // ---- x1 = x + rms(o, post_attention_norm); rms(x1, ffn_norm); gate and up ---------------------
-            norm_pair(a.o_at, post, next, x, own, false, [&] { ask_o(N, 0); ask_o(N, 1); }, [] {}, [] {});
             {
+                put_quad(*reinterpret_cast<const f4_t*>(sh.u + own.at), lane, own.on, sh.opnd[wave], sh.mult[wave]);
+                own_lds();
                 int op[2];
                 i4_t D[kOwn], E[kOwn];
                 read_operand(op, sh.opnd[wave], lane);
+                ask_down(L, 3);
+                ask_o(N, 0);
+                ask_o(N, 1);
                 steps(tg, op, D);
                 steps(tu, op, E);
                 publish(fold(tg, own.blocks.count, D, sh.mult[wave]), 0);
                 publish(fold(tu, own.blocks.count, E, sh.mult[wave]), 1);
             }
             meet();
-            meet();
             // ---- down --------------------------------------------------------------------------------------
             {
                 const uint32_t at = 32 * d_first + 4 * min(lane, 8 * max(d_own.count, 1u) - 1);
-                const f4_t hv = ld4(a.h_at, at);
-                arrived();
-                ask_q(N, 0);
-                ask_q(N, 1);
-                ask_q(N, 2);
-                norm_weights(L.weights[2], L.weights[3]);
+                f4_t hv;
+                uint32_t looks = 0;
+                do hv = ld4(set_of(l) + a.h_at, at); while (empty(hv) && again(looks));
                 put_quad(hv, lane, lane < 8 * d_own.count, sh.opnd[wave], sh.mult[wave]);
-                ask_gate(N, 0);
                 own_lds();
                 int op[2];
                 i4_t D[kOwnDown];
                 read_operand(op, sh.opnd[wave], lane);
+                ask_gate(N, 0);
+                ask_gate(N, 1);
                 steps(td, op, D);
-                publish(fold(td, d_own.count, D, sh.mult[wave]), 0);
+                publish(fold(td, d_own.count, D, sh.mult[wave]), 2);
             }
-            meet();
             const Tokens tn = tokens_of(sh, ln, N.ring_mask, slot);
+            ask_rows(rows, N.ring_k, N.ring_v, tn, tn.t0, wave, lane);
+            gamma = ask_gamma(N);
             meet();
-            // ---- x = x1 + rms(down, post_ffw_norm); rms(x, next block's attn_norm or the output norm) -----
-            norm_pair(a.d_at, post, next, x, own, l + 1 == a.layers && slot == 0, [&] { ask_gate(N, 1); },
-                      [&] { ask_gate(N, 2); ask_rows(rows, N.ring_k, N.ring_v, tn, tn.t0, wave, lane); gamma = ask_gamma(N); }, [&] { ask_up(N, 0); });
+            // ---- x = x1 + rms(down, post_ffw_norm), u = rms(x, next block's attn_norm or the output norm) by the last wave ---
+            meet();
+            put_quad(*reinterpret_cast<const f4_t*>(sh.u + own.at), lane, own.on, sh.opnd[wave], sh.mult[wave]);
+            own_lds();
         }
     }
 };
@@ -870,7 +973,7 @@ __global__ void __launch_bounds__(kThreads) drafter_blocks_kernel(const DArgs a)
     const uint32_t row = uniform(xcc_id());   // the model has one KV head: a row an XCD
     if (row >= a.rows) return;
     const uint32_t lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-    Pass<G> pass {a, sh, lane, wave, blockIdx.x / 8, row, 0,
+    Pass<G> pass {a, sh, lane, wave, blockIdx.x / 8, row, 1.0f / static_cast<float>(a.H),
                   __builtin_amdgcn_make_buffer_rsrc(a.exchange + size_t(row) * a.exchange_bytes, 0, static_cast<int>(a.exchange_bytes), 0x00020000)};
     // The arguments' lines, once, all at a time: they come from far, and a block's pointers otherwise cost a wait at each first use.
     {
@@ -916,10 +1019,12 @@ static uint32_t lay_out(const guffin_model_desc& m, DArgs& a) {
     };
     a.qkv_at = take((m.q_heads + 2) * kHd);
     a.out_at = take(kGroups * m.q_heads * kHd);
-    a.ml_at = take(kGroups * m.q_heads * 2);
+    a.ml_at = take(kGroups * kMl);
     a.o_at = take(kParts * m.hidden);
     a.d_at = take(kParts * m.hidden);
     a.h_at = take(m.ffn);
+    a.set_bytes = used;
+    used += a.set_bytes;
     a.kv_at = take(std::min(m.layer_count, kLayers) * kHd);   // a key and a value a block, fp16
     return used;
 }

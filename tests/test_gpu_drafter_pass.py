@@ -159,6 +159,24 @@ def test_a_row_keeps_a_nan_and_says_so(hip):
     assert words[0] != 0 and words[0] == words[1]
 
 
+@pytest.mark.parametrize("which", [0, 1, 2, 3, 4, 5])
+def test_a_gamma_of_all_ones_is_no_missing_word(hip, which):
+    """The pass hands words over by themselves, a word of all ones being one that is still to come: a NaN that looks like it ends in
+    the status word all the same, without a wait that gives up."""
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=2, vocab=1024, ring_global=1024)
+    host = model.HostModel(shape, seed=9, position=100)
+    host.norm[0][which].view(np.uint32)[:] = 0xFFFFFFFF
+    devm = model.DeviceModel.from_host(host)
+    hip.set_forward_mode(2)
+    out = devm.forward(torch.tensor([5], dtype=torch.int32, device="cuda"), 100)
+    torch.cuda.synchronize()
+    hip.set_forward_mode(0)
+    assert not bool(torch.isfinite(out[0]).any())
+    assert int(out[4].item()) != 0 and int(out[4].item()) & 64 == 0 and hip.lib().guffin_hip_resident_enabled() == 1
+
+
 @pytest.mark.parametrize("rows", [1, 2])
 def test_a_model_without_head_norms(hip, rows):
     """Null gammas leave the head norms out, also on the widths of the drafter's own pass."""
