@@ -30,15 +30,17 @@
 //   * The eighth wave has no weights.  It adds the workers' partial sums and stores them; so its looks at the planes do not wait
 //     behind a weight request.
 //   * Attention: a wave a query (four waves are one a SIMD: eight would share the issue slots), a token per 16 lanes with a
-//     running softmax of their own, merged over lanes by register swaps; a list's first 20 tokens lie in LDS before the phase.
+//     running softmax of their own, merged over lanes by register swaps; a list's first 20 tokens lie in LDS before the phase,
+//     three chunks of 20 more are on their way.
 //
 //   * Rows depend on each other through keys and values alone.  A row writes a copy of its own past its L2, raises a flag for the block, and
 //     the workgroups whose part of the list holds an earlier row's wait for that row's flag and take them over into LDS -- the last
 //     wave, which has no weights under way, while the others prepare the queries.  Every row is one hand-over behind the row before
 //     from the first block on, so the wait is short after that; and a row's operations are those of a pass by itself.
 //
-// 270M-shaped model, whole pass at position 150 / 4096: one row 226 / 279 us (288 / 342 with acknowledged stores, a counter and norms shared by
-// the workers).  (resident_blocks_kernel, three launches: one row 606 / 652, two 777 / 888; one launch per operator: 559 / 581 and 609 / 653.)
+// 270M-shaped model, whole pass at position 150 / 4096 / 8180: one row 225 / 260 / 282 us, two rows 232 / 266 / 287; eight rows appended at 150 312 with
+// the host's part.  (With acknowledged stores, a counter, norms shared by the workers and a chunk ahead through their registers 288 / 342 /
+// 387, 302 / 346 / 392, 379; resident_blocks_kernel, three launches: one row 606 / 652, two 777 / 888; one launch per operator: 559 / 581 and 609 / 653.)
 // rms error of the hidden row against 64 bits, one block, where no K/V rounding falls the other way: 6.2e-8 (6.5e-8 before).
 #include "common.hpp"
 #include "receipt.hpp"
@@ -57,7 +59,8 @@ constexpr uint32_t kMaxWidth = 640;       // hidden width: three blocks a worker
 constexpr uint32_t kMaxFfn = 2048;        // a gate / up tile pair a workgroup
 constexpr int kOwn = 3, kOwnO = 2, kOwnDown = 4;          // blocks per worker: of the hidden width, of o, of down
 constexpr uint32_t kTile = 64 * 34;       // a wave tile of one Q8_0 block (gemv_packed.hip has the layout)
-constexpr uint32_t kChunk = 20;           // tokens whose keys and values lie in LDS (a window of 512: 17 a workgroup)
+constexpr uint32_t kChunk = 20;           // tokens whose keys and values lie in LDS together (a window of 512: 17 a workgroup)
+constexpr uint32_t kSlots = 4;            // chunks in LDS: one in work, three on their way (60 requests of 63 that a wave can have)
 
 constexpr uint32_t kMl = 32;              // words between two workgroups' maxima and sums: a cache line each
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;  // a word that nobody has handed over yet
@@ -105,7 +108,7 @@ struct Shared {
     float mult[kWorkers][4];
     float head[kWaves][kHd];                       // a wave's query (then its output, where several waves share a query)
     float2 ml[kWaves];
-    uint16_t k_s[kChunk][kHd], v_s[kChunk][kHd];   // ring rows of a chunk of this workgroup's tokens
+    uint16_t k_s[kSlots][kChunk][kHd], v_s[kSlots][kChunk][kHd];   // ring rows of chunks of this workgroup's tokens
     uint16_t kp_s[kRunRows][kHd], vp_s[kRunRows][kHd];   // the private rows among them
     float weight[kWorkers][kGroups];               // a worker's partition weights, those of lane group g at 8 g ..
     uint32_t schedule[kLayers][4];                 // first ring position, ring count, first private row, private rows (this one the last)
@@ -247,25 +250,41 @@ __device__ __forceinline__ Tokens tokens_of(const Shared& sh, uint32_t l, uint32
     return t;
 }
 
-// A worker's share of a chunk: up to three of its 20 pairs of rows (ten of keys, ten of values), half a wave a row.  Asked for
-// through a buffer resource: lanes past the last token ask beyond its end, which reads zeros and touches no memory.
+// Where lane's 16 bytes of a chunk's rows 2 pair, 2 pair + 1 lie in a ring, half a wave a row.  Asked for through a buffer resource: lanes
+// past the last token ask beyond its end, which reads zeros and touches no memory.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ring_of(const uint16_t* ring, const Tokens& t) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ring), 0, static_cast<int>((t.mask + 1) * (2 * kHd)), 0x00020000);
+}
+__device__ __forceinline__ int ring_place(const Tokens& t, uint32_t chunk, uint32_t pair, uint32_t lane) {
+    const uint32_t token = chunk + 2 * pair + (lane >> 5);
+    return token < t.t1 && token < t.n_ring ? static_cast<int>(((t.first + token) & t.mask) * (2 * kHd) + 16 * (lane & 31u)) : -1024;
+}
+// A worker's share of the first chunk: up to three of its 20 pairs of rows (ten of keys, ten of values).
 struct Rows { uint4 v[3]; };
-__device__ __forceinline__ void ask_rows(Rows& to, const uint16_t* ring_k, const uint16_t* ring_v, const Tokens& t, uint32_t chunk, uint32_t wave, uint32_t lane) {
+__device__ __forceinline__ void ask_rows(Rows& to, const uint16_t* ring_k, const uint16_t* ring_v, const Tokens& t, uint32_t wave, uint32_t lane) {
 #pragma unroll
     for (uint32_t i = 0; i < 3; ++i) {
-        const uint32_t pair = wave + kWorkers * i, row = 2 * (pair % (kChunk / 2)) + (lane >> 5), token = chunk + row;
-        const __amdgpu_buffer_rsrc_t ring = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pair < kChunk / 2 ? ring_k : ring_v), 0,
-                                                                              static_cast<int>((t.mask + 1) * (2 * kHd)), 0x00020000);
-        const bool there = pair < kChunk && token < t.t1 && token < t.n_ring;
-        const int at = there ? static_cast<int>(((t.first + token) & t.mask) * (2 * kHd) + 16 * (lane & 31u)) : -1024;
-        to.v[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ring, at, 0, 0));
+        const uint32_t pair = wave + kWorkers * i;
+        const int at = pair < kChunk ? ring_place(t, t.t0, pair % (kChunk / 2), lane) : -1024;
+        to.v[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ring_of(pair < kChunk / 2 ? ring_k : ring_v, t), at, 0, 0));
     }
 }
 __device__ __forceinline__ void put_rows(Shared& sh, const Rows& from, uint32_t wave, uint32_t lane) {
 #pragma unroll
     for (uint32_t i = 0; i < 3; ++i) {
         const uint32_t pair = wave + kWorkers * i, row = 2 * (pair % (kChunk / 2)) + (lane >> 5);
-        if (pair < kChunk) *reinterpret_cast<uint4*>(&(pair < kChunk / 2 ? sh.k_s : sh.v_s)[row][8 * (lane & 31u)]) = from.v[i];
+        if (pair < kChunk) *reinterpret_cast<uint4*>(&(pair < kChunk / 2 ? sh.k_s : sh.v_s)[0][row][8 * (lane & 31u)]) = from.v[i];
+    }
+}
+// chunk `number` of the list (not the first) straight into its place in LDS, by one wave: kChunk requests
+__device__ __forceinline__ void ask_chunk(Shared& sh, const uint16_t* ring_k, const uint16_t* ring_v, const Tokens& t, uint32_t number, uint32_t lane) {
+    const __amdgpu_buffer_rsrc_t keys = ring_of(ring_k, t), values = ring_of(ring_v, t);
+    const uint32_t slot = number % kSlots;
+#pragma unroll
+    for (uint32_t pair = 0; pair < kChunk / 2; ++pair) {
+        const int at = ring_place(t, t.t0 + kChunk * number, pair, lane);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(keys, (__attribute__((address_space(3))) void*)&sh.k_s[slot][2 * pair][0], 16, at, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(values, (__attribute__((address_space(3))) void*)&sh.v_s[slot][2 * pair][0], 16, at, 0, 0, 0);
     }
 }
 
@@ -422,15 +441,20 @@ struct Pass {
         return load_head_norm(L.weights[wave == PREPARING ? 5 : 4], lane);
     }
 
-    // Every query of the row against this workgroup's tokens.  The first chunk's rows lie in LDS, `rows` holds this worker's share
-    // of the second one; a token per 16 lanes, lane s of them with dimensions 8s .. 8s+7 and 128 + 8s .. 128 + 8s + 7.
-    template <typename First, typename Second>
-    __device__ __forceinline__ void attend(uint32_t l, const DLayer& L, const Tokens& t, const HeadNorm& gamma, Rows& rows, First first_request, Second second_request) {
+    // Every query of the row against this workgroup's tokens; a token per 16 lanes, lane s of them with dimensions 8s .. 8s+7 and 128 +
+    // 8s .. 128 + 8s + 7.  The first chunk's rows lie in LDS; the others are the last wave's to bring (LAST), which has nothing else under
+    // way, three of them ahead of the one in work (position 4096, seven chunks: 9.2 us a block instead of 15.0 with one ahead through
+    // registers of the workers, rounds one after the other; 4.9 of it would be the rows alone).
+    template <bool LAST, typename First, typename Second>
+    __device__ __forceinline__ void attend(uint32_t l, const DLayer& L, const Tokens& t, const HeadNorm& gamma, First first_request, Second second_request) {
         constexpr uint32_t ROUNDS = (kChunk + STEP - 1) / STEP;
         const uint32_t query = wave / WPQ, s16 = lane & 15u;
         const float2* rope = sh.rope[L.local ? 0 : 1];
         // private rows among this workgroup's tokens: this row's key and value are prepared here, a wave each, earlier rows' come
         // from their XCDs
+        const uint32_t chunks = (t.t1 - t.t0 + kChunk - 1) / kChunk;
+        if constexpr (LAST)
+            for (uint32_t c = 1; c < min(chunks, kSlots); ++c) ask_chunk(sh, L.ring_k, L.ring_v, t, c, lane);
         const uint32_t own = t.priv_count - 1, priv_from = max(t.t0, t.n_ring) - t.n_ring, priv_to = max(t.t1, t.n_ring) - t.n_ring;
         const bool owner = priv_from <= own && own < priv_to, peers = min(priv_to, own) > priv_from;
         const bool prepares = owner && wave >= PREPARING && wave < PREPARING + 2, is_key = wave == PREPARING;
@@ -486,82 +510,85 @@ struct Pass {
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-        for (uint32_t chunk = t.t0; chunk < t.t1; chunk += kChunk) {
-            const uint32_t chunk_end = min(chunk + kChunk, t.t1);
-            if (wave < ATTENDING) {
+        for (uint32_t number = 0; number < chunks; ++number) {
+            const uint32_t chunk = t.t0 + kChunk * number, chunk_end = min(chunk + kChunk, t.t1), in_work = number % kSlots;
+            if (!LAST && wave < ATTENDING) {
                 const uint32_t mine = 4 * (wave % WPQ) + (lane >> 4);   // this lane's token of a round, from the chunk's first
-                float s[ROUNDS];
-                // a token's row: a private one, or the chunk's (past the last token zeros, or what the chunk before left)
+                // a token's row: a private one, or the chunk's (zeros past the last token)
                 auto row_at = [&](uint32_t at, const uint16_t (*ring)[kHd], const uint16_t (*priv)[kHd]) {
                     return (chunk + at >= t.n_ring && chunk + at < t.t1 ? priv[chunk + at - t.n_ring] : ring[min(at, kChunk - 1)]) + 8 * s16;
                 };
+                // N rounds without a branch between them, each row asked for a round ahead, four chains a score: a round by itself
+                // is 800 cycles, most of it waiting (position 4096, seven chunks: 9.2 us a block instead of 13.5)
+                auto rounds = [&]<uint32_t N>() {
+                    float s[N];
+                    uint4 ahead[2];   // the next round's key or value
+                    auto ask = [&](uint32_t at, const uint16_t (*ring)[kHd], const uint16_t (*priv)[kHd]) {
+                        const uint16_t* from = row_at(at, ring, priv);
+                        ahead[0] = *reinterpret_cast<const uint4*>(from);
+                        ahead[1] = *reinterpret_cast<const uint4*>(from + 128);
+                        asm volatile("" ::: "memory");   // here
+                        lane = opaque(lane);             // no rounds' addresses kept: there are no registers for them
+                    };
+                    ask(mine, sh.k_s[in_work], sh.kp_s);
 #pragma unroll
-                for (uint32_t u = 0; u < ROUNDS; ++u) {
-                    s[u] = -INFINITY;
-                    if (chunk + STEP * u + 4 * (wave % WPQ) < chunk_end) {
-                        const uint32_t at = STEP * u + mine, token = chunk + at;
-                        const uint16_t* key = row_at(at, sh.k_s, sh.kp_s);
-                        float d[2];
+                    for (uint32_t u = 0; u < N; ++u) {
+                        const uint32_t w[8] = {ahead[0].x, ahead[0].y, ahead[0].z, ahead[0].w, ahead[1].x, ahead[1].y, ahead[1].z, ahead[1].w};
+                        if (u + 1 < N) ask(STEP * (u + 1) + mine, sh.k_s[in_work], sh.kp_s);
+                        else ask(mine, sh.v_s[in_work], sh.vp_s);
+                        float d[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                        for (int p = 0; p < 2; ++p) {
-                            const uint4 k4 = *reinterpret_cast<const uint4*>(key + 128 * p);
-                            const uint32_t w[4] = {k4.x, k4.y, k4.z, k4.w};
-                            d[p] = 0.f;
+                        for (int i = 0; i < 4; ++i)
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                const half2_t h2 = __builtin_bit_cast(half2_t, w[i]);
-                                d[p] = fmaf(static_cast<float>(h2.x), q[2 * p + (i >> 1)][2 * (i & 1)], d[p]);
-                                d[p] = fmaf(static_cast<float>(h2.y), q[2 * p + (i >> 1)][2 * (i & 1) + 1], d[p]);
+                            for (int p = 0; p < 2; ++p) {
+                                const half2_t h2 = __builtin_bit_cast(half2_t, w[4 * p + i]);
+                                d[2 * p] = fmaf(static_cast<float>(h2.x), q[2 * p + (i >> 1)][2 * (i & 1)], d[2 * p]);
+                                d[2 * p + 1] = fmaf(static_cast<float>(h2.y), q[2 * p + (i >> 1)][2 * (i & 1) + 1], d[2 * p + 1]);
                             }
-                        }
-                        const float dot = row16_sum(d[0] + d[1]);
-                        s[u] = token < chunk_end ? dot : -INFINITY;
+                        const float dot = row16_sum((d[0] + d[1]) + (d[2] + d[3]));
+                        s[u] = chunk + STEP * u + mine < chunk_end ? dot : -INFINITY;
                     }
-                }
-                float top = m;
+                    float top = m;
 #pragma unroll
-                for (uint32_t u = 0; u < ROUNDS; ++u) top = fmaxf(top, s[u]);
-                const float base = top == -INFINITY ? 0.f : top;   // nothing attended so far: every weight is zero
-                if (chunk != t.t0) {
-                    const float keep = expf(m - base);
-                    sum *= keep;
+                    for (uint32_t u = 0; u < N; ++u) top = fmaxf(top, s[u]);
+                    const float base = top == -INFINITY ? 0.f : top;   // nothing attended so far: every weight is zero
+                    if (number != 0) {
+                        const float keep = expf(m - base);
+                        sum *= keep;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[i] *= keep;
-                }
-                m = top;
+                        for (int i = 0; i < 16; ++i) acc[i] *= keep;
+                    }
+                    m = top;
 #pragma unroll
-                for (uint32_t u = 0; u < ROUNDS; ++u) {
-                    if (chunk + STEP * u + 4 * (wave % WPQ) < chunk_end) {
-                        const uint32_t at = STEP * u + mine;
-                        const uint16_t* value = row_at(at, sh.v_s, sh.vp_s);
+                    for (uint32_t u = 0; u < N; ++u) {
                         const float p = expf(s[u] - base);
                         sum += p;
-                        if (chunk + at < chunk_end) {
+                        const uint32_t w[8] = {ahead[0].x, ahead[0].y, ahead[0].z, ahead[0].w, ahead[1].x, ahead[1].y, ahead[1].z, ahead[1].w};
+                        if (u + 1 < N) ask(STEP * (u + 1) + mine, sh.v_s[in_work], sh.vp_s);
 #pragma unroll
-                            for (int b = 0; b < 2; ++b) {
-                                const uint4 v4 = *reinterpret_cast<const uint4*>(value + 128 * b);
-                                const uint32_t w[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) {
-                                    const half2_t h2 = __builtin_bit_cast(half2_t, w[i]);
-                                    acc[8 * b + 2 * i] = fmaf(static_cast<float>(h2.x), p, acc[8 * b + 2 * i]);
-                                    acc[8 * b + 2 * i + 1] = fmaf(static_cast<float>(h2.y), p, acc[8 * b + 2 * i + 1]);
-                                }
-                            }
+                        for (int i = 0; i < 8; ++i) {
+                            const half2_t h2 = __builtin_bit_cast(half2_t, w[i]);
+                            acc[2 * i] = fmaf(static_cast<float>(h2.x), p, acc[2 * i]);
+                            acc[2 * i + 1] = fmaf(static_cast<float>(h2.y), p, acc[2 * i + 1]);
                         }
                     }
-                }
+                };
+                if (chunk_end - chunk <= STEP * (ROUNDS / 2)) rounds.template operator()<ROUNDS / 2>();
+                else rounds.template operator()<ROUNDS>();
             }
-            if (chunk + kChunk < t.t1) {   // a longer list: the next chunk takes this one's place
-                meet();
-                if (wave < kWorkers) {
-                    put_rows(sh, rows, wave, lane);
-                    ask_rows(rows, L.ring_k, L.ring_v, t, chunk + 2 * kChunk, wave, lane);
+            if (number + 1 < chunks) {   // the next chunk has arrived, and this one's place is another's
+                if constexpr (LAST) {
+                    const uint32_t younger = min(chunks - 1, number + kSlots - 1) - (number + 1);   // chunks asked for behind the next
+                    if (younger == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kChunk) : "memory");
+                    else if (younger == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kChunk) : "memory");
+                    else arrived();
                 }
                 meet();
+                if constexpr (LAST)
+                    if (number + kSlots < chunks) ask_chunk(sh, L.ring_k, L.ring_v, t, number + kSlots, lane);
             }
         }
-        if (wave >= ATTENDING) return;
+        if (LAST || wave >= ATTENDING) return;
         // the four token groups of the wave: a common maximum, then halves of the values exchanged for halves of the lanes
         const float top = swap32_max(swap16_max(m)), base = top == -INFINITY ? 0.f : top, f = expf(m - base);
         sum = swap32_sum(swap16_sum(sum * f));
@@ -735,8 +762,7 @@ struct Pass {
             const uint32_t set = set_of(l);
             enter();
             const Tokens t = tokens_of(sh, l, L.ring_mask, slot);
-            Rows none;
-            const HeadNorm gamma {};
+            const HeadNorm none {};
             stamp(l, 0);
             meet();
             if (slot < TA) st(set + a.qkv_at, slot * 64 + lane, workers_sum(0));
@@ -744,7 +770,7 @@ struct Pass {
             ask_row(post, L.weights[0]);
             ask_row(next, L.weights[1]);
             stamp(l, 1);
-            attend(l, L, t, gamma, none, [] {}, [] {});
+            attend<true>(l, L, t, none, [] {}, [] {});
             meet();
             if constexpr (WPQ > 1) publish_attention(l);
             stamp(l, 2);
@@ -826,7 +852,7 @@ struct Pass {
             for (int i = 0; i < kOwn; ++i) ask_gate(L, i);
             for (int i = 0; i < 1; ++i) ask_up(L, i);
             const Tokens t = tokens_of(sh, 0, L.ring_mask, slot);
-            ask_rows(rows, L.ring_k, L.ring_v, t, t.t0, wave, lane);
+            ask_rows(rows, L.ring_k, L.ring_v, t, wave, lane);
             gamma = ask_gamma(L);
         }
         // the operand that the launch starts from
@@ -853,10 +879,9 @@ struct Pass {
             put_rows(sh, rows, wave, lane);
             meet();
             const Tokens t = tokens_of(sh, l, L.ring_mask, slot);
-            if (t.t0 + kChunk < t.t1) ask_rows(rows, L.ring_k, L.ring_v, t, t.t0 + kChunk, wave, lane);
             if (l == 0) meet();
             // ---- attention ---------------------------------------------------------------------------------
-            attend(l, L, t, gamma, rows, [&] { ask_q(N, 0); ask_q(N, 1); ask_q(N, 2); }, [&] { ask_up(L, 1); ask_up(L, 2); });
+            attend<false>(l, L, t, gamma, [&] { ask_q(N, 0); ask_q(N, 1); ask_q(N, 2); }, [&] { ask_up(L, 1); ask_up(L, 2); });
             meet();
             // ---- merge of the partitions for this wave's 64 elements, o-projection ------------------------
             if (merges) {
@@ -956,7 +981,7 @@ struct Pass {
                 publish(fold(td, d_own.count, D, sh.mult[wave]), 2);
             }
             const Tokens tn = tokens_of(sh, ln, N.ring_mask, slot);
-            ask_rows(rows, N.ring_k, N.ring_v, tn, tn.t0, wave, lane);
+            ask_rows(rows, N.ring_k, N.ring_v, tn, wave, lane);
             gamma = ask_gamma(N);
             meet();
             // ---- x = x1 + rms(down, post_ffw_norm), u = rms(x, next block's attn_norm or the output norm) by the last wave ---

@@ -72,6 +72,27 @@ def test_the_pass_equals_the_per_operator_pass(hip, gfo, heads, hidden, ffn, lay
     assert rel_rms(got[0].cpu().numpy(), oracle) <= 1e-3
 
 
+# Lists of four and of five chunks of 20 tokens a workgroup to the token (three are asked for ahead of the one in work), of six and
+# seven with a few tokens in the last one, and the longest that a ring holds.
+@pytest.mark.parametrize("heads", [1, 2, 4])
+@pytest.mark.parametrize("rows,position", [(1, 2558), (1, 2560), (2, 3199), (1, 3205), (1, 4095), (2, 5000), (1, 8191)])
+def test_long_lists_equal_the_per_operator_pass(hip, heads, rows, position):
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=2, vocab=1024, ring_global=8192, q_heads=heads, hidden=128, ffn=256, global_period=2)
+    devm = model.DeviceModel.random(shape, seed=heads, position=position)
+    tokens = torch.tensor([17, 999][:rows], dtype=torch.int32, device="cuda")
+    print("long list", heads, rows, position, flush=True)
+    out = []
+    for mode in (1, 2):
+        hip.set_forward_mode(mode)
+        out.append(devm.forward(tokens, position))
+        torch.cuda.synchronize()
+    hip.set_forward_mode(0)
+    assert int(out[0][4].item()) == 0 and int(out[1][4].item()) == 0
+    assert rel_rms(out[1][0].cpu().numpy(), out[0][0].cpu().numpy()) <= 1e-4
+
+
 # heads, hidden, ffn, layers, window, first position, runs: rows of a launch that attend each other's keys from the first token on,
 # across a window's start (also one shorter than a run), in lists of several chunks a workgroup, over more blocks than a launch takes
 RUNS = [(4, 640, 2048, 2, 512, 0, (8, 8, 8)), (4, 640, 2048, 2, 512, 505, (8, 3, 24)), (4, 640, 2048, 3, 512, 1276, (2, 8, 7)),
