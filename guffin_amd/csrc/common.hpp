@@ -224,6 +224,28 @@ __device__ __forceinline__ float wave_max(float v) {
 // their way out, a trip to memory in the middle of a chain.)  What waves exchange through memory needs the other.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Sum of one word of each of `count` waves in LDS, `stride` words apart, in wave order.  All of up to MOST words are read ahead of the
+// first add: a loop over a count known at run time waits for the words it is left with (up to seven) one after the other, 0.04 us
+// each at the end of a launch.  MOST words have to lie there; -0 leaves a sum as it is.
+template <int MOST>
+__device__ __forceinline__ float sum_of_waves(const float* at, uint32_t stride, uint32_t count) {
+    float v[MOST];
+#pragma unroll
+    for (int w = 0; w < MOST; ++w) v[w] = at[w * stride];
+    float t = v[0];
+#pragma unroll
+    for (int w = 1; w < MOST; ++w) t += uint32_t(w) < count ? v[w] : -0.f;
+    return t;
+}
+
+// 1 / sqrt(mean + eps) of a sum of squares, per_width = 1 / width.  The root's reciprocal (an ulp) and one step of Newton's: no
+// further off than a division, a root and a division, which are 40 instructions behind each other where a norm waits for them.
+__device__ __forceinline__ float inverse_rms(float sum, float per_width, float eps) {
+    const float mean = fmaf(sum, per_width, eps), y = __builtin_amdgcn_rsqf(mean);
+    const float better = fmaf(0.5f * y, fmaf(-(mean * y), y, 1.0f), y);
+    return mean == INFINITY ? 0.f : better;
+}
+
 // Sum of `planes` partial planes in plane order; loads are issued four at a time so that the
 // adds, not the memory latency, form the dependent chain.
 __device__ __forceinline__ float load_planes(const float* p, uint32_t planes, size_t plane_stride) {

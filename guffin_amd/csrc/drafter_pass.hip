@@ -675,7 +675,7 @@ struct Pass {
         return r;
     }
     // 1 / rms of the row
-    __device__ __forceinline__ float inverse_rms(const RowQuads& r) const {
+    __device__ __forceinline__ float over_rms(const RowQuads& r) const {
         float ss[kQuads];
 #pragma unroll
         for (int i = 0; i < kQuads; ++i) {
@@ -685,22 +685,19 @@ struct Pass {
         float all = ss[0];
 #pragma unroll
         for (int i = 1; i < kQuads; ++i) all += ss[i];
-        const float mean = lanes_sum(all) * per_width + a.eps;
-        // the root's reciprocal and one step of Newton's: as close as a root and a division, in a third of their instructions
-        const float y = __builtin_amdgcn_rsqf(mean), better = fmaf(0.5f * y, fmaf(-(mean * y), y, 1.0f), y);
-        return mean == INFINITY ? 0.f : better;
+        return inverse_rms(lanes_sum(all), per_width, a.eps);
     }
     // x = x + rms(v, post), then rms(x, next) for the workers.  outputs: also written to memory (the state after the launch's last block).
     __device__ __forceinline__ void norm_pair(RowQuads v, const RowQuads& post, RowQuads next, RowQuads& x, bool outputs) const {
         const uint32_t H = a.H;
-        float inv = inverse_rms(v);
+        float inv = over_rms(v);
 #pragma unroll
         for (int i = 0; i < kQuads; ++i) v.v[i] *= post.v[i];
 #pragma unroll
         for (int i = 0; i < kQuads; ++i)
 #pragma unroll
             for (int k = 0; k < 4; ++k) x.v[i][k] = fmaf(v.v[i][k], inv, x.v[i][k]);
-        inv = inverse_rms(x);
+        inv = over_rms(x);
 #pragma unroll
         for (int i = 0; i < kQuads; ++i) next.v[i] *= x.v[i];
 #pragma unroll

@@ -216,8 +216,8 @@ __device__ __forceinline__ void finish_tile(float (&acc)[R], float* __restrict__
     __syncthreads();
     if (threadIdx.x < R * 64) {
         const uint32_t r = threadIdx.x >> 6;
-        float t = red[r * 64 + lane];
-        for (uint32_t w = 1; w < W; ++w) t += red[(w * R + r) * 64 + lane];
+        const float* at = red + r * 64 + lane;
+        const float t = W <= 4 ? sum_of_waves<4>(at, R * 64, W) : W <= 8 ? sum_of_waves<8>(at, R * 64, W) : sum_of_waves<16>(at, R * 64, W);
         part[(size_t(plane) * R + r) * N + ct * kTileCols + lane] = t;
     }
 }
@@ -299,9 +299,8 @@ gateup_geglu_kernel(const uint8_t* __restrict__ gate_tiles, const uint8_t* __res
     __syncthreads();
     if (threadIdx.x < R * 64) {
         const uint32_t r = threadIdx.x >> 6;
-        float g = red[r * 64 + lane], u = red[(W * R + r) * 64 + lane];
-        for (uint32_t w = 1; w < W; ++w) { g += red[(w * R + r) * 64 + lane]; u += red[((W + w) * R + r) * 64 + lane]; }
-        const float v = geglu_value(g, u);
+        const float* at = red + r * 64 + lane;   // (at most eight waves each)
+        const float v = geglu_value(sum_of_waves<8>(at, R * 64, W), sum_of_waves<8>(at + W * R * 64, R * 64, W));
         h[size_t(r) * F + blockIdx.x * kTileCols + lane] = v;
         vals[r * 64 + lane] = v;
     }

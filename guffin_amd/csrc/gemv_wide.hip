@@ -112,8 +112,7 @@ gemv_wide_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1,
     }
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < rows * 64; i += 64 * W) {
-        float t = red[i];
-        for (uint32_t w = 1; w < W; ++w) t += red[w * kWideRows * 64 + i];
+        const float t = sum_of_waves<WAVES>(red + i, kWideRows * 64, W);
         part[(size_t(blockIdx.y) * rows + (i >> 6)) * N + ct * kTileCols + (i & 63u)] = t;
     }
 }
@@ -133,9 +132,8 @@ gateup_wide_kernel(const uint8_t* __restrict__ gate_tiles, const uint8_t* __rest
     run_wide<DTYPE>(is_up ? up_tiles : gate_tiles, xsums, K, nblk, blockIdx.x, b0, b1, red + wave * kWideRows * 64, lane);
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < rows * 64; i += 128 * W) {
-        float g = red[i], u = red[W * kWideRows * 64 + i];
-        for (uint32_t w = 1; w < W; ++w) { g += red[w * kWideRows * 64 + i]; u += red[(W + w) * kWideRows * 64 + i]; }
-        const float v = geglu_value(g, u);
+        const float v = geglu_value(sum_of_waves<kWideWaves / 2>(red + i, kWideRows * 64, W),
+                                    sum_of_waves<kWideWaves / 2>(red + W * kWideRows * 64 + i, kWideRows * 64, W));
         h[size_t(i >> 6) * F + blockIdx.x * kTileCols + (i & 63u)] = v;
         vals[i] = v;
     }

@@ -179,9 +179,10 @@ rms_norm_add_norm_kernel(const float* __restrict__ x, uint32_t planes, size_t pl
 // The same for the common shape (at most four planes, 16-byte aligned rows, width a multiple of 8
 // and at most 8 x 1024): a thread owns 8 consecutive columns from the operands to the receipt, so
 // every operand is requested at once (one trip to memory instead of one per plane batch) and
-// nothing is staged in LDS but the per-wave sums.  A chain of one trip, two sums over the row and the
-// stores, which all stand at its end: 4.8 us for 3840 columns (5.0 with
-// the first stores ahead of the second sum, whose barriers waited for them).
+// nothing is staged in LDS but the per-wave sums.  A chain of one trip (115 KB a row, 0.8 us of what a CU takes), two sums over
+// the row and the stores, which all stand at its end: 4.4 us for two rows of 3840 columns, of which 3.4 are any launch that
+// reads what the one before wrote (4.5 with a division, a root and a division a norm, the waves' sums in a loop and the stores'
+// pointers asked for between the sums; 5.0 with the first stores ahead of the second sum, whose barriers waited for them).
 constexpr int kFastPlanes = 4;
 __device__ __forceinline__ float4 ld4(const float* p, bool on) {
     return on ? *reinterpret_cast<const float4*>(p) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -193,16 +194,15 @@ rms_norm_add_norm_regs_kernel(const float* __restrict__ x, const float* __restri
                               const float* __restrict__ gamma_next, size_t plane_stride, uint32_t planes, uint32_t width,
                               float eps, uint32_t rows, float* __restrict__ out_residual,
                               float* __restrict__ out_norm, float* __restrict__ out_sums, uint32_t* __restrict__ status) {
-    __shared__ float scratch[2][16];   // the waves' sums: of the first norm, of the second
+    __shared__ __attribute__((aligned(16))) float scratch[2][16];   // the waves' sums: of the first norm, of the second
     const uint32_t r = blockIdx.x, item = threadIdx.x;
     const bool active = item < width / 8;
     auto row_sum = [&](float own, float* sums) {
         own = wave_sum(own);
         if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = own;
         lds_barrier();
-        float t = 0.f;
-        for (uint32_t i = 0; i < (width + 511) / 512; ++i) t += sums[i];  // same order on every thread
-        return t;
+        const uint32_t waves = (width + 511) / 512;   // same order on every thread
+        return waves <= 8 ? sum_of_waves<8>(sums, 1, waves) : sum_of_waves<16>(sums, 1, waves);
     };
     const size_t col = active ? item * 8u : 0u, at = size_t(r) * width + col;
     float4 p[kFastPlanes][2], res4[2], gp4[2], gn4[2];
@@ -214,6 +214,9 @@ rms_norm_add_norm_regs_kernel(const float* __restrict__ x, const float* __restri
 #pragma unroll
         for (int s = 0; s < kFastPlanes; ++s) p[s][h] = ld4(x + s * plane_stride + at + 4 * h, active && uint32_t(s) < planes);
     }
+    // The stores' pointers are not in registers when a wave starts; asked for here they travel beside the operands.
+    asm volatile("" ::"s"(out_residual), "s"(out_norm), "s"(out_sums), "s"(status));
+    const float per_width = 1.0f / static_cast<float>(width);
     float v[8], a[8], gp[8], gn[8], res[8];
     unpack4(p[0][0], v); unpack4(p[0][1], v + 4);
 #pragma unroll
@@ -227,25 +230,24 @@ rms_norm_add_norm_regs_kernel(const float* __restrict__ x, const float* __restri
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
-    float total = row_sum(ss, scratch[0]);
-    float inv = 1.0f / sqrtf(total / static_cast<float>(width) + eps);
+    float inv = inverse_rms(row_sum(ss, scratch[0]), per_width, eps);
     unpack4(gp4[0], gp); unpack4(gp4[1], gp + 4);
     unpack4(gn4[0], gn); unpack4(gn4[1], gn + 4);
     unpack4(res4[0], res); unpack4(res4[1], res + 4);
-    bool bad = false;
     ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const float t = active ? v[i] * inv * gp[i] + res[i] : 0.f;
-        bad |= !isfinite(t);
-        v[i] = t;
-        ss = fmaf(t, t, ss);
+        v[i] = active ? fmaf(v[i] * gp[i], inv, res[i]) : 0.f;
+        ss = fmaf(v[i], v[i], ss);
     }
-    total = row_sum(ss, scratch[1]);
-    inv = 1.0f / sqrtf(total / static_cast<float>(width) + eps);
+    inv = inverse_rms(row_sum(ss, scratch[1]), per_width, eps);
     float y[8];
+    bool bad = false;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = v[i] * inv * gn[i];
+    for (int i = 0; i < 8; ++i) {
+        y[i] = v[i] * gn[i] * inv;
+        bad |= !isfinite(v[i]);
+    }
     if (active) {
         *reinterpret_cast<float4*>(out_residual + at) = make_float4(v[0], v[1], v[2], v[3]);
         *reinterpret_cast<float4*>(out_residual + at + 4) = make_float4(v[4], v[5], v[6], v[7]);

@@ -117,6 +117,13 @@ def test_packed_gemv_parity(hip, gfo, dtype, K, N, rows):
     assert np.all(np.abs(y.astype(np.float64) - yc) <= 2e-5 * scale)
 
 
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("waves", [2, 3, 4, 5, 7, 8, 9, 15, 16])
+def test_a_column_tile_over_any_number_of_waves(hip, gfo, dtype, waves):
+    """200 column tiles of as many blocks as a workgroup has waves: their sums are read four, eight or sixteen at a time."""
+    test_packed_gemv_parity(hip, gfo, dtype, 256 * waves, 12800, 2)
+
+
 @pytest.mark.parametrize("dtype,K,N", [(1, 3840, 2048), (2, 3840, 2048), (2, 15360, 512), (0, 640, 1024), (1, 15360, 256)])
 def test_packed_two_row_rows_equal_one_row_calls(hip, dtype, K, N):
     w = hip.repack(dtype, dev(synth.make_weight(dtype, K, N, 9)), K, N)

@@ -339,3 +339,23 @@ def test_kv_rows_move_between_views_at_any_word_offset(hip, offset_bytes):
         hip.kv_cache_copy(half_word, ring_v, backup_k, backup_v, position, 2, cap - 1, 3)
     with pytest.raises(hip.GuffinError):
         hip.publish_run(run_k, run_v, half_word, ring_v, position, cap - 1)
+
+
+@pytest.mark.parametrize("width", [8, 504, 512, 520, 3840, 4096, 4104, 8192])
+@pytest.mark.parametrize("planes", [1, 4])
+def test_norm_pair_over_any_number_of_waves(hip, width, planes):
+    """One to sixteen waves a row, the last one full or with a single thread.  Every value is a few roundings of 2^-24 from the exact one;
+    a sum of squares beyond the floats' range leaves the residual alone, as a division by an infinite root does."""
+    import torch
+    gen = torch.Generator().manual_seed(width + planes)
+    x = torch.randn(planes, 2, width, generator=gen)
+    gp, gn, res = (torch.randn(s, generator=gen) for s in ((width,), (width,), (2, width)))
+    run = lambda t: hip.rms_norm_add_norm(t.cuda(), gp.cuda(), res.cuda(), gn.cuda(), planes=planes if planes > 1 else None)
+    norm = lambda t, g: t / ((t * t).mean(-1, keepdim=True) + 1e-6).sqrt() * g.double()
+    want = res.double() + norm(x.double().sum(0), gp)
+    got = run(x if planes > 1 else x[0])
+    for g, w in ((got[0], want), (got[1], norm(want, gn))):
+        err = (g.cpu().double() - w).abs() / (w.abs() + (w * w).mean(-1, keepdim=True).sqrt())
+        assert float(err.max()) <= 12 * 2.0 ** -24
+    huge = run((x if planes > 1 else x[0]) * 1e25)
+    assert torch.equal(huge[0].cpu(), res)
