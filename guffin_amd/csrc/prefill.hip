@@ -117,9 +117,9 @@ prefill_attention_kernel(const float* __restrict__ q, const uint16_t* __restrict
 }
 
 // ---- the same attention on the matrix core ------------------------------------------------
-// Values are contracted over tokens, so the B operand needs 8 consecutive tokens of one output
-// dimension: a small pass first writes V^T, [kv_heads][T / 32][256][32] fp16 (a tile in one piece: with rows of T tokens an operand
-// took half of each of sixteen lines), for the virtual tokens
+// Values are contracted over tokens, so a lane's operand is eight tokens of one output dimension, those whose probabilities the lane has:
+// a small pass first writes V^T, [kv_heads][T / 32][256][32] fp16 (a tile in one piece: with rows of T tokens an operand
+// took half of each of sixteen lines), a dimension's 32 tokens in the order of value_token, for the virtual tokens
 // base32 .. base32 + T (T a multiple of 32; tokens outside [first_visible, end) are zero).
 __global__ void __launch_bounds__(256)
 transpose_values_kernel(const uint16_t* __restrict__ ring_v, const uint16_t* __restrict__ run_v,
@@ -147,7 +147,7 @@ transpose_values_kernel(const uint16_t* __restrict__ ring_v, const uint16_t* __r
     for (int t = 0; t < 16; ++t) w[t] = uint32_t(tile[2 * t][dim]) | (uint32_t(tile[2 * t + 1][dim]) << 16);
     uint4* dst = reinterpret_cast<uint4*>(vt + size_t(kvh) * HD * T + (size_t(v0) * HD + dim * 32));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+    for (int i = 0; i < 4; ++i) dst[i] = make_uint4(w[2 * i], w[2 * i + 1], w[8 + 2 * i], w[8 + 2 * i + 1]);   // value_token's order
 }
 
 __device__ __forceinline__ void split_half8(const float (&x)[8], uint4& hi, uint4& lo) {
@@ -192,8 +192,9 @@ __device__ __forceinline__ void emit_attention(const AttentionOut& to, const flo
 }
 
 // a workgroup's LDS: its waves' outputs of an A tile, their states and the merged ones (queries and probabilities take less)
-constexpr uint32_t attention_lds(uint32_t nt, uint32_t waves) { return waves * 16384 + (waves + 1) * nt * 16 * 2 * 4; }
-static_assert(attention_lds(2, 4) >= 2 * (16384 + 4 * 16 * 32 * 4));
+constexpr uint32_t kOutPitch = 256 + 4;   // floats between two pairs' outputs there: 16 lanes that store four dimensions each touch every bank once
+constexpr uint32_t attention_lds(uint32_t nt, uint32_t waves) { return waves * 16 * kOutPitch * 4 + (waves + 1) * nt * 16 * 2 * 4; }
+static_assert(attention_lds(2, 4) >= 2 * 16384);
 
 // grid (kv_heads * ceil(rows * group / (16 NT)), 1, parts), W waves.  Heads run fastest and the last rows come first: consecutive
 // workgroups go to different XCDs, so with eight KV heads an L2 holds one head's keys and values, and the longest lists of a causal
@@ -202,11 +203,17 @@ static_assert(attention_lds(2, 4) >= 2 * (16384 + 4 * 16 * 32 * 4));
 // wave walks its own 32-token tiles (tile index = wave mod W) with its own online softmax state and its own output
 // accumulators; the states are merged at the end.  A run of few rows is cut into parts so that the chip is full; their
 // states are merged by prefill_attention_merge_kernel.
-//   scores   S = Q K^T: queries (scaled, fp16 hi + lo, staged once in LDS in operand order) as A,
-//            keys straight from their fp16 rows as B (a lane reads 8 dims of one key per MFMA)
-//   softmax  a tile that every row sees whole needs no masks, and the accumulators are rescaled only where a maximum moved
-//   values   O += P V: probabilities times 2^10 as fp16 hi + lo through a wave-private LDS
-//            transpose as A, V^T rows as B
+//   scores   S^T = K Q^T: keys straight from their fp16 rows as A (a lane reads 8 dims of one key per MFMA), queries (scaled, fp16
+//            hi + lo, staged once in LDS in operand order) as B.  So a lane has eight scores of one pair, tokens 4 lg .. 4 lg + 3 of
+//            either half of the tile, and four lanes all of that pair's
+//   softmax  over those eight and two swaps of lanes; the denominator stays the lane's own until the end.  A tile that every row
+//            sees whole needs no masks, and the accumulators are rescaled only where a maximum moved
+//   values   O^T += V^T P^T: the lane's own probabilities times 2^10 as fp16 hi + lo as B, V^T rows as A, whose tokens lie in that
+//            order; so a lane has four dimensions of its pair an instruction
+// (S = Q K^T, four pairs a lane: a maximum and a sum over 16 lanes for each, the probabilities through LDS to become an operand and
+// the outputs through LDS word by word: 37 rows at 1500 12.1 us, 333 rows 16.8, 2048 rows 108, the drafter's 1000 21.4; so 10.2, 15.1,
+// 99 and 19.7.  Of the 37 rows' 7.6 behind the launch 2.7 are until the queries are staged, 2.0 until the scores, 0.4 the softmax, 0.9
+// the values, 1.5 the merge.)
 template <int NT, int W>
 __global__ void __launch_bounds__(64 * W, W == 4 ? 2 : 1)
 prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __restrict__ ring_k,
@@ -222,7 +229,6 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
     uint8_t* qa = lds;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 15, lg = lane >> 4;
-    float* pt = reinterpret_cast<float*>(lds + NT * 16384) + wave * (kPairs * 32);   // [NT][16 pairs][32 tokens]
     const uint32_t kvh = blockIdx.x % kv_heads, group = 1u << group_shift;
     const uint32_t r0 = ((((rows << group_shift) + kPairs - 1) / kPairs) - 1 - blockIdx.x / kv_heads) * (kPairs >> group_shift);
     const size_t row_stride = size_t(kv_heads) * HD;
@@ -269,12 +275,11 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the keys stay on their way
 
-    float m[NT][4], l[NT][4];
-    float4_t O[NT][16];
+    float m[NT], l[NT];   // of pair 16 g + j: its maximum; the sum over this lane's tokens
+    float4_t O[NT][16];   // [dt]: dimensions 16 dt + 4 lg .. + 3
 #pragma unroll
     for (int g = 0; g < NT; ++g) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) { m[g][r] = -INFINITY; l[g][r] = 0.f; }
+        m[g] = -INFINITY; l[g] = 0.f;
 #pragma unroll
         for (int dt = 0; dt < 16; ++dt) O[g][dt] = float4_t{0.f, 0.f, 0.f, 0.f};
     }
@@ -298,11 +303,11 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
             for (int half = 1; half >= 0; --half)
 #pragma unroll
                 for (int g = 0; g < NT; ++g) {
-                    const half8_t a = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(qa + ((g * 8 + ks) * 2 + half) * 1024 + lane * 16));
+                    const half8_t q8 = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4*>(qa + ((g * 8 + ks) * 2 + half) * 1024 + lane * 16));
 #pragma unroll
                     for (int c = 0; c < 2; ++c) {
                         float4_t& sum = half == 0 && ks < 4 ? S[g][c] : rest[g][c];
-                        sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8_t, kb[c][ks]),
+                        sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, kb[c][ks]), q8,
                                                                      ks == 0 ? float4_t{0.f, 0.f, 0.f, 0.f} : sum, 0, 0, 0);
                     }
                 }
@@ -312,66 +317,57 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
             for (int c = 0; c < 2; ++c) S[g][c] += rest[g][c];
         if constexpr (NT > 1) __builtin_amdgcn_sched_barrier(0);   // the keys' registers become the values'
         if constexpr (NT > 1) ask_values(0);
-        // online softmax of the lane group's four pairs of a tile; a pair's 32 scores sit in 16 lanes x 2
+        // online softmax of a pair's 32 scores, eight in each of four lanes
         if (!(t0 >= last_first && t0 + 31 <= position + r0)) {
 #pragma unroll
-            for (int g = 0; g < NT; ++g)
+            for (int g = 0; g < NT; ++g) {
+                const uint32_t row = r0 + ((16 * g + j) >> group_shift), pos = position + row;
+                const uint32_t first = (window && pos + 1 > window) ? pos + 1 - window : 0u;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t row = r0 + ((16 * g + 4 * lg + r) >> group_shift), pos = position + row;
-                    const uint32_t first = (window && pos + 1 > window) ? pos + 1 - window : 0u;
+                for (int c = 0; c < 2; ++c)
 #pragma unroll
-                    for (int c = 0; c < 2; ++c) {
-                        const uint32_t kp = t0 + 16 * c + j;
+                    for (int r = 0; r < 4; ++r) {
+                        const uint32_t kp = t0 + 16 * c + 4 * lg + r;
                         if (!(row < rows && kp <= pos && kp >= first)) S[g][c][r] = -INFINITY;
                     }
-                }
+            }
         }
-        float top[NT][4];
+        float top[NT];
         bool moved = false;
 #pragma unroll
-        for (int g = 0; g < NT; ++g)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                top[g][r] = fmaxf(m[g][r], row16_max(fmaxf(S[g][0][r], S[g][1][r])));
-                moved |= top[g][r] > m[g][r];
-            }
+        for (int g = 0; g < NT; ++g) {
+            float t = fmaxf(fmaxf(fmaxf(S[g][0][0], S[g][0][1]), fmaxf(S[g][0][2], S[g][0][3])),
+                            fmaxf(fmaxf(S[g][1][0], S[g][1][1]), fmaxf(S[g][1][2], S[g][1][3])));
+            t = both_max(rows_beside(__float_as_uint(t)));
+            top[g] = fmaxf(m[g], both_max(halves_beside(__float_as_uint(t))));
+            moved |= top[g] > m[g];
+        }
         if (__ballot(moved)) {
 #pragma unroll
-            for (int g = 0; g < NT; ++g)
+            for (int g = 0; g < NT; ++g) {
+                const float resc = top[g] == -INFINITY ? 1.f : exp_of(m[g] - top[g]);
+                l[g] *= resc;
+                m[g] = top[g];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float resc = top[g][r] == -INFINITY ? 1.f : exp_of(m[g][r] - top[g][r]);
-                    l[g][r] *= resc;
-                    m[g][r] = top[g][r];
-#pragma unroll
-                    for (int dt = 0; dt < 16; ++dt) O[g][dt][r] *= resc;
-                }
-        }
-#pragma unroll
-        for (int g = 0; g < NT; ++g)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float from = m[g][r] == -INFINITY ? 0.f : m[g][r];   // nothing seen yet: every score is -inf
-                const float p0 = exp_of(S[g][0][r] - from), p1 = exp_of(S[g][1][r] - from);
-                l[g][r] += row16_sum(p0 + p1);
-                pt[(g * 16 + 4 * lg + r) * 32 + j] = p0 * kProbScale;
-                pt[(g * 16 + 4 * lg + r) * 32 + 16 + j] = p1 * kProbScale;
+                for (int dt = 0; dt < 16; ++dt) O[g][dt] *= resc;
             }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
         half8_t pa[NT][2];
 #pragma unroll
         for (int g = 0; g < NT; ++g) {
-            const float* src = pt + (g * 16 + j) * 32 + 8 * lg;  // A lane (pair j, tokens 8 lg .. 8 lg + 7)
-            const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
-            const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            const float from = m[g] == -INFINITY ? 0.f : m[g];   // nothing seen yet: every score is -inf
+            float x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x[k] = exp_of(S[g][k >> 2][k & 3] - from);
+            l[g] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x[k] *= kProbScale;
             uint4 hi, lo;
             split_half8(x, hi, lo);
             pa[g][0] = __builtin_bit_cast(half8_t, hi);
             pa[g][1] = __builtin_bit_cast(half8_t, lo);
         }
+        __builtin_amdgcn_sched_barrier(0);   // the next keys are asked for here and not ahead of the softmax: there are no registers for that
         auto values = [&](int first) {
 #pragma unroll
             for (int half = 0; half < 2; ++half)
@@ -379,7 +375,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
                 for (int i = 0; i < VB; ++i)
 #pragma unroll
                     for (int g = 0; g < NT; ++g)
-                        O[g][first + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[g][half], __builtin_bit_cast(half8_t, vb[i]), O[g][first + i], 0, 0, 0);
+                        O[g][first + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, vb[i]), pa[g][half], O[g][first + i], 0, 0, 0);
         };
         if constexpr (NT == 1) {
             if (ti + W < end) ask_keys(ti + W, kb);
@@ -390,46 +386,43 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
             ask_values(8);
             values(8);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     // Merge the waves' states through LDS, an A tile at a time: every wave's outputs, scaled to the common maximum by their own
     // wave, have room together and are summed in wave order by whoever stores them.  (One wave behind the other over the same slots:
     // three more passes over them,
     // 14 us of a workgroup's 65 at 2048 rows instead of 9.)
-    float* ob = reinterpret_cast<float*>(lds);  // [wave][dt][4][64 lanes]; the query operands and the probabilities are dead now
-    constexpr uint32_t kWaveSlots = 4096;       // of one wave's outputs
+    float* ob = reinterpret_cast<float*>(lds);  // [wave][16 pairs][kOutPitch]; the query operands are dead now
+    constexpr uint32_t kWaveSlots = 16 * kOutPitch;   // of one wave's outputs
     float* states = reinterpret_cast<float*>(lds + W * kWaveSlots * 4);   // [wave][pair][2]
     float* ml = states + W * kPairs * 2;        // [pair][2], merged
-    __syncthreads();
-    if (j == 0)
 #pragma unroll
-        for (int g = 0; g < NT; ++g)
+    for (int g = 0; g < NT; ++g) {
+        l[g] = both_sum(rows_beside(__float_as_uint(l[g])));
+        l[g] = both_sum(halves_beside(__float_as_uint(l[g])));
+    }
+    if (lg == 0)   // (behind the queries' operands, which others may still read)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                *reinterpret_cast<float2*>(states + (wave * kPairs + 16 * g + 4 * lg + r) * 2) = make_float2(m[g][r], l[g][r]);
+        for (int g = 0; g < NT; ++g) *reinterpret_cast<float2*>(states + (wave * kPairs + 16 * g + j) * 2) = make_float2(m[g], l[g]);
     __syncthreads();
 #pragma unroll
     for (int g = 0; g < NT; ++g) {
         if (g > 0) __syncthreads();   // the tile before has been read
+        const uint32_t pair = 16 * g + j;
+        float2 st[W];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t pair = 16 * g + 4 * lg + r;
-            float2 st[W];
+        for (int w = 0; w < W; ++w) st[w] = *reinterpret_cast<const float2*>(states + (w * kPairs + pair) * 2);
+        float M = st[0].x;
 #pragma unroll
-            for (int w = 0; w < W; ++w) st[w] = *reinterpret_cast<const float2*>(states + (w * kPairs + pair) * 2);
-            float M = st[0].x;
+        for (int w = 1; w < W; ++w) M = fmaxf(M, st[w].x);
+        const float mine = m[g] == -INFINITY ? 0.f : exp_of(m[g] - M);
+        float* slots = ob + wave * kWaveSlots + j * kOutPitch + 4 * lg;
 #pragma unroll
-            for (int w = 1; w < W; ++w) M = fmaxf(M, st[w].x);
+        for (int dt = 0; dt < 16; ++dt) *reinterpret_cast<float4_t*>(slots + 16 * dt) = O[g][dt] * mine;
+        if (wave == 0 && lg == 0) {
             float den = 0.f;
 #pragma unroll
             for (int w = 0; w < W; ++w) den += st[w].x == -INFINITY ? 0.f : st[w].y * exp_of(st[w].x - M);
-            const float mine = m[g][r] == -INFINITY ? 0.f : exp_of(m[g][r] - M);
-            float* slots = ob + wave * kWaveSlots + r * 64 + lane;
-#pragma unroll
-            for (int dt = 0; dt < 16; ++dt) slots[dt * 256] = O[g][dt][r] * mine;
-            if (wave == 0 && j == 0) *reinterpret_cast<float2*>(ml + pair * 2) = make_float2(M, den);
+            *reinterpret_cast<float2*>(ml + pair * 2) = make_float2(M, den);
         }
         __syncthreads();
 #pragma unroll 1
@@ -437,7 +430,7 @@ prefill_attention_mfma_kernel(const float* __restrict__ q, const uint16_t* __res
             const uint32_t i = kStep * n + threadIdx.x / 32, c8 = threadIdx.x % 32, p = 16 * g + i;
             const uint32_t row = r0 + (p >> group_shift), head = kvh * group + (p & (group - 1));
             if (row >= rows) continue;
-            const float* src = ob + (((c8 >> 1) * 4 + (i & 3)) * 64 + 8 * (c8 & 1) + 16 * (i >> 2));
+            const float* src = ob + i * kOutPitch + 8 * c8;
             float v[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) {

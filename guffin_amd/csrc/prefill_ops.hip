@@ -263,11 +263,11 @@ prefill_qkv_kernel(const float* __restrict__ q_planes, const float* __restrict__
             *reinterpret_cast<uint4*>(&tile[token][8 * d8]) = val;
         }
         lds_barrier();
-        const uint32_t dim = threadIdx.x >> 2, t0 = 8 * (threadIdx.x & 3);   // four threads: a dimension's 32 tokens
+        const uint32_t dim = threadIdx.x >> 2, lg = threadIdx.x & 3;   // four threads: a dimension's 32 tokens
         uint32_t o[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = uint32_t(tile[t0 + 2 * t][dim]) | (uint32_t(tile[t0 + 2 * t + 1][dim]) << 16);
-        *reinterpret_cast<uint4*>(a.vt + size_t(kvh) * HD * a.T + size_t(v0) * HD + 32 * dim + t0) = make_uint4(o[0], o[1], o[2], o[3]);
+        for (int t = 0; t < 4; ++t) o[t] = uint32_t(tile[value_token(lg, 2 * t)][dim]) | (uint32_t(tile[value_token(lg, 2 * t + 1)][dim]) << 16);
+        *reinterpret_cast<uint4*>(a.vt + size_t(kvh) * HD * a.T + size_t(v0) * HD + 32 * dim + 8 * lg) = make_uint4(o[0], o[1], o[2], o[3]);
     }
     if (bad && a.status) atomicOr(a.status, GUFFIN_STATUS_KV_NONFINITE);
 }

@@ -30,6 +30,8 @@ inline ValueSpan value_span(uint32_t rows, uint32_t position, uint32_t window) {
     const uint32_t base32 = first & ~31u;
     return {first, base32, (position + rows - base32 + 31u) & ~31u};
 }
+// Element e of k-slice lg of a dimension's 32 tokens in V^T: the tokens whose probabilities lane group lg has (four of either half).
+__host__ __device__ constexpr uint32_t value_token(uint32_t lg, uint32_t e) { return (e < 4 ? 0u : 12u) + 4 * lg + e; }
 // The matrix-core path wants one, two or four query heads per KV head, and K/V rows and queries at 16-byte addresses.
 bool prefill_attention_on_matrix_core(const void* q, const void* ring_k, const void* ring_v, const void* run_k, const void* run_v,
                                       uint32_t q_heads, uint32_t kv_heads);
@@ -50,7 +52,7 @@ struct QkvRun {
     const float *q_planes, *k_planes, *v_planes;   // planes of [rows][heads * 256]
     const float *q_norm, *k_norm, *rope_table;     // table [rows][128] of cos, sin
     float* q_out; uint16_t *k_out, *v_out;         // [rows][heads * 256]
-    const uint16_t* ring_v; uint16_t* vt;          // vt [kv_heads][T / 32][256][32]
+    const uint16_t* ring_v; uint16_t* vt;          // vt [kv_heads][T / 32][256][32], tokens as value_token has them
     uint32_t planes, rows, q_heads, kv_heads, position, ring_mask, first_visible, base32, T, head_groups;
     float eps;
     uint32_t* status;
