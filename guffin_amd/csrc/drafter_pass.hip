@@ -276,10 +276,22 @@ __device__ __forceinline__ void put_rows(Shared& sh, const Rows& from, uint32_t 
         if (pair < kChunk) *reinterpret_cast<uint4*>(&(pair < kChunk / 2 ? sh.k_s : sh.v_s)[0][row][8 * (lane & 31u)]) = from.v[i];
     }
 }
-// chunk `number` of the list (not the first) straight into its place in LDS, by one wave: kChunk requests
+// chunk `number` of the list (not the first) straight into its place in LDS, by one wave: kChunk requests.  (Requests into LDS want
+// whole 16 bytes: rings that lie off them go through the wave's registers.)
 __device__ __forceinline__ void ask_chunk(Shared& sh, const uint16_t* ring_k, const uint16_t* ring_v, const Tokens& t, uint32_t number, uint32_t lane) {
     const __amdgpu_buffer_rsrc_t keys = ring_of(ring_k, t), values = ring_of(ring_v, t);
     const uint32_t slot = number % kSlots;
+    if ((reinterpret_cast<uintptr_t>(ring_k) | reinterpret_cast<uintptr_t>(ring_v)) & 15u) {
+#pragma unroll 1
+        for (uint32_t pair = 0; pair < kChunk / 2; ++pair) {
+            const int at = ring_place(t, t.t0 + kChunk * number, pair, lane);
+            const uint4 k = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(keys, at, 0, 0));
+            const uint4 v = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(values, at, 0, 0));
+            *reinterpret_cast<uint4*>(&sh.k_s[slot][2 * pair + (lane >> 5)][8 * (lane & 31u)]) = k;
+            *reinterpret_cast<uint4*>(&sh.v_s[slot][2 * pair + (lane >> 5)][8 * (lane & 31u)]) = v;
+        }
+        return;
+    }
 #pragma unroll
     for (uint32_t pair = 0; pair < kChunk / 2; ++pair) {
         const int at = ring_place(t, t.t0 + kChunk * number, pair, lane);

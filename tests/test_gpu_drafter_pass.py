@@ -218,3 +218,27 @@ def test_a_model_without_head_norms(hip, rows):
         out.append(got[0].cpu().numpy())
     hip.set_forward_mode(0)
     assert rel_rms(out[1], out[0]) <= 1e-4 and rel_rms(out[0], normed) > 1e-2
+
+
+@pytest.mark.parametrize("off", [2, 4, 8, 12])
+def test_rings_that_lie_off_16_bytes(hip, off):
+    """Lists of several chunks a workgroup, whose later chunks go straight into LDS where the rings are aligned: the same bits."""
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=2, vocab=1024, ring_global=4096, hidden=128, ffn=256, global_period=2)
+    devm = model.DeviceModel.random(shape, seed=off, position=4000)
+    tokens = torch.tensor([17], dtype=torch.int32, device="cuda")
+    hip.set_forward_mode(0)
+    want = devm.forward(tokens, 4000)[0].clone()
+    kept = []
+    for l in range(shape.layers):
+        for rings, field in ((devm.ring_k, "ring_k"), (devm.ring_v, "ring_v")):
+            ring = rings[l]
+            words = torch.empty(ring.numel() + 16, dtype=torch.int16, device="cuda")
+            words[off // 2:off // 2 + ring.numel()] = ring.view(torch.int16).flatten()
+            kept.append(words)
+            setattr(devm.layers[l], field, words.data_ptr() + off)
+    got = devm.forward(tokens, 4000)
+    torch.cuda.synchronize()
+    assert int(got[4].item()) == 0 and hip.lib().guffin_hip_resident_enabled() == 1
+    assert torch.equal(got[0], want)
