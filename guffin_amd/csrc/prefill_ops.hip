@@ -15,15 +15,13 @@
 namespace guffin {
 namespace {
 
-// scratch: nobody else's, and used once; waves: of the workgroup
+// scratch: 16 floats, nobody else's, and used once; waves: of the workgroup
 __device__ __forceinline__ float block_total(float v, float* scratch, uint32_t waves) {
     v = wave_sum(v);
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (lane == 0) scratch[wv] = v;
     lds_barrier();
-    float t = 0.f;
-    for (uint32_t i = 0; i < waves; ++i) t += scratch[i];  // same order on every thread
-    return t;
+    return waves <= 8 ? sum_of_waves<8>(scratch, 1, waves) : sum_of_waves<16>(scratch, 1, waves);  // same order on every thread
 }
 
 // 8 consecutive floats of `planes` planes, summed in plane order; up to B planes are requested before the first add
@@ -76,7 +74,7 @@ __device__ __forceinline__ uint32_t row_of(uint32_t b, uint32_t rows) {
 __global__ void __launch_bounds__(1024)
 prefill_norm_kernel(const float* __restrict__ x, const float* __restrict__ gamma, uint8_t* __restrict__ image, uint32_t rows,
                     uint32_t width, float eps, uint32_t* __restrict__ status) {
-    __shared__ float scratch[16];
+    __shared__ __attribute__((aligned(16))) float scratch[16];
     const uint32_t r = row_of(blockIdx.x, rows), t = threadIdx.x;
     const bool active = t < width / 8;
     float v[8] = {}, g[8] = {};
@@ -84,7 +82,7 @@ prefill_norm_kernel(const float* __restrict__ x, const float* __restrict__ gamma
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
-    const float inv = 1.0f / sqrtf(block_total(ss, scratch, (width + 511) / 512) / static_cast<float>(width) + eps);
+    const float inv = inverse_rms(block_total(ss, scratch, (width + 511) / 512), 1.0f / static_cast<float>(width), eps);
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < 8; ++i) { v[i] = v[i] * inv * g[i]; bad |= !isfinite(v[i]); }
@@ -110,7 +108,7 @@ prefill_joint_kernel(const float* __restrict__ x, const float* __restrict__ resi
         static_cast<U4a4*>(run.ring_v)[dst] = static_cast<const U4a4*>(run.run_v)[size_t(row) * run.row_vec + c];
         return;
     }
-    __shared__ float scratch[2][16];
+    __shared__ __attribute__((aligned(16))) float scratch[2][16];
     const uint32_t r = row_of(blockIdx.x, rows), t = threadIdx.x;
     const bool active = t < width / 8;
     const size_t at = size_t(r) * width + 8 * t;
@@ -121,22 +119,27 @@ prefill_joint_kernel(const float* __restrict__ x, const float* __restrict__ resi
         load8_words(gamma_next + 8 * t, gn);
         sum_planes8<B>(x + at, planes, plane_stride, v);
     }
+    // what only the stores need, asked for beside the operands (see rms_norm_add_norm_regs_kernel)
+    asm volatile("" ::"s"(out_residual), "s"(out_norm), "s"(image), "s"(status));
+    const float per_width = 1.0f / static_cast<float>(width);
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
-    float inv = 1.0f / sqrtf(block_total(ss, scratch[0], (width + 511) / 512) / static_cast<float>(width) + eps);
-    bool bad = false;
+    float inv = inverse_rms(block_total(ss, scratch[0], (width + 511) / 512), per_width, eps);
     ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        v[i] = v[i] * inv * gp[i] + res[i];
-        bad |= !isfinite(v[i]);
+        v[i] = fmaf(v[i] * gp[i], inv, res[i]);
         ss = fmaf(v[i], v[i], ss);
     }
-    inv = 1.0f / sqrtf(block_total(ss, scratch[1], (width + 511) / 512) / static_cast<float>(width) + eps);
+    inv = inverse_rms(block_total(ss, scratch[1], (width + 511) / 512), per_width, eps);
     if (active) store8(out_residual + at, v);
+    bool bad = false;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = v[i] * inv * gn[i];
+    for (int i = 0; i < 8; ++i) {
+        bad |= !isfinite(v[i]);
+        v[i] = v[i] * gn[i] * inv;
+    }
     if (active) {
         if (image) emit_image_values(v, t, r, image_layout(rows, width), image);
         else store8_words(out_norm + at, v);
@@ -220,7 +223,7 @@ prefill_qkv_kernel(const float* __restrict__ q_planes, const float* __restrict__
                 }
         }
         float ss = fmaf(v[0], v[0], fmaf(v[1], v[1], fmaf(v[2], v[2], v[3] * v[3])));
-        const float normed = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(HD) + a.eps), inv = gamma ? normed : 1.f;
+        const float normed = inverse_rms(wave_sum(ss), 1.0f / HD, a.eps), inv = gamma ? normed : 1.f;
         v[0] = v[0] * inv * g0.x; v[1] = v[1] * inv * g0.y; v[2] = v[2] * inv * g1.x; v[3] = v[3] * inv * g1.y;
         const float o0 = __fsub_rn(__fmul_rn(v[0], rot.x), __fmul_rn(v[2], rot.y)), o1 = __fsub_rn(__fmul_rn(v[1], rot.z), __fmul_rn(v[3], rot.w));
         const float o2 = __fadd_rn(__fmul_rn(v[0], rot.y), __fmul_rn(v[2], rot.x)), o3 = __fadd_rn(__fmul_rn(v[1], rot.w), __fmul_rn(v[3], rot.z));
