@@ -99,6 +99,15 @@ __device__ __forceinline__ void hist_add(uint32_t* hist, bool valid, uint32_t bi
     if ((todo >> lane) & 1u) atomicAdd(&hist[bin], 1u);
 }
 
+// The same where the bins were made to spread the words: lanes of one wave rarely share one, and each counts for itself.
+__device__ __forceinline__ void hist_add_spread(uint32_t* hist, bool valid, uint32_t bin, uint32_t lane) {
+    const uint64_t live = __ballot(valid);
+    if (!live) return;
+    const uint32_t first = __builtin_amdgcn_readlane(bin, __ffsll(static_cast<long long>(live)) - 1);
+    if (__popcll(__ballot(valid && bin == first)) > 8) hist_add(hist, valid, bin, lane);
+    else if (valid) atomicAdd(&hist[bin], 1u);
+}
+
 // Writes one row of the result from its `retain` selected keys (candidate order) and appends the logits of
 // the row's history tokens; all threads of the workgroup call it after the keys are complete.  raised: the row's status word;
 // whole: the record is new memory, what it does not use becomes zero.
@@ -317,8 +326,8 @@ topk_merge_kernel(const float* __restrict__ logits, const uint64_t* __restrict__
 // arrival is whoever draws the last ticket.  Up to kCollectCap keys of a row are sorted in LDS, however they
 // lie: the common list holds what the places of a single collector leave of that many.  A row with more is
 // selected exactly, and slowly, by a radix select over the whole row in that workgroup.
-// 262144 logits: 64 of two rows 8.8 us (10.6 with an exact bound and every key through one reservation), what a compact law
-// of 64 needs of one row 8.8 (15.4 with its best 257 in order).  Ties, both launches and the call: 300 to 2000 keys 18 to 29 us,
+// 262144 logits: 64 of two rows 6.8 us (an exact bound and every key through one reservation cost 1.8 more), a compact law of 64
+// and its proposal 10.5.  Ties, both launches and the call: 300 to 2000 keys 18 to 29 us,
 // beyond 2048 keys 920.
 constexpr uint32_t kSeg = 256, kMaxSegs = 1024, kCollectTile = 4096, kCollectCap = 2048;
 struct Nothing {};
@@ -353,7 +362,7 @@ segment_max_kernel(const float* __restrict__ logits, uint32_t vocab, uint32_t se
     for (uint32_t u = 0; u < kSeg / 64; ++u) {
         const uint32_t t = seg * kSeg + u * 64 + lane;
         if (t < vocab) {
-            const uint32_t o = ordered_bits(lr[t] / divisor);
+            const uint32_t o = ordered_bits(divisor == 1.f ? lr[t] : lr[t] / divisor);
             best = o > best ? o : best;
         }
     }
@@ -394,6 +403,7 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t* __restrict__
     __shared__ uint64_t sel[kCollectCap];
     __shared__ uint64_t keys[512];
     __shared__ uint32_t s_bin, s_above, s_in, s_last, s_count;
+    __shared__ uint32_t s_low[16], s_top[16];   // the waves' least (inverted) and largest maxima
     const uint32_t row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, collectors = (vocab + kCollectTile - 1) / kCollectTile;
     uint32_t* row_ws = ws + size_t(row) * kThresholdRowWords;
     uint32_t* counter = row_ws + kMaxSegs;
@@ -416,39 +426,57 @@ threshold_select_kernel(const float* __restrict__ logits, uint32_t* __restrict__
     const uint32_t hc = history_count ? history_count[size_t(row) * row_stride] : 0;
     // ---- the bound: at or below the largest segment maximum but `least` - 1 (there are as many by the launch's condition), with
     // no more than an eighth of `least` maxima too many above it; every further byte would cost a pass, most rows stop after two
+    // The first pass has 256 bins between the least and the largest maximum: maxima are alike, and the top byte of their bits says
+    // next to nothing.  (Passes from the top byte down, equal bins counted by one lane: 64 of two rows 8.8 us, so 6.8.)
     const uint32_t least = sure ? sure : retain;
-    uint32_t prefix = 0, remaining = least, shift = 24;
-    for (;; shift -= 8) {
-        if (tid < 256) hist[tid] = 0;
-        __syncthreads();
-        hist_add(hist, tid < segs && (shift == 24 || (word >> (shift + 8)) == prefix), (word >> shift) & 255u, lane);
+    const uint32_t wave_top = wave_max_u32(tid < segs ? word : 0u), wave_low = wave_max_u32(tid < segs ? ~word : 0u);
+    if (lane == 0) { s_top[tid >> 6] = wave_top; s_low[tid >> 6] = wave_low; }
+    if (tid < 256) hist[tid] = 0;
+    if (tid == 0) s_count = 0;
+    __syncthreads();
+    auto of_waves = [](uint32_t v) {   // the largest of sixteen, in every lane
+        v = max(v, lane_cross_u32<0xB1, 0xF>(v));
+        v = max(v, lane_cross_u32<0x4E, 0xF>(v));
+        v = max(v, lane_cross_u32<0x141, 0xF>(v));
+        v = max(v, lane_cross_u32<0x140, 0xF>(v));
+        return __builtin_amdgcn_readfirstlane(v);
+    };
+    const uint32_t top = of_waves(s_top[lane & 15u]);
+    uint32_t bound = ~of_waves(s_low[lane & 15u]);   // the lower edge of bin 0, then of the bin that was found
+    uint32_t remaining = least, bins = 256u, shift = top > bound ? 24u - min(24u, static_cast<uint32_t>(__clz(static_cast<int>(top - bound)))) : 0u;
+    for (;;) {
+        const uint32_t bin = (word - bound) >> shift;
+        hist_add_spread(hist, tid < segs && word >= bound && bin < bins, bin, lane);
         __syncthreads();
         if (tid < 64) find_bin(hist, remaining, lane, s_bin, s_above, s_in);
-        if (tid == 0) s_count = 0;
         __syncthreads();
-        prefix = (prefix << 8) | s_bin;
+        bound += s_bin << shift;
         remaining -= s_above;
         if (shift == 0 || s_in - remaining <= least / 8) break;
+        const uint32_t finer = shift > 8 ? shift - 8 : 0u;
+        bins = 1u << (shift - finer);
+        shift = finer;
+        if (tid < 256) hist[tid] = 0;
+        __syncthreads();
     }
-    const uint32_t bound = prefix << shift;
     // ---- collect: this workgroup's keys into LDS, then into its places and, past them, the row's common list ----
     bool bad = false;
+    auto collect = [&](auto scaled) {   // (sixteen waves and exact division: dividing by one is not free)
 #pragma unroll
-    for (uint32_t u = 0; u < kCollectTile / 1024; ++u) {
-        const uint32_t t = token_of(u);
-        bool hit = false;
-        uint64_t key = 0;
-        if (t < vocab) {
-            const float v = mine[u] / divisor;
-            bad |= (!isfinite(v) || !isfinite(mine[u])) && !(suppressed_ok && mine[u] == -INFINITY);
-            key = make_key(v, t);
-            hit = static_cast<uint32_t>(key >> 32) >= bound;
+        for (uint32_t u = 0; u < kCollectTile / 1024; ++u) {
+            const uint32_t t = token_of(u);
+            if (t < vocab) {
+                const float v = scaled(mine[u]);
+                bad |= (!isfinite(v) || !isfinite(mine[u])) && !(suppressed_ok && mine[u] == -INFINITY);
+                if (ordered_bits(v) >= bound) {
+                    const uint32_t at = atomicAdd(&s_count, 1u);
+                    if (at < kCollectCap) sel[at] = make_key(v, t);
+                }
+            }
         }
-        if (hit) {
-            const uint32_t at = atomicAdd(&s_count, 1u);
-            if (at < kCollectCap) sel[at] = key;
-        }
-    }
+    };
+    if (divisor == 1.f) collect([](float x) { return x; });
+    else collect([&](float x) { return x / divisor; });
     __syncthreads();
     const uint32_t found = s_count;
     if (tid < kSlots && tid < found) shared_store(places + blockIdx.x * kSlots + tid, sel[tid]);

@@ -111,23 +111,6 @@ __device__ __forceinline__ void note_first(bool hit, uint32_t index, uint32_t* t
     if (hits && (threadIdx.x & 63u) == 0) atomicMin(to, index + static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(hits))) - 1u);
 }
 
-// Sort of the first n keys in LDS by rank, n at most the workgroup's size: every thread counts the keys that go
-// before its own (all lanes read the same word: a broadcast) and drops its key at that place.  Three barriers
-// instead of the bitonic network's one per stage (28 for 128 keys, 45 for 512).
-// Distinct keys, ascending: a permutation of the n places.
-__device__ __forceinline__ void rank_sort_ascending(uint64_t* keys, uint32_t n) {
-    __syncthreads();
-    const uint32_t t = threadIdx.x;
-    const uint64_t mine = t < n ? keys[t] : 0;
-    uint32_t rank = 0;
-    if (t < n)
-#pragma unroll 8
-        for (uint32_t j = 0; j < n; ++j) rank += keys[j] < mine;
-    __syncthreads();
-    if (t < n) keys[rank] = mine;
-    __syncthreads();
-}
-
 // The law from the best 257 scores (sorted, score = logit / T).  The 256 threads of a workgroup (those that are left of a
 // larger one) call it: thread t with entry t, counted or not, all with the record's count and status and entry 256's score.
 __device__ __forceinline__ void compact_law(const LawCall& call, uint32_t avail, uint32_t raised, uint32_t found_token, float found_logit, float more) {
@@ -140,7 +123,8 @@ __device__ __forceinline__ void compact_law(const LawCall& call, uint32_t avail,
     __shared__ uint64_t keys[256];
     __shared__ float score[256], weight[256], running[256];
     __shared__ uint64_t edge[257];
-    __shared__ uint32_t s_n, s_first, s_bad, s_chosen;
+    __shared__ uint32_t ids[256];
+    __shared__ uint32_t s_first, s_bad, s_chosen, s_word;
     const uint32_t t = threadIdx.x;
     const bool usable = options_valid(opt) && opt.temperature > 0.f && opt.top_k <= 64 && avail >= 1;
     const uint32_t k = usable ? (opt.top_k < avail ? opt.top_k : avail) : 1u;
@@ -154,32 +138,32 @@ __device__ __forceinline__ void compact_law(const LawCall& call, uint32_t avail,
     // entry that is below the cutoff or -inf
     note_first(!(t < avail && !(my_logit < cutoff) && my_logit != -INFINITY), t, &s_first);
     __syncthreads();
-    if (t == 0) {
-        uint32_t st = 0, n = 0;
-        if (!usable) st = GUFFIN_STATUS_LAW_INVALID;
-        if (raised & GUFFIN_STATUS_NONFINITE) st = GUFFIN_STATUS_LAW_INVALID | GUFFIN_STATUS_NONFINITE;
-        if (!st) {
-            n = s_first;
-            if (n == 256u && avail > 256u) {   // all 256 are in: a 257th eligible entry overflows the compact law
-                if (!(more < cutoff) && more != -INFINITY) n = 257u;
-            }
-            if (n == 0) st = GUFFIN_STATUS_LAW_INVALID;  // nothing eligible
-            if (n > 256) st = GUFFIN_STATUS_LAW_INVALID | 32u;  // support overflow: needs the full-vocabulary law
+    uint32_t st = 0, n = 0;   // every thread's own, all alike
+    if (!usable) st = GUFFIN_STATUS_LAW_INVALID;
+    if (raised & GUFFIN_STATUS_NONFINITE) st = GUFFIN_STATUS_LAW_INVALID | GUFFIN_STATUS_NONFINITE;
+    if (!st) {
+        n = s_first;
+        if (n == 256u && avail > 256u) {   // all 256 are in: a 257th eligible entry overflows the compact law
+            if (!(more < cutoff) && more != -INFINITY) n = 257u;
         }
-        s_n = st ? 0 : n;
+        if (n == 0) st = GUFFIN_STATUS_LAW_INVALID;  // nothing eligible
+        if (n > 256) st = GUFFIN_STATUS_LAW_INVALID | 32u;  // support overflow: needs the full-vocabulary law
+    }
+    if (t == 0) {
         if (full_error) *full_error = 0;
         if (st == (GUFFIN_STATUS_LAW_INVALID | 32u) && full_error) { law->count = kLawFull; *proposal = 0xFFFFFFFFu; }
         else if (st) { atomicOr(status, st); law->count = 0; *proposal = 0xFFFFFFFFu; }
     }
-    __syncthreads();
-    const uint32_t n = s_n;
-    if (n == 0) {
+    if (st) {
         if (whole) { law->ids[t] = 0; law->cdf[t] = 0; if (t == 0) { law->pad = 0; law->cdf[256] = 0; } }
         return;
     }
-    score[t] = t < n ? my_logit : -INFINITY;
-    weight[t] = t < n ? law_exp(my_logit - first_logit) : 0.f;
+    // An entry's weight against the best one, which the filters always leave: the weights of the law are these, those of what is
+    // filtered zero.
+    const float own_weight = t < n ? law_exp(my_logit - first_logit) : 0.f;
+    weight[t] = own_weight;
     __syncthreads();
+    if (t == 64) s_word = injected ? injected->word : step_draws(seed, step).word;   // another wave's, beside the sums
     if (t == 0) {  // descending-tail top-p / min-p in the reference's sequential order
         // the tail sums from the last entry down; the last of them, in slot 0 (always kept), is the total: the
         // same adds in the same order
@@ -198,25 +182,24 @@ __device__ __forceinline__ void compact_law(const LawCall& call, uint32_t avail,
         }
     }
     __syncthreads();
-    if (t > 0 && t < n) {
-        const bool keep = (opt.top_p >= 1.0f || __fdiv_rn(running[t], running[0]) > __fsub_rn(1.0f, opt.top_p))
-                          && (opt.min_p <= 0.0f || weight[t] >= opt.min_p);
-        if (!keep) score[t] = -INFINITY;
+    const bool keep = t == 0 || ((opt.top_p >= 1.0f || __fdiv_rn(running[t], running[0]) > __fsub_rn(1.0f, opt.top_p))
+                                 && (opt.min_p <= 0.0f || own_weight >= opt.min_p));
+    // ascending token id; the weight rides in the low half of the key
+    keys[t] = t < n ? (uint64_t(my_token) << 32) | __float_as_uint(keep ? own_weight : 0.f) : ~uint64_t{0};
+    __syncthreads();
+    {   // places: the keys that go before one's own, counted by one, two or four neighbouring lanes
+        const uint32_t part_bits = n <= 64 ? 2 : n <= 128 ? 1 : 0, i = t >> part_bits, part = t & ((1u << part_bits) - 1);
+        const uint64_t mine = keys[i];
+        uint32_t rank = 0;
+#pragma unroll 8
+        for (uint32_t j = part; j < n; j += 1u << part_bits) rank += keys[j] < mine;
+        if (part_bits >= 1) rank += lane_cross_u32<0xB1, 0xF>(rank);
+        if (part_bits >= 2) rank += lane_cross_u32<0x4E, 0xF>(rank);
+        if (i < n && part == 0) {   // (weight: zeros behind the last entry as before)
+            ids[rank] = static_cast<uint32_t>(mine >> 32);
+            weight[rank] = __uint_as_float(static_cast<uint32_t>(mine));
+        }
     }
-    __syncthreads();
-    // ascending token id; the score rides in the low half of the key
-    keys[t] = t < n ? (uint64_t(my_token) << 32) | __float_as_uint(score[t]) : ~uint64_t{0};
-    rank_sort_ascending(keys, n);   // entries beyond the support are all-ones keys already in their final place
-    score[t] = t < n ? __uint_as_float(static_cast<uint32_t>(keys[t])) : -INFINITY;
-    __syncthreads();
-    {   // the maximum of the support (a maximum does not depend on the order it is taken in)
-        const float wave_best = wave_max(t < n ? score[t] : -INFINITY);
-        if ((t & 63u) == 0) weight[t >> 6] = wave_best;
-    }
-    __syncthreads();
-    const float maximum = fmaxf(fmaxf(weight[0], weight[1]), fmaxf(weight[2], weight[3]));
-    __syncthreads();
-    weight[t] = t < n ? law_exp(__fsub_rn(score[t], maximum)) : 0.f;
     __syncthreads();
     if (t == 0) {   // the f32 running sums in token order; the quotients and edges are per-lane work
         ordered_sums(weight, n, running);
@@ -233,12 +216,11 @@ __device__ __forceinline__ void compact_law(const LawCall& call, uint32_t avail,
         edge[t + 1] = next;
     }
     __syncthreads();
-    const StepDraws d = injected ? *injected : step_draws(seed, step);
     if (t < n) {
         const uint64_t last = edge[t];
         if (next < last || next > kMassTotal || (t == n - 1 && next != kMassTotal)) s_bad = 1;
-        if (uint64_t(d.word) >= last && uint64_t(d.word) < next) s_chosen = static_cast<uint32_t>(keys[t] >> 32);
-        law->ids[t] = static_cast<uint32_t>(keys[t] >> 32);
+        if (uint64_t(s_word) >= last && uint64_t(s_word) < next) s_chosen = ids[t];
+        law->ids[t] = ids[t];
         law->cdf[t + 1] = next;
     } else if (whole) {
         law->ids[t] = 0;

@@ -272,10 +272,10 @@ law_cdf_select_kernel(uint32_t vocab, bool greedy, uint64_t seed, uint64_t step,
 // =========================================================================================
 // One workgroup of two teams, a candidate row each: whether row 1 is wanted is known only at the end, and by then its law is
 // ready.  The kernel is a chain of short dependent steps, so what it costs is their number: everything is requested at once;
-// duplicates and places come out of one walk over the record; a sum whose order matters is one lane's, the compensated sum of
-// the same terms another wave's beside it and the masses of q a third's; running sums are kept, so that a draw is found by all
+// duplicates and places come out of one walk over the record; a sum whose order matters is one lane's, the masses of q another
+// wave's beside it; running sums are kept, so that a draw is found by all
 // lanes at once; at temperatures of 1 and 0 the tempered weights are the raw ones and their sums are not taken twice.
-// An accepted proposal over 64 candidates takes 12.0 us (25.0 with a row after the other, and a step after the other inside).
+// An accepted proposal over 64 candidates takes 10.2 us (twice that with a row after the other, and a step after the other inside).
 constexpr uint32_t kTeam = kMaxCandidates;   // threads of a row, a candidate each
 
 struct Prepared {
@@ -290,29 +290,19 @@ struct RowScratch {
     uint64_t keys[kMaxCandidates], sorted[kMaxCandidates];
     float raw[kMaxCandidates];
     double w[kMaxTopK];              // raw weights, zeros behind the last entry
-    double compensated[kMaxTopK];    // compensated running sums of the weights
+    double lost[kMaxTopK];           // what the running sums of the weights lost, entry by entry; then the sums of that
     uint32_t hist[kHistoryCap];
     uint32_t kept, cut;              // ends of the top-p and min-p prefixes
     uint32_t dup, unique, flag, pick;
     int err;
 };
 
-// Neumaier's compensated sum over v[0] ... v[i], for every i; zeros past the end change nothing
-__device__ __forceinline__ void compensated_sums(const double* __restrict__ v, uint32_t n, double* __restrict__ out) {
-    double total = 0.0, correction = 0.0, x[8];
-    for (uint32_t i0 = 0; i0 < n; i0 += 8) {
-#pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) x[k] = v[i0 + k];
-#pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) {
-            const double w = x[k], sum = total + w;
-            correction += total >= w ? (total - sum) + w : (w - sum) + total;
-            total = sum;
-            x[k] = total + correction;
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) out[i0 + k] = x[k];
-    }
+// Neumaier's compensated sum over v[0] ... v[i] is run[i] plus the sum of what its additions lost: the terms of that sum are every
+// lane's own where the running sums are known, and what is left of the order are additions.  (All of it by one lane, an entry after
+// the other, beside the plain sums: an accepted proposal 10.4 us, so 10.2.)
+__device__ __forceinline__ double lost_by(const double* __restrict__ v, const double* __restrict__ run, uint32_t i) {
+    const double w = v[i], total = i ? run[i - 1] : 0.0, sum = run[i];
+    return total >= w ? (total - sum) + w : (w - sum) + total;
 }
 // the reference's consistency check of a law's stored total against its compensated sum
 __device__ __forceinline__ bool total_holds(double total, double stored, uint32_t count) {
@@ -479,7 +469,6 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
     __syncthreads();
     if (t == 0) ordered_sums(sc.w, count, out.run);
     if (team == 0) {
-        if (t == 64 && plain) compensated_sums(sc.w, count, sc.compensated);
         if (!target_to_draft && t >= 128 && t - 128 < count) q[t - 128] = law_mass(q_law, full_cdf, vocab, out.token[t - 128], nullptr);
     } else if (t == 128) {
         uint64_t begin = 0;   // a law that failed leaves no proposal
@@ -502,9 +491,11 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
         if (t < kMaxTopK) out.weight[t] = t < count ? exp(static_cast<double>(below) / static_cast<double>(opt.temperature)) : 0.0;
         __syncthreads();
         if (t == 0) ordered_sums(out.weight, count, out.run);
-        if (t == 64 && team == 0) compensated_sums(out.weight, count, sc.compensated);
         __syncthreads();
     }
+    if (team == 0 && t < kMaxTopK) sc.lost[t] = t < count ? lost_by(out.weight, out.run, t) : 0.0;
+    __syncthreads();
+    if (team == 0 && t == 64) ordered_sums(sc.lost, count, sc.lost);
     const double norm = count ? out.run[count - 1] : 0.0;
     if (!rc && (!isfinite(norm) || norm <= 0.0)) rc = -7;
     if (t == 0) { out.count = rc ? 0u : count; out.total = norm; if (team == 1) sc.err = rc; }
@@ -533,7 +524,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
     double proposed = 0.0, normalization = -1.0;
     if (head && !code) {
         auto unit = [](double u) { return isfinite(u) && u >= 0.0 && u < 1.0; };
-        normalization = scratch[0].compensated[count - 1];
+        normalization = norm + scratch[0].lost[count - 1];
         const bool valid = total_usable(count, norm) && !sc.flag && total_holds(normalization, norm, count);
         uint64_t gathered = 0;
         for (uint32_t w = 0; w < kTeam / 64; ++w) gathered += wave_mass[w];
@@ -567,7 +558,10 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
     }
     __syncthreads();
     if (head && t == 0) ordered_sums(residual.weight, excess, residual.run);
-    if (head && t == 64) compensated_sums(residual.weight, excess, sc.compensated);
+    __syncthreads();
+    if (head && t < kMaxTopK) sc.lost[t] = t < excess ? lost_by(residual.weight, residual.run, t) : 0.0;
+    __syncthreads();
+    if (head && t == 0) ordered_sums(sc.lost, excess, sc.lost);
     __syncthreads();
     const double acceptance = s_acceptance, residual_total = excess ? residual.run[excess - 1] : 0.0;
     const bool decided = code == 0;
@@ -583,7 +577,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
             if (scratch[1].err) code = scratch[1].err - 100;
             else note_first(t < after.count && d.u_next * after.total < after.run[t], t, &sc.pick);
         } else {
-            if (!total_usable(excess, residual_total) || !total_holds(sc.compensated[excess - 1], residual_total, excess)) code = -26;
+            if (!total_usable(excess, residual_total) || !total_holds(residual_total + sc.lost[excess - 1], residual_total, excess)) code = -26;
             else {
                 if (t < excess && !weight_usable(residual.weight[t], residual_total)) sc.flag = 1;
                 note_first(t < excess && d.u_residual * residual_total < residual.run[t], t, &sc.pick);

@@ -140,3 +140,26 @@ def test_a_fresh_law_clears_what_it_does_not_write(vocab, ties):
         assert status == 48 and proposal.view(torch.int32).item() == -1   # refused, more than fit, and nothing else
     else:
         assert status == 0 and proposal.view(torch.int32).item() in order[:5].tolist()
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 255, 256])
+@pytest.mark.parametrize("top_p,min_p", [(1.0, 0.0), (0.9, 0.0), (1.0, 0.4), (0.7, 0.1)])
+def test_a_law_s_places_are_the_oracle_s(n, top_p, min_p):
+    """Supports on both sides of 64 and 128 entries, whose places one, two or four lanes find: ids, edges and proposal to the bit, also
+    where a filter left entries without mass and at divisors of one and others."""
+    from oracle import gfo
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(262144).astype(np.float32)
+    order, top_k = np.argsort(-x, kind="stable"), min(n, 64)
+    x[order[top_k - 1:n]] = x[order[top_k - 1]]   # ties with the last place make up the rest
+    for temperature, word in ((1.0, 5), (0.7, (1 << 32) - 1), (1.3, 1 << 31)):
+        draws = np.zeros(1, hip.draws_dtype)
+        draws["word"] = word
+        law, proposal, status = hip.draft_law(torch.from_numpy(x).cuda(), hip.SamplerOptions(temperature, top_k, top_p, min_p, 1.0),
+                                              draws=torch.from_numpy(draws.view(np.uint8)).cuda())
+        law = law.cpu().numpy().view(hip.law_dtype)[0]
+        rc, want = gfo.draft_law_compact(x, gfo.SamplerOptions(temperature, top_k, top_p, min_p, 1.0))
+        assert rc == 0 and int(status.item()) == 0 and int(law["count"]) == want.count <= n
+        n = want.count
+        assert list(law["ids"][:n]) == list(want.ids[:n]) and list(law["cdf"][:n + 1]) == list(want.cdf[:n + 1])
+        assert int(proposal.item()) & 0xFFFFFFFF == gfo.lib().gfo_draft_select(C.byref(want), C.c_uint32(word))
