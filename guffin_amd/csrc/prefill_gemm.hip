@@ -21,7 +21,10 @@
 //
 // A workgroup is four waves on the same R * 16 rows and four neighbouring column tiles.  The A operand of a 64-element
 // chunk goes from memory to LDS without passing registers, two chunks ahead in three rotating buffers, one barrier per
-// chunk; weights are private to a wave and requested half a block ahead.
+// chunk; weights are private to a wave and requested half a block ahead.  A barrier waits for the chunk it opens and leaves everything younger
+// on its way, weights too: waits are counts of requests, so requests have a fixed order (in_order()).  Waiting for the weights as well, with the
+// first of them asked for behind the first barrier, blocks of 12B shapes took, us, so / as it is: 16 rows 95.9 / 93.4, 37 rows 123.4 / 121.3, 96 rows
+// 169.9 / 168.4, 333 rows 428.8 / 424.1; of Q4_K alone 16 rows 88.8 / 86.6, 100 rows 190.4 / 183.0, 192 rows 246.6 / 242.4.
 //
 // What bounds it: the instructions that form B.  A loop of one matrix and V packed vector instructions (sixteen independent chains of the one, eight
 // of the other, two waves a SIMD) takes 8.9, 10.2, 10.6, 12.2 and 13.6 ns of a SIMD for V = 0 to 4, 1.4 more for each further one; a
@@ -131,7 +134,15 @@ __device__ __forceinline__ uint4_t from_lds16(const uint8_t* at) { return *reint
 __device__ __forceinline__ uint2_t from_lds8(const uint8_t* at) { return *reinterpret_cast<const uint2_t*>(at); }
 // the wave's requests but the N youngest have arrived and its LDS accesses are done, and so have every wave's
 template <int N>
+__device__ __forceinline__ void arrived() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory"); }
+template <int N>
 __device__ __forceinline__ void arrive() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
+// requests on either side keep their order, which the counts above rely on
+__device__ __forceinline__ void in_order() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
 
 // What a launch brings.  A kernel takes it as words and pointers in this order: the first fourteen words of a launch's arguments
 // are in registers when a wave starts (a build flag), as long as no struct stands among them.
@@ -258,6 +269,7 @@ template <int R, bool HALVES>
 __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint8_t* stage, const uint8_t* tile_base,
                                         uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4], uint32_t mid, float4_t* kept_sums) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q4_K);
+    constexpr int kHalf = 4;                        // requests of a half block's quants
     constexpr int V = (26 + 4 * R - 1) / (4 * R);   // vector instructions behind each matrix instruction
     // Up to three row tiles the fold is woven in as well: a tile's beside the next tile's products, the last one's beside the
     // second half's first products.  Four leave no registers for that (2048 x 3840 x 15360: 446 us against 440 by itself).
@@ -299,18 +311,20 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
     ask_half(b0, 0, q[0]);
     ask_head(b0);
     feed.ask(4 * b0, 0);
-    asm volatile("" ::: "memory");   // in this order
-    ask_half(b0, 1, q[1]);
+    in_order();
     feed.ask(4 * b0 + 1, 1);
-    asm volatile("" ::: "memory");
+    in_order();
+    ask_half(b0, 1, q[1]);
+    in_order();
     feed.ask(4 * b0 + 2, 2);
-    arrive<2 * R>();
+    arrive<2 * R + kHalf>();
     scales(b0, 0);
     read_half<R>(stage, 1, lane16, lo);
     q4_operands<0, 0>(q[0], sc, operands[0]);
     q4_operands<0, 1>(q[0], sc, operands[0]);
     uint32_t rd = 0;   // the buffer of the chunk in work
-    for (uint32_t blk = b0; blk < b1; ++blk) {
+    uint32_t blk = b0;   // (no test ahead of the first block: behind one, the first weights would be asked for after the first meeting)
+    do {
         if constexpr (!WOVEN) { lane = lane_again(); j = lane & 15; lg = lane >> 4; lane16 = feed.lane16 = lane * 16; }   // no register to keep addresses in
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
         if constexpr (HALVES) {
@@ -342,6 +356,9 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
         auto group = [&]<int G>() {
             half8_t (&b)[4] = operands[G & 1], (&bn)[4] = operands[(G + 1) & 1];
             const uint8_t* now = stage + rd * S::kChunk + (G & 1) * (2048 * R);
+            if constexpr (G == 3) ask_half(next, 0, q[0]);   // the half's last operands were formed beside the group before
+            if constexpr (G == 7) ask_half(next, 1, q[1]);
+            if constexpr ((G & 3) == 3) in_order();
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (G == 3) scales(blk, 1);
             if constexpr (WOVEN && G == 3) fold_scales();
@@ -361,15 +378,12 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
                 weave<4 * R, V, R>();
             }
             if constexpr (G & 1) {
-                arrive<R>();
-                if constexpr (G == 1) {
-                    ask_block(blk);
-                    ask_head(next);
-                    asm volatile("" ::: "memory");   // in this order: the fold reads the multipliers behind the next meeting
-                }
-                if constexpr (G == 3) ask_half(next, 0, q[0]);
-                if constexpr (G == 7) ask_half(next, 1, q[1]);
+                // What may still be on its way: the chunk asked for at the last meeting and half a block of weights, asked for a group
+                // before this meeting (3, 7) or the last one (1, 5); at 3 the next header as well (the fold wants the multipliers).
+                arrive<R + kHalf + (G == 3 ? 1 : 0)>();
+                if constexpr (G == 1) { ask_block(blk); in_order(); }
                 feed.ask(4 * blk + (G >> 1) + 3, rd);
+                if constexpr (G == 1) { in_order(); ask_head(next); }
                 rd = rd == 2 ? 0 : rd + 1;
             }
             const uint8_t* then = stage + rd * S::kChunk + ((G + 1) & 1) * (2048 * R);
@@ -427,7 +441,7 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-    }
+    } while (++blk < b1);
 }
 
 // ---- Q6_K ------------------------------------------------------------------------------------------------
@@ -496,6 +510,7 @@ template <int R>
 __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& feed, uint8_t* stage, const uint8_t* tile_base,
                                         uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q6_K);
+    constexpr int kHalf = 8;   // requests of a half block's quants
     constexpr int V0 = (60 + 4 * R - 1) / (4 * R), V1 = (38 + 4 * R - 1) / (4 * R);
     using S = Stage<R>;
     const uint32_t lane = threadIdx.x & 63, wv = feed.wv, j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
@@ -522,23 +537,27 @@ __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& fee
     ask_half(b0, 0);
     ask_head(b0);
     feed.ask(4 * b0, 0);
-    asm volatile("" ::: "memory");   // in this order
-    ask_half(b0, 1);
+    in_order();
     feed.ask(4 * b0 + 1, 1);
-    asm volatile("" ::: "memory");
+    in_order();
+    ask_half(b0, 1);
+    in_order();
     feed.ask(4 * b0 + 2, 2);
-    arrive<2 * R>();
+    arrive<2 * R + kHalf>();
     scales(b0, 0);
     read_half<R>(stage, 0, lane16, hi);
     q6_quants<0>(ql[0], qh[0], operands[0]);
     q6_scaled<0>(sc, operands[0], rest);
-    uint32_t rd = 0;
-    for (uint32_t blk = b0; blk < b1; ++blk) {
+    uint32_t rd = 0, blk = b0;
+    do {
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
         auto group = [&]<int G>() {
             constexpr int H = ((G + 1) & 7) >> 2, QD = (G + 1) & 3;   // the next group's half block and place
             half8_t (&b)[4] = operands[G & 1], (&bn)[4] = operands[(G + 1) & 1];
             const uint8_t* now = stage + rd * S::kChunk + (G & 1) * (2048 * R);
+            if constexpr (G == 3) ask_half(next, 0);
+            if constexpr (G == 7) ask_half(next, 1);
+            if constexpr ((G & 3) == 3) in_order();
             __builtin_amdgcn_sched_barrier(0);
             read_half<R>(now, 1, lane16, lo);
             q6_quants<QD>(ql[H], qh[H], bn);
@@ -550,14 +569,13 @@ __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& fee
             products<R, false>(hi, b, D);
             weave<4 * R, V1, 0>();
             if constexpr (G & 1) {
-                arrive<R>();
+                arrive<R + kHalf + (G == 3 ? 2 : 0)>();   // as the Q4_K walk, a header being two requests
                 if constexpr (G == 1) {
                     if (wv == 2) to_lds4(feed.img, stage + S::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (blk * L.mpad + rt0 * 16) * 4);
-                    ask_head(next);
+                    in_order();
                 }
-                if constexpr (G == 3) ask_half(next, 0);
-                if constexpr (G == 7) ask_half(next, 1);
                 feed.ask(4 * blk + (G >> 1) + 3, rd);
+                if constexpr (G == 1) { in_order(); ask_head(next); }
                 rd = rd == 2 ? 0 : rd + 1;
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -586,7 +604,7 @@ __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& fee
                 for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(d[cg] * mult[i], D[cg][r][i], acc[cg][r][i]);
         }
         __builtin_amdgcn_sched_barrier(0);
-    }
+    } while (++blk < b1);
 }
 
 // The same for four row tiles, where the accumulators leave no registers for operands formed ahead: column groups by pairs,
@@ -596,6 +614,7 @@ template <int R>
 __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed, uint8_t* stage, const uint8_t* tile_base,
                                              uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q6_K);
+    constexpr int kHalf = 8;   // requests of a half block's quants
     using S = Stage<R>;
     const uint32_t wv = feed.wv;
     uint32_t lane = lane_again(), j = lane & 15, lg = lane >> 4, lane16 = lane * 16;
@@ -621,25 +640,28 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
     ask_half(b0, 0);
     ask_head(b0);
     feed.ask(4 * b0, 0);
-    asm volatile("" ::: "memory");   // in this order
+    asm volatile("" ::: "memory");
     feed.ask(4 * b0 + 1, 1);
-    uint32_t rd = 0, wr = 2;
-    for (uint32_t blk = b0; blk < b1; ++blk) {
+    uint32_t rd = 0, wr = 2, blk = b0;
+    do {
         lane = lane_again(); j = lane & 15; lg = lane >> 4; lane16 = feed.lane16 = lane * 16;   // no register to keep addresses in
         sel = lane >= 32 ? 0x07030501u : 0x06020400u;
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;
         auto group = [&]<int G>() {
             constexpr int H = G >> 2, QD = G & 3;
             if constexpr ((G & 1) == 0) {
-                arrive<R>();
+                // the last meeting's requests may still be on their way: a chunk and, at 2 and 6, a half block's quants, at 4 a header
+                arrive<R + (G == 0 ? 0 : G == 4 ? 2 : kHalf)>();
                 if constexpr (G == 0) {
-                    ask_half(blk, 1);
                     if (wv == 2) to_lds4(feed.img, stage + S::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (blk * L.mpad + rt0 * 16) * 4);
+                    ask_half(blk, 1);
                     scales(blk, 0);
                 }
                 if constexpr (G == 2) ask_head(next);
                 if constexpr (G == 4) { ask_half(next, 0); scales(blk, 1); }
+                asm volatile("" ::: "memory");
                 feed.ask(4 * blk + (G >> 1) + 2, wr);
+                asm volatile("" ::: "memory");
             }
             const uint8_t* from = stage + rd * S::kChunk + (G & 1) * (2048 * R);
             half8_t hi[R], lo[R], b[4], rest[4];
@@ -677,7 +699,7 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(d[cg] * mult[i], D[cg][r][i], acc[cg][r][i]);
         }
-    }
+    } while (++blk < b1);
 }
 
 // grid (row chunks, column groups of 256 over all segments, k-slices), so that an XCD's L2 keeps its share of the image, or as
