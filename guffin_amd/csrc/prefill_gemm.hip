@@ -262,12 +262,9 @@ __device__ __forceinline__ void products(const half8_t (&a)[R], const half8_t (&
 // next region's A operands come from LDS and the next group's B operands are formed, so a wave by itself keeps the matrix
 // pipe and the vector pipe busy together.  A chunk's last lo half is in registers when its last region starts: there the
 // workgroup meets, the next chunk has arrived and the one after the next but one is asked for in place of the old.
-// HALVES: the sums start anew at block `mid`, the first half's wait in LDS (`kept_sums`, [4 R][256 threads]): a slice of twice the length
-// rounds as two slices, and the planes, the workgroups' first trips and the next operator's reads are those of one.
-constexpr uint32_t kKeptStride = 256;   // of a thread's quads: the workgroup's
-template <int R, bool HALVES>
+template <int R>
 __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint8_t* stage, const uint8_t* tile_base,
-                                        uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4], uint32_t mid, float4_t* kept_sums) {
+                                        uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
     constexpr uint32_t TB = kCols * block_bytes(GUFFIN_Q4_K);
     constexpr int kHalf = 4;                        // requests of a half block's quants
     constexpr int V = (26 + 4 * R - 1) / (4 * R);   // vector instructions behind each matrix instruction
@@ -327,19 +324,6 @@ __device__ __forceinline__ void q4_walk(const ImageLayout& L, Feed<R> feed, uint
     do {
         if constexpr (!WOVEN) { lane = lane_again(); j = lane & 15; lg = lane >> 4; lane16 = feed.lane16 = lane * 16; }   // no register to keep addresses in
         const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
-        if constexpr (HALVES) {
-            if (blk == mid) {
-                float4_t* to = kept_sums + wv * 64 + lane_again();
-#pragma unroll
-                for (int cg = 0; cg < 4; ++cg)
-#pragma unroll
-                    for (int r = 0; r < R; ++r) {
-                        float(&sum)[4] = acc[cg][r];
-                        to[(cg * R + r) * kKeptStride] = float4_t{sum[0], sum[1], sum[2], sum[3]};
-                        sum[0] = sum[1] = sum[2] = sum[3] = 0.f;
-                    }
-            }
-        }
         float dh[4];   // the first half's sums leave their chain for acc (no bias term yet)
         auto fold_scales = [&] {
 #pragma unroll
@@ -703,22 +687,32 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
 }
 
 // grid (row chunks, column groups of 256 over all segments, k-slices), so that an XCD's L2 keeps its share of the image, or as
-// row_ways has it; 256 threads.
-template <int R, int KINDS, bool HALVES = false>
-__global__ void __launch_bounds__(256, 2)
+// row_ways has it; 256 threads a team.
+// Two teams take half a slice each on operands of their own and add up through LDS: where a compute unit has one workgroup, a second wave a
+// SIMD issues beside the first, and a slice rounds as two while its planes, and the next operator's reads of them, are those of one.  (R = 1, one
+// wave a SIMD 5840 clocks a block, two 8170 for both.  One team taking both halves one after the other, and twice the slices where that was
+// faster, blocks of 12B shapes, us, so / by teams: 10 rows 92.5 / 89.0, 20 rows 105.2 / 102.6, 96 rows 168.5 / 165.8, 128 rows 199.0 / 196.2; of
+// Q4_K alone 37 rows 116.8 / 113.8, 100 rows 183.0 / 174.0.  52 to 64 rows lose a little, 140.3 / 141.4.)
+template <int R, int KINDS, int TEAMS = 1>
+__global__ void __launch_bounds__(256 * TEAMS, 2)
 prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const uint8_t* __restrict__ blob,
                     uint32_t M, uint32_t K, uint32_t n0, uint32_t n1, uint32_t n2, uint32_t form, float* __restrict__ y0,
                     float* __restrict__ y1, float* __restrict__ y2) {
-    __shared__ __attribute__((aligned(16))) uint8_t stage[Stage<R>::kBytes];
+    // (two stages pass what a kernel may declare for itself)
+    __shared__ __attribute__((aligned(16))) uint8_t one[TEAMS == 1 ? Stage<R>::kBytes : 16];
+    extern __shared__ __attribute__((aligned(16))) uint8_t two[];
+    uint8_t* const stages = TEAMS == 1 ? one : two;
     const ImageLayout L = image_layout(M, K);
-    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wv = wave & 3, team = TEAMS == 1 ? 0u : wave >> 2;
+    uint8_t* const stage = stages + team * Stage<R>::kBytes;
     const GemmPlace at = place_of<R>(M, n0, n1, n2, form);
     const uint32_t slices = form & ((1u << kSliceBits) - 1);
     if (at.slice >= slices) return;
     const GemmSegment seg = segment_of(at.group, t0, t1, t2, n0, n1, n2, form, y0, y1, y2);
     const uint32_t tile_index = seg.first + wv, nblk = K / 256, rt0 = at.chunk * R;
     const bool valid = tile_index < seg.columns;   // a wave past the last tile works on tile 0 and stores nothing
-    const uint32_t b0 = at.slice * nblk / slices, b1 = (at.slice + 1) * nblk / slices;
+    const uint32_t part = TEAMS * at.slice + team, parts = TEAMS * slices;
+    const uint32_t b0 = part * nblk / parts, b1 = (part + 1) * nblk / parts;
     Feed<R> feed;
     feed.img = make_resource(blob, static_cast<uint32_t>(L.bytes));
     feed.stage = stage;
@@ -727,7 +721,6 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
     feed.base = rt0 * 2048 + (wv & 1) * (1024 * R);
     feed.wv = wv;
     feed.last = 4 * b1 - 1;
-    extern __shared__ float4_t first_sums[];   // HALVES: [4 R][256 threads]
     // a whole form per format: what they share would have to lie in the same registers for both
     auto run = [&](auto walk, uint32_t bytes) {
         float acc[4][R][4];
@@ -738,35 +731,56 @@ prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ 
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[cg][r][i] = 0.f;
         walk(L, feed, stage, seg.tiles + size_t(valid ? tile_index : 0) * nblk * (kCols * bytes), rt0, b0, b1, acc);
-        if constexpr (HALVES) {
-            const float4_t* from = first_sums + wv * 64 + lane_again();
-#pragma unroll
-            for (int cg = 0; cg < 4; ++cg)
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const float4_t first = from[(cg * R + r) * kKeptStride];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[cg][r][i] = first[i] + acc[cg][r][i];
-                }
-        }
         // the chunks asked for past the end are still on their way into this workgroup's LDS
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (!valid) return;
         const uint32_t N = seg.columns * kCols;
         float* y = seg.y + at.slice * (uint64_t(M) * N);
         const uint32_t lane = lane_again(), col = tile_index * kCols + (lane & 15), row0 = rt0 * 16 + 4 * (lane >> 4);
+        auto store = [&]<int C0, int C1>() {
 #pragma unroll
-        for (int r = 0; r < R; ++r)
+            for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t row = row0 + 16 * r + i;
-                if (row < M)
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t row = row0 + 16 * r + i;
+                    if (row < M)
 #pragma unroll
-                    for (int cg = 0; cg < 4; ++cg) y[size_t(row) * N + col + 16 * cg] = acc[cg][r][i];
-            }
+                        for (int cg = C0; cg < C1; ++cg) y[size_t(row) * N + col + 16 * cg] = acc[cg][r][i];
+                }
+        };
+        if constexpr (TEAMS == 1) {
+            if (valid) store.template operator()<0, 4>();
+        } else {
+            // the team with a block less meets as often as the other one
+            const uint32_t other = part ^ 1u, others = (other + 1) * nblk / parts - other * nblk / parts;
+            for (uint32_t n = 4 * (b1 - b0); n < 4 * others; ++n) asm volatile("s_barrier" ::: "memory");
+            arrive<0>();
+            // a team's sums of two column groups to the other one, which finishes and stores them
+            float4_t* const swap = reinterpret_cast<float4_t*>(stages) + wv * 64 + lane;   // [team][column group][row tile][256]
+            auto finish = [&]<int OWN>() {
+                constexpr int GIVEN = 2 - OWN;
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float(&give)[4] = acc[GIVEN + c][r];
+                        swap[(GIVEN * R + c * R + r) * 256] = float4_t{give[0], give[1], give[2], give[3]};
+                    }
+                arrive<0>();
+                if (!valid) return;
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float4_t more = swap[(OWN * R + c * R + r) * 256];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[OWN + c][r][i] += more[i];
+                    }
+                store.template operator()<OWN, OWN + 2>();
+            };
+            if (team == 0) finish.template operator()<0>(); else finish.template operator()<2>();
+        }
     };
-    auto q4 = [&](auto&&... args) { q4_walk<R, HALVES>(args..., (2 * at.slice + 1) * nblk / (2 * slices), first_sums); };
-    if (KINDS == 1 || (KINDS == 3 && seg.dtype == GUFFIN_Q4_K)) run(q4, block_bytes(GUFFIN_Q4_K));
+    if (KINDS == 1 || (KINDS == 3 && seg.dtype == GUFFIN_Q4_K)) run(q4_walk<R>, block_bytes(GUFFIN_Q4_K));
     else if constexpr (KINDS != 1 && R == 4) run(q6_walk_wide<R>, block_bytes(GUFFIN_Q6_K));
     else if constexpr (KINDS != 1) run(q6_walk<R>, block_bytes(GUFFIN_Q6_K));
 }
@@ -1006,7 +1020,6 @@ uint32_t row_ways(uint32_t chunks, uint32_t units, bool q8) {
     return (dealt + turn - 1) / turn > (even + turn - 1) / turn ? 0 : ways;
 }
 
-constexpr uint32_t kept_bytes(uint32_t R) { return 4 * R * kKeptStride * sizeof(float4_t); }
 int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M, uint32_t K,
                 uint32_t slices, uint32_t R, bool halves) {
     if (count > 3 || slices >= 1u << kSliceBits) return fail(GUFFIN_E_SHAPE, "prefill_gemm: at most three matrices and 31 slices");
@@ -1022,7 +1035,7 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
     }
     if (halves && (kinds != 1 || 2 * slices > K / 256)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: a slice in halves is two blocks of Q4_K at least");
     const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
-    dim3 grid(chunks, groups, slices), block(256);
+    dim3 grid(chunks, groups, slices), block(halves ? 512 : 256);
     const uint32_t units = groups * slices;
     if (const uint32_t ways = row_ways(chunks, units, kinds == 4u)) {
         const uint32_t others = 8 / ways;
@@ -1032,7 +1045,7 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
 #define GUFFIN_PG_ARGS a.tiles[0], a.tiles[1], a.tiles[2], a.blob, a.M, a.K, a.columns[0], a.columns[1], a.columns[2], a.form, a.y[0], a.y[1], a.y[2]
 #define GUFFIN_PG(R_) \
     do { \
-        if (halves) launch((prefill_gemm_kernel<R_, 1, true>), grid, block, kept_bytes(R_), s, GUFFIN_PG_ARGS); \
+        if (halves) launch((prefill_gemm_kernel<R_, 1, 2>), grid, block, 2 * Stage<R_>::kBytes, s, GUFFIN_PG_ARGS); \
         else if (kinds == 1) launch(prefill_gemm_kernel<R_, 1>, grid, block, 0, s, GUFFIN_PG_ARGS); \
         else if (kinds == 2) launch(prefill_gemm_kernel<R_, 2>, grid, block, 0, s, GUFFIN_PG_ARGS); \
         else if (kinds == 3) launch(prefill_gemm_kernel<R_, 3>, grid, block, 0, s, GUFFIN_PG_ARGS); \
@@ -1069,7 +1082,7 @@ constexpr SplitCosts kLong = {{5.0f, 6.2f, 7.5f, 8.5f}, {{0.6f, 0.82f, 1.0f, 1.3
 constexpr float kPlaneRounding[3] = {0.f, 0.54f, 1.2f};
 constexpr float rounding(uint32_t units, uint32_t S, uint32_t halves, float plane) { return float(units) / float(S << halves) + plane * float(S + halves); }
 
-constexpr float kHalvesCost = 0.04f;   // us a row tile: through LDS and back (fitted: 17 to 32 rows keep four slices of gate + up, 20 rows 5169 us instead of 5290)
+constexpr float kHalvesCost = 2.0f;   // us: twice the first trips at once, sums from team to team
 struct SplitShape { uint32_t units, groups, width, most; bool q8; float unit[4]; };   // units: what a slice is made of; unit: of a workgroup, the mean over the launch
 SplitShape split_shape(const PrefillMatrix* m, uint32_t count, uint32_t K, uint32_t most, const SplitCosts& costs) {
     SplitShape s {};
@@ -1101,12 +1114,12 @@ PrefillSplit cheapest_split(const SplitShape& s, const SplitCosts& costs, uint32
             if (best.slices && fixed >= least) break;   // grows with S
             for (uint32_t halves = 0; halves <= most_halves; ++halves) {
                 const uint32_t n = chunks * s.groups * S;
-                // (halves: the sums that wait leave room for one workgroup of three or four row tiles a compute unit)
+                // (halves: two teams are what a compute unit takes)
                 if (!allowed(R, S, halves) || (halves && n > cus)) continue;
                 // the last, partly filled turn overlaps the one before it: half of it counts
-                const float turns = std::max(costs.alone[R - 1], 0.5f * (float((n + cus - 1) / cus) + float(n) / float(cus)));
-                const float cost = fixed + turns * (costs.workgroup + float(halves) * kHalvesCost * float(R)
-                                                    + float((s.units + S - 1) / S) * s.unit[R - 1] / float(s.groups));
+                const float turns = halves ? 1.f : std::max(costs.alone[R - 1], 0.5f * (float((n + cus - 1) / cus) + float(n) / float(cus)));
+                const uint32_t units = halves ? 2 * ((s.units + 2 * S - 1) / (2 * S)) : (s.units + S - 1) / S;   // a team's, each beside the other's
+                const float cost = fixed + float(halves) * kHalvesCost + turns * (costs.workgroup + float(units) * s.unit[R - 1] / float(s.groups));
                 if (!best.slices || cost < least) { best = {R, S, halves}; least = cost; }
             }
         }
@@ -1139,8 +1152,8 @@ PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint3
 }  // namespace
 
 int prefill_gemm_init() {
-    return allow_lds(prefill_gateup_q8_kernel<4>, GatedStage<4>::kBytes) && allow_lds((prefill_gemm_kernel<2, 1, true>), kept_bytes(2))
-        && allow_lds((prefill_gemm_kernel<3, 1, true>), kept_bytes(3)) && allow_lds((prefill_gemm_kernel<4, 1, true>), kept_bytes(4)) ? 0 : -1;
+    return allow_lds(prefill_gateup_q8_kernel<4>, GatedStage<4>::kBytes) && allow_lds((prefill_gemm_kernel<2, 1, 2>), 2 * Stage<2>::kBytes)
+        && allow_lds((prefill_gemm_kernel<3, 1, 2>), 2 * Stage<3>::kBytes) && allow_lds((prefill_gemm_kernel<4, 1, 2>), 2 * Stage<4>::kBytes) ? 0 : -1;
 }
 
 // The fewest row tiles a workgroup with which every workgroup has a compute unit, as long as more than half of them have work: a

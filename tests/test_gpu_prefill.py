@@ -768,3 +768,10 @@ def test_a_run_without_head_norms(hip, q_norm, k_norm):
     assert int(status.item()) == 0 and int(st.item()) == 0
     want = one.cpu().numpy().astype(np.float64)[0]
     assert np.max(np.abs(hidden[19].cpu().numpy() - want)) <= 2e-4 * np.sqrt((want ** 2).mean())
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("rows", [6, 16, 17, 32, 33, 72, 80, 97, 100])
+def test_two_teams_a_workgroup(hip, rows, mixed):
+    """Where a workgroup's two teams take half a slice each: of 15 blocks in two and four slices the teams' shares differ by a block."""
+    test_a_short_run_s_splits_are_those_of_shorter_runs(hip, rows, mixed)
