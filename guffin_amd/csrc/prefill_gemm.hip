@@ -477,6 +477,22 @@ __device__ __forceinline__ void q6_scaled(const uint32_t (&scw)[4], half8_t (&q)
     if constexpr (C0 == 0) two.template operator()<0>();
     if constexpr (C1 == 4) two.template operator()<1>();
 }
+// the same of one column group
+template <int QD, int CG>
+__device__ __forceinline__ void q6_scaled_one(const uint32_t (&scw)[4], half8_t& q, half8_t& rest) {
+    const half2_t s = both<CG & 1>(h2(__builtin_amdgcn_perm(0x64646464u, scw[2 * (CG >> 1) + (QD >> 1)], pair_bytes(QD & 1))) - splat(1152.f));
+    const uint4 v = __builtin_bit_cast(uint4, q);
+    const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+    uint32_t p[4], r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const half2_t prod = s * h2(x[k]);
+        p[k] = u2(prod);
+        r[k] = u2(__builtin_elementwise_fma(s, h2(x[k]), -prod));
+    }
+    q = as_half8(p[0], p[1], p[2], p[3]);
+    rest = as_half8(r[0], r[1], r[2], r[3]);
+}
 // a half block's scale words from the waves' headers: lanes of k-slices 0, 1 take a group's first scale, of 2, 3 its second
 __device__ __forceinline__ void q6_scale_words(const uint8_t* head, int half, uint32_t j, uint32_t sel, uint32_t (&sc)[4]) {
 #pragma unroll
@@ -591,9 +607,10 @@ __device__ __forceinline__ void q6_walk(const ImageLayout& L, const Feed<R>& fee
     } while (++blk < b1);
 }
 
-// The same for four row tiles, where the accumulators leave no registers for operands formed ahead: column groups by pairs,
-// the compiler's order, and the second wave of the SIMD to fill the gaps (the woven form spills: 2048 x 15360 x 3840 takes
-// 772 us instead of 614).  The workgroup meets at a chunk's start; the chunk after the next is asked for there.
+// The same for four row tiles, where the accumulators leave no registers for a whole group's operands formed ahead: a region takes one
+// column group, its rest and its products with hi and lo, while the next column group's operands are formed; the compiler's order
+// inside a region and the second wave of the SIMD fill the gaps.  2048 x 15360 x 3840, us, two column groups' operands formed ahead of their
+// products / so: 521 / 504 (575 / 560 on a part whose clock falls further); 25.8 clocks a matrix instruction at 2.45 vector instructions.
 template <int R>
 __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed, uint8_t* stage, const uint8_t* tile_base,
                                              uint32_t rt0, uint32_t b0, uint32_t b1, float (&acc)[4][R][4]) {
@@ -608,6 +625,7 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
     uint4 ql[2][4];
     uint2 qh[2][4];
     uint32_t sc[4];
+    half8_t hi[R], lo[R], b[4], rest[4];
     float4_t D[4][R];
     auto ask_half = [&](uint32_t blk, int h) {
 #pragma unroll
@@ -621,47 +639,64 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
         to_lds4(tile, heads + (blk & 1) * 5120 + 1024, lane < 32 ? lane * 4 : 0, blk * TB + 13312);
     };
     auto scales = [&](uint32_t blk, int half) { q6_scale_words(heads + (blk & 1) * 5120, half, j, sel, sc); };
+    auto form = [&]<int G, int CG>() {
+        q6_quants<G & 3, CG, CG + 1>(ql[(G & 7) >> 2], qh[(G & 7) >> 2], b);
+        q6_scaled_one<G & 3, CG>(sc, b[CG], rest[CG]);
+    };
     ask_half(b0, 0);
     ask_head(b0);
     feed.ask(4 * b0, 0);
-    asm volatile("" ::: "memory");
+    in_order();
     feed.ask(4 * b0 + 1, 1);
-    uint32_t rd = 0, wr = 2, blk = b0;
+    in_order();
+    ask_half(b0, 1);
+    in_order();
+    feed.ask(4 * b0 + 2, 2);
+    arrive<2 * R + kHalf>();
+    scales(b0, 0);
+    read_half<R>(stage, 0, lane16, hi);
+    form.template operator()<0, 0>();
+    uint32_t rd = 0, blk = b0;
     do {
         lane = lane_again(); j = lane & 15; lg = lane >> 4; lane16 = feed.lane16 = lane * 16;   // no register to keep addresses in
         sel = lane >= 32 ? 0x07030501u : 0x06020400u;
-        const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;
+        const uint32_t next = blk + 1 < b1 ? blk + 1 : blk;   // the last block asks for itself again
         auto group = [&]<int G>() {
-            constexpr int H = G >> 2, QD = G & 3;
-            if constexpr ((G & 1) == 0) {
-                // the last meeting's requests may still be on their way: a chunk and, at 2 and 6, a half block's quants, at 4 a header
-                arrive<R + (G == 0 ? 0 : G == 4 ? 2 : kHalf)>();
-                if constexpr (G == 0) {
-                    if (wv == 2) to_lds4(feed.img, stage + S::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (blk * L.mpad + rt0 * 16) * 4);
-                    ask_half(blk, 1);
-                    scales(blk, 0);
-                }
-                if constexpr (G == 2) ask_head(next);
-                if constexpr (G == 4) { ask_half(next, 0); scales(blk, 1); }
-                asm volatile("" ::: "memory");
-                feed.ask(4 * blk + (G >> 1) + 2, wr);
-                asm volatile("" ::: "memory");
-            }
-            const uint8_t* from = stage + rd * S::kChunk + (G & 1) * (2048 * R);
-            half8_t hi[R], lo[R], b[4], rest[4];
-            read_half<R>(from, 0, lane16, hi);
-            read_half<R>(from, 1, lane16, lo);
-            auto pair = [&]<int C>() {
-                q6_quants<QD, C, C + 2>(ql[H], qh[H], b);
-                q6_scaled<QD, C, C + 2>(sc, b, rest);
-                products<R, G == 0, C, C + 2>(hi, b, D);
-                products<R, false, C, C + 2>(lo, b, D);
-                products<R, false, C, C + 2>(hi, rest, D);
+            const uint8_t* now = stage + rd * S::kChunk + (G & 1) * (2048 * R);
+            auto column = [&]<int CG>() {
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (CG == 0) read_half<R>(now, 1, lane16, lo);
+                form.template operator()<G, CG + 1>();
+                products<R, G == 0, CG, CG + 1>(hi, rest, D);
+                products<R, false, CG, CG + 1>(hi, b, D);
+                products<R, false, CG, CG + 1>(lo, b, D);
             };
-            pair.template operator()<0>();
+            column.template operator()<0>();
+            column.template operator()<1>();
+            column.template operator()<2>();
+            if constexpr (G == 3) ask_half(next, 0);   // the half's last operands are formed
+            if constexpr (G == 7) ask_half(next, 1);
+            if constexpr ((G & 3) == 3) in_order();
+            if constexpr (G == 3) scales(blk, 1);
+            if constexpr (G == 7) scales(next, 0);
             __builtin_amdgcn_sched_barrier(0);
-            pair.template operator()<2>();
-            if constexpr (G & 1) { rd = rd == 2 ? 0 : rd + 1; wr = wr == 2 ? 0 : wr + 1; }
+            form.template operator()<G + 1, 0>();
+            products<R, G == 0, 3, 4>(hi, rest, D);
+            products<R, false, 3, 4>(hi, b, D);
+            if constexpr (G & 1) {
+                arrive<R + kHalf + (G == 3 ? 2 : 0)>();   // as the walk above
+                if constexpr (G == 1) {
+                    if (wv == 2) to_lds4(feed.img, stage + S::kMult, lane * 4, static_cast<uint32_t>(L.mult_off) + (blk * L.mpad + rt0 * 16) * 4);
+                    in_order();
+                }
+                feed.ask(4 * blk + (G >> 1) + 3, rd);
+                if constexpr (G == 1) { in_order(); ask_head(next); }
+                rd = rd == 2 ? 0 : rd + 1;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            read_half<R>(stage + rd * S::kChunk + ((G + 1) & 1) * (2048 * R), 0, lane16, hi);
+            products<R, false, 3, 4>(lo, b, D);
+            __builtin_amdgcn_sched_barrier(0);
         };
         group.template operator()<0>();
         group.template operator()<1>();
@@ -683,6 +718,7 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[cg][r][i] = fmaf(d[cg] * mult[i], D[cg][r][i], acc[cg][r][i]);
         }
+        __builtin_amdgcn_sched_barrier(0);
     } while (++blk < b1);
 }
 
@@ -1136,10 +1172,8 @@ PrefillSplit split_for(const PrefillMatrix* m, uint32_t count, uint32_t M, uint3
     const PrefillSplit bar[2] = {cheapest_split(shape, kLong, last - 15, any), cheapest_split(shape, kLong, last, any)};
     bool q4 = true;
     for (uint32_t i = 0; i < count; ++i) q4 &= m[i].dtype == GUFFIN_Q4_K;
-    // (Q6_K in four row tiles adds up in another order, 1 % further off: q6_walk_wide)
-    const uint32_t tallest = q4 || (bar[0].row_tiles == 4 && bar[1].row_tiles == 4) ? 4 : 3;
-    auto close = [&](uint32_t R, uint32_t S, uint32_t halves) {
-        if (R > tallest || (halves && 2 * S > std::max(bar[0].slices, bar[1].slices))) return false;   // halves stand for two of its slices
+    auto close = [&](uint32_t, uint32_t S, uint32_t halves) {
+        if (halves && 2 * S > std::max(bar[0].slices, bar[1].slices)) return false;   // halves stand for two of its slices
         for (uint32_t i = 0; i < count; ++i)
             for (const PrefillSplit& b : bar)
                 if (rounding(shape.units, S, halves, kPlaneRounding[m[i].dtype]) > rounding(shape.units, b.slices, 0, kPlaneRounding[m[i].dtype])) return false;
