@@ -775,3 +775,17 @@ def test_a_run_without_head_norms(hip, q_norm, k_norm):
 def test_two_teams_a_workgroup(hip, rows, mixed):
     """Where a workgroup's two teams take half a slice each: of 15 blocks in two and four slices the teams' shares differ by a block."""
     test_a_short_run_s_splits_are_those_of_shorter_runs(hip, rows, mixed)
+
+
+@pytest.mark.parametrize("K,N", [(256, 64), (512, 320), (768, 64), (2048, 640), (288, 64)])
+@pytest.mark.parametrize("M", [3, 16, 17, 40, 300, 1000])
+def test_q8_spans(hip, gfo, K, N, M):
+    """Spans of 256 whose blocks add up before the row's multiplier, one and several of them, and spans of one block; rows and blocks of
+    very different size.  Bar: as for row tiles."""
+    w = synth.make_weight(0, K, N, seed=K)
+    x = synth.make_activation(M, K, seed=M)
+    x[M - 1] *= 1e4
+    x[:, K // 2:] *= 1e-3
+    tiles = hip.repack(0, dev(w), K, N)
+    y = hip.prefill_gemm(0, tiles, hip.prefill_pack(dev(x)), M, K, N).cpu().numpy()
+    assert_within_operator_bound(gfo, 0, w, x, y, K, N, matrix_path=True)
