@@ -359,3 +359,17 @@ def test_norm_pair_over_any_number_of_waves(hip, width, planes):
         assert float(err.max()) <= 12 * 2.0 ** -24
     huge = run((x if planes > 1 else x[0]) * 1e25)
     assert torch.equal(huge[0].cpu(), res)
+
+
+@pytest.mark.parametrize("rows_of", [0.0, 1e-20])
+def test_norm_pair_of_rows_and_an_epsilon_below_the_normal_floats(hip, rows_of):
+    """1 / sqrt(1e-40) and the like are ordinary floats, so a row of zeros stays one and a tiny row comes out as in 64 bits; the mean itself
+    is a denormal of 2^-149's places, half of one of which in 1e-40 is 2^-18 of it, and twice a root's half of that is allowed."""
+    import torch
+    gen = torch.Generator().manual_seed(5)
+    x = rows_of * torch.randn(2, 3840, generator=gen)
+    res, ones = torch.zeros(2, 3840), torch.ones(3840)
+    got = hip.rms_norm_add_norm(x.cuda(), ones.cuda(), res.cuda(), ones.cuda(), eps=1e-40)
+    want = x.double() / ((x.double() ** 2).mean(-1, keepdim=True) + 1e-40).sqrt()
+    err = (got[0].cpu().double() - want).abs().max()
+    assert float(err) <= 2.0 ** -18 * float(want.abs().max())
