@@ -844,36 +844,6 @@ ShortRun short_run_layout(const guffin_model_desc& m, uint32_t rows, uint32_t po
     return r;
 }
 
-int check_ring_alignment(const guffin_model_desc& m) {
-    for (uint32_t l = 0; l < m.layer_count; ++l)
-        if ((reinterpret_cast<uintptr_t>(m.layers[l].ring_k) | reinterpret_cast<uintptr_t>(m.layers[l].ring_v)) & 3u)
-            return fail(GUFFIN_E_ALIGN, "prefill_rows: ring rows must be 4-byte aligned");
-    return GUFFIN_OK;
-}
-
-// A short run of a model that the drafter's pass covers: passes of up to eight rows side by side, each followed by its K/V rows' way to the
-// rings.  A pass costs what its chain of phases costs, the tiled form its 9 launches a block whatever they do.  270M shapes, us, tiled / so: 2
-// rows at 0 670 / 227, 8 rows at 0, 700 and 4000 719 / 246, 803 / 279, 818 / 298, 9 rows at 0 723 / 466, 16 rows at the same 736 / 490, 816 /
-// 554, 834 / 594; three passes would be no less than the tiled form: 24 rows 731, 816 and 833.
-constexpr uint32_t kRowRuns = 2 * kRunRows;
-struct RowRuns { uint8_t* pass; uint16_t *priv_k, *priv_v; uint64_t bytes; };
-bool row_runs_fit(const guffin_model_desc& m, uint32_t rows) {
-    return rows <= kRowRuns && rows <= m.ring_local && rows <= m.ring_global && drafter_pass_fits(m);
-}
-RowRuns row_runs_layout(const guffin_model_desc& m, uint8_t* base) {
-    Arena ar {base, 0, 0};
-    const uint64_t words = uint64_t(m.layer_count) * kRunRows * m.kv_heads * m.head_dim;
-    RowRuns r {};
-    r.pass = ar.take<uint8_t>(forward_run_bytes(m));
-    r.priv_k = ar.take<uint16_t>(words);
-    r.priv_v = ar.take<uint16_t>(words);
-    r.bytes = (ar.used + 255) & ~uint64_t{255};
-    return r;
-}
-uint64_t with_row_runs(const guffin_model_desc& m, uint32_t rows, uint64_t bytes) {
-    return row_runs_fit(m, std::min(rows, kRowRuns)) ? std::max(bytes, row_runs_layout(m, nullptr).bytes) : bytes;
-}
-
 __global__ void fill_positions_kernel(uint32_t* positions, uint32_t rows, uint32_t position) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < rows) positions[i] = position + i;
@@ -884,13 +854,12 @@ __global__ void fill_positions_kernel(uint32_t* positions, uint32_t rows, uint32
 
 extern "C" uint64_t guffin_hip_prefill_scratch_bytes(const guffin_model_desc* model, uint32_t rows) {
     if (!model || rows == 0 || guffin::validate_model(model)) return 0;
-    return guffin::with_row_runs(*model, rows, guffin::prefill_layout(*model, rows, guffin::prefill_most_pieces(*model, rows), nullptr).bytes);
+    return guffin::prefill_layout(*model, rows, guffin::prefill_most_pieces(*model, rows), nullptr).bytes;
 }
 
 extern "C" uint64_t guffin_hip_prefill_run_bytes(const guffin_model_desc* model, uint32_t rows) {
     if (!model || rows == 0 || guffin::validate_model(model)) return 0;
-    const uint64_t bytes = guffin::prefill_layout(*model, rows, guffin::prefill_pieces(*model, rows), nullptr).bytes;
-    return rows <= guffin::kRowRuns ? guffin::with_row_runs(*model, rows, bytes) : bytes;
+    return guffin::prefill_layout(*model, rows, guffin::prefill_pieces(*model, rows), nullptr).bytes;
 }
 
 extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* model, const uint32_t* tokens,
@@ -910,23 +879,12 @@ extern "C" int guffin_hip_prefill_rows(void* stream, const guffin_model_desc* mo
         uint8_t* base = static_cast<uint8_t*>(scratch);
         const ShortRun r = short_run_layout(m, rows, position, base);
         if (r.bytes <= scratch_bytes) {
-            GUFFIN_TRY(check_ring_alignment(m));
+            for (uint32_t l = 0; l < m.layer_count; ++l)
+                if ((reinterpret_cast<uintptr_t>(m.layers[l].ring_k) | reinterpret_cast<uintptr_t>(m.layers[l].ring_v)) & 3u)
+                    return fail(GUFFIN_E_ALIGN, "prefill_rows: ring rows must be 4-byte aligned");
             GUFFIN_TRY(forward_rows(hs, m, tokens, rows, position, layout(m, rows, position, base, false), r.priv_k, r.priv_v, out_hidden, nullptr, status));
             const uint32_t path[kWideRows] = {0, 1, 2, 3};
             return kv_move_rows(hs, m, KvMove::Put, nullptr, nullptr, 0, position, rows, r.priv_k, r.priv_v, rows, path);
-        }
-    }
-    if (g_forward_mode == 0 && forward_run_chosen(m) && row_runs_fit(m, rows)) {
-        const RowRuns r = row_runs_layout(m, static_cast<uint8_t*>(scratch));
-        if (r.bytes <= scratch_bytes) {
-            GUFFIN_TRY(check_ring_alignment(m));
-            for (uint32_t at = 0; at < rows; at += kRunRows) {
-                const uint32_t n = std::min(kRunRows, rows - at), path[kRunRows] = {0, 1, 2, 3, 4, 5, 6, 7};
-                GUFFIN_TRY(forward_run(hs, m, tokens + at, n, position + at, r.pass, r.priv_k, r.priv_v, out_hidden + size_t(at) * m.hidden, nullptr,
-                                       nullptr, status));
-                GUFFIN_TRY(kv_move_rows(hs, m, KvMove::Put, nullptr, nullptr, 0, position + at, n, r.priv_k, r.priv_v, n, path));
-            }
-            return GUFFIN_OK;
         }
     }
     const uint32_t H = m.hidden, QW = m.q_heads * m.head_dim, KW = m.kv_heads * m.head_dim;

@@ -242,57 +242,3 @@ def test_rings_that_lie_off_16_bytes(hip, off):
     torch.cuda.synchronize()
     assert int(got[4].item()) == 0 and hip.lib().guffin_hip_resident_enabled() == 1
     assert torch.equal(got[0], want)
-
-
-# first position, rows, local ring, window: pieces of eight rows and what is left of them, one row more than two pieces take (the tiled
-# form on both sides), behind a ring that wraps inside the run, a window shorter than the run, and the longest list of a chunk and more
-@pytest.mark.parametrize("position,rows,ring,window", [(0, 2, 128, 48), (0, 7, 128, 48), (120, 8, 128, 48), (122, 9, 128, 48), (250, 16, 128, 48),
-                                                       (0, 16, 16, 5), (11, 15, 16, 16), (60, 17, 128, 48), (1990, 13, 512, 512)])
-def test_short_prefill_runs_equal_the_tiled_form(hip, position, rows, ring, window):
-    """Hidden rows to 2e-4 of their RMS (fp32 sums of exact products in another order, fp16 K/V rows that may round the other way), the
-    rings' rows up to such ties and untouched where the run has none."""
-    import torch
-    from guffin_amd import model
-    shape = replace(model.GEMMA3_270M, layers=6, vocab=2048, ring_global=2048, ring_local=ring, sliding_window=window)
-    devm = model.DeviceModel.random(shape, seed=rows, position=position)
-    rings = [r.clone() for r in devm.ring_k + devm.ring_v]
-    tokens = torch.from_numpy(np.random.default_rng(rows).integers(2, shape.vocab, rows).astype(np.int32)).cuda()
-    out = []
-    print("prefill run", position, rows, ring, window, flush=True)
-    for mode in (1, 0):
-        for ring_now, before in zip(devm.ring_k + devm.ring_v, rings):
-            ring_now.copy_(before)
-        hip.set_forward_mode(mode)
-        hidden, status = devm.prefill(tokens, position)
-        torch.cuda.synchronize()
-        assert int(status.item()) == 0 and hip.lib().guffin_hip_resident_enabled() == 1
-        out.append((hidden.cpu().numpy().astype(np.float64), [r.clone() for r in devm.ring_k + devm.ring_v]))
-    hip.set_forward_mode(0)
-    scale = np.sqrt((out[0][0] ** 2).mean(axis=-1, keepdims=True))
-    assert np.max(np.abs(out[1][0] - out[0][0]) / scale) <= 2e-4
-    for i, (a, b) in enumerate(zip(out[0][1], out[1][1])):
-        cap = a.shape[0]
-        written = torch.zeros(cap, dtype=torch.bool, device="cuda")
-        written[[(position + r) & (cap - 1) for r in range(rows)]] = True
-        assert torch.equal(b[~written], rings[i][~written])
-        assert float((a[written] == b[written]).float().mean()) >= 0.95
-        assert torch.allclose(a[written].view(torch.float16).float(), b[written].view(torch.float16).float(), rtol=2.0 ** -9, atol=1e-3)
-
-
-def test_a_prefill_arena_of_the_tiled_form_alone(hip):
-    """An arena that was sized for no passes takes the tiled form, to the bit."""
-    import ctypes as C
-    import torch
-    from guffin_amd import model
-    shape = replace(model.GEMMA3_270M, layers=6, vocab=2048, ring_global=256, ring_local=128, sliding_window=48)
-    devm = model.DeviceModel.random(shape, seed=3, position=0)
-    tokens = torch.tensor([5, 9, 700], dtype=torch.int32, device="cuda")
-    hip.set_forward_mode(1)
-    want = devm.prefill(tokens, 0)[0]
-    hip.set_forward_mode(0)
-    other = devm.prefill(tokens, 0)[0]
-    nbytes = hip._calls.guffin_hip_prefill_run_bytes(C.byref(devm.desc), 3) - 256
-    arena, got, status = torch.empty(nbytes, dtype=torch.uint8, device="cuda"), torch.empty_like(want), hip.new_status()
-    hip.check(hip._calls.guffin_hip_prefill_rows(hip._raw_stream(), C.byref(devm.desc), tokens.data_ptr(), 3, 0, arena.data_ptr(), nbytes,
-                                                 got.data_ptr(), status.data_ptr()))
-    assert int(status.item()) == 0 and torch.equal(got, want) and not torch.equal(other, want)

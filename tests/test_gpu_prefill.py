@@ -770,6 +770,34 @@ def test_a_run_without_head_norms(hip, q_norm, k_norm):
     assert np.max(np.abs(hidden[19].cpu().numpy() - want)) <= 2e-4 * np.sqrt((want ** 2).mean())
 
 
+@pytest.mark.parametrize("rows", [2, 8, 9, 16])
+def test_a_drafter_s_short_prompt_waits_for_nobody(hip, rows):
+    """A run of prompt rows is ordinary launches, also where the model's decode rows go through a pass whose workgroups wait for each
+    other: waits that all give up at once leave its rows, its rings and its status word what they are."""
+    import torch
+    from dataclasses import replace
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=3, vocab=2048, ring_global=512, ring_local=128, sliding_window=48)
+    devm = model.DeviceModel.random(shape, seed=rows, position=130)
+    rings = [r.clone() for r in devm.ring_k + devm.ring_v]
+    tokens = dev(np.random.default_rng(rows).integers(2, shape.vocab, rows).astype(np.int32))
+    out = []
+    print("drafter prompt, spin limit 0", rows, flush=True)
+    try:
+        for polls in (1 << 20, 0):
+            for now, before in zip(devm.ring_k + devm.ring_v, rings):
+                now.copy_(before)
+            hip.set_spin_limit(polls)
+            hidden, status = devm.prefill(tokens, 130)
+            torch.cuda.synchronize()
+            assert int(status.item()) == 0
+            out.append([hidden] + [r.clone() for r in devm.ring_k + devm.ring_v])
+    finally:
+        hip.set_spin_limit(1 << 20)
+        hip.set_forward_mode(0)
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("rows", [6, 16, 17, 32, 33, 72, 80, 97, 100])
 def test_two_teams_a_workgroup(hip, rows, mixed):
