@@ -1096,6 +1096,12 @@ uint32_t row_ways(uint32_t chunks, uint32_t units, bool q8) {
     return (dealt + turn - 1) / turn > (even + turn - 1) / turn ? 0 : ways;
 }
 
+// (columns come by 64, planes lie in arenas of 256 bytes)
+__global__ void __launch_bounds__(256) zero_planes_kernel(float* planes, uint64_t quads) {
+    const uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (i < quads) reinterpret_cast<float4_t*>(planes)[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+}
+
 int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uint8_t* image, float* const* y, uint32_t M, uint32_t K,
                 uint32_t slices, uint32_t R, bool halves) {
     if (count > 3 || slices >= 1u << kSliceBits) return fail(GUFFIN_E_SHAPE, "prefill_gemm: at most three matrices and 31 slices");
@@ -1110,6 +1116,7 @@ int gemm_launch(hipStream_t s, const PrefillMatrix* m, uint32_t count, const uin
         kinds |= m[i].dtype == GUFFIN_Q4_K ? 1u : m[i].dtype == GUFFIN_Q6_K ? 2u : 4u;
     }
     if (halves && (kinds != 1 || 2 * slices > K / 256)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: a slice in halves is two blocks of Q4_K at least");
+    if (kinds != 4 && slices > K / 256) return fail(GUFFIN_E_SHAPE, "prefill_gemm: a slice of a K-quant is a block at least");   // its walk begins with one unasked
     const uint32_t chunks = (M + 16 * R - 1) / (16 * R);
     dim3 grid(chunks, groups, slices), block(halves ? 512 : 256);
     const uint32_t units = groups * slices;
@@ -1276,8 +1283,15 @@ int prefill_gemm_planes(hipStream_t s, const PrefillMatrix* m, uint32_t count, c
     }
     if (image_layout(M, K).bytes >= (size_t(1) << 31)) return fail(GUFFIN_E_SHAPE, "prefill_gemm: the image of M x K exceeds 2 GiB, split the rows");
     if (q8 && k) {   // the formats' workgroups walk K in different units: a launch each
-        for (uint32_t i = 0; i < count; ++i)
-            if (int rc = prefill_gemm_planes(s, m + i, 1, image, y + i, M, K, split)) return rc;
+        for (uint32_t i = 0; i < count; ++i) {
+            // The cut is by Q8_0's finer units.  Where it has more slices than a K-quant has blocks, each block is a slice of its own, in order,
+            // and the planes behind them are zeros: so the kernels, whose walks have a block at least, need no test of their own.
+            const uint32_t blocks = m[i].dtype == GUFFIN_Q8_0 ? split.slices : std::min(split.slices, K / 256);
+            if (int rc = prefill_gemm_planes(s, m + i, 1, image, y + i, M, K, {split.row_tiles, blocks, split.halves})) return rc;
+            const uint64_t plane = uint64_t(M) * m[i].N, quads = (split.slices - blocks) * plane / 4;
+            if (quads) launch(zero_planes_kernel, dim3(static_cast<uint32_t>((quads + 255) / 256)), dim3(256), 0, s, y[i] + blocks * plane, quads);
+            if (int rc = check_launch("prefill_gemm planes")) return rc;
+        }
         return GUFFIN_OK;
     }
     return gemm_launch(s, m, count, image, y, M, K, split.slices, split.row_tiles, split.halves);

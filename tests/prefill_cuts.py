@@ -30,16 +30,16 @@ def bar(name, rows):
     return [s for first, s in BAR[name] if first <= rows][-1]
 
 
-def matrices(name):
-    K, parts = PRODUCTS[name]
-    return K, (Matrix * len(parts))(*[Matrix(dtype, None, n) for dtype, n in parts])
+def cut_of(K, parts, rows):
+    """The library's cut of a run of `rows` through one launch of `parts` ((format, N))."""
+    f = hip.lib()._ZN6guffin13prefill_splitEPKNS_13PrefillMatrixEjjj
+    f.argtypes, f.restype = [C.POINTER(Matrix), C.c_uint32, C.c_uint32, C.c_uint32], Split
+    return f((Matrix * len(parts))(*[Matrix(dtype, None, n) for dtype, n in parts]), len(parts), rows, K)
 
 
 def split(name, rows):
-    f = hip.lib()._ZN6guffin13prefill_splitEPKNS_13PrefillMatrixEjjj
-    f.argtypes, f.restype = [C.POINTER(Matrix), C.c_uint32, C.c_uint32, C.c_uint32], Split
-    K, m = matrices(name)
-    return f(m, len(m), rows, K)
+    K, parts = PRODUCTS[name]
+    return cut_of(K, parts, rows)
 
 
 def planes(parts, image, M, K, cut):

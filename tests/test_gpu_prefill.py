@@ -101,6 +101,31 @@ def test_a_slice_in_halves_is_the_sum_of_two_slices(hip, M, row_tiles, K, slices
     assert torch.equal(whole, parts[0::2] + parts[1::2])
 
 
+@pytest.mark.parametrize("K,rows", [(1024, 5), (1024, 40), (1024, 100), (2048, 16), (2048, 33), (2048, 40)])
+def test_more_slices_than_blocks(hip, K, rows):
+    """q, k and v of one block in three formats: the launch is cut by Q8_0's units of 64, which leaves slices of the others without a
+    block (looked at first).  Such a plane is zeros to the bit; the planes' sums are held to the bar of the other cuts, against 64 bits."""
+    import torch
+    from prefill_cuts import Split, cut_of, planes
+    formats = ((1, 1024), (2, 256), (0, 256))
+    cut = cut_of(K, formats, rows)
+    assert cut.slices > K // 256
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows)
+    x = torch.randn((rows, K), device="cuda", generator=gen)
+    weights = [dev(synth.make_weight(dtype, K, N, seed=dtype)) for dtype, N in formats]
+    parts = [(dtype, hip.repack(dtype, w, K, N), N) for w, (dtype, N) in zip(weights, formats)]
+    for row_tiles in (cut.row_tiles, 1, 2, 3, 4):
+        print("more slices than blocks", K, rows, row_tiles, cut.slices, flush=True)
+        for w, (dtype, N), y in zip(weights, formats, planes(parts, hip.prefill_pack(x), rows, K, Split(row_tiles, cut.slices, 0))):
+            if dtype:
+                assert int((y == 0).all(2).all(1).sum()) == cut.slices - K // 256
+            want = x.double() @ hip.dequant(dtype, w, N * K // synth.BLOCK_ELEMS[dtype]).view(N, K).double().T.contiguous()
+            got = y.double().sum(0)
+            assert float(((got - want).pow(2).mean() / want.pow(2).mean()).sqrt()) <= 4e-7
+            assert float((got - want).abs().max() / want.pow(2).mean().sqrt()) <= 1e-5
+
+
 @pytest.mark.parametrize("name,rows", [("gate_up", 24), ("gate_up", 37), ("gate_up", 55), ("gate_up", 64), ("gate_up", 100), ("gate_up", 144),
                                        ("qkv4", 80), ("qkv4", 176), ("down4", 150), ("o", 20), ("o", 40), ("o", 104), ("down", 60)])
 def test_a_short_run_s_sums_are_as_close_as_in_the_long_runs_slices(hip, name, rows):
