@@ -241,6 +241,8 @@ __device__ __forceinline__ float sum_of_waves(const float* at, uint32_t stride, 
 // 1 / sqrt(mean + eps) of a sum of squares, per_width = 1 / width.  The root's reciprocal (an ulp) and one step of Newton's: no
 // further off than a division, a root and a division, which are 40 instructions behind each other where a norm waits for them.
 // The instruction takes a denormal for zero; a row of zeros with an epsilon as small as that goes 2^24 times as large, beside the other.
+// (A value meets this factor ahead of its gamma: the row's values by it are at most the root of its width, where a value times a gamma can
+// pass either end of the floats.)
 __device__ __forceinline__ float inverse_rms(float sum, float per_width, float eps) {
     const float mean = fmaf(sum, per_width, eps);
     const float y = mean < 0x1p-126f ? __builtin_amdgcn_rsqf(mean * 0x1p24f) * 0x1p12f : __builtin_amdgcn_rsqf(mean);

@@ -700,21 +700,17 @@ struct Pass {
         return inverse_rms(lanes_sum(all), per_width, a.eps);
     }
     // x = x + rms(v, post), then rms(x, next) for the workers.  outputs: also written to memory (the state after the launch's last block).
-    __device__ __forceinline__ void norm_pair(RowQuads v, const RowQuads& post, RowQuads next, RowQuads& x, bool outputs) const {
+    __device__ __forceinline__ void norm_pair(const RowQuads& v, const RowQuads& post, const RowQuads& next, RowQuads& x, bool outputs) const {
         const uint32_t H = a.H;
         float inv = over_rms(v);
 #pragma unroll
-        for (int i = 0; i < kQuads; ++i) v.v[i] *= post.v[i];
-#pragma unroll
         for (int i = 0; i < kQuads; ++i)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) x.v[i][k] = fmaf(v.v[i][k], inv, x.v[i][k]);
+            for (int k = 0; k < 4; ++k) x.v[i][k] = fmaf(v.v[i][k] * inv, post.v[i][k], x.v[i][k]);
         inv = over_rms(x);
 #pragma unroll
-        for (int i = 0; i < kQuads; ++i) next.v[i] *= x.v[i];
-#pragma unroll
         for (int i = 0; i < kQuads; ++i) {
-            const f4_t u = next.v[i] * inv;
+            const f4_t u = x.v[i] * inv * next.v[i];
             if (mine(i)) {
                 *reinterpret_cast<f4_t*>(sh.u + quad_at(i)) = u;
                 if (outputs) {

@@ -237,7 +237,7 @@ rms_norm_add_norm_regs_kernel(const float* __restrict__ x, const float* __restri
     ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        v[i] = active ? fmaf(v[i] * gp[i], inv, res[i]) : 0.f;
+        v[i] = active ? fmaf(v[i] * inv, gp[i], res[i]) : 0.f;
         ss = fmaf(v[i], v[i], ss);
     }
     inv = inverse_rms(row_sum(ss, scratch[1]), per_width, eps);
@@ -245,7 +245,7 @@ rms_norm_add_norm_regs_kernel(const float* __restrict__ x, const float* __restri
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        y[i] = v[i] * gn[i] * inv;
+        y[i] = v[i] * inv * gn[i];
         bad |= !isfinite(v[i]);
     }
     if (active) {

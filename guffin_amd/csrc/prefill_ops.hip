@@ -129,7 +129,7 @@ prefill_joint_kernel(const float* __restrict__ x, const float* __restrict__ resi
     ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        v[i] = fmaf(v[i] * gp[i], inv, res[i]);
+        v[i] = fmaf(v[i] * inv, gp[i], res[i]);
         ss = fmaf(v[i], v[i], ss);
     }
     inv = inverse_rms(block_total(ss, scratch[1], (width + 511) / 512), per_width, eps);
@@ -138,7 +138,7 @@ prefill_joint_kernel(const float* __restrict__ x, const float* __restrict__ resi
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         bad |= !isfinite(v[i]);
-        v[i] = v[i] * gn[i] * inv;
+        v[i] = v[i] * inv * gn[i];
     }
     if (active) {
         if (image) emit_image_values(v, t, r, image_layout(rows, width), image);

@@ -242,3 +242,36 @@ def test_rings_that_lie_off_16_bytes(hip, off):
     torch.cuda.synchronize()
     assert int(got[4].item()) == 0 and hip.lib().guffin_hip_resident_enabled() == 1
     assert torch.equal(got[0], want)
+
+
+@pytest.mark.parametrize("path", ["operators", "pass", "prompt"])
+def test_gammas_far_from_their_values(hip, path):
+    """Rows of 2^-12 under an epsilon that lets them be normalised, and gammas of 2^-124: value times gamma is a denormal of a few places,
+    normalised value times gamma an ordinary float, and the bits of a larger gamma's, scaled, up to the last place of the few results that
+    are denormals all the same.  (Embedded rows are zeros, so a block's first norm pair has the attention's outputs alone, and the second one
+    adds nothing.)"""
+    import torch
+    from guffin_amd import model
+    shape = replace(model.GEMMA3_270M, layers=1, vocab=1024, ring_global=1024, eps=2.0 ** -40)
+    devm = model.DeviceModel.random(shape, seed=3, position=3)
+    devm.ring_v[0].mul_(2.0 ** -17)
+    embed = torch.zeros(shape.vocab * shape.hidden // 32 * 34, dtype=torch.uint8, device="cuda")
+    post, nothing = torch.empty(shape.hidden, device="cuda"), torch.zeros(shape.hidden, device="cuda")
+    devm.desc.embed_rows, devm.layers[0].norm[3], devm.layers[0].norm[5] = embed.data_ptr(), post.data_ptr(), nothing.data_ptr()
+    hip.set_forward_mode({"operators": 1, "pass": 2, "prompt": 0}[path])
+
+    def run(gamma_post, gamma_out):
+        post.fill_(gamma_post)
+        devm.out_norm.fill_(gamma_out)
+        tokens = torch.tensor([5, 7], dtype=torch.int32, device="cuda")
+        hidden, status = devm.prefill(tokens.repeat(3), 3) if path == "prompt" else devm.forward(tokens, 3)[::4]
+        assert int(status.item()) == 0
+        return hidden.cpu().double()
+    plain, scaled = run(2.0 ** -12, 1.0), run(2.0 ** -12, 2.0 ** -124)
+    assert 0.5 <= float(plain.pow(2).mean().sqrt()) <= 1.0
+    assert float((scaled - plain * 2.0 ** -124).abs().max()) <= 2.0 ** -149
+    # rows of 2^-70 and less leave the second norm's epsilon alone: its factor is 2^20
+    plain, scaled = run(2.0 ** -70, 2.0 ** 80), run(2.0 ** -124, 2.0 ** 80)
+    hip.set_forward_mode(0)
+    assert float(plain.abs().max()) >= 2.0 ** 29
+    assert float((scaled * 2.0 ** 54 - plain).abs().max()) <= 2.0 ** (-149 + 20 + 80 + 54)

@@ -373,3 +373,24 @@ def test_norm_pair_of_rows_and_an_epsilon_below_the_normal_floats(hip, rows_of):
     want = x.double() / ((x.double() ** 2).mean(-1, keepdim=True) + 1e-40).sqrt()
     err = (got[0].cpu().double() - want).abs().max()
     assert float(err) <= 2.0 ** -18 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("planes", [1, 6])
+def test_norm_pair_of_values_that_their_gammas_would_take_out_of_range(hip, planes):
+    """A value and its gamma may lie so far apart that their product is no float although the normalised value's is: gammas that are powers
+    of two give the bits of gammas of one, scaled.  Of results that are denormals the last place is 2^-149; a row whose sum of
+    squares passes the floats is zero times any gamma."""
+    import torch
+    gen = torch.Generator().manual_seed(planes)
+    x = torch.randn(2, 3840, generator=gen)
+    ones, none = torch.ones(3840), torch.zeros(2, 3840)
+    run = lambda v, gp, res, gn: [t.cpu() for t in hip.rms_norm_add_norm((v[None] * torch.tensor([1.0] + [0.0] * (planes - 1))[:, None, None] if planes > 1 else v).cuda(),
+                                                                          gp.cuda(), res.cuda(), gn.cuda(), eps=2.0 ** -60, planes=planes if planes > 1 else None)[:2]]
+    for size, gamma in ((2.0 ** 56, 2.0 ** 100), (2.0 ** -20, 2.0 ** -124)):
+        plain, scaled = run(x * size, ones, none, ones), run(x * size, gamma * ones, none, ones)
+        assert float((scaled[0].double() - plain[0].double() * gamma).abs().max()) <= 2.0 ** -149
+        plain, scaled = run(x, 0 * ones, x * size, ones), run(x, 0 * ones, x * size, gamma * ones)
+        assert torch.equal(plain[0], x * size) and bool(torch.isfinite(plain[1]).all())
+        assert float((scaled[1].double() - plain[1].double() * gamma).abs().max()) <= 2.0 ** -149
+    huge = run(x * 1e25, 2.0 ** 100 * ones, x, ones)
+    assert torch.equal(huge[0], x)
