@@ -275,7 +275,7 @@ law_cdf_select_kernel(uint32_t vocab, bool greedy, uint64_t seed, uint64_t step,
 // duplicates and places come out of one walk over the record; a sum whose order matters is one lane's, the masses of q another
 // wave's beside it; running sums are kept, so that a draw is found by all
 // lanes at once; at temperatures of 1 and 0 the tempered weights are the raw ones and their sums are not taken twice.
-// An accepted proposal over 64 candidates takes 10.2 us (twice that with a row after the other, and a step after the other inside).
+// An accepted proposal over 64 candidates takes 10.0 us (twice that with a row after the other, and a step after the other inside).
 constexpr uint32_t kTeam = kMaxCandidates;   // threads of a row, a candidate each
 
 struct Prepared {
@@ -290,7 +290,8 @@ struct RowScratch {
     uint64_t keys[kMaxCandidates], sorted[kMaxCandidates];
     float raw[kMaxCandidates];
     double w[kMaxTopK];              // raw weights, zeros behind the last entry
-    double lost[kMaxTopK];           // what the running sums of the weights lost, entry by entry; then the sums of that
+    double lost[kMaxTopK];           // what the running sums of the weights lost, entry by entry
+    double lost_all;
     uint32_t hist[kHistoryCap];
     uint32_t kept, cut;              // ends of the top-p and min-p prefixes
     uint32_t dup, unique, flag, pick;
@@ -299,7 +300,7 @@ struct RowScratch {
 
 // Neumaier's compensated sum over v[0] ... v[i] is run[i] plus the sum of what its additions lost: the terms of that sum are every
 // lane's own where the running sums are known, and what is left of the order are additions.  (All of it by one lane, an entry after
-// the other, beside the plain sums: an accepted proposal 10.4 us, so 10.2.)
+// the other, beside the plain sums: an accepted proposal 10.4 us, so 10.0.)
 __device__ __forceinline__ double lost_by(const double* __restrict__ v, const double* __restrict__ run, uint32_t i) {
     const double w = v[i], total = i ? run[i - 1] : 0.0, sum = run[i];
     return total >= w ? (total - sum) + w : (w - sum) + total;
@@ -495,7 +496,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
     }
     if (team == 0 && t < kMaxTopK) sc.lost[t] = t < count ? lost_by(out.weight, out.run, t) : 0.0;
     __syncthreads();
-    if (team == 0 && t == 64) ordered_sums(sc.lost, count, sc.lost);
+    if (team == 0 && t == 64) sc.lost_all = ordered_sums<double>(sc.lost, count, nullptr);
     const double norm = count ? out.run[count - 1] : 0.0;
     if (!rc && (!isfinite(norm) || norm <= 0.0)) rc = -7;
     if (t == 0) { out.count = rc ? 0u : count; out.total = norm; if (team == 1) sc.err = rc; }
@@ -524,7 +525,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
     double proposed = 0.0, normalization = -1.0;
     if (head && !code) {
         auto unit = [](double u) { return isfinite(u) && u >= 0.0 && u < 1.0; };
-        normalization = norm + scratch[0].lost[count - 1];
+        normalization = norm + scratch[0].lost_all;
         const bool valid = total_usable(count, norm) && !sc.flag && total_holds(normalization, norm, count);
         uint64_t gathered = 0;
         for (uint32_t w = 0; w < kTeam / 64; ++w) gathered += wave_mass[w];
@@ -561,7 +562,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
     __syncthreads();
     if (head && t < kMaxTopK) sc.lost[t] = t < excess ? lost_by(residual.weight, residual.run, t) : 0.0;
     __syncthreads();
-    if (head && t == 0) ordered_sums(sc.lost, excess, sc.lost);
+    if (head && t == 0) sc.lost_all = ordered_sums<double>(sc.lost, excess, nullptr);
     __syncthreads();
     const double acceptance = s_acceptance, residual_total = excess ? residual.run[excess - 1] : 0.0;
     const bool decided = code == 0;
@@ -577,7 +578,7 @@ spec_accept_kernel(const Candidates* __restrict__ rows, const DraftLaw* __restri
             if (scratch[1].err) code = scratch[1].err - 100;
             else note_first(t < after.count && d.u_next * after.total < after.run[t], t, &sc.pick);
         } else {
-            if (!total_usable(excess, residual_total) || !total_holds(residual_total + sc.lost[excess - 1], residual_total, excess)) code = -26;
+            if (!total_usable(excess, residual_total) || !total_holds(residual_total + sc.lost_all, residual_total, excess)) code = -26;
             else {
                 if (t < excess && !weight_usable(residual.weight[t], residual_total)) sc.flag = 1;
                 note_first(t < excess && d.u_residual * residual_total < residual.run[t], t, &sc.pick);
