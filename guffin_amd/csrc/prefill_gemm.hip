@@ -134,8 +134,6 @@ __device__ __forceinline__ uint4_t from_lds16(const uint8_t* at) { return *reint
 __device__ __forceinline__ uint2_t from_lds8(const uint8_t* at) { return *reinterpret_cast<const uint2_t*>(at); }
 // the wave's requests but the N youngest have arrived and its LDS accesses are done, and so have every wave's
 template <int N>
-__device__ __forceinline__ void arrived() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory"); }
-template <int N>
 __device__ __forceinline__ void arrive() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
 
 // requests on either side keep their order, which the counts above rely on
@@ -451,36 +449,13 @@ __device__ __forceinline__ void q6_quants(const uint4 (&ql)[4], const uint2 (&qh
         q[cg] = as_half8(o[0], o[1], o[2], o[3]);
     }
 }
-// times the lane's scale (a scale covers 16 elements; a word holds those of two column groups for two groups, int8 + 128): q
-// becomes the nearest half of the product, rest what that rounding left
-template <int QD, int C0 = 0, int C1 = 4>
-__device__ __forceinline__ void q6_scaled(const uint32_t (&scw)[4], half8_t (&q)[4], half8_t (&rest)[4]) {
-    auto column = [&]<int CG>(half2_t pair) {
-        const half2_t s = both<CG & 1>(pair);
-        const uint4 v = __builtin_bit_cast(uint4, q[CG]);
-        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
-        uint32_t p[4], r[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const half2_t prod = s * h2(x[k]);
-            p[k] = u2(prod);
-            r[k] = u2(__builtin_elementwise_fma(s, h2(x[k]), -prod));
-        }
-        q[CG] = as_half8(p[0], p[1], p[2], p[3]);
-        rest[CG] = as_half8(r[0], r[1], r[2], r[3]);
-    };
-    auto two = [&]<int P>() {
-        const half2_t pair = h2(__builtin_amdgcn_perm(0x64646464u, scw[2 * P + (QD >> 1)], pair_bytes(QD & 1))) - splat(1152.f);
-        column.template operator()<2 * P>(pair);
-        column.template operator()<2 * P + 1>(pair);
-    };
-    if constexpr (C0 == 0) two.template operator()<0>();
-    if constexpr (C1 == 4) two.template operator()<1>();
+// both column groups' scales of the pair P (a scale covers 16 elements; a word holds those of two column groups for two groups, int8 + 128)
+template <int QD, int P>
+__device__ __forceinline__ half2_t q6_scales(const uint32_t (&scw)[4]) {
+    return h2(__builtin_amdgcn_perm(0x64646464u, scw[2 * P + (QD >> 1)], pair_bytes(QD & 1))) - splat(1152.f);
 }
-// the same of one column group
-template <int QD, int CG>
-__device__ __forceinline__ void q6_scaled_one(const uint32_t (&scw)[4], half8_t& q, half8_t& rest) {
-    const half2_t s = both<CG & 1>(h2(__builtin_amdgcn_perm(0x64646464u, scw[2 * (CG >> 1) + (QD >> 1)], pair_bytes(QD & 1))) - splat(1152.f));
+// times the lane's scale: q becomes the nearest half of the product, rest what that rounding left
+__device__ __forceinline__ void q6_times(half2_t s, half8_t& q, half8_t& rest) {
     const uint4 v = __builtin_bit_cast(uint4, q);
     const uint32_t x[4] = {v.x, v.y, v.z, v.w};
     uint32_t p[4], r[4];
@@ -492,6 +467,16 @@ __device__ __forceinline__ void q6_scaled_one(const uint32_t (&scw)[4], half8_t&
     }
     q = as_half8(p[0], p[1], p[2], p[3]);
     rest = as_half8(r[0], r[1], r[2], r[3]);
+}
+template <int QD>
+__device__ __forceinline__ void q6_scaled(const uint32_t (&scw)[4], half8_t (&q)[4], half8_t (&rest)[4]) {
+    auto two = [&]<int P>() {
+        const half2_t pair = q6_scales<QD, P>(scw);
+        q6_times(both<0>(pair), q[2 * P], rest[2 * P]);
+        q6_times(both<1>(pair), q[2 * P + 1], rest[2 * P + 1]);
+    };
+    two.template operator()<0>();
+    two.template operator()<1>();
 }
 // a half block's scale words from the waves' headers: lanes of k-slices 0, 1 take a group's first scale, of 2, 3 its second
 __device__ __forceinline__ void q6_scale_words(const uint8_t* head, int half, uint32_t j, uint32_t sel, uint32_t (&sc)[4]) {
@@ -641,7 +626,7 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
     auto scales = [&](uint32_t blk, int half) { q6_scale_words(heads + (blk & 1) * 5120, half, j, sel, sc); };
     auto form = [&]<int G, int CG>() {
         q6_quants<G & 3, CG, CG + 1>(ql[(G & 7) >> 2], qh[(G & 7) >> 2], b);
-        q6_scaled_one<G & 3, CG>(sc, b[CG], rest[CG]);
+        q6_times(both<CG & 1>(q6_scales<G & 3, (CG >> 1)>(sc)), b[CG], rest[CG]);
     };
     ask_half(b0, 0);
     ask_head(b0);
