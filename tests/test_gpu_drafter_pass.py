@@ -220,14 +220,15 @@ def test_a_model_without_head_norms(hip, rows):
     assert rel_rms(out[1], out[0]) <= 1e-4 and rel_rms(out[0], normed) > 1e-2
 
 
+@pytest.mark.parametrize("heads,rows", [(4, 1), (4, 2), (2, 1), (1, 2)])
 @pytest.mark.parametrize("off", [2, 4, 8, 12])
-def test_rings_that_lie_off_16_bytes(hip, off):
+def test_rings_that_lie_off_16_bytes(hip, off, heads, rows):
     """Lists of several chunks a workgroup, whose later chunks go straight into LDS where the rings are aligned: the same bits."""
     import torch
     from guffin_amd import model
-    shape = replace(model.GEMMA3_270M, layers=2, vocab=1024, ring_global=4096, hidden=128, ffn=256, global_period=2)
+    shape = replace(model.GEMMA3_270M, layers=2, vocab=1024, ring_global=4096, hidden=128, ffn=256, global_period=2, q_heads=heads)
     devm = model.DeviceModel.random(shape, seed=off, position=4000)
-    tokens = torch.tensor([17], dtype=torch.int32, device="cuda")
+    tokens = torch.tensor([17, 999][:rows], dtype=torch.int32, device="cuda")
     hip.set_forward_mode(0)
     want = devm.forward(tokens, 4000)[0].clone()
     kept = []

@@ -826,7 +826,12 @@ def test_a_drafter_s_short_prompt_waits_for_nobody(hip, rows):
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("rows", [6, 16, 17, 32, 33, 72, 80, 97, 100])
 def test_two_teams_a_workgroup(hip, rows, mixed):
-    """Where a workgroup's two teams take half a slice each: of 15 blocks in two and four slices the teams' shares differ by a block."""
+    """Where a workgroup's two teams take half a slice each (looked at first): of 15 blocks in one and two slices the teams' shares differ by a
+    block; the runs have one, two, three and four row tiles a workgroup."""
+    from prefill_cuts import split
+    cuts = [split(name, rows) for name in (("qkv4", "o", "gate_up", "down4") if mixed else ("qkv", "o", "gate_up", "down"))]
+    assert cuts[2].halves and cuts[2].row_tiles == min(-(-rows // 16), 4 if rows > 96 else 3), [(c.row_tiles, c.slices, c.halves) for c in cuts]
+    assert 15 % (2 * cuts[2].slices)
     test_a_short_run_s_splits_are_those_of_shorter_runs(hip, rows, mixed)
 
 
@@ -842,3 +847,27 @@ def test_q8_spans(hip, gfo, K, N, M):
     tiles = hip.repack(0, dev(w), K, N)
     y = hip.prefill_gemm(0, tiles, hip.prefill_pack(dev(x)), M, K, N).cpu().numpy()
     assert_within_operator_bound(gfo, 0, w, x, y, K, N, matrix_path=True)
+
+
+@pytest.mark.parametrize("K,slices", [(512, 2), (512, 3), (768, 5), (1024, 3), (1024, 8), (2048, 7), (2048, 16), (640, 3), (672, 4)])
+@pytest.mark.parametrize("row_tiles,M", [(1, 13), (2, 32), (2, 45), (3, 48), (4, 61)])
+def test_q8_slices_that_begin_inside_a_span(hip, K, slices, row_tiles, M):
+    """Slices are cut by chunks of 64, spans of 256 are four of them: a slice's first and last span may be a part of one, and where K is no
+    multiple of 256 a span is a block and the last chunk may have a single one.  The rms error of such sums is 1.1e-7 to 1.7e-7 of the
+    result's; a part of a span under another's multiplier, or left out, is off by a share of the result itself."""
+    import torch
+    from prefill_cuts import Split, planes
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(K + M)
+    x = torch.randn((M, K), device="cuda", generator=gen)
+    x *= torch.exp2(torch.randint(-9, 1, (M, -(-K // 256)), device="cuda", generator=gen).float()).repeat_interleave(256, 1)[:, :K]
+    w = dev(synth.make_weight(0, K, 64 * 5, seed=K))
+    want = x.double() @ hip.dequant(0, w, 64 * 5 * K // 32).view(64 * 5, K).double().T.contiguous()
+    y, = planes([(0, hip.repack(0, w, K, 64 * 5), 64 * 5)], hip.prefill_pack(x), M, K, Split(row_tiles, slices, 0))
+    ends = [32 * min(K // 32, 2 * (s * ((K // 32 + 1) // 2) // slices)) for s in range(slices + 1)]
+    for s in range(slices):
+        part = slice(ends[s], ends[s + 1])
+        one = x[:, part].double() @ hip.dequant(0, w, 64 * 5 * K // 32).view(64 * 5, K)[:, part].double().T.contiguous()
+        assert float((y[s].double() - one).abs().max() / one.pow(2).mean().sqrt()) <= 1e-5
+    got = y.double().sum(0)
+    assert float(((got - want).pow(2).mean() / want.pow(2).mean()).sqrt()) <= 4e-7
