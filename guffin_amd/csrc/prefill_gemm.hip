@@ -15,6 +15,7 @@
 // the order of a chain counts: Q4_K takes a group's lo half ahead of its hi half and ends a chain after half a block.  rms
 // error against 64 bits in 1e-7 of the result's rms, 333 rows, K = 3840 (Q4_K), 15360 (Q6_K), 2048 (Q8_0): normal activations
 // 1.51, 2.16, 1.61; of a 512-fold range 1.57, 2.20, 1.65; every 97th 200-fold 1.63, 2.29, 1.68; all positive 0.87, 2.16, 1.59.
+// Those of Q8_0 are three and four row tiles'; up to two add a span up under d alone: 1.06, 1.11, 1.17, 1.05.
 // (Kernels of 8 rows, hi and lo in accumulators of their own and Q6_K's -32 a term by itself: 1.56, 3.80, 2.68; 2.24, 4.10,
 // 2.74; 3.31, 12.7, 2.88; 0.88, 6.34, 5.21.  Q4_K hi before lo over whole blocks: 1.78, 1.84, 1.87, 0.78, and 4 % faster.  Its
 // minima or quants as denormal halves need no bias, but the instruction then drops the places they lack: 1.59 on normal ones.)
@@ -713,7 +714,8 @@ __device__ __forceinline__ void q6_walk_wide(const ImageLayout& L, Feed<R> feed,
 // SIMD issues beside the first, and a slice rounds as two while its planes, and the next operator's reads of them, are those of one.  (R = 1, one
 // wave a SIMD 5840 clocks a block, two 8170 for both.  One team taking both halves one after the other, and twice the slices where that was
 // faster, blocks of 12B shapes, us, so / by teams: 10 rows 92.5 / 89.0, 20 rows 105.2 / 102.6, 96 rows 168.5 / 165.8, 128 rows 199.0 / 196.2; of
-// Q4_K alone 37 rows 116.8 / 113.8, 100 rows 183.0 / 174.0.  52 to 64 rows lose a little, 140.3 / 141.4.)
+// Q4_K alone 37 rows 116.8 / 113.8, 100 rows 183.0 / 174.0.  52 to 64 rows lose a little, 140.3 / 141.4; without halves they take 0.3-1.1 % more
+// again.)
 template <int R, int KINDS, int TEAMS = 1>
 __global__ void __launch_bounds__(256 * TEAMS, 2)
 prefill_gemm_kernel(const uint8_t* __restrict__ t0, const uint8_t* __restrict__ t1, const uint8_t* __restrict__ t2, const uint8_t* __restrict__ blob,

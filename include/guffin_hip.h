@@ -460,7 +460,8 @@ int guffin_hip_forward_tree_rows(void* stream, const guffin_model_desc* model, c
  * of 1 or 2 rows have no resident form and run one launch per operator in every mode.  The resident pass keeps one workgroup per CU for a
  * group of blocks, gives each of the 8 XCDs one KV head (models with 8 KV heads; one XCD for a single KV
  * head) and moves a block's intermediate rows through that XCD's L2; only the two reductions of a block
- * cross XCDs.  Every wait in it is bounded by the spin limit (polls of a counter): a workgroup that gives up
+ * cross XCDs.  Every wait in it is bounded by the spin limit (polls of a counter; in the drafter's own pass also
+ * looks at the words that are to come): a workgroup that gives up
  * raises GUFFIN_STATUS_SYNC in the status word and the launch still ends.  Same results as the
  * per-operator path up to fp32 summation order; a row's arithmetic does not depend on the row count in
  * the projections.  No counterpart in the reference (its command buffers are per operator).

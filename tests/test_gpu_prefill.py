@@ -853,7 +853,7 @@ def test_q8_spans(hip, gfo, K, N, M):
 @pytest.mark.parametrize("row_tiles,M", [(1, 13), (2, 32), (2, 45), (3, 48), (4, 61)])
 def test_q8_slices_that_begin_inside_a_span(hip, K, slices, row_tiles, M):
     """Slices are cut by chunks of 64, spans of 256 are four of them: a slice's first and last span may be a part of one, and where K is no
-    multiple of 256 a span is a block and the last chunk may have a single one.  The rms error of such sums is 1.1e-7 to 1.7e-7 of the
+    multiple of 256 a span is a block and the last chunk may have a single one.  The rms error of such sums is 1.0e-7 to 1.7e-7 of the
     result's; a part of a span under another's multiplier, or left out, is off by a share of the result itself."""
     import torch
     from prefill_cuts import Split, planes
